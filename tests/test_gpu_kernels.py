@@ -281,6 +281,34 @@ def test_the_wide_tiles_of_gemm_generic_sum_in_the_same_order(m, n, k):
     assert float(out[:, :4].abs().max()) == 0.0 and float(out[:, n + 4:].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 64, 256), (64, 65, 260), (65, 63, 1028), (200, 33, 3001), (1500, 1500, 1100), (1499, 1503, 2052),
+                                   (2200, 2242, 1030)])
+def test_gemm_generic_cut_over_workgroups_sums_in_the_same_order(m, n, k):
+    """The tiled product with K whole, in slabs and in ranges, at sizes that end inside a tile, a step, a range and a slab:
+    bit for bit the rows that the weight stream gives eight at a time, with a bias and accumulating; from 16-bit operands
+    bit for bit what the same values give in 32-bit."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w = torch.randn(m, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    bias, base = torch.randn(n, generator=g).to(DEV), torch.randn(m, n, generator=g).to(DEV)
+    whole, added = torch.full((m, n), float("nan"), device=DEV), base.clone()
+    kernels.gemm_generic(a, w, bias, whole)
+    kernels.gemm_generic(a, w, bias, added, accumulate=True)
+    assert _rel(whole, a.double() @ w.double().T + bias.double()) < 2e-6
+    padded = torch.nn.functional.pad(a, (0, -k % 4)), torch.nn.functional.pad(w, (0, -k % 4))   # the stream takes K in fours
+    for start in (0, (m - 8) // 2, m - 8):
+        rows = slice(start, start + 8)
+        few, more = torch.empty(8, n, device=DEV), base[rows].clone()
+        kernels.gemm_generic(padded[0][rows], padded[1], bias, few)
+        kernels.gemm_generic(padded[0][rows], padded[1], bias, more, accumulate=True)
+        assert torch.equal(few, whole[rows]) and torch.equal(more, added[rows]), start
+    ha, hw = a.to(torch.bfloat16), w.to(torch.bfloat16)
+    mixed, again = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n, device=DEV)
+    kernels.gemm_generic(ha, hw, bias, mixed)
+    kernels.gemm_generic(ha.float(), hw.float(), bias, again)
+    assert torch.equal(mixed, again.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 4), (3, 70, 36), (8, 3584, 1536), (9, 129, 1028), (16, 1000, 4096), (40, 200, 520),
                                    (64, 333, 2052)])
 def test_gemm_stream_against_float64(m, n, k):

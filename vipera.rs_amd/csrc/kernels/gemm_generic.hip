@@ -17,10 +17,12 @@
 //     never ends at -0);
 //   * the element is +0 + s0 + s1 + ... over its slabs in ascending order, then + bias, then,
 //     when accumulating, old + that.
-// Three kernels follow it. gemm_stream_kernel, for up to 64 rows of A in 32-bit operands, is a stream
-// of the weights: the product of a few tokens is bound by the bytes of W. gemm_generic_kernel is a
-// plain tiled product for everything else, gemm_generic_wide_kernel its twin with larger tiles for
-// 128 rows of A and more.
+// Two kernels follow it. gemm_stream_kernel, for up to 64 rows of A in 32-bit operands, is a stream
+// of the weights: the product of a few tokens is bound by the bytes of W. gemm_matrix_kernel, for
+// everything else, runs on the matrix cores: v_mfma_f32_32x32x2_f32 computes each of its outputs as
+// fma(a[k + 1], w[k + 1], fma(a[k], w[k], c)), rounded after every product (compared with fmaf chains bit
+// for bit, values of all magnitudes, denormal, infinite and NaN ones included), so a chain of these
+// instructions over ascending k is the range's chain above.
 #include "common.h"
 
 namespace {
@@ -28,204 +30,128 @@ constexpr int RANGE_K = 256, SLAB_RANGES = 4, SLAB_K = RANGE_K * SLAB_RANGES;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------------------
-// The tiled product: any operand types, any M. A thread owns a 4 x 4 block of outputs and walks K in
-// steps of 16 through LDS; the three levels of sums above are three sets of accumulators.
-constexpr int BM = 64, BN = 64, BK = 16, TM = 4, TN = 4;
+// The tiled product: any operand types, any M. A workgroup owns 64 x 64 outputs, its four waves 32 x 32 each; K in
+// steps of 16 through two LDS stages, the next step's loads on their way into registers while a step is multiplied, one
+// barrier a step.
+//
+// What bounds it: the matrix cores' 32-bit rate (64 cycles for 32 x 32 x 2, 157 TFLOP/s over the chip) where the
+// tiles fill the chip, the number of workgroups where they do not, and the bytes of W below some 64 rows of A. A wave reads two
+// LDS values per 64 cycles of the matrix core, so LDS is idle. Tiles of 128 x 64 and 128 x 128 ask the caches for less but
+// hold two and four times the accumulators in three sets (the sums' levels), which leaves fewer waves to hide a step's
+// barrier: 2,048 x 37,888 x 3,584 takes 5.23 ms (106 TFLOP/s) here, 5.56 and 6.71 ms with those.
+//
+// UNITS: 0: a workgroup walks all of K and stores C. 1 or 4: a workgroup (blockIdx.y) owns one range or one slab of
+// K and stores its sum to `parts` [unit][M][N]; gemm_parts_finish_kernel adds them, in the order above.
+constexpr int TILE = 64, BK = 16, TILE_ROW = BK + 4;   // a row's 16 k and 4 floats of padding: 8 lanes' 16 bytes lie in 32 different banks
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
-template <typename TA, typename TW, typename TC, bool ACCUMULATE>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
-                                                           const float* __restrict__ bias, TC* __restrict__ C,
-                                                           int M, int N, int K, long long lda, long long ldc) {
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Ws[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int ty = tid / 16, tx = tid % 16;
-  float acc[TM][TN], slab[TM][TN], total[TM][TN];
+// Four consecutive k of a row as floats; VECTOR: K is a multiple of 4 and rows are aligned for one load (a row past
+// the end and a k past the end are read at the last place and cleared by the caller where it matters).
+template <typename T, bool VECTOR>
+__device__ __forceinline__ f32x4_t fetch4(const T* __restrict__ row, int k, int K) {
+  f32x4_t v;
+  if constexpr (VECTOR) {
+    const int at = min(k, K - 4);
+    if constexpr (sizeof(T) == 4) {
+      v = *(const f32x4_t*)(row + at);
+    } else {
+      const bf16x4_t raw = *(const bf16x4_t*)(row + at);
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+      for (int e = 0; e < 4; ++e) v[e] = (float)raw[e];
+    }
+  } else {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = slab[i][j] = total[i][j] = 0.f;
+    for (int e = 0; e < 4; ++e) v[e] = to_float<T>(row[min(k + e, K - 1)]);
+  }
+  return v;
+}
 
-  // each thread stages 4 elements of A and 4 of W per k-tile: row = tid / 4, k = (tid % 4) * 4 + e
-  const int lr = tid / 4, lk = (tid % 4) * 4;
-  for (int k0 = 0; k0 < K; k0 += BK) {
+template <typename TA, typename TW, typename TC, bool ACCUMULATE, int UNITS, bool VECTOR>
+__global__ __launch_bounds__(256) void gemm_matrix_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
+                                                          const float* __restrict__ bias, TC* __restrict__ C,
+                                                          float* __restrict__ parts, int M, int N, int K, long long lda,
+                                                          long long ldc) {
+  __shared__ __attribute__((aligned(16))) float As[2][TILE][TILE_ROW];
+  __shared__ __attribute__((aligned(16))) float Ws[2][TILE][TILE_ROW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the tiles of one run of W's rows follow each other, so that they read it at about the same time
+  const int m_tiles = (M + TILE - 1) / TILE;
+  const int m0 = blockIdx.x % m_tiles * TILE, n0 = blockIdx.x / m_tiles * TILE;
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int k_begin = UNITS ? blockIdx.y * (UNITS * RANGE_K) : 0;
+  const int k_end = UNITS ? min(K, k_begin + UNITS * RANGE_K) : K;
+  f32x16_t acc, slab, total;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = slab[r] = total[r] = 0.f;
+
+  // A thread stages k 4 q .. 4 q + 3 of row tid / 4 of both operands. Instruction t of a step takes k 2 t from lanes
+  // 0 to 31 and k 2 t + 1 from lanes 32 to 63, so a row lies in LDS as its eight even k, then its eight odd ones: a
+  // lane's next four operands are one 16-byte read.
+  const int lr = tid >> 2, q = tid & 3;
+  const TA* a_row = A + (size_t)min(m0 + lr, M - 1) * lda;   // a row past the end is a copy of the last and is not stored
+  const TW* w_row = W + (size_t)min(n0 + lr, N - 1) * K;
+  f32x4_t ra, rw;
+  auto fetch = [&](int k0) {
+    ra = fetch4<TA, VECTOR>(a_row, k0 + 4 * q, K);
+    rw = fetch4<TW, VECTOR>(w_row, k0 + 4 * q, K);
+  };
+  auto stage = [&](int buf, int k0) {
+    const int left = k_end - (k0 + 4 * q);   // a k past the end adds 0 * 0, which changes no sum
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int k = k0 + lk + e;
-      const int am = m0 + lr, wn = n0 + lr;
-      As[lk + e][lr] = (am < M && k < K) ? to_float<TA>(A[(size_t)am * lda + k]) : 0.f;
-      Ws[lk + e][lr] = (wn < N && k < K) ? to_float<TW>(W[(size_t)wn * K + k]) : 0.f;
+      ra[e] = e < left ? ra[e] : 0.f;
+      rw[e] = e < left ? rw[e] : 0.f;
     }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      float a[TM], w[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = As[kk][ty * TM + i];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) w[j] = Ws[kk][tx * TN + j];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-    }
-    __syncthreads();
-    const int done = k0 + BK;  // a multiple of 16, as the range and slab lengths are
-    if (done % RANGE_K == 0 || done >= K) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          slab[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
-        }
-    }
-    if (done % SLAB_K == 0 || done >= K) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          total[i][j] += slab[i][j];
-          slab[i][j] = 0.f;
-        }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + ty * TM + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + tx * TN + j;
-      if (n >= N) continue;
-      float v = total[i][j];
-      if (bias) v += bias[n];
-      TC* dst = C + (size_t)m * ldc + n;
-      if (ACCUMULATE)
-        *dst = from_float<TC>(to_float<TC>(*dst) + v);
-      else
-        *dst = from_float<TC>(v);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// The same product for 128 rows of A and more (prompts): a 128 x 128 tile, a thread owns 8 x 8 outputs (rows
-// 4 ty .. + 3 and 64 + 4 ty .. + 3, columns likewise with tx), so that a step of k costs four 16-byte LDS reads for
-// 64 FMAs where the 4 x 4 block above pays two for 16 and is bound by LDS as much as by arithmetic. The next
-// 16 k of both operands are on their way from memory into registers while this tile's are multiplied, and go
-// into the other half of a double LDS buffer: one barrier per 16 k. Every output element's sums are those of
-// the kernel above, in the same order.
-constexpr int WIDE = 128, WIDE_ROW = WIDE + 4;
-
-template <typename T>
-__device__ __forceinline__ void fetch4(const T* __restrict__ base, long long ld, int row, int rows, int k, int K,
-                                       bool vector_ok, float (&dst)[4]) {
-  if (row < rows && k + 3 < K && vector_ok) {
-    if constexpr (sizeof(T) == 4) {
-      const f32x4_t v = *(const f32x4_t*)(base + (size_t)row * ld + k);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[e] = v[e];
-      return;
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) dst[e] = (row < rows && k + e < K) ? to_float<T>(base[(size_t)row * ld + k + e]) : 0.f;
-}
-
-template <typename TA, typename TW, typename TC, bool ACCUMULATE>
-__global__ __launch_bounds__(256) void gemm_generic_wide_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
-                                                                const float* __restrict__ bias, TC* __restrict__ C,
-                                                                int M, int N, int K, long long lda, long long ldc,
-                                                                int a_vector_ok, int w_vector_ok) {
-  __shared__ __attribute__((aligned(16))) float As[2][BK][WIDE_ROW];
-  __shared__ __attribute__((aligned(16))) float Ws[2][BK][WIDE_ROW];
-  const int tid = threadIdx.x;
-  const int m0 = blockIdx.y * WIDE, n0 = blockIdx.x * WIDE;
-  const int ty = tid / 16, tx = tid % 16;
-  float acc[8][8], slab[8][8], total[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = slab[i][j] = total[i][j] = 0.f;
-
-  // a thread stages rows tid / 4 and 64 + tid / 4 of both operands, k (tid % 4) * 4 .. + 3 of the tile
-  const int lr = tid / 4, lk = (tid % 4) * 4;
-  float ra[2][4], rw[2][4];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      fetch4<TA>(A, lda, m0 + h * 64 + lr, M, k0 + lk, K, a_vector_ok, ra[h]);
-      fetch4<TW>(W, K, n0 + h * 64 + lr, N, k0 + lk, K, w_vector_ok, rw[h]);
-    }
+    *(f32x2_t*)(As[buf][lr] + 2 * q) = f32x2_t{ra[0], ra[2]};
+    *(f32x2_t*)(As[buf][lr] + 8 + 2 * q) = f32x2_t{ra[1], ra[3]};
+    *(f32x2_t*)(Ws[buf][lr] + 2 * q) = f32x2_t{rw[0], rw[2]};
+    *(f32x2_t*)(Ws[buf][lr] + 8 + 2 * q) = f32x2_t{rw[1], rw[3]};
   };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        As[buf][lk + e][h * 64 + lr] = ra[h][e];
-        Ws[buf][lk + e][h * 64 + lr] = rw[h][e];
-      }
-  };
-  fetch(0);
-  stage(0);
+  fetch(k_begin);
+  stage(0, k_begin);
   __syncthreads();
   int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    const bool more = k0 + BK < K;
+  const int in_tile = lane & 31, half = (lane >> 5) * 8;
+  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
+    const bool more = k0 + BK < k_end;
     if (more) fetch(k0 + BK);
-#pragma unroll 4
-    for (int kk = 0; kk < BK; ++kk) {
-      float a[8], w[8];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const f32x4_t av = *(const f32x4_t*)&As[buf][kk][h * 64 + ty * 4];
-        const f32x4_t wv = *(const f32x4_t*)&Ws[buf][kk][h * 64 + tx * 4];
+    for (int t4 = 0; t4 < 2; ++t4) {
+      const f32x4_t a = *(const f32x4_t*)&As[buf][wm + in_tile][half + 4 * t4];
+      const f32x4_t w = *(const f32x4_t*)&Ws[buf][wn + in_tile][half + 4 * t4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          a[h * 4 + e] = av[e];
-          w[h * 4 + e] = wv[e];
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+      for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], w[t], acc, 0, 0, 0);
     }
-    if (more) stage(buf ^ 1);
+    if (more) stage(buf ^ 1, k0 + BK);
     __syncthreads();
     buf ^= 1;
     const int done = k0 + BK;
-    if (done % RANGE_K == 0 || done >= K) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          slab[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
-        }
+    if constexpr (UNITS != 1) {
+      if (done % RANGE_K == 0 || !more) {
+        slab += acc;
+        acc = 0.f;
+      }
     }
-    if (done % SLAB_K == 0 || done >= K) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          total[i][j] += slab[i][j];
-          slab[i][j] = 0.f;
-        }
+    if constexpr (UNITS == 0) {
+      if (done % SLAB_K == 0 || !more) {
+        total += slab;
+        slab = 0.f;
+      }
     }
   }
+  // a lane holds column lane % 32 of its tile, rows 8 (r / 4) + 4 (lane / 32) + r % 4
+  const int n = n0 + wn + in_tile;
+  if (n >= N) return;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + (i / 4) * 64 + ty * 4 + i % 4;
+  for (int r = 0; r < 16; ++r) {
+    const int m = m0 + wm + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
     if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int n = n0 + (j / 4) * 64 + tx * 4 + j % 4;
-      if (n >= N) continue;
-      float v = total[i][j];
+    if constexpr (UNITS != 0) {
+      parts[((size_t)blockIdx.y * M + m) * N + n] = UNITS == 1 ? acc[r] : slab[r];
+    } else {
+      float v = total[r];
       if (bias) v += bias[n];
       TC* dst = C + (size_t)m * ldc + n;
       if (ACCUMULATE)
@@ -236,33 +162,109 @@ __global__ __launch_bounds__(256) void gemm_generic_wide_kernel(const TA* __rest
   }
 }
 
-template <typename TA, typename TW, typename TC>
-int launch(const void* A, const void* W, const float* bias, void* C, int M, int N, int K, long long lda,
-           long long ldc, int accumulate, hipStream_t s) {
-  // the wide tiles where they are enough to occupy a quarter of the GPU at least (2,048 x 37,888 x 3,584: 7.9 ms
-  // against 15.1, 90 % of the rate of unpacked FMAs; 200 x 1,000 x 520, 16 tiles: 107 us against 81)
-  const long long wide_tiles = (long long)((M + WIDE - 1) / WIDE) * ((N + WIDE - 1) / WIDE);
-  if (M >= WIDE && N >= WIDE && wide_tiles >= 64) {
-    dim3 grid((N + WIDE - 1) / WIDE, (M + WIDE - 1) / WIDE);
-    // 16-byte loads where every row of an operand starts on a 16-byte boundary
-    const int a_ok = sizeof(TA) == 4 && ((uintptr_t)A % 16 == 0) && lda % 4 == 0;
-    const int w_ok = sizeof(TW) == 4 && ((uintptr_t)W % 16 == 0) && K % 4 == 0;
-    if (accumulate)
-      gemm_generic_wide_kernel<TA, TW, TC, true><<<grid, 256, 0, s>>>((const TA*)A, (const TW*)W, bias, (TC*)C, M, N, K, lda,
-                                                                      ldc, a_ok, w_ok);
-    else
-      gemm_generic_wide_kernel<TA, TW, TC, false><<<grid, 256, 0, s>>>((const TA*)A, (const TW*)W, bias, (TC*)C, M, N, K, lda,
-                                                                       ldc, a_ok, w_ok);
-    VK_LAUNCH_CHECK();
-    return 0;
+// C = the sum of the parts (+ bias) (+ old C): units of `per_slab` to a slab (4: ranges, 1: slabs), slabs in order.
+// Four consecutive columns a thread where N allows, so that the parts are read 16 bytes at a time.
+template <typename TC, bool ACCUMULATE, int COLUMNS>
+__global__ __launch_bounds__(256) void gemm_parts_finish_kernel(const float* __restrict__ parts,
+                                                                const float* __restrict__ bias, TC* __restrict__ C,
+                                                                int M, int N, long long ldc, int units, int per_slab) {
+  const long long at = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * COLUMNS;
+  if (at >= (long long)M * N) return;
+  const int m = (int)(at / N), n = (int)(at % N);
+  float total[COLUMNS];
+#pragma unroll
+  for (int e = 0; e < COLUMNS; ++e) total[e] = 0.f;
+  const size_t stride = (size_t)M * N;
+  for (int u = 0; u < units; u += per_slab) {
+    float slab[COLUMNS];
+#pragma unroll
+    for (int e = 0; e < COLUMNS; ++e) slab[e] = 0.f;
+#pragma unroll
+    for (int r = 0; r < SLAB_RANGES; ++r) {
+      if (r < per_slab && u + r < units) {
+        const float* from = parts + (size_t)(u + r) * stride + at;
+        if constexpr (COLUMNS == 4) {
+          const f32x4_t v = *(const f32x4_t*)from;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) slab[e] += v[e];
+        } else {
+          slab[0] += from[0];
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < COLUMNS; ++e) total[e] += slab[e];
   }
-  dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-  if (accumulate)
-    gemm_generic_kernel<TA, TW, TC, true><<<grid, 256, 0, s>>>((const TA*)A, (const TW*)W, bias, (TC*)C, M, N, K, lda, ldc);
+#pragma unroll
+  for (int e = 0; e < COLUMNS; ++e) {
+    float v = total[e];
+    if (bias) v += bias[n + e];
+    TC* dst = C + (size_t)m * ldc + n + e;
+    if (ACCUMULATE)
+      *dst = from_float<TC>(to_float<TC>(*dst) + v);
+    else
+      *dst = from_float<TC>(v);
+  }
+}
+
+// How K is cut for a product of M x N: whole (0), in slabs (4) or in ranges (1), so that the workgroups fill the chip
+// (256 CUs, four workgroups each). Measured on tiles x K, us whole / slabs / ranges, weights from memory:
+//   many tiles need no cut, and the parts' way through memory costs: 2,432 x 896: 187 / - / 215; 912 x 896: 83 / - / 89;
+//   2,240 x 1,536: 306 / 315 / 340; but 608 x 896: 67 / - / 63 and 1,120 x 1,536: 183 / 160 / 163;
+//   slabs where those are enough: 384 x 8,960: 446 / 315 / 351; 56 x 18,944: 792 / 121 / 130; 512 x 1,536: 82 / 79 / 85;
+//   ranges below: 112 x 4,864: 175 / 72 / 67; 256 x 1,536: 61 / 50 / 45; 84 x 896: 36 / - / 18; 14 x 4,864: 175 / 43 / 29.
+int matrix_units(int M, int N, int K) {
+  const long long tiles = (long long)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
+  const int ranges = (K + RANGE_K - 1) / RANGE_K, slabs = (K + SLAB_K - 1) / SLAB_K;
+  if (ranges == 1 || ranges > 65535 || tiles >= (slabs == 1 ? 900 : 1200)) return 0;
+  const int units = slabs > 1 && tiles * slabs >= 700 ? SLAB_RANGES : 1;
+  // at most 256 MB of parts (2,048 x 2,048 outputs in 16 slabs)
+  return (long long)(units == 1 ? ranges : slabs) * M * N <= 64ll * 1024 * 1024 ? units : 0;
+}
+
+template <typename TA, typename TW, typename TC, bool ACCUMULATE, int UNITS>
+int launch_tiles(const TA* A, const TW* W, const float* bias, TC* C, float* parts, int M, int N, int K, long long lda,
+                 long long ldc, hipStream_t s) {
+  const long long tiles = (long long)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
+  if (tiles > 0x7fffffff) return VK_UNSUPPORTED_SIZE;
+  dim3 grid((unsigned)tiles, UNITS ? (K + UNITS * RANGE_K - 1) / (UNITS * RANGE_K) : 1);
+  // loads of four k where every row of both operands starts on a boundary of their size
+  const bool vector = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0;
+  if (vector)
+    gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, true><<<grid, 256, 0, s>>>(A, W, bias, C, parts, M, N, K, lda, ldc);
   else
-    gemm_generic_kernel<TA, TW, TC, false><<<grid, 256, 0, s>>>((const TA*)A, (const TW*)W, bias, (TC*)C, M, N, K, lda, ldc);
+    gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, false><<<grid, 256, 0, s>>>(A, W, bias, C, parts, M, N, K, lda, ldc);
   VK_LAUNCH_CHECK();
   return 0;
+}
+
+template <typename TC, bool ACCUMULATE>
+int launch_finish(const float* parts, const float* bias, TC* C, int M, int N, long long ldc, int units, int per_slab,
+                  hipStream_t s) {
+  const long long outputs = (long long)M * N;
+  if (N % 4 == 0)
+    gemm_parts_finish_kernel<TC, ACCUMULATE, 4><<<(unsigned)((outputs / 4 + 255) / 256), 256, 0, s>>>(parts, bias, C, M, N, ldc, units, per_slab);
+  else
+    gemm_parts_finish_kernel<TC, ACCUMULATE, 1><<<(unsigned)((outputs + 255) / 256), 256, 0, s>>>(parts, bias, C, M, N, ldc, units, per_slab);
+  VK_LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename TA, typename TW, typename TC>
+int launch(const void* A_, const void* W_, const float* bias, void* C_, int M, int N, int K, long long lda, long long ldc,
+           int accumulate, int units, float* parts, hipStream_t s) {
+  const TA* A = (const TA*)A_;
+  const TW* W = (const TW*)W_;
+  TC* C = (TC*)C_;
+  if (units == 0)
+    return accumulate ? launch_tiles<TA, TW, TC, true, 0>(A, W, bias, C, parts, M, N, K, lda, ldc, s)
+                      : launch_tiles<TA, TW, TC, false, 0>(A, W, bias, C, parts, M, N, K, lda, ldc, s);
+  const int status = units == 1 ? launch_tiles<TA, TW, float, false, 1>(A, W, nullptr, nullptr, parts, M, N, K, lda, ldc, s)
+                                : launch_tiles<TA, TW, float, false, SLAB_RANGES>(A, W, nullptr, nullptr, parts, M, N, K, lda, ldc, s);
+  if (status != 0) return status;
+  const int count = (K + units * RANGE_K - 1) / (units * RANGE_K), per_slab = SLAB_RANGES / units;
+  return accumulate ? launch_finish<TC, true>(parts, bias, C, M, N, ldc, count, per_slab, s)
+                    : launch_finish<TC, false>(parts, bias, C, M, N, ldc, count, per_slab, s);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -473,24 +475,49 @@ extern "C" int vk_gemm_stream(const float* A, const float* W, const float* bias,
   return 0;
 }
 
+namespace {
+int dispatch(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C, int c_dtype, int M, int N,
+             int K, long long lda, long long ldc, int accumulate, int units, float* parts, hipStream_t s) {
+  switch (a_dtype * 4 + w_dtype * 2 + c_dtype) {
+    case 0: return launch<float, float, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 1: return launch<float, float, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 2: return launch<float, bf16_t, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 3: return launch<float, bf16_t, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 4: return launch<bf16_t, float, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 5: return launch<bf16_t, float, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 6: return launch<bf16_t, bf16_t, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+    case 7: return launch<bf16_t, bf16_t, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
+  }
+  return VK_BAD_ARGUMENT;
+}
+}  // namespace
+
 // dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.
 extern "C" int vk_gemm_generic(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
                                int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
                                void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldc < N) return VK_BAD_ARGUMENT;
-  if ((M + BM - 1) / BM > 65535) return VK_UNSUPPORTED_SIZE;
-  hipStream_t s = (hipStream_t)stream;
-  const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
-  switch (key) {
-    case 0: return launch<float, float, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 1: return launch<float, float, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 2: return launch<float, bf16_t, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 3: return launch<float, bf16_t, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 4: return launch<bf16_t, float, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 5: return launch<bf16_t, float, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 6: return launch<bf16_t, bf16_t, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case 7: return launch<bf16_t, bf16_t, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-  }
-  return VK_BAD_ARGUMENT;
+  if ((M + TILE - 1) / TILE > 65535) return VK_UNSUPPORTED_SIZE;
+  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, 0, nullptr, (hipStream_t)stream);
+}
+
+// Floats of workspace that vk_gemm_generic_split wants for an M x N product over K (0: it is not split).
+extern "C" long long vk_gemm_generic_workspace(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int units = matrix_units(M, N, K);
+  return units ? (long long)((K + units * RANGE_K - 1) / (units * RANGE_K)) * M * N : 0;
+}
+
+// The same product, with K split over workgroups where the tiles alone are too few. `parts`: a workspace of
+// vk_gemm_generic_workspace(M, N, K) floats, aligned to 16 bytes.
+extern "C" int vk_gemm_generic_split(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
+                                     int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
+                                     float* parts, long long part_floats, void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || lda < K || ldc < N) return VK_BAD_ARGUMENT;
+  if ((M + TILE - 1) / TILE > 65535) return VK_UNSUPPORTED_SIZE;
+  if (vk_gemm_generic_workspace(M, N, K) > part_floats || ((uintptr_t)parts & 15)) return VK_BAD_ARGUMENT;
+  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, matrix_units(M, N, K), parts,
+                  (hipStream_t)stream);
 }

@@ -81,13 +81,13 @@ def _cache_ok(k_cache, v_cache, kv_heads: int, head_dim: int, dtype) -> bool:
 _signatures_done = set()
 
 
-def _fn(module: str, name: str, argtypes, key: str = None):
+def _fn(module: str, name: str, argtypes, key: str = None, restype=ctypes.c_int):
     library = load_module(module)
     fn = getattr(library, name)
     key = key or name
     if key not in _signatures_done:
         fn.argtypes = argtypes
-        fn.restype = ctypes.c_int
+        fn.restype = restype
         _signatures_done.add(key)
     return fn
 
@@ -224,7 +224,7 @@ def fill_normal(out: torch.Tensor, key: int, std: float, offset: float = 0.0) ->
 # ----------------------------------------------------------------------------------------------
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                  accumulate: bool = False) -> None:
-    """``out (+)= a @ w.T + bias`` in 32-bit FMA; ``a`` and ``out`` may be row-strided views."""
+    """``out (+)= a @ w.T + bias`` with every product and sum in 32 bits; ``a`` and ``out`` may be row-strided views."""
     _dev(a, w, bias, out)
     _need(a.dim() == 2 and w.dim() == 2 and out.dim() == 2, "gemm: operands must be matrices")
     m, k = a.shape
@@ -239,17 +239,23 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
         _need(out.dtype == torch.float32, "gemm: accumulation needs a float32 output")
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
     ldc = out.stride(0) if m > 1 else max(out.stride(0), n)
-    if (m <= 64 and a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0 and lda % 4 == 0
+    if (m <= 8 and a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0 and lda % 4 == 0
             and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and k < 65535 * 1024):
-        # up to 64 tokens in 32-bit: a stream of the weights (the same sums in the same order as the tiled kernel)
+        # up to 8 tokens in 32-bit: a stream of the weights (the same sums in the same order as the tiled kernel, whose
+        # matrix cores pass the stream's FMAs from there on: 9,728 x 896 at 8 tokens 20.4 us against 21.2, at 16 42.8 against
+        # 21.6; 37,888 x 3,584 at 8 tokens 117 against 204, at 16 219 against 196)
         slabs = _split_k_workspace(a.device, ((k + 1023) // 1024) * m * n, "stream")
         fn = _fn("gemm_generic", "vk_gemm_stream", [_p, _p, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p, _ll, _p])
         _status(fn(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc, 1 if accumulate else 0,
                    _ptr(slabs), slabs.numel(), _stream()), "gemm_stream")
         return
-    fn = _fn("gemm_generic", "vk_gemm_generic", [_p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p])
+    # K split over workgroups where the tiles are too few; the parts belong to this call alone, on whatever stream it runs
+    floats = _fn("gemm_generic", "vk_gemm_generic_workspace", [_i, _i, _i], restype=_ll)(m, n, k)
+    parts = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
+    fn = _fn("gemm_generic", "vk_gemm_generic_split",
+             [_p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p, _ll, _p])
     _status(fn(_ptr(a), _dt(a, "a"), _ptr(w), _dt(w, "w"), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc,
-               1 if accumulate else 0, _stream()), "gemm_generic")
+               1 if accumulate else 0, _ptr(parts), floats, _stream()), "gemm_generic")
 
 
 # ----------------------------------------------------------------------------------------------
