@@ -247,6 +247,37 @@ def test_experts_with_and_without_a_gate(tokens, width, ff, experts, top, plain,
         assert rel_err(got, want) < tol and torch.equal(stream.cpu(), torch.from_numpy(got).to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("tile_rows", [128, 256])
+@pytest.mark.parametrize("plain, weigh_input", [("relu2", False), (None, True)])
+@pytest.mark.parametrize("tokens, width, ff, experts, top", [(37, 64, 64, 5, 2), (130, 320, 192, 3, 1), (700, 192, 448, 3, 2), (330, 128, 64, 1, 1)])
+def test_experts_in_tiles_loaded_straight_into_lds(tokens, width, ff, experts, top, plain, weigh_input, tile_rows):
+    """Widths in whole steps of 64, from one step on: experts with no pairs, with fewer than a wave's rows, one more and many more
+    than a tile's; columns that end inside a tile; activations in rows further apart than they are long.  Against 64 bits, whose
+    distance is that of one rounding to 16 bits in front of the last sum (2^-9 at most, a third of it on average)."""
+    from vipera_rs_amd.ops import kernels
+
+    g = torch.Generator(device="cuda").manual_seed(tokens + ff)
+    h = torch.randn(tokens, width + 64, device="cuda", generator=g).to(torch.bfloat16)[:, :width]
+    z = torch.randn(tokens, experts, device="cuda", generator=g) + (torch.arange(experts, device="cuda") == 1) * 2.0
+    if experts > 3:
+        z[:, 3] = -30.0                                   # nobody's choice
+    gate, up = ((torch.randn(experts, ff, width, device="cuda", generator=g) * width ** -0.5).to(torch.bfloat16) for _ in range(2))
+    down = (torch.randn(experts, width, ff, device="cuda", generator=g) * ff ** -0.5).to(torch.bfloat16)
+    ids, w, offsets, order, tiles, count = route(kernels, z, top, tile_rows)
+    act = torch.full((tokens * top, ff), float("nan"), dtype=torch.bfloat16, device="cuda")
+    pair_out, residual = torch.full((tokens * top, width), float("nan"), device="cuda"), torch.empty(tokens, width, device="cuda")
+    kernels.moe_experts(h, None if plain else gate, up, down, offsets, order, tiles, count, w, top, float("inf"), 1.0, act, pair_out,
+                        residual, False, weigh_input, tile_rows, plain=plain)
+    want = torch.zeros(tokens, width, dtype=torch.float64, device="cuda")
+    for j in range(top):
+        e, share = ids.view(tokens, top)[:, j].long(), w.view(tokens, top)[:, j:j + 1].double()
+        x = h.double() * (share if weigh_input else 1.0)
+        u = torch.bmm(up[e].double(), x[:, :, None])[:, :, 0]
+        y = torch.relu(u) ** 2 if plain else torch.nn.functional.silu(torch.bmm(gate[e].double(), x[:, :, None])[:, :, 0]) * u
+        want += (1.0 if weigh_input else share) * torch.bmm(down[e].double(), y[:, :, None])[:, :, 0]
+    assert rel_err(residual.cpu().numpy(), want.cpu().numpy()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [40, 50, 1000, 4096, 5000])
 def test_a_norm_behind_and_a_layer_norm_in_front_in_one_launch(width, dtype):

@@ -2,7 +2,7 @@
 //
 // A step's T tokens each choose `top` of E experts: P = T * top pairs, pair p = t * top + j.  The pairs are
 // grouped by expert (`order[i]` is the pair at sorted place i, `offsets[e]` the first place of expert e) and cut
-// into tiles of 64 places (128 on the matrix cores, 16 where a step has few pairs) that never span two experts; a
+// into tiles of 64 places (128 or 256 on the matrix cores, 16 where a step has few pairs) that never span two experts; a
 // product's workgroup owns one tile and some output columns.  The grid is sized for the most tiles there can be, and workgroups past `num_tiles` (which only the
 // device knows) leave at once.  Which place a pair gets depends on the order in which the counters were bumped,
 // but no value does: a pair's row is computed alone, an FMA chain in k order per output element, and the
@@ -10,7 +10,7 @@
 #include "common.h"
 #include "group_tile.h"
 
-constexpr int MOE_TILE = 64;      // places per tile of the 32-bit products; the matrix-core products take 128
+constexpr int MOE_TILE = 64;      // places per tile of the 32-bit products; the matrix-core products take 128 or more
 constexpr int MOE_FEW = 16;       // or 16, where the products are streams of the weights
 
 // ---------------------------------------------------------------------------------------------
@@ -304,7 +304,8 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ act
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same two products on the matrix cores (bfloat16): tiles of 128 places, see group_tile.h.  A workgroup of the
+// The same two products on the matrix cores (bfloat16) for widths that are no multiples of 64: tiles of 128 places, see
+// group_tile.h.  A workgroup of the
 // gate/up product owns 64 columns of an expert's width: each wave holds gate and up of the same 32 columns.
 __global__ __launch_bounds__(256) void moe_gate_up_mma_kernel(const __bf16* __restrict__ h, long long ldh,
                                                               const __bf16* __restrict__ wg,
@@ -421,6 +422,111 @@ __global__ __launch_bounds__(256) void moe_down_mma_kernel(const __bf16* __restr
         if (col < width) dst[col] = acc[tn][tm][i];
       }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same products with operands loaded straight into LDS, for widths that are multiples of 64 (group_tile_direct).
+// FORM 0: gate and up, a workgroup owns BN / 2 columns of either; 1: up alone; 2: down.
+//
+// What bounds them: with few pairs an expert the bytes of the weights (32 experts of 1,024 x 2,048, 268 MB for gate and
+// up: 57 us at 64 pairs an expert, 4.7 TB/s), with many the way of the operands from L2 into LDS (about 11 TB/s over the
+// chip: 1.3 GB for 256 pairs an expert in tiles of 128 x 128) and whole rounds of workgroups over the CUs.  2,048 tokens,
+// top 4 of 32: gate and up 150 to 118 us, down 107 to 70 (tiles of 128 x 128 staged through registers before); 512 tokens,
+// up without a gate 61 to 41, down 48 to 30.
+//
+// A workgroup's number says which XCD it runs on (the remainder by eight): each XCD takes a run of neighbouring tiles,
+// and walks them column block by column block, so that the few tiles of an expert read its weights at the same time
+// through one L2.
+template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
+                                                                 const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
+                                                                 const int* __restrict__ offsets,
+                                                                 const int* __restrict__ order, const int* __restrict__ tiles,
+                                                                 const int* __restrict__ num_tiles, int top, int K, int N,
+                                                                 float limit, float alpha, int plain,
+                                                                 const float* __restrict__ in_weights,
+                                                                 __bf16* __restrict__ act, float* __restrict__ pair_out) {
+  constexpr int COLUMNS = FORM == 0 ? BN / 2 : BN, TM = BM / WM / 16, TN = BN / WN / 16;
+  const int blocks = (N + COLUMNS - 1) / COLUMNS, count_tiles = num_tiles[0];
+  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int t0 = (int)((long long)count_tiles * xcd / 8), own = (int)((long long)count_tiles * (xcd + 1) / 8) - t0;
+  if (at >= own * blocks) return;
+  const int tile = t0 + at % own, n0 = at / own * COLUMNS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ unsigned rows[BM];
+  const int e = tiles[2 * tile], first = tiles[2 * tile + 1];
+  const int count = min(BM, offsets[e + 1] - first);
+  for (int i = threadIdx.x; i < BM; i += WM * WN * 64)
+    rows[i] = i < count ? (unsigned)((FORM == 2 ? first + i : order[first + i] / top) * ldi * 2) : GT_NO_ROW;
+  __syncthreads();
+  // weight row r of the tile: the wave's rows are its columns of the gate, then the same columns of up
+  auto column = [&](int r) {
+    if constexpr (FORM != 0) return n0 + r;
+    const int wave_rows = TN * 16, half = TN * 8;
+    return n0 + r / wave_rows * half + r % half;
+  };
+  const long long matrix = (long long)e * N * K, matrix_bytes = (long long)N * K * 2;
+  gt_f32x4 acc[TN][TM];
+  group_tile_direct<BM, BN, WM, WN, STAGES>(
+      gt_view(in, in_bytes), [&](int r) { return rows[r]; }, gt_view(w0 + matrix, matrix_bytes), gt_view(w1 + matrix, matrix_bytes),
+      [&](int r) { const int c = column(r); return c < N ? (unsigned)c * (unsigned)K * 2u : GT_NO_ROW; },
+      [&](int r) { return FORM == 0 && (r / (TN * 8)) % 2 == 1; }, K, count, lds, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm) {
+    const int r = wm * (BM / WM) + tm * 16 + lr;
+    if (r >= count) continue;
+    const float w = FORM != 2 && in_weights ? in_weights[order[first + r]] : 1.f;
+    float* dst = FORM == 2 ? pair_out + (long long)order[first + r] * N : nullptr;
+#pragma unroll
+    for (int tn = 0; tn < (FORM == 0 ? TN / 2 : TN); ++tn) {
+      const int col = n0 + wn * (COLUMNS / WN) + tn * 16 + lg * 4;
+      if (col >= N) continue;                  // N is a multiple of 8: all four or none
+      if constexpr (FORM == 2) {
+        *(gt_f32x4*)(dst + col) = acc[tn][tm];
+      } else {
+        bf16x4 out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          out[i] = (__bf16)(FORM == 0 ? expert_act(w * acc[tn][tm][i], w * acc[tn + TN / 2][tm][i], limit, alpha)
+                                      : plain_act(w * acc[tn][tm][i], plain));
+        *(bf16x4*)(act + (long long)(first + r) * N + col) = out;
+      }
+    }
+  }
+}
+
+template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
+static int launch_direct(const __bf16* in, long long in_rows, long long ldi, const __bf16* w0, const __bf16* w1,
+                         const int* offsets, const int* order, const int* tiles, const int* num_tiles, int max_tiles, int top,
+                         int K, int N, float limit, float alpha, int plain, const float* in_weights, __bf16* act,
+                         float* pair_out, hipStream_t s) {
+  constexpr int COLUMNS = FORM == 0 ? BN / 2 : BN, lds_bytes = gt_direct_lds<BM, BN, STAGES>();
+  static bool sized = false;
+  if (!sized) {
+    const hipError_t e = hipFuncSetAttribute((const void*)moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    sized = true;
+  }
+  // an XCD has at most ceil(tiles / 8) of the tiles, whatever their number turns out to be
+  const long long grid = 8ll * ((max_tiles + 7) / 8) * ((N + COLUMNS - 1) / COLUMNS);
+  if (grid > 0x7fffffff) return VK_UNSUPPORTED_SIZE;
+  moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES><<<(unsigned)grid, WM * WN * 64, lds_bytes, s>>>(
+      in, ((in_rows - 1) * ldi + K) * 2, ldi, w0, w1, offsets, order, tiles, num_tiles, top, K, N, limit, alpha, plain, in_weights,
+      act, pair_out);
+  VK_LAUNCH_CHECK();
+  return 0;
+}
+
+// Tiles of 128 x 128 outputs (two workgroups a CU) or 256 x 256 (one): moe_tile_rows in ops/kernels.py chooses.  Tiles of
+// 320 x 128 were measured too: the fastest where 256 pairs fall to every expert alike (2,048 tokens 180 us against 204 with the
+// weighted sum), the slowest as soon as the experts differ (239 to 247 against 198 to 205), so they are not in.
+template <int FORM, typename... Args>
+static int launch_direct_tiles(int tile_rows, Args... args) {
+  if (tile_rows == GT_WIDE) return launch_direct<FORM, GT_WIDE, 256, 2, 4, 2>(args...);
+  return launch_direct<FORM, GT_TILE, 128, 2, 4, 2>(args...);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -575,10 +681,17 @@ static inline bool moe_on_matrix_cores(int dtype, int width, int ff, long long l
   return dtype == DT_BF16 && width % 8 == 0 && ff % 8 == 0 && ldh % 8 == 0;
 }
 
+// Whether their tiles load straight into LDS: widths in whole steps, and operands within a buffer view each.
+static inline bool moe_loads_direct(int width, int ff, int num_tokens, int top, long long ldh) {
+  return width % GT_BK == 0 && ff % GT_BK == 0 && num_tokens * ldh * 2 <= GT_VIEW_BYTES &&
+         (long long)num_tokens * top * ff * 2 <= GT_VIEW_BYTES && (long long)width * ff * 2 <= GT_VIEW_BYTES;
+}
+
 extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int groups, int keep,
                             int all_scores, const float* correction, float weight_scale, long long ld, int* ids,
                             float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
-  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW) return VK_BAD_ARGUMENT;
+  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE)
+    return VK_BAD_ARGUMENT;
   if (groups < 1 || keep < 1 || keep > groups || experts % groups != 0) return VK_BAD_ARGUMENT;
   if (groups > WAVE) return VK_UNSUPPORTED_SIZE;
   if (keep < groups && (long long)keep * (experts / groups) < top) return VK_BAD_ARGUMENT;
@@ -641,6 +754,25 @@ extern "C" int vk_moe_experts(const void* h, long long ldh, const void* wg, cons
                                                                               offsets, order, tiles, num_tiles, top, ff, width,
                                                                               limit, alpha, 0, nullptr, nullptr, pair_out);
       VK_LAUNCH_CHECK();
+      return launch_combine(pair_out, out_weights, num_tokens, top, width, residual, accumulate, with, s);
+    }
+    if (moe_loads_direct(width, ff, num_tokens, top, ldh)) {
+      const __bf16 *x = (const __bf16*)h, *g = (const __bf16*)wg, *u = (const __bf16*)wu, *d = (const __bf16*)wd;
+      __bf16* a = (__bf16*)act;
+      const int max_tiles = vk_moe_max_tiles(pairs, experts, tile_rows);
+      int status;
+      if (tile_rows != GT_TILE && tile_rows != GT_WIDE) return VK_BAD_ARGUMENT;
+      if (plain)
+        status = launch_direct_tiles<1>(tile_rows, x, (long long)num_tokens, ldh, u, u, offsets, order, tiles, num_tiles, max_tiles,
+                                        top, width, ff, limit, alpha, plain, in_weights, a, (float*)nullptr, s);
+      else
+        status = launch_direct_tiles<0>(tile_rows, x, (long long)num_tokens, ldh, g, u, offsets, order, tiles, num_tiles, max_tiles,
+                                        top, width, ff, limit, alpha, 0, in_weights, a, (float*)nullptr, s);
+      if (status != 0) return status;
+      status = launch_direct_tiles<2>(tile_rows, (const __bf16*)a, (long long)pairs, (long long)ff, d, d, offsets, order, tiles,
+                                      num_tiles, max_tiles, top, ff, width, limit, alpha, 0, (const float*)nullptr,
+                                      (__bf16*)nullptr, pair_out, s);
+      if (status != 0) return status;
       return launch_combine(pair_out, out_weights, num_tokens, top, width, residual, accumulate, with, s);
     }
     if (tile_rows != GT_TILE) return VK_BAD_ARGUMENT;

@@ -1307,13 +1307,30 @@ def head_linear(a: torch.Tensor, a_head_stride: int, k: int, w: torch.Tensor, ou
 MOE_STREAM_PAIRS = 10     # pairs per expert, on average, up to which the experts' products are streams of the weights
 
 
-def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int) -> int:
+def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int, gated: bool = True) -> int:
     """Places per tile of the experts' products for activations ``h`` of ``pairs`` (token, choice) pairs: on the matrix cores
-    (bfloat16, widths that are multiples of 8) 128, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The grouping
-    has to be made for the same number."""
+    (bfloat16, widths that are multiples of 8) 128 or 256, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The
+    grouping has to be made for the same number.
+
+    With widths in whole steps of 64 the tiles are 128 x 128 outputs (two workgroups a CU) or 256 x 256 (one), and a chip full
+    of the second takes 1.6 times as long as one of the first (32 experts of 1,024 x 2,048, gate and up: 60 against 37 us, down
+    37 against 23).  Experts are taken to fill their last tile to a half, as they do when tokens prefer some of them:
+    3,000 tokens, top 4 of 32, products and sum 267 us in tiles of 128, 217 to 231 in 256 (282 where half the tokens choose
+    one expert); 2,048 tokens 198 to 205 and 206 to 214; 1,383 tokens 150 to 164 and 133 (all experts alike) to 192."""
     if not (h.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and h.stride(0) % 8 == 0):
         return 64
-    return 16 if pairs <= MOE_STREAM_PAIRS * experts else 128
+    if pairs <= MOE_STREAM_PAIRS * experts:
+        return 16
+    tokens = max(1, h.shape[0])
+    if width % 64 or ff % 64 or max(tokens * h.stride(0), pairs * ff, width * ff) * 2 >= 2 ** 31 - 1:
+        return 128
+
+    def cost(rows: int, columns: int, slots: int) -> float:
+        tiles = experts * (pairs / experts / rows + 0.5)
+        fills = lambda n: max(1.0, tiles * -(-n // columns) / slots)
+        return fills(2 * ff if gated else ff) * width + fills(width) * ff
+
+    return 256 if 1.6 * cost(256, 256, 256) < 0.95 * cost(128, 128, 512) else 128
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 64) -> int:
@@ -1339,7 +1356,7 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     _f32(weights, "moe_route: weights")
     _need(ids.numel() == tokens * top and weights.numel() == tokens * top and order.numel() == tokens * top
           and offsets.numel() == experts + 1 and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and num_tiles.numel() == 1 and tile_rows in (16, 64, 128), "moe_route: output sizes")
+          and num_tiles.numel() == 1 and tile_rows in (16, 64, 128, 256), "moe_route: output sizes")
     _need(1 <= keep <= groups <= 64 and experts % groups == 0 and (keep == groups or keep * (experts // groups) >= top),
           f"moe_route: {keep} of {groups} groups of {experts} experts for top {top}")
     mode = {"sigmoid": 2, "steered": 3}.get(all_scores, 1 if all_scores else 0)
@@ -1393,7 +1410,7 @@ def moe_experts(h: torch.Tensor, w_gate: Optional[torch.Tensor], w_up: torch.Ten
     _i32(offsets, order, tiles, num_tiles)
     _need(offsets.numel() == experts + 1 and order.numel() == tokens * top
           and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, 128),
+          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, 128, 256),
           "moe_experts: grouping (made by moe_route with the tile_rows that moe_tile_rows gives)")
     fn = _fn("moe", "vk_moe_experts", [_p, _ll, _p, _p, _p, _i, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f, _f, _i, _p, _p,
                                        _p, _i, _i, _p, _p, _ll, _p, _p])

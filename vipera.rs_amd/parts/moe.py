@@ -156,7 +156,7 @@ class MixtureOfExperts(FeedForward):
         rows = torch.empty((tokens, self.w_router.shape[0]), dtype=torch.float32, device=device)
         linear(h, self.w_router, self.b_router, rows)
         logits = rows[:, self.router_col:self.router_col + self.experts]
-        tile_rows = kernels.moe_tile_rows(h, self.hidden, self.inter, pairs, self.experts)
+        tile_rows = kernels.moe_tile_rows(h, self.hidden, self.inter, pairs, self.experts, gated=self.plain is None)
         ints = torch.empty(2 * pairs + self.experts + 2 + 2 * kernels.moe_max_tiles(pairs, self.experts, tile_rows),
                            dtype=torch.int32, device=device)
         ids, order = ints[:pairs], ints[pairs:2 * pairs]
