@@ -209,45 +209,6 @@ def test_the_convolution_and_the_selective_scan_alone(sizes):
     assert bool(torch.isnan(state[0]).all())
 
 
-@pytest.mark.parametrize("channels, states", [(300, 5), (40, 8), (257, 16), (64, 20), (12, 64)])
-def test_the_selective_scan_cut_in_time(channels, states):
-    """Portions that end on, before and behind a segment's edge, from zeros and from a state, beside single tokens, against 64
-    bits; with step sizes from almost none to ones that leave nothing of the state; rows outside the entries' stay as they are.
-    The bound is the one of the walk token by token: 32-bit sums of some hundred terms."""
-    from vipera_rs_amd.ops import kernels
-
-    lengths, firsts = (32, 1, 33, 200, 31, 1, 64, 2), (0, 4, 7, 0, 0, 0, 3, 5)
-    tokens, entries = sum(lengths), len(lengths)
-    g = torch.Generator(device="cuda").manual_seed(channels)
-    rand = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
-    x, z, dt = rand(tokens, channels), rand(tokens, channels), 2.0 * rand(tokens, channels) - 2.0
-    low, skip, dt_bias = rand(tokens, 3 + 2 * states), rand(channels), rand(channels)
-    a_log = torch.log1p(15.0 * torch.rand(channels, states, device="cuda", generator=g))
-    b, c = low[:, 3:3 + states], low[:, 3 + states:]
-    floats = kernels.selective_scan_channel_floats(states)
-    state = rand(entries + 1, channels * floats + 3)
-    before = state.clone()
-    ints = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
-    starts, slots = np.cumsum((0,) + lengths), list(range(entries, 0, -1))
-    want, rate = torch.empty(tokens, channels, dtype=torch.float64, device="cuda"), -torch.exp(a_log.double())
-    steps = torch.nn.functional.softplus(dt.double() + dt_bias.double())
-    ends = {}
-    for e in range(entries):
-        S = before[slots[e], :channels * floats].view(channels, floats)[:, :states].double() * (firsts[e] != 0)
-        for t in range(starts[e], starts[e + 1]):
-            S = torch.exp(steps[t][:, None] * rate) * S + (steps[t] * x[t].double())[:, None] * b[t].double()[None]
-            want[t] = (S @ c[t].double() + skip.double() * x[t].double()) * torch.nn.functional.silu(z[t].double())
-        ends[e] = S
-    out = torch.full((tokens, channels), float("nan"), device="cuda")
-    kernels.selective_scan(x, dt.clone(), dt_bias, b, c, a_log, skip, z, state, ints(starts), ints(firsts), ints(slots), out, entries,
-                           longest=max(lengths), shortest=min(lengths))
-    assert rel_err(out.cpu().numpy(), want.cpu().numpy()) < 4e-6
-    for e in range(entries):
-        got = state[slots[e], :channels * floats].view(channels, floats)[:, :states]
-        assert rel_err(got.cpu().numpy(), ends[e].cpu().numpy()) < 4e-6, f"entry {e}"
-    assert torch.equal(state[0], before[0]) and torch.equal(state[:, channels * floats:], before[:, channels * floats:])
-
-
 # --- each mechanism alone: models of one layer ---------------------------------------------------------------------
 def only_left(part):
     return Z.parallel(part, Z.right(16, 4, 2, 2), 1.0, 0.0)

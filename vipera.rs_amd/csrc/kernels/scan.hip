@@ -417,9 +417,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     const float* __restrict__ bmat, const float* __restrict__ cmat, long long ldbc, const float* __restrict__ a_log,
     const float* __restrict__ skip, const float* __restrict__ z, long long ldz, float* __restrict__ state,
     long long state_stride, const int* __restrict__ entry_start, const int* __restrict__ entry_first,
-    const int* __restrict__ slots, int C, int N, int prepared, int singles_only, TO* __restrict__ out) {
+    const int* __restrict__ slots, int C, int N, int prepared, TO* __restrict__ out) {
   const int e = blockIdx.x;
-  if (singles_only && entry_start[e + 1] - entry_start[e] != 1) return;
   const int lane = threadIdx.x & 63;
   const int part = lane & 15;
   const int ch_raw = blockIdx.y * SCAN_CHANNELS + (lane >> 4);
@@ -524,12 +523,12 @@ extern "C" int vk_scan_prepare(float* dt, long long lddt, const float* dt_bias, 
 
 extern "C" long long vk_selective_scan_channel_floats(int states) { return 16LL * lanes_share(states); }
 
-static int launch_selective_scan(const float* x, const float* dtraw, long long lddt, const float* dt_bias,
+extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long lddt, const float* dt_bias,
                                  const float* bmat, const float* cmat, long long ldbc, const float* a_log,
                                  const float* skip, const float* z, long long ldz, float* state,
                                  long long state_stride, const int* entry_start, const int* entry_first,
-                                 const int* slots, int num_entries, int C, int N, int prepared, int singles_only,
-                                 void* out, int out_dtype, void* stream) {
+                                 const int* slots, int num_entries, int C, int N, int prepared, void* out,
+                                 int out_dtype, void* stream) {
   if (num_entries <= 0) return 0;
   if (C < 1 || N < 1) return VK_BAD_ARGUMENT;
   if (N > 256) return VK_UNSUPPORTED_SIZE;
@@ -540,7 +539,7 @@ static int launch_selective_scan(const float* x, const float* dtraw, long long l
 #define VK_SS(RR, TO)                                                                                               \
   selective_scan_kernel<RR, TO><<<grid, SCAN_THREADS, 0, s>>>(x, dtraw, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, \
                                                               z, ldz, state, state_stride, entry_start, entry_first, \
-                                                              slots, C, N, prepared, singles_only, (TO*)out)
+                                                              slots, C, N, prepared, (TO*)out)
 #define VK_SS_R(TO)                       \
   switch (lanes_share(N)) {               \
     case 1: VK_SS(1, TO); break;          \
@@ -555,228 +554,5 @@ static int launch_selective_scan(const float* x, const float* dtraw, long long l
 #undef VK_SS_R
 #undef VK_SS
   VK_LAUNCH_CHECK();
-  return 0;
-}
-
-extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long lddt, const float* dt_bias,
-                                 const float* bmat, const float* cmat, long long ldbc, const float* a_log,
-                                 const float* skip, const float* z, long long ldz, float* state,
-                                 long long state_stride, const int* entry_start, const int* entry_first,
-                                 const int* slots, int num_entries, int C, int N, int prepared, void* out,
-                                 int out_dtype, void* stream) {
-  return launch_selective_scan(x, dtraw, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, z, ldz, state, state_stride, entry_start,
-                               entry_first, slots, num_entries, C, N, prepared, 0, out, out_dtype, stream);
-}
-
-// ---------------------------------------------------------------------------------------------
-// The selective scan of prompts' portions, cut in time.  The recurrence is diagonal, so a segment of SEGMENT tokens can
-// start from zeros: with s_local its end from there, an end from S is exp(A sum(dt)) S + s_local.  Three launches: every
-// segment's end from zeros (and the step sizes' softplus, left in place of dt), the segments' starts one after the other,
-// every segment again from its start, with the outputs.
-//
-// A lane owns a channel with all its states in registers, so that a sum over the states needs no other lane, loads and
-// stores are whole rows of channels, and a token's B and C are the same numbers for the whole wave.  What bounds it is the
-// exponential per token, channel and state (a quarter of the vector rate), taken twice; the form above, sixteen lanes to a
-// channel, walks a portion's tokens one by one on one wave a SIMD (4,096 channels) and is bound by that chain.  4,096
-// channels of 16 states, portions of 1,000 and 834 tokens: 355 us with what that form has taken ahead, 123 here; one of 2,048
-// tokens 575 and 139.
-constexpr int SEGMENT = 32;
-
-// -exp(a_log) log2(e) of a channel's states, zeros past N (and no state there ever leaves zero).
-template <int NP>
-__device__ __forceinline__ void segment_rates(const float* __restrict__ a_log, int N, float (&a)[NP]) {
-#pragma unroll
-  for (int n = 0; n < NP; ++n) a[n] = n < N ? -expf(a_log[min(n, N - 1)]) * 1.44269504088896341f : 0.f;
-}
-
-// The segment of a workgroup and its place in the workspace: entry e's segments lie from entry_start[e] / SEGMENT + e on.
-struct Segment {
-  int t0, t1, slot;
-  bool last, any;
-};
-__device__ __forceinline__ Segment segment_of(const int* __restrict__ entry_start, int e, int index) {
-  const int start = entry_start[e], end = entry_start[e + 1], t0 = start + index * SEGMENT;
-  return Segment{t0, min(t0 + SEGMENT, end), start / SEGMENT + e + index, t0 + SEGMENT >= end, t0 < end && end - start > 1};
-}
-
-// Grid (segments of the longest entry, ceil(C / 256), entries).  OUTPUT false: the end from zeros into `ends`
-// [slot][NP][C], the sum of the step sizes into `steps` [slot][C], softplus(dt + dt_bias) into dt.  OUTPUT true: from the
-// starts in `ends`, with dt as the first launch left it; an entry's last segment leaves its state row.
-template <int NP, bool OUTPUT, typename TO>
-__global__ __launch_bounds__(256) void scan_segment_kernel(
-    const float* __restrict__ x, float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
-    const float* __restrict__ bmat, const float* __restrict__ cmat, long long ldbc, const float* __restrict__ a_log,
-    const float* __restrict__ skip, const float* __restrict__ z, long long ldz, float* __restrict__ state,
-    long long state_stride, int channel_floats, const int* __restrict__ entry_start, const int* __restrict__ slots, int C,
-    int N, float* __restrict__ ends, float* __restrict__ steps, TO* __restrict__ out) {
-  const int e = blockIdx.z;
-  const Segment seg = segment_of(entry_start, e, blockIdx.x);
-  if (!seg.any) return;      // the whole workgroup
-  // the segment's B and C, zeros past N, so that a token's are read by all lanes at one address
-  __shared__ __attribute__((aligned(16))) float b_rows[SEGMENT][NP], c_rows[OUTPUT ? SEGMENT : 1][NP];
-  for (int i = threadIdx.x; i < SEGMENT * NP; i += 256) {
-    const int j = i / NP, n = i % NP;
-    const long long from = (long long)min(seg.t0 + j, seg.t1 - 1) * ldbc + min(n, N - 1);
-    b_rows[j][n] = n < N ? bmat[from] : 0.f;
-    if (OUTPUT) c_rows[j][n] = n < N ? cmat[from] : 0.f;
-  }
-  __syncthreads();
-  const int c = blockIdx.y * 256 + threadIdx.x;
-  if (c >= C) return;
-  float a[NP], s[NP];
-  segment_rates<NP>(a_log + (long long)c * N, N, a);
-  float* mine = ends + (long long)seg.slot * NP * C + c;
-#pragma unroll
-  for (int n = 0; n < NP; ++n) s[n] = OUTPUT ? mine[(long long)n * C] : 0.f;
-  const float bias = dt_bias[c], d = skip[c];
-  float sum_dt = 0.f;
-  constexpr int AHEAD = 4;     // tokens whose numbers are on their way while the ones before are worked on
-  float nx[AHEAD], ndt[AHEAD], nz[AHEAD];
-  auto fetch = [&](int first) {
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      const long long t = min(first + j, seg.t1 - 1);
-      nx[j] = x[t * C + c];
-      ndt[j] = dt[t * lddt + c];
-      if (OUTPUT) nz[j] = z[t * ldz + c];
-    }
-  };
-  fetch(seg.t0);
-  for (int tb = seg.t0; tb < seg.t1; tb += AHEAD) {
-    float cx[AHEAD], cdt[AHEAD], cz[AHEAD];
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      cx[j] = nx[j];
-      cdt[j] = ndt[j];
-      cz[j] = OUTPUT ? nz[j] : 0.f;
-    }
-    if (OUTPUT || tb + AHEAD < seg.t1) fetch(tb + AHEAD);
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      const int t = tb + j;
-      if (t >= seg.t1) break;
-      const float* b = b_rows[t - seg.t0];
-      const float step = OUTPUT ? cdt[j] : scan_softplus(cdt[j] + bias), dtx = step * cx[j];
-      if (!OUTPUT) {
-        dt[(long long)t * lddt + c] = step;
-        sum_dt += step;
-      }
-      float y[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int n = 0; n < NP; ++n) {
-        s[n] = fmaf(__builtin_amdgcn_exp2f(step * a[n]), s[n], dtx * b[n]);
-        if (OUTPUT) y[n & 3] = fmaf(s[n], c_rows[t - seg.t0][n], y[n & 3]);
-      }
-      if (OUTPUT) out[(long long)t * C + c] = from_float<TO>(fmaf(d, cx[j], (y[0] + y[1]) + (y[2] + y[3])) * scan_silu(cz[j]));
-    }
-  }
-  if (!OUTPUT) {
-#pragma unroll
-    for (int n = 0; n < NP; ++n) mine[(long long)n * C] = s[n];
-    steps[(long long)seg.slot * C + c] = sum_dt;
-  } else if (seg.last) {
-    float* row = state + (long long)slots[e] * state_stride + (long long)c * channel_floats;
-#pragma unroll
-    for (int n = 0; n < NP; ++n)
-      if (n < channel_floats) row[n] = s[n];
-  }
-}
-
-// The segments' starts in place of their ends: a thread per (state, channel) walks an entry's segments.
-// Grid (ceil(NP C / 256), entries).
-template <int NP>
-__global__ __launch_bounds__(256) void scan_starts_kernel(const float* __restrict__ a_log, const float* __restrict__ state,
-                                                          long long state_stride, int channel_floats,
-                                                          const int* __restrict__ entry_start,
-                                                          const int* __restrict__ entry_first,
-                                                          const int* __restrict__ slots, int C, int N,
-                                                          float* __restrict__ ends, const float* __restrict__ steps) {
-  const int e = blockIdx.y;
-  const int at = blockIdx.x * 256 + threadIdx.x;
-  if (at >= NP * C) return;
-  const int n = at / C, c = at % C;
-  const int start = entry_start[e], tokens = entry_start[e + 1] - start, count = (tokens + SEGMENT - 1) / SEGMENT;
-  if (tokens <= 1) return;
-  const float a = n < N ? -expf(a_log[(long long)c * N + min(n, N - 1)]) * 1.44269504088896341f : 0.f;
-  float s = 0.f;
-  if (entry_first[e] != 0 && n < N) s = state[(long long)slots[e] * state_stride + (long long)c * channel_floats + n];
-  float* mine = ends + (long long)(start / SEGMENT + e) * NP * C + at;
-  const float* sum = steps + (long long)(start / SEGMENT + e) * C + c;
-  constexpr int AHEAD = 8;
-  for (int k0 = 0; k0 < count; k0 += AHEAD) {
-    float end[AHEAD], dt[AHEAD];
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      const long long k = min(k0 + j, count - 1);
-      end[j] = mine[k * NP * C];
-      dt[j] = sum[k * C];
-    }
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      if (k0 + j >= count) break;
-      mine[(long long)(k0 + j) * NP * C] = s;
-      s = fmaf(__builtin_amdgcn_exp2f(dt[j] * a), s, end[j]);
-    }
-  }
-}
-
-static inline int segment_states(int N) { return N <= 8 ? 8 : N <= 16 ? 16 : N <= 32 ? 32 : 64; }
-
-// Floats of workspace for a step of num_tokens tokens in num_entries entries.
-extern "C" long long vk_selective_scan_segments_workspace(int num_tokens, int num_entries, int C, int N) {
-  return ((long long)num_tokens / SEGMENT + num_entries) * (segment_states(N) + 1) * C;
-}
-
-// `longest`: tokens of the longest entry (or more); `singles`: whether there may be entries of one token, which the form
-// above takes in a launch of its own (a segment of one token would be three launches' work for a state read and written
-// once).  dt of the others is overwritten with softplus(dt + dt_bias).  N at most 64.
-extern "C" int vk_selective_scan_segments(const float* x, float* dt, long long lddt, const float* dt_bias, const float* bmat,
-                                          const float* cmat, long long ldbc, const float* a_log, const float* skip,
-                                          const float* z, long long ldz, float* state, long long state_stride,
-                                          const int* entry_start, const int* entry_first, const int* slots, int num_tokens,
-                                          int num_entries, int longest, int singles, int C, int N, float* work, long long work_floats,
-                                          void* out, int out_dtype, void* stream) {
-  if (num_entries <= 0 || num_tokens <= 0) return 0;
-  if (C < 1 || N < 1 || longest < 1) return VK_BAD_ARGUMENT;
-  if (N > 64 || num_entries > 65535 || (C + 255) / 256 > 65535 || (long long)C * 64 > 0x7fffffff) return VK_UNSUPPORTED_SIZE;
-  const int floats = (int)vk_selective_scan_channel_floats(N);
-  if (state_stride < (long long)C * floats) return VK_BAD_ARGUMENT;
-  if (vk_selective_scan_segments_workspace(num_tokens, num_entries, C, N) > work_floats) return VK_BAD_ARGUMENT;
-  if (singles) {
-    const int status = launch_selective_scan(x, dt, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, z, ldz, state, state_stride,
-                                             entry_start, entry_first, slots, num_entries, C, N, 0, 1, out, out_dtype, stream);
-    if (status != 0) return status;
-  }
-  hipStream_t s = (hipStream_t)stream;
-  const long long places = (long long)num_tokens / SEGMENT + num_entries;
-  float* steps = work + places * segment_states(N) * C;
-  const dim3 grid((longest + SEGMENT - 1) / SEGMENT, (C + 255) / 256, num_entries);
-#define VK_SEGMENTS(NP, TO)                                                                                                 \
-  do {                                                                                                                     \
-    scan_segment_kernel<NP, false, float><<<grid, 256, 0, s>>>(x, dt, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, z, ldz,  \
-                                                               state, state_stride, floats, entry_start, slots, C, N, work, \
-                                                               steps, nullptr);                                             \
-    VK_LAUNCH_CHECK();                                                                                                     \
-    scan_starts_kernel<NP><<<dim3((NP * C + 255) / 256, num_entries), 256, 0, s>>>(a_log, state, state_stride, floats,       \
-                                                                                   entry_start, entry_first, slots, C, N,   \
-                                                                                   work, steps);                            \
-    VK_LAUNCH_CHECK();                                                                                                     \
-    scan_segment_kernel<NP, true, TO><<<grid, 256, 0, s>>>(x, dt, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, z, ldz,      \
-                                                           state, state_stride, floats, entry_start, slots, C, N, work,     \
-                                                           steps, (TO*)out);                                                \
-    VK_LAUNCH_CHECK();                                                                                                     \
-  } while (0)
-#define VK_SEGMENTS_N(TO)                   \
-  switch (segment_states(N)) {              \
-    case 8: VK_SEGMENTS(8, TO); break;      \
-    case 16: VK_SEGMENTS(16, TO); break;    \
-    case 32: VK_SEGMENTS(32, TO); break;    \
-    default: VK_SEGMENTS(64, TO); break;    \
-  }
-  if (out_dtype == DT_F32) { VK_SEGMENTS_N(float) }
-  else if (out_dtype == DT_BF16) { VK_SEGMENTS_N(bf16_t) }
-  else return VK_BAD_ARGUMENT;
-#undef VK_SEGMENTS_N
-#undef VK_SEGMENTS
   return 0;
 }

@@ -1685,29 +1685,15 @@ def causal_conv(x: torch.Tensor, conv: torch.Tensor, bias: Optional[torch.Tensor
                _ptr(out_run), _dt(out_run, "out_run") if out_run is not None else 0, _stream()), "causal_conv")
 
 
-SELECTIVE_SCAN_SEGMENT_STATES = 64       # states a channel that one lane keeps in registers
-# tokens of a step's longest portion from which on its portions are cut in time: 4,096 channels of 16 states, us of the walk
-# token by token (with what it has taken ahead) against the three launches: 64 tokens 26 and 44, 100 34 and 43, 200 66 and 47
-SELECTIVE_SCAN_SEGMENT_TOKENS = 128
-
-
-def selective_scan_segments(longest: int, states: int) -> bool:
-    """Whether :func:`selective_scan` is to run a step whose longest entry has ``longest`` tokens cut in time."""
-    return longest >= SELECTIVE_SCAN_SEGMENT_TOKENS and states <= SELECTIVE_SCAN_SEGMENT_STATES
-
-
 def selective_scan(x: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
                    a_log: torch.Tensor, skip: torch.Tensor, z: torch.Tensor, state: torch.Tensor,
                    entry_start: torch.Tensor, entry_first_pos: torch.Tensor, slots: torch.Tensor, out: torch.Tensor,
-                   num_entries: int, prepared: bool = False, longest: int = 0, shortest: int = 1) -> None:
+                   num_entries: int, prepared: bool = False) -> None:
     """The selective scan over the step's entries in 32-bit: per channel ``c`` and state ``n``
     ``step = softplus(dt + dt_bias); S <- exp(step * -exp(a_log)) S + step x b; y = S . c + skip x``, and
     ``out = y * silu(z)``.  ``x [T, C]`` contiguous; ``dt``, ``z`` row-strided views ``[T, C]``; ``b`` and ``c``
     row-strided views ``[T, N]`` of one buffer; ``state`` starts with ``C * selective_scan_channel_floats(N)`` floats.
-    ``prepared``: ``dt`` already holds ``softplus(dt + dt_bias)`` and ``z`` already ``silu(z)`` (:func:`scan_prepare`).
-    ``longest`` > 0, the tokens of the step's longest entry (:func:`selective_scan_segments` says from how many on): the
-    portions run cut in time, with their ``dt`` overwritten by ``softplus(dt + dt_bias)``; ``shortest``: the tokens of the
-    shortest entry."""
+    ``prepared``: ``dt`` already holds ``softplus(dt + dt_bias)`` and ``z`` already ``silu(z)`` (:func:`scan_prepare`)."""
     _dev(x, dt, dt_bias, b, c, a_log, skip, z, state, entry_start, entry_first_pos, slots, out)
     tokens, channels = x.shape
     states = a_log.shape[1]
@@ -1727,17 +1713,6 @@ def selective_scan(x: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, b: 
           and state.shape[1] >= channels * selective_scan_channel_floats(states), "selective_scan: state row too short")
     _i32(entry_start, entry_first_pos, slots)
     _entries_ok((entry_start, entry_first_pos, slots), num_entries)
-    if longest:
-        _need(not prepared and states <= SELECTIVE_SCAN_SEGMENT_STATES, "selective_scan: segments")
-        floats = _fn("scan", "vk_selective_scan_segments_workspace", [_i, _i, _i, _i], restype=_ll)(tokens, num_entries, channels, states)
-        work = torch.empty(floats, dtype=torch.float32, device=x.device)
-        fn = _fn("scan", "vk_selective_scan_segments", [_p, _p, _ll, _p, _p, _p, _ll, _p, _p, _p, _ll, _p, _ll, _p, _p, _p, _i, _i,
-                                                        _i, _i, _i, _i, _p, _ll, _p, _i, _p])
-        _status(fn(_ptr(x), _ptr(dt), dt.stride(0), _ptr(dt_bias), _ptr(b), _ptr(c), b.stride(0), _ptr(a_log), _ptr(skip),
-                   _ptr(z), z.stride(0), _ptr(state), state.stride(0), _ptr(entry_start), _ptr(entry_first_pos), _ptr(slots),
-                   tokens, num_entries, int(longest), 1 if shortest <= 1 else 0, channels, states, _ptr(work), floats, _ptr(out), _dt(out, "out"),
-                   _stream()), "selective_scan")
-        return
     fn = _fn("scan", "vk_selective_scan", [_p, _p, _ll, _p, _p, _p, _ll, _p, _p, _p, _ll, _p, _ll, _p, _p, _p, _i, _i, _i,
                                            _i, _p, _i, _p])
     _status(fn(_ptr(x), _ptr(dt), dt.stride(0), _ptr(dt_bias), _ptr(b), _ptr(c), b.stride(0), _ptr(a_log), _ptr(skip),

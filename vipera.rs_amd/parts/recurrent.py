@@ -521,16 +521,14 @@ class SelectiveScan(Mixer):
         linear(steps, self.w_dt, None, dt)
         y = self.runtime.empty((tokens, self.inner))
         z = xz[:, self.inner:]
-        segments = kernels.selective_scan_segments(batch.max_count, self.states)
-        ahead = not batch.all_single and not segments
-        if ahead:   # a short portion of a prompt: the step sizes' softplus and the gate's silu once, ahead of the recurrence
+        ahead = not batch.all_single
+        if ahead:   # a prompt's portion: the step sizes' softplus and the gate's silu once, ahead of the recurrence
             gate = torch.empty((tokens, self.inner), **f32)
             kernels.scan_prepare(dt, self.dt_b, z, gate)
             z = gate
         kernels.selective_scan(x32, dt, self.dt_b, low[:, self.rank:self.rank + self.states],
                                low[:, self.rank + self.states:], self.a_log, self.skip, z, state,
-                               batch.entry_start, batch.entry_first_pos, batch.slots, y, entries, prepared=ahead,
-                               longest=batch.max_count if segments else 0, shortest=min(batch.host_counts))
+                               batch.entry_start, batch.entry_first_pos, batch.slots, y, entries, prepared=ahead)
         linear(y, self.w_o, None, residual, accumulate=accumulate)
 
 
