@@ -209,6 +209,58 @@ def test_the_convolution_and_the_selective_scan_alone(sizes):
     assert bool(torch.isnan(state[0]).all())
 
 
+@pytest.mark.parametrize("sizes", [(2, 10, 14), (2, 16, 9), (3, 24, 8), (1, 32, 16), (2, 64, 40), (2, 100, 7), (3, 128, 17), (1, 200, 5), (1, 256, 9)])
+def test_prompts_portions_walk_to_the_same_bits(sizes):
+    """The walk in blocks of tokens against the one token behind token: lengths around the blocks, fresh and continued states,
+    row widths with and without 16-byte alignment."""
+    from vipera_rs_amd.ops import kernels
+
+    heads, dim, vdim = sizes
+    lengths, firsts = (15, 1, 16, 33, 8, 50), (0, 7, 3, 0, 1, 2)
+    rng = np.random.default_rng(9)
+    dev = lambda a, dt=torch.float32: torch.tensor(np.asarray(a), dtype=dt, device="cuda")
+    tokens, qk, floats = sum(lengths), heads * dim, heads * kernels.decay_rule_head_floats(dim, vdim)
+    meta = (dev(np.cumsum([0, *lengths]), torch.int32), dev(firsts, torch.int32), dev([3, 0, 6, 1, 4, 2], torch.int32))
+    start = dev(rng.standard_normal((8, floats + 3)))
+    decay = dev(np.linspace(0.6, 0.99, heads))
+    for extra in (0, 1):
+        proj = dev(rng.standard_normal((tokens, 2 * qk + heads * vdim + extra)))
+        got = []
+        for short in (True, False):
+            state, out = start.clone(), torch.full((tokens, heads * vdim), float("nan"), device="cuda")
+            kernels.decay_rule(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + heads * vdim], False, decay, state, *meta,
+                               heads, dim, vdim, out, len(lengths), short_entries=short)
+            got.append((out, state))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), f"{extra} more columns"
+
+
+@pytest.mark.parametrize("sizes", [(18, 5), (40, 16), (7, 33), (33, 20), (16, 64), (20, 65)])
+def test_a_prepared_selective_scan_walks_to_the_same_bits(sizes):
+    """Steps and gates taken beforehand (the walk in blocks of tokens, up to 64 states) against those taken inside (token
+    behind token): the same functions of the same numbers."""
+    from vipera_rs_amd.ops import kernels
+
+    channels, states = sizes
+    lengths, firsts = (15, 1, 16, 33, 50), (0, 7, 3, 0, 1)
+    rng = np.random.default_rng(10)
+    dev = lambda a, dt=torch.float32: torch.tensor(np.asarray(a), dtype=dt, device="cuda")
+    tokens, floats = sum(lengths), channels * kernels.selective_scan_channel_floats(states)
+    meta = (dev(np.cumsum([0, *lengths]), torch.int32), dev(firsts, torch.int32), dev([3, 0, 5, 1, 2], torch.int32))
+    start = dev(rng.standard_normal((6, floats + 3)))
+    x, z, dt = (dev(rng.standard_normal((tokens, channels))) for _ in range(3))
+    low = dev(rng.standard_normal((tokens, 3 + 2 * states)))
+    a_log, skip, dt_bias = dev(rng.uniform(-1.5, 1.0, (channels, states))), dev(rng.standard_normal(channels)), dev(rng.uniform(-2.0, 0.0, channels))
+    got = []
+    for prepared in (False, True):
+        state, out, step, gate = start.clone(), torch.full_like(x, float("nan")), dt.clone(), z.clone()
+        if prepared:
+            kernels.scan_prepare(step, dt_bias, z, gate)
+        kernels.selective_scan(x, step, dt_bias, low[:, 3:3 + states], low[:, 3 + states:], a_log, skip, gate, state, *meta, out,
+                               len(lengths), prepared)
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 # --- each mechanism alone: models of one layer ---------------------------------------------------------------------
 def only_left(part):
     return Z.parallel(part, Z.right(16, 4, 2, 2), 1.0, 0.0)

@@ -153,12 +153,147 @@ __global__ __launch_bounds__(SCAN_THREADS) void decay_rule_kernel(const float* _
   }
 }
 
+// The same for prompts' portions, with every token's sum and state formed exactly as above.  A workgroup of two waves takes the
+// tokens in blocks through two LDS stages, a block's numbers on their way into registers while the block before is worked on;
+// a whole block is unrolled without a branch, two tokens side by side and the next two's LDS reads before them, so that neither
+// a read nor a sum, which nothing waits for, is waited for alone; lane j of a channel's sixteen keeps token j's sum, so that a block is stored at once.  Above, a token's eight
+// dependent FMAs, four exchanges and a store behind a branch stand in a row on less than a wave a SIMD.  Now the vector
+// instructions of a token bound it (about 33 for 8 key channels a lane).  ALL: dim = 16 R; VEC: and 16-byte rows.
+// Grid (entries, heads, ceil(vdim / 8)).  16 heads of 128 x 128, against that walk: one portion of 2,048 tokens 549 -> 214 us, portions of 1,000 and
+// 834 269 -> 147 us, of 512 138 -> 55 us (without the reads ahead 291, 160 and 75 us).  Short entries stay above: the stages cost
+// a single token more than they save.
+constexpr int RUN_WAVES = 2, RUN_THREADS = RUN_WAVES * 64, RUN_COLS = 4 * RUN_WAVES;
+template <int R, bool ALL, bool VEC>
+__global__ __launch_bounds__(RUN_THREADS) void decay_run_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                long long ldqk, const float* __restrict__ v, long long ldv,
+                                                                const float* __restrict__ decay, float* __restrict__ state,
+                                                                long long state_stride, const int* __restrict__ entry_start,
+                                                                const int* __restrict__ entry_first,
+                                                                const int* __restrict__ slots, int heads, int dim, int vdim,
+                                                                float* __restrict__ o) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int KEYS = 16 * R, BLOCK = R <= 8 ? 16 : 8, QUADS = 8 * R;     // QUADS: 16-byte pieces of a token's k and q
+  constexpr int LOADS = BLOCK * QUADS / RUN_THREADS, STEP = RUN_THREADS / QUADS;
+  static_assert(RUN_THREADS % QUADS == 0 && BLOCK * RUN_COLS <= RUN_THREADS, "a thread's pieces lie in one column");
+  __shared__ __attribute__((aligned(16))) float kq[2][BLOCK][2 * KEYS];
+  __shared__ float vals[2][BLOCK][RUN_COLS];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & 63, part = lane & 15;
+  const int v0 = blockIdx.z * RUN_COLS, mine = (tid >> 6) * 4 + (lane >> 4), vch = v0 + mine;
+  const bool live = vch < vdim;
+  const int vcol = h * vdim + min(vch, vdim - 1);
+  const int t0 = entry_start[e], t1 = entry_start[e + 1];
+  if (t1 <= t0) return;       // the whole workgroup
+  const bool fresh = entry_first[e] == 0;
+  const float rate = decay[h];
+  float* row = state + (long long)slots[e] * state_stride + ((long long)h * vdim + min(vch, vdim - 1)) * KEYS + part * R;
+  float s[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const float old = row[r];
+    s[r] = (fresh || (!ALL && part * R + r >= dim)) ? 0.f : old;
+  }
+  // this thread's pieces of a block: keys (or queries) key .. key + 3 of tokens tid / QUADS + i STEP; a token past the end is
+  // the last one again, a key channel past dim zero
+  const int piece = tid % QUADS, key = piece % (4 * R) * 4, of = tid / QUADS;
+  const float* from = (piece < 4 * R ? k : q) + (long long)h * dim;
+  // in LDS a lane's n-th pieces lie side by side over the sixteen lanes, so that these read them without bank conflicts
+  constexpr int FLOATS = R < 4 ? R : 4;
+  const int place = R <= 4 ? key : (key / 4 % (R / 4) * 16 + key / R) * 4;
+  f32x4 held[LOADS];
+  float held_v = 0.f;
+  const float* v_from = v + h * vdim + min(v0 + tid % RUN_COLS, vdim - 1);
+  auto fetch = [&](int first) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const float* src = from + (long long)min(first + of + i * STEP, t1 - 1) * ldqk;
+      if constexpr (VEC) {
+        held[i] = *(const f32x4*)(src + key);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) held[i][n] = src[ALL ? key + n : min(key + n, dim - 1)];
+      }
+    }
+    held_v = v_from[(long long)min(first + tid / RUN_COLS, t1 - 1) * ldv];
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      if constexpr (!ALL) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) held[i][n] = key + n < dim ? held[i][n] : 0.f;
+      }
+      *(f32x4*)&kq[buf][of + i * STEP][piece < 4 * R ? place : KEYS + place] = held[i];
+    }
+    if (tid < BLOCK * RUN_COLS) vals[buf][tid / RUN_COLS][tid % RUN_COLS] = held_v;
+  };
+  fetch(t0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int tb = t0; tb < t1; tb += BLOCK, buf ^= 1) {
+    const bool more = tb + BLOCK < t1;
+    if (more) fetch(tb + BLOCK);
+    float sums = 0.f;    // lane j of a channel's sixteen: token j's sum
+    auto token = [&](int j, const float (&kj)[R], const float (&qj)[R], float value) {
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        s[r] = fmaf(rate, s[r], kj[r] * value);
+        sum = fmaf(s[r], qj[r], sum);
+      }
+      sum = row16_sum(sum);
+      sums = part == j ? sum : sums;
+    };
+    auto read = [&](int j, float (&kj)[R], float (&qj)[R], float& value) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int at = r / FLOATS * 16 * FLOATS + part * FLOATS + r % FLOATS;
+        kj[r] = kq[buf][j][at];
+        qj[r] = kq[buf][j][KEYS + at];
+      }
+      value = vals[buf][j][mine];
+    };
+    const int count = min(BLOCK, t1 - tb);
+    if (count == BLOCK) {
+      float kp[2][2][R], qp[2][2][R], vp[2][2];     // two tokens at a time, the next two's reads before them
+      read(0, kp[0][0], qp[0][0], vp[0][0]);
+      read(1, kp[0][1], qp[0][1], vp[0][1]);
+#pragma unroll
+      for (int j = 0; j < BLOCK; j += 2) {
+        const int now = j / 2 & 1;
+        if (j + 2 < BLOCK) {
+          read(j + 2, kp[now ^ 1][0], qp[now ^ 1][0], vp[now ^ 1][0]);
+          read(j + 3, kp[now ^ 1][1], qp[now ^ 1][1], vp[now ^ 1][1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        token(j, kp[now][0], qp[now][0], vp[now][0]);
+        token(j + 1, kp[now][1], qp[now][1], vp[now][1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int j = 0; j < count; ++j) {
+        float kj[R], qj[R], value;
+        read(j, kj, qj, value);
+        token(j, kj, qj, value);
+      }
+    }
+    if (live && part < count) o[(long long)(tb + part) * heads * vdim + vcol] = sums;
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  }
+  if (live) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) row[r] = s[r];
+  }
+}
+
 extern "C" long long vk_decay_rule_head_floats(int dim, int vdim) { return (long long)vdim * 16 * lanes_share(dim); }
 
-extern "C" int vk_decay_rule(const float* q, const float* k, long long ldqk, const float* v, long long ldv, int act,
+static int launch_decay_rule(const float* q, const float* k, long long ldqk, const float* v, long long ldv, int act,
                              const float* decay, float* state, long long state_stride, const int* entry_start,
                              const int* entry_first, const int* slots, int num_entries, int heads, int dim, int vdim,
-                             float* o, void* stream) {
+                             int runs, float* o, void* stream) {
   if (num_entries <= 0) return 0;
   if (heads < 1 || dim < 1 || vdim < 1 || heads > 65535) return VK_BAD_ARGUMENT;
   if (dim > 256) return VK_UNSUPPORTED_SIZE;
@@ -167,6 +302,28 @@ extern "C" int vk_decay_rule(const float* q, const float* k, long long ldqk, con
   if (grid.z > 65535) return VK_UNSUPPORTED_SIZE;
   hipStream_t s = (hipStream_t)stream;
   const int share = lanes_share(dim);
+  if (runs) {
+    const dim3 run_grid(num_entries, heads, (vdim + RUN_COLS - 1) / RUN_COLS);
+    const bool quads = dim == 16 * share && ldqk % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & 15) == 0;
+#define VK_RUN_AS(RR, ALL, VEC)                                                                                              \
+  decay_run_kernel<RR, ALL, VEC><<<run_grid, RUN_THREADS, 0, s>>>(q, k, ldqk, v, ldv, decay, state, state_stride, entry_start, \
+                                                                  entry_first, slots, heads, dim, vdim, o)
+#define VK_RUN(RR)                              \
+  if (quads) VK_RUN_AS(RR, true, true);         \
+  else if (dim == 16 * RR) VK_RUN_AS(RR, true, false); \
+  else VK_RUN_AS(RR, false, false)
+    switch (share) {
+      case 1: VK_RUN(1); break;
+      case 2: VK_RUN(2); break;
+      case 4: VK_RUN(4); break;
+      case 8: VK_RUN(8); break;
+      default: VK_RUN(16); break;
+    }
+#undef VK_RUN
+#undef VK_RUN_AS
+    VK_LAUNCH_CHECK();
+    return 0;
+  }
   const bool vec = share >= 4 && dim == 16 * share && ldqk % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & 15) == 0;
 #define VK_DR(RR, VV)                                                                                                 \
   decay_rule_kernel<RR, VV><<<grid, SCAN_THREADS, 0, s>>>(q, k, ldqk, v, ldv, act, decay, state, state_stride,        \
@@ -181,6 +338,23 @@ extern "C" int vk_decay_rule(const float* q, const float* k, long long ldqk, con
 #undef VK_DR
   VK_LAUNCH_CHECK();
   return 0;
+}
+
+extern "C" int vk_decay_rule(const float* q, const float* k, long long ldqk, const float* v, long long ldv, int act,
+                             const float* decay, float* state, long long state_stride, const int* entry_start,
+                             const int* entry_first, const int* slots, int num_entries, int heads, int dim, int vdim,
+                             float* o, void* stream) {
+  return launch_decay_rule(q, k, ldqk, v, ldv, act, decay, state, state_stride, entry_start, entry_first, slots, num_entries,
+                           heads, dim, vdim, 0, o, stream);
+}
+
+// For steps that hold portions of prompts; the inputs' activation is the caller's.
+extern "C" int vk_decay_rule_runs(const float* q, const float* k, long long ldqk, const float* v, long long ldv,
+                                  const float* decay, float* state, long long state_stride, const int* entry_start,
+                                  const int* entry_first, const int* slots, int num_entries, int heads, int dim, int vdim,
+                                  float* o, void* stream) {
+  return launch_decay_rule(q, k, ldqk, v, ldv, 0, decay, state, state_stride, entry_start, entry_first, slots, num_entries,
+                           heads, dim, vdim, 1, o, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -497,6 +671,151 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
   }
 }
 
+// The same for prompts' portions (`prepared`) and up to 64 states, with every token's sum and state formed exactly as above.  A
+// workgroup of four waves (sixteen channels) takes the tokens in blocks of sixteen through two LDS stages, where a state's (a
+// channel's) numbers of neighbouring tokens lie side by side, so that a lane reads four tokens' at once; a block's numbers are on
+// their way into registers while the block before is worked on.  A whole block is unrolled without a branch: the exponentials,
+// products and exchanges of neighbouring tokens, which wait for nothing but the state's one FMA a token, fill each other's
+// latencies.  Lane j of a channel's sixteen keeps token j's sum and finishes that token's output, so that a block's gate, skip and
+// store are one instruction each.  Now the vector instructions of a token bound it (about 25 and an exponential for a state a
+// lane); above it was their latencies, one behind the other on a wave a SIMD.  ALL: N = 16 R.  4,096 channels of 16 states,
+// against that walk: portions of 1,000 and 834 tokens 278 -> 118 us, one of 2,048 473 -> 172 us, of 512 120 -> 45 us.  Beyond
+// 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
+template <int R, bool ALL, typename TO>
+__global__ __launch_bounds__(256) void selective_run_kernel(
+    const float* __restrict__ x, const float* __restrict__ dt, long long lddt, const float* __restrict__ bmat,
+    const float* __restrict__ cmat, long long ldbc, const float* __restrict__ a_log, const float* __restrict__ skip,
+    const float* __restrict__ z, long long ldz, float* __restrict__ state, long long state_stride,
+    const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots, int C, int N,
+    TO* __restrict__ out) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int BLOCK = 16, ROW = BLOCK + 4, STATES = 16 * R;
+  __shared__ __attribute__((aligned(16))) float bc[2][2][STATES][ROW];     // B and C: [state][token]
+  __shared__ __attribute__((aligned(16))) float xdz[2][3][16][ROW];        // x, dt and the gate: [channel][token]
+  const int e = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, part = lane & 15, mine = (tid >> 6) * 4 + (lane >> 4);
+  const int ch_raw = blockIdx.y * 16 + mine, ch = min(ch_raw, C - 1);
+  const bool live = ch_raw < C;
+  const int t0 = entry_start[e], t1 = entry_start[e + 1];
+  if (t1 <= t0) return;       // the whole workgroup
+  const bool fresh = entry_first[e] == 0;
+  float* row = state + (long long)slots[e] * state_stride + (long long)ch * STATES + part * R;
+  float s[R], a[R];
+  bool in[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int n = part * R + r;
+    in[r] = ALL || n < N;
+    const float old = row[r];
+    s[r] = (fresh || !in[r]) ? 0.f : old;
+    a[r] = -expf(a_log[(long long)ch * N + (ALL ? n : min(n, N - 1))]);
+  }
+  const float d = skip[ch];
+  // this thread's numbers of a block: state tid % STATES of tokens tid / STATES + i (256 / STATES), channel tid % 16 of token
+  // tid / 16; a token past the end is the last one again
+  const int state_of = tid % STATES, bc_token = tid / STATES, ch_token = tid / 16;
+  const int bc_col = ALL ? state_of : min(state_of, N - 1);
+  const long long ch_col = min((int)blockIdx.y * 16 + tid % 16, C - 1);
+  float held_b[R], held_c[R], held_x, held_dt, held_z;
+  auto fetch = [&](int first) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const long long at = (long long)min(first + bc_token + i * (256 / STATES), t1 - 1) * ldbc + bc_col;
+      held_b[i] = bmat[at];
+      held_c[i] = cmat[at];
+    }
+    const long long t = min(first + ch_token, t1 - 1);
+    held_x = x[t * C + ch_col];
+    held_dt = dt[t * lddt + ch_col];
+    held_z = z[t * ldz + ch_col];
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      bc[buf][0][state_of][bc_token + i * (256 / STATES)] = held_b[i];
+      bc[buf][1][state_of][bc_token + i * (256 / STATES)] = held_c[i];
+    }
+    xdz[buf][0][tid % 16][ch_token] = held_x;
+    xdz[buf][1][tid % 16][ch_token] = held_dt;
+    xdz[buf][2][tid % 16][ch_token] = held_z;
+  };
+  fetch(t0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int tb = t0; tb < t1; tb += BLOCK, buf ^= 1) {
+    const bool more = tb + BLOCK < t1;
+    if (more) fetch(tb + BLOCK);
+    float sums = 0.f;
+    const int count = min(BLOCK, t1 - tb);
+    if (count == BLOCK) {
+      f32x4 x4[2], dt4[2], b4[2][R], c4[2][R];     // four tokens at a time, the next four's reads before them
+      auto read = [&](int j4, int to) {
+        x4[to] = *(const f32x4*)&xdz[buf][0][mine][j4];
+        dt4[to] = *(const f32x4*)&xdz[buf][1][mine][j4];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          b4[to][r] = *(const f32x4*)&bc[buf][0][part * R + r][j4];
+          c4[to][r] = *(const f32x4*)&bc[buf][1][part * R + r][j4];
+        }
+      };
+      read(0, 0);
+#pragma unroll
+      for (int j4 = 0; j4 < BLOCK; j4 += 4) {
+        const int now = j4 / 4 & 1;
+        if (j4 + 4 < BLOCK) read(j4 + 4, now ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // in phases, each of them over the four tokens, so that none of their chains is waited for alone
+        float keep[4][R], add[4][R], sum[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            keep[j][r] = expf(dt4[now][j] * a[r]);
+            add[j][r] = in[r] ? dt4[now][j] * x4[now][j] * b4[now][r][j] : 0.f;
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          sum[j] = 0.f;
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            s[r] = fmaf(keep[j][r], s[r], add[j][r]);
+            sum[j] = fmaf(s[r], in[r] ? c4[now][r][j] : 0.f, sum[j]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] = row16_sum(sum[j]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sums = part == j4 + j ? sum[j] : sums;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int j = 0; j < count; ++j) {
+        const float step = xdz[buf][1][mine][j], dtx = step * xdz[buf][0][mine][j];
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          s[r] = fmaf(expf(step * a[r]), s[r], in[r] ? dtx * bc[buf][0][part * R + r][j] : 0.f);
+          sum = fmaf(s[r], in[r] ? bc[buf][1][part * R + r][j] : 0.f, sum);
+        }
+        sum = row16_sum(sum);
+        sums = part == j ? sum : sums;
+      }
+    }
+    if (live && part < count)
+      out[(long long)(tb + part) * C + ch] = from_float<TO>(fmaf(d, xdz[buf][0][mine][part], sums) * xdz[buf][2][mine][part]);
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  }
+  if (live) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) row[r] = s[r];
+  }
+}
+
 // dt[t, c] <- softplus(dt[t, c] + dt_bias[c]) in place and gate[t, c] = silu(z[t, c]): what the scan of a prompt's
 // portion would otherwise compute token behind token.
 __global__ void scan_prepare_kernel(float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
@@ -536,7 +855,18 @@ extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long l
   dim3 grid(num_entries, (C + SCAN_CHANNELS - 1) / SCAN_CHANNELS);
   if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
   hipStream_t s = (hipStream_t)stream;
+  const dim3 run_grid(num_entries, (C + 15) / 16);
+#define VK_SS_RUN(RR, ALL, TO)                                                                                        \
+  selective_run_kernel<RR, ALL, TO><<<run_grid, 256, 0, s>>>(x, dtraw, lddt, bmat, cmat, ldbc, a_log, skip, z, ldz, state, \
+                                                             state_stride, entry_start, entry_first, slots, C, N, (TO*)out)
 #define VK_SS(RR, TO)                                                                                               \
+  if constexpr (RR <= 4) {                                                                                          \
+    if (prepared) {                                                                                                 \
+      if (N == 16 * RR) VK_SS_RUN(RR, true, TO);                                                                    \
+      else VK_SS_RUN(RR, false, TO);                                                                                \
+      break;                                                                                                        \
+    }                                                                                                               \
+  }                                                                                                                 \
   selective_scan_kernel<RR, TO><<<grid, SCAN_THREADS, 0, s>>>(x, dtraw, lddt, dt_bias, bmat, cmat, ldbc, a_log, skip, \
                                                               z, ldz, state, state_stride, entry_start, entry_first, \
                                                               slots, C, N, prepared, (TO*)out)
@@ -553,6 +883,7 @@ extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long l
   else return VK_BAD_ARGUMENT;
 #undef VK_SS_R
 #undef VK_SS
+#undef VK_SS_RUN
   VK_LAUNCH_CHECK();
   return 0;
 }

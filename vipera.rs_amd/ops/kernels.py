@@ -1611,11 +1611,12 @@ def selective_scan_channel_floats(states: int) -> int:
 
 def decay_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, silu_inputs: bool, decay: torch.Tensor,
                state: torch.Tensor, entry_start: torch.Tensor, entry_first_pos: torch.Tensor, slots: torch.Tensor,
-               heads: int, dim: int, vdim: int, out: torch.Tensor, num_entries: int) -> None:
+               heads: int, dim: int, vdim: int, out: torch.Tensor, num_entries: int, short_entries: bool = True) -> None:
     """Linear attention with a fixed decay per head, ``S <- decay S + k v^T; o = S^T q``, over the step's entries in
     32-bit; ``q`` and ``k`` are row-strided views ``[T, heads * dim]`` with one stride, ``v [T, heads * vdim]``;
     ``silu_inputs``: all three pass through silu as they are read.  ``state [slots + 1, floats]`` starts with
-    ``heads * decay_rule_head_floats(dim, vdim)`` floats of this layer."""
+    ``heads * decay_rule_head_floats(dim, vdim)`` floats of this layer.  ``short_entries`` False: the step holds portions of
+    prompts (without ``silu_inputs``); the results are the same bits."""
     _dev(q, k, v, decay, state, entry_start, entry_first_pos, slots, out)
     tokens = out.shape[0]
     for t, what in ((q, "q"), (k, "k"), (v, "v"), (decay, "decay"), (state, "state"), (out, "out")):
@@ -1631,6 +1632,12 @@ def decay_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, silu_inputs: b
         raise UnsupportedError(f"decay_rule: a key width of {dim} is above the kernel's limit of {DECAY_RULE_MAX_KEY_DIM}")
     _i32(entry_start, entry_first_pos, slots)
     _entries_ok((entry_start, entry_first_pos, slots), num_entries)
+    if not short_entries and not silu_inputs:
+        fn = _fn("scan", "vk_decay_rule_runs", [_p, _p, _ll, _p, _ll, _p, _p, _ll, _p, _p, _p, _i, _i, _i, _i, _p, _p])
+        _status(fn(_ptr(q), _ptr(k), q.stride(0), _ptr(v), v.stride(0), _ptr(decay), _ptr(state), state.stride(0),
+                   _ptr(entry_start), _ptr(entry_first_pos), _ptr(slots), num_entries, heads, dim, vdim, _ptr(out), _stream()),
+                "decay_rule")
+        return
     fn = _fn("scan", "vk_decay_rule", [_p, _p, _ll, _p, _ll, _i, _p, _p, _ll, _p, _p, _p, _i, _i, _i, _i, _p, _p])
     _status(fn(_ptr(q), _ptr(k), q.stride(0), _ptr(v), v.stride(0), 1 if silu_inputs else 0, _ptr(decay), _ptr(state),
                state.stride(0), _ptr(entry_start), _ptr(entry_first_pos), _ptr(slots), num_entries, heads, dim, vdim,

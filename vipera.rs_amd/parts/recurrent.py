@@ -440,7 +440,8 @@ class DecayAttention(Mixer):
             q, k, v = ready[:, :self.qk], ready[:, self.qk:2 * self.qk], ready[:, 2 * self.qk:]
             inside = False
         kernels.decay_rule(q, k, v, inside, self.decay, state, batch.entry_start,
-                           batch.entry_first_pos, batch.slots, self.heads, self.dim, self.vdim, o, entries)
+                           batch.entry_first_pos, batch.slots, self.heads, self.dim, self.vdim, o, entries,
+                           short_entries=batch.all_single)
         gated = self.runtime.empty((tokens, self.vw))
         if self.norm_kind == "head":
             if self.gate == "none":
