@@ -392,3 +392,65 @@ def test_the_trace_runner_replays_a_schedule(tmp_path, g2):
     for step, want in rows.items():
         got = np.fromfile(out / f"{step}.f32", dtype="<f4").reshape(len(want), cfg["vocab"])
         assert rel_err(got, np.stack(want)) < TOL["float32"]
+
+
+@pytest.mark.parametrize("rule", ["delta", "delta_channel", "wkv"])
+@pytest.mark.parametrize("sizes", [(1, 2, 20, 9), (2, 4, 64, 16), (1, 3, 72, 8), (2, 2, 128, 24), (1, 1, 200, 5)])
+def test_prompts_recurrences_in_whole_and_partial_blocks(rule, sizes):
+    """The walks in blocks of sixteen tokens: a portion at once (whole blocks) and cut into portions of all remainders (its
+    state carried between them) give the same bits, and the recurrence in 64 bits."""
+    from vipera_rs_amd.ops import kernels
+
+    kv_heads, heads, dim, vdim = sizes
+    vdim = dim if rule == "wkv" else vdim
+    lengths = (50, 17)
+    rng = np.random.default_rng(11)
+    tokens = sum(lengths)
+    q, k = (rng.standard_normal((tokens, kv_heads, dim)) for _ in range(2))
+    k /= np.linalg.norm(k, axis=2, keepdims=True)
+    v, beta = rng.standard_normal((tokens, heads, vdim)), rng.uniform(0.1, 0.9, (tokens, heads))
+    keep, bonus = rng.uniform(0.6, 0.99, (tokens, heads, dim)), rng.standard_normal((heads, dim))
+    if rule == "delta":
+        keep[:] = keep[:, :, :1]
+    want = np.zeros((tokens, heads, vdim))
+    for lo, hi in ((0, 50), (50, 67)):
+        state = np.zeros((heads, dim, vdim))
+        for t in range(lo, hi):
+            for h in range(heads):
+                kk, qq = k[t, h // (heads // kv_heads)], q[t, h // (heads // kv_heads)]
+                if rule == "wkv":
+                    kv = np.outer(kk, v[t, h])
+                    want[t, h] = (state[h] + bonus[h][:, None] * kv).T @ qq
+                    state[h] = keep[t, h][:, None] * state[h] + kv
+                else:
+                    state[h] *= keep[t, h][:, None]
+                    state[h] += np.outer(kk, beta[t, h] * (v[t, h] - state[h].T @ kk))
+                    want[t, h] = state[h].T @ qq
+    dev = lambda a, dt=torch.float32: torch.tensor(np.asarray(a), dtype=dt, device="cuda").contiguous()
+    flat = lambda a: dev(a.reshape(tokens, -1))
+    spread = lambda a: flat(np.repeat(a, heads // kv_heads, axis=1))
+    channels = 2 * kv_heads * dim + heads * vdim
+    qkv = torch.cat([flat(q), flat(k), flat(v)] + ([flat(keep)] if rule == "delta_channel" else []), dim=1)
+    r_, k_, v_, w_, beta_, keep_ = spread(q), spread(k), flat(v), flat(keep), dev(beta), dev(keep[:, :, 0])
+
+    def walk(cuts):
+        state = torch.full((3, heads * kernels.recurrent_head_floats(dim, vdim)), float("nan"), device="cuda")
+        out, done = torch.full((tokens, heads * vdim), float("nan"), device="cuda"), [0, 0]
+        for sizes_now in cuts:      # the next tokens of both requests, gathered into one step
+            rows = [list(range(50 * r + done[r], 50 * r + done[r] + n)) for r, n in enumerate(sizes_now)]
+            at = dev(rows[0] + rows[1], torch.long)
+            meta = (dev(np.cumsum([0, *sizes_now]), torch.int32), dev(done, torch.int32), dev([2, 0], torch.int32))
+            got = torch.empty((len(at), heads * vdim), device="cuda")
+            if rule == "wkv":
+                kernels.wkv_rule(r_[at], k_[at], v_[at], w_[at], dev(np.zeros(heads * dim)), dev(bonus.reshape(-1)), state, *meta, dim, heads,
+                                 got, 2, decayed=True)
+            else:
+                kernels.delta_rule(qkv[at][:, :channels], beta_[at], keep_[at] if rule == "delta" else None, state, *meta, kv_heads, dim,
+                                   heads, vdim, got, 2, channel_decay_col=channels if rule == "delta_channel" else -1)
+            out[at] = got
+            done = [d + n for d, n in zip(done, sizes_now)]
+        return out, state[[0, 2]]
+
+    whole, cut = walk([lengths]), walk([(1, 2), (15, 1), (16, 14), (18, 0)])
+    assert torch.equal(whole[0], cut[0]) and torch.equal(whole[1], cut[1])
+    assert rel_err(whole[0].cpu().numpy(), want.reshape(tokens, -1)) < 4e-6     # dim terms a sum and 1 / (1 - keep) tokens' roundings

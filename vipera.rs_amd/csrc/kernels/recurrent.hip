@@ -343,30 +343,43 @@ __global__ __launch_bounds__(256) void wkv_rule_kernel(
 // them each (64 Q >= the state's padded key width), so that one prompt of a few thousand tokens is heads x value
 // channels waves, two or more to a SIMD, each with a short step per token: Q terms a lane, four DPP exchanges inside
 // the rows, and the four rows' sums read by every lane.  A workgroup is eight waves (eight value channels) that share a
-// block's k, q (r, k, decay) in LDS.  What a thread fetches of a block is worked out once, before the first block.
+// block's k, q (r, k, decay) in LDS.  A whole block is unrolled without a branch, with a token's (four tokens') LDS reads
+// before the arithmetic of the token (four) before it, so that only the recurrence itself is waited for: the delta rule's
+// dot product, six exchanges and update, about 130 ns a token at two waves a SIMD; the time mixing has one FMA a token
+// there and its vector instructions and LDS reads bound it.  With a loop of one branch a token, reads right before their
+// use and a number's address worked out by its thread: delta rule, 16 heads of 128 x 128, 2,048 tokens 400 -> 262 us,
+// portions of 1,000 and 834 314 -> 213 us, with a decay per key channel 422 -> 280 and 333 -> 226 us; time mixing, 32
+// heads of 64, 292 -> 157 and 197 -> 114 us.
 constexpr int SCAN_COLS = 8;
 constexpr int SCAN_THREADS = SCAN_COLS * 64;
 
-__device__ __forceinline__ float wave_total(float v) {
-  v = row_sum16(v);
-  const int bits = __float_as_int(v);
-  return __int_as_float(__builtin_amdgcn_readlane(bits, 0)) + __int_as_float(__builtin_amdgcn_readlane(bits, 16)) +
-         (__int_as_float(__builtin_amdgcn_readlane(bits, 32)) + __int_as_float(__builtin_amdgcn_readlane(bits, 48)));
+// (row 0 + row 1) + (row 2 + row 3), to every lane, of a number that is the same in a row's lanes: row 0's joins row 1's
+// and row 2's row 3's, then the first two row 3, whose last lane everybody reads.
+__device__ __forceinline__ float rows_total(float v) {
+  v = dpp_add<0x143>(dpp_add<0x142>(v));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// A block's fetch plan: element x = tid + i * SCAN_THREADS of the block is token x / ROW, column x % ROW; `plan[i]` is
-// token * 2^24 + the column's offset inside the token's row of the source, or -1 for an element that is always zero.
+__device__ __forceinline__ float wave_total(float v) { return rows_total(row_sum16(v)); }
+
+// How a block gets into LDS: a wave takes whole pieces of sixty-four numbers of one token and one kind (k, q, ...), so
+// that where a piece begins is worked out by the scalar unit and a lane only adds its own number; the sixteen tokens'
+// eight values are 128 threads'.  A fetch only issues loads, the same number in every thread and none inside a
+// branch, from addresses that exist whatever the block holds: the entry's last token stands in for tokens past its end,
+// which are never worked on, and a channel past the last is the last one, stored as zero.  A loaded number is first used
+// when it is stored into LDS, a block later, so that nothing waits for memory before the block in between has been
+// worked on.  (Every thread working out its own numbers' addresses took a third of the walk's vector instructions.)
 template <int Q, bool CH>
 __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
     const float* __restrict__ qkv, long long ldq, int g_col, const float* __restrict__ beta,
     const float* __restrict__ decay, float* __restrict__ state, long long state_stride,
     const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots,
     int kv_heads, int dim, int heads, int vdim, int key_pad, int value_pad, float* __restrict__ out) {
-  constexpr int DP = 64 * Q, VOFF = (CH ? 3 : 2) * DP, ROW = VOFF + SCAN_COLS, COUNT = REC_BLOCK * ROW;
-  constexpr int LOADS = (COUNT + SCAN_THREADS - 1) / SCAN_THREADS;
-  __shared__ float rows[COUNT];
+  constexpr int DP = 64 * Q, KINDS = CH ? 3 : 2, VOFF = KINDS * DP, ROW = VOFF + SCAN_COLS;
+  constexpr int TOKENS = REC_BLOCK / SCAN_COLS, PIECES = TOKENS * KINDS * Q;     // a wave's tokens of a block, and their pieces
+  __shared__ float rows[REC_BLOCK * ROW];
   __shared__ float gates[REC_BLOCK][2];
-  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d0 = lane * Q;
   const int v0 = blockIdx.z * SCAN_COLS, v = v0 + wave;
   const bool live = v < vdim;
@@ -378,68 +391,99 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
   float S[Q];
 #pragma unroll
   for (int i = 0; i < Q; ++i) S[i] = (!fresh && kept && d0 + i < key_pad) ? mine[i] : 0.f;
-  int plan[LOADS];
+  int from[Q];        // the lane's number of a piece in each part of a row of key channels
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int x = tid + i * SCAN_THREADS, j = x / ROW, col = x % ROW;
-    int within = -1;
-    if (x < COUNT) {
-      if (col < DP) { if (col < dim) within = kh * dim + col; }
-      else if (col < 2 * DP) { if (col - DP < dim) within = (kv_heads + kh) * dim + col - DP; }
-      else if (CH && col < VOFF) { if (col - 2 * DP < dim) within = g_col + h * dim + col - 2 * DP; }
-      else if (v0 + col - VOFF < vdim) within = 2 * kv_heads * dim + h * vdim + v0 + col - VOFF;
-    }
-    plan[i] = within < 0 ? -1 : (j << 24) | within;
-  }
-  // A fetch only issues loads, every thread the same number of them and none inside a branch, from addresses that
-  // exist whatever the block holds (the entry's last token stands in for tokens past its end, which are never worked
-  // on; column 0 for numbers that are always zero).  A loaded number is first used when it is stored into LDS, a block
-  // later, so that nothing waits for memory before the block in between has been worked on.
-  float held[LOADS], held_gate;
+  for (int c = 0; c < Q; ++c) from[c] = min(c * 64 + lane, dim - 1);
+  const int value_j = tid / SCAN_COLS & (REC_BLOCK - 1), value_col = min(v0 + tid % SCAN_COLS, vdim - 1);
+  const float* values = qkv + 2 * kv_heads * dim + h * vdim + value_col;
+  float held[PIECES], held_value, held_gate;
   const float* gate_src = ((tid & 1) && !CH ? decay : beta) + h;
   auto fetch = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int t = min(t0 + (plan[i] >> 24 & 127), end - 1);
-      held[i] = qkv[(long long)t * ldq + (plan[i] < 0 ? 0 : plan[i] & 0xFFFFFF)];
+    for (int i = 0; i < PIECES; ++i) {
+      const int j = wave * TOKENS + i / (KINDS * Q), kind = i / Q % KINDS;
+      const int col = kind == 0 ? kh * dim : kind == 1 ? (kv_heads + kh) * dim : g_col + h * dim;
+      held[i] = (qkv + (long long)min(t0 + j, end - 1) * ldq + col)[from[i % Q]];
     }
+    held_value = values[(long long)min(t0 + value_j, end - 1) * ldq];
     held_gate = gate_src[(long long)min(t0 + ((tid >> 1) & (REC_BLOCK - 1)), end - 1) * heads];
   };
   fetch(start);
   for (int t0 = start; t0 < end; t0 += REC_BLOCK) {
     __syncthreads();     // the block before has been read
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i)
-      if (tid + i * SCAN_THREADS < COUNT) rows[tid + i * SCAN_THREADS] = plan[i] < 0 ? 0.f : held[i];
+    for (int i = 0; i < PIECES; ++i) {
+      const int j = wave * TOKENS + i / (KINDS * Q), kind = i / Q % KINDS;
+      rows[j * ROW + kind * DP + i % Q * 64 + lane] = i % Q * 64 + lane < dim ? held[i] : 0.f;
+    }
+    if (tid < REC_BLOCK * SCAN_COLS) rows[value_j * ROW + VOFF + tid % SCAN_COLS] = v0 + tid % SCAN_COLS < vdim ? held_value : 0.f;
     if (tid < 2 * REC_BLOCK) gates[tid >> 1][tid & 1] = held_gate;
     __syncthreads();
     fetch(min(t0 + REC_BLOCK, end - 1));
     const int count = min(REC_BLOCK, end - t0);
     float outs = 0.f;      // lane j of every row: its row's part of token j's read-out, which nothing waits for
-    for (int j = 0; j < count; ++j) {
+    auto read = [&](int j, float (&kk)[Q], float (&qq)[Q], float (&gg)[Q], float& b, float& val) {
       const float* row = rows + j * ROW;
-      const float b = gates[j][0], g = gates[j][1], val = row[VOFF + wave];
-      float kk[Q], qq[Q];
+      b = gates[j][0];
+      val = row[VOFF + wave];
+      const float g = gates[j][1];
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
         kk[i] = row[DP + d0 + i];
         qq[i] = row[d0 + i];
+        gg[i] = CH ? row[2 * DP + d0 + i] : g;
       }
-      float dot = 0.f;
+    };
+    // token j's update, with the read-out of the token before from the same state beside it: the update's chain (a dot
+    // product, six exchanges, a lane's sum to all) is what a token costs, and the read-out's lies in its gaps
+    auto token = [&](int j, const float (&kk)[Q], const float (&gg)[Q], float b, float val, const float (&before)[Q]) {
+      float dot = 0.f, o = 0.f;
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        S[i] *= CH ? row[2 * DP + d0 + i] : g;
+        o = fmaf(S[i], before[i], o);
+        S[i] *= gg[i];
         dot = fmaf(S[i], kk[i], dot);
       }
-      const float u = b * (val - wave_total(dot));
+      // the two sums' exchanges in turn: between two of one chain the chip would have to wait
+#define VK_STEP(CTRL)                 \
+  dot = dpp_add<CTRL>(dot);           \
+  if (j) o = dpp_add<CTRL>(o);        \
+  __builtin_amdgcn_sched_barrier(0);
+      VK_STEP(0xB1)
+      VK_STEP(0x4E)
+      VK_STEP(0x141)
+      VK_STEP(0x140)
+#undef VK_STEP
+      const float u = b * (val - rows_total(dot));
+#pragma unroll
+      for (int i = 0; i < Q; ++i) S[i] = fmaf(kk[i], u, S[i]);
+      if (j) outs = (lane & (REC_BLOCK - 1)) == j - 1 ? o : outs;
+    };
+    auto read_out = [&](int j, const float (&qq)[Q]) {
       float o = 0.f;
 #pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        S[i] = fmaf(kk[i], u, S[i]);
-        o = fmaf(S[i], qq[i], o);
-      }
+      for (int i = 0; i < Q; ++i) o = fmaf(S[i], qq[i], o);
       o = row_sum16(o);
       outs = (lane & (REC_BLOCK - 1)) == j ? o : outs;
+    };
+    float kk[2][Q], qq[3][Q], gg[2][Q], b[2], val[2];
+    if (count == REC_BLOCK) {      // a token's LDS reads go before the arithmetic of the token before it
+      read(0, kk[0], qq[0], gg[0], b[0], val[0]);
+#pragma unroll
+      for (int j = 0; j < REC_BLOCK; ++j) {
+        const int now = j & 1, next = now ^ 1;
+        if (j + 1 < REC_BLOCK) read(j + 1, kk[next], qq[(j + 1) % 3], gg[next], b[next], val[next]);
+        __builtin_amdgcn_sched_barrier(0);
+        token(j, kk[now], gg[now], b[now], val[now], qq[(j + 2) % 3]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      read_out(REC_BLOCK - 1, qq[(REC_BLOCK - 1) % 3]);
+    } else {
+      for (int j = 0; j < count; ++j) {
+        read(j, kk[0], qq[0], gg[0], b[0], val[0]);
+        token(0, kk[0], gg[0], b[0], val[0], qq[0]);
+        read_out(j, qq[0]);
+      }
     }
     outs += __shfl_xor(outs, 16, 64);     // (row 0 + row 1) + (row 2 + row 3), in every row
     outs += __shfl_xor(outs, 32, 64);
@@ -452,7 +496,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
   }
 }
 
-// An LDS row of a token: [r: 64Q | k: 64Q | w: 64Q | v: 8]; sources differ by column, so the plan keeps which.
+// An LDS row of a token: [r: 64Q | k: 64Q | w: 64Q | v: 8].
 template <int Q>
 __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
     const float* __restrict__ r, long long ldr, const float* __restrict__ k, long long ldk, const float* __restrict__ v,
@@ -460,9 +504,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
     const float* __restrict__ bonus, float* __restrict__ state, long long state_stride,
     const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots, int dim,
     int heads, int key_pad, int value_pad, int decayed, float* __restrict__ out) {
-  constexpr int DP = 64 * Q, ROW = 3 * DP + SCAN_COLS, COUNT = REC_BLOCK * ROW, LOADS = (COUNT + SCAN_THREADS - 1) / SCAN_THREADS;
-  __shared__ float rows[COUNT];
-  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int DP = 64 * Q, ROW = 3 * DP + SCAN_COLS, TOKENS = REC_BLOCK / SCAN_COLS, PIECES = TOKENS * 3 * Q;
+  __shared__ float rows[REC_BLOCK * ROW];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d0 = lane * Q;
   const int v0 = blockIdx.z * SCAN_COLS, col_v = v0 + wave;
   const bool live = col_v < dim;
@@ -476,55 +521,84 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
     S[i] = (!fresh && kept && d0 + i < key_pad) ? mine[i] : 0.f;
     U[i] = d0 + i < dim ? bonus[h * dim + d0 + i] : 0.f;
   }
-  // kind * 2^28 + token * 2^21 + offset inside the head's dim (kinds: 0 r, 1 k, 2 decay, 3 value), or -1
-  int plan[LOADS];
+  int from[Q];
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int x = tid + i * SCAN_THREADS, j = x / ROW, col = x % ROW;
-    const int kind = col < DP ? 0 : col < 2 * DP ? 1 : col < 3 * DP ? 2 : 3;
-    const int d = kind < 3 ? col - kind * DP : v0 + col - 3 * DP;
-    plan[i] = (x < COUNT && d < dim) ? (kind << 28) | (j << 21) | d : -1;
-  }
-  // A fetch only issues loads, the same number in every thread and none inside a branch, from addresses that exist
-  // whatever the block holds; a loaded number is first used when it is stored into LDS, a block later.
-  float held[LOADS];
+  for (int c = 0; c < Q; ++c) from[c] = min(c * 64 + lane, dim - 1);
+  const int value_j = tid / SCAN_COLS & (REC_BLOCK - 1);
+  const float* values = v + h * dim + min(v0 + tid % SCAN_COLS, dim - 1);
+  float held[PIECES], held_value;
   auto fetch = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int kind = plan[i] >> 28 & 3, d = plan[i] < 0 ? 0 : plan[i] & 0x1FFFFF;
-      const long long t = min(t0 + (plan[i] >> 21 & 127), end - 1);
-      const float* base = kind == 0 ? r + t * ldr : kind == 1 ? k + t * ldk : kind == 2 ? wraw + t * ldw : v + t * ldv;
-      held[i] = base[h * dim + d];
+    for (int i = 0; i < PIECES; ++i) {
+      const int j = wave * TOKENS + i / (3 * Q), kind = i / Q % 3;
+      const long long t = min(t0 + j, end - 1);
+      held[i] = ((kind == 0 ? r + t * ldr : kind == 1 ? k + t * ldk : wraw + t * ldw) + h * dim)[from[i % Q]];
     }
+    held_value = values[min(t0 + value_j, end - 1) * ldv];
   };
   fetch(start);
   for (int t0 = start; t0 < end; t0 += REC_BLOCK) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
+    for (int i = 0; i < PIECES; ++i) {
+      const int j = wave * TOKENS + i / (3 * Q), kind = i / Q % 3;
       float value = held[i];
-      if (!decayed) {      // the same for every thread: the caller has not turned wraw into the decay yet
-        const float shift = w0[h * dim + (plan[i] < 0 ? 0 : plan[i] & 0x1FFFFF)];
-        value = (plan[i] >> 28 & 3) == 2 ? expf(-expf(value + shift)) : value;
-      }
-      if (tid + i * SCAN_THREADS < COUNT) rows[tid + i * SCAN_THREADS] = plan[i] < 0 ? 0.f : value;
+      if (kind == 2 && !decayed) value = expf(-expf(value + w0[h * dim + from[i % Q]]));     // wraw is not the decay yet
+      rows[j * ROW + kind * DP + i % Q * 64 + lane] = i % Q * 64 + lane < dim ? value : 0.f;
     }
+    if (tid < REC_BLOCK * SCAN_COLS) rows[value_j * ROW + 3 * DP + tid % SCAN_COLS] = v0 + tid % SCAN_COLS < dim ? held_value : 0.f;
     __syncthreads();
     fetch(min(t0 + REC_BLOCK, end - 1));
     const int count = min(REC_BLOCK, end - t0);
     float outs = 0.f;      // lane j of every row: its row's part of token j's read-out, which nothing waits for
-    for (int j = 0; j < count; ++j) {
+    constexpr int AHEAD = Q == 1 ? 4 : 2;      // tokens read from LDS before the arithmetic of the AHEAD before them
+    float rr[2][AHEAD][Q], kk[2][AHEAD][Q], ww[2][AHEAD][Q], val[2][AHEAD];
+    auto read = [&](int j, int of, int n) {
       const float* row = rows + j * ROW;
-      const float val = row[3 * DP + wave];
+      val[of][n] = row[3 * DP + wave];
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        rr[of][n][i] = row[d0 + i];
+        kk[of][n][i] = row[DP + d0 + i];
+        ww[of][n][i] = row[2 * DP + d0 + i];
+      }
+    };
+    auto token = [&](int of, int n) {
       float o = 0.f;
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        const float kv = row[DP + d0 + i] * val;
-        o = fmaf(fmaf(U[i], kv, S[i]), row[d0 + i], o);
-        S[i] = fmaf(row[2 * DP + d0 + i], S[i], kv);
+        const float kv = kk[of][n][i] * val[of][n];
+        o = fmaf(fmaf(U[i], kv, S[i]), rr[of][n][i], o);
+        S[i] = fmaf(ww[of][n][i], S[i], kv);
       }
-      o = row_sum16(o);
-      outs = (lane & (REC_BLOCK - 1)) == j ? o : outs;
+      return o;
+    };
+    if (count == REC_BLOCK) {
+#pragma unroll
+      for (int n = 0; n < AHEAD; ++n) read(n, 0, n);
+#pragma unroll
+      for (int j = 0; j < REC_BLOCK; j += AHEAD) {
+        const int of = j / AHEAD & 1;
+        if (j + AHEAD < REC_BLOCK) {
+#pragma unroll
+          for (int n = 0; n < AHEAD; ++n) read(j + AHEAD + n, of ^ 1, n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float o[AHEAD];
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) o[n] = token(of, n);
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) o[n] = row_sum16(o[n]);
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) outs = (lane & (REC_BLOCK - 1)) == j + n ? o[n] : outs;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int j = 0; j < count; ++j) {
+        read(j, 0, 0);
+        const float o = row_sum16(token(0, 0));
+        outs = (lane & (REC_BLOCK - 1)) == j ? o : outs;
+      }
     }
     outs += __shfl_xor(outs, 16, 64);     // (row 0 + row 1) + (row 2 + row 3), in every row
     outs += __shfl_xor(outs, 32, 64);
@@ -955,7 +1029,7 @@ extern "C" int vk_delta_rule_strided(const float* qkv, long long ldq, int g_col,
   if (dim > 256 || heads > 65535) return VK_UNSUPPORTED_SIZE;
   const long long C = 2LL * kv_heads * dim + (long long)heads * vdim;
   if (ldq < C || (g_col < 0 && !decay) || (g_col >= 0 && g_col + (long long)heads * dim > ldq)) return VK_BAD_ARGUMENT;
-  if (ldq >= (1 << 24)) return VK_UNSUPPORTED_SIZE;      // the prompt form keeps a column in 24 bits
+  if (ldq >= (1 << 24)) return VK_UNSUPPORTED_SIZE;      // refused in both forms alike
   dim3 grid(num_entries, heads, (vdim + REC_COLS - 1) / REC_COLS);
   hipStream_t s = (hipStream_t)stream;
   const int key_pad = 16 * rows_of(dim), value_pad = (vdim + REC_COLS - 1) / REC_COLS * REC_COLS;
