@@ -67,6 +67,60 @@ def test_gemm_bf16_every_tiling_of_the_tiled_kernel(tiling, ranges):
         kernels.gemm_bf16_force_tiling(-1)
 
 
+@pytest.mark.parametrize("tiling", [13, 14, 15])
+@pytest.mark.parametrize("ranges", [1, 2, 3, 8])
+def test_the_small_tilings_give_the_bits_of_the_large_one(tiling, ranges):
+    """64x64 and 128x64 tiles with three and four LDS stages, K split over workgroups or its ranges added up in one:
+    the same sums in the same order as the 128x128 tiles with as many ranges.  Tails in both directions, runs shorter
+    than the stages, ranges that end in every stage and that K does not fill."""
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.linear import interleave_gate_up
+    try:
+        for m, n, k in [(129, 33, 64), (200, 96, 128), (257, 130, 192), (300, 264, 256), (150, 64, 1600), (513, 301, 1088), (140, 520, 4096)]:
+            g = torch.Generator().manual_seed(m + n + k)
+            a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+            w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+            bias, base = torch.randn(n, generator=g).to(DEV), torch.randn(m, n, generator=g).to(DEV)
+            fused = interleave_gate_up(w[:n // 16 * 16], w[:n // 16 * 16].flip(0).contiguous())
+            got = []
+            for now in (9, tiling):
+                kernels.gemm_bf16_force_tiling(now, ranges)
+                outs = [torch.full((m, n), 7.0, device=DEV), torch.full((m, n), 7.0, dtype=torch.bfloat16, device=DEV), base.clone(),
+                        torch.full((m, n // 16 * 16), 7.0, dtype=torch.bfloat16, device=DEV)]
+                kernels.gemm_bf16(a, w, bias, outs[0])
+                kernels.gemm_bf16(a, w, None, outs[1])
+                kernels.gemm_bf16(a, w, None, outs[2], accumulate=True)
+                kernels.gemm_bf16_gated(a, fused, outs[3])
+                got.append(outs)
+            assert all(torch.equal(x, y) for x, y in zip(*got)), (m, n, k)
+            assert _rel(got[1][0], a.double() @ w.double().T + bias.double()) < 1e-5, (m, n, k)
+    finally:
+        kernels.gemm_bf16_force_tiling(-1)
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 33, 2048), (512, 1057, 2048), (300, 64, 8192), (512, 2576, 512), (1000, 640, 1536), (700, 5120, 8256)])
+def test_the_tiles_chosen_for_a_product_do_not_change_its_bits(m, n, k):
+    """Past 128 tokens a product that takes 128x128 tiles may be carried out by smaller ones: the same bits as the
+    128x128 tiles give with one of the splits that are tried."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    out = torch.empty(m, n, device=DEV)
+    kernels.gemm_bf16(a, w, None, out)
+    assert _rel(out, a.double() @ w.double().T) < 1e-5
+    same = []
+    try:
+        for ranges in (1, 2, 4, 8):
+            kernels.gemm_bf16_force_tiling(9, ranges)
+            other = torch.empty(m, n, device=DEV)
+            kernels.gemm_bf16(a, w, None, other)
+            same.append(torch.equal(out, other))
+    finally:
+        kernels.gemm_bf16_force_tiling(-1)
+    assert any(same)
+
+
 @pytest.mark.parametrize("tiling", [0, 9, 7, 5, 6])
 def test_the_tiled_kernel_computes_the_same_in_every_order_of_its_tiles(tiling):
     """The workgroups walk the tiles in blocks of a few rows of tiles (chosen by shape, forced here): every tile is

@@ -429,9 +429,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const __bf16* _
 //   multiply the second half.
 // K ranges must be multiples of 64 (the launcher sends other shapes to gemm_tile_kernel). Four stages of
 // 32 k, which give a load three short steps to arrive instead of one long one, were slower.
+// FOLD: one workgroup works through all of K and adds up the ranges' sums itself (k_per_range of K each).
 // STAGES 3 (for up to 128 tokens, where the product is a stream of the weights and a CU's bytes in flight are
 // what bounds it): step s + 3 is requested when step s's stage is free, and the barrier of a step waits for
-// step s + 1 only, so the loads of two steps are in flight instead of one.
+// step s + 1 only, so the loads of two steps are in flight instead of one; STAGES 4 likewise.
 constexpr int DIRECT_ROW = BK * 2;  // bytes per LDS row
 
 // Until none of the wave's vector memory loads is in flight (s_waitcnt vmcnt(0), the other counters left
@@ -445,7 +446,7 @@ __device__ __forceinline__ void wait_own_loads_but() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
-template <int BM, int BN, int WM, int WN, typename TC, bool ACCUMULATE, bool GATED, int STAGES = 2>
+template <int BM, int BN, int WM, int WN, typename TC, bool ACCUMULATE, bool GATED, int STAGES = 2, bool FOLD = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __bf16* __restrict__ A,
                                                                           const __bf16* __restrict__ W,
                                                                           const float* __restrict__ bias,
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
                                                                           int k_per_range,
                                                                           long long range_stride, TileNorm norm) {
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  const int k_begin = blockIdx.y * k_per_range, k_end = min(K, k_begin + k_per_range);
+  const int k_begin = FOLD ? 0 : blockIdx.y * k_per_range, k_end = FOLD ? K : min(K, k_begin + k_per_range);
   C += (size_t)blockIdx.y * range_stride;
   constexpr int WAVES = WM * WN;
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide among the waves' loads");
   constexpr int STAGE = (BM + BN) * DIRECT_ROW;
   constexpr int LOADS = A_LOADS + W_LOADS;
-  static_assert(STAGES == 2 || STAGES == 3, "two or three LDS stages");
+  static_assert(STAGES >= 2 && STAGES <= 4, "two to four LDS stages");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];  // [STAGES][BM + BN][128]
 
   const int total = tiles_m * tiles_n;
@@ -531,11 +532,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
   bf16x8 fa0[TM], fw0[TN], fa1[TM], fw1[TN];
   __shared__ float part_sums[WAVES * 64];
   issue_loads(0, 0);
-  if (steps > 1) issue_loads(1, 1);
-  if (STAGES == 3 && steps > 2) issue_loads(2, 2);
+#pragma unroll
+  for (int i = 1; i < STAGES; ++i)
+    if (steps > i) issue_loads(i, i);
   tile_norm_parts<BM, WAVES * 64>(norm, m0, M, tid, part_sums);  // behind the first requests, before the first wait
-  if (STAGES == 3 && steps > 2) {
-    wait_own_loads_but<2 * LOADS>();  // step 0 has arrived; the other two stay in flight
+  if (STAGES > 2 && steps >= STAGES) {
+    wait_own_loads_but<(STAGES > 2 ? STAGES - 1 : 0) * LOADS>();  // step 0 has arrived; the others stay in flight
   } else {
     wait_own_loads();
   }
@@ -573,12 +575,44 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
     __builtin_amdgcn_sched_barrier(0);
   };
   int s = 0, stage = 0;
-  auto advance = [&]() { stage = stage + 1 == STAGES ? 0 : stage + 1; };
+  // FOLD: the sums of every k_per_range of K are added up as gemm_reduce_kernel adds the partial sums of as many workgroups
+  f32x4 folded[FOLD ? TN : 1][FOLD ? TM : 1];
+  int fold_at = k_per_range / BK;
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) folded[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        folded[i][j] += acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  auto advance = [&]() {
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    if constexpr (FOLD) {
+      if (s == fold_at) {
+        fold();
+        fold_at += k_per_range / BK;
+      }
+    }
+  };
   for (; s + STAGES < steps; ++s, advance())   // with three stages the step after next stays in flight
     step(s, stage, std::true_type{}, std::true_type{}, std::integral_constant<int, STAGES - 2>{});
   for (; s + 1 < steps; ++s, advance())
     step(s, stage, std::false_type{}, std::true_type{}, std::integral_constant<int, 0>{});
   step(s, stage, std::false_type{}, std::false_type{}, std::integral_constant<int, 0>{});
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = folded[i][j] + acc[i][j];
+  }
 
   tile_epilogue<BM, WAVES * 64, TM, TN, TC, ACCUMULATE, GATED>(acc, C, ldc, M, N, K, bias, (vector_ok & 1) != 0,
                                                                m0 + wm * TM * 16, n0 + wn * TN * 16, lr, lg, norm,
@@ -1732,14 +1766,15 @@ int launch_mid(const __bf16* A, const __bf16* W, const float* bias, TC* C, float
 
 int g_tile_group_m = 0;   // 0: chosen by shape; else the rows of tiles per block of tile_of, for measurements
 
-template <bool DIRECT, int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, int STAGES>
+template <bool DIRECT, int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, int STAGES, bool FOLD = false>
 constexpr auto tile_kernel() {
-  if constexpr (DIRECT) return gemm_tile_direct_kernel<BM, BN, WM, WN, TC, ACC, GATED, STAGES>;
+  if constexpr (DIRECT) return gemm_tile_direct_kernel<BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD>;
   else return gemm_tile_kernel<BM, BN, WM, WN, TC, ACC, GATED>;
 }
 
 // DIRECT: the kernel that loads straight into LDS; K must be a multiple of 64. STAGES: its LDS stages.
-template <int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, bool DIRECT = false, int STAGES = 2>
+// FOLD: one workgroup a tile adds up its K ranges itself.
+template <int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, bool DIRECT = false, int STAGES = 2, bool FOLD = false>
 int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, int M, int N, int K, long long lda,
                    long long ldc, int vector_ok, int ranges, float* partial, hipStream_t s, const TileNorm& norm) {
   static_assert(DIRECT || STAGES == 2, "only the direct kernel has a third stage");
@@ -1753,16 +1788,17 @@ int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, i
   const long long at_once = (long long)(compute_units() / XCDS) * (lds_bytes * 2 <= 160 * 1024 ? 2 : 1);
   const int group_m = g_tile_group_m > 0 ? (g_tile_group_m < tiles_m ? g_tile_group_m : tiles_m)
                                          : tile_group_rows(tiles_m, grid / XCDS < at_once ? grid / XCDS : at_once, BM, BN);
-  if (ranges <= 1 || GATED) {
+  const int k_per_range = ((K + ranges - 1) / ranges + BK - 1) / BK * BK;
+  if (ranges <= 1 || GATED || FOLD) {
     static bool configured = false;
-    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, TC, ACC, GATED, STAGES>();
+    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD>();
     if (!configured) {
       hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (e != hipSuccess) return (int)e;
       configured = true;
     }
     kernel<<<(int)grid, WM * WN * 64, lds_bytes, s>>>(A, W, bias, C, M, N, K, lda, ldc, tiles_m, tiles_n, group_m,
-                                                      vector_ok, K, 0, norm);
+                                                      vector_ok, FOLD ? k_per_range : K, 0, norm);
     VK_LAUNCH_CHECK();
     return 0;
   }
@@ -1775,7 +1811,6 @@ int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, i
       if (e != hipSuccess) return (int)e;
       configured_partial = true;
     }
-    const int k_per_range = ((K + ranges - 1) / ranges + BK - 1) / BK * BK;
     const int used = (K + k_per_range - 1) / k_per_range;
     kernel<<<dim3((unsigned)grid, used), WM * WN * 64, lds_bytes, s>>>(A, W, nullptr, partial, M, N, K, lda, N, tiles_m,
                                                                        tiles_n, group_m, (N & 3) == 0 ? 1 : 0,
@@ -1886,8 +1921,34 @@ TilePlan choose_tile_plan(int M, int N, int K, long long partial_floats, bool di
   return best;
 }
 
+// Past 128 tokens, where choose_tile_plan takes 128x128 tiles: the tiling that carries the same plan out. Such a launch
+// is a few dozen to a few hundred workgroups, and what bounds it is the latency of a K step on the CUs that have one
+// (0.5 us with two stages), not the matrix cores. So the tiles are cut further, with more stages in flight: 64x64 with
+// four stages (0.2 us a step) while these find a CU each, else 128x64 with three, two workgroups to a CU; and K is not
+// split over workgroups any more but by each for itself, which adds its ranges' sums in the same order without
+// partial sums in memory and a second launch. Every output is the same sum in the same order, with the same bits.
+// 512 tokens, K 2,048: 2,048 rows 21.8 -> 9.6 us, 1,057 rows in four ranges 21.5 -> 10.2, 2,576 rows 22.3 -> 13.1;
+// 1,834 tokens on 1,024 rows 22.4 -> 14.1, 2,048 on 2,048 25.8 -> 23.7, on 3,072 rows of 768 18.1 -> 16.9.
+// Where few tiles have a long K, its split over workgroups (13) is faster than the walk (14): 512 tokens on 64 rows in
+// four ranges 7.8 against 9.0 us; both by the estimate of 0.19 us a step and 3.5 us and the sums' bytes for the split.
+// The 128x128 tiles stay beyond three 128x64 tiles a CU, where nothing was measured to gain, and where they come close to
+// one a CU by themselves and K is long, so that the bytes per product count (700 tokens, 5,120 rows of 8,960: 71.7 us
+// against 77.2; of 2,048, 31.4 against 28.1), or where the split of small tiles would come to many a CU.
+int smaller_tiles(int M, int N, int K, int ranges) {
+  const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  const long long middle = (long long)((M + 127) / 128) * ((N + 63) / 64);
+  const long long whole = (long long)((M + 127) / 128) * ((N + 127) / 128) * ranges;
+  if (small > g_compute_units)
+    return middle <= 3LL * g_compute_units && (K <= 8192 || whole * 10 < 9LL * g_compute_units) ? 15 : 9;
+  const double steps = K / 64 * 0.19e-6;
+  const double split = steps / ranges + 3.5e-6 + (2.0 * ranges + 1.0) * 4.0 * M * N / 6e12;
+  if (ranges == 1 || steps <= split) return 14;
+  return small * ranges <= 4LL * g_compute_units ? 13 : 9;
+}
+
 // Tilings: 0, 2, 3, 4 the staged kernel at 128x128, 256x128, 128x256, 256x256; 9, 7, 8, 5 the same tiles
-// with the kernel that loads straight into LDS, which needs K to be a multiple of 64, and 6 that kernel at
+// with the kernel that loads straight into LDS, which needs K to be a multiple of 64; 13 and 15 that kernel at 64x64
+// and 128x64, 14 at 64x64 with the K ranges of one tile in one workgroup (15 always so); and 6 that kernel at
 // 256x192 (2,048 tokens x 4,608 rows are 192 such tiles for 256 CUs, against 144 of 256x256).
 template <typename TC, bool ACC, bool GATED = false>
 int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int M, int N, int K, long long lda,
@@ -1896,11 +1957,12 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
   const bool direct = (K & 63) == 0;
   TilePlan plan = choose_tile_plan(M, N, K, (GATED || !partial) ? 0 : partial_floats, direct, GATED);
   if (g_tile_config >= 0) plan = TilePlan{g_tile_config, g_tile_ranges > 1 && !GATED && partial ? g_tile_ranges : 1};
+  else if (direct && plan.config == 9 && M > 128 && !norm.sumsq) plan.config = smaller_tiles(M, N, K, plan.ranges);
   if (plan.ranges > 1 && (long long)plan.ranges * M * N > partial_floats) plan.ranges = 1;
-  if (plan.config >= 10 && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
+  if (plan.config >= 10 && plan.config <= 12 && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
   if (!direct) {
     switch (plan.config) { case 5: case 6: plan.config = 4; break; case 7: plan.config = 2; break; case 8: plan.config = 3; break;
-                           case 9: case 10: case 11: case 12: plan.config = 0; break; }
+                           case 9: case 10: case 11: case 12: case 13: case 14: case 15: plan.config = 0; break; }
   }
   const int r = plan.ranges;
 #define VK_TILE(BMV, BNV, WMV, WNV, DIRECTV) \
@@ -1925,6 +1987,23 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
       case 12: VK_TILE_DEEP(128, 224, 4, 1);
     }
   }
+#define VK_TILE_SMALL(BMV, BNV, STAGESV, FOLDV)                                                                       \
+  return launch_tile_as<BMV, BNV, 4, 2, TC, ACC, GATED, true, STAGESV, FOLDV>(A, W, bias, C, M, N, K, lda, ldc, vector_ok, r, \
+                                                                              partial, s, norm)
+  switch (plan.config) {
+    case 14:
+      if constexpr (!GATED) {
+        if (r > 1) VK_TILE_SMALL(64, 64, 4, true);
+      }
+      [[fallthrough]];
+    case 13: VK_TILE_SMALL(64, 64, 4, false);
+    case 15:
+      if constexpr (!GATED) {
+        if (r > 1) VK_TILE_SMALL(128, 64, 3, true);
+      }
+      VK_TILE_SMALL(128, 64, 3, false);
+  }
+#undef VK_TILE_SMALL
   switch (plan.config) {
     case 5: VK_TILE(256, 256, 4, 2, true);
     case 6: VK_TILE(256, 192, 4, 2, true);

@@ -721,7 +721,8 @@ def gemm_bf16_gated_tile_scaled(scaled: torch.Tensor, w: torch.Tensor, out: torc
 
 TILE_TILINGS = {0: "128x128 staged", 2: "256x128 staged", 3: "128x256 staged", 4: "256x256 staged",
                 9: "128x128 direct", 7: "256x128 direct", 8: "128x256 direct", 5: "256x256 direct", 6: "256x192 direct",
-                10: "128x96 direct, gated only", 11: "128x160 direct, gated only", 12: "128x224 direct, gated only"}
+                10: "128x96 direct, gated only", 11: "128x160 direct, gated only", 12: "128x224 direct, gated only",
+                13: "64x64 direct", 14: "64x64 direct, ranges in one workgroup", 15: "128x64 direct, ranges in one workgroup"}
 
 
 def gemm_bf16_force_tiling(tiling: int = -1, ranges: int = 1, stages: int = 0) -> None:
