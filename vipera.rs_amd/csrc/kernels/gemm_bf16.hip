@@ -8,9 +8,9 @@
 //     lane l, register j of an accumulator  <->  C[token l % 16][column 4 * (l / 16) + j]
 //
 // Kernels:
-//   gemm_tile    more than 64 tokens (prompts). An output tile per workgroup (256x256 down to 128x128,
-//                chosen with a split of K by an estimate of the time), K in steps of 64 through two LDS
-//                stages, one barrier per step. Workgroups are renumbered so that those running on one XCD
+//   gemm_tile    more than 64 tokens (prompts). An output tile per workgroup (256x256 down to 64x64,
+//                chosen with a split of K by an estimate of the time), K in steps of 64 through two to four
+//                LDS stages, one barrier per step. Workgroups are renumbered so that those running on one XCD
 //                (one L2) work on neighbouring tiles. Two kernels: gemm_tile_direct_kernel loads both
 //                operands straight into LDS (unpadded rows, chunks swizzled) and pipelines the LDS reads
 //                against the products inside each wave; it takes K in multiples of 64. gemm_tile_kernel

@@ -477,7 +477,7 @@ def logit_bias(logits: torch.Tensor, rows: torch.Tensor, tokens: torch.Tensor, v
 # ----------------------------------------------------------------------------------------------
 def gemm_bf16_supported(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     """Whether the matrix-core kernels take these operands (16-byte chunks along K, rows short enough for their
-    32-bit offsets); what they do not take goes to the 32-bit FMA kernel."""
+    32-bit offsets); what they do not take goes to the 32-bit kernel."""
     k = a.shape[1]
     return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype in _DT and k % 8 == 0
             and k < GEMM_BF16_MAX_K and a.stride(0) < GEMM_BF16_MAX_K

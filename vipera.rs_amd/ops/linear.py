@@ -2,7 +2,7 @@
 
 All-bfloat16 operands whose rows are 16-byte aligned go to the matrix-core kernels; every other
 combination (the 32-bit run, or a matrix kept in 32-bit inside a bfloat16 run) goes to the
-32-bit FMA kernel.  Among the matrix-core kernels the number of rows of ``a`` (tokens) decides:
+32-bit kernel.  Among the matrix-core kernels the number of rows of ``a`` (tokens) decides:
 
 * many (prompts): the LDS-tiled kernel;
 * up to 64 (decoding), and up to 128 for small weights (:func:`streams_weights`): the

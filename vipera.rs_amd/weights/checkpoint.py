@@ -129,7 +129,7 @@ def kept_dtype(spec: TensorSpec, stored: torch.dtype, run_dtype: torch.dtype, ke
     A matrix is converted once, when it is loaded, to the run's dtype, whatever floating-point type the folder
     stores it in (32-bit, 16-bit float or bfloat16; to bfloat16 by rounding to nearest even): the run's kernels and
     the memory a plan predicts are then those of the run's dtype, not of the file's.  ``keep_float32``: a matrix
-    stored in 32-bit stays in 32-bit in a bfloat16 run (its products then go through the 32-bit FMA kernel, at a
+    stored in 32-bit stays in 32-bit in a bfloat16 run (its products then go through the 32-bit kernel, at a
     fraction of the speed).  Vectors (norm weights, biases) are always 32-bit, which widens a 16-bit one exactly and
     leaves a 32-bit one as it is; integer tables become int32.
     """
