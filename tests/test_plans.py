@@ -176,3 +176,11 @@ def test_a_32_bit_product_of_9_to_16_tokens_streams_its_weights_where_they_are_m
         assert all(gemm_streams_weights_f32(m, n, k) for m in (1, 8))
         assert all(gemm_streams_weights_f32(m, n, k) == ((n, k) in heads) for m in (9, 12, 16))
         assert not any(gemm_streams_weights_f32(m, n, k) for m in (17, 64, 2048))
+
+
+def test_the_cut_of_a_32_bit_product_is_asked_for_once_for_a_size(monkeypatch):
+    from vipera_rs_amd.ops import kernels
+    asked, real = [], kernels._fn
+    monkeypatch.setattr(kernels, "_fn", lambda *args, **named: asked.append(args[1]) or real(*args, **named))
+    first = kernels._gemm_generic_parts(77, 1155, 899)
+    assert asked == ["vk_gemm_generic_workspace"] and first == kernels._gemm_generic_parts(77, 1155, 899) and len(asked) == 1
