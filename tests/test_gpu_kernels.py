@@ -363,6 +363,25 @@ def test_gemm_generic_cut_over_workgroups_sums_in_the_same_order(m, n, k):
     assert torch.equal(mixed, again.to(torch.bfloat16))
 
 
+def test_gemm_generic_needs_no_memory_for_its_parts():
+    """Where the memory for the parts of a cut K is not there, the product runs uncut: the same bits."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(3)
+    a, w = torch.randn(128, 16384, generator=g).to(DEV), torch.randn(1024, 16384, generator=g).to(DEV)
+    want, out = torch.empty(128, 1024, device=DEV), torch.full((128, 1024), float("nan"), device=DEV)
+    assert kernels._gemm_generic_parts(128, 1024, 16384) == 64 * 128 * 1024
+    kernels.gemm_generic(a, w, None, want)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved(DEV) + 2 ** 22      # the parts are 32 MB
+    try:
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory, 0)
+        kernels.gemm_generic(a, w, None, out)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, 0)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 4), (3, 70, 36), (8, 3584, 1536), (9, 129, 1028), (16, 1000, 4096), (40, 200, 520),
                                    (64, 333, 2052)])
 def test_gemm_stream_against_float64(m, n, k):

@@ -270,11 +270,21 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
         _status(fn(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc, 1 if accumulate else 0,
                    _ptr(slabs), slabs.numel(), _stream()), "gemm_stream")
         return
-    # K split over workgroups where the tiles are too few; the parts belong to this call alone, on whatever stream it runs
+    # K split over workgroups where the tiles are too few; the parts belong to this call alone, on whatever stream it runs.
+    # Where the memory for them is not there a workgroup walks all of K instead: the same bits, more time.
+    parts = None
     floats = _gemm_generic_parts(m, n, k)
-    parts = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
-    fn = _fn("gemm_generic", "vk_gemm_generic_split",
-             [_p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p, _ll, _p])
+    if floats:
+        try:
+            parts = torch.empty(floats, dtype=torch.float32, device=a.device)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    if parts is None:
+        fn = _fn("gemm_generic", "vk_gemm_generic", [_p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p])
+        _status(fn(_ptr(a), _dt(a, "a"), _ptr(w), _dt(w, "w"), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc,
+                   1 if accumulate else 0, _stream()), "gemm_generic")
+        return
+    fn = _fn("gemm_generic", "vk_gemm_generic_split", [_p, _i, _p, _i, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p, _ll, _p])
     _status(fn(_ptr(a), _dt(a, "a"), _ptr(w), _dt(w, "w"), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc,
                1 if accumulate else 0, _ptr(parts), floats, _stream()), "gemm_generic")
 
