@@ -382,6 +382,27 @@ def test_gemm_generic_needs_no_memory_for_its_parts():
     assert torch.equal(out, want)
 
 
+def test_gemm_generic_of_more_tiles_than_one_launch_takes():
+    """Past 2^32 threads in its tiles a product is several launches: 1,048,576 x 65,600 outputs, 138 GB in bfloat16."""
+    from vipera_rs_amd.ops import kernels
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info(DEV)[0] < 150e9:
+        pytest.skip("needs 138 GB of free device memory for its output")
+    m, n = 1048576, 65600
+    a = (torch.arange(m, device=DEV) % 251 - 125).float()[:, None]      # whole numbers, and products below 2^8 times a power of two
+    w = 2.0 ** (torch.arange(n, device=DEV) % 13 - 6).float()[:, None]
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    try:
+        kernels.gemm_generic(a, w, None, out)
+        for rows in (slice(0, 3), slice(m // 2, m // 2 + 3), slice(m - 3, m)):
+            assert torch.equal(out[rows], (a[rows] * w.T).to(torch.bfloat16))
+        for columns in (slice(0, 70), slice(n // 2, n // 2 + 70), slice(n - 200, n)):
+            assert torch.equal(out[:, columns], (a * w[columns].T).to(torch.bfloat16))
+    finally:
+        del out
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 4), (3, 70, 36), (8, 3584, 1536), (9, 129, 1028), (16, 1000, 4096), (40, 200, 520),
                                    (64, 333, 2052)])
 def test_gemm_stream_against_float64(m, n, k):

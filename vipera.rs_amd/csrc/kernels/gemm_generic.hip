@@ -225,16 +225,24 @@ int matrix_units(int M, int N, int K) {
 template <typename TA, typename TW, typename TC, bool ACCUMULATE, int UNITS>
 int launch_tiles(const TA* A, const TW* W, const float* bias, TC* C, float* parts, int M, int N, int K, long long lda,
                  long long ldc, hipStream_t s) {
-  const long long tiles = (long long)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
-  if (tiles > 0x7fffffff) return VK_UNSUPPORTED_SIZE;
-  dim3 grid((unsigned)tiles, UNITS ? (K + UNITS * RANGE_K - 1) / (UNITS * RANGE_K) : 1);
+  const long long m_tiles = (M + TILE - 1) / TILE, n_tiles = (N + TILE - 1) / TILE;
   // loads of four k where every row of both operands starts on a boundary of their size
   const bool vector = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0;
-  if (vector)
-    gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, true><<<grid, 256, 0, s>>>(A, W, bias, C, parts, M, N, K, lda, ldc);
-  else
-    gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, false><<<grid, 256, 0, s>>>(A, W, bias, C, parts, M, N, K, lda, ldc);
-  VK_LAUNCH_CHECK();
+  // A launch counts its threads in 32 bits, and past them leaves tiles out without an error: so many columns are several
+  // launches (one is enough where K is cut, which takes few tiles)
+  const long long slice = min(n_tiles, 0xffffffffll / 256 / m_tiles);
+  for (long long n0 = 0; n0 < n_tiles; n0 += slice) {
+    const long long first = n0 * TILE;
+    dim3 grid((unsigned)(m_tiles * min(slice, n_tiles - n0)), UNITS ? (K + UNITS * RANGE_K - 1) / (UNITS * RANGE_K) : 1);
+    const int columns = (int)min((long long)N - first, slice * TILE);
+    const TW* w = W + first * K;
+    const float* b = bias ? bias + first : nullptr;
+    if (vector)
+      gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, true><<<grid, 256, 0, s>>>(A, w, b, C + first, parts, M, columns, K, lda, ldc);
+    else
+      gemm_matrix_kernel<TA, TW, TC, ACCUMULATE, UNITS, false><<<grid, 256, 0, s>>>(A, w, b, C + first, parts, M, columns, K, lda, ldc);
+    VK_LAUNCH_CHECK();
+  }
   return 0;
 }
 
