@@ -278,6 +278,33 @@ def test_experts_in_tiles_loaded_straight_into_lds(tokens, width, ff, experts, t
     assert rel_err(residual.cpu().numpy(), want.cpu().numpy()) < 2.0 ** -8
 
 
+def test_experts_of_more_tiles_than_one_row_of_a_grid_takes():
+    """4,096 experts of 64 x 131,072: 2^32 threads and more in the tiles of the product in front (69 GB of weights, shared by
+    its two halves and the product behind)."""
+    from vipera_rs_amd.ops import kernels
+
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 80e9:
+        pytest.skip("needs 71 GB of free device memory for its weights")
+    experts, width, ff = 4096, 64, 131072
+    up = torch.empty(experts, ff, width, dtype=torch.bfloat16, device="cuda").normal_(0.0, 0.125)
+    down = up.view(experts, width, ff)
+    h = torch.randn(experts, width, device="cuda").to(torch.bfloat16)
+    ids, w, offsets, order, tiles, count = route(kernels, 9.0 * torch.eye(experts, device="cuda"), 1, 128)    # token e to expert e
+    act = torch.full((experts, ff), float("nan"), dtype=torch.bfloat16, device="cuda")
+    pair_out, residual = torch.full((experts, width), float("nan"), device="cuda"), torch.empty(experts, width, device="cuda")
+    try:
+        kernels.moe_experts(h, up, up, down, offsets, order, tiles, count, w, 1, float("inf"), 1.0, act, pair_out, residual, False, False, 128)
+        assert not bool(torch.isnan(act).any()) and not bool(torch.isnan(residual).any())
+        for e in (0, 1, 2047, 4094, 4095):
+            u = up[e].double() @ h[e].double()
+            want = down[e].double() @ (torch.nn.functional.silu(u) * u)
+            assert rel_err(residual[e].cpu().numpy(), want.cpu().numpy()) < 2.0 ** -8     # the activation's rounding to 16 bits
+    finally:
+        del up, down, act
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [40, 50, 1000, 4096, 5000])
 def test_a_norm_behind_and_a_layer_norm_in_front_in_one_launch(width, dtype):

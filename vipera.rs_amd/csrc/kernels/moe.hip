@@ -436,7 +436,8 @@ __global__ __launch_bounds__(256) void moe_down_mma_kernel(const __bf16* __restr
 //
 // A workgroup's number says which XCD it runs on (the remainder by eight): each XCD takes a run of neighbouring tiles,
 // and walks them column block by column block, so that the few tiles of an expert read its weights at the same time
-// through one L2.
+// through one L2.  Grid (a multiple of eight at or above the tiles there can be, column blocks): a row of the grid holds a column
+// block's share of every XCD, so that the numbers run on from row to row.  In one row they passed the 2^32 threads that a launch takes.
 template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
                                                                  const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* _
                                                                  __bf16* __restrict__ act, float* __restrict__ pair_out) {
   constexpr int COLUMNS = FORM == 0 ? BN / 2 : BN, TM = BM / WM / 16, TN = BN / WN / 16;
   const int blocks = (N + COLUMNS - 1) / COLUMNS, count_tiles = num_tiles[0];
-  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int xcd = blockIdx.x & 7, at = (blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3);
   const int t0 = (int)((long long)count_tiles * xcd / 8), own = (int)((long long)count_tiles * (xcd + 1) / 8) - t0;
   if (at >= own * blocks) return;
   const int tile = t0 + at % own, n0 = at / own * COLUMNS;
@@ -511,9 +512,9 @@ static int launch_direct(const __bf16* in, long long in_rows, long long ldi, con
     sized = true;
   }
   // an XCD has at most ceil(tiles / 8) of the tiles, whatever their number turns out to be
-  const long long grid = 8ll * ((max_tiles + 7) / 8) * ((N + COLUMNS - 1) / COLUMNS);
-  if (grid > 0x7fffffff) return VK_UNSUPPORTED_SIZE;
-  moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES><<<(unsigned)grid, WM * WN * 64, lds_bytes, s>>>(
+  const dim3 grid(8 * ((max_tiles + 7) / 8), (N + COLUMNS - 1) / COLUMNS);
+  if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
+  moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES><<<grid, WM * WN * 64, lds_bytes, s>>>(
       in, ((in_rows - 1) * ldi + K) * 2, ldi, w0, w1, offsets, order, tiles, num_tiles, top, K, N, limit, alpha, plain, in_weights,
       act, pair_out);
   VK_LAUNCH_CHECK();
