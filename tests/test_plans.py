@@ -184,3 +184,19 @@ def test_the_cut_of_a_32_bit_product_is_asked_for_once_for_a_size(monkeypatch):
     monkeypatch.setattr(kernels, "_fn", lambda *args, **named: asked.append(args[1]) or real(*args, **named))
     first = kernels._gemm_generic_parts(77, 1155, 899)
     assert asked == ["vk_gemm_generic_workspace"] and first == kernels._gemm_generic_parts(77, 1155, 899) and len(asked) == 1
+
+
+def test_past_128_tokens_small_tiles_carry_out_a_128x128_plan_unless_its_tiles_fill_the_gpu():
+    """The tiling and the ranges of K.  Tilings 9: 128x128, 13: 64x64 with K split, 14: 64x64 that walk K, 15: 128x64 that walk K."""
+    from vipera_rs_amd.ops.kernels import gemm_bf16_tile_plan as plan
+    assert plan(512, 2048, 2048) == (14, 1) and plan(512, 1057, 2048) == (14, 4) and plan(512, 64, 2048) == (13, 4)
+    assert plan(512, 2576, 2048) == (15, 1) and plan(700, 5120, 2048) == (15, 1)           # more than a 64x64 tile a CU
+    assert plan(2819, 768, 1280, gated=True) == (15, 1) and plan(300, 1024, 768, gated=True) == (14, 1)
+    # as many ranges as fill the CUs with 128x128 tiles: these stay, or walk K where it has four
+    assert plan(330, 7488, 7168) == (9, 2) and plan(353, 3168, 6400) == (9, 4) and plan(301, 4288, 6848) == (9, 4)
+    assert plan(1879, 256, 8192) == (9, 8) and plan(953, 512, 6400) == (9, 8) and plan(468, 1792, 4352) == (14, 4)
+    assert plan(161, 1792, 10496) == (13, 8)       # 256 tokens' worth of 128x128 tiles for 161
+    # one 128x128 tile a CU at the most, however long K is
+    assert all(plan(700, 5120, k, gated=True) == (15, 1) for k in (1024, 8192, 12288)) and plan(277, 10880, 4096, gated=True) == (15, 1)
+    assert plan(277, 10976, 4096, gated=True) == (9, 1) and plan(270, 13312, 8192, gated=True) == (9, 1)
+    assert plan(512, 2048, 2040)[0] == 0           # no whole steps of 64

@@ -1928,22 +1928,37 @@ TilePlan choose_tile_plan(int M, int N, int K, long long partial_floats, bool di
 // split over workgroups any more but by each for itself, which adds its ranges' sums in the same order without
 // partial sums in memory and a second launch. Every output is the same sum in the same order, with the same bits.
 // 512 tokens, K 2,048: 2,048 rows 21.8 -> 9.6 us, 1,057 rows in four ranges 21.5 -> 10.2, 2,576 rows 22.3 -> 13.1;
-// 1,834 tokens on 1,024 rows 22.4 -> 14.1, 2,048 on 2,048 25.8 -> 23.7, on 3,072 rows of 768 18.1 -> 16.9.
+// 1,834 tokens on 1,024 rows 22.4 -> 14.1, 2,048 on 2,048 25.8 -> 23.7, on 3,072 rows of 768 18.1 -> 16.9; gated, 700
+// tokens on 5,120 rows of 2,048 32.7 -> 26.1, of 12,288 167 -> 149.
 // Where few tiles have a long K, its split over workgroups (13) is faster than the walk (14): 512 tokens on 64 rows in
 // four ranges 7.8 against 9.0 us; both by the estimate of 0.19 us a step and 3.5 us and the sums' bytes for the split.
-// The 128x128 tiles stay beyond three 128x64 tiles a CU, where nothing was measured to gain, and where they come close to
-// one a CU by themselves and K is long, so that the bytes per product count (700 tokens, 5,120 rows of 8,960: 71.7 us
-// against 77.2; of 2,048, 31.4 against 28.1), or where the split of small tiles would come to many a CU.
+// The 128x128 tiles stay where they and their ranges are more than one workgroup a CU (270 tokens, gated, 13,312 rows of
+// 8,192, 312 tiles: 116 us, 126 as 128x64; 330 tokens, 7,488 rows of 7,168 in two ranges: 72 and 83). From three quarters of
+// one a CU on the split small tiles (13) lose as well, by 2 to 10 %, unless the 128x128 tiles multiply a fifth more rows and
+// columns than there are: four ranges are walked (468 tokens, 1,792 rows of 4,352: 17.7 us, 23.6 split, 22.5 as 128x128),
+// eight stay (1,879 tokens, 256 rows of 8,192: 21.9 us, 24.2 split, 26.9 walked). All with the weights in memory; where a
+// small weight is in the caches already and K is 1,024 or less, 128x64 tiles of which some CUs have two are 2 to 5 % behind
+// the 128x128 ones, as they are 5 to 10 % ahead from memory.
 int smaller_tiles(int M, int N, int K, int ranges) {
   const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  const long long middle = (long long)((M + 127) / 128) * ((N + 63) / 64);
-  const long long whole = (long long)((M + 127) / 128) * ((N + 127) / 128) * ranges;
-  if (small > g_compute_units)
-    return middle <= 3LL * g_compute_units && (K <= 8192 || whole * 10 < 9LL * g_compute_units) ? 15 : 9;
+  const long long tiles = (long long)((M + 127) / 128) * ((N + 127) / 128), whole = tiles * ranges;
+  if (small > g_compute_units) return whole <= g_compute_units ? 15 : 9;
   const double steps = K / 64 * 0.19e-6;
   const double split = steps / ranges + 3.5e-6 + (2.0 * ranges + 1.0) * 4.0 * M * N / 6e12;
   if (ranges == 1 || steps <= split) return 14;
+  if (whole * 4 > 3LL * g_compute_units) {
+    if (ranges <= 4) return 14;
+    if (small * 11 > tiles * 36) return 9;
+  }
   return small * ranges <= 4LL * g_compute_units ? 13 : 9;
+}
+
+// What launch_tile carries out: `scaled`: with a norm's factors.
+TilePlan tile_plan(int M, int N, int K, long long partial_floats, bool gated, bool scaled) {
+  const bool direct = (K & 63) == 0;
+  TilePlan plan = choose_tile_plan(M, N, K, partial_floats, direct, gated);
+  if (direct && plan.config == 9 && M > 128 && !scaled) plan.config = smaller_tiles(M, N, K, plan.ranges);
+  return plan;
 }
 
 // Tilings: 0, 2, 3, 4 the staged kernel at 128x128, 256x128, 128x256, 256x256; 9, 7, 8, 5 the same tiles
@@ -1955,9 +1970,8 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
                 long long ldc, int vector_ok, float* partial, long long partial_floats, hipStream_t s,
                 const TileNorm& norm = TileNorm{}) {
   const bool direct = (K & 63) == 0;
-  TilePlan plan = choose_tile_plan(M, N, K, (GATED || !partial) ? 0 : partial_floats, direct, GATED);
+  TilePlan plan = tile_plan(M, N, K, (GATED || !partial) ? 0 : partial_floats, GATED, norm.sumsq != nullptr);
   if (g_tile_config >= 0) plan = TilePlan{g_tile_config, g_tile_ranges > 1 && !GATED && partial ? g_tile_ranges : 1};
-  else if (direct && plan.config == 9 && M > 128 && !norm.sumsq) plan.config = smaller_tiles(M, N, K, plan.ranges);
   if (plan.ranges > 1 && (long long)plan.ranges * M * N > partial_floats) plan.ranges = 1;
   if (plan.config >= 10 && plan.config <= 12 && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
   if (!direct) {
@@ -2366,5 +2380,14 @@ extern "C" int vk_gemm_bf16_tile_config(int tiling, int ranges, int stages) {
   g_tile_config = tiling;
   g_tile_ranges = ranges;
   g_tile_stages = stages;
+  return 0;
+}
+
+// The tiling and the ranges of K that a tiled product of these sizes is given (without a norm's factors).
+extern "C" int vk_gemm_bf16_tile_plan(int M, int N, int K, long long partial_floats, int gated, int* tiling, int* ranges) {
+  if (M <= 0 || N <= 0 || K <= 0) return VK_BAD_ARGUMENT;
+  const TilePlan plan = tile_plan(M, N, K, gated ? 0 : partial_floats, gated != 0, false);
+  *tiling = plan.config;
+  *ranges = plan.ranges;
   return 0;
 }
