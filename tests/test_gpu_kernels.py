@@ -363,6 +363,40 @@ def test_gemm_generic_cut_over_workgroups_sums_in_the_same_order(m, n, k):
     assert torch.equal(mixed, again.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("k", [4, 200, 260, 1100])
+@pytest.mark.parametrize("values", ["spread", "small operands", "small products", "small sums", "overflow", "special"])
+def test_the_matrix_instruction_is_two_fused_multiply_adds_for_all_values(values, k):
+    """The tiles on the matrix cores (70 rows) against the weight stream's FMA chains (8 rows at a time), bit for bit, NaN for
+    NaN: magnitudes over the whole range of exponents, denormal operands, products and sums, overflow, infinities, NaN and
+    zeros of both signs.  With one product per element both are the product rounded once, denormal results included."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(k)
+    scale = lambda rows, low, high: 2.0 ** torch.randint(low, high, (rows, k), generator=g).double()
+    a, w = torch.randn(70, k, generator=g).double(), torch.randn(90, k, generator=g).double()
+    exponents = {"spread": (-60, 60, -60, 60), "small operands": (-148, -126, 100, 126), "small products": (-80, -60, -80, -60),
+                 "small sums": (-68, -65, -68, -65), "overflow": (50, 66, 50, 66), "special": (-3, 3, -3, 3)}[values]
+    a, w = (a * scale(70, *exponents[:2])).float(), (w * scale(90, *exponents[2:])).float()
+    if values == "special":
+        for x, row in ((a, 5), (w, 7)):
+            x[row, 0], x[row + 1, 1], x[row + 2, 2] = float("inf"), float("-inf"), float("nan")
+            x[row + 3], x[row + 4], x[row + 5, 3] = 0.0, -0.0, 3.4e38
+    if k == 4:
+        a[:, 1:], w[:, 1:] = 0.0, 0.0          # one product per element
+    a, w = a.to(DEV), w.to(DEV)
+    tiles, stream = torch.empty(70, 90, device=DEV), torch.empty(70, 90, device=DEV)
+    kernels.gemm_generic(a, w, None, tiles)
+    for first in range(0, 70, 7):
+        kernels.gemm_generic(a[first:first + 7], w, None, stream[first:first + 7])
+    nan = torch.isnan(stream)
+    bits = lambda x: x.masked_fill(torch.isnan(x), 0.0).view(torch.int32)
+    assert torch.equal(torch.isnan(tiles), nan) and torch.equal(bits(tiles), bits(stream))
+    if values.startswith("small"):
+        denormal = a if values == "small operands" else stream
+        assert bool(((denormal != 0.0) & (denormal.abs() < 2.0 ** -126)).any())
+    if k == 4 and values != "special":
+        assert torch.equal(tiles, (a[:, :1].double() * w[:, :1].double().T).float())
+
+
 def test_gemm_generic_needs_no_memory_for_its_parts():
     """Where the memory for the parts of a cut K is not there, the product runs uncut: the same bits."""
     from vipera_rs_amd.ops import kernels
