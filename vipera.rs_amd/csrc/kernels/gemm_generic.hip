@@ -114,28 +114,30 @@ __global__ __launch_bounds__(256) void gemm_matrix_kernel(const TA* __restrict__
   __syncthreads();
   int buf = 0;
   const int in_tile = lane & 31, half = (lane >> 5) * 8;
-  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-    const bool more = k0 + BK < k_end;
-    if (more) fetch(k0 + BK);
+  for (int k0 = k_begin; k0 < k_end;) {
+    // a range's steps in a loop of their own, which touches no sum but acc: with the sums added up behind a branch of every
+    // step the compiler moves all three sets between the two register files in each of them
+    const int range_end = min(k_end, k0 + RANGE_K);
+    for (; k0 < range_end; k0 += BK) {
+      const bool more = k0 + BK < k_end;
+      if (more) fetch(k0 + BK);
 #pragma unroll
-    for (int t4 = 0; t4 < 2; ++t4) {
-      const f32x4_t a = *(const f32x4_t*)&As[buf][wm + in_tile][half + 4 * t4];
-      const f32x4_t w = *(const f32x4_t*)&Ws[buf][wn + in_tile][half + 4 * t4];
+      for (int t4 = 0; t4 < 2; ++t4) {
+        const f32x4_t a = *(const f32x4_t*)&As[buf][wm + in_tile][half + 4 * t4];
+        const f32x4_t w = *(const f32x4_t*)&Ws[buf][wn + in_tile][half + 4 * t4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], w[t], acc, 0, 0, 0);
-    }
-    if (more) stage(buf ^ 1, k0 + BK);
-    __syncthreads();
-    buf ^= 1;
-    const int done = k0 + BK;
-    if constexpr (UNITS != 1) {
-      if (done % RANGE_K == 0 || !more) {
-        slab += acc;
-        acc = 0.f;
+        for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], w[t], acc, 0, 0, 0);
       }
+      if (more) stage(buf ^ 1, k0 + BK);
+      __syncthreads();
+      buf ^= 1;
+    }
+    if constexpr (UNITS != 1) {
+      slab += acc;
+      acc = 0.f;
     }
     if constexpr (UNITS == 0) {
-      if (done % SLAB_K == 0 || !more) {
+      if (k0 % SLAB_K == 0 || k0 >= k_end) {
         total += slab;
         slab = 0.f;
       }
