@@ -48,9 +48,10 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
 // Four consecutive k of a row as floats; VECTOR: K is a multiple of 4 and rows are aligned for one load (a row past
-// the end and a k past the end are read at the last place and cleared by the caller where it matters).
+// the end and a k past the end are read at the last place and cleared by the caller where it matters).  whole: no k of
+// the step lies past the end, the same for all lanes (a place of its own for every k costs an odd K a tenth of its rate).
 template <typename T, bool VECTOR>
-__device__ __forceinline__ f32x4_t fetch4(const T* __restrict__ row, int k, int K) {
+__device__ __forceinline__ f32x4_t fetch4(const T* __restrict__ row, int k, int K, bool whole) {
   f32x4_t v;
   if constexpr (VECTOR) {
     const int at = min(k, K - 4);
@@ -61,6 +62,9 @@ __device__ __forceinline__ f32x4_t fetch4(const T* __restrict__ row, int k, int 
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = (float)raw[e];
     }
+  } else if (whole) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = to_float<T>(row[k + e]);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = to_float<T>(row[min(k + e, K - 1)]);
@@ -94,8 +98,9 @@ __global__ __launch_bounds__(256) void gemm_matrix_kernel(const TA* __restrict__
   const TW* w_row = W + (size_t)min(n0 + lr, N - 1) * K;
   f32x4_t ra, rw;
   auto fetch = [&](int k0) {
-    ra = fetch4<TA, VECTOR>(a_row, k0 + 4 * q, K);
-    rw = fetch4<TW, VECTOR>(w_row, k0 + 4 * q, K);
+    const bool whole = k0 + BK <= K;
+    ra = fetch4<TA, VECTOR>(a_row, k0 + 4 * q, K, whole);
+    rw = fetch4<TW, VECTOR>(w_row, k0 + 4 * q, K, whole);
   };
   auto stage = [&](int buf, int k0) {
     const int left = k_end - (k0 + 4 * q);   // a k past the end adds 0 * 0, which changes no sum
