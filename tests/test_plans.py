@@ -169,15 +169,6 @@ def test_prompt_tiles_are_halved_between_sixteen_waves_only_where_a_cu_would_be_
     assert not halves_prompt_tiles(0, 28, 0, 0, 256)
 
 
-def test_a_32_bit_product_of_9_to_16_tokens_streams_its_weights_where_they_are_many():
-    from vipera_rs_amd.ops.kernels import gemm_streams_weights_f32
-    small, heads = ((896, 896), (9728, 896), (37888, 1536), (896, 4864)), ((151936, 896), (151936, 1536), (37888, 3584), (9728, 8960))
-    for n, k in small + heads:
-        assert all(gemm_streams_weights_f32(m, n, k) for m in (1, 8))
-        assert all(gemm_streams_weights_f32(m, n, k) == ((n, k) in heads) for m in (9, 12, 16))
-        assert not any(gemm_streams_weights_f32(m, n, k) for m in (17, 64, 2048))
-
-
 def test_the_cut_of_a_32_bit_product_is_asked_for_once_for_a_size(monkeypatch):
     from vipera_rs_amd.ops import kernels
     asked, real = [], kernels._fn

@@ -230,21 +230,6 @@ def _gemm_generic_parts(m: int, n: int, k: int) -> int:
     return _fn("gemm_generic", "vk_gemm_generic_workspace", [_i, _i, _i], restype=_ll)(m, n, k)
 
 
-def gemm_streams_weights_f32(m: int, n: int, k: int) -> bool:
-    """Whether a 32-bit product of ``m`` tokens runs as a stream of the weights instead of in tiles on the matrix cores.
-
-    Up to 8 tokens always: the stream is bound by the weights' bytes there.  At 9 to 16 its FMAs bound it: its
-    workgroups (64 weight rows of 1,024 k, two at a time on each of 256 CUs) take 41.5 us a round, whatever part of the
-    round and of their k there is.  The tiles take 10 us and their weights at 2.4 TB/s, 1.8 where they walk K whole.
-    At 16 tokens, stream / tiles, us: 37,888 x 3,584 210 / 226, 151,936 x 896 210 / 296, 9,728 x 8,960 128 / 158, but
-    9,728 x 896 43 / 22, 37,888 x 1,536 123 / 108, 151,936 x 512 202 / 176; of 55 sizes the estimate picks the slower one
-    at none by more than 2 %.  From 17 tokens on the tiles were faster at every size (151,936 x 896: 557 / 307)."""
-    if m <= 8 or m > 16:
-        return m <= 8
-    rounds = -(-(-(-n // 64) * -(-k // 1024)) // 512)
-    return 41.5 * rounds < 10.0 + n * k * 4 / (2.4e6 if _gemm_generic_parts(m, n, k) else 1.8e6)
-
-
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                  accumulate: bool = False) -> None:
     """``out (+)= a @ w.T + bias`` with every product and sum in 32 bits; ``a`` and ``out`` may be row-strided views."""
@@ -262,9 +247,12 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
         _need(out.dtype == torch.float32, "gemm: accumulation needs a float32 output")
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
     ldc = out.stride(0) if m > 1 else max(out.stride(0), n)
-    if (gemm_streams_weights_f32(m, n, k) and a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0
-            and lda % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and k < 65535 * 1024):
-        # a stream of the weights (the same sums in the same order as the tiled kernel)
+    if (m <= 8 and a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0 and lda % 4 == 0
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and k < 65535 * 1024):
+        # up to 8 tokens in 32-bit: a stream of the weights (the same sums in the same order as the tiled kernel, whose
+        # matrix cores pass the stream's FMAs from there on: 9,728 x 896 at 8 tokens 21.2 us against 23.1, at 16 43.3 against
+        # 22.7; 37,888 x 3,584 at 8 tokens 117 against 196, at 16 213 against 188; 151,936 x 896 113 against 206 and 212
+        # against 201; of 55 sizes one is faster as a stream at 16, 1,024 x 18,944 with 51.2 against 53.3)
         slabs = _split_k_workspace(a.device, ((k + 1023) // 1024) * m * n, "stream")
         fn = _fn("gemm_generic", "vk_gemm_stream", [_p, _p, _p, _p, _i, _i, _i, _i, _ll, _ll, _i, _p, _ll, _p])
         _status(fn(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), _dt(out, "out"), m, n, k, lda, ldc, 1 if accumulate else 0,
