@@ -24,6 +24,7 @@ SIGNATURES = {
     "plain_rope_kvwrite": [P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, I, P],
     "plain_swiglu": [P, P, I, I, I, I, P],
     "plain_gemm_generic": [P, I, P, I, P, P, I, I, I, I, LL, LL, I, P],
+    "plain_gemm_generic_split": [P, I, P, I, P, P, I, I, I, I, LL, LL, I, P, LL, P],
     "plain_gemm_stream": [P, P, P, P, I, I, I, I, LL, LL, I, P, LL, P],
     "plain_gemm_bf16": [P, P, P, P, I, I, I, I, LL, LL, I, I, I, P, LL, P],
     "plain_gemm_bf16_mid": [P, P, P, P, I, I, I, I, LL, LL, I, I, I, P, LL, P],

@@ -197,11 +197,18 @@ extern "C" int plain_gemm_generic(const void* A, int a_dtype, const void* W, int
   return 0;
 }
 
-// the 32-bit weight stream for up to 64 tokens; the workspace shapes the kernel's work only
+// with K cut over workgroups; the workspace shapes the kernel's work only
+extern "C" int plain_gemm_generic_split(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
+                                        int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
+                                        float*, long long, void*) {
+  return plain_gemm_generic(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, nullptr);
+}
+
+// the 32-bit weight stream for up to 8 tokens; the workspace shapes the kernel's work only
 extern "C" int plain_gemm_stream(const float* A, const float* W, const float* bias, void* C, int c_dtype, int M, int N,
                                  int K, long long lda, long long ldc, int accumulate, float*, long long, void*) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || M > 64 || !known(c_dtype) || lda < K || ldc < N || (accumulate && c_dtype != DT_F32)) return BAD_ARGUMENT;
+  if (K <= 0 || M > 8 || !known(c_dtype) || lda < K || ldc < N || (accumulate && c_dtype != DT_F32)) return BAD_ARGUMENT;
   product(A, DT_F32, W, DT_F32, bias, C, c_dtype, M, N, K, lda, ldc, accumulate != 0);
   return 0;
 }

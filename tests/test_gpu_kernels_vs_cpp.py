@@ -255,7 +255,7 @@ def _kernel_with_pointer(name):
     return fn
 
 
-PRODUCTS = [(1, 48, 64), (7, 300, 96), (33, 1000, 264), (65, 130, 72), (200, 257, 136), (300, 520, 1024), (515, 384, 192)]
+PRODUCTS = [(1, 48, 64), (7, 300, 96), (8, 130, 1096), (33, 1000, 264), (65, 130, 72), (200, 257, 136), (300, 520, 1024), (515, 384, 192)]
 
 
 @pytest.mark.parametrize("m,n,k", PRODUCTS)
@@ -264,7 +264,14 @@ def test_products_beside_their_twins(m, n, k):
     a, w, bias = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g), torch.randn(n, generator=g)
     (got, want), = both("gemm_generic", "gemm_generic", [a, 0, w, 0, bias, torch.empty(m, n), 0, m, n, k, k, n, 0, None], [5])
     assert rel_err(got.numpy(), want.double().numpy()) < 2e-6
-    if m <= 64 and k % 4 == 0:
+    from vipera_rs_amd.ops.kernels import _gemm_generic_parts
+    floats = _gemm_generic_parts(m, n, k)
+    assert (floats > 0) == (k > 256)
+    for into, base in ((0, torch.empty(m, n)), (1, torch.empty(m, n, dtype=torch.bfloat16)), (2, torch.randn(m, n, generator=g))):
+        (got, want), = both("gemm_generic", "gemm_generic_split", [a, 0, w, 0, bias, base, into % 2, m, n, k, k, n, into // 2,
+                                                                   torch.empty(max(floats, 1)), floats, None], [5])
+        assert rel_err(got.float().numpy(), want.double().numpy()) < (6e-3 if into == 1 else 2e-6)
+    if m <= 8 and k % 4 == 0:
         slabs = torch.empty(((k + 1023) // 1024) * m * n)
         (got, want), = both("gemm_generic", "gemm_stream", [a, w, bias, torch.randn(m, n, generator=g), 0, m, n, k, k, n, 1, slabs,
                                                             slabs.numel(), None], [3])

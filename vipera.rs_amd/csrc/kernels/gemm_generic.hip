@@ -17,7 +17,7 @@
 //     never ends at -0);
 //   * the element is +0 + s0 + s1 + ... over its slabs in ascending order, then + bias, then,
 //     when accumulating, old + that.
-// Two kernels follow it. gemm_stream_kernel, for up to 64 rows of A in 32-bit operands, is a stream
+// Two kernels follow it. gemm_stream_kernel, for up to 8 rows of A in 32-bit operands, is a stream
 // of the weights: the product of a few tokens is bound by the bytes of W. gemm_matrix_kernel, for
 // everything else, runs on the matrix cores: v_mfma_f32_32x32x2_f32 computes each of its outputs as
 // fma(a[k + 1], w[k + 1], fma(a[k], w[k], c)), rounded after every product (compared with fmaf chains bit
@@ -216,10 +216,10 @@ __global__ __launch_bounds__(256) void gemm_parts_finish_kernel(const float* __r
 
 // How K is cut for a product of M x N: whole (0), in slabs (4) or in ranges (1), so that the workgroups fill the chip
 // (256 CUs, four workgroups each). Measured on tiles x K, us whole / slabs / ranges, weights from memory:
-//   many tiles need no cut, and the parts' way through memory costs: 2,432 x 896: 187 / - / 215; 912 x 896: 83 / - / 89;
-//   2,240 x 1,536: 306 / 315 / 340; but 608 x 896: 67 / - / 63 and 1,120 x 1,536: 183 / 160 / 163;
-//   slabs where those are enough: 384 x 8,960: 446 / 315 / 351; 56 x 18,944: 792 / 121 / 130; 512 x 1,536: 82 / 79 / 85;
-//   ranges below: 112 x 4,864: 175 / 72 / 67; 256 x 1,536: 61 / 50 / 45; 84 x 896: 36 / - / 18; 14 x 4,864: 175 / 43 / 29.
+//   many tiles need no cut, and the parts' way through memory costs: 2,432 x 896: 193 / - / 221; 912 x 896: 82 / - / 87;
+//   2,240 x 1,536: 296 / 293 / 331; but 608 x 896: 64 / - / 64 and 1,120 x 1,536: 181 / 161 / 174;
+//   slabs where those are enough: 384 x 8,960: 426 / 295 / 335; 56 x 18,944: 729 / 117 / 138; 512 x 1,536: 75 / 74 / 84;
+//   ranges below: 112 x 4,864: 177 / 69 / 66; 256 x 1,536: 54 / 49 / 46; 84 x 896: 32 / - / 18; 14 x 4,864: 154 / 40 / 24.
 int matrix_units(int M, int N, int K) {
   const long long tiles = (long long)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
   const int ranges = (K + RANGE_K - 1) / RANGE_K, slabs = (K + SLAB_K - 1) / SLAB_K;
@@ -283,7 +283,7 @@ int launch(const void* A_, const void* W_, const float* bias, void* C_, int M, i
 }
 
 // ---------------------------------------------------------------------------------------------
-// The weight stream, for 32-bit A and W and up to 64 rows of A. A workgroup of four waves owns 64 rows
+// The weight stream, for 32-bit A and W and up to 8 rows of A. A workgroup of four waves owns 64 rows
 // of W and one slab of K; wave w owns range w of the slab, and each of its lanes one row of W, whose
 // chain over the range's k it computes for all rows of A (MT accumulators). What a lane needs of W is
 // consecutive in memory, which is the opposite of what 64 lanes should request together: so W goes
@@ -311,9 +311,8 @@ template <int MT>
 __global__ __launch_bounds__(256) void gemm_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                           float* __restrict__ slabs, int M, int N, int K,
                                                           long long lda) {
-  constexpr int A_LOADS = (MT + 7) / 8;                 // a load instruction brings 32 k of eight rows of A
-  constexpr int STAGE = W_STAGE + A_LOADS * 1024;
-  constexpr int LOADS = W_LOADS + A_LOADS;
+  static_assert(MT <= 8, "a load instruction brings 32 k of eight rows of A");
+  constexpr int STAGE = W_STAGE + 1024, LOADS = W_LOADS + 1;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -326,7 +325,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(const float* __restric
   for (int m = 0; m < MT; ++m) acc[m] = 0.f;
 
   // what this lane fetches with each load instruction of a stage: of W, chunk (slot ^ swizzle) of row 8 i + sub_row;
-  // of A, chunk `slot` of row 8 i + sub_row. A row past the end is a copy of the last one and is not stored; a
+  // of A, chunk `slot` of row sub_row. A row past the end is a copy of the last one and is not stored; a
   // chunk past the end of K is a copy of the last one and is never multiplied.
   const int sub_row = lane >> 3, slot = lane & 7;
   const float* w_from[W_LOADS];
@@ -343,11 +342,8 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(const float* __restric
     for (int i = 0; i < W_LOADS; ++i)
       __builtin_amdgcn_global_load_lds((global_ptr)(w_from[i] + min(k_sub + w_chunk[i], K - 4)),
                                        (lds_ptr)(to + i * 1024), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(A + (size_t)min(i * 8 + sub_row, M - 1) * lda + min(k_sub + (slot << 2), K - 4)),
-          (lds_ptr)(to + W_STAGE + i * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((global_ptr)(A + (size_t)min(sub_row, M - 1) * lda + min(k_sub + (slot << 2), K - 4)),
+                                     (lds_ptr)(to + W_STAGE), 16, 0, 0);
   };
   const unsigned my_row = (unsigned)(lane * (SUB_K * 4)), my_swizzle = (unsigned)((lane >> 1) & 7);
   if (k_begin < k_end) {
@@ -431,7 +427,7 @@ __global__ __launch_bounds__(256) void gemm_stream_finish_kernel(const float* __
 template <int MT>
 int launch_stream_as(const float* A, const float* W, float* slabs, int M, int N, int K, long long lda, int num_slabs,
                      hipStream_t s) {
-  constexpr int lds_bytes = 4 * 2 * (W_STAGE + (MT + 7) / 8 * 1024);
+  constexpr int lds_bytes = 4 * 2 * (W_STAGE + 1024);
   static_assert(4 * MT * STREAM_ROWS * 4 <= lds_bytes, "the ranges' sums reuse the stages");
   static bool configured = false;
   if (!configured) {
@@ -447,18 +443,13 @@ int launch_stream_as(const float* A, const float* W, float* slabs, int M, int N,
 }
 }  // namespace
 
-// Floats of workspace that vk_gemm_stream needs for an M x N product over K.
-extern "C" long long vk_gemm_stream_workspace(int M, int N, int K) {
-  return (long long)((K + SLAB_K - 1) / SLAB_K) * M * N;
-}
-
-// The weight stream: float A (row stride lda, a multiple of 4) and W, M <= 64, K a multiple of 4, 16-byte aligned
-// operands; C float or bfloat16. `slabs`: workspace of vk_gemm_stream_workspace(M, N, K) floats.
+// The weight stream: float A (row stride lda, a multiple of 4) and W, M <= 8, K a multiple of 4, 16-byte aligned
+// operands; C float or bfloat16. `slabs`: workspace of ceil(K / 1024) M N floats.
 extern "C" int vk_gemm_stream(const float* A, const float* W, const float* bias, void* C, int c_dtype, int M, int N,
                               int K, long long lda, long long ldc, int accumulate, float* slabs,
                               long long slab_floats, void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64) return VK_UNSUPPORTED_SIZE;
+  if (M > 8) return VK_UNSUPPORTED_SIZE;
   if (K < 4 || (K & 3) || (lda & 3) || lda < K || ldc < N || !slabs) return VK_BAD_ARGUMENT;
   if (((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return VK_BAD_ARGUMENT;
   if (accumulate && c_dtype != DT_F32) return VK_BAD_ARGUMENT;
@@ -469,10 +460,7 @@ extern "C" int vk_gemm_stream(const float* A, const float* W, const float* bias,
   if (M <= 1) status = launch_stream_as<1>(A, W, slabs, M, N, K, lda, num_slabs, s);
   else if (M <= 2) status = launch_stream_as<2>(A, W, slabs, M, N, K, lda, num_slabs, s);
   else if (M <= 4) status = launch_stream_as<4>(A, W, slabs, M, N, K, lda, num_slabs, s);
-  else if (M <= 8) status = launch_stream_as<8>(A, W, slabs, M, N, K, lda, num_slabs, s);
-  else if (M <= 16) status = launch_stream_as<16>(A, W, slabs, M, N, K, lda, num_slabs, s);
-  else if (M <= 32) status = launch_stream_as<32>(A, W, slabs, M, N, K, lda, num_slabs, s);
-  else status = launch_stream_as<64>(A, W, slabs, M, N, K, lda, num_slabs, s);
+  else status = launch_stream_as<8>(A, W, slabs, M, N, K, lda, num_slabs, s);
   if (status != 0) return status;
   const long long outputs = (long long)M * N;
   const unsigned blocks = (unsigned)((outputs + 255) / 256);
@@ -507,7 +495,7 @@ int dispatch(const void* A, int a_dtype, const void* W, int w_dtype, const float
 }
 }  // namespace
 
-// dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.
+// K whole in every workgroup, which needs no workspace. dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.
 extern "C" int vk_gemm_generic(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
                                int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
                                void* stream) {
