@@ -98,27 +98,34 @@ def test_the_small_tilings_give_the_bits_of_the_large_one(tiling, ranges):
         kernels.gemm_bf16_force_tiling(-1)
 
 
-@pytest.mark.parametrize("m,n,k", [(129, 33, 2048), (512, 1057, 2048), (300, 64, 8192), (512, 2576, 512), (1000, 640, 1536), (700, 5120, 8256)])
-def test_the_tiles_chosen_for_a_product_do_not_change_its_bits(m, n, k):
-    """Past 128 tokens a product that takes 128x128 tiles may be carried out by smaller ones: the same bits as the
-    128x128 tiles give with one of the splits that are tried."""
+@pytest.mark.parametrize("m,n,k,tiling", [(129, 33, 2048, 13), (512, 64, 2048, 13), (161, 1792, 10496, 13), (512, 2048, 512, 14),
+                                          (512, 1057, 2048, 14), (468, 1792, 4352, 14), (512, 2576, 512, 15), (700, 5120, 2048, 15),
+                                          (140, 5536, 1600, 15), (330, 7488, 7168, 9), (953, 512, 6400, 9)])
+def test_the_tiles_chosen_for_a_product_do_not_change_its_bits(m, n, k, tiling):
+    """Past 128 tokens a product planned as 128x128 tiles may be carried out by smaller ones: it is at these sizes, one beside
+    each line of the choice, with the bits that the 128x128 tiles give with the planned ranges of K."""
     from vipera_rs_amd.ops import kernels
     g = torch.Generator().manual_seed(m + n + k)
     a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
     w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
-    out = torch.empty(m, n, device=DEV)
+    out, other = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    chosen, ranges = kernels.gemm_bf16_tile_plan(m, n, k)
+    assert chosen == tiling
     kernels.gemm_bf16(a, w, None, out)
     assert _rel(out, a.double() @ w.double().T) < 1e-5
-    same = []
     try:
-        for ranges in (1, 2, 4, 8):
-            kernels.gemm_bf16_force_tiling(9, ranges)
-            other = torch.empty(m, n, device=DEV)
-            kernels.gemm_bf16(a, w, None, other)
-            same.append(torch.equal(out, other))
+        kernels.gemm_bf16_force_tiling(9, ranges)
+        kernels.gemm_bf16(a, w, None, other)
     finally:
         kernels.gemm_bf16_force_tiling(-1)
-    assert any(same)
+    assert torch.equal(out, other)
+    if ranges > 1:      # and no other number of ranges gives them
+        try:
+            kernels.gemm_bf16_force_tiling(9, ranges // 2)
+            kernels.gemm_bf16(a, w, None, other)
+        finally:
+            kernels.gemm_bf16_force_tiling(-1)
+        assert not torch.equal(out, other)
 
 
 @pytest.mark.parametrize("tiling", [0, 9, 7, 5, 6])
@@ -267,8 +274,9 @@ def test_gemm_generic_against_float64(m, n, k, dtypes):
 @pytest.mark.parametrize("k", [64, 200, 256, 1100, 2600])
 def test_gemm_generic_does_not_depend_on_the_batch(k):
     """Every output element is summed in one fixed order (chains over ranges of 256 k, four ranges to a slab, slabs in
-    ascending order), whichever kernel computes it: the weight stream that takes up to 64 tokens gives bit for bit
-    the rows of the tiled kernel that takes 70, alone or in any company, with and without a bias, accumulating or not."""
+    ascending order), whichever kernel computes it: the weight stream that takes up to 8 tokens and the tiles that take 33 and
+    64 give bit for bit the rows of the tiles that take 70, alone or in any company, with and without a bias, accumulating
+    or not."""
     from vipera_rs_amd.ops import kernels
     g = torch.Generator().manual_seed(k)
     a = torch.randn(70, k, generator=g).to(DEV)
@@ -278,7 +286,7 @@ def test_gemm_generic_does_not_depend_on_the_batch(k):
     whole = torch.empty(70, 90, device=DEV)
     kernels.gemm_generic(a, w, None, whole)
     assert _rel(whole, a.double() @ w.double().T) < 2e-6
-    for rows in ([37], [0, 1], list(range(5, 12)), list(range(3, 36)), list(range(6, 70))):
+    for rows in ([37], [0, 1], list(range(5, 12)), list(range(50, 58)), list(range(61, 70)), list(range(3, 36)), list(range(6, 70))):
         part = torch.empty(len(rows), 90, device=DEV)
         kernels.gemm_generic(a[rows].contiguous(), w, None, part)
         assert torch.equal(part, whole[rows]), f"{len(rows)} rows"      # bit for bit
@@ -295,10 +303,10 @@ def test_gemm_generic_does_not_depend_on_the_batch(k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1024, 1024, 520), (1030, 1100, 1027), (1500, 905, 258), (1153, 1025, 2052)])
-def test_the_wide_tiles_of_gemm_generic_sum_in_the_same_order(m, n, k):
-    """128 rows and more on enough tiles take 128 x 128 tiles with 8 x 8 outputs a thread: against 64-bit, and bit
-    for bit the rows that the 64 x 64 tiles give 70 rows at a time and the weight stream 33 at a time; with a bias,
-    accumulating, into bfloat16, from bfloat16 activations, and with rows that start off a 16-byte boundary."""
+def test_many_tiles_of_gemm_generic_sum_in_the_same_order(m, n, k):
+    """Against 64-bit, and bit for bit the rows that the tiles give 70 and 33 rows at a time and, where K is in fours, the weight
+    stream 8 at a time; with a bias, accumulating, into bfloat16, from bfloat16 activations, and with rows that start off a
+    16-byte boundary."""
     from vipera_rs_amd.ops import kernels
     g = torch.Generator().manual_seed(m + n + k)
     a = torch.randn(m, k, generator=g).to(DEV)
@@ -308,7 +316,7 @@ def test_the_wide_tiles_of_gemm_generic_sum_in_the_same_order(m, n, k):
     whole = torch.full((m, n), float("nan"), device=DEV)
     kernels.gemm_generic(a, w, bias, whole)
     assert _rel(whole, a.double() @ w.double().T + bias.double()) < 2e-6
-    for rows in (70, 33):
+    for rows in (70, 33, 8):
         for start in (0, 128 * 3 + 5, m - rows):
             part = torch.empty(rows, n, device=DEV)
             kernels.gemm_generic(a[start:start + rows], w, bias, part)
@@ -437,11 +445,10 @@ def test_gemm_generic_of_more_tiles_than_one_launch_takes():
         torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 64, 4), (3, 70, 36), (8, 3584, 1536), (9, 129, 1028), (16, 1000, 4096), (40, 200, 520),
-                                   (64, 333, 2052)])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 4), (2, 200, 520), (3, 70, 36), (4, 1000, 4096), (5, 129, 1028), (7, 333, 2052), (8, 3584, 1536)])
 def test_gemm_stream_against_float64(m, n, k):
     """The 32-bit weight stream at sizes of its own: K that ends inside a chunk of 32, a range and a slab, rows of
-    W that do not fill a workgroup's 64, every count of tokens' class."""
+    W that do not fill a workgroup's 64, every count of tokens' class, filled and not."""
     from vipera_rs_amd.ops import kernels
     g = torch.Generator().manual_seed(m * n + k)
     a = torch.randn(m, k, generator=g).to(DEV)
