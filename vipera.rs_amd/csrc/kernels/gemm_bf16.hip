@@ -433,6 +433,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const __bf16* _
 // STAGES 3 (for up to 128 tokens, where the product is a stream of the weights and a CU's bytes in flight are
 // what bounds it): step s + 3 is requested when step s's stage is free, and the barrier of a step waits for
 // step s + 1 only, so the loads of two steps are in flight instead of one; STAGES 4 likewise.
+// group_tile_direct (group_tile.h) is the same loop over gathered rows; a change to one is to be weighed for the other.
 constexpr int DIRECT_ROW = BK * 2;  // bytes per LDS row
 
 // Until none of the wave's vector memory loads is in flight (s_waitcnt vmcnt(0), the other counters left

@@ -98,6 +98,9 @@ __device__ __forceinline__ void group_tile_mma(ARow a_row, WRow w_row, int K, un
 // instruction fills 1 KB: 8 rows, lane L the 16 bytes at 16 L); chunk c of row r sits in slot c ^ (r % 8), so that 16
 // rows read the same chunk from different banks.  A wave reads the operands of a half step while it multiplies the other half.
 //
+// The main loop is that of gemm_tile_direct_kernel (gemm_bf16.hip), whose rows lie a stride apart; a change to one is to be
+// weighed for the other.
+//
 // Every row's place is a byte offset of its own, so rows may be gathered; a row that does not exist has GT_NO_ROW and
 // reads zero without touching memory.
 constexpr int GT_WIDE = 256;                                     // rows of activations of its larger tile
