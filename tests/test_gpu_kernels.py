@@ -405,6 +405,44 @@ def test_the_matrix_instruction_is_two_fused_multiply_adds_for_all_values(values
         assert torch.equal(tiles, (a[:, :1].double() * w[:, :1].double().T).float())
 
 
+def test_cut_products_in_a_captured_step():
+    """Products whose K is cut, one behind the other in a graph: their parts come from the graph's memory, and every replay gives
+    the eager bits whatever the program allocates and computes in between."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(8)
+    a, w0 = torch.randn(24, 1100, generator=g).to(DEV), torch.randn(900, 1100, generator=g).to(DEV)
+    w1, x = torch.randn(1100, 900, generator=g).to(DEV) / 30, torch.empty_like(a)
+    assert kernels._gemm_generic_parts(24, 900, 1100) and kernels._gemm_generic_parts(24, 1100, 900)
+
+    def step():
+        x.copy_(a)
+        for _ in range(3):
+            hidden = torch.empty(24, 900, device=DEV)
+            kernels.gemm_generic(x, w0, None, hidden)
+            kernels.gemm_generic(hidden, w1, None, x, accumulate=True)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for turn in range(4):
+        a.normal_()
+        step()
+        torch.cuda.synchronize()
+        want = x.clone()
+        x.fill_(float("nan"))
+        noise = [torch.full((24, 900, 5), float(turn), device=DEV) for _ in range(4)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(x, want), turn
+        del noise
+
+
 def test_gemm_generic_needs_no_memory_for_its_parts():
     """Where the memory for the parts of a cut K is not there, the product runs uncut: the same bits."""
     from vipera_rs_amd.ops import kernels
