@@ -635,7 +635,7 @@ def test_attention_kernels_against_plain_softmax(case, dtype, stale):
                              skip_single_of=es)
         assert _rel(out3.cpu(), want) < tol, "32-bit decode kernel beside the general one"
         if kernels.attn_prefill_f32_supported(qkv_d, k_d, hd):
-            # the portions on the 32-bit kernel that walks the positions in LDS tiles; tiles of 128 or of 64 tokens
+            # the portions on the 32-bit kernel that walks the positions in tiles; tiles of 128 or of 64 tokens
             for tile_tokens in (128, 64):
                 tiles = [x for e, n in enumerate(counts) if n > 1 for off in range(0, n, tile_tokens) for x in (e, off)]
                 rows = [t for e, n in enumerate(counts) if n > 1 for t in range(starts[e], starts[e + 1])]
@@ -1085,3 +1085,41 @@ def test_a_steps_words_are_fetched_from_pinned_host_memory(count):
     assert int(out.min()) == 5 and int(out.max()) == 5
     with pytest.raises(InvalidArgumentError):
         kernels.fetch_words(torch.zeros(count, dtype=torch.int32), out)   # pageable memory is refused on the host
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(3, 1, 16), (4, 2, 80), (2, 2, 128), (120, 60, 16)])
+@pytest.mark.parametrize("bs", [4, 20, 64, 192])
+@pytest.mark.parametrize("window,keep", [(0, 0), (70, 0), (40, 5), (30, 130), (-48, 0)])
+def test_32_bit_prompt_attention_at_the_edges_of_its_tiles(heads, kv_heads, hd, bs, window, keep):
+    """Portions of 15 to 65 tokens that begin on both sides of a tile of 64 positions, pages that divide a tile, do not, or
+    hold several; windows that have given pages back (what those and the free slots hold is NaN), first positions that stay
+    visible, a sink, a cap, a bias by distance and a gate; few heads (16 tokens a workgroup) and many (32).  The general kernel
+    sums a score in the same order and the softmax over other tiles: 2e-6 as in the tests of both against 64 bits."""
+    from types import SimpleNamespace
+    from vipera_rs_amd.ops import kernels
+    entries = [(15, 15), (80, 17), (129, 65), (263, 16)]
+    counts, first = [n for _, n in entries], [kv - n for kv, n in entries]
+    cache = _Paged([kv for kv, _ in entries], kv_heads, hd, bs, torch.float32, heads * 7 + bs, stale_nan=True)
+    table = cache.table
+    if window:
+        lowest = [max(0, f + 1 - window) if window > 0 else f - f % -window for f in first]
+        table = cache.with_pages_given_back(lowest)
+        kept = min((keep + bs - 1) // bs, table.shape[1])
+        table[:, :kept] = cache.table[:, :kept]
+    starts = [sum(counts[:e]) for e in range(len(counts) + 1)]
+    T = starts[-1]
+    g = torch.Generator().manual_seed(hd + bs)
+    qkv = torch.randn(T, (heads + 2 * kv_heads) * hd, generator=g).to(DEV)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    positions, entry_of = ints([f + i for f, n in zip(first, counts) for i in range(n)]), ints([e for e, n in enumerate(counts) for _ in range(n)])
+    tiles = ints([x for e, n in enumerate(counts) for off in range(0, n, 64) for x in (e, off)])
+    k, v, table = cache.k.to(DEV), cache.v.to(DEV), table.to(DEV)
+    plain = SimpleNamespace(sink=None, rel=None, keep_first=keep, gate=None)
+    full = SimpleNamespace(sink=torch.randn(heads, generator=g).to(DEV), rel=torch.randn(heads, 90, generator=g).to(DEV), keep_first=keep,
+                           gate=torch.randn(T, heads, generator=g).to(DEV))
+    for extras, cap in ((plain, 0.0), (full, 5.0)):
+        want, got = torch.zeros(T, heads * hd, device=DEV), torch.full((T, heads * hd), float("nan"), device=DEV)
+        kernels.attn_generic(qkv, k, v, want, positions, entry_of, table, heads, kv_heads, hd, hd ** -0.5, window, softcap=cap, extras=extras)
+        kernels.attn_prefill_f32(qkv, k, v, got, tiles, 64, ints(starts), ints(first), table, heads, kv_heads, hd, hd ** -0.5, window,
+                                 softcap=cap, extras=extras)
+        assert _rel(got.cpu(), want.cpu().double()) < 2e-6

@@ -12,6 +12,8 @@
 //
 // Cache layout: K [page, kv_head, slot, head_dim], V transposed [page, kv_head, head_dim, slot];
 // page of position p = table[entry, p / block_size].
+#include <type_traits>
+
 #include "attn_extras.h"
 
 namespace {
@@ -336,208 +338,310 @@ __global__ __launch_bounds__(64) void attn_combine_f32_kernel(const float* __res
 
 // ---------------------------------------------------------------------------------------------
 // Prompt portions in 32-bit. The general kernel gives every (token, query head) a workgroup that walks all of the
-// token's positions alone: 2,048 tokens x 28 heads read the cache 58 GB over per layer. Here a workgroup owns 64
+// token's positions alone: 2,048 tokens x 28 heads read the cache 58 GB over per layer. Here a workgroup owns 16 RB
 // consecutive tokens of one entry and one query head and walks the positions in tiles of 64 that begin at
 // multiples of 64 (so which positions share a tile, and with it a token's arithmetic, depends on the position alone,
-// not on how the prompt was cut): the K tile and the V^T tile go into LDS as they lie in the pages (rows padded by 16
-// bytes, so that sixteen lanes reading sixteen consecutive rows spread over the banks), slots past the last
-// position of the tile's tokens as zeros (a weight of zero times whatever a free slot holds must stay zero), and so
-// are positions before the first one that the tile's first token sees: a window has passed them, and their page
-// may have been given back (its id in the table is then -1 and must not be followed).
-//   scores   thread (ty, tx) of 16 x 16 owns tokens 4 ty .. 4 ty + 3 and positions tx, tx + 16, tx + 32, tx + 48: a
-//            dot product is an FMA chain over the head width in ascending order;
-//   softmax  online over the tiles (crates/vipera-backend-cpu/src/model.rs:1840-1857 is the plain form): a row's
+// not on how the prompt was cut).  Both products run on the matrix cores: v_mfma_f32_16x16x4_f32 computes each of its
+// outputs as four FMAs in ascending k on top of c (compared with fmaf chains bit for bit), so the sums are those of
+// FMA chains:
+//   scores   wave w owns the tile's positions 16 w .. 16 w + 15 for all of the workgroup's tokens: an FMA chain over the
+//            head width in ascending order;
+//   softmax  online over the tiles (crates/vipera-backend-cpu/src/model.rs:1840-1857 is the plain form): thread (ty, tx) of
+//            16 x 16 owns positions tx, tx + 16, tx + 32, tx + 48 of tokens ty, ty + 16, ...; a row's
 //            maximum and sum over the sixteen lanes that share it in a fixed tree, library-grade exp;
-//   output   the weights go through LDS; thread (ty, tx) owns the same four tokens and dims tx, tx + 16, ...: an
-//            FMA chain over the tile's positions in ascending order.
-// Head widths that are multiples of 16 up to 128 (the tiles of a wider head do not fit a CU's LDS) and pages of a
-// multiple of 4 positions; anything else stays with the general kernel.
-constexpr int PF_TILE = 64;
-template <int DPT>   // the head width is 16 * DPT
+//   output   wave w owns dims 16 w .. 16 w + 15 (and 64 further on): an FMA chain over the tile's positions in ascending order.
+// No two waves read the same of K or V, so both go from memory into registers, sixteen bytes a lane, K of the next tile
+// while this one's softmax runs; what the matrix instruction wants of a lane (one k of four) comes out of two lane
+// exchanges a register pair. Only scores and weights go through LDS, in two buffers, two barriers a tile. Positions past the
+// tokens' last one and those before the first one that the first token sees (a window has passed them, their page may have
+// been given back and its id in the table is then -1) are read at the last position instead; their scores are masked and
+// their values count as zeros (a weight of zero times whatever a free slot holds must stay zero).
+//
+// What bounds it: a few hundred tokens have little to multiply (333 tokens of 14 heads of 64: 0.2 GFLOP a layer, 1.3 us of
+// the chip), and their last tokens' walk takes some 2.6 us a tile, one wave a SIMD issuing some 600 instructions; long prompts
+// run at 80 TFLOP/s (their matrix instructions wait for the softmax between the products). us, with both products on
+// vector FMAs in LDS tiles of 64 tokens (the same sums) and so: 333 tokens of 14 heads of 64 66 and 19; 2,048 of them 378 and
+// 182; 4,096 tokens of 28 heads of 128 7,570 and 1,970. Asking for a tile's keys and pages a whole tile ahead gained nothing.
+// Head widths that are multiples of 16 up to 128 and pages of a multiple of 4 positions; anything else stays with the
+// general kernel.
+constexpr int PF_TILE = 64, PF_ROW = PF_TILE + 4;   // a row of scores: eight lanes' 16 bytes of consecutive rows lie in 32 different banks
+typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
+
+// r[e] holds k 4 g + e in lane group g = lane / 16; afterwards r[t] holds k 4 t + g.
+__device__ __forceinline__ void transpose_lane_groups(float (&r)[4]) {
+  auto swap = [](float& x, float& y, auto wide) {
+    const unsigned a = __builtin_bit_cast(unsigned, x), b = __builtin_bit_cast(unsigned, y);
+    if constexpr (decltype(wide)::value) {
+      const auto s = __builtin_amdgcn_permlane32_swap(a, b, false, false);   // the upper half of x and the lower half of y
+      x = __builtin_bit_cast(float, (unsigned)s[0]);
+      y = __builtin_bit_cast(float, (unsigned)s[1]);
+    } else {
+      const auto s = __builtin_amdgcn_permlane16_swap(a, b, false, false);   // x's odd groups and y's even ones
+      x = __builtin_bit_cast(float, (unsigned)s[0]);
+      y = __builtin_bit_cast(float, (unsigned)s[1]);
+    }
+  };
+  swap(r[0], r[1], std::false_type{});
+  swap(r[2], r[3], std::false_type{});
+  swap(r[0], r[2], std::true_type{});
+  swap(r[1], r[3], std::true_type{});
+}
+
+// The maximum and the sum over 16 neighbouring lanes, as a tree over lanes 1, 2, 4 and 8 apart, without LDS: once a quad
+// holds one value, a mirrored half row brings that of the lane 4 apart, and a mirrored row that of the lane 8 apart.
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float max16(float v) {
+  v = fmaxf(v, lane_move<0xB1>(v));
+  v = fmaxf(v, lane_move<0x4E>(v));
+  v = fmaxf(v, lane_move<0x141>(v));
+  return fmaxf(v, lane_move<0x140>(v));
+}
+__device__ __forceinline__ float sum16(float v) {
+  v += lane_move<0xB1>(v);
+  v += lane_move<0x4E>(v);
+  v += lane_move<0x141>(v);
+  return v + lane_move<0x140>(v);
+}
+
+template <int DPT, int RB>   // the head width is 16 * DPT, the workgroup's tokens 16 * RB
 __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     const float* __restrict__ q, long long q_stride, const float* __restrict__ k_cache,
     const float* __restrict__ v_cache, float* __restrict__ out, const int* __restrict__ tiles,
     const int* __restrict__ entry_start, const int* __restrict__ entry_first_pos, const int* __restrict__ block_table,
     int table_width, int block_size, int heads, int kv_heads, float scale, int window, float softcap, int tile_tokens,
     AttnExtras ex) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int HD = 16 * DPT, QROW = HD + 4, VROW = PF_TILE + 4;
-  extern __shared__ __attribute__((aligned(16))) float pf_lds[];
-  float* q_s = pf_lds;                     // [64][QROW]
-  float* k_s = q_s + PF_TILE * QROW;       // [64][QROW]
-  float* v_s = k_s + PF_TILE * QROW;       // [HD][VROW], transposed as in the pages
-  float* p_s = v_s + HD * VROW;            // [64][VROW]
-  const int parts = tile_tokens / PF_TILE;                 // workgroups per tile of the step's list
+  constexpr int HD = 16 * DPT, ROWS = 16 * RB, OB = (DPT + 3) / 4;
+  __shared__ __attribute__((aligned(16))) float sw_s[2][ROWS][PF_ROW];   // scores, then weights
+  __shared__ float rescale_s[2][ROWS];
+  const int parts = tile_tokens / ROWS;                    // workgroups per tile of the step's list
   // the list comes with the tiles that see most positions last; workgroups start in the order of their index, and the
   // long ones should start first, so that the short ones fill the gaps at the end
   const int index = gridDim.x - 1 - blockIdx.x;
   const int tile = index / parts, part = index % parts, h = blockIdx.y;
-  const int entry = tiles[2 * tile], offset = tiles[2 * tile + 1] + part * PF_TILE;
+  const int entry = tiles[2 * tile], offset = tiles[2 * tile + 1] + part * ROWS;
   const int count = entry_start[entry + 1] - entry_start[entry];
   if (offset >= count) return;
-  const int rows = min(PF_TILE, count - offset);
+  const int rows = min(ROWS, count - offset);
   const int tok0 = entry_start[entry] + offset, pos0 = entry_first_pos[entry] + offset;
   const int last_pos = pos0 + rows - 1;
   const int kvh = h / (heads / kv_heads);
   const int* table = block_table + (size_t)entry * table_width;
   const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
 
-  for (int i = tid; i < PF_TILE * (HD / 4); i += 256) {
-    const int r = i / (HD / 4), c = (i % (HD / 4)) * 4;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (r < rows) v = *(const f32x4*)(q + (size_t)(tok0 + r) * q_stride + (size_t)h * HD + c);
-    *(f32x4*)(q_s + r * QROW + c) = v;
+  float qf[RB][DPT * 4];   // a row past the end is a copy of the last and is not stored
+#pragma unroll
+  for (int b = 0; b < RB; ++b) {
+    const float* row = q + (size_t)(tok0 + min(16 * b + lr, rows - 1)) * q_stride + (size_t)h * HD + 4 * lg;
+#pragma unroll
+    for (int u = 0; u < DPT; ++u) {
+      const pf_f32x4 v = *(const pf_f32x4*)(row + 16 * u);
+      float r[4] = {v[0], v[1], v[2], v[3]};
+      transpose_lane_groups(r);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) qf[b][4 * u + t] = r[t];
+    }
   }
-  float m[4], l[4], o[4][DPT];
+  float m[RB], l[RB];
+  pf_f32x4 o[OB][RB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
+  for (int b = 0; b < RB; ++b) {
+    m[b] = -INFINITY;
+    l[b] = 0.f;
 #pragma unroll
-    for (int j = 0; j < DPT; ++j) o[i][j] = 0.f;
+    for (int d = 0; d < OB; ++d) o[d][b] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int lowest = first_visible(pos0, window);   // the first token's first position
   // the tiles of the first positions that stay visible whatever the window has passed come first (those that the
   // window's own tiles do not hold anyway), then the tiles from the window's first position on
   const int keep = ex.keep_first;
   const int first_tile = lowest / PF_TILE, kept_tiles = min((keep + PF_TILE - 1) / PF_TILE, first_tile);
-  for (int it = 0;; ++it) {
-    const int kv0 = (it < kept_tiles ? it : first_tile + (it - kept_tiles)) * PF_TILE;
-    if (kv0 > last_pos) break;
-    __syncthreads();   // the tile before has been read
-    for (int i = tid; i < PF_TILE * (HD / 4); i += 256) {
-      const int r = i / (HD / 4), c = (i % (HD / 4)) * 4, p = kv0 + r;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if ((p >= lowest || p < keep) && p <= last_pos)   // below `lowest` the window has passed: the page may have been given back
-        v = *(const f32x4*)(k_cache + (((size_t)table[p / block_size] * kv_heads + kvh) * block_size + p % block_size) * HD + c);
-      *(f32x4*)(k_s + r * QROW + c) = v;
-    }
-    for (int i = tid; i < HD * (PF_TILE / 4); i += 256) {
-      const int d = i / (PF_TILE / 4), c = (i % (PF_TILE / 4)) * 4, p = kv0 + c;   // four positions of one page
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if ((p + 3 >= lowest || p < keep) && p <= last_pos) {   // the four share a page, which is held if any of them is visible
-        v = *(const f32x4*)(v_cache + (((size_t)table[p / block_size] * kv_heads + kvh) * HD + d) * block_size + p % block_size);
+  auto tile_begin = [&](int it) { return (it < kept_tiles ? it : first_tile + (it - kept_tiles)) * PF_TILE; };
+  // a tile that every token sees whole needs no masks
+  const int lowest_of_last = first_visible(last_pos, window);
+  auto whole = [&](int kv0) { return kv0 >= lowest_of_last && kv0 + PF_TILE - 1 <= pos0; };
+  // Where a tile's positions lie: its first position's page index is the same for all lanes; a lane's position is at most 63
+  // further on, which a 16-bit reciprocal divides exactly (pages of 64 positions and more: a comparison).
+  const int reciprocal = block_size < PF_TILE ? 65536 / block_size + 1 : 0;
+  const int long_page = block_size < PF_TILE ? 0x7fffffff : block_size;
+  auto pages_in = [&](int rem) { return (int)(((unsigned)rem * (unsigned)reciprocal) >> 16) + (rem >= long_page ? 1 : 0); };
+  const size_t page_floats = (size_t)kv_heads * block_size * HD;
+  const float* k_head = k_cache + (size_t)kvh * block_size * HD + 4 * lg;
+  const float* v_head = v_cache + (size_t)kvh * block_size * HD;
+  int v_row[OB];   // the lane's dims; past the head width the last one, which is not stored
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if ((p + e < lowest && p + e >= keep) || p + e > last_pos) v[e] = 0.f;
+  for (int d = 0; d < OB; ++d) v_row[d] = min(16 * (wave + 4 * d) + lr, HD - 1) * block_size;
+  auto held = [&](int p) { return (p >= lowest || p < keep) && p <= last_pos; };
+  // a held place of a tile for the lanes whose own is not
+  auto stand_in = [&](int it, int kv0) {
+    return it < kept_tiles ? min(PF_TILE - 1, keep - 1 - kv0) : kv0 < lowest ? lowest - kv0 : min(PF_TILE - 1, last_pos - kv0);
+  };
+  pf_f32x4 k_raw[DPT];
+  auto fetch_k = [&](int it, int kv0, int index0, auto is_whole) {
+    int off = 16 * wave + lr;
+    if constexpr (!decltype(is_whole)::value) off = held(kv0 + off) ? off : stand_in(it, kv0);
+    const int rem = kv0 - index0 * block_size + off, pages = pages_in(rem);
+    const float* row = k_head + (size_t)table[index0 + pages] * page_floats + (rem - pages * block_size) * HD;
+#pragma unroll
+    for (int u = 0; u < DPT; ++u) k_raw[u] = *(const pf_f32x4*)(row + 16 * u);
+  };
+  auto walk_tile = [&](int it, int kv0, int& index0, int buf, auto is_whole) {
+    constexpr bool WHOLE = decltype(is_whole)::value;
+    // the values of four positions of a page and one dim per lane and load
+    pf_f32x4 v_raw[OB][4];
+    const float* v_at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      int off = 16 * u + 4 * lg;
+      if constexpr (!WHOLE) {
+        const int p = kv0 + off;
+        off = (p + 3 >= lowest || p < keep) && p <= last_pos ? off : stand_in(it, kv0) & ~3;
       }
-      *(f32x4*)(v_s + d * VROW + c) = v;
+      const int rem = kv0 - index0 * block_size + off, pages = pages_in(rem);
+      v_at[u] = v_head + (size_t)table[index0 + pages] * page_floats + (rem - pages * block_size);
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int d = 0; d < OB; ++d) v_raw[d][u] = *(const pf_f32x4*)(v_at[u] + v_row[d]);
+    // ---- scores
+    pf_f32x4 s[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) s[b] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < DPT; ++u) {
+      float kf[4] = {k_raw[u][0], k_raw[u][1], k_raw[u][2], k_raw[u][3]};
+      transpose_lane_groups(kf);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int b = 0; b < RB; ++b) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t], qf[b][4 * u + t], s[b], 0, 0, 0);
+    }
+    // the next tile's keys
+    if (const int next = tile_begin(it + 1); next <= last_pos) {
+      if (it + 1 == kept_tiles) index0 = next / block_size;
+      else index0 += pages_in(kv0 - index0 * block_size + PF_TILE % block_size) + PF_TILE / block_size;
+      if (whole(next)) fetch_k(it + 1, next, index0, std::true_type{});
+      else fetch_k(it + 1, next, index0, std::false_type{});
+    }
+    // a lane holds token lr's scores of positions 16 wave + 4 lg .. + 3
+#pragma unroll
+    for (int b = 0; b < RB; ++b) *(pf_f32x4*)&sw_s[buf][16 * b + lr][16 * wave + 4 * lg] = s[b];
     __syncthreads();
-    float s[4][4];
+    // ---- softmax; weights go back where the scores were, as k 4 t + g of every 16 at 4 g + t (a row stays with its wave)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int b = 0; b < RB; ++b) {
+      const int row = 16 * b + ty;
+      float sc[4], best = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[i][j] = 0.f;
-    auto score_step = [&](int c) {
-      f32x4 qv[4], kv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) qv[i] = *(const f32x4*)(q_s + (4 * ty + i) * QROW + c);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) kv[j] = *(const f32x4*)(k_s + (tx + 16 * j) * QROW + c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < 4; ++j) sc[j] = sw_s[buf][row][tx + 16 * j] * scale;
+      const int qpos = pos0 + row;
+      if (softcap > 0.f || ex.rel) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          s[i][j] = fmaf(qv[i][0], kv[j][0], s[i][j]);
-          s[i][j] = fmaf(qv[i][1], kv[j][1], s[i][j]);
-          s[i][j] = fmaf(qv[i][2], kv[j][2], s[i][j]);
-          s[i][j] = fmaf(qv[i][3], kv[j][3], s[i][j]);
+          sc[j] = capped(sc[j], softcap);
+          if (ex.rel) sc[j] += distance_bias(ex, h, max(qpos - (kv0 + tx + 16 * j), 0));
         }
-    };
-    // A head of up to 64 dims is few enough steps for the compiler to unroll them all and hoist every load, which
-    // spills 96 registers at a width of 64: two steps at a time there (2,048 tokens of 14 heads 902 to 372 us; a
-    // width of 32 191 to 202). Wider heads keep the compiler's own choice (limited to two, a width of 128 ran 15 %
-    // slower).
-    if constexpr (DPT <= 4) {
-#pragma unroll 2
-      for (int c = 0; c < HD; c += 4) score_step(c);
-    } else {
-      for (int c = 0; c < HD; c += 4) score_step(c);
-    }
+      }
+      if constexpr (!WHOLE) {
+        const int first = first_visible(qpos, window);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int qpos = pos0 + 4 * ty + i;
-      const int first = first_visible(qpos, window);
-      float best = -INFINITY;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int p = kv0 + tx + 16 * j;
-        const bool sees = 4 * ty + i < rows && p <= qpos && (p >= first || p < keep);
-        s[i][j] = sees ? capped(s[i][j] * scale, softcap) : -INFINITY;
-        if (ex.rel && sees) s[i][j] += distance_bias(ex, h, qpos - p);
-        best = fmaxf(best, s[i][j]);
+        for (int j = 0; j < 4; ++j) {
+          const int p = kv0 + tx + 16 * j;
+          sc[j] = p <= qpos && (p >= first || p < keep) ? sc[j] : -INFINITY;
+        }
       }
 #pragma unroll
-      for (int off = 1; off < 16; off <<= 1) best = fmaxf(best, __shfl_xor(best, off));
-      const float m_new = fmaxf(m[i], best);
+      for (int j = 0; j < 4; ++j) best = fmaxf(best, sc[j]);
+      const float m_new = fmaxf(m[b], max16(best));
       float sum = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float w = s[i][j] > -INFINITY ? expf(s[i][j] - m_new) : 0.f;
-        p_s[(4 * ty + i) * VROW + tx + 16 * j] = w;
+        const float w = sc[j] > -INFINITY ? expf(sc[j] - m_new) : 0.f;
+        sw_s[buf][row][16 * j + 4 * (tx & 3) + (tx >> 2)] = w;
         sum += w;
       }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off);
-      const float rescale = m[i] > -INFINITY ? expf(m[i] - m_new) : 0.f;   // nothing seen so far: the sums are zero
-      l[i] = l[i] * rescale + sum;
-      m[i] = m_new;
-#pragma unroll
-      for (int j = 0; j < DPT; ++j) o[i][j] *= rescale;
+      sum = sum16(sum);
+      const float rescale = m[b] > -INFINITY ? expf(m[b] - m_new) : 0.f;   // nothing seen so far: the sums are zero
+      l[b] = l[b] * rescale + sum;
+      m[b] = m_new;
+      if (tx == 0) rescale_s[buf][row] = rescale;
     }
     __syncthreads();
-    auto output_step = [&](int c) {
-      f32x4 pv[4];
+    // ---- output: a lane holds token lr's dims 16 (wave + 4 d) + 4 lg .. + 3
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pv[i] = *(const f32x4*)(p_s + (4 * ty + i) * VROW + c);
+    for (int b = 0; b < RB; ++b) {
+      const float rescale = rescale_s[buf][16 * b + lr];
 #pragma unroll
-      for (int j = 0; j < DPT; ++j) {
-        const f32x4 vv = *(const f32x4*)(v_s + (tx + 16 * j) * VROW + c);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          o[i][j] = fmaf(pv[i][0], vv[0], o[i][j]);
-          o[i][j] = fmaf(pv[i][1], vv[1], o[i][j]);
-          o[i][j] = fmaf(pv[i][2], vv[2], o[i][j]);
-          o[i][j] = fmaf(pv[i][3], vv[3], o[i][j]);
-        }
-      }
-    };
-    if constexpr (DPT <= 4) {
-#pragma unroll 2
-      for (int c = 0; c < PF_TILE; c += 4) output_step(c);
-    } else {
-      for (int c = 0; c < PF_TILE; c += 4) output_step(c);
+      for (int d = 0; d < OB; ++d) o[d][b] *= rescale;
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      pf_f32x4 w[RB];
+#pragma unroll
+      for (int b = 0; b < RB; ++b) w[b] = *(const pf_f32x4*)&sw_s[buf][16 * b + lr][16 * u + 4 * lg];
+#pragma unroll
+      for (int d = 0; d < OB; ++d) {
+        float vf[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vf[e] = WHOLE || held(kv0 + 16 * u + 4 * lg + e) ? v_raw[d][u][e] : 0.f;
+        transpose_lane_groups(vf);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int b = 0; b < RB; ++b) o[d][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t], w[b][t], o[d][b], 0, 0, 0);
+      }
+    }
+  };
+  int index0 = tile_begin(0) / block_size;
+  fetch_k(0, tile_begin(0), index0, std::false_type{});
+  for (int it = 0;; ++it) {
+    const int kv0 = tile_begin(it);
+    if (kv0 > last_pos) break;
+    if (whole(kv0)) walk_tile(it, kv0, index0, it & 1, std::true_type{});
+    else walk_tile(it, kv0, index0, it & 1, std::false_type{});
   }
+  __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (4 * ty + i >= rows) continue;
-    float* dst = out + (size_t)(tok0 + 4 * ty + i) * heads * HD + (size_t)h * HD;
-    const float whole = l[i] + sink_term(ex, h, m[i]), gate = output_gate(ex, tok0 + 4 * ty + i, h);
+  for (int b = 0; b < RB; ++b)
+    if (tx == 0) rescale_s[0][16 * b + ty] = l[b] + sink_term(ex, h, m[b]);
+  __syncthreads();
 #pragma unroll
-    for (int j = 0; j < DPT; ++j) dst[tx + 16 * j] = o[i][j] / whole * gate;
+  for (int b = 0; b < RB; ++b) {
+    const int row = 16 * b + lr;
+    if (row >= rows) continue;
+    float* dst = out + (size_t)(tok0 + row) * heads * HD + (size_t)h * HD + 4 * lg;
+    const float sum = rescale_s[0][row], gate = output_gate(ex, tok0 + row, h);
+#pragma unroll
+    for (int d = 0; d < OB; ++d) {
+      if (wave + 4 * d >= DPT) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[16 * (wave + 4 * d) + r] = o[d][b][r] / sum * gate;
+    }
   }
 }
 
+// 16-token blocks of a workgroup for a step of `items` pairs (64 tokens, head): one while those are about one workgroup a CU,
+// two above, which read the keys and values half as often. us with one / two (and with four, slower at every size):
+// 140 tokens, 12 heads of 128 (48 items) 13.1 / 17.6; 333, 14 heads of 64 (84) 18.8 / 20.4; 400, 12 of 128 (96) 37.7 / 34.4;
+// 512 behind 1,000, 14 of 64 (112) 70.0 / 68.5; 4,096, 28 of 128 (1,792) 2,231 / 1,971.
+inline int prefill_f32_row_blocks(long long items) { return items <= 90 ? 1 : 2; }
+
 template <int DPT>
-int launch_prefill_f32(dim3 grid, hipStream_t s, const float* q, long long q_stride, const float* k_cache,
+int launch_prefill_f32(int num_tiles, hipStream_t s, const float* q, long long q_stride, const float* k_cache,
                        const float* v_cache, float* out, const int* tiles, const int* entry_start,
                        const int* entry_first_pos, const int* block_table, int table_width, int block_size, int heads,
-                       int kv_heads, float scale, int window, float softcap, int tile_tokens, AttnExtras ex) {
-  constexpr int HD = 16 * DPT;
-  constexpr int lds_bytes = (2 * PF_TILE * (HD + 4) + HD * (PF_TILE + 4) + PF_TILE * (PF_TILE + 4)) * 4;
-  static_assert(lds_bytes <= 160 * 1024, "a CU has 160 KB of LDS");
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_f32_kernel<DPT>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
-  attn_prefill_f32_kernel<DPT><<<grid, 256, lds_bytes, s>>>(q, q_stride, k_cache, v_cache, out, tiles, entry_start,
-                                                            entry_first_pos, block_table, table_width, block_size,
-                                                            heads, kv_heads, scale, window, softcap, tile_tokens, ex);
+                       int kv_heads, float scale, int window, float softcap, int tile_tokens, int row_blocks, AttnExtras ex) {
+  dim3 grid((unsigned)((long long)num_tiles * (tile_tokens / (16 * row_blocks))), heads);
+#define VK_PF(RBV)                                                                                                    \
+  attn_prefill_f32_kernel<DPT, RBV><<<grid, 256, 0, s>>>(q, q_stride, k_cache, v_cache, out, tiles, entry_start,       \
+                                                         entry_first_pos, block_table, table_width, block_size, heads, \
+                                                         kv_heads, scale, window, softcap, tile_tokens, ex)
+  if (row_blocks == 1) VK_PF(1); else VK_PF(2);
+#undef VK_PF
   return 0;
 }
 
@@ -674,12 +778,12 @@ extern "C" int vk_attn_prefill_f32_ext(const float* q, long long q_stride, const
   const long long groups = (long long)num_tiles * (tile_tokens / PF_TILE);
   if (groups > 0x7fffffffLL) return VK_UNSUPPORTED_SIZE;
   hipStream_t s = (hipStream_t)stream;
-  dim3 grid((unsigned)groups, heads);
+  const int row_blocks = prefill_f32_row_blocks(groups * heads);
   int status = 0;
 #define VK_PF(DPTV)                                                                                                  \
   case DPTV:                                                                                                         \
-    status = launch_prefill_f32<DPTV>(grid, s, q, q_stride, k_cache, v_cache, out, tiles, entry_start, entry_first_pos, \
-                                      block_table, table_width, block_size, heads, kv_heads, scale, window, softcap, tile_tokens, ex); \
+    status = launch_prefill_f32<DPTV>(num_tiles, s, q, q_stride, k_cache, v_cache, out, tiles, entry_start, entry_first_pos, \
+                                      block_table, table_width, block_size, heads, kv_heads, scale, window, softcap, tile_tokens, row_blocks, ex); \
     break;
   switch (hd / 16) { VK_PF(1) VK_PF(2) VK_PF(3) VK_PF(4) VK_PF(5) VK_PF(6) VK_PF(7) VK_PF(8) }
 #undef VK_PF

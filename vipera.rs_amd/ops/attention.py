@@ -165,7 +165,7 @@ def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, h
                                      chunks, dense=batch.all_single, join=join, softcap=softcap, extras=extras)
         return
     # the 32-bit run: single tokens on the kernel that splits their positions into chunks and shares the reads among
-    # the query heads of a key head, prompt portions on the kernel that walks the positions in LDS tiles; what
+    # the query heads of a key head, prompt portions on the matrix cores' 32-bit instructions; what
     # either does not take (odd widths, pages that are no multiple of 4) is left to the general kernel
     singles = bool(batch.num_decode_entries) and kernels.attn_decode_f32_supported(qkv, k_cache, head_dim)
     portions = bool(batch.num_prefill_tiles) and kernels.attn_prefill_f32_supported(qkv, k_cache, head_dim)

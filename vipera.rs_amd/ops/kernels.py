@@ -379,7 +379,7 @@ def attn_decode_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                *attn_extras_args(extras, heads, window, out.shape[0]), _stream()), "attn_decode_f32")
 
 
-ATTN_PREFILL_F32_MAX_HEAD_DIM = 128   # the K, V and weight tiles of a wider head do not fit a CU's LDS
+ATTN_PREFILL_F32_MAX_HEAD_DIM = 128   # a wave keeps its tokens' q and a tile's keys and values in registers
 
 
 def attn_prefill_f32_supported(q: torch.Tensor, k_cache: torch.Tensor, head_dim: int) -> bool:
@@ -395,7 +395,7 @@ def attn_prefill_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                      block_table: torch.Tensor, heads: int, kv_heads: int, head_dim: int, scale: float,
                      window: int, softcap: float = 0.0, extras=None) -> None:
     """32-bit attention of the entries' tiles listed in ``tiles`` (pairs: entry, first token within it; ``tile_tokens``
-    tokens a tile, a multiple of 64): 64 tokens of one head a workgroup, the positions in LDS tiles of 64."""
+    tokens a tile, a multiple of 64): 16 or 32 tokens of one head a workgroup, the positions in tiles of 64."""
     _dev(q, k_cache, v_cache, out, tiles, entry_start, entry_first_pos, block_table)
     _need(attn_prefill_f32_supported(q, k_cache, head_dim), "attn_prefill_f32: 32-bit operands, a head width that is a "
           "multiple of 16 up to 128, pages of a multiple of 4 positions")
