@@ -371,6 +371,36 @@ def test_gemm_generic_cut_over_workgroups_sums_in_the_same_order(m, n, k):
     assert torch.equal(mixed, again.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("m,n,k,form", [(17, 33, 260, 1), (9, 1150, 896, 1), (16, 130, 4864, 1), (128, 1155, 1020, 2), (25, 1530, 8964, 2),
+                                        (333, 1100, 1024, 3), (257, 1150, 516, 3), (64, 1536, 8964, 4), (260, 9731, 900, 5),
+                                        (1000, 3001, 1028, 5), (65, 17930, 1540, 6), (400, 17921, 1036, 7), (2050, 6001, 260, 7)])
+def test_each_form_of_the_32_bit_product_sums_in_the_same_order(m, n, k, form):
+    """At sizes that take each kernel and end inside its tiles, steps, ranges and slabs: bit for bit the rows that the weight
+    stream gives eight at a time, with a bias and accumulating; into and from rows of another stride, also where outputs do
+    not lie on 16 bytes."""
+    import ctypes
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.build import load_module
+    chosen = load_module("gemm_generic").vk_gemm_generic_form
+    chosen.argtypes, chosen.restype = [ctypes.c_int] * 3 + [ctypes.c_longlong], ctypes.c_int
+    assert chosen(m, n, k, kernels._gemm_generic_parts(m, n, k)) == form
+    g = torch.Generator(DEV).manual_seed(m + n + k)
+    randn = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    strided, w, bias, base = randn(m, k + 4), randn(n, k), randn(n), randn(m, n)
+    a = strided[:, :k]
+    whole, added, wide = torch.full((m, n), float("nan"), device=DEV), base.clone(), torch.zeros(m, n + 9, device=DEV)
+    kernels.gemm_generic(a, w, bias, whole)
+    kernels.gemm_generic(a, w, bias, added, accumulate=True)
+    kernels.gemm_generic(a.contiguous(), w, bias, wide[:, 4:n + 4])
+    assert torch.equal(wide[:, 4:n + 4], whole) and float(wide[:, :4].abs().max()) == 0.0 and float(wide[:, n + 4:].abs().max()) == 0.0
+    for start in (0, (m - 8) // 2, m - 8):
+        rows = slice(start, start + 8)
+        few, more = torch.empty(8, n, device=DEV), base[rows].clone()
+        kernels.gemm_generic(a[rows], w, bias, few)
+        kernels.gemm_generic(a[rows], w, bias, more, accumulate=True)
+        assert torch.equal(few, whole[rows]) and torch.equal(more, added[rows]), start
+
+
 @pytest.mark.parametrize("k", [4, 200, 260, 1100])
 @pytest.mark.parametrize("values", ["spread", "small operands", "small products", "small sums", "overflow", "special"])
 def test_the_matrix_instruction_is_two_fused_multiply_adds_for_all_values(values, k):

@@ -17,12 +17,15 @@
 //     never ends at -0);
 //   * the element is +0 + s0 + s1 + ... over its slabs in ascending order, then + bias, then,
 //     when accumulating, old + that.
-// Two kernels follow it. gemm_stream_kernel, for up to 8 rows of A in 32-bit operands, is a stream
-// of the weights: the product of a few tokens is bound by the bytes of W. gemm_matrix_kernel, for
-// everything else, runs on the matrix cores: v_mfma_f32_32x32x2_f32 computes each of its outputs as
+// Every kernel follows it. gemm_stream_kernel, for up to 8 rows of A in 32-bit operands, is a stream
+// of the weights: the product of a few tokens is bound by the bytes of W. Everything else runs on the
+// matrix cores, gemm_matrix_kernel for any types and rows, gemm_rows_kernel and gemm_slab_kernel for
+// 32-bit operands whose rows start on 16 bytes: v_mfma_f32_32x32x2_f32 computes each of its outputs as
 // fma(a[k + 1], w[k + 1], fma(a[k], w[k], c)), rounded after every product (compared with fmaf chains bit
 // for bit, values of all magnitudes, denormal, infinite and NaN ones included), so a chain of these
 // instructions over ascending k is the range's chain above.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -169,6 +172,381 @@ __global__ __launch_bounds__(256) void gemm_matrix_kernel(const TA* __restrict__
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same product where A, W and C are 32-bit and every row starts on 16 bytes: operands go from memory straight into LDS
+// (buffer loads with the lds modifier: no staging registers, no LDS stores) several steps ahead.  What the matrix instruction
+// wants of a lane, one k of two (or of four: v_mfma_f32_16x16x4_f32, four FMAs in ascending k on top of c, compared with fmaf
+// chains bit for bit), comes out of the 16 bytes it reads by lane exchanges (Fragment).  Two kernels:
+//   gemm_rows_kernel   a workgroup walks all of K
+//   gemm_slab_kernel   a workgroup owns one slab of K, wave w range w of it: the ranges' sums meet in LDS, and where K is one
+//                      slab that is the output, with no second launch; else parts and gemm_parts_finish_kernel
+// What bounds them: a wave alone on its SIMD reaches 70 % of the matrix cores' rate in the loop (every LDS read, load and lane
+// exchange between two products costs it some 5 to 30 cycles, and several waves a SIMD gain nothing beside them); below a round
+// of tiles, a range's chain: 128 instructions of 64 cycles, 3.4 us. Tiles of 128 x 128 are no faster at any size.
+// A row past the end is a copy of the last one and is not stored; a k past the end reads as zero (an offset past the view).
+constexpr unsigned NO_CHUNK = 0x80000000u;            // past the end of every view, and so are the steps behind it
+constexpr long long VIEW_BYTES = 0x7fffffffll;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_view(const float* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)VIEW_BYTES, 0x00020000);
+}
+
+// Until at most N of the wave's vector memory loads are in flight (they complete in the order of their issue).
+template <int N>
+__device__ __forceinline__ void loads_but() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
+
+// A block of BLOCK rows of an operand, 16 k: what a lane reads of it, and in which order the matrix instruction wants that.
+// 16 rows: one chunk of four k, lane group g = lane / 16 chunk g; instruction t wants k 4 t + g. 32 rows: chunks h and 2 + h
+// (h = lane / 32); instruction 4 c + t wants k 8 c + 2 t + h.
+template <int BLOCK>
+struct Fragment {
+  f32x4_t v[BLOCK / 16];
+  __device__ __forceinline__ static int row(int lane) { return lane & (BLOCK - 1); }
+  __device__ __forceinline__ static int chunk(int lane, int i) { return BLOCK == 16 ? lane >> 4 : 2 * i + (lane >> 5); }
+  __device__ __forceinline__ float operator()(int t) const { return v[t / 4][t % 4]; }
+  __device__ __forceinline__ void order() {
+    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int i = 0; i < BLOCK / 16; ++i) {
+      const u32x4_t r = __builtin_bit_cast(u32x4_t, v[i]);
+      u32x4_t to;
+      if constexpr (BLOCK == 16) {
+        const auto s01 = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);   // the first's odd groups and the second's even ones
+        const auto s23 = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
+        const auto s02 = __builtin_amdgcn_permlane32_swap(s01[0], s23[0], false, false);   // the first's upper half and the second's lower
+        const auto s13 = __builtin_amdgcn_permlane32_swap(s01[1], s23[1], false, false);
+        to = u32x4_t{s02[0], s13[0], s02[1], s13[1]};
+      } else {
+        const auto s01 = __builtin_amdgcn_permlane32_swap(r[0], r[1], false, false);
+        const auto s23 = __builtin_amdgcn_permlane32_swap(r[2], r[3], false, false);
+        to = u32x4_t{s01[0], s23[0], s01[1], s23[1]};
+      }
+      v[i] = __builtin_bit_cast(f32x4_t, to);
+    }
+  }
+};
+template <int BLOCK> struct Sums;
+template <> struct Sums<16> { typedef f32x4_t type; };
+template <> struct Sums<32> { typedef f32x16_t type; };
+__device__ __forceinline__ f32x4_t matrix_step(float w, float a, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, c, 0, 0, 0); }
+__device__ __forceinline__ f32x16_t matrix_step(float w, float a, f32x16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(w, a, c, 0, 0, 0); }
+// where a lane's four sums q of a block lie: row of A, first column
+template <int BLOCK> __device__ __forceinline__ int sum_column(int lane, int q) { return BLOCK == 16 ? 4 * (lane >> 4) : 8 * q + 4 * (lane >> 5); }
+
+// Four consecutive outputs of a row (as far as they exist): + bias, + old, in that order.  quads: every four lie on 16 bytes
+// and exist together.
+template <bool ACCUMULATE>
+__device__ __forceinline__ void store_outputs(float* __restrict__ C, const float* __restrict__ bias, f32x4_t v, int m, int n, int M,
+                                              int N, long long ldc, bool quads) {
+  if (m >= M || n >= N) return;
+  float* dst = C + (size_t)m * ldc + n;
+  if (quads) {
+    if (bias) v += *(const f32x4_t*)(bias + n);
+    if (ACCUMULATE) v = *(const f32x4_t*)dst + v;
+    *(f32x4_t*)dst = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (n + e >= N) break;
+    float x = v[e];
+    if (bias) x += bias[n + e];
+    dst[e] = ACCUMULATE ? dst[e] + x : x;
+  }
+}
+
+// Hints for the order of what was written since the last such line: LDS reads and loads go out one by one between the products,
+// or two lane exchanges at a time.  All reads and loads ahead of the products made every wave wait for the others' at the LDS and
+// address units: 112 TFLOP/s at 2,048 x 4,096 x 4,096.
+template <int PRODUCTS, int READS, int LOADS>
+__device__ __forceinline__ void between_products() {
+  if constexpr (READS + LOADS == 0) {
+#pragma unroll
+    for (int i = 0; i < PRODUCTS; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one matrix instruction
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // two others
+    }
+  } else {
+    constexpr int MOST = READS > LOADS ? READS : LOADS;
+    constexpr int EACH = MOST <= PRODUCTS ? 1 : (MOST + PRODUCTS - 1) / PRODUCTS;
+#pragma unroll
+    for (int i = 0; i < PRODUCTS; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (i * EACH < READS) __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);   // LDS reads
+      if (i * EACH < LOADS) __builtin_amdgcn_sched_group_barrier(0x020, EACH, 0);   // loads
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// A workgroup's outputs over all of K: WM x WN waves, each TM x TN blocks of 32 x 32; steps of 32 k through STAGES stages, the
+// loads of STAGES - 1 steps in flight.  LDS rows are 128 bytes, unpadded (a load instruction fills 1 KB: 8 rows, lane L the 16
+// bytes at 16 L); chunk c of row r sits in slot c ^ (r % 8), so that 16 rows read the same chunk from different banks.  A wave
+// reads the operands of a half step while it multiplies the first half of the other and orders them during its second half.
+// SLABS: K has several.
+template <int TM, int TN, int WM, int WN, int STAGES, bool SLABS, bool ACCUMULATE>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                 const float* __restrict__ bias, float* __restrict__ C, int M,
+                                                                 int N, int K, long long lda, long long ldc, bool quads) {
+  typedef __attribute__((address_space(3))) void* lds_at;
+  typedef Fragment<32> Frag;
+  constexpr int WAVES = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, STEP = 32, ROW = STEP * 4;
+  constexpr int A_LOADS = BM / 8 / WAVES, W_LOADS = BN / 8 / WAVES, LOADS = A_LOADS + W_LOADS, STAGE = (BM + BN) * ROW;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide among the waves' loads");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN, lr = Frag::row(lane);
+  const int m_tiles = (M + BM - 1) / BM;
+  const int m0 = blockIdx.x % m_tiles * BM, n0 = blockIdx.x / m_tiles * BN;
+  const __amdgpu_buffer_rsrc_t a_view = row_view(A + (size_t)m0 * lda), w_view = row_view(W + (size_t)n0 * K);
+  const int ld_row = lane >> 3, ld_chunk = (lane & 7) ^ (lane >> 3);
+  unsigned a_off[A_LOADS], w_off[W_LOADS];
+#pragma unroll
+  for (int i = 0; i < A_LOADS; ++i)
+    a_off[i] = (unsigned)(min(m0 + (wave * A_LOADS + i) * 8 + ld_row, M - 1) - m0) * (unsigned)(lda * 4) + ld_chunk * 16;
+#pragma unroll
+  for (int i = 0; i < W_LOADS; ++i)
+    w_off[i] = (unsigned)(min(n0 + (wave * W_LOADS + i) * 8 + ld_row, N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
+  auto issue = [&](int stage, int step) {
+    unsigned char* to_a = lds + stage * STAGE + wave * A_LOADS * 1024;
+    unsigned char* to_w = lds + stage * STAGE + BM * ROW + wave * W_LOADS * 1024;
+    const unsigned kb = step * STEP + ld_chunk * 4 < K ? (unsigned)step * ROW : NO_CHUNK;
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_view, (lds_at)(to_a + i * 1024), 16, (int)(a_off[i] + kb), 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < W_LOADS; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_view, (lds_at)(to_w + i * 1024), 16, (int)(w_off[i] + kb), 0, 0, 0);
+  };
+  unsigned at_a[2], at_w[2];   // the lane's two chunks of the first half step; bit 6 of the place: the second half
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned slot = (unsigned)((Frag::chunk(lane, i) ^ (lr & 7)) * 16);
+    at_a[i] = (unsigned)((wm * TM * 32 + lr) * ROW) + slot;
+    at_w[i] = (unsigned)((BM + wn * TN * 32 + lr) * ROW) + slot;
+  }
+  auto read = [&](int stage, int half, Frag (&fa)[TM], Frag (&fw)[TN]) {
+    const unsigned char* base = lds + stage * STAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) fw[t].v[i] = *(const f32x4_t*)(base + (at_w[i] ^ (half * 64)) + t * 32 * ROW);
+#pragma unroll
+      for (int t = 0; t < TM; ++t) fa[t].v[i] = *(const f32x4_t*)(base + (at_a[i] ^ (half * 64)) + t * 32 * ROW);
+    }
+  };
+  f32x16_t acc[TN][TM], slab[TN][TM], total[TN][TM];
+#pragma unroll
+  for (int n = 0; n < TN; ++n)
+#pragma unroll
+    for (int m = 0; m < TM; ++m) acc[n][m] = slab[n][m] = total[n][m] = 0.f;
+  auto multiply = [&](const Frag (&fa)[TM], const Frag (&fw)[TN], int half) {
+#pragma unroll
+    for (int t = 4 * half; t < 4 * half + 4; ++t)
+#pragma unroll
+      for (int n = 0; n < TN; ++n)
+#pragma unroll
+        for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n](t), fa[m](t), acc[n][m]);
+  };
+  auto order = [&](Frag (&fa)[TM], Frag (&fw)[TN]) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t) fw[t].order();
+#pragma unroll
+    for (int t = 0; t < TM; ++t) fa[t].order();
+  };
+  const int steps = (K + STEP - 1) / STEP;
+  Frag fa0[TM], fw0[TN], fa1[TM], fw1[TN];
+#pragma unroll
+  for (int i = 0; i < STAGES; ++i) issue(i, i);        // a step past the end loads zeros
+  loads_but<(STAGES - 1) * LOADS>();
+  __syncthreads();
+  read(0, 0, fa0, fw0);
+  order(fa0, fw0);
+  int stage = 0, s = 0;
+  for (int slabs_done = 0; s < steps;) {
+    // a range's steps in a loop of their own, which touches no sum but acc
+    const int range_end = min(steps, s + RANGE_K / STEP);
+    for (; s < range_end; ++s) {
+      const int next = stage + 1 == STAGES ? 0 : stage + 1;
+      read(stage, 1, fa1, fw1);
+      multiply(fa0, fw0, 0);
+      between_products<4 * TM * TN, 2 * (TM + TN), 0>();
+      order(fa1, fw1);
+      multiply(fa0, fw0, 1);
+      between_products<4 * TM * TN, 0, 0>();
+      loads_but<(STAGES - 2) * LOADS>();
+      __syncthreads();                                 // step s + 1 is there, and nobody reads this step's stage any more
+      read(next, 0, fa0, fw0);
+      issue(stage, s + STAGES);
+      multiply(fa1, fw1, 0);
+      between_products<4 * TM * TN, 2 * (TM + TN), LOADS>();
+      order(fa0, fw0);
+      multiply(fa1, fw1, 1);
+      between_products<4 * TM * TN, 0, 0>();
+      stage = next;
+    }
+    const bool slab_ends = ++slabs_done % SLAB_RANGES == 0 || s == steps;
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        slab[n][m] += acc[n][m];
+        acc[n][m] = 0.f;
+        if constexpr (SLABS) {
+          if (slab_ends) {
+            total[n][m] += slab[n][m];
+            slab[n][m] = 0.f;
+          }
+        }
+      }
+  }
+  loads_but<0>();                                      // no load may write LDS that the next workgroup has
+  auto store = [&](bool in_quads) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        const f32x16_t& sum = SLABS ? total[n][m] : slab[n][m];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          store_outputs<ACCUMULATE>(C, bias, f32x4_t{sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]},
+                                    m0 + (wm * TM + m) * 32 + lr, n0 + (wn * TN + n) * 32 + sum_column<32>(lane, q), M, N, ldc, in_quads);
+      }
+  };
+  if (quads) store(true);
+  else store(false);
+}
+
+// A workgroup's BLOCK TM x BLOCK TN outputs over one slab (blockIdx.y), a range a wave.  A wave has stages of its own, of 16 k,
+// and waits for no other before the ranges' sums meet.  LDS rows are 64 bytes (a load instruction: 16 rows); chunk c of row r
+// sits in slot c ^ (r / 4 % 4): a chunk of 16 rows lies in all banks.
+template <int BLOCK, int TM, int TN, int STAGES, bool PARTS, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                        const float* __restrict__ bias, float* __restrict__ C,
+                                                        float* __restrict__ parts, int M, int N, int K, long long lda,
+                                                        long long ldc, bool quads) {
+  typedef __attribute__((address_space(3))) void* lds_at;
+  typedef Fragment<BLOCK> Frag;
+  typedef typename Sums<BLOCK>::type Sum;
+  constexpr int STEP = 16, HALVES = BLOCK / 16, A_GROUPS = TM * HALVES, GROUPS = (TM + TN) * HALVES, STAGE = GROUPS * 1024;
+  constexpr int QUADS = BLOCK == 16 ? 1 : 4, SUM_QUADS = TM * TN * QUADS;
+  static_assert(SUM_QUADS * 1024 <= STAGES * STAGE, "the ranges' sums reuse the stages");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m_tiles = (M + BLOCK * TM - 1) / (BLOCK * TM);
+  const int m0 = blockIdx.x % m_tiles * (BLOCK * TM), n0 = blockIdx.x / m_tiles * (BLOCK * TN);
+  const int k_begin = blockIdx.y * SLAB_K + wave * RANGE_K, k_end = min(K, k_begin + RANGE_K);
+  unsigned char* mine = lds + wave * (STAGES * STAGE);
+  Sum acc[TN][TM];
+#pragma unroll
+  for (int n = 0; n < TN; ++n)
+#pragma unroll
+    for (int m = 0; m < TM; ++m) acc[n][m] = 0.f;
+  if (k_begin < k_end) {
+    const __amdgpu_buffer_rsrc_t a_view = row_view(A + (size_t)m0 * lda + k_begin), w_view = row_view(W + (size_t)n0 * K + k_begin);
+    const int ld_row = lane >> 2, ld_chunk = (lane & 3) ^ (lane >> 4), left = k_end - k_begin;
+    unsigned off[GROUPS];
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g)
+      off[g] = (g < A_GROUPS ? (unsigned)(min(m0 + 16 * g + ld_row, M - 1) - m0) * (unsigned)(lda * 4)
+                             : (unsigned)(min(n0 + 16 * (g - A_GROUPS) + ld_row, N - 1) - n0) * (unsigned)(K * 4)) + ld_chunk * 16;
+    auto issue = [&](int stage, int step) {
+      unsigned char* to = mine + stage * STAGE;
+      const unsigned kb = step * STEP + ld_chunk * 4 < left ? (unsigned)(step * STEP * 4) : NO_CHUNK;
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(g < A_GROUPS ? a_view : w_view, (lds_at)(to + g * 1024), 16, (int)(off[g] + kb), 0, 0, 0);
+    };
+    const int lr = Frag::row(lane);
+    unsigned at[HALVES];
+#pragma unroll
+    for (int i = 0; i < HALVES; ++i) at[i] = (unsigned)(lr * 64 + ((Frag::chunk(lane, i) ^ (lr >> 2 & 3)) * 16));
+    auto read = [&](int stage, Frag (&fa)[TM], Frag (&fw)[TN]) {
+      const unsigned char* base = mine + stage * STAGE;
+#pragma unroll
+      for (int i = 0; i < HALVES; ++i) {
+#pragma unroll
+        for (int t = 0; t < TN; ++t) fw[t].v[i] = *(const f32x4_t*)(base + (TM + t) * HALVES * 1024 + at[i]);
+#pragma unroll
+        for (int t = 0; t < TM; ++t) fa[t].v[i] = *(const f32x4_t*)(base + t * HALVES * 1024 + at[i]);
+      }
+    };
+    constexpr int INSTRUCTIONS = 4 * HALVES, FIRST = INSTRUCTIONS / 2;
+    auto multiply = [&](const Frag (&fa)[TM], const Frag (&fw)[TN], auto from, auto to) {
+#pragma unroll
+      for (int t = decltype(from)::value; t < decltype(to)::value; ++t)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n](t), fa[m](t), acc[n][m]);
+    };
+    auto order = [&](Frag (&fa)[TM], Frag (&fw)[TN]) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) fw[t].order();
+#pragma unroll
+      for (int t = 0; t < TM; ++t) fa[t].order();
+    };
+    const int steps = (left + STEP - 1) / STEP;
+    Frag fa0[TM], fw0[TN], fa1[TM], fw1[TN];
+#pragma unroll
+    for (int i = 0; i < STAGES; ++i) issue(i, i);      // a step past the end loads zeros
+    loads_but<(STAGES - 1) * GROUPS>();
+    asm volatile("" ::: "memory");
+    read(0, fa0, fw0);
+    order(fa0, fw0);
+    int stage = 0;
+    // fa, fw: this step's operands, in order; the next one's are read while their first half is multiplied
+    auto step = [&](int s, Frag (&fa)[TM], Frag (&fw)[TN], Frag (&na)[TM], Frag (&nw)[TN]) {
+      const int next = stage + 1 == STAGES ? 0 : stage + 1;
+      __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this step's operands are in registers, its stage is free
+      asm volatile("" ::: "memory");
+      issue(stage, s + STAGES);
+      loads_but<(STAGES - 1) * GROUPS>();              // step s + 1 is there
+      asm volatile("" ::: "memory");
+      read(next, na, nw);
+      multiply(fa, fw, std::integral_constant<int, 0>{}, std::integral_constant<int, FIRST>{});
+      between_products<FIRST * TM * TN, GROUPS, 0>();
+      order(na, nw);
+      multiply(fa, fw, std::integral_constant<int, FIRST>{}, std::integral_constant<int, INSTRUCTIONS>{});
+      between_products<FIRST * TM * TN, 0, 0>();
+      stage = next;
+    };
+    int s = 0;
+    for (; s + 2 <= steps; s += 2) {
+      step(s, fa0, fw0, fa1, fw1);
+      step(s + 1, fa1, fw1, fa0, fw0);
+    }
+    if (s < steps) step(s, fa0, fw0, fa1, fw1);
+    loads_but<0>();
+  }
+  __syncthreads();                                     // every wave is done with its stages
+  float* sums = (float*)lds;                           // [wave][four sums][lane][4]
+#pragma unroll
+  for (int n = 0; n < TN; ++n)
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q)
+        *(f32x4_t*)(sums + (((size_t)wave * SUM_QUADS + (n * TM + m) * QUADS + q) * 64 + lane) * 4) =
+            f32x4_t{acc[n][m][4 * q], acc[n][m][4 * q + 1], acc[n][m][4 * q + 2], acc[n][m][4 * q + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int b0 = 0; b0 < SUM_QUADS; b0 += 4) {
+    const int b = b0 + wave;
+    if (b >= SUM_QUADS) break;
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < SLAB_RANGES; ++w) v += *(const f32x4_t*)(sums + (((size_t)w * SUM_QUADS + b) * 64 + lane) * 4);
+    const int q = b % QUADS, m = b / QUADS % TM, n = b / QUADS / TM;
+    const int row = m0 + BLOCK * m + Frag::row(lane), column = n0 + BLOCK * n + sum_column<BLOCK>(lane, q);
+    if constexpr (PARTS) store_outputs<false>(parts + (size_t)blockIdx.y * M * N, nullptr, v, row, column, M, N, N, N % 4 == 0);
+    else store_outputs<ACCUMULATE>(C, bias, v, row, column, M, N, ldc, quads);
+  }
+}
+
 // C = the sum of the parts (+ bias) (+ old C): units of `per_slab` to a slab (4: ranges, 1: slabs), slabs in order.
 // Four consecutive columns a thread where N allows, so that the parts are read 16 bytes at a time.
 template <typename TC, bool ACCUMULATE, int COLUMNS>
@@ -280,6 +658,130 @@ int launch(const void* A_, const void* W_, const float* bias, void* C_, int M, i
   const int count = (K + units * RANGE_K - 1) / (units * RANGE_K), per_slab = SLAB_RANGES / units;
   return accumulate ? launch_finish<TC, true>(parts, bias, C, M, N, ldc, count, per_slab, s)
                     : launch_finish<TC, false>(parts, bias, C, M, N, ldc, count, per_slab, s);
+}
+
+// Whether four outputs at a time lie on 16 bytes, in C and in the bias.
+inline bool stores_quads(const float* C, const float* bias, int N, long long ldc) {
+  return N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0 && ((uintptr_t)bias & 15) == 0;
+}
+
+template <int TM, int TN, int WM, int WN, int STAGES>
+int launch_rows(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, long long lda, long long ldc,
+                int accumulate, hipStream_t s) {
+  constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, lds_bytes = STAGES * (BM + BN) * 128;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipSuccess;
+    for (const void* f : {(const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, false, false>, (const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, false, true>,
+                          (const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, true, false>, (const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, true, true>})
+      if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  const unsigned tiles = (unsigned)(((M + BM - 1) / BM) * ((N + BN - 1) / BN));
+  const bool quads = stores_quads(C, bias, N, ldc);
+#define VK_ROWS(SLABS, ACC) gemm_rows_kernel<TM, TN, WM, WN, STAGES, SLABS, ACC><<<tiles, 64 * WM * WN, lds_bytes, s>>>(A, W, bias, C, M, N, K, lda, ldc, quads)
+  if (K <= SLAB_K) { if (accumulate) VK_ROWS(false, true); else VK_ROWS(false, false); }
+  else { if (accumulate) VK_ROWS(true, true); else VK_ROWS(true, false); }
+#undef VK_ROWS
+  VK_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int BLOCK, int TM, int TN, int STAGES>
+int launch_slabs(const float* A, const float* W, const float* bias, float* C, float* parts, int M, int N, int K, long long lda,
+                 long long ldc, int accumulate, hipStream_t s) {
+  constexpr int BM = BLOCK * TM, BN = BLOCK * TN, lds_bytes = 4 * STAGES * (BM + BN) * 64;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipSuccess;
+    for (const void* f : {(const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, false>, (const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, true>,
+                          (const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, true, false>})
+      if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  const int slabs = (K + SLAB_K - 1) / SLAB_K;
+  const bool quads = stores_quads(C, bias, N, ldc);
+  const dim3 grid((unsigned)(((M + BM - 1) / BM) * ((N + BN - 1) / BN)), slabs);
+  if (slabs > 1) gemm_slab_kernel<BLOCK, TM, TN, STAGES, true, false><<<grid, 256, lds_bytes, s>>>(A, W, nullptr, nullptr, parts, M, N, K, lda, 0, false);
+  else if (accumulate) gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, true><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
+  else gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, false><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
+  VK_LAUNCH_CHECK();
+  if (slabs == 1) return 0;
+  return accumulate ? launch_finish<float, true>(parts, bias, C, M, N, ldc, slabs, 1, s)
+                    : launch_finish<float, false>(parts, bias, C, M, N, ldc, slabs, 1, s);
+}
+
+// Which kernel an all-32-bit product of aligned rows takes.  Both cut M x N into tiles, one a workgroup; the last round of
+// tiles over the 256 CUs is as long as a full one while the rounds are few.  Times in us as measured (weights from memory), of
+// a round and beside the rounds:
+//   slab, 16 x 32 outputs   2.9 + 3.9 a round (tiles x slabs)    9 x 1,152 x 896: 6.7 (14.1 as 64 x 64 tiles cut over workgroups)
+//         32 x 32           3.2 + 6.4                            128 x 1,152 x 896: 9.4 (15.0)
+//         48 x 32           4.5 + 9.3                            333 x 1,152 x 896: 14.2 (20.3)
+//         64 x 64           3 + 22                               64 x 1,536 x 8,960: 32.7 (40.3)
+//     and, with several slabs, 5 for adding the parts and their way through memory
+//   rows, 64 x 64           7.5 + 0.0193 K a round               2,048 x 2,560 x 2,048: 210 (232)
+//         32 x 128          8 + 0.0207 K                         65 x 17,920 x 1,536: 68.9 (92.9)
+//         64 x 128          8 + 0.0365 K                         333 x 9,728 x 896: 72.8 (81.7); 2,048 x 37,888 x 3,584: 4,757 (5,358)
+// Over 112 sizes from 9 to 2,048 rows the choice takes 0.80 of the time of the 64 x 64 tiles (geometric mean), and 1.07 of it at
+// worst (512 x 1,536 x 1,536).  Those tiles keep a product where their cut of K is estimated to be faster (200 x 1,536 x 8,960: 87.8
+// against 93.7), any other type, and rows off 16 bytes.
+enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128 };
+
+inline double rounds(long long tiles) { return tiles <= 3 * 256 ? (double)((tiles + 255) / 256) : tiles / 256.0 + 0.35; }
+
+// The same estimate for the 64 x 64 tiles, as they are cut (matrix_units).
+inline double estimate_matrix(int M, int N, int K, int units) {
+  const double tiles = (double)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
+  if (units == 0) return 7 + fmax(1.0, tiles / 256 + 0.3) * K * 0.0205;
+  const int cuts = (K + units * RANGE_K - 1) / (units * RANGE_K);
+  const double parts = (double)cuts * M * N * 8 / 6e6, per_cu = tiles * cuts / 256;
+  return units == 1 ? 9.5 + fmax(5.0, (per_cu + 0.35) * 5.2) + parts : 9 + fmax(19.5, (per_cu + 0.15) * 18.5) + parts;
+}
+
+Direct direct_plan(int M, int N, int K, long long part_floats) {
+  struct Form { Direct form; int rows, columns; double beside, round; };
+  constexpr Form forms[] = {{SLAB_16_32, 16, 32, 2.9, 3.9}, {SLAB_32_32, 32, 32, 3.2, 6.4}, {SLAB_48_32, 48, 32, 4.5, 9.3},
+                            {SLAB_64_64, 64, 64, 3.0, 22.0}, {ROWS_64_64, 64, 64, 7.5, 0.0193}, {ROWS_32_128, 32, 128, 8.0, 0.0207},
+                            {ROWS_64_128, 64, 128, 8.0, 0.0365}};
+  const long long slabs = (K + SLAB_K - 1) / SLAB_K;
+  const bool parts_fit = slabs == 1 || slabs * M * N <= part_floats;
+  double best = 0.97 * estimate_matrix(M, N, K, part_floats > 0 ? matrix_units(M, N, K) : 0);
+  Direct chosen = NOT_DIRECT;
+  for (const Form& f : forms) {
+    const bool slab = f.form <= SLAB_64_64;
+    const long long tiles = (long long)((M + f.rows - 1) / f.rows) * ((N + f.columns - 1) / f.columns);
+    if ((slab && !parts_fit) || tiles > 0xffffffffll / 256) continue;
+    double us;
+    if (slab) us = f.beside + f.round * rounds(tiles * slabs) + (slabs == 1 ? 0.0 : 5.0 + (double)slabs * M * N * 8 / 6e6);
+    else us = f.beside + f.round * K * rounds(tiles) * (K > SLAB_K && tiles <= 256 ? 1.07 : 1.0);
+    if (us < best) best = us, chosen = f.form;
+  }
+  return chosen;
+}
+
+int launch_direct(Direct form, const float* A, const float* W, const float* bias, float* C, float* parts, int M, int N, int K,
+                  long long lda, long long ldc, int accumulate, hipStream_t s) {
+  switch (form) {
+    case SLAB_16_32: return launch_slabs<16, 1, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_32_32: return launch_slabs<32, 1, 1, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_48_32: return launch_slabs<16, 3, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_64_64: return launch_slabs<32, 2, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_64_64: return launch_rows<1, 1, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_32_128: return launch_rows<1, 1, 1, 4, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_64_128: return launch_rows<1, 2, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case NOT_DIRECT: break;
+  }
+  return VK_BAD_ARGUMENT;
+}
+
+// Rows of 32-bit operands that start on 16 bytes, and tiles whose bytes lie within a view.
+constexpr long long DIRECT_MAX_ROW = 4000000;
+static_assert(128 * DIRECT_MAX_ROW * 4 < VIEW_BYTES, "a tile has up to 128 rows");
+inline bool direct_takes(const void* A, int a_dtype, const void* W, int w_dtype, int c_dtype, int K, long long lda) {
+  return a_dtype == DT_F32 && w_dtype == DT_F32 && c_dtype == DT_F32 && K % 4 == 0 && lda % 4 == 0 && lda <= DIRECT_MAX_ROW &&
+         K <= DIRECT_MAX_ROW && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -480,7 +982,11 @@ extern "C" int vk_gemm_stream(const float* A, const float* W, const float* bias,
 
 namespace {
 int dispatch(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C, int c_dtype, int M, int N,
-             int K, long long lda, long long ldc, int accumulate, int units, float* parts, hipStream_t s) {
+             int K, long long lda, long long ldc, int accumulate, float* parts, long long part_floats, hipStream_t s) {
+  if (direct_takes(A, a_dtype, W, w_dtype, c_dtype, K, lda))
+    if (const Direct form = direct_plan(M, N, K, part_floats); form != NOT_DIRECT)
+      return launch_direct(form, (const float*)A, (const float*)W, bias, (float*)C, parts, M, N, K, lda, ldc, accumulate, s);
+  const int units = parts ? matrix_units(M, N, K) : 0;
   switch (a_dtype * 4 + w_dtype * 2 + c_dtype) {
     case 0: return launch<float, float, float>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
     case 1: return launch<float, float, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, accumulate, units, parts, s);
@@ -495,14 +1001,19 @@ int dispatch(const void* A, int a_dtype, const void* W, int w_dtype, const float
 }
 }  // namespace
 
-// K whole in every workgroup, which needs no workspace. dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.
+// The kernel that an all-32-bit product of aligned rows takes with a workspace of part_floats (direct_plan); 0: the 64 x 64 tiles.
+extern "C" int vk_gemm_generic_form(int M, int N, int K, long long part_floats) {
+  return M <= 0 || N <= 0 || K <= 0 || (K & 3) || K > DIRECT_MAX_ROW ? 0 : (int)direct_plan(M, N, K, part_floats);
+}
+
+// Without a workspace: no sums go through memory. dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.
 extern "C" int vk_gemm_generic(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
                                int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
                                void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldc < N) return VK_BAD_ARGUMENT;
   if ((M + TILE - 1) / TILE > 65535) return VK_UNSUPPORTED_SIZE;
-  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, 0, nullptr, (hipStream_t)stream);
+  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, nullptr, 0, (hipStream_t)stream);
 }
 
 // Floats of workspace that vk_gemm_generic_split wants for an M x N product over K (0: it is not split).
@@ -521,6 +1032,6 @@ extern "C" int vk_gemm_generic_split(const void* A, int a_dtype, const void* W, 
   if (K <= 0 || lda < K || ldc < N) return VK_BAD_ARGUMENT;
   if ((M + TILE - 1) / TILE > 65535) return VK_UNSUPPORTED_SIZE;
   if (vk_gemm_generic_workspace(M, N, K) > part_floats || ((uintptr_t)parts & 15)) return VK_BAD_ARGUMENT;
-  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, matrix_units(M, N, K), parts,
+  return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, parts, part_floats,
                   (hipStream_t)stream);
 }
