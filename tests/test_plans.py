@@ -191,3 +191,27 @@ def test_past_128_tokens_small_tiles_carry_out_a_128x128_plan_unless_its_tiles_f
     assert all(plan(700, 5120, k, gated=True) == (15, 1) for k in (1024, 8192, 12288)) and plan(277, 10880, 4096, gated=True) == (15, 1)
     assert plan(277, 10976, 4096, gated=True) == (9, 1) and plan(270, 13312, 8192, gated=True) == (9, 1)
     assert plan(512, 2048, 2040)[0] == 0           # no whole steps of 64
+
+
+def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
+    """Chunks as long as one another are few enough to run at once, never leave a position out and never outnumber what was
+    allowed for."""
+    import random
+    from vipera_rs_amd.ops.attention import cut_prompt_tiles
+    reaches = lambda *portions: [first + min(off + 128, n) for first, n in portions for off in range(0, n, 128)]
+    assert cut_prompt_tiles(reaches((1194, 512), (2389, 456), (3584, 399)), 12, 128, 0, 256) == (16, 4)
+    assert cut_prompt_tiles(reaches((1900, 100)), 14, 64, 0, 256) == (4, 8)
+    assert cut_prompt_tiles(reaches((0, 1000), (0, 834)), 16, 128, 0, 256) is None
+    assert cut_prompt_tiles(reaches((0, 2048)), 28, 128, 0, 256) is None                   # more items than CUs
+    assert cut_prompt_tiles(reaches((3000, 200)), 12, 96, 0, 256) is None and cut_prompt_tiles([], 12, 128, 0, 256) is None
+    assert cut_prompt_tiles(reaches((8000, 200)), 12, 128, 100, 256) is None               # a window of 100: short walks
+    rng = random.Random(3)
+    for _ in range(300):
+        tiles = sorted(rng.randrange(1, rng.choice([200, 2000, 30000])) for _ in range(rng.randrange(1, 20)))
+        heads, window = rng.choice([1, 8, 14, 28]), rng.choice([0, 0, 512, -512])
+        plan = cut_prompt_tiles(tiles, heads, rng.choice([64, 128, 256]), window, 256)
+        if plan is not None:
+            chunk, most = plan
+            assert chunk >= 4 and chunk * most * 64 >= max(tiles)
+            if not window:
+                assert heads * sum(-(-t // (64 * chunk)) for t in tiles) <= 2 * 256

@@ -71,6 +71,8 @@ class StepBatch:
     sum_decode_kv_len: int = 0     # positions that the single-token entries see, added up (a captured step: assumed)
     max_tile_reach: int = 0        # positions that the last token of the longest prompt tile sees (no window counted)
     sum_tile_reach: int = 0        # the same, added over the prompt tiles
+    tile_reaches: Sequence[int] = ()                  # the same, tile by tile
+    cuts_tiles_by_length: bool = False   # whether attention may cut prompt tiles by their single lengths (set by the model)
 
 
 @dataclass
@@ -90,6 +92,7 @@ class PackedStep:
     max_tile_reach: int = 0
     sum_tile_reach: int = 0
     sum_decode_kv_len: int = 0
+    tile_reaches: Sequence[int] = ()
 
     def flat(self) -> np.ndarray:
         return np.concatenate([s.reshape(-1) for s in self.sections]) if self.sections else np.zeros(0, np.int32)
@@ -195,7 +198,8 @@ def pack_entries(entries: Sequence[StepEntry], cache, vocab_size: int, min_table
                 sources]
     sections += tables
     return PackedStep(sections, widths, T, E, len(rows), counts_all, [int(v) for v in first], [int(v) for v in slots],
-                      int(kv_len.max()), max_decode_kv, max(tile_reach, default=0), sum(tile_reach), sum_decode_kv)
+                      int(kv_len.max()), max_decode_kv, max(tile_reach, default=0), sum(tile_reach), sum_decode_kv,
+                      tile_reach)
 
 
 def batch_from_buffer(packed: PackedStep, dev: torch.Tensor) -> StepBatch:
@@ -218,6 +222,7 @@ def batch_from_buffer(packed: PackedStep, dev: torch.Tensor) -> StepBatch:
         num_prefill_tiles=packed.sections[8].size // 2, num_decode_entries=packed.sections[9].size,
         max_decode_kv_len=packed.max_decode_kv_len, max_tile_reach=packed.max_tile_reach,
         sum_tile_reach=packed.sum_tile_reach, sum_decode_kv_len=packed.sum_decode_kv_len,
+        tile_reaches=packed.tile_reaches,
     )
 
 

@@ -126,6 +126,8 @@ class DecoderModel:
         if self.rejoin is None and any(entry.rejoins for entry in self.schedule):
             raise InvalidArgumentError("the run order has entries that rejoin the embedding's output, but no part that does it")
         self.vocab_size = self.head.vocab
+        self.routes = any(spec.ffn is not None and getattr(part_class("ffn", spec.ffn.kind), "routes", False)
+                          for spec in config.layer_specs())
         self.loaded = False
 
     def tensor_specs(self) -> List[TensorSpec]:
@@ -159,6 +161,7 @@ class DecoderModel:
         # must launch it too, or the graph would replay with what an earlier run left
         batch.shared.clear()
         batch.launch_plans.clear()
+        batch.cuts_tiles_by_length = not self.routes
         x = self.embedding.embed(batch)
         tokens = x.shape[0]
         incoming = None

@@ -107,7 +107,8 @@ PROMPT_CHUNK_MIN_TILES = 8   # a chunk of a prompt tile's positions is at least 
 
 def chunks_prompt_tiles(num_tiles: int, heads: int, longest: int, total: int, cus: int):
     """``(chunk_tiles, max_chunks)`` if the prompt kernel should cut every tile's positions into chunks of
-    ``chunk_tiles`` steps of 64, a workgroup each, and merge them with a second kernel, else None.  For a model of
+    ``chunk_tiles`` steps of 64, a workgroup each, and merge them with a second kernel, else None, by the tiles' longest and
+    total length (:func:`cut_prompt_tiles` knows them all).  For a model of
     few heads, whose (tile, head) items are fewer than the CUs (12 heads and four portions of 512 tokens are 192
     items) and as long as their prompts, so that the one deepest in its prompt sets the time.  The chunks are sized
     to give every CU about two workgroups (sizes for one to six measured the same); a tile's partial results (128
@@ -131,6 +132,55 @@ def chunks_prompt_tiles(num_tiles: int, heads: int, longest: int, total: int, cu
     return chunk_tiles, -(-longest_steps // chunk_tiles)
 
 
+# us as measured by padded head width: of a step of 64 positions and beside the steps, for a workgroup that takes a tile alone
+# (halved between sixteen waves where the width allows), for chunks of which a CU has one at the most, and two
+PROMPT_COSTS = {64: ((0.9, 5.0), (0.96, 10.7, 0.015), (0.95, 17.0, 0.015)), 128: ((1.35, 5.5), (2.1, 7.0, 0.025), (2.5, 4.0, 0.025)),
+                256: ((3.1, 6.0), (2.84, 13.6, 0.027), None)}
+
+
+def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int):
+    """:func:`chunks_prompt_tiles` where the tiles' lengths are known one by one (``reaches``: the positions that the last token
+    of each sees, no window counted): the chunk length whose workgroups, counted tile by tile, are at most one a CU, or 1.7 a
+    CU (two, less what the XCDs differ by: one more runs behind all others), and that takes the least time by this estimate, if
+    that is less than nine tenths of what the tiles take uncut.  us a layer, uncut (halved) against cut, the merge included: four tiles of 16
+    heads of 128 that end at 1,664 to 2,048 positions 47.7 / 30.3; twelve of 12 heads that end at 1,322 to 3,983 87.0 / 52.2;
+    the sixteen of one prompt of 2,048, 12 heads, 47.4 / 39.8; two of 14 heads of 64 at 2,000 32.7 / 15.0; and left uncut: eight
+    and seven tiles of 1,000 and 834 tokens, 16 heads, 29.2 / 31.6; a prompt of 2,048 at 28 heads 63.2 / 69.5."""
+    items = len(reaches) * heads
+    costs = PROMPT_COSTS.get(head_dim)
+    if items <= 0 or items > cus or costs is None:
+        return None
+    seen = [min(r, abs(window) + 128) if window else r for r in reaches]
+    steps = [(r + 63) // 64 for r in seen]
+    longest = max(steps)
+    (alone, alone_beside), one, two = costs
+    best, chosen = 0.9 * (alone * longest + alone_beside), None
+    for chunk in range(4, longest):
+        counts = [-(-s // chunk) for s in steps]
+        groups = heads * sum(counts)
+        cost = one if groups <= cus else two if groups <= 1.7 * cus else None
+        if cost is None:
+            continue
+        us = cost[0] * chunk + cost[1] + cost[2] * groups
+        if us < best:
+            best, chosen = us, chunk
+    return None if chosen is None else (chosen, -(-((max(reaches) + 63) // 64) // chosen))
+
+
+def _prompt_plan(batch, k_cache, heads: int, kv_heads: int, head_dim: int, window: int, cus: int):
+    """``(chunk_tiles and max_chunks, or None; whether tiles are halved)``, once for a step's layers of one geometry."""
+    chunked = None
+    if kernels.attn_bf16_prefill_loads_directly(k_cache, kv_heads, head_dim):
+        # A router's closest calls turn on the last bits of what comes before it, so a model that has one keeps the cuts, and
+        # with them the order of its attention's sums, that the tiles' total gives.
+        if getattr(batch, "cuts_tiles_by_length", False):
+            chunked = cut_prompt_tiles(batch.tile_reaches, heads, head_dim, window, cus)
+        else:
+            chunked = chunks_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach, batch.sum_tile_reach, cus)
+    return chunked, chunked is None and halves_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach,
+                                                            batch.sum_tile_reach, cus)
+
+
 def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, head_dim, scale, window,
                     softcap: float = 0.0, extras: Optional[AttentionExtras] = None) -> None:
     """``window`` > 0: a token sees the last that many positions; < 0: the positions of its own block of ``-window``
@@ -140,12 +190,10 @@ def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, h
         extras = None
     if kernels.attn_bf16_supported(qkv, k_cache, head_dim):
         if batch.num_prefill_tiles:
-            cus = kernels.compute_units(qkv.device)
-            chunked = None
-            if kernels.attn_bf16_prefill_loads_directly(k_cache, kv_heads, head_dim):
-                chunked = chunks_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach, batch.sum_tile_reach, cus)
-            split = chunked is None and halves_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach,
-                                                            batch.sum_tile_reach, cus)
+            key = ("prompt tiles", heads, kv_heads, head_dim, window, k_cache.shape[2])
+            if key not in batch.shared:
+                batch.shared[key] = _prompt_plan(batch, k_cache, heads, kv_heads, head_dim, window, kernels.compute_units(qkv.device))
+            chunked, split = batch.shared[key]
             kernels.attn_bf16_prefill(qkv, k_cache, v_cache, out, batch.prefill_tiles, batch.entry_start,
                                       batch.entry_first_pos, table, heads, kv_heads, head_dim, scale, window, split,
                                       *(chunked or (0, 0)), softcap=softcap, extras=extras)
