@@ -28,8 +28,8 @@ def _dt(tensor: torch.Tensor, what: str) -> int:
     return _DT[tensor.dtype]
 
 
-def _ptr(tensor: Optional[torch.Tensor]):
-    return _p(tensor.data_ptr()) if tensor is not None else _p(0)
+def _ptr(tensor: Optional[torch.Tensor]) -> Optional[int]:
+    return tensor.data_ptr() if tensor is not None else None
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -40,13 +40,18 @@ def _stream():
     """The current stream's handle.  Through torch's raw accessors where it has them: ``torch.cuda.current_stream()``
     builds a Python object on every call, which was a quarter of the host's time for a step launched kernel by kernel."""
     if _raw_stream is not None and _raw_device is not None:
-        return _p(_raw_stream(_raw_device()))
-    return _p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(_raw_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _need(cond: bool, text: str) -> None:
     if not cond:
         raise InvalidArgumentError(text)
+
+
+def _refuse(text: str) -> None:
+    """Where the text is put together from the operands, which costs more than the check it belongs to."""
+    raise InvalidArgumentError(text)
 
 
 def _dev(*tensors: Optional[torch.Tensor]) -> None:
@@ -79,17 +84,17 @@ def _cache_ok(k_cache, v_cache, kv_heads: int, head_dim: int, dtype) -> bool:
             and v_cache.is_contiguous())
 
 
-_signatures_done = set()
+_functions: dict = {}
 
 
 def _fn(module: str, name: str, argtypes, key: str = None, restype=ctypes.c_int):
-    library = load_module(module)
-    fn = getattr(library, name)
-    key = key or name
-    if key not in _signatures_done:
+    """The launcher ``name`` of ``module`` with its signature set (kept under ``key``, where modules share names)."""
+    fn = _functions.get(key or name)
+    if fn is None:
+        fn = getattr(load_module(module), name)
         fn.argtypes = argtypes
         fn.restype = restype
-        _signatures_done.add(key)
+        _functions[key or name] = fn
     return fn
 
 
@@ -237,7 +242,8 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     _need(a.dim() == 2 and w.dim() == 2 and out.dim() == 2, "gemm: operands must be matrices")
     m, k = a.shape
     n = w.shape[0]
-    _need(w.shape[1] == k and out.shape == (m, n), f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
+    if not (w.shape[1] == k and out.shape == (m, n)):
+        _refuse(f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
     _need(a.stride(1) == 1 and out.stride(1) == 1 and w.is_contiguous(), "gemm: inner strides must be 1")
     _need(a.stride(0) >= k or m == 1, "gemm: a's row stride")
     _need(out.stride(0) >= n or m == 1, "gemm: out's row stride")
@@ -505,14 +511,16 @@ def gemm_bf16_supported(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> 
 
 
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
-              accumulate: bool = False, skinny_limit: int = 64, skinny_shape: int = 0) -> None:
-    """``out (+)= a @ w.T + bias`` on the matrix cores: bfloat16 products, 32-bit sums."""
+              accumulate: bool = False, skinny_limit: int = 64, skinny_shape: int = 0, supported: bool = False) -> None:
+    """``out (+)= a @ w.T + bias`` on the matrix cores: bfloat16 products, 32-bit sums.  ``supported``: the caller has
+    just found :func:`gemm_bf16_supported` true of the operands."""
     _dev(a, w, bias, out)
     _need(a.dim() == 2 and w.dim() == 2 and out.dim() == 2, "gemm: operands must be matrices")
     m, k = a.shape
     n = w.shape[0]
-    _need(w.shape[1] == k and out.shape == (m, n), f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
-    _need(gemm_bf16_supported(a, w, out), "gemm_bf16: operands must be bfloat16, K a multiple of 8, rows 16-byte aligned")
+    if not (w.shape[1] == k and out.shape == (m, n)):
+        _refuse(f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
+    _need(supported or gemm_bf16_supported(a, w, out), "gemm_bf16: operands must be bfloat16, K a multiple of 8, rows 16-byte aligned")
     if bias is not None:
         _need(bias.dtype == torch.float32 and bias.numel() == n and bias.is_contiguous(), "gemm: bias must be float32 [n]")
     if accumulate:
@@ -893,16 +901,18 @@ def _split_k_workspace(device: torch.device, floats: int, kind: str) -> torch.Te
 
 
 def gemm_bf16_mid(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
-                  accumulate: bool = False, ranges: int = 1, rows_per_wave: int = 2) -> None:
+                  accumulate: bool = False, ranges: int = 1, rows_per_wave: int = 2, supported: bool = False) -> None:
     """``out (+)= a @ w.T + bias`` for at most 128 rows of ``a``: activations shared through LDS, weights
-    streamed; ``ranges`` > 1 splits K over workgroups and adds the ranges' partial sums in a second kernel."""
+    streamed; ``ranges`` > 1 splits K over workgroups and adds the ranges' partial sums in a second kernel.  ``supported``
+    as in :func:`gemm_bf16`."""
     _dev(a, w, bias, out)
     _need(a.dim() == 2 and w.dim() == 2 and out.dim() == 2, "gemm: operands must be matrices")
     m, k = a.shape
     n = w.shape[0]
     _need(m <= 128, "gemm_bf16_mid takes at most 128 rows")
-    _need(w.shape[1] == k and out.shape == (m, n), f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
-    _need(gemm_bf16_supported(a, w, out), "gemm_bf16: operands must be bfloat16, K a multiple of 8, rows 16-byte aligned")
+    if not (w.shape[1] == k and out.shape == (m, n)):
+        _refuse(f"gemm: shapes {tuple(a.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)}")
+    _need(supported or gemm_bf16_supported(a, w, out), "gemm_bf16: operands must be bfloat16, K a multiple of 8, rows 16-byte aligned")
     _need((rows_per_wave in (1, 2) or 108 <= rows_per_wave <= 116) and ranges >= 1,
           "gemm_bf16_mid: rows_per_wave is 1 or 2 (or 108 to 116: one tile with 8 to 16 rows), ranges at least 1")
     if bias is not None:
@@ -939,7 +949,8 @@ def gemm_bf16_gated_act(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kin
     _dev(a, w, out)
     m, k = a.shape
     n = w.shape[0]
-    _need(kind in ("silu", "gelu_tanh"), f"gemm_gated: activation {kind!r}")
+    if not (kind in ("silu", "gelu_tanh")):
+        _refuse(f"gemm_gated: activation {kind!r}")
     _need(w.shape[1] == k and out.shape == (m, n // 2) and n % 32 == 0, "gemm_gated: shapes")
     _need(gemm_bf16_supported(a, w, out) and out.dtype == torch.bfloat16, "gemm_gated: operands must be bfloat16")
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
@@ -969,7 +980,8 @@ def gemm_bf16_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_pe
 
 # ----------------------------------------------------------------------------------------------
 def _f32(tensor: torch.Tensor, what: str) -> None:
-    _need(tensor.dtype == torch.float32 and tensor.is_contiguous(), f"{what} must be contiguous float32")
+    if not (tensor.dtype == torch.float32 and tensor.is_contiguous()):
+        _refuse(f"{what} must be contiguous float32")
 
 
 def _i32(*tensors: torch.Tensor) -> None:
@@ -986,7 +998,8 @@ def dyt(x: torch.Tensor, alpha: torch.Tensor, weight: torch.Tensor, bias: torch.
     _need(x.dim() == 2 and x.dtype == torch.float32 and x.is_contiguous(), "dyt: x must be contiguous float32 [tokens, width]")
     _need(alpha.dtype == torch.float32 and alpha.numel() == 1, "dyt: alpha must be one float32")
     for name, t in (("weight", weight), ("bias", bias)):
-        _need(t.dtype == torch.float32 and t.numel() == width and t.is_contiguous(), f"dyt: {name} must be float32 [width]")
+        if not (t.dtype == torch.float32 and t.numel() == width and t.is_contiguous()):
+            _refuse(f"dyt: {name} must be float32 [width]")
     count = x.shape[0] if rows is None else rows.numel()
     if rows is not None:
         _i32(rows)
@@ -1005,7 +1018,8 @@ def dyt_pair(x: torch.Tensor, first, second, out1: torch.Tensor, out2: torch.Ten
         _dev(x, alpha, weight, bias)
         _need(alpha.dtype == torch.float32 and alpha.numel() == 1, "dyt_pair: alpha must be one float32")
         for name, t in (("weight", weight), ("bias", bias)):
-            _need(t.dtype == torch.float32 and t.numel() == width and t.is_contiguous(), f"dyt_pair: {name} must be float32 [width]")
+            if not (t.dtype == torch.float32 and t.numel() == width and t.is_contiguous()):
+                _refuse(f"dyt_pair: {name} must be float32 [width]")
     _dev(out1, out2)
     _need(out1.shape == x.shape and out2.shape == x.shape and out1.is_contiguous() and out2.is_contiguous()
           and out1.dtype == out2.dtype, "dyt_pair: outputs")
@@ -1086,7 +1100,8 @@ def delta_prepare(proj: torch.Tensor, conv: torch.Tensor, state: torch.Tensor, c
     _f32(beta, "delta_prepare: beta")
     if a_col >= 0:
         for name, t in (("a_log", a_log), ("dt_bias", dt_bias)):
-            _need(t is not None and t.dtype == torch.float32 and t.numel() == heads, f"delta_prepare: {name}")
+            if not (t is not None and t.dtype == torch.float32 and t.numel() == heads):
+                _refuse(f"delta_prepare: {name}")
         _need(decay is not None and decay.shape == (tokens, heads), "delta_prepare: decay")
         _f32(decay, "delta_prepare: decay")
     fn = _fn("recurrent", "vk_delta_prepare_strided",
@@ -1104,7 +1119,8 @@ def channel_decay(raw: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
     _dev(raw, a_log, dt_bias, out)
     tokens = raw.shape[0]
     for name, t in (("raw", raw), ("out", out)):
-        _need(t.dtype == torch.float32 and t.shape == (tokens, heads * dim) and t.stride(1) == 1, f"channel_decay: {name}")
+        if not (t.dtype == torch.float32 and t.shape == (tokens, heads * dim) and t.stride(1) == 1):
+            _refuse(f"channel_decay: {name}")
     _need(a_log.dtype == torch.float32 and a_log.numel() == heads and a_log.is_contiguous(), "channel_decay: a_log")
     _need(dt_bias.dtype == torch.float32 and dt_bias.numel() == heads * dim and dt_bias.is_contiguous(),
           "channel_decay: dt_bias")
@@ -1197,9 +1213,11 @@ def wkv_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wraw: torch.Tens
     _dev(r, k, v, wraw, w0, bonus, state, entry_start, entry_first, slots, out)
     tokens, width = out.shape[0], heads * dim
     for name, t in (("r", r), ("k", k), ("v", v), ("wraw", wraw)):
-        _need(t.dtype == torch.float32 and t.shape == (tokens, width) and t.stride(1) == 1, f"wkv_rule: {name}")
+        if not (t.dtype == torch.float32 and t.shape == (tokens, width) and t.stride(1) == 1):
+            _refuse(f"wkv_rule: {name}")
     for name, t in (("w0", w0), ("bonus", bonus)):
-        _need(t.dtype == torch.float32 and t.numel() == width and t.is_contiguous(), f"wkv_rule: {name}")
+        if not (t.dtype == torch.float32 and t.numel() == width and t.is_contiguous()):
+            _refuse(f"wkv_rule: {name}")
     _f32(out, "wkv_rule: out")
     _need(out.shape == (tokens, width), "wkv_rule: out shape")
     _need(state.dim() == 2 and state.dtype == torch.float32 and state.is_contiguous()
@@ -1381,7 +1399,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     _dev(logits, ids, weights, offsets, order, tiles, num_tiles)
     tokens, experts = logits.shape
     _f32s(logits, "moe_route: logits")      # rows may lie further apart than they are long (a view of some columns)
-    _need(1 <= top <= min(experts, 64), f"moe_route: top {top} of {experts} experts")
+    if not (1 <= top <= min(experts, 64)):
+        _refuse(f"moe_route: top {top} of {experts} experts")
     _i32(ids, offsets, order, tiles, num_tiles)
     _f32(weights, "moe_route: weights")
     _need(ids.numel() == tokens * top and weights.numel() == tokens * top and order.numel() == tokens * top
@@ -1455,7 +1474,8 @@ def moe_experts(h: torch.Tensor, w_gate: Optional[torch.Tensor], w_up: torch.Ten
 # --- norms behind a sublayer, sums of two streams, activations ------------------------------------------
 def _f32s(tensor: torch.Tensor, what: str) -> None:
     """32-bit with unit inner stride; rows may lie further apart than they are long (a view of some columns)."""
-    _need(tensor.dtype == torch.float32 and tensor.stride(-1) == 1, f"{what} must be float32 with a unit inner stride")
+    if not (tensor.dtype == torch.float32 and tensor.stride(-1) == 1):
+        _refuse(f"{what} must be float32 with a unit inner stride")
 
 
 def rmsnorm_add(y: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.Tensor,
@@ -1514,7 +1534,8 @@ def token_side(x: torch.Tensor, e: torch.Tensor, gate: torch.Tensor, proj: torch
           and proj.is_contiguous(), "token_side: shapes")
     for t, what in ((norm, "norm"), (next_weight, "next_weight"), (next_bias, "next_bias")):
         if t is not None:
-            _need(t.dtype == torch.float32 and t.numel() == width and t.is_contiguous(), f"token_side: {what}")
+            if not (t.dtype == torch.float32 and t.numel() == width and t.is_contiguous()):
+                _refuse(f"token_side: {what}")
     if next_out is not None:
         _need(next_weight is not None and next_kind in ("rms", "layer") and next_out.shape == x.shape
               and next_out.is_contiguous() and next_out.dtype == torch.bfloat16, "token_side: next_out")
@@ -1541,7 +1562,8 @@ ACTIVATIONS = {"none": 0, "relu2": 1, "silu": 2, "gelu_tanh": 3, "sigmoid": 4}
 def activation(x: torch.Tensor, kind: str, out: torch.Tensor, mul: Optional[torch.Tensor] = None) -> None:
     """``out = act(x) (* mul)`` elementwise; all three may be row-strided views of either dtype.  ``kind``: none (a change of type), relu2 (the square of relu), silu, gelu_tanh, sigmoid."""
     _dev(x, out, mul)
-    _need(kind in ACTIVATIONS, f"activation: kind {kind!r}; known: {', '.join(ACTIVATIONS)}")
+    if not (kind in ACTIVATIONS):
+        _refuse(f"activation: kind {kind!r}; known: {', '.join(ACTIVATIONS)}")
     rows, width = out.shape
     _need(x.shape == out.shape and x.stride(1) == 1 and out.stride(1) == 1, "activation: shapes")
     if mul is not None:
@@ -1893,7 +1915,8 @@ def head_finish(attn: torch.Tensor, out: torch.Tensor, heads: int, vdim: int, wi
     _need(attn.shape == (tokens, heads * maps * width) and attn.is_contiguous() and maps in (1, 2), "head_finish: attn shape")
     _need(out.shape == (tokens, heads * vdim) and out.is_contiguous() and out.dtype == attn.dtype, "head_finish: out shape")
     _need(vdim <= width and vdim <= 256, "head_finish: widths")
-    _need(gate_kind in _GATE_ACTS, f"head_finish: gate {gate_kind!r}")
+    if not (gate_kind in _GATE_ACTS):
+        _refuse(f"head_finish: gate {gate_kind!r}")
     ldg = 0
     if gate is not None:
         _need(gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == tokens and gate.stride(1) == 1
@@ -1927,7 +1950,8 @@ def row_gate_add(y: torch.Tensor, gate: torch.Tensor, gate_kind: str, out: torch
     _need(y.dtype == torch.float32 and out.dtype == torch.float32 and y.shape == out.shape and y.dim() == 2
           and y.is_contiguous() and out.is_contiguous(), "row_gate_add: two contiguous 32-bit matrices of one shape")
     _need(gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == y.shape[0], "row_gate_add: gate")
-    _need(gate_kind in _GATE_ACTS, f"row_gate_add: gate {gate_kind!r}")
+    if not (gate_kind in _GATE_ACTS):
+        _refuse(f"row_gate_add: gate {gate_kind!r}")
     fn = _fn("heads", "vk_row_gate_add", [_p, _p, _ll, _i, _p, _i, _i, _i, _p])
     _status(fn(_ptr(y), _ptr(gate), gate.stride(0), _GATE_ACTS[gate_kind], _ptr(out), y.shape[0], y.shape[1],
                1 if accumulate else 0, _stream()), "row_gate_add")
@@ -1960,7 +1984,8 @@ def streams_step(src: torch.Tensor, streams: int, y: Optional[torch.Tensor], mix
         _need(mix is not None and share is not None, "streams_step: an output joins through mix and share")
         for t, shape, what in ((y, (tokens, width), "y"), (mix, (streams, streams), "mix"), (share, (streams,), "share")):
             _f32(t, "streams_step: " + what)
-            _need(t.shape == shape, f"streams_step: {what} shape")
+            if not (t.shape == shape):
+                _refuse(f"streams_step: {what} shape")
     if dst is not None:
         _f32(dst, "streams_step: dst")
         _need(y is not None and rows is None and dst.shape == (tokens, streams, width), "streams_step: dst")
@@ -1976,7 +2001,8 @@ def streams_step(src: torch.Tensor, streams: int, y: Optional[torch.Tensor], mix
         _need(out.shape == (count, width) and out.is_contiguous(), "streams_step: out shape")
     for t, what in ((weight, "weight"), (bias, "bias")):
         if t is not None:
-            _need(t.dtype == torch.float32 and t.numel() == width and t.is_contiguous(), f"streams_step: {what}")
+            if not (t.dtype == torch.float32 and t.numel() == width and t.is_contiguous()):
+                _refuse(f"streams_step: {what}")
     _need(norm in STREAM_NORMS, "streams_step: norm")
     held = src.dim() == 3
     fn = _fn("streams", "vk_streams_step", [_p, _ll, _ll, _p, _p, _p, _p, _p, _i, _p, _p, _f, _p, _p, _i, _i, _i, _i, _p])
@@ -2020,7 +2046,8 @@ def state_space(x: torch.Tensor, b: torch.Tensor, c: torch.Tensor, dt: torch.Ten
     _need(out.shape == (tokens, heads * vdim) and out.is_contiguous(), "state_space: out")
     for t, what in ((dt_bias, "dt_bias"), (a_log, "a_log"), (skip, "skip")):
         _f32(t, "state_space: " + what)
-        _need(t.numel() == heads, f"state_space: {what} is one number per head")
+        if not (t.numel() == heads):
+            _refuse(f"state_space: {what} is one number per head")
     if states > STATE_SPACE_MAX_STATES:
         raise UnsupportedError(f"state_space: {states} states are above the kernel's limit of {STATE_SPACE_MAX_STATES}")
     _need(state.dim() == 2 and state.stride(1) == 1 and state.stride(0) % 4 == 0 and state.data_ptr() % 16 == 0

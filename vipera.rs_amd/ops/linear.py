@@ -96,10 +96,10 @@ def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
         m, k = a.shape
         n = w.shape[0]
         if not streams_weights(m, n, k) or streams_in_wave_order(m, n, k):
-            kernels.gemm_bf16(a, w, bias, out, accumulate)
+            kernels.gemm_bf16(a, w, bias, out, accumulate, supported=True)
         else:
             ranges, rows_per_wave = mid_plan(m, n, k)
-            kernels.gemm_bf16_mid(a, w, bias, out, accumulate, ranges, rows_per_wave)
+            kernels.gemm_bf16_mid(a, w, bias, out, accumulate, ranges, rows_per_wave, supported=True)
     else:
         kernels.gemm_generic(a, w, bias, out, accumulate)
     return out
