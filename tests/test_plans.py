@@ -215,3 +215,18 @@ def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
             assert chunk >= 4 and chunk * most * 64 >= max(tiles)
             if not window:
                 assert heads * sum(-(-t // (64 * chunk)) for t in tiles) <= 2 * 256
+
+
+def test_few_requests_of_short_contexts_take_short_chunks():
+    from vipera_rs_amd.ops.attention import short_decode_plan
+    assert short_decode_plan(512, 1, 2, 1, 64) == (64, 8, True) and short_decode_plan(513, 1, 2, 1, 64) == (32, 17, False)
+    assert short_decode_plan(256, 8, 4, 1, 128) == (32, 8, True) and short_decode_plan(512, 8, 4, 1, 128) == (32, 16, False)
+    assert short_decode_plan(1024, 8, 4, 1, 128) == (64, 16, False) and short_decode_plan(2048, 8, 4, 1, 128) is None
+    assert short_decode_plan(4096, 1, 4, 1, 128) == (64, 64, False) and short_decode_plan(4097, 1, 4, 1, 128) is None
+    assert short_decode_plan(512, 80, 2, 1, 64) is None and short_decode_plan(300, 1, 2, 1, 256) is None
+    for length in range(1, 4500, 7):
+        for entries, kv, dim in ((1, 2, 64), (3, 4, 128), (40, 2, 64)):
+            plan = short_decode_plan(length, entries, kv, 1, dim)
+            if plan is not None:
+                chunk, chunks, join = plan
+                assert chunk % 32 == 0 and chunk * chunks >= length and (chunks <= 8 if join else chunks <= 64)

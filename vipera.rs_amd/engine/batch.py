@@ -72,7 +72,9 @@ class StepBatch:
     max_tile_reach: int = 0        # positions that the last token of the longest prompt tile sees (no window counted)
     sum_tile_reach: int = 0        # the same, added over the prompt tiles
     tile_reaches: Sequence[int] = ()                  # the same, tile by tile
-    cuts_tiles_by_length: bool = False   # whether attention may cut prompt tiles by their single lengths (set by the model)
+    # whether attention may cut positions into chunks of any length (set by the model): a router's closest calls turn on the last
+    # bits of what comes before it, so a model that has one keeps the chunks, and with them the order of the sums, that it had
+    free_sum_order: bool = False
 
 
 @dataclass

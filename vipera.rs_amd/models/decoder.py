@@ -161,7 +161,7 @@ class DecoderModel:
         # must launch it too, or the graph would replay with what an earlier run left
         batch.shared.clear()
         batch.launch_plans.clear()
-        batch.cuts_tiles_by_length = not self.routes
+        batch.free_sum_order = not self.routes
         x = self.embedding.embed(batch)
         tokens = x.shape[0]
         incoming = None

@@ -89,6 +89,32 @@ def joins_decode_chunks(chunks: int, num_entries: int, kv_heads: int, head_block
     return chunks <= kernels.ATTN_DECODE_JOINED_CHUNKS and pairs >= 0.8 * cus
 
 
+def short_decode_plan(max_kv_len: int, num_entries: int, kv_heads: int, head_blocks: int, head_dim: int):
+    """``(chunk, chunks, join)`` for few requests of short contexts at head widths of 64 and 128, else None: a wave walks its
+    chunk 32 positions at a time, each step a round trip to memory, so that while the waves are few they should be as short
+    as the merge allows.
+
+    * Up to eight chunks of 64 positions (a head of 64) or 32 (of 128): one workgroup a (request, key head), a wave a
+      chunk, which merges them itself.
+    * Chunks of 32 while a request has at most 32 of them and the waves are at most 512; chunks of 64 up to 64 and 512.
+
+    us a layer in a captured step, against chunks of 128 and a merge: one request of 512 positions, two key heads of 64
+    5.9 / 8.4, eight 6.8 / 9.2; of 128 6.8 / 9.0, eight with four key heads 8.1 / 9.7; one of 1,000 7.9 / 9.9, of 2,000
+    8.5 / 10.1, of 4,096 (four key heads) 10.0 / 10.3; past 512 waves even (eight requests of 1,000, four key heads: 10.5 to
+    10.8 with chunks of 32, 64 and 128)."""
+    if head_dim not in (64, 128):
+        return None
+    pairs = num_entries * kv_heads * head_blocks
+    own = 4096 // head_dim
+    if max_kv_len <= kernels.ATTN_DECODE_JOINED_CHUNKS * own and pairs <= 128:
+        return own, max(1, -(-max_kv_len // own)), True
+    for chunk, most in ((32, 32), (64, 64)):
+        chunks = -(-max_kv_len // chunk)
+        if chunks <= most and pairs * chunks <= 512:
+            return chunk, chunks, False
+    return None
+
+
 def halves_prompt_tiles(num_tiles: int, heads: int, longest: int, total: int, cus: int) -> bool:
     """Whether the prompt kernel should give every (tile, head) a workgroup of sixteen waves that halve the
     tile's positions between them: when a CU would otherwise be left with a single workgroup of eight for most of
@@ -171,9 +197,7 @@ def _prompt_plan(batch, k_cache, heads: int, kv_heads: int, head_dim: int, windo
     """``(chunk_tiles and max_chunks, or None; whether tiles are halved)``, once for a step's layers of one geometry."""
     chunked = None
     if kernels.attn_bf16_prefill_loads_directly(k_cache, kv_heads, head_dim):
-        # A router's closest calls turn on the last bits of what comes before it, so a model that has one keeps the cuts, and
-        # with them the order of its attention's sums, that the tiles' total gives.
-        if getattr(batch, "cuts_tiles_by_length", False):
+        if getattr(batch, "free_sum_order", False):
             chunked = cut_prompt_tiles(batch.tile_reaches, heads, head_dim, window, cus)
         else:
             chunked = chunks_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach, batch.sum_tile_reach, cus)
@@ -201,10 +225,15 @@ def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, h
             group = heads // kv_heads
             visible = batch.max_decode_kv_len
             head_blocks = (group + 15) // 16
-            chunk, chunks = decode_chunking(visible, batch.num_decode_entries, kv_heads, head_blocks,
-                                            batch.sum_decode_kv_len)
-            join = joins_decode_chunks(chunks, batch.num_decode_entries, kv_heads, head_blocks,
-                                       kernels.compute_units(qkv.device), head_dim)
+            plan = None
+            if getattr(batch, "free_sum_order", False):
+                plan = short_decode_plan(visible, batch.num_decode_entries, kv_heads, head_blocks, head_dim)
+            if plan is None:
+                chunk, chunks = decode_chunking(visible, batch.num_decode_entries, kv_heads, head_blocks,
+                                                batch.sum_decode_kv_len)
+                plan = chunk, chunks, joins_decode_chunks(chunks, batch.num_decode_entries, kv_heads, head_blocks,
+                                                          kernels.compute_units(qkv.device), head_dim)
+            chunk, chunks, join = plan
             batch.launch_plans.append((chunk, chunks, join))
             partial = None if join else torch.empty(batch.num_decode_entries * heads * chunks * (head_dim + 2),
                                                     dtype=torch.float32, device=qkv.device)
