@@ -98,6 +98,54 @@ def test_the_small_tilings_give_the_bits_of_the_large_one(tiling, ranges):
         kernels.gemm_bf16_force_tiling(-1)
 
 
+@pytest.mark.parametrize("tiling", [16, 17, 18, 19, 20])
+@pytest.mark.parametrize("ranges", [1, 3])
+def test_the_tiles_of_whole_products_give_the_bits_of_the_128x128_ones(tiling, ranges):
+    """192x64, 128x128, 192x128 and 192x192 tiles with two to four LDS stages: tails of a row and a column, runs shorter than
+    the stages and runs that end in every stage, several rounds of tiles, plain, added to a residual and gated."""
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.linear import interleave_gate_up
+    try:
+        for m, n, k in [(129, 33, 64), (193, 65, 128), (385, 193, 192), (192, 192, 256), (191, 300, 320), (577, 129, 1088), (140, 520, 2048)]:
+            g = torch.Generator().manual_seed(m + n + k)
+            a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+            w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+            bias, base = torch.randn(n, generator=g).to(DEV), torch.randn(m, n, generator=g).to(DEV)
+            fused = interleave_gate_up(w[:n // 16 * 16], w[:n // 16 * 16].flip(0).contiguous())
+            got = []
+            for now in (9, tiling):
+                kernels.gemm_bf16_force_tiling(now, ranges)
+                outs = [torch.full((m, n), 7.0, device=DEV), torch.full((m, n), 7.0, dtype=torch.bfloat16, device=DEV), base.clone(),
+                        torch.full((m, n // 16 * 16), 7.0, dtype=torch.bfloat16, device=DEV)]
+                kernels.gemm_bf16(a, w, bias, outs[0])
+                kernels.gemm_bf16(a, w, None, outs[1])
+                kernels.gemm_bf16(a, w, None, outs[2], accumulate=True)
+                kernels.gemm_bf16_gated(a, fused, outs[3])
+                got.append(outs)
+            assert all(torch.equal(x, y) for x, y in zip(*got)), (m, n, k)
+            assert _rel(got[1][0], a.double() @ w.double().T + bias.double()) < 1e-5, (m, n, k)
+    finally:
+        kernels.gemm_bf16_force_tiling(-1)
+
+
+@pytest.mark.parametrize("m,n,k,tiling", [(1396, 1536, 1536, 16), (783, 4096, 2048, 17), (1000, 4608, 3584, 18), (2210, 4096, 1024, 19),
+                                          (910, 9216, 2048, 20)])
+def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    assert kernels.gemm_bf16_tile_carried_out(m, n, k) == tiling
+    out, other = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    kernels.gemm_bf16(a, w, None, out)
+    try:
+        kernels.gemm_bf16_force_tiling(kernels.gemm_bf16_tile_plan(m, n, k)[0])
+        kernels.gemm_bf16(a, w, None, other)
+    finally:
+        kernels.gemm_bf16_force_tiling(-1)
+    assert torch.equal(out, other)
+
+
 @pytest.mark.parametrize("m,n,k,tiling", [(129, 33, 2048, 13), (512, 64, 2048, 13), (161, 1792, 10496, 13), (512, 2048, 512, 14),
                                           (512, 1057, 2048, 14), (468, 1792, 4352, 14), (512, 2576, 512, 15), (700, 5120, 2048, 15),
                                           (140, 5536, 1600, 15), (330, 7488, 7168, 9), (953, 512, 6400, 9)])

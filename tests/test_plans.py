@@ -193,6 +193,16 @@ def test_past_128_tokens_small_tiles_carry_out_a_128x128_plan_unless_its_tiles_f
     assert plan(512, 2048, 2040)[0] == 0           # no whole steps of 64
 
 
+def test_a_plan_of_one_range_takes_the_tile_of_the_least_rounds():
+    """16: 192x64, 17: 128x128 of three stages, 18 and 19: 192x128 of three and two, 20: 192x192."""
+    from vipera_rs_amd.ops.kernels import gemm_bf16_tile_carried_out as carried, gemm_bf16_tile_plan as plan
+    assert carried(1396, 1536, 1536) == 16 and carried(783, 4096, 2048) == 17 and carried(1000, 4608, 3584) == 18
+    assert carried(2048, 4608, 3584, output_bytes=2) == 19 and carried(311, 22016, 2048, gated=True) == 20
+    assert carried(2048, 37888, 3584, gated=True) == 5 and carried(2048, 3584, 18944) == 7 and carried(1000, 2048, 1536) == 15
+    for sizes in ((100, 4608, 3584), (512, 2048, 2048), (330, 7488, 7168), (1396, 1536, 8960), (700, 4096, 2040)):
+        assert carried(*sizes) == plan(*sizes)[0]       # up to 128 tokens, 64x64 tiles, ranges, no whole steps of 64
+
+
 def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
     """Chunks as long as one another are few enough to run at once, never leave a position out and never outnumber what was
     allowed for."""

@@ -203,7 +203,7 @@ struct TileNorm {
 // barrier before the first product makes the parts visible; tile_norm_factor adds them in ascending order.
 template <int BM, int THREADS>
 __device__ __forceinline__ void tile_norm_parts(const TileNorm& norm, int m0, int M, int tid, float* part_sums) {
-  static_assert(THREADS % BM == 0, "whole threads per token");
+  if constexpr (THREADS % BM != 0) return;   // such tiles are not launched with a norm (launch_tile_as refuses it)
   constexpr int PER = THREADS / BM, AHEAD = 32;
   if (!norm.sumsq) return;
   const int token = tid % BM, part = tid / BM;
@@ -235,7 +235,7 @@ __device__ __forceinline__ void tile_epilogue(f32x4 (&acc)[TN][TM], TC* __restri
                                               int K, const float* __restrict__ bias, bool vector_ok, int wave_m,
                                               int wave_n, int lr, int lg, const TileNorm& norm,
                                               const float* part_sums, int wave_token, bool gelu = false) {
-  if (norm.sumsq) {
+  if (THREADS % BM == 0 && norm.sumsq) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       const float inv = tile_norm_factor<BM, THREADS>(norm, part_sums, wave_token + tm * 16 + lr, K);
@@ -1781,6 +1781,7 @@ int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, i
   static_assert(DIRECT || STAGES == 2, "only the direct kernel has a third stage");
   constexpr int lds_bytes = DIRECT ? STAGES * (BM + BN) * DIRECT_ROW : 2 * (BM + BN) * ROW * (int)sizeof(__bf16);
   static_assert(lds_bytes + WM * WN * 64 * 4 <= 160 * 1024, "a CU has 160 KB of LDS (the stages and the norm's sums)");
+  if (WM * WN * 64 % BM != 0 && norm.sumsq) return VK_UNSUPPORTED_SIZE;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const long long total = (long long)tiles_m * tiles_n;
   const long long grid = (total + XCDS - 1) / XCDS * XCDS;
@@ -1962,10 +1963,68 @@ TilePlan tile_plan(int M, int N, int K, long long partial_floats, bool gated, bo
   return plan;
 }
 
+// The tile that carries out a product whose K is in one piece (ranges 1) and whose plan says tiles of 128x64 or more. The
+// plan's estimate ranks by whole rounds of a few tiles; between them lie tiles that come in one round where the planned one
+// needs a little more than one, or half a round of a larger one: 192x64 (1,396 tokens on 1,536 rows are 264 tiles of 128x64,
+// eight CUs with two, and 192 of 192x64), 128x128 and 192x128 with three LDS stages, one workgroup a CU; 192x128 with two
+// stages, 80 KB, two to a CU (2,048 tokens on 4,608 rows are 396 of these, 192 of 256x192); 192x192 with three stages. What
+// bounds a step of K is the LDS reads of its fragments and a barrier, so that a step of a larger tile takes less time per
+// product, and a third stage about a third off the step of a workgroup that is alone on its CU.
+// Each tile's time is estimated as `beside` + K / 64 * (rounds) + `output` per MB of results moved, in us: a full round takes
+// `high` a step, one filled to a share f `low` + (high - low) f; where two workgroups share a CU, two full rounds take `pair`
+// together, and a second round filled to f the share `alone` + (1 - alone) f of what it adds. 16, 17 and 18 are for one round:
+// in more they lose to the larger tiles. Fitted to 81 products (the seven
+// designs' and Qwen2's shapes, 129 to 2,500 tokens, weights from memory; 5 % off on average): the tiles picked take 0.93 of
+// the planned ones' time over the 53 that are planned in one range and larger tiles, and 1 % more than the fastest of each; a tile is changed only for an estimate below
+// 0.98 of the planned one's. us, planned to picked: 1,396 tokens on 2,048 rows of 1,536 21.4 -> 14.8, on 1,536
+// rows 19.7 -> 16.2, 1,383 on 2,048 of 2,048 24.4 -> 18.2, 1,000 on 4,608 of 3,584 49.0 -> 37.8, 1,014 on 3,584 of 3,584
+// 48.3 -> 38.8; gated: 1,396 on 17,920 of 1,536 89.8 -> 80.7, 622 on 5,120 of 2,048 25.0 -> 20.1, 311 on 22,016 46.1 -> 36.2.
+// Every output is one sum over K in ascending steps of 32 whatever the tile, so the bits are the same.
+struct TileCost { int config, tokens, rows, resident; double beside, low, high, pair, alone, output; };
+constexpr TileCost WHOLE_TILES[] = {
+    {5, 256, 256, 1, 6.6, 1.17, 1.52, 0, 0, 0.164},     {6, 256, 192, 1, 4.4, 0.97, 1.28, 0, 0, 0.192},
+    {7, 256, 128, 1, 4.9, 0.62, 0.86, 0, 0, 0.176},     {9, 128, 128, 2, 2.0, 0.63, 0.84, 1.02, 0.68, 0.103},
+    {15, 128, 64, 2, 2.6, 0.28, 0.41, 0.69, 0.75, 0.091}, {16, 192, 64, 1, 3.7, 0.34, 0.44, 0, 0, 0.153},
+    {17, 128, 128, 1, 3.2, 0.41, 0.53, 0, 0, 0.174},    {18, 192, 128, 1, 5.3, 0.48, 0.59, 0, 0, 0.148},
+    {19, 192, 128, 2, 3.0, 0.71, 0.94, 1.32, 0.40, 0.115}, {20, 192, 192, 1, 6.4, 0.63, 0.96, 0, 0, 0.100}};
+double whole_tile_us(const TileCost& t, int M, int N, int K, double output_bytes) {
+  const long long groups = (long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows);
+  const long long full = groups / g_compute_units;
+  const double rest = (double)(groups % g_compute_units) / g_compute_units;
+  const double last = rest > 0 ? t.low + (t.high - t.low) * rest : 0;
+  double rounds = full * t.high + last;
+  if (t.resident == 2) {
+    rounds = full / 2 * t.pair + last;
+    if (full & 1) rounds = full / 2 * t.pair + t.high + (rest > 0 ? (t.pair - t.high) * (t.alone + (1 - t.alone) * rest) : 0);
+  }
+  return t.beside + K / 64 * rounds + t.output * 1e-6 * M * N * output_bytes;
+}
+// output_bytes: per product row and token (a gated product writes one 16-bit result for two rows).
+int whole_tile(int planned, int M, int N, int K, double output_bytes) {
+  int best = planned;
+  double best_us = -1;
+  for (const TileCost& t : WHOLE_TILES)
+    if (t.config == planned) best_us = 0.98 * whole_tile_us(t, M, N, K, output_bytes);
+  if (best_us < 0) return planned;   // the staged kernel's, and 64x64 tiles, which come in one round where they are planned
+  for (const TileCost& t : WHOLE_TILES) {
+    if (t.config == planned) continue;
+    if (t.config >= 16 && t.config <= 18 &&
+        (long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows) > g_compute_units)
+      continue;
+    const double us = whole_tile_us(t, M, N, K, output_bytes);
+    if (us < best_us) {
+      best_us = us;
+      best = t.config;
+    }
+  }
+  return best;
+}
+
 // Tilings: 0, 2, 3, 4 the staged kernel at 128x128, 256x128, 128x256, 256x256; 9, 7, 8, 5 the same tiles
 // with the kernel that loads straight into LDS, which needs K to be a multiple of 64; 13 and 15 that kernel at 64x64
 // and 128x64, 14 at 64x64 with the K ranges of one tile in one workgroup (15 always so); and 6 that kernel at
-// 256x192 (2,048 tokens x 4,608 rows are 192 such tiles for 256 CUs, against 144 of 256x256).
+// 256x192 (2,048 tokens x 4,608 rows are 192 such tiles for 256 CUs, against 144 of 256x256). 16 to 20: see whole_tile;
+// with a norm's factors, which are summed by a power of two of threads a token, they fall back to 9.
 template <typename TC, bool ACC, bool GATED = false>
 int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int M, int N, int K, long long lda,
                 long long ldc, int vector_ok, float* partial, long long partial_floats, hipStream_t s,
@@ -1973,11 +2032,14 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
   const bool direct = (K & 63) == 0;
   TilePlan plan = tile_plan(M, N, K, (GATED || !partial) ? 0 : partial_floats, GATED, norm.sumsq != nullptr);
   if (g_tile_config >= 0) plan = TilePlan{g_tile_config, g_tile_ranges > 1 && !GATED && partial ? g_tile_ranges : 1};
+  else if (direct && M > 128 && plan.ranges == 1 && !norm.sumsq) 
+    plan.config = whole_tile(plan.config, M, N, K, GATED ? 1.0 : sizeof(TC) * (ACC ? 2.0 : 1.0));
   if (plan.ranges > 1 && (long long)plan.ranges * M * N > partial_floats) plan.ranges = 1;
+  if (plan.config >= 16 && norm.sumsq) plan.config = 9;
   if (plan.config >= 10 && plan.config <= 12 && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
   if (!direct) {
     switch (plan.config) { case 5: case 6: plan.config = 4; break; case 7: plan.config = 2; break; case 8: plan.config = 3; break;
-                           case 9: case 10: case 11: case 12: case 13: case 14: case 15: plan.config = 0; break; }
+                           default: if (plan.config >= 9) plan.config = 0; }
   }
   const int r = plan.ranges;
 #define VK_TILE(BMV, BNV, WMV, WNV, DIRECTV) \
@@ -2019,6 +2081,17 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
       VK_TILE_SMALL(128, 64, 3, false);
   }
 #undef VK_TILE_SMALL
+#define VK_TILE_WHOLE(BMV, BNV, STAGESV)                                                                              \
+  return launch_tile_as<BMV, BNV, 4, 2, TC, ACC, GATED, true, STAGESV>(A, W, bias, C, M, N, K, lda, ldc, vector_ok, r, partial, \
+                                                                       s, norm)
+  switch (plan.config) {
+    case 16: VK_TILE_WHOLE(192, 64, 4);
+    case 17: VK_TILE_WHOLE(128, 128, 3);
+    case 18: VK_TILE_WHOLE(192, 128, 3);
+    case 19: VK_TILE_WHOLE(192, 128, 2);
+    case 20: VK_TILE_WHOLE(192, 192, 3);
+  }
+#undef VK_TILE_WHOLE
   switch (plan.config) {
     case 5: VK_TILE(256, 256, 4, 2, true);
     case 6: VK_TILE(256, 192, 4, 2, true);
@@ -2390,5 +2463,14 @@ extern "C" int vk_gemm_bf16_tile_plan(int M, int N, int K, long long partial_flo
   const TilePlan plan = tile_plan(M, N, K, gated ? 0 : partial_floats, gated != 0, false);
   *tiling = plan.config;
   *ranges = plan.ranges;
+  return 0;
+}
+
+// The tiling that carries this plan out (see whole_tile). output_bytes: 4 or 2 by the results' type, 8 where they are added.
+extern "C" int vk_gemm_bf16_tile_carried_out(int M, int N, int K, long long partial_floats, int gated, int output_bytes,
+                                             int* tiling) {
+  if (M <= 0 || N <= 0 || K <= 0) return VK_BAD_ARGUMENT;
+  const TilePlan plan = tile_plan(M, N, K, gated ? 0 : partial_floats, gated != 0, false);
+  *tiling = (K & 63) == 0 && M > 128 && plan.ranges == 1 ? whole_tile(plan.config, M, N, K, gated ? 1.0 : output_bytes) : plan.config;
   return 0;
 }

@@ -749,17 +749,30 @@ def gemm_bf16_gated_tile_scaled(scaled: torch.Tensor, w: torch.Tensor, out: torc
 TILE_TILINGS = {0: "128x128 staged", 2: "256x128 staged", 3: "128x256 staged", 4: "256x256 staged",
                 9: "128x128 direct", 7: "256x128 direct", 8: "128x256 direct", 5: "256x256 direct", 6: "256x192 direct",
                 10: "128x96 direct, gated only", 11: "128x160 direct, gated only", 12: "128x224 direct, gated only",
-                13: "64x64 direct", 14: "64x64 direct, ranges in one workgroup", 15: "128x64 direct, ranges in one workgroup"}
+                13: "64x64 direct", 14: "64x64 direct, ranges in one workgroup", 15: "128x64 direct, ranges in one workgroup",
+                16: "192x64 direct", 17: "128x128 direct, three stages", 18: "192x128 direct, three stages",
+                19: "192x128 direct, two stages", 20: "192x192 direct"}
 
 
 def gemm_bf16_tile_plan(m: int, n: int, k: int, gated: bool = False) -> Tuple[int, int]:
     """The tiling (a key of ``TILE_TILINGS``) and the number of ranges of K that the tiled kernel of :func:`gemm_bf16` (or
-    :func:`gemm_bf16_gated`) takes for these sizes."""
+    :func:`gemm_bf16_gated`) plans for these sizes; the ranges decide the bits.  A plan of one range may be carried out by
+    another tiling with the same bits: :func:`gemm_bf16_tile_carried_out`."""
     tiling, ranges = _i(), _i()
     fn = _fn("gemm_bf16", "vk_gemm_bf16_tile_plan", [_i, _i, _i, _ll, _i, _p, _p])
     _status(fn(m, n, k, min(8 * m * n, _TILE_WORKSPACE_FLOATS), 1 if gated else 0, ctypes.addressof(tiling),
                ctypes.addressof(ranges)), "gemm_bf16_tile_plan")
     return tiling.value, ranges.value
+
+
+def gemm_bf16_tile_carried_out(m: int, n: int, k: int, gated: bool = False, output_bytes: int = 4) -> int:
+    """The tiling (a key of ``TILE_TILINGS``) that carries out the plan of :func:`gemm_bf16_tile_plan`; ``output_bytes``: 4 or 2
+    by the type of the results, 8 where they are added to what is there."""
+    tiling = _i()
+    fn = _fn("gemm_bf16", "vk_gemm_bf16_tile_carried_out", [_i, _i, _i, _ll, _i, _i, _p])
+    _status(fn(m, n, k, min(8 * m * n, _TILE_WORKSPACE_FLOATS), 1 if gated else 0, output_bytes, ctypes.addressof(tiling)),
+            "gemm_bf16_tile_carried_out")
+    return tiling.value
 
 
 def gemm_bf16_force_tiling(tiling: int = -1, ranges: int = 1, stages: int = 0) -> None:
