@@ -917,6 +917,36 @@ def test_decode_attention_at_the_benchmark_head_shapes(heads, kv_heads, hd, batc
     assert _rel(out.cpu(), want) < 1.2e-2, "32-bit-arithmetic kernel on the bfloat16 cache"
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd,window,keep", [(14, 2, 64, 0, 0), (4, 1, 128, 0, 0), (8, 4, 128, 200, 70), (3, 3, 64, 96, 0)])
+def test_prompt_tiles_shared_between_workgroups_and_narrow_addresses_give_the_same_bits(heads, kv_heads, hd, window, keep):
+    """Tiles whose tokens end in the first and the second half, at a wave's edge and one past it, behind nothing and behind
+    hundreds of positions; offsets of 32 bits against addresses of 64 for every form of the kernel."""
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.attention import AttentionExtras
+    bs, dtype = 16, torch.bfloat16
+    entries = [(2, 2), (64, 64), (65, 65), (500, 17), (900, 129), (333, 333), (1300, 208)]   # (positions after the step, tokens)
+    cache = _Paged([kv for kv, _ in entries], kv_heads, hd, bs, dtype, seed=hd + heads)
+    counts, first = [n for _, n in entries], [kv - n for kv, n in entries]
+    starts = [sum(counts[:e]) for e in range(len(counts) + 1)]
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    qkv = dev(torch.randn(starts[-1], (heads + 2 * kv_heads) * hd, generator=torch.Generator().manual_seed(heads)).to(dtype))
+    tiles = sorted((first[e] + off, e, off) for e, n in enumerate(counts) for off in range(0, n, 128))
+    arrays = [dev(torch.tensor(x, dtype=torch.int32)) for x in ([x for _, e, off in tiles for x in (e, off)], starts, first)]
+    k, v, table = dev(cache.k), dev(cache.v), dev(cache.table)
+    extras = AttentionExtras(keep_first=keep) if keep else None
+
+    def run(split, pages, chunk_tiles=0, max_chunks=0):
+        out = torch.full((starts[-1], heads * hd), 7.0, dtype=dtype, device=DEV)
+        kernels.attn_bf16_prefill(qkv, k, v, out, *arrays, table, heads, kv_heads, hd, hd ** -0.5, window, split, chunk_tiles,
+                                  max_chunks, extras=extras, cache_pages=pages)
+        return out
+
+    halved = run(1, None)
+    assert torch.equal(run(2, None), halved) and torch.equal(run(2, 0), halved) and torch.equal(run(1, 0), halved)
+    assert torch.equal(run(0, None), run(0, 0)) and torch.equal(run(0, None, 3, 8), run(0, 0, 3, 8))
+    assert _rel(run(0, None), halved.double()) < 1.2e-2
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", BENCH_HEADS, ids=[f"h{h}kv{k}" for h, k, _ in BENCH_HEADS])
 def test_prompt_attention_at_the_benchmark_head_shapes(heads, kv_heads, hd):
     """One prompt of 2,048 tokens from position 0 and one portion of 512 tokens from position 3,584 in one step."""

@@ -26,6 +26,8 @@
 #include "attn_extras.h"
 #include "pipeline.h"
 
+#include <type_traits>
+
 #ifndef HDP
 #define HDP 128
 #endif
@@ -567,8 +569,6 @@ constexpr int PD_C = HDP / 8;                           // 16-byte chunks of a K
 constexpr int PD_KBYTES = PT_KV * PD_ROWB;              // K tile: 64 rows
 constexpr int PD_VBYTES = HDP * 128;                    // V^T tile: HDP rows of 64 positions
 constexpr int PD_STAGE = PD_KBYTES + PD_VBYTES;
-constexpr int PD_KLOADS = PD_KBYTES / 1024 / PT_WAVES;  // load instructions per wave and tile
-constexpr int PD_VLOADS = PD_VBYTES / 1024 / PT_WAVES;
 constexpr int PD_ROWS_PER_LOAD = 1024 / PD_ROWB;
 constexpr bool PD_CAN_SPLIT = 4 * PD_STAGE <= 128 * 1024;  // two halves with two stages each
 
@@ -581,21 +581,36 @@ __device__ __forceinline__ int k_swizzle(int r) {
 
 constexpr int PD_PARTIAL_ROW = HDP + 4;   // floats of a column's partial result: the weighted sum, max, sum, and padding to 16 bytes
 
-template <bool SPLIT, bool CHUNKED = false>
-__global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_prefill_direct_kernel(
+// PARTS 2 (with SPLIT): the tile's 128 columns are shared between two workgroups of eight waves, each of which walks the tile's
+// positions, in the halves of the whole tile: every column's sums are those of PARTS 1. For items that are no more than the CUs:
+// what a step costs a CU is its waves' products, exponentials and LDS reads, behind one another. us, one workgroup a tile against two: 512 tokens
+// of 16 heads of 128 at 1,536 47.3 / 35.5, 1,000 of 12 28.2 / 22.3, 333 of 14 heads of 64 10.7 / 8.5, 1,200 of 16 (160 tiles) 31.3 /
+// 26.5, 1,834 of 16 (240) 28.2 / 28.1; a quarter of the columns a workgroup measured as a half does where it has a CU and up to
+// twice as long where it has not. With half the waves there are the registers to spread the next tile's loads over this one's parts and to
+// take the tile that holds the end in a loop of its own (38.2 to 35.5 of the first), which cost the other forms their second
+// workgroup a CU (61 to 82 us).
+//
+// WIDE: the cache is 4 GB or more, and a load's address is 64 bits wide; else it is an offset behind a buffer descriptor, which
+// takes fewer vector instructions and registers (one prompt of 2,048 tokens, 28 heads, whole tiles 69.3 to 60.6 us, halved 59.5 to 57.2).
+template <bool SPLIT, bool CHUNKED, int PARTS, bool WIDE>
+__global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void attn_prefill_direct_kernel(
     const __bf16* __restrict__ q, long long q_stride, const __bf16* __restrict__ k_cache,
     const __bf16* __restrict__ v_cache, __bf16* __restrict__ out, const int* __restrict__ tiles,
     const int* __restrict__ entry_start, const int* __restrict__ entry_first_pos,
     const int* __restrict__ block_table, int table_width, int block_size, int heads, int kv_heads, float scale,
-    int window, float softcap, int cus, float* __restrict__ partial, int chunk_tiles, int max_chunks, AttnExtras ex) {
+    int window, float softcap, int cus, float* __restrict__ partial, int chunk_tiles, int max_chunks,
+    unsigned cache_bytes, AttnExtras ex) {
   static_assert(!(SPLIT && CHUNKED), "a chunk is taken by a workgroup of eight waves");
+  static_assert(PARTS == 1 || (SPLIT && PT_WAVES % PARTS == 0), "only halved tiles are shared");
+  constexpr int WAVES = PT_WAVES / PARTS;                                           // of a half
+  constexpr int PD_KLOADS = PD_KBYTES / 1024 / WAVES, PD_VLOADS = PD_VBYTES / 1024 / WAVES;   // load instructions per wave and tile
   typedef __attribute__((address_space(3))) void* lds_ptr;
   typedef __attribute__((address_space(1))) const void* global_ptr;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];  // [2][K tile | V^T tile]
   constexpr int hd = HDP;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int wave_of_group = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = SPLIT ? wave_of_group >> 3 : 0, wave = SPLIT ? wave_of_group & 7 : wave_of_group;
+  const int half = SPLIT ? wave_of_group / WAVES : 0, wave = SPLIT ? wave_of_group % WAVES : wave_of_group;
   unsigned char* lds_half = lds_raw + half * 2 * PD_STAGE;
   // work items as in attn_prefill_kernel: long ones first, paired with short ones on a CU (SPLIT: one
   // workgroup per CU, longest first)
@@ -605,7 +620,7 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
   // fetches those tiles once (with numbers in a row, every head of a group ran on another XCD). Every other run
   // of 8 groups is dealt to the XCDs in the opposite order: the items come sorted by length, and dealt one way
   // only the first XCDs would get the longer item of every run.
-  const int heads_per_key = heads / kv_heads;
+  const int heads_per_key = heads / kv_heads * PARTS;   // the parts of an item read the same K and V as well
   auto by_xcd = [&](int number, int count) {
     const int block = 8 * heads_per_key;
     if (number >= count / block * block) return number;
@@ -620,9 +635,9 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
   const int chunk = CHUNKED ? (int)blockIdx.x / total : 0;
   const int item = CHUNKED ? total - 1 - by_xcd((int)blockIdx.x % total, total)
                            : SPLIT ? total - 1 - by_xcd((int)blockIdx.x, total) : (round & 1) ? taken : total - 1 - taken;
-  const int tile = item / heads;
+  const int tile = item / (heads * PARTS), part = item % PARTS;
   const int entry = tiles[2 * tile], tile_off = tiles[2 * tile + 1];
-  const int h = item % heads, kvh = h / (heads / kv_heads);
+  const int h = item / PARTS % heads, kvh = h / (heads / kv_heads);
   const int tok0 = entry_start[entry], count = entry_start[entry + 1] - tok0;
   const int first_pos = entry_first_pos[entry];
   const int* table = block_table + (size_t)entry * table_width;
@@ -637,8 +652,9 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
   const int all_tiles = walk.count(end);
   const int chunks = CHUNKED ? (all_tiles + chunk_tiles - 1) / chunk_tiles : 1;
   if (CHUNKED && chunk >= chunks) return;   // the whole workgroup, before any barrier
+  if (PARTS > 1 && part * WAVES * 16 >= tile_cols) return;   // a last tile's columns end before this part: likewise
 
-  const int q_off = tile_off + wave * 16;
+  const int q_off = tile_off + (part * WAVES + wave) * 16;
   const int c = q_off + lr;
   const bool col_ok = c < count;
   const int col_pos = col_ok ? first_pos + c : -1;
@@ -688,19 +704,28 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
 #pragma unroll
     for (int i = 0; i < PD_VLOADS; ++i) v_page[i] = table[min(max(tp + v_tab[i], page_lo), page_hi)];
   };
-  auto issue = [&](int stage) {
+  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(k_cache), 0, (int)cache_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(v_cache), 0, (int)cache_bytes, 0x00020000);
+  auto load = [&](const __bf16* cache, __amdgpu_buffer_rsrc_t rsrc, int page, unsigned in, unsigned char* to) {
+    if constexpr (WIDE)
+      __builtin_amdgcn_global_load_lds((global_ptr)((const char*)cache + ((size_t)(unsigned)page * page_bytes + in)), (lds_ptr)to,
+                                       16, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)to, 16, (int)((unsigned)page * page_bytes + in), 0, 0, 0);
+  };
+  auto issue = [&](int stage, int quarter) {   // a quarter of a tile's loads
     unsigned char* to_k = lds_half + stage * PD_STAGE + wave * PD_KLOADS * 1024;
     unsigned char* to_v = lds_half + stage * PD_STAGE + PD_KBYTES + wave * PD_VLOADS * 1024;
 #pragma unroll
     for (int i = 0; i < PD_KLOADS; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)((const char*)k_cache + ((size_t)(unsigned)k_page[i] * page_bytes + k_in[i])),
-          (lds_ptr)(to_k + i * 1024), 16, 0, 0);
+      if (i % 4 == quarter) load(k_cache, k_rsrc, k_page[i], k_in[i], to_k + i * 1024);
 #pragma unroll
     for (int i = 0; i < PD_VLOADS; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)((const char*)v_cache + ((size_t)(unsigned)v_page[i] * page_bytes + v_in[i])),
-          (lds_ptr)(to_v + i * 1024), 16, 0, 0);
+      if ((PD_KLOADS + i) % 4 == quarter) load(v_cache, v_rsrc, v_page[i], v_in[i], to_v + i * 1024);
+  };
+  auto issue_all = [&](int stage) {
+#pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter) issue(stage, quarter);
   };
 
   // a lane's operand addresses within a stage
@@ -718,7 +743,8 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
   const float cap_raw = softcap > 0.f ? softcap / scale : 0.f, cap_inv = softcap > 0.f ? scale / softcap : 0.f;
   const float* rel_row = ex.rel ? ex.rel + (size_t)h * (ex.rel_far + 1) : nullptr;
   const float inv_scale = 1.f / scale;
-  auto tile_body = [&](bool masked, int p0, const unsigned char* base) {
+  // `next` (PARTS 2): whether the next tile's loads go out between this one's parts, into `next_stage`
+  auto tile_body = [&](bool masked, int p0, const unsigned char* base, bool next, int next_stage) {
     // ---- scores: tile sub = 2 st + t holds positions p0 + 32 st + 8 g + 4 t + j in register j of lane group g
     f32x4 s[4];
 #pragma unroll
@@ -730,6 +756,7 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], acc, 0, 0, 0);
       }
       s[sub] = acc;
+      if (PARTS > 1 && (sub & 1) && next) issue(next_stage, sub >> 1);
     }
     if (softcap > 0.f) {   // raw scores whose product with the scale is the capped score
 #pragma unroll
@@ -782,19 +809,26 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
       }
       l += sum;
     }
-    const bool tail = p0 + PT_KV > end;
+    if (PARTS > 1 && next) issue(next_stage, 2);
+    auto weigh = [&](auto tail) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
+      for (int dt = 0; dt < DT; ++dt) {
+        if (PARTS > 1 && dt == DT / 2 && next) issue(next_stage, 3);
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        bf16x8 vf = *(const bf16x8*)(base + v_at[st] + dt * 16 * 128);
-        if (tail) {
-          const int kept = end - (p0 + st * 32 + lg * 8);
-          vf = keep_before_end(vf, kept, kept - 4);
+        for (int st = 0; st < 2; ++st) {
+          bf16x8 vf = *(const bf16x8*)(base + v_at[st] + dt * 16 * 128);
+          if (tail) {
+            const int kept = end - (p0 + st * 32 + lg * 8);
+            vf = keep_before_end(vf, kept, kept - 4);
+          }
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[st], o[dt], 0, 0, 0);
         }
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[st], o[dt], 0, 0, 0);
       }
-    }
+    };
+    const bool tail = p0 + PT_KV > end;
+    if constexpr (PARTS == 1) weigh(tail);
+    else if (tail) weigh(std::true_type{});
+    else weigh(std::false_type{});
   };
 
   // this half's tiles: all of them, or with SPLIT the first or the second half of them (both halves pass the
@@ -803,27 +837,35 @@ __global__ __launch_bounds__(SPLIT ? 2 * PT_THREADS : PT_THREADS) void attn_pref
   const int my_tiles = half ? all_tiles - steps : steps;
   const int my_first = CHUNKED ? chunk * chunk_tiles : half ? steps : 0;   // in tiles of the walk
   lookup(walk.at(my_first));
-  if (my_tiles > 0) issue(0);
+  if (my_tiles > 0) issue_all(0);
   lookup(walk.at(my_first + 1));
   wait_own_loads();
   __syncthreads();
   int stage = 0;
   for (int i = 0; i < steps; ++i) {
     const int p0 = walk.at(my_first + i);
-    if (i + 1 < my_tiles) {
-      issue(stage ^ 1);            // nobody reads that stage any more: the barrier that ended the last tile
-      lookup(walk.at(my_first + i + 2));
+    const bool next = i + 1 < my_tiles;   // into the stage that nobody reads any more: the barrier that ended the last tile
+    const bool sees = i < my_tiles && p0 < wave_end && (p0 + PT_KV > wave_begin || p0 < ex.keep_first);
+    const bool masked = !(p0 + PT_KV - 1 <= wave_first && p0 >= wave_lo_max);
+    if constexpr (PARTS == 1) {
+      if (next) {
+        issue_all(stage ^ 1);
+        lookup(walk.at(my_first + i + 2));
+      }
+      if (sees) tile_body(masked, p0, lds_half + stage * PD_STAGE, next, stage ^ 1);
+    } else {
+      if (sees) tile_body(masked, p0, lds_half + stage * PD_STAGE, next, stage ^ 1);
+      else if (next) issue_all(stage ^ 1);
+      if (next) lookup(walk.at(my_first + i + 2));
     }
-    if (i < my_tiles && p0 < wave_end && (p0 + PT_KV > wave_begin || p0 < ex.keep_first))
-      tile_body(!(p0 + PT_KV - 1 <= wave_first && p0 >= wave_lo_max), p0, lds_half + stage * PD_STAGE);
     wait_own_loads();   // a barrier alone does not wait for loads that write LDS
     __syncthreads();
     stage ^= 1;
   }
   if constexpr (SPLIT) {
     // the second half hands its state over in LDS (every tile has been read: the loop's last barrier)
-    f32x4* hand_o = (f32x4*)lds_raw;                                        // [8 waves][DT][64 lanes]
-    float* hand_ml = (float*)(lds_raw + PT_WAVES * DT * 64 * sizeof(f32x4));  // [8 waves][64 lanes][m, l]
+    f32x4* hand_o = (f32x4*)lds_raw;                                        // [waves of a half][DT][64 lanes]
+    float* hand_ml = (float*)(lds_raw + WAVES * DT * 64 * sizeof(f32x4));  // [waves of a half][64 lanes][m, l]
     if (half) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) hand_o[(wave * DT + dt) * 64 + lane] = o[dt];
@@ -1133,18 +1175,20 @@ extern "C" int vk_attn_bf16_hdp() { return HDP; }
 // tiles: pairs (entry, first token of the tile within the entry), 128 tokens per tile; best sorted by the
 // number of positions a tile sees, rising (any order gives the same result). split: nonzero asks for workgroups
 // of sixteen waves that halve a tile's positions between them, where the kernel in use has that form (few tiles
-// of very different lengths); the result is the same up to rounding.
+// of very different lengths); the result is the same up to rounding. split 2: such halves, with the tile's tokens shared
+// between two workgroups; the same bits as split 1.
 // chunk_tiles > 0 (with the kernel that loads straight into LDS; ignored otherwise): a tile's steps of 64 positions
 // are cut into chunks of that many, a workgroup each, of which no tile has more than `max_chunks`; `partial` holds
 // num_tiles * heads * max_chunks * 128 * (padded head width + 4) floats.
 // sink, rel, rel_far, keep_first, gate, gate_ld: see attn_extras.h (null and 0: none of them).
-extern "C" int vk_attn_bf16_prefill_ext(const void* q, long long q_stride, const void* k_cache, const void* v_cache,
+// cache_pages: pages that either cache holds (0: not known; what it is used for is whether offsets fit 32 bits).
+extern "C" int vk_attn_bf16_prefill_pages(const void* q, long long q_stride, const void* k_cache, const void* v_cache,
                                     void* out, const int* tiles, int num_tiles, const int* entry_start,
                                     const int* entry_first_pos, const int* block_table, int table_width,
                                     int block_size, int heads, int kv_heads, int hd, float scale, int window, float softcap,
                                     int split, float* partial, long long partial_floats, int chunk_tiles,
                                     int max_chunks, const float* sink, const float* rel, int rel_far, int keep_first,
-                                    const float* gate, long long gate_ld, void* stream) {
+                                    const float* gate, long long gate_ld, long long cache_pages, void* stream) {
   const AttnExtras ex{sink, rel, rel_far, keep_first, gate, gate_ld};
   if (rel_far < 0 || keep_first < 0 || (keep_first > 0 && window <= 0)) return VK_BAD_ARGUMENT;
   if (num_tiles <= 0) return 0;
@@ -1172,22 +1216,25 @@ extern "C" int vk_attn_bf16_prefill_ext(const void* q, long long q_stride, const
   }
   if ((long long)num_tiles * heads > 0x7fffffffLL) return VK_UNSUPPORTED_SIZE;
 #ifdef VK_PREFILL_DIRECT
+  const long long page_bytes = (long long)kv_heads * block_size * hd * 2;
+  const bool wide = cache_pages <= 0 || cache_pages > 0xFFFFFFFFll / page_bytes;
+  const unsigned cache_bytes = wide ? 0 : (unsigned)(cache_pages * page_bytes);
   if (fast && hd == HDP && block_size >= 8 && chunk_tiles > 0) {  // the kernel that loads straight into LDS, in chunks
     if (max_chunks <= 0 || !partial || ((uintptr_t)partial & 15) ||
         (long long)num_tiles * heads * max_chunks * PT_TOKENS * PD_PARTIAL_ROW > partial_floats)
       return VK_BAD_ARGUMENT;
     if ((long long)num_tiles * heads * max_chunks > 0x7fffffffLL) return VK_UNSUPPORTED_SIZE;
-    auto chunked = attn_prefill_direct_kernel<false, true>;
-    static bool chunked_configured = false;
-    if (!chunked_configured) {
+    auto chunked = wide ? attn_prefill_direct_kernel<false, true, 1, true> : attn_prefill_direct_kernel<false, true, 1, false>;
+    static bool chunked_configured[2] = {false, false};
+    if (!chunked_configured[wide]) {
       hipError_t e = hipFuncSetAttribute((const void*)chunked, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * PD_STAGE);
       if (e != hipSuccess) return (int)e;
-      chunked_configured = true;
+      chunked_configured[wide] = true;
     }
     chunked<<<num_tiles * heads * max_chunks, PT_THREADS, 2 * PD_STAGE, (hipStream_t)stream>>>(
         (const __bf16*)q, q_stride, (const __bf16*)k_cache, (const __bf16*)v_cache, (__bf16*)out, tiles, entry_start,
         entry_first_pos, block_table, table_width, block_size, heads, kv_heads, scale, window, softcap, cus, partial,
-        chunk_tiles, max_chunks, ex);
+        chunk_tiles, max_chunks, cache_bytes, ex);
     VK_LAUNCH_CHECK();
     attn_prefill_merge_kernel<<<dim3(num_tiles, heads, PT_TOKENS * (HDP / 4) / 256), 256, 0, (hipStream_t)stream>>>(
         partial, (__bf16*)out, tiles, entry_start, entry_first_pos, heads, scale, window, softcap, chunk_tiles, max_chunks, ex);
@@ -1196,20 +1243,27 @@ extern "C" int vk_attn_bf16_prefill_ext(const void* q, long long q_stride, const
   }
   if (fast && hd == HDP && block_size >= 8) {  // the kernel that loads straight into LDS
     const bool halves = split != 0 && PD_CAN_SPLIT;
-    auto direct = attn_prefill_direct_kernel<false>;
+    const int parts = halves && split == 2 ? 2 : 1;
+    if ((long long)num_tiles * heads * parts > 0x7fffffffLL) return VK_UNSUPPORTED_SIZE;
+    auto direct = wide ? attn_prefill_direct_kernel<false, false, 1, true> : attn_prefill_direct_kernel<false, false, 1, false>;
     if constexpr (PD_CAN_SPLIT) {
-      if (halves) direct = attn_prefill_direct_kernel<true>;
+      if (parts == 2)
+        direct = wide ? attn_prefill_direct_kernel<true, false, 2, true> : attn_prefill_direct_kernel<true, false, 2, false>;
+      else if (halves)
+        direct = wide ? attn_prefill_direct_kernel<true, false, 1, true> : attn_prefill_direct_kernel<true, false, 1, false>;
     }
     const int direct_lds = (halves ? 4 : 2) * PD_STAGE;
-    static bool direct_configured[2] = {false, false};
-    if (!direct_configured[halves]) {
+    static bool direct_configured[6] = {false, false, false, false, false, false};
+    const int which = (halves ? parts : 0) * 2 + (wide ? 1 : 0);
+    if (!direct_configured[which]) {
       hipError_t e = hipFuncSetAttribute((const void*)direct, hipFuncAttributeMaxDynamicSharedMemorySize, direct_lds);
       if (e != hipSuccess) return (int)e;
-      direct_configured[halves] = true;
+      direct_configured[which] = true;
     }
-    direct<<<num_tiles * heads, halves ? 2 * PT_THREADS : PT_THREADS, direct_lds, (hipStream_t)stream>>>(
+    direct<<<num_tiles * heads * parts, (halves ? 2 * PT_THREADS : PT_THREADS) / parts, direct_lds, (hipStream_t)stream>>>(
         (const __bf16*)q, q_stride, (const __bf16*)k_cache, (const __bf16*)v_cache, (__bf16*)out, tiles, entry_start,
-        entry_first_pos, block_table, table_width, block_size, heads, kv_heads, scale, window, softcap, cus, nullptr, 0, 1, ex);
+        entry_first_pos, block_table, table_width, block_size, heads, kv_heads, scale, window, softcap, cus, nullptr, 0, 1,
+        cache_bytes, ex);
     VK_LAUNCH_CHECK();
     return 0;
   }
@@ -1219,6 +1273,19 @@ extern "C" int vk_attn_bf16_prefill_ext(const void* q, long long q_stride, const
       entry_first_pos, block_table, table_width, block_size, heads, kv_heads, hd, scale, window, softcap, cus, ex);
   VK_LAUNCH_CHECK();
   return 0;
+}
+
+extern "C" int vk_attn_bf16_prefill_ext(const void* q, long long q_stride, const void* k_cache, const void* v_cache,
+                                    void* out, const int* tiles, int num_tiles, const int* entry_start,
+                                    const int* entry_first_pos, const int* block_table, int table_width,
+                                    int block_size, int heads, int kv_heads, int hd, float scale, int window, float softcap,
+                                    int split, float* partial, long long partial_floats, int chunk_tiles,
+                                    int max_chunks, const float* sink, const float* rel, int rel_far, int keep_first,
+                                    const float* gate, long long gate_ld, void* stream) {
+  return vk_attn_bf16_prefill_pages(q, q_stride, k_cache, v_cache, out, tiles, num_tiles, entry_start, entry_first_pos,
+                                    block_table, table_width, block_size, heads, kv_heads, hd, scale, window, softcap, split,
+                                    partial, partial_floats, chunk_tiles, max_chunks, sink, rel, rel_far, keep_first, gate,
+                                    gate_ld, 0, stream);
 }
 
 extern "C" int vk_attn_bf16_prefill_capped(const void* q, long long q_stride, const void* k_cache, const void* v_cache,

@@ -158,9 +158,9 @@ def chunks_prompt_tiles(num_tiles: int, heads: int, longest: int, total: int, cu
     return chunk_tiles, -(-longest_steps // chunk_tiles)
 
 
-# us as measured by padded head width: of a step of 64 positions and beside the steps, for a workgroup that takes a tile alone
-# (halved between sixteen waves where the width allows), for chunks of which a CU has one at the most, and two
-PROMPT_COSTS = {64: ((0.9, 5.0), (0.96, 10.7, 0.015), (0.95, 17.0, 0.015)), 128: ((1.35, 5.5), (2.1, 7.0, 0.025), (2.5, 4.0, 0.025)),
+# us as measured by padded head width: of a step of 64 positions and beside the steps, for a tile that is taken whole
+# (halved, and its tokens shared between two workgroups, where the width allows), for chunks of which a CU has one at the most, and two
+PROMPT_COSTS = {64: ((0.66, 4.8), (0.96, 10.7, 0.015), (0.95, 17.0, 0.015)), 128: ((0.95, 6.2), (2.1, 7.0, 0.025), (2.5, 4.0, 0.025)),
                 256: ((3.1, 6.0), (2.84, 13.6, 0.027), None)}
 
 
@@ -194,15 +194,19 @@ def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int):
 
 
 def _prompt_plan(batch, k_cache, heads: int, kv_heads: int, head_dim: int, window: int, cus: int):
-    """``(chunk_tiles and max_chunks, or None; whether tiles are halved)``, once for a step's layers of one geometry."""
+    """``(chunk_tiles and max_chunks, or None; 0, or 1 where tiles are halved, or 2 where two workgroups share such a tile's
+    tokens)``, once for a step's layers of one geometry.  Two where the tiles are no more than the CUs: the same bits in 0.75
+    to 1 of the time (see attn_prefill_direct_kernel; 448 tiles on 256 CUs 57 and 81 us)."""
     chunked = None
     if kernels.attn_bf16_prefill_loads_directly(k_cache, kv_heads, head_dim):
         if getattr(batch, "free_sum_order", False):
             chunked = cut_prompt_tiles(batch.tile_reaches, heads, head_dim, window, cus)
         else:
             chunked = chunks_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach, batch.sum_tile_reach, cus)
-    return chunked, chunked is None and halves_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach,
-                                                            batch.sum_tile_reach, cus)
+    if chunked is not None or not halves_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach,
+                                                      batch.sum_tile_reach, cus):
+        return chunked, 0
+    return None, 2 if batch.num_prefill_tiles * heads <= cus else 1
 
 
 def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, head_dim, scale, window,

@@ -818,13 +818,16 @@ ATTN_PREFILL_PARTIAL_ROW_EXTRA = 4   # floats beside the padded head width in a 
 def attn_bf16_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
                       tiles: torch.Tensor, entry_start: torch.Tensor, entry_first_pos: torch.Tensor,
                       block_table: torch.Tensor, heads: int, kv_heads: int, head_dim: int, scale: float,
-                      window: int, split: bool = False, chunk_tiles: int = 0, max_chunks: int = 0,
-                      softcap: float = 0.0, extras=None) -> None:
+                      window: int, split: int = 0, chunk_tiles: int = 0, max_chunks: int = 0,
+                      softcap: float = 0.0, extras=None, cache_pages: Optional[int] = None) -> None:
     """Attention of the entries' 128-token tiles listed in ``tiles`` (pairs: entry, first token within it).
     ``split``: workgroups of sixteen waves that halve a tile's positions between them and merge at the end, where
-    the kernel in use has that form (for few tiles of very different lengths); the same result up to rounding.
+    the kernel in use has that form (for few tiles of very different lengths); the same result up to rounding.  2: such
+    halves, with a tile's tokens shared between two workgroups, and the same bits as 1.
     ``chunk_tiles`` > 0 (where :func:`attn_bf16_prefill_loads_directly`): a tile's steps of 64 positions are cut into
     chunks of that many, a workgroup each, and a second kernel merges them; no tile may have more than ``max_chunks``."""
+    if cache_pages is None:      # 0, for tests: addresses of 64 bits, as for caches of 4 GB and more
+        cache_pages = k_cache.shape[0]
     _dev(q, k_cache, v_cache, out, tiles, entry_start, entry_first_pos, block_table)
     _need(attn_bf16_supported(q, k_cache, head_dim), "attn_bf16: operands must be bfloat16 with 16-byte rows")
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= heads * head_dim, "attention: q")
@@ -844,14 +847,14 @@ def attn_bf16_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     else:
         chunk_tiles = max_chunks = 0
     module = f"attn_bf16_hd{attn_bf16_padded_width(head_dim)}"
-    fn = _fn(module, "vk_attn_bf16_prefill_ext",
-             [_p, _ll, _p, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _f, _i, _f, _i, _p, _ll, _i, _i, _p, _p, _i, _i, _p, _ll, _p],
+    fn = _fn(module, "vk_attn_bf16_prefill_pages",
+             [_p, _ll, _p, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _i, _f, _i, _f, _i, _p, _ll, _i, _i, _p, _p, _i, _i, _p, _ll, _ll, _p],
              key=module + ".prefill")
     _status(fn(_ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(tiles), num_tiles,
                _ptr(entry_start), _ptr(entry_first_pos), _ptr(block_table), block_table.shape[1], k_cache.shape[2],
-               heads, kv_heads, head_dim, float(scale), int(window), float(softcap), 1 if split else 0, _ptr(partial),
+               heads, kv_heads, head_dim, float(scale), int(window), float(softcap), int(split), _ptr(partial),
                partial.numel() if partial is not None else 0, int(chunk_tiles), int(max_chunks),
-               *attn_extras_args(extras, heads, window, out.shape[0]), _stream()),
+               *attn_extras_args(extras, heads, window, out.shape[0]), cache_pages, _stream()),
             "attn_bf16_prefill")
 
 
