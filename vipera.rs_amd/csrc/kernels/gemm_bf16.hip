@@ -2020,6 +2020,24 @@ int whole_tile(int planned, int M, int N, int K, double output_bytes) {
   return best;
 }
 
+// The tiling and ranges that launch_tile carries out, worked out once for a size: the estimates of two dozen plans and ten tiles
+// take a microsecond or two, which is what a step of a few hundred tokens of a small model, launched eagerly, waits for. Each thread
+// keeps the last plan of every slot of its own table; the answer depends on nothing but the key.
+TilePlan carried_out(int M, int N, int K, long long partial_floats, bool gated, bool scaled, double output_bytes) {
+  struct Kept { long long floats; int M, N, K, form; TilePlan plan; };
+  constexpr int SLOTS = 512;
+  thread_local Kept table[SLOTS] = {};
+  const int form = (gated ? 1 : 0) | (scaled ? 2 : 0) | (int)output_bytes << 2 | g_tile_stages << 8;
+  const unsigned hash = ((unsigned)M * 0x9E3779B1u ^ (unsigned)N * 0x85EBCA6Bu ^ (unsigned)K * 0xC2B2AE35u ^ (unsigned)form * 0x27D4EB2Fu);
+  Kept& kept = table[(hash ^ hash >> 15) % SLOTS];
+  if (kept.M != M || kept.N != N || kept.K != K || kept.form != form || kept.floats != partial_floats) {
+    TilePlan plan = tile_plan(M, N, K, partial_floats, gated, scaled);
+    if ((K & 63) == 0 && M > 128 && plan.ranges == 1 && !scaled) plan.config = whole_tile(plan.config, M, N, K, output_bytes);
+    kept = Kept{partial_floats, M, N, K, form, plan};
+  }
+  return kept.plan;
+}
+
 // Tilings: 0, 2, 3, 4 the staged kernel at 128x128, 256x128, 128x256, 256x256; 9, 7, 8, 5 the same tiles
 // with the kernel that loads straight into LDS, which needs K to be a multiple of 64; 13 and 15 that kernel at 64x64
 // and 128x64, 14 at 64x64 with the K ranges of one tile in one workgroup (15 always so); and 6 that kernel at
@@ -2470,7 +2488,6 @@ extern "C" int vk_gemm_bf16_tile_plan(int M, int N, int K, long long partial_flo
 extern "C" int vk_gemm_bf16_tile_carried_out(int M, int N, int K, long long partial_floats, int gated, int output_bytes,
                                              int* tiling) {
   if (M <= 0 || N <= 0 || K <= 0) return VK_BAD_ARGUMENT;
-  const TilePlan plan = tile_plan(M, N, K, gated ? 0 : partial_floats, gated != 0, false);
-  *tiling = (K & 63) == 0 && M > 128 && plan.ranges == 1 ? whole_tile(plan.config, M, N, K, gated ? 1.0 : output_bytes) : plan.config;
+  *tiling = carried_out(M, N, K, gated ? 0 : partial_floats, gated != 0, false, gated ? 1.0 : output_bytes).config;
   return 0;
 }
