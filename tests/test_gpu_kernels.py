@@ -138,12 +138,36 @@ def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):
     assert kernels.gemm_bf16_tile_carried_out(m, n, k) == tiling
     out, other = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
     kernels.gemm_bf16(a, w, None, out)
+    assert kernels.gemm_bf16_tile_launched()[0] == tiling
     try:
         kernels.gemm_bf16_force_tiling(kernels.gemm_bf16_tile_plan(m, n, k)[0])
         kernels.gemm_bf16(a, w, None, other)
+        assert kernels.gemm_bf16_tile_launched()[0] == kernels.gemm_bf16_tile_plan(m, n, k)[0]
     finally:
         kernels.gemm_bf16_force_tiling(-1)
     assert torch.equal(out, other)
+
+
+@pytest.mark.parametrize("m,n,k", [(399, 4288, 512), (288, 8320, 1024), (1435, 5440, 256), (695, 5440, 2048), (1805, 8896, 512),
+                                   (512, 1056, 2048), (512, 64, 2048), (330, 7488, 7168), (100, 4608, 3584), (700, 4096, 2040)])
+def test_a_product_launches_the_tile_that_the_plan_names_and_works_it_out_once(m, n, k):
+    """For results of 32 and 16 bits, results added to what is there and gated ones, at sizes where these take different tiles,
+    with and without ranges of K, up to 128 tokens and over a K of no whole steps of 64."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    calls = [(4, False, lambda: kernels.gemm_bf16(a, w, None, torch.empty(m, n, device=DEV))),
+             (2, False, lambda: kernels.gemm_bf16(a, w, None, torch.empty(m, n, dtype=torch.bfloat16, device=DEV))),
+             (8, False, lambda: kernels.gemm_bf16(a, w, None, torch.zeros(m, n, device=DEV), accumulate=True)),
+             (2, True, lambda: kernels.gemm_bf16_gated(a, w, torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)))]
+    for output_bytes, gated, call in calls:
+        call()
+        tiling, ranges, plans = kernels.gemm_bf16_tile_launched()
+        assert tiling == kernels.gemm_bf16_tile_carried_out(m, n, k, gated, output_bytes), (output_bytes, gated)
+        assert ranges == kernels.gemm_bf16_tile_plan(m, n, k, gated)[1], (output_bytes, gated)
+        call()
+        assert kernels.gemm_bf16_tile_launched() == (tiling, ranges, plans), "a plan kept for these sizes was worked out again"
 
 
 @pytest.mark.parametrize("m,n,k,tiling", [(129, 33, 2048, 13), (512, 64, 2048, 13), (161, 1792, 10496, 13), (512, 2048, 512, 14),

@@ -775,6 +775,15 @@ def gemm_bf16_tile_carried_out(m: int, n: int, k: int, gated: bool = False, outp
     return tiling.value
 
 
+def gemm_bf16_tile_launched() -> Tuple[int, int, int]:
+    """For tests: the tiling (a key of ``TILE_TILINGS``; -1: none yet) and the ranges that this thread's last tiled launch took, and
+    how many plans the thread has worked out."""
+    tiling, ranges, plans = _i(), _i(), _ll()
+    fn = _fn("gemm_bf16", "vk_gemm_bf16_tile_launched", [_p, _p, _p])
+    _status(fn(ctypes.addressof(tiling), ctypes.addressof(ranges), ctypes.addressof(plans)), "gemm_bf16_tile_launched")
+    return tiling.value, ranges.value, plans.value
+
+
 def gemm_bf16_force_tiling(tiling: int = -1, ranges: int = 1, stages: int = 0) -> None:
     """For tests and measurements: make the tiled kernel of :func:`gemm_bf16` and :func:`gemm_bf16_gated`
     use one tiling (a key of ``TILE_TILINGS``) and split K into ``ranges``; ``-1`` gives the choice back
