@@ -971,6 +971,68 @@ def test_prompt_tiles_shared_between_workgroups_and_narrow_addresses_give_the_sa
     assert _rel(run(0, None), halved.double()) < 1.2e-2
 
 
+# heads, kv_heads, hd, window, first positions kept, (positions after the step, tokens) of the prompts, positions of single tokens,
+# whether sums may be reordered (no router), the prompts' (chunk, chunks; split), the single tokens' (chunk, chunks, joined)
+DISPATCHED = [
+    (16, 4, 128, 2048, 0, [(6000, 512)], [], True, ((6, 6), 0), None),          # cut by what the window leaves
+    (16, 4, 128, 2048, 130, [(6000, 512)], [], True, ((7, 6), 0), None),
+    (16, 4, 128, 2048, 0, [(6000, 512)], [], False, ((12, 8), 0), None),
+    (4, 1, 256, -1500, 0, [(4000, 200)], [700], False, ((8, 8), 0), (128, 6, False)),
+    (14, 2, 64, 0, 0, [(2000, 100)], [], True, ((4, 8), 0), None),
+    (12, 2, 128, 0, 0, [(3000, 200), (700, 65)], [600, 40], True, ((4, 12), 0), (32, 19, False)),
+    (8, 4, 128, 0, 0, [(333, 333), (200, 17)], [], True, (None, 2), None),      # halved and shared between two workgroups
+    (3, 3, 64, 96, 70, [(500, 300), (65, 65)], [], False, (None, 2), None),
+    (14, 2, 64, 0, 0, [], [512], True, None, (64, 8, True)),                    # short chunks, joined by the workgroup
+    (14, 2, 64, 0, 0, [], [449, 1, 64, 65, 300], True, None, (64, 8, True)),
+    (12, 2, 128, 150, 40, [], [256, 31, 129], True, None, (32, 8, True)),
+    (28, 4, 128, 0, 0, [], [1000, 1, 33, 970, 64, 500, 999, 128], True, None, (64, 16, False)),
+    (14, 2, 64, 200, 0, [], [1500, 3], True, None, (64, 24, False)),
+]
+
+
+@pytest.mark.parametrize("extended", [False, True], ids=["plain", "extended"])
+@pytest.mark.parametrize("case", DISPATCHED, ids=[f"h{c[0]}d{c[2]}w{c[3]}-{i}" for i, c in enumerate(DISPATCHED)])
+def test_paged_attention_with_the_plans_of_known_lengths_and_short_contexts(case, extended):
+    """The dispatch over cut, halved and shared prompt tiles and over short decode chunks, of models with and without a router,
+    against the kernel of 32-bit arithmetic; ``extended``: with a cap, a sink, a bias by distance and a gate."""
+    from types import SimpleNamespace
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.attention import AttentionExtras, paged_attention
+    heads, kv_heads, hd, window, keep, prompts, singles, free, prompt_plan, decode_plan = case
+    entries = prompts + [(kv, 1) for kv in singles]
+    cache = _Paged([kv for kv, _ in entries], kv_heads, hd, 16, torch.bfloat16, seed=hd + heads, stale_nan=True)
+    counts, first = [n for _, n in entries], [kv - n for kv, n in entries]
+    starts = [sum(counts[:e]) for e in range(len(counts) + 1)]
+    g = torch.Generator().manual_seed(heads)
+    qkv = torch.randn(starts[-1], (heads + 2 * kv_heads) * hd, generator=g).to(torch.bfloat16).to(DEV)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    tiles = sorted((first[e] + off, e, off) for e, n in enumerate(counts) if n > 1 for off in range(0, n, 128))
+    reaches = [pos + min(128, counts[e] - off) for pos, e, off in tiles]
+    batch = SimpleNamespace(
+        num_prefill_tiles=len(tiles), prefill_tiles=ints([x for _, e, off in tiles for x in (e, off)]), tile_reaches=reaches,
+        max_tile_reach=max(reaches, default=0), sum_tile_reach=sum(reaches), entry_start=ints(starts), entry_first_pos=ints(first),
+        num_decode_entries=len(singles), decode_entries=ints(list(range(len(prompts), len(entries)))), max_decode_kv_len=max(singles, default=0),
+        sum_decode_kv_len=sum(singles), all_single=not prompts, shared={}, launch_plans=[], free_sum_order=free)
+    table = cache.table
+    if window and not keep:    # what the window has passed has been given back (a layer that keeps first positions keeps all pages)
+        table = cache.with_pages_given_back([max(0, f + 1 - window) if window > 0 else f - f % -window for f in first])
+    k, v, table = cache.k.to(DEV), cache.v.to(DEV), table.to(DEV)
+    extras, cap = AttentionExtras(keep_first=keep), 0.0
+    if extended:
+        extras, cap = AttentionExtras(sink=torch.randn(heads, generator=g).to(DEV), rel=torch.randn(heads, 90, generator=g).to(DEV), keep_first=keep,
+                                      gate=torch.randn(starts[-1], heads, generator=g).to(DEV)), 5.0
+    want, got = (torch.full((starts[-1], heads * hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    kernels.attn_generic(qkv, k, v, want, ints([f + i for f, n in zip(first, counts) for i in range(n)]),
+                         ints([e for e, n in enumerate(counts) for _ in range(n)]), table, heads, kv_heads, hd, hd ** -0.5, window,
+                         softcap=cap, extras=extras)
+    paged_attention(qkv, k, v, got, batch, table, heads, kv_heads, hd, hd ** -0.5, window, cap, extras)
+    assert list(batch.shared.values()) == ([prompt_plan] if prompts else [])
+    assert batch.launch_plans == ([decode_plan] if singles else [])
+    for e in range(len(entries)):
+        rows = slice(starts[e], starts[e + 1])
+        assert _rel(got[rows], want[rows].double()) < 1.2e-2, entries[e]
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", BENCH_HEADS, ids=[f"h{h}kv{k}" for h, k, _ in BENCH_HEADS])
 def test_prompt_attention_at_the_benchmark_head_shapes(heads, kv_heads, hd):
     """One prompt of 2,048 tokens from position 0 and one portion of 512 tokens from position 3,584 in one step."""

@@ -203,6 +203,69 @@ def test_a_plan_of_one_range_takes_the_tile_of_the_least_rounds():
         assert carried(*sizes) == plan(*sizes)[0]       # up to 128 tokens, 64x64 tiles, ranges, no whole steps of 64
 
 
+def _walked(reach, tokens, window, keep_first=0):
+    """Steps that the kernel's walk makes of a tile of so many tokens whose last one sees ``reach`` positions (TileWalk)."""
+    pos = reach - tokens
+    first = (max(pos + 1 - window, 0) if window > 0 else pos - pos % -window if window < 0 else 0) // 64 * 64
+    kept = min((keep_first + 63) // 64, first // 64)
+    return kept + (reach - first + 63) // 64
+
+
+def test_the_steps_of_a_prompt_tile_are_those_of_the_kernels_walk():
+    from vipera_rs_amd.ops.attention import prompt_tile_steps
+    for window, keep in ((0, 0), (1, 0), (64, 0), (100, 7), (512, 64), (512, 65), (512, 4000), (2048, 300), (-64, 0), (-100, 0), (-512, 0)):
+        for reach in (*range(1, 420), *range(1000, 1200), *range(30000, 30200)):
+            steps = prompt_tile_steps(reach, window, keep)
+            assert steps == _walked(reach, min(reach, 128), window, keep)
+            assert steps >= max(_walked(reach, n, window, keep) for n in range(1, min(reach, 128) + 1))
+
+
+def test_cut_prompt_tiles_ask_for_no_more_than_their_walks():
+    """Workgroups and memory are those of the longest walk through the window, and 512 MB of partial results at the most."""
+    import random
+    from vipera_rs_amd.ops.attention import cut_prompt_tiles
+    portion = lambda first, n: [first + min(off + 128, n) for off in range(0, n, 128)]
+    for window, heads in ((2048, 16), (-2048, 16), (4096, 16), (2048, 8), (1024, 4)):
+        for first in (3000, 30000, 120000):
+            for dim in (64, 128, 256):
+                plan = cut_prompt_tiles(portion(first, 512), heads, dim, window, 256)
+                assert plan is None or 4 * heads * plan[1] <= 2 * 256, (window, heads, first, dim, plan)
+    rng = random.Random(7)
+    for _ in range(600):
+        tiles = sorted(rng.randrange(128, rng.choice([400, 4000, 130000])) for _ in range(rng.randrange(1, 120)))
+        heads, window, dim = rng.choice([1, 2, 14]), rng.choice([0, 0, 700, 5000, -3000]), rng.choice([64, 128, 256])
+        keep = rng.choice([0, 4, 1000]) if window > 0 else 0
+        plan = cut_prompt_tiles(tiles, heads, dim, window, 256, keep)
+        if plan is not None:
+            longest = max(_walked(t, 128, window, keep) for t in tiles)
+            assert plan[1] == -(-longest // plan[0]) and len(tiles) * heads * plan[1] * 128 * (dim + 4) * 4 <= 512 << 20
+
+
+def test_the_chunk_of_cut_prompt_tiles_is_the_best_of_all():
+    import random
+    from vipera_rs_amd.ops.attention import PROMPT_COSTS, PROMPT_PARTIAL_BYTES, cut_prompt_tiles, prompt_tile_steps
+    rng = random.Random(11)
+    plans = 0
+    for _ in range(500):
+        tiles = sorted(rng.randrange(1, rng.choice([600, 3000, 30000])) for _ in range(rng.randrange(1, rng.choice([6, 60]))))
+        heads, window, dim, cus = rng.choice([1, 3, 12]), rng.choice([0, 0, 2500, -4000]), rng.choice([64, 128, 256]), rng.choice([256, 304])
+        steps, items = [prompt_tile_steps(t, window) for t in tiles], len(tiles) * heads
+        (alone, beside), one, two = PROMPT_COSTS[dim]
+        best, want = 0.9 * (alone * max(steps) + beside), None
+        for chunk in range(4, max(steps) if items <= cus else 0):
+            groups = heads * sum(-(-s // chunk) for s in steps)
+            cost = one if groups <= cus else two if groups <= 1.7 * cus else None
+            most = -(-max(steps) // chunk)
+            if cost is None or items * most * 128 * (dim + 4) * 4 > PROMPT_PARTIAL_BYTES:
+                continue
+            us = cost[0] * chunk + cost[1] + cost[2] * groups
+            if us < best:
+                best, want = us, (chunk, most)
+        assert cut_prompt_tiles(tiles, heads, dim, window, cus) == want
+        plans += want is not None
+    assert plans > 100
+
+
 def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
     """Chunks as long as one another are few enough to run at once, never leave a position out and never outnumber what was
     allowed for."""
@@ -222,7 +285,7 @@ def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
         plan = cut_prompt_tiles(tiles, heads, rng.choice([64, 128, 256]), window, 256)
         if plan is not None:
             chunk, most = plan
-            assert chunk >= 4 and chunk * most * 64 >= max(tiles)
+            assert chunk >= 4 and chunk * most >= max(_walked(t, n, window) for t in tiles for n in (1, 64, 127, 128) if n <= t)
             if not window:
                 assert heads * sum(-(-t // (64 * chunk)) for t in tiles) <= 2 * 256
 

@@ -164,43 +164,66 @@ PROMPT_COSTS = {64: ((0.66, 4.8), (0.96, 10.7, 0.015), (0.95, 17.0, 0.015)), 128
                 256: ((3.1, 6.0), (2.84, 13.6, 0.027), None)}
 
 
-def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int):
+PROMPT_PARTIAL_BYTES = 512 << 20   # the most that the partial results of cut prompt tiles may take
+
+
+def prompt_tile_steps(reach: int, window: int, keep_first: int = 0) -> int:
+    """The steps of 64 positions that the prompt kernel walks for a tile of 128 tokens whose last one sees ``reach`` positions (no
+    window counted), and the most for a shorter tile that ends there: those from the first position that the tile's first
+    token sees on, and those of the ``keep_first`` first positions that stay visible (``TileWalk`` in ``attn_bf16.hip``)."""
+    pos = max(reach - 128, 0)
+    first = max(pos + 1 - window, 0) if window > 0 else pos - pos % -window if window < 0 else 0
+    return -(-reach // 64) - max(0, first // 64 - -(-keep_first // 64))
+
+
+def _cut_workgroups(steps, heads: int, chunk: int) -> int:
+    return heads * sum(-(-s // chunk) for s in steps)
+
+
+def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int, keep_first: int = 0):
     """:func:`chunks_prompt_tiles` where the tiles' lengths are known one by one (``reaches``: the positions that the last token
     of each sees, no window counted): the chunk length whose workgroups, counted tile by tile, are at most one a CU, or 1.7 a
     CU (two, less what the XCDs differ by: one more runs behind all others), and that takes the least time by this estimate, if
     that is less than nine tenths of what the tiles take uncut.  us a layer, uncut (halved) against cut, the merge included: four tiles of 16
     heads of 128 that end at 1,664 to 2,048 positions 47.7 / 30.3; twelve of 12 heads that end at 1,322 to 3,983 87.0 / 52.2;
     the sixteen of one prompt of 2,048, 12 heads, 47.4 / 39.8; two of 14 heads of 64 at 2,000 32.7 / 15.0; and left uncut: eight
-    and seven tiles of 1,000 and 834 tokens, 16 heads, 29.2 / 31.6; a prompt of 2,048 at 28 heads 63.2 / 69.5."""
+    and seven tiles of 1,000 and 834 tokens, 16 heads, 29.2 / 31.6; a prompt of 2,048 at 28 heads 63.2 / 69.5.
+
+    Every tile is given the chunks of the longest one, workgroups and partial results: no chunk is so short that these come to
+    more than ``PROMPT_PARTIAL_BYTES`` (many shallow tiles beside a deep one), and a window counts as what the walk through it
+    makes (512 tokens of 16 heads of 128 behind 30,000 positions, a window of 2,048: with chunks for the whole reach 39.7 us a
+    layer and 330 MB, so 32.5 and 26; behind 120,000 83.5 and 32.4 us)."""
     items = len(reaches) * heads
     costs = PROMPT_COSTS.get(head_dim)
     if items <= 0 or items > cus or costs is None:
         return None
-    seen = [min(r, abs(window) + 128) if window else r for r in reaches]
-    steps = [(r + 63) // 64 for r in seen]
+    steps = [prompt_tile_steps(r, window, keep_first) for r in reaches]
     longest = max(steps)
+    most_chunks = PROMPT_PARTIAL_BYTES // (items * 128 * (head_dim + kernels.ATTN_PREFILL_PARTIAL_ROW_EXTRA) * 4)
+    if most_chunks < 2:
+        return None
+    shortest = max(4, -(-longest // most_chunks))
     (alone, alone_beside), one, two = costs
     best, chosen = 0.9 * (alone * longest + alone_beside), None
-    for chunk in range(4, longest):
-        counts = [-(-s // chunk) for s in steps]
-        groups = heads * sum(counts)
+    for chunk in range(shortest, longest):
+        groups = _cut_workgroups(steps, heads, chunk)
         cost = one if groups <= cus else two if groups <= 1.7 * cus else None
         if cost is None:
             continue
         us = cost[0] * chunk + cost[1] + cost[2] * groups
         if us < best:
             best, chosen = us, chunk
-    return None if chosen is None else (chosen, -(-((max(reaches) + 63) // 64) // chosen))
+    return None if chosen is None else (chosen, -(-longest // chosen))
 
 
-def _prompt_plan(batch, k_cache, heads: int, kv_heads: int, head_dim: int, window: int, cus: int):
+def _prompt_plan(batch, k_cache, heads: int, kv_heads: int, head_dim: int, window: int, keep_first: int, cus: int):
     """``(chunk_tiles and max_chunks, or None; 0, or 1 where tiles are halved, or 2 where two workgroups share such a tile's
     tokens)``, once for a step's layers of one geometry.  Two where the tiles are no more than the CUs: the same bits in 0.75
     to 1 of the time (see attn_prefill_direct_kernel; 448 tiles on 256 CUs 57 and 81 us)."""
     chunked = None
     if kernels.attn_bf16_prefill_loads_directly(k_cache, kv_heads, head_dim):
         if getattr(batch, "free_sum_order", False):
-            chunked = cut_prompt_tiles(batch.tile_reaches, heads, head_dim, window, cus)
+            chunked = cut_prompt_tiles(batch.tile_reaches, heads, head_dim, window, cus, keep_first)
         else:
             chunked = chunks_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach, batch.sum_tile_reach, cus)
     if chunked is not None or not halves_prompt_tiles(batch.num_prefill_tiles, heads, batch.max_tile_reach,
@@ -218,9 +241,11 @@ def paged_attention(qkv, k_cache, v_cache, out, batch, table, heads, kv_heads, h
         extras = None
     if kernels.attn_bf16_supported(qkv, k_cache, head_dim):
         if batch.num_prefill_tiles:
-            key = ("prompt tiles", heads, kv_heads, head_dim, window, k_cache.shape[2])
+            keep_first = extras.keep_first if extras is not None else 0
+            key = ("prompt tiles", heads, kv_heads, head_dim, window, keep_first, k_cache.shape[2])
             if key not in batch.shared:
-                batch.shared[key] = _prompt_plan(batch, k_cache, heads, kv_heads, head_dim, window, kernels.compute_units(qkv.device))
+                batch.shared[key] = _prompt_plan(batch, k_cache, heads, kv_heads, head_dim, window, keep_first,
+                                                 kernels.compute_units(qkv.device))
             chunked, split = batch.shared[key]
             kernels.attn_bf16_prefill(qkv, k_cache, v_cache, out, batch.prefill_tiles, batch.entry_start,
                                       batch.entry_first_pos, table, heads, kv_heads, head_dim, scale, window, split,
