@@ -266,6 +266,18 @@ def test_the_chunk_of_cut_prompt_tiles_is_the_best_of_all():
     assert plans > 100
 
 
+def test_a_cut_of_prompt_tiles_is_found_in_a_few_looks_however_deep(monkeypatch):
+    from vipera_rs_amd.ops import attention
+    looks = []
+    counted = attention._cut_workgroups
+    monkeypatch.setattr(attention, "_cut_workgroups", lambda *a: looks.append(1) or counted(*a))
+    for reach in (500, 2048, 8192, 32768, 131072):
+        for tiles, heads, dim in ((16, 14, 64), (4, 12, 128), (16, 1, 128), (19, 4, 256), (1, 28, 128)):
+            looks.clear()
+            attention.cut_prompt_tiles([max(128, reach - 128 * i) for i in range(tiles)], heads, dim, 0, 256)
+            assert len(looks) <= 40, (reach, tiles, heads, dim, len(looks))
+
+
 def test_prompt_tiles_of_known_lengths_are_cut_where_it_pays():
     """Chunks as long as one another are few enough to run at once, never leave a position out and never outnumber what was
     allowed for."""

@@ -192,7 +192,8 @@ def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int, 
     Every tile is given the chunks of the longest one, workgroups and partial results: no chunk is so short that these come to
     more than ``PROMPT_PARTIAL_BYTES`` (many shallow tiles beside a deep one), and a window counts as what the walk through it
     makes (512 tokens of 16 heads of 128 behind 30,000 positions, a window of 2,048: with chunks for the whole reach 39.7 us a
-    layer and 330 MB, so 32.5 and 26; behind 120,000 83.5 and 32.4 us)."""
+    layer and 330 MB, so 32.5 and 26; behind 120,000 83.5 and 32.4 us).  Workgroups only fall as chunks grow, so that the
+    shortest chunk that keeps to either limit is found by halving, and a few more beyond it may be shorter still."""
     items = len(reaches) * heads
     costs = PROMPT_COSTS.get(head_dim)
     if items <= 0 or items > cus or costs is None:
@@ -205,14 +206,23 @@ def cut_prompt_tiles(reaches, heads: int, head_dim: int, window: int, cus: int, 
     shortest = max(4, -(-longest // most_chunks))
     (alone, alone_beside), one, two = costs
     best, chosen = 0.9 * (alone * longest + alone_beside), None
-    for chunk in range(shortest, longest):
-        groups = _cut_workgroups(steps, heads, chunk)
-        cost = one if groups <= cus else two if groups <= 1.7 * cus else None
-        if cost is None:
-            continue
-        us = cost[0] * chunk + cost[1] + cost[2] * groups
-        if us < best:
-            best, chosen = us, chunk
+    if best <= min(cost[0] * shortest + cost[1] for cost in (one, two) if cost is not None):
+        return None
+
+    def shortest_within(limit):
+        low, high = max(shortest, -(-heads * sum(steps) // limit)), longest
+        while low < high:
+            middle = (low + high) // 2
+            low, high = (low, middle) if _cut_workgroups(steps, heads, middle) <= limit else (middle + 1, high)
+        return low
+
+    alone_from = shortest_within(cus)     # from here on a CU has one workgroup at the most
+    for cost, chunk, end in ((two, shortest_within(int(1.7 * cus)), alone_from), (one, alone_from, longest)):
+        while cost is not None and chunk < end and cost[0] * chunk + cost[1] + cost[2] * items < best:
+            us = cost[0] * chunk + cost[1] + cost[2] * _cut_workgroups(steps, heads, chunk)
+            if us < best:
+                best, chosen = us, chunk
+            chunk += 1
     return None if chosen is None else (chosen, -(-longest // chosen))
 
 
