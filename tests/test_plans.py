@@ -315,3 +315,36 @@ def test_few_requests_of_short_contexts_take_short_chunks():
             if plan is not None:
                 chunk, chunks, join = plan
                 assert chunk % 32 == 0 and chunk * chunks >= length and (chunks <= 8 if join else chunks <= 64)
+
+
+def test_attention_keeps_the_order_of_its_sums_in_every_model_that_may_route():
+    from types import SimpleNamespace
+    import gilidra_helpers
+    import helpers
+    import lurirax_helpers
+    import muzasun_helpers
+    import rebidra_helpers
+    import zeladra_helpers
+    import zulesun_helpers
+    from vipera_rs_amd.config import config_from_dict
+    from vipera_rs_amd.models.decoder import routes_tokens
+    from vipera_rs_amd.parts import FeedForward, register_ffn, unregister
+    seen = set()
+    for data in (helpers.CONFIG_B, gilidra_helpers.G1, gilidra_helpers.G2, lurirax_helpers.L1, lurirax_helpers.L2, muzasun_helpers.M1,
+                 muzasun_helpers.M2, rebidra_helpers.R1, rebidra_helpers.R2, zeladra_helpers.Z1, zulesun_helpers.Z1):
+        config = config_from_dict(data)
+        routed = any(spec.ffn is not None and "experts" in spec.ffn.params for spec in config.layer_specs())
+        assert routes_tokens(config) == routed, config.architecture
+        seen.add(routed)
+    assert seen == {True, False}
+
+    class Unsaid(FeedForward):
+        pass
+
+    register_ffn("unsaid", Unsaid)
+    try:
+        layers = [SimpleNamespace(ffn=SimpleNamespace(kind=kind)) for kind in ("gated_mlp", "mlp", "none")] + [SimpleNamespace(ffn=None)]
+        assert not routes_tokens(SimpleNamespace(layer_specs=lambda: layers))
+        assert routes_tokens(SimpleNamespace(layer_specs=lambda: layers + [SimpleNamespace(ffn=SimpleNamespace(kind="unsaid"))]))
+    finally:
+        unregister("ffn", "unsaid")

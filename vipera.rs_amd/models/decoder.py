@@ -109,6 +109,11 @@ def declare_cache_needs(config: ModelConfig) -> List[CacheNeed]:
     return needs
 
 
+def routes_tokens(config: ModelConfig) -> bool:
+    """Whether any layer's feed-forward may choose among experts (:attr:`FeedForward.routes`), from the configuration alone."""
+    return any(spec.ffn is not None and part_class("ffn", spec.ffn.kind).routes for spec in config.layer_specs())
+
+
 class DecoderModel:
     def __init__(self, config: ModelConfig, runtime):
         self.config = config
@@ -126,8 +131,7 @@ class DecoderModel:
         if self.rejoin is None and any(entry.rejoins for entry in self.schedule):
             raise InvalidArgumentError("the run order has entries that rejoin the embedding's output, but no part that does it")
         self.vocab_size = self.head.vocab
-        self.routes = any(spec.ffn is not None and getattr(part_class("ffn", spec.ffn.kind), "routes", False)
-                          for spec in config.layer_specs())
+        self.routes = routes_tokens(config)
         self.loaded = False
 
     def tensor_specs(self) -> List[TensorSpec]:

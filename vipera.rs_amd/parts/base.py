@@ -192,6 +192,10 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    #: whether it may choose among experts by its input: the closest of such choices turn on the last bits of what comes
+    #: before them, so attention keeps the order of its sums in a model that has one.  A part that makes none says so.
+    routes = True
+
     #: as :attr:`Mixer.can_overwrite`
     can_overwrite = False
 

@@ -105,6 +105,7 @@ class TokenSide(FeedForward):
     has it at hand (``wants_stream``), else it is made here.  ``params``: ``hidden``,
     ``dim``, ``index``, ``eps``, ``activation`` ("gelu_tanh" unless given), ``name``; tensors ``<name>.gate | proj | norm``."""
 
+    routes = False
     applies_following = True
 
     def __init__(self, spec: PartSpec, prefix: str, runtime):

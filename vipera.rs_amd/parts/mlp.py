@@ -23,6 +23,8 @@ class GatedMLP(FeedForward):
     """``params``: ``hidden``, ``intermediate``, ``name``; tensors ``<name>.gate_proj.weight | up_proj.weight |
     down_proj.weight``, or as ``params["tensors"]`` names them (keys ``gate``, ``up``, ``down``)."""
 
+    routes = False
+
     @staticmethod
     def _names(spec: PartSpec, prefix: str):
         names = {"gate": "gate_proj.weight", "up": "up_proj.weight", "down": "down_proj.weight"}
@@ -109,6 +111,8 @@ class GatedMLP(FeedForward):
 class NoFeedForward(FeedForward):
     """A layer without a feed-forward: adds nothing."""
 
+    routes = False
+
     def forward(self, h, batch, residual, **_unused) -> None:
         return None
 
@@ -118,6 +122,7 @@ class PlainMLP(FeedForward):
     the square of relu; "silu"; "gelu_tanh"), ``name``; tensors ``<name>.up`` and ``<name>.down`` (or as
     ``params["tensors"]`` names them)."""
 
+    routes = False
     can_overwrite = True
 
     def __init__(self, spec: PartSpec, prefix: str, runtime):

@@ -42,8 +42,6 @@ class MixtureOfExperts(FeedForward):
     "plain"), ``activation`` (of the plain form), ``router_bias``, ``name``; tensors ``<name>.router``,
     ``<name>.e<i>.gate | up | down`` and ``<name>.shared.gate | up | down``."""
 
-    routes = True
-
     def __init__(self, spec: PartSpec, prefix: str, runtime):
         super().__init__(spec, prefix, runtime)
         p = spec.params
