@@ -354,8 +354,9 @@ __global__ __launch_bounds__(64) void attn_combine_f32_kernel(const float* __res
 // while this one's softmax runs; what the matrix instruction wants of a lane (one k of four) comes out of two lane
 // exchanges a register pair. Only scores and weights go through LDS, in two buffers, two barriers a tile. Positions past the
 // tokens' last one and those before the first one that the first token sees (a window has passed them, their page may have
-// been given back and its id in the table is then -1) are read at the last position instead; their scores are masked and
-// their values count as zeros (a weight of zero times whatever a free slot holds must stay zero).
+// been given back and its id in the table is then -1) are read at a place of the tile that is held (stand_in: the first one that
+// is seen, the last first position that stays visible, or the tokens' last one); their scores are masked and their values
+// count as zeros (a weight of zero times whatever a free slot holds must stay zero).
 //
 // What bounds it: a few hundred tokens have little to multiply (333 tokens of 14 heads of 64: 0.2 GFLOP a layer, 1.3 us of
 // the chip), and their last tokens' walk takes some 2.6 us a tile, one wave a SIMD issuing some 600 instructions; long prompts
@@ -625,9 +626,10 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
 }
 
 // 16-token blocks of a workgroup for a step of `items` pairs (64 tokens, head): one while those are about one workgroup a CU,
-// two above, which read the keys and values half as often. us with one / two (and with four, slower at every size):
-// 140 tokens, 12 heads of 128 (48 items) 13.1 / 17.6; 333, 14 heads of 64 (84) 18.8 / 20.4; 400, 12 of 128 (96) 37.7 / 34.4;
-// 512 behind 1,000, 14 of 64 (112) 70.0 / 68.5; 4,096, 28 of 128 (1,792) 2,231 / 1,971.
+// two above, which read the keys and values half as often. us with one / two (and with four, slower at every size), from
+// position 0: 12 heads of 128 16.3 / 22.7 (48 items), 34.3 / 35.5 (84), 41.2 / 39.2 (96), 28 of them 2,231 / 1,971 (1,792); behind
+// 1,000 positions 61.5 / 88.4, 104.5 / 101.7, 111.6 / 105.2. One line for all widths: heads of 96 cross at the same place, narrower
+// ones later (14 of 64 behind 1,000 60.0 / 62.5 at 84 items, 62.8 / 65.2 at 98, 67.0 / 67.6 at 112; 8 of 32 58.9 / 64.8 at 96).
 inline int prefill_f32_row_blocks(long long items) { return items <= 90 ? 1 : 2; }
 
 template <int DPT>

@@ -3,7 +3,7 @@
 A bfloat16 run whose head width and page size allow 16-byte reads uses the matrix-core kernels: one
 launch for the tiles of multi-token entries (prompt portions), one (plus the merge) for the entries
 that hold a single token, whose positions are split into chunks.  The 32-bit run has a split kernel for
-single tokens too (chunks of 256 positions) and a tiled one for prompt portions (64 tokens of a head a
+single tokens too (chunks of 256 positions) and a tiled one for prompt portions (16 or 32 tokens of a head a
 workgroup); everything of odd sizes uses the general 32-bit kernel, which serves both kinds alike.
 """
 from __future__ import annotations
