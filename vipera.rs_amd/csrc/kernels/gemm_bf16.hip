@@ -433,6 +433,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const __bf16* _
 // STAGES 3 (for up to 128 tokens, where the product is a stream of the weights and a CU's bytes in flight are
 // what bounds it): step s + 3 is requested when step s's stage is free, and the barrier of a step waits for
 // step s + 1 only, so the loads of two steps are in flight instead of one; STAGES 4 likewise.
+// W_STAGES: stages of the weight's rows alone, which come from memory where the activations' come from a cache, each read by
+// all workgroups of its row of tiles: 256x256 tiles leave room for a third one, and their step of K, which waited for the
+// weights (1.5 us, of which the matrix cores work 0.9), has two steps' time for them. A step's weights are requested behind its
+// activations, so at the barrier the newest request of weights may stay in flight. Weights from memory, two stages to three: gate/up
+// of 2,048 tokens on 37,888 rows of 3,584 456 to 426 us (1.31 PFLOP/s), of 1,000 tokens 257 to 240, 1,396 on 17,920 of 1,536
+// 79.3 to 77.2; 256x192 tiles: 2,048 on 6,144 rows of 2,048 47.8 to 45.5, on 3,584 of 18,944 350 to 288; 128x128 tiles, two to a
+// CU: 1,396 on 17,920 of 1,536 92.1 to 88.2, on 1,536 of 8,960 115 to 98. No faster with a third one: 256x128 (three of both: 240
+// us either way at 3,584 rows of 18,944), 192x192; slower: the weights' loads spread over the other half of the step.
 // group_tile_direct (group_tile.h) is the same loop over gathered rows; a change to one is to be weighed for the other.
 constexpr int DIRECT_ROW = BK * 2;  // bytes per LDS row
 
@@ -447,7 +455,8 @@ __device__ __forceinline__ void wait_own_loads_but() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
-template <int BM, int BN, int WM, int WN, typename TC, bool ACCUMULATE, bool GATED, int STAGES = 2, bool FOLD = false>
+template <int BM, int BN, int WM, int WN, typename TC, bool ACCUMULATE, bool GATED, int STAGES = 2, bool FOLD = false,
+          int W_STAGES = STAGES>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __bf16* __restrict__ A,
                                                                           const __bf16* __restrict__ W,
                                                                           const float* __restrict__ bias,
@@ -463,10 +472,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
   constexpr int A_LOADS = BM / 8 / WAVES, W_LOADS = BN / 8 / WAVES;  // load instructions per wave and step
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide among the waves' loads");
-  constexpr int STAGE = (BM + BN) * DIRECT_ROW;
-  constexpr int LOADS = A_LOADS + W_LOADS;
+  constexpr int A_STAGE = BM * DIRECT_ROW, W_STAGE = BN * DIRECT_ROW, W_BASE = STAGES * A_STAGE;
+  constexpr int LOADS = A_LOADS + W_LOADS, W_MORE = W_STAGES - STAGES, W_AHEAD = W_MORE * W_LOADS;
   static_assert(STAGES >= 2 && STAGES <= 4, "two to four LDS stages");
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];  // [STAGES][BM + BN][128]
+  static_assert(W_MORE == 0 || W_MORE == 1, "at most one stage more for the weight");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];  // [STAGES][BM][128], [W_STAGES][BN][128]
 
   const int total = tiles_m * tiles_n;
   const int per_xcd = (total + XCDS - 1) / XCDS;
@@ -499,27 +509,30 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
 #pragma unroll
   for (int i = 0; i < W_LOADS; ++i)
     w_off[i] = (unsigned)((((size_t)(wave * W_LOADS + i) * 8 + ld_row) * K + ld_chunk * 8 + k_begin) * 2);
-  auto issue_loads = [&](int stage, int step) {
-    unsigned char* to_a = lds_raw + stage * STAGE + wave * A_LOADS * 1024;
-    unsigned char* to_w = lds_raw + stage * STAGE + BM * DIRECT_ROW + wave * W_LOADS * 1024;
+  auto issue_a = [&](int stage, int step) {
+    unsigned char* to = lds_raw + stage * A_STAGE + wave * A_LOADS * 1024;
     const unsigned kb = (unsigned)step * (BK * 2);
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_view.rsrc, (lds_ptr)(to_a + i * 1024), 16, (int)(a_off[i] + kb), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_view.rsrc, (lds_ptr)(to + i * 1024), 16, (int)(a_off[i] + kb), 0, 0, 0);
+  };
+  auto issue_w = [&](int stage, int step) {
+    unsigned char* to = lds_raw + W_BASE + stage * W_STAGE + wave * W_LOADS * 1024;
+    const unsigned kb = (unsigned)step * (BK * 2);
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_view.rsrc, (lds_ptr)(to_w + i * 1024), 16, (int)(w_off[i] + kb), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_view.rsrc, (lds_ptr)(to + i * 1024), 16, (int)(w_off[i] + kb), 0, 0, 0);
   };
   // a lane's fragment chunks within a stage: row lr of each 16-row tile, chunk lg (first half of the step)
   // or lg + 4 (second half), which differ in bit 6 of the byte offset
   const unsigned frag_a = (unsigned)((wm * TM * 16 + lr) * DIRECT_ROW + ((lg ^ (lr & 7)) * 16));
-  const unsigned frag_w = (unsigned)(BM * DIRECT_ROW + (wn * TN * 16 + lr) * DIRECT_ROW + ((lg ^ (lr & 7)) * 16));
-  auto read_fragments = [&](int stage, int half, bf16x8 (&fa)[TM], bf16x8 (&fw)[TN]) {
-    const unsigned char* base = lds_raw + stage * STAGE;
+  const unsigned frag_w = (unsigned)(W_BASE + (wn * TN * 16 + lr) * DIRECT_ROW + ((lg ^ (lr & 7)) * 16));
+  auto read_fragments = [&](int a_stage, int w_stage, int half, bf16x8 (&fa)[TM], bf16x8 (&fw)[TN]) {
+    const unsigned char *a_base = lds_raw + a_stage * A_STAGE, *w_base = lds_raw + w_stage * W_STAGE;
 #pragma unroll
-    for (int t = 0; t < TN; ++t) fw[t] = *(const bf16x8*)(base + (frag_w ^ (half * 64)) + t * 16 * DIRECT_ROW);
+    for (int t = 0; t < TN; ++t) fw[t] = *(const bf16x8*)(w_base + (frag_w ^ (half * 64)) + t * 16 * DIRECT_ROW);
 #pragma unroll
-    for (int t = 0; t < TM; ++t) fa[t] = *(const bf16x8*)(base + (frag_a ^ (half * 64)) + t * 16 * DIRECT_ROW);
+    for (int t = 0; t < TM; ++t) fa[t] = *(const bf16x8*)(a_base + (frag_a ^ (half * 64)) + t * 16 * DIRECT_ROW);
   };
   auto multiply = [&](const bf16x8 (&fa)[TM], const bf16x8 (&fw)[TN]) {
 #pragma unroll
@@ -531,19 +544,25 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
 
   const int steps = (k_end - k_begin) / BK;
   bf16x8 fa0[TM], fw0[TN], fa1[TM], fw1[TN];
-  __shared__ float part_sums[WAVES * 64];
-  issue_loads(0, 0);
+  float* part_sums = (float*)lds_raw;   // with a stage more for the weight, the norm's sums follow when the stages are done with
+  if constexpr (W_MORE == 0) {
+    __shared__ float sums[WAVES * 64];
+    part_sums = sums;
+  }
+  if constexpr (W_MORE > 0) issue_w(0, 0);
 #pragma unroll
-  for (int i = 1; i < STAGES; ++i)
-    if (steps > i) issue_loads(i, i);
-  tile_norm_parts<BM, WAVES * 64>(norm, m0, M, tid, part_sums);  // behind the first requests, before the first wait
-  if (STAGES > 2 && steps >= STAGES) {
-    wait_own_loads_but<(STAGES > 2 ? STAGES - 1 : 0) * LOADS>();  // step 0 has arrived; the others stay in flight
+  for (int i = 0; i < STAGES; ++i) {
+    if (steps > i) issue_a(i, i);
+    if (steps > i + W_MORE) issue_w(i + W_MORE, i + W_MORE);
+  }
+  if constexpr (W_MORE == 0) tile_norm_parts<BM, WAVES * 64>(norm, m0, M, tid, part_sums);  // behind the first requests, before the first wait
+  if (steps >= W_STAGES) {
+    wait_own_loads_but<(STAGES - 1) * LOADS + W_AHEAD>();  // step 0 has arrived; the others stay in flight
   } else {
     wait_own_loads();
   }
   __syncthreads();
-  read_fragments(0, 0, fa0, fw0);
+  read_fragments(0, 0, 0, fa0, fw0);
   // Hints for the instruction order within a half step: the LDS reads and the loads go out one by one
   // between products, so that their issue hides behind the matrix core's work instead of stalling it.
   auto interleave = [](auto lds_reads, auto loads) {
@@ -558,24 +577,31 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
     });
     __builtin_amdgcn_sched_group_barrier(0x008, TM * TN, 0);
   };
-  // `in_flight`: how many later steps' loads may stay in flight at the barrier (all of a step's loads that were
-  // issued before them have then arrived)
-  auto step = [&](int s, int stage, auto with_loads, auto with_next, auto in_flight) {
-    const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
-    read_fragments(stage, 1, fa1, fw1);
+  // with_loads: 0 none, 1 the activations' where they still have a step to come, 2 both operands'. `in_flight`: how many of the
+  // wave's last loads may stay in flight at the barrier (all of step s + 1 were issued before them and have then arrived)
+  auto step = [&](int s, int a_stage, int w_stage, auto with_loads, auto with_next, auto in_flight) {
+    constexpr int LOADING = decltype(with_loads)::value;
+    const int a_next = a_stage + 1 == STAGES ? 0 : a_stage + 1, w_next = w_stage + 1 == W_STAGES ? 0 : w_stage + 1;
+    read_fragments(a_stage, w_stage, 1, fa1, fw1);
     multiply(fa0, fw0);
     interleave(std::integral_constant<int, TM + TN>{}, std::integral_constant<int, 0>{});
     __builtin_amdgcn_sched_barrier(0);  // the products stay on this side: they cover the reads above
-    wait_own_loads_but<decltype(in_flight)::value * LOADS>();
+    wait_own_loads_but<decltype(in_flight)::value>();
     __syncthreads();
-    if constexpr (decltype(with_loads)::value) issue_loads(stage, s + STAGES);
-    if constexpr (decltype(with_next)::value) read_fragments(next_stage, 0, fa0, fw0);
+    if constexpr (LOADING == 1) {
+      if (s + STAGES < steps) issue_a(a_stage, s + STAGES);
+    }
+    if constexpr (LOADING == 2) {
+      issue_a(a_stage, s + STAGES);
+      issue_w(w_stage, s + W_STAGES);
+    }
+    if constexpr (decltype(with_next)::value) read_fragments(a_next, w_next, 0, fa0, fw0);
     multiply(fa1, fw1);
     interleave(std::integral_constant<int, decltype(with_next)::value ? TM + TN : 0>{},
-               std::integral_constant<int, decltype(with_loads)::value ? LOADS : 0>{});
+               std::integral_constant<int, LOADING == 2 ? LOADS : 0>{});
     __builtin_amdgcn_sched_barrier(0);
   };
-  int s = 0, stage = 0;
+  int s = 0, stage = 0, w_stage = 0;
   // FOLD: the sums of every k_per_range of K are added up as gemm_reduce_kernel adds the partial sums of as many workgroups
   f32x4 folded[FOLD ? TN : 1][FOLD ? TM : 1];
   int fold_at = k_per_range / BK;
@@ -596,6 +622,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
   };
   auto advance = [&]() {
     stage = stage + 1 == STAGES ? 0 : stage + 1;
+    w_stage = w_stage + 1 == W_STAGES ? 0 : w_stage + 1;
     if constexpr (FOLD) {
       if (s == fold_at) {
         fold();
@@ -603,16 +630,24 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
       }
     }
   };
-  for (; s + STAGES < steps; ++s, advance())   // with three stages the step after next stays in flight
-    step(s, stage, std::true_type{}, std::true_type{}, std::integral_constant<int, STAGES - 2>{});
+  for (; s + W_STAGES < steps; ++s, advance())   // with three stages the step after next stays in flight
+    step(s, stage, w_stage, std::integral_constant<int, 2>{}, std::true_type{},
+         std::integral_constant<int, (STAGES - 2) * LOADS + W_AHEAD>{});
   for (; s + 1 < steps; ++s, advance())
-    step(s, stage, std::false_type{}, std::true_type{}, std::integral_constant<int, 0>{});
-  step(s, stage, std::false_type{}, std::false_type{}, std::integral_constant<int, 0>{});
+    step(s, stage, w_stage, std::integral_constant<int, W_MORE>{}, std::true_type{}, std::integral_constant<int, 0>{});
+  step(s, stage, w_stage, std::integral_constant<int, 0>{}, std::false_type{}, std::integral_constant<int, 0>{});
   if constexpr (FOLD) {
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] = folded[i][j] + acc[i][j];
+  }
+  if constexpr (W_MORE > 0) {
+    if (norm.sumsq) {
+      __syncthreads();   // nobody reads a stage any more, and no load into one is in flight
+      tile_norm_parts<BM, WAVES * 64>(norm, m0, M, tid, part_sums);
+      __syncthreads();
+    }
   }
 
   tile_epilogue<BM, WAVES * 64, TM, TN, TC, ACCUMULATE, GATED>(acc, C, ldc, M, N, K, bias, (vector_ok & 1) != 0,
@@ -1767,20 +1802,22 @@ int launch_mid(const __bf16* A, const __bf16* W, const float* bias, TC* C, float
 
 int g_tile_group_m = 0;   // 0: chosen by shape; else the rows of tiles per block of tile_of, for measurements
 
-template <bool DIRECT, int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, int STAGES, bool FOLD = false>
+template <bool DIRECT, int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, int STAGES, bool FOLD = false, int W_STAGES = STAGES>
 constexpr auto tile_kernel() {
-  if constexpr (DIRECT) return gemm_tile_direct_kernel<BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD>;
+  if constexpr (DIRECT) return gemm_tile_direct_kernel<BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD, W_STAGES>;
   else return gemm_tile_kernel<BM, BN, WM, WN, TC, ACC, GATED>;
 }
 
-// DIRECT: the kernel that loads straight into LDS; K must be a multiple of 64. STAGES: its LDS stages.
-// FOLD: one workgroup a tile adds up its K ranges itself.
-template <int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, bool DIRECT = false, int STAGES = 2, bool FOLD = false>
+// DIRECT: the kernel that loads straight into LDS; K must be a multiple of 64. STAGES: its LDS stages, W_STAGES: those of
+// the weight's rows. FOLD: one workgroup a tile adds up its K ranges itself.
+template <int BM, int BN, int WM, int WN, typename TC, bool ACC, bool GATED, bool DIRECT = false, int STAGES = 2, bool FOLD = false,
+          int W_STAGES = STAGES>
 int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, int M, int N, int K, long long lda,
                    long long ldc, int vector_ok, int ranges, float* partial, hipStream_t s, const TileNorm& norm) {
-  static_assert(DIRECT || STAGES == 2, "only the direct kernel has a third stage");
-  constexpr int lds_bytes = DIRECT ? STAGES * (BM + BN) * DIRECT_ROW : 2 * (BM + BN) * ROW * (int)sizeof(__bf16);
-  static_assert(lds_bytes + WM * WN * 64 * 4 <= 160 * 1024, "a CU has 160 KB of LDS (the stages and the norm's sums)");
+  static_assert(DIRECT || W_STAGES == 2, "only the direct kernel has a third stage");
+  constexpr int lds_bytes = DIRECT ? (STAGES * BM + W_STAGES * BN) * DIRECT_ROW : 2 * (BM + BN) * ROW * (int)sizeof(__bf16);
+  constexpr int norm_bytes = W_STAGES > STAGES ? 0 : WM * WN * 64 * 4;
+  static_assert(lds_bytes + norm_bytes <= 160 * 1024, "a CU has 160 KB of LDS (the stages and the norm's sums)");
   if (WM * WN * 64 % BM != 0 && norm.sumsq) return VK_UNSUPPORTED_SIZE;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const long long total = (long long)tiles_m * tiles_n;
@@ -1793,7 +1830,7 @@ int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, i
   const int k_per_range = ((K + ranges - 1) / ranges + BK - 1) / BK * BK;
   if (ranges <= 1 || GATED || FOLD) {
     static bool configured = false;
-    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD>();
+    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, TC, ACC, GATED, STAGES, FOLD, W_STAGES>();
     if (!configured) {
       hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (e != hipSuccess) return (int)e;
@@ -1807,7 +1844,7 @@ int launch_tile_as(const __bf16* A, const __bf16* W, const float* bias, TC* C, i
   // K split over workgroups: float partial sums [range, M, N], then the ranges are added in ascending order
   if constexpr (!GATED) {
     static bool configured_partial = false;
-    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, float, false, false, STAGES>();
+    auto kernel = tile_kernel<DIRECT, BM, BN, WM, WN, float, false, false, STAGES, false, W_STAGES>();
     if (!configured_partial) {
       hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (e != hipSuccess) return (int)e;
@@ -2121,9 +2158,12 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
     case 20: VK_TILE_WHOLE(192, 192, 3);
   }
 #undef VK_TILE_WHOLE
+#define VK_TILE_W3(BMV, BNV)                                                                                          \
+  return launch_tile_as<BMV, BNV, 4, 2, TC, ACC, GATED, true, 2, false, 3>(A, W, bias, C, M, N, K, lda, ldc, vector_ok, r, \
+                                                                           partial, s, norm)
   switch (plan.config) {
-    case 5: VK_TILE(256, 256, 4, 2, true);
-    case 6: VK_TILE(256, 192, 4, 2, true);
+    case 5: VK_TILE_W3(256, 256);
+    case 6: VK_TILE_W3(256, 192);
     case 7:  // three stages fit this tile's LDS, and its loads per product are the most of the 256-token tiles
       if (g_tile_stages != 2)
         return launch_tile_as<256, 128, 4, 2, TC, ACC, GATED, true, 3>(A, W, bias, C, M, N, K, lda, ldc, vector_ok, r,
@@ -2134,7 +2174,7 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
       // past 128 tokens eight waves of 32 x 64 instead of four of 64 x 64: such tiles run where the tiles are few, often
       // one workgroup to a CU, and twice the waves hide more of its waits (2,048 tokens on 2,048 x 2,048: 30.1 to
       // 26.9 us, 512 tokens on 2,048 x 1,536: 16.5 to 12.1; nowhere slower)
-      if (!deep) VK_TILE(128, 128, 4, 2, true);
+      if (!deep) VK_TILE_W3(128, 128);
       VK_TILE_DEEP(128, 128, 2, 2);
     case 2: VK_TILE(256, 128, 4, 2, false);
     case 3: VK_TILE(128, 256, 2, 4, false);
@@ -2142,6 +2182,7 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
     default: VK_TILE(128, 128, 2, 2, false);
   }
 #undef VK_TILE_DEEP
+#undef VK_TILE_W3
 #undef VK_TILE
 }
 }  // namespace
