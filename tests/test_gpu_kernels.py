@@ -128,6 +128,65 @@ def test_the_tiles_of_whole_products_give_the_bits_of_the_128x128_ones(tiling, r
         kernels.gemm_bf16_force_tiling(-1)
 
 
+@pytest.mark.parametrize("tiling", [5, 6, 9])
+def test_tiles_with_a_third_stage_of_the_weight_give_the_bits_of_the_others(tiling):
+    """Runs of K shorter than the stages, as long, and ending in every pair of stages (64 to 640), whole and in ranges, with tails
+    of a row and a column: the bits of the 256x128 tiles, whose operands have three stages each."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(tiling)
+    for m, n in ((257, 288), (300, 416)):
+        for k in (64, 128, 192, 256, 320, 384, 640, 1152):
+            a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+            w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+            for ranges in (1, 2):
+                got = []
+                try:
+                    for one in (tiling, 7):
+                        kernels.gemm_bf16_force_tiling(one, ranges)
+                        outs = [torch.full((m, n), 7.0, device=DEV), torch.full((m, n // 2), 7.0, dtype=torch.bfloat16, device=DEV)]
+                        kernels.gemm_bf16(a, w, None, outs[0])
+                        kernels.gemm_bf16_gated(a, w, outs[1])
+                        got.append(outs)
+                finally:
+                    kernels.gemm_bf16_force_tiling(-1)
+                assert all(torch.equal(x, y) for x, y in zip(*got)), (m, n, k, ranges)
+                assert _rel(got[0][0], a.double() @ w.double().T) < 1e-5
+
+
+@pytest.mark.parametrize("rows,tiling", [(32, 21), (96, 21), (64 * 256, 21), (64 * 256 + 32, 22), (96 * 256, 22), (96 * 256 + 32, 23),
+                                         (128 * 256 + 32, 24), (160 * 256 + 32, 25), (224 * 256, 25), (224 * 256 + 32, 23)])
+def test_gated_products_of_up_to_64_tokens_take_tiles_of_64_with_the_same_bits(rows, tiling):
+    """At each width of a tile, its last number of weight rows and the next one's first: the bits of the 128x128 tiles, with and
+    without the norm before the product, whichever of the LDS-shared kernel's plans asks."""
+    from vipera_rs_amd.ops import kernels
+    if kernels.compute_units(torch.device(DEV)) != 256:
+        pytest.skip("the widths follow the number of CUs")
+    for m, k in ((17, 64), (33, 192), (64, 320), (5, 128)):
+        g = torch.Generator().manual_seed(rows + m)
+        a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+        w = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+        groups, stride = 5, kernels.follow_stride(m)
+        sumsq = (torch.rand(groups * stride, generator=g) * k / groups).to(DEV)
+        assert kernels.gemm_bf16_tile_carried_out(m, rows, k, gated=True) == tiling
+        got = []
+        try:
+            for forced in (-1, 9):
+                kernels.gemm_bf16_force_tiling(forced)
+                outs = [torch.full((m, rows // 2), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(4)]
+                kernels.gemm_bf16_gated(a, w, outs[0], 3)
+                kernels.gemm_bf16_gated_tile_scaled(a, w, outs[1], sumsq, groups, 1e-5)
+                for plan in (1, 2):
+                    kernels.gemm_bf16_gated(a, w, outs[1 + plan], plan)
+                got.append(outs)
+        finally:
+            kernels.gemm_bf16_force_tiling(-1)
+        assert all(torch.equal(x, y) for x, y in zip(*got)) and torch.equal(got[0][0], got[0][2]) and torch.equal(got[0][0], got[0][3])
+        product = a.double() @ w.double().T
+        blocks = product.view(m, rows // 32, 2, 16)
+        gate, up = blocks[:, :, 0].reshape(m, -1), blocks[:, :, 1].reshape(m, -1)
+        assert _rel(got[0][0], up * gate / (1 + torch.exp(-gate))) < 8e-3
+
+
 @pytest.mark.parametrize("m,n,k,tiling", [(1396, 1536, 1536, 16), (783, 4096, 2048, 17), (1000, 4608, 3584, 18), (2210, 4096, 1024, 19),
                                           (910, 9216, 2048, 20)])
 def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):

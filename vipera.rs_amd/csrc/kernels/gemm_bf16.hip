@@ -195,18 +195,20 @@ struct TileNorm {
   float eps = 0.f;
 };
 
-// At the start of a tile kernel the THREADS / BM threads of a token each add every
-// (THREADS / BM)-th group, in ascending order, and leave their part in part_sums[part * BM + token] (a token past M
+// At the start of a tile kernel the threads of a token (THREADS / BM of them; two in tiles of 64 tokens, which take over from
+// tiles of 128 on 256 threads: the same sums) each add every so many-th group, in ascending order, and leave their part in part_sums[part * BM + token] (a token past M
 // takes the last one's, which nothing uses). A thread requests 32 groups at a time at clamped addresses before it
 // adds any: one round trip to memory for up to 64 groups on two threads, behind the tile's first operand requests,
 // where a loop of a load and an addition at a time cost the gate/up product of 2,048 tokens 69 us of 437. The
 // barrier before the first product makes the parts visible; tile_norm_factor adds them in ascending order.
 template <int BM, int THREADS>
+constexpr int NORM_PARTS = BM <= 64 ? 2 : THREADS / BM;
+template <int BM, int THREADS>
 __device__ __forceinline__ void tile_norm_parts(const TileNorm& norm, int m0, int M, int tid, float* part_sums) {
   if constexpr (THREADS % BM != 0) return;   // such tiles are not launched with a norm (launch_tile_as refuses it)
-  constexpr int PER = THREADS / BM, AHEAD = 32;
-  if (!norm.sumsq) return;
+  constexpr int PER = NORM_PARTS<BM, THREADS>, AHEAD = 32;
   const int token = tid % BM, part = tid / BM;
+  if (!norm.sumsq || part >= PER) return;
   const float* of_token = norm.sumsq + min(m0 + token, M - 1);
   float squares = 0.f;
   for (int base = part; base < norm.groups; base += AHEAD * PER) {
@@ -223,7 +225,7 @@ template <int BM, int THREADS>
 __device__ __forceinline__ float tile_norm_factor(const TileNorm& norm, const float* part_sums, int token, int K) {
   float squares = 0.f;
 #pragma unroll
-  for (int part = 0; part < THREADS / BM; ++part) squares += part_sums[part * BM + token];
+  for (int part = 0; part < NORM_PARTS<BM, THREADS>; ++part) squares += part_sums[part * BM + token];
   return 1.0f / sqrtf(squares / (float)K + norm.eps);
 }
 
@@ -2057,6 +2059,23 @@ int whole_tile(int planned, int M, int N, int K, double output_bytes) {
   return best;
 }
 
+// The gated product of up to 64 tokens: tiles of 64 tokens and of the fewest weight rows with which every tile finds a CU; past
+// 224 x CUs rows 128 of them, two tiles to a CU. A launch is a stream of the weights beside which every tile reads all
+// activations, and tiles of 128 tokens spend half their loads, LDS and products on tokens that are not there. More bytes of the
+// weight in flight (up to nine stages) are slower, not faster. Every output is one sum over K in ascending steps of 32, as in the
+// tiles of 128 tokens and in the kernel that shares the activations through LDS where it does not turn its chunks. us, weights
+// from memory, 17 and 64 tokens: 9,728 rows of 896 (LDS-shared before) 8.6 -> 7.7 and 10.6 -> 8.8 in tiles of 64 rows; 17,920 of 1,536
+// (LDS-shared, tiles) 20.1 -> 14.7 and 19.4 -> 17.1 in 96; 22,016 of 2,048 (48 and 64 tokens, tiles) 24.6 -> 22.9 and 24.8 -> 23.2 in 96;
+// 27,648 of 5,120 57.1 -> 51.5 and 58.7 -> 55.4 in 128; 37,888 of 3,584 55.0 -> 48.7 and 52.5 -> 49.9 in 160; 55,296 of 5,120 105 -> 97 and
+// 103 -> 100 in 224; 59,136 of 8,192 (64 tokens) 186 -> 175 in 128. The next wider or narrower tile is 5 to 40 % slower each time.
+struct FewTile { int config, rows; };
+constexpr FewTile FEW_TILES[] = {{21, 64}, {22, 96}, {23, 128}, {24, 160}, {25, 224}};
+int few_tokens_tile(int N) {
+  for (const FewTile& t : FEW_TILES)
+    if ((N + t.rows - 1) / t.rows <= g_compute_units) return t.config;
+  return 23;
+}
+
 // What this thread's last tiled launch took, and the plans it has worked out so far, for tests.
 struct TileLaunched { int config, ranges; long long plans; };
 thread_local TileLaunched g_tile_launched = {-1, 0, 0};
@@ -2079,6 +2098,7 @@ TilePlan carried_out(int M, int N, int K, long long partial_floats, bool gated, 
     ++g_tile_launched.plans;
     TilePlan plan = tile_plan(M, N, K, (long long)most_ranges * M * N, gated, scaled);
     if ((K & 63) == 0 && M > 128 && plan.ranges == 1 && !scaled) plan.config = whole_tile(plan.config, M, N, K, output_bytes);
+    if ((K & 63) == 0 && M <= 64 && gated) plan.config = few_tokens_tile(N);
     kept = Kept{M, N, K, form, plan};
   }
   return kept.plan;
@@ -2088,7 +2108,8 @@ TilePlan carried_out(int M, int N, int K, long long partial_floats, bool gated, 
 // with the kernel that loads straight into LDS, which needs K to be a multiple of 64; 13 and 15 that kernel at 64x64
 // and 128x64, 14 at 64x64 with the K ranges of one tile in one workgroup (15 always so); and 6 that kernel at
 // 256x192 (2,048 tokens x 4,608 rows are 192 such tiles for 256 CUs, against 144 of 256x256). 16 to 20: see whole_tile;
-// with a norm's factors, which are summed by a power of two of threads a token, they fall back to 9.
+// with a norm's factors, which are summed by a power of two of threads a token, they fall back to 9. 21 to 25: see
+// few_tokens_tile; 10 to 12 and these exist for the gated product only.
 template <typename TC, bool ACC, bool GATED = false>
 int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int M, int N, int K, long long lda,
                 long long ldc, int vector_ok, float* partial, long long partial_floats, hipStream_t s,
@@ -2099,8 +2120,8 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
   else plan = carried_out(M, N, K, (GATED || !partial) ? 0 : partial_floats, GATED, norm.sumsq != nullptr,
                           GATED ? 1.0 : sizeof(TC) * (ACC ? 2.0 : 1.0));
   if (plan.ranges > 1 && (long long)plan.ranges * M * N > partial_floats) plan.ranges = 1;
-  if (plan.config >= 16 && norm.sumsq) plan.config = 9;
-  if (plan.config >= 10 && plan.config <= 12 && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
+  if (plan.config >= 16 && plan.config <= 20 && norm.sumsq) plan.config = 9;
+  if (((plan.config >= 10 && plan.config <= 12) || plan.config >= 21) && !GATED) plan.config = 9;   // the narrow tiles exist for the gated product only
   if (!direct) {
     switch (plan.config) { case 5: case 6: plan.config = 4; break; case 7: plan.config = 2; break; case 8: plan.config = 3; break;
                            default: if (plan.config >= 9) plan.config = 0; }
@@ -2120,6 +2141,9 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
                                                                          partial, s, norm);                          \
     VK_TILE(BMV, BNV, WMV, WNV, true);                                                                               \
   }
+#define VK_TILE_FEW(BNV, WNV, STAGESV)                                                                                \
+  return launch_tile_as<64, BNV, 4, WNV, TC, ACC, GATED, true, STAGESV>(A, W, bias, C, M, N, K, lda, ldc, vector_ok, r, partial, \
+                                                                        s, norm)
   const bool deep = tile_is_deep(M);
   if constexpr (GATED) {
     switch (plan.config) {
@@ -2128,6 +2152,11 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
       case 10: VK_TILE_DEEP(128, 96, 4, 1);
       case 11: VK_TILE_DEEP(128, 160, 4, 1);
       case 12: VK_TILE_DEEP(128, 224, 4, 1);
+      case 21: VK_TILE_FEW(64, 2, 4);
+      case 22: VK_TILE_FEW(96, 1, 4);
+      case 23: VK_TILE_FEW(128, 1, 3);
+      case 24: VK_TILE_FEW(160, 1, 3);
+      case 25: VK_TILE_FEW(224, 1, 3);
     }
   }
 #define VK_TILE_SMALL(BMV, BNV, STAGESV, FOLDV)                                                                       \
@@ -2182,6 +2211,7 @@ int launch_tile(const __bf16* A, const __bf16* W, const float* bias, TC* C, int 
     default: VK_TILE(128, 128, 2, 2, false);
   }
 #undef VK_TILE_DEEP
+#undef VK_TILE_FEW
 #undef VK_TILE_W3
 #undef VK_TILE
 }
@@ -2308,7 +2338,8 @@ extern "C" int vk_gemm_bf16_mid_no_alloc(const void* A, const void* W, const flo
 // out[M, N / 2] = up * silu(gate) of the product with a fused gate/up weight W[N, K] whose rows are
 // interleaved in groups of 16 (see store_gated). bfloat16 in and out; N a multiple of 32.
 // More than 64 tokens: the tiled kernel; up to 64: the LDS-shared kernel with one K range and `rows_per_wave`
-// (1 or 2) tiles of 16 rows per wave, or with `rows_per_wave` 0 the kernel that keeps the activations resident
+// (1 or 2) tiles of 16 rows per wave (from 17 tokens on, and for K in whole steps of 64 but not of 2,048, the tiled kernel with the
+// same sums in the same order), or with `rows_per_wave` 0 the kernel that keeps the activations resident
 // in LDS (up to 16 tokens, K a multiple of 128, tokens x K within LDS; anything else is refused), or with
 // `rows_per_wave` 3 the tiled kernel.
 extern "C" int vk_gemm_bf16_gated(const void* A, const void* W, void* C, int M, int N, int K, long long lda,
@@ -2321,7 +2352,10 @@ extern "C" int vk_gemm_bf16_gated(const void* A, const void* W, void* C, int M, 
   const __bf16* a = (const __bf16*)A;
   const __bf16* w = (const __bf16*)W;
   __bf16* c = (__bf16*)C;
-  if (M > 64 || rows_per_wave == 3) return launch_tile<__bf16, false, true>(a, w, nullptr, c, M, N, K, lda, ldc, 0, nullptr, 0, s);
+  // what the LDS-shared kernel would do in K's own order, the tiles of 64 tokens do faster from 17 tokens on (few_tokens_tile)
+  const bool tiled = (rows_per_wave == 1 || rows_per_wave == 2) && M > 16 && (K & 63) == 0 && (K & 2047) != 0;
+  if (M > 64 || rows_per_wave == 3 || tiled)
+    return launch_tile<__bf16, false, true>(a, w, nullptr, c, M, N, K, lda, ldc, 0, nullptr, 0, s);
   if (rows_per_wave == 0) return launch_resident_gated<false>(a, w, c, M, N, K, lda, ldc, nullptr, 0, 0.f, s);
   const int cb = (M + 15) / 16;
 #define VK_GATED(CBV, RTV)                                                                                         \

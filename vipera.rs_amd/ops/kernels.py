@@ -751,7 +751,8 @@ TILE_TILINGS = {0: "128x128 staged", 2: "256x128 staged", 3: "128x256 staged", 4
                 10: "128x96 direct, gated only", 11: "128x160 direct, gated only", 12: "128x224 direct, gated only",
                 13: "64x64 direct", 14: "64x64 direct, ranges in one workgroup", 15: "128x64 direct, ranges in one workgroup",
                 16: "192x64 direct", 17: "128x128 direct, three stages", 18: "192x128 direct, three stages",
-                19: "192x128 direct, two stages", 20: "192x192 direct"}
+                19: "192x128 direct, two stages", 20: "192x192 direct", 21: "64x64 direct, gated, up to 64 tokens",
+                22: "64x96 direct, gated", 23: "64x128 direct, gated", 24: "64x160 direct, gated", 25: "64x224 direct, gated"}
 
 
 def gemm_bf16_tile_plan(m: int, n: int, k: int, gated: bool = False) -> Tuple[int, int]:
