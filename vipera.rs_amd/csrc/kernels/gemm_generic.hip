@@ -717,17 +717,25 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
 // tiles over the 256 CUs is as long as a full one while the rounds are few.  Times in us as measured (weights from memory), of
 // a round and beside the rounds:
 //   slab, 16 x 32 outputs   2.9 + 3.9 a round (tiles x slabs)    9 x 1,152 x 896: 6.7 (14.1 as 64 x 64 tiles cut over workgroups)
-//         32 x 32           3.2 + 6.4                            128 x 1,152 x 896: 9.4 (15.0)
+//         32 x 32           3.2 + 6.2                            128 x 1,152 x 896: 9.1 (15.0)
 //         48 x 32           4.5 + 9.3                            333 x 1,152 x 896: 14.2 (20.3)
-//         64 x 64           3 + 22                               64 x 1,536 x 8,960: 32.7 (40.3)
+//   slabs of 64 columns: by how many a CU holds at a time (Residents)
+//         32 x 64           15, 26.5, 32 for 1, 2, 3             200 x 896 x 4,864: 34.6 (37.0 as 32 x 32)
+//         48 x 64           20.5, 33                             333 x 896 x 4,864: 44.0 (55.5 as 64 x 64 tiles cut over workgroups)
+//         64 x 64           23, 38.5                             64 x 1,536 x 8,960: 31 (40.3)
 //     and, with several slabs, 5 for adding the parts and their way through memory
 //   rows, 64 x 64           7.5 + 0.0193 K a round               2,048 x 2,560 x 2,048: 210 (232)
 //         32 x 128          8 + 0.0207 K                         65 x 17,920 x 1,536: 68.9 (92.9)
 //         64 x 128          8 + 0.0365 K                         333 x 9,728 x 896: 72.8 (81.7); 2,048 x 37,888 x 3,584: 4,757 (5,358)
-// Over 112 sizes from 9 to 2,048 rows the choice takes 0.80 of the time of the 64 x 64 tiles (geometric mean), and 1.07 of it at
-// worst (512 x 1,536 x 1,536).  Those tiles keep a product where their cut of K is estimated to be faster (200 x 1,536 x 8,960: 87.8
-// against 93.7), any other type, and rows off 16 bytes.
-enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128 };
+// A slab's wave has a chain of loads and sums of its own, and what hides it is other workgroups of the CU, not more of its own
+// stages: with 2 stages instead of 4 two workgroups of 64 x 64 fit, which take 0.91 of the time over 216 sizes from 12 to
+// 2,048 rows (0.75 to 0.98 at each), and with 3 instead of 4 three of 32 x 32 (0.96); the tiles of 48 x 64 and 32 x 64 read less
+// for each output than narrower ones and leave room for 2 and 3 on a CU.  The choice takes 0.966 of the time it took without these
+// (geometric mean), 0.72 at best (65 x 2,048 x 11,008: 60.9 against 84.2) and 1.05 at worst (256 x 2,560 x 2,048: 43.7 against 41.8).
+// Over 112 sizes from 9 to 2,048 rows it took 0.80 of the time of the 64 x 64 tiles cut over workgroups without them, and 1.07 of
+// it at worst.  Those keep a product where their cut of K is estimated to be faster (512 x 896 x 4,864), any other
+// type, and rows off 16 bytes.
+enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128, SLAB_32_64, SLAB_48_64 };
 
 inline double rounds(long long tiles) { return tiles <= 3 * 256 ? (double)((tiles + 255) / 256) : tiles / 256.0 + 0.35; }
 
@@ -740,23 +748,46 @@ inline double estimate_matrix(int M, int N, int K, int units) {
   return units == 1 ? 9.5 + fmax(5.0, (per_cu + 0.35) * 5.2) + parts : 9 + fmax(19.5, (per_cu + 0.15) * 18.5) + parts;
 }
 
+// Slabs of 64 columns: `resident` of them run on a CU at a time, and together they take us[resident - 1] for theirs.  The last
+// ones to start share a CU with as many others as are left; past two full rounds those of several slabs overlap.  Weights
+// whose rows are a multiple of 8 KB apart arrive 1.06 times as slowly, and 32 x 64 falls behind over rows of more than 8,192
+// (200 x 2,048 x 11,008: 169 us, 149 as 64 x 64 tiles cut over workgroups).
+struct Residents { Direct form; int rows, resident; double us[3], long_rows; };
+inline double resident_rounds(const Residents& f, long long tiles, int K) {
+  const long long chip = 256ll * f.resident, full = tiles / chip, left = tiles % chip;
+  const double round = f.us[f.resident - 1], last = left ? f.us[(left + 255) / 256 - 1] : 0.0;
+  return (full >= 2 && K > SLAB_K ? ((double)tiles / chip - 0.2) * round : full * round + last) *
+         (K % 2048 == 0 ? 1.06 : 1.0) * (K > 8192 ? f.long_rows : 1.0);
+}
+
 Direct direct_plan(int M, int N, int K, long long part_floats) {
   struct Form { Direct form; int rows, columns; double beside, round; };
-  constexpr Form forms[] = {{SLAB_16_32, 16, 32, 2.9, 3.9}, {SLAB_32_32, 32, 32, 3.2, 6.4}, {SLAB_48_32, 48, 32, 4.5, 9.3},
-                            {SLAB_64_64, 64, 64, 3.0, 22.0}, {ROWS_64_64, 64, 64, 7.5, 0.0193}, {ROWS_32_128, 32, 128, 8.0, 0.0207},
-                            {ROWS_64_128, 64, 128, 8.0, 0.0365}};
+  constexpr Form slab_forms[] = {{SLAB_16_32, 16, 32, 2.9, 3.9}, {SLAB_32_32, 32, 32, 3.2, 6.2}, {SLAB_48_32, 48, 32, 4.5, 9.3}};
+  constexpr Residents wide_slabs[] = {{SLAB_32_64, 32, 3, {15.0, 26.5, 32.0}, 1.2}, {SLAB_48_64, 48, 2, {20.5, 33.0}, 1.0},
+                                       {SLAB_64_64, 64, 2, {23.0, 38.5}, 1.0}};
+  constexpr Form row_forms[] = {{ROWS_64_64, 64, 64, 7.5, 0.0193}, {ROWS_32_128, 32, 128, 8.0, 0.0207}, {ROWS_64_128, 64, 128, 8.0, 0.0365}};
   const long long slabs = (K + SLAB_K - 1) / SLAB_K;
-  const bool parts_fit = slabs == 1 || slabs * M * N <= part_floats;
+  const double parts = slabs == 1 ? 0.0 : 5.0 + (double)slabs * M * N * 8 / 6e6;
   double best = 0.97 * estimate_matrix(M, N, K, part_floats > 0 ? matrix_units(M, N, K) : 0);
   Direct chosen = NOT_DIRECT;
-  for (const Form& f : forms) {
-    const bool slab = f.form <= SLAB_64_64;
-    const long long tiles = (long long)((M + f.rows - 1) / f.rows) * ((N + f.columns - 1) / f.columns);
-    if ((slab && !parts_fit) || tiles > 0xffffffffll / 256) continue;
-    double us;
-    if (slab) us = f.beside + f.round * rounds(tiles * slabs) + (slabs == 1 ? 0.0 : 5.0 + (double)slabs * M * N * 8 / 6e6);
-    else us = f.beside + f.round * K * rounds(tiles) * (K > SLAB_K && tiles <= 256 ? 1.07 : 1.0);
-    if (us < best) best = us, chosen = f.form;
+  auto tiles = [&](int rows, int columns) { return (long long)((M + rows - 1) / rows) * ((N + columns - 1) / columns); };
+  auto offer = [&](Direct form, long long count, double us) {
+    if (count <= 0xffffffffll / 256 && us < best) best = us, chosen = form;
+  };
+  if (slabs == 1 || slabs * M * N <= part_floats) {
+    for (const Form& f : slab_forms) {
+      const long long count = tiles(f.rows, f.columns);
+      offer(f.form, count, f.beside + f.round * rounds(count * slabs) + parts);
+    }
+    for (const Residents& f : wide_slabs) {
+      if (M <= 32) break;              // one row of tiles: narrower ones have more of the weight in flight (24 x 17,920 x 1,536: 40 against 45 us)
+      const long long count = tiles(f.rows, 64);
+      offer(f.form, count, resident_rounds(f, count * slabs, K) + parts);
+    }
+  }
+  for (const Form& f : row_forms) {
+    const long long count = tiles(f.rows, f.columns);
+    offer(f.form, count, f.beside + f.round * K * rounds(count) * (K > SLAB_K && count <= 256 ? 1.07 : 1.0));
   }
   return chosen;
 }
@@ -765,9 +796,11 @@ int launch_direct(Direct form, const float* A, const float* W, const float* bias
                   long long lda, long long ldc, int accumulate, hipStream_t s) {
   switch (form) {
     case SLAB_16_32: return launch_slabs<16, 1, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_32_32: return launch_slabs<32, 1, 1, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_32_32: return launch_slabs<32, 1, 1, 3>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
     case SLAB_48_32: return launch_slabs<16, 3, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_64_64: return launch_slabs<32, 2, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_32_64: return launch_slabs<32, 1, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_48_64: return launch_slabs<16, 3, 4, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_64_64: return launch_slabs<32, 2, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
     case ROWS_64_64: return launch_rows<1, 1, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
     case ROWS_32_128: return launch_rows<1, 1, 1, 4, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
     case ROWS_64_128: return launch_rows<1, 2, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
