@@ -532,10 +532,10 @@ def test_each_form_of_the_32_bit_product_sums_in_the_same_order(m, n, k, form):
         assert torch.equal(few, whole[rows]) and torch.equal(more, added[rows]), start
 
 
-@pytest.mark.parametrize("m,n,k,form", [(101, 9725, 1020, 8), (77, 1761, 2052, 8), (103, 1041, 11012, 8), (515, 1150, 900, 9),
+@pytest.mark.parametrize("m,n,k,form", [(333, 9725, 900, 8), (39, 3037, 2052, 8), (35, 779, 11012, 8), (515, 1150, 900, 9),
                                         (36, 4979, 2052, 9), (333, 895, 4868, 9), (162, 4283, 1020, 4), (553, 105, 11012, 4)])
-def test_slabs_of_64_columns_sum_in_the_same_order(m, n, k, form):
-    """The tiles of 32 x 64, 48 x 64 and 64 x 64 outputs over one slab and several, ending inside a tile, a step, a range and a
+def test_wide_slabs_of_the_32_bit_product_sum_in_the_same_order(m, n, k, form):
+    """The tiles of 48 x 48, 48 x 64 and 64 x 64 outputs over one slab and several, ending inside a tile, a step, a range and a
     slab, as their neighbours above."""
     test_each_form_of_the_32_bit_product_sums_in_the_same_order(m, n, k, form)
 

@@ -21,10 +21,9 @@
 // of the weights: the product of a few tokens is bound by the bytes of W. Everything else runs on the
 // matrix cores, gemm_matrix_kernel for any types and rows, gemm_rows_kernel and gemm_slab_kernel for
 // 32-bit operands whose rows start on 16 bytes: v_mfma_f32_32x32x2_f32 computes each of its outputs as
-// fma(a[k + 1], w[k + 1], fma(a[k], w[k], c)), rounded after every product (compared with fmaf chains bit
-// for bit, values of all magnitudes, denormal, infinite and NaN ones included), so a chain of these
-// instructions over ascending k is the range's chain above.
-#include <type_traits>
+// fma(a[k + 1], w[k + 1], fma(a[k], w[k], c)), rounded after every product, and v_mfma_f32_16x16x4_f32 as
+// four of these (compared with fmaf chains bit for bit, values of all magnitudes, denormal, infinite and
+// NaN ones included), so a chain of either over ascending k is the range's chain above.
 
 #include "common.h"
 
@@ -174,15 +173,17 @@ __global__ __launch_bounds__(256) void gemm_matrix_kernel(const TA* __restrict__
 
 // ---------------------------------------------------------------------------------------------
 // The same product where A, W and C are 32-bit and every row starts on 16 bytes: operands go from memory straight into LDS
-// (buffer loads with the lds modifier: no staging registers, no LDS stores) several steps ahead.  What the matrix instruction
-// wants of a lane, one k of two (or of four: v_mfma_f32_16x16x4_f32, four FMAs in ascending k on top of c, compared with fmaf
-// chains bit for bit), comes out of the 16 bytes it reads by lane exchanges (Fragment).  Two kernels:
+// (buffer loads with the lds modifier: no staging registers, no LDS stores) several steps ahead.  Lane group
+// g = lane / 16 gives v_mfma_f32_16x16x4_f32 k 4 t + g of its row, which it reads from LDS as such, 4 bytes, two blocks of
+// 16 rows with one instruction.  Two kernels:
 //   gemm_rows_kernel   a workgroup walks all of K
 //   gemm_slab_kernel   a workgroup owns one slab of K, wave w range w of it: the ranges' sums meet in LDS, and where K is one
 //                      slab that is the output, with no second launch; else parts and gemm_parts_finish_kernel
-// What bounds them: a wave alone on its SIMD reaches 70 % of the matrix cores' rate in the loop (every LDS read, load and lane
-// exchange between two products costs it some 5 to 30 cycles, and several waves a SIMD gain nothing beside them); below a round
-// of tiles, a range's chain: 128 instructions of 64 cycles, 3.4 us. Tiles of 128 x 128 are no faster at any size.
+// What bounds them: the matrix cores, and the cycles that each LDS read and load between two products takes of its wave.  Lanes
+// that read 16 bytes of four k and exchange them took more of those (four exchanges for each such read): 333 x 1,152 x 896 in
+// tiles of 48 x 32 15.4 us, 12.4 now; 333 x 9,728 x 896 in tiles of 64 x 128 74.1, 68.0 now.  Below a round of tiles a range's
+// chain is what a call waits for: 64 instructions of 32 cycles for each 16 x 16 outputs of a wave.  Tiles of more outputs are
+// faster at no size: those of 112 x 128 for 333 x 9,728 x 896 fit one round and take 64.4 us, 62.1 as 48 x 48 over one slab.
 // A row past the end is a copy of the last one and is not stored; a k past the end reads as zero (an offset past the view).
 constexpr unsigned NO_CHUNK = 0x80000000u;            // past the end of every view, and so are the steps behind it
 constexpr long long VIEW_BYTES = 0x7fffffffll;
@@ -198,43 +199,10 @@ __device__ __forceinline__ void loads_but() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
-// A block of BLOCK rows of an operand, 16 k: what a lane reads of it, and in which order the matrix instruction wants that.
-// 16 rows: one chunk of four k, lane group g = lane / 16 chunk g; instruction t wants k 4 t + g. 32 rows: chunks h and 2 + h
-// (h = lane / 32); instruction 4 c + t wants k 8 c + 2 t + h.
-template <int BLOCK>
-struct Fragment {
-  f32x4_t v[BLOCK / 16];
-  __device__ __forceinline__ static int row(int lane) { return lane & (BLOCK - 1); }
-  __device__ __forceinline__ static int chunk(int lane, int i) { return BLOCK == 16 ? lane >> 4 : 2 * i + (lane >> 5); }
-  __device__ __forceinline__ float operator()(int t) const { return v[t / 4][t % 4]; }
-  __device__ __forceinline__ void order() {
-    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-    for (int i = 0; i < BLOCK / 16; ++i) {
-      const u32x4_t r = __builtin_bit_cast(u32x4_t, v[i]);
-      u32x4_t to;
-      if constexpr (BLOCK == 16) {
-        const auto s01 = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);   // the first's odd groups and the second's even ones
-        const auto s23 = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
-        const auto s02 = __builtin_amdgcn_permlane32_swap(s01[0], s23[0], false, false);   // the first's upper half and the second's lower
-        const auto s13 = __builtin_amdgcn_permlane32_swap(s01[1], s23[1], false, false);
-        to = u32x4_t{s02[0], s13[0], s02[1], s13[1]};
-      } else {
-        const auto s01 = __builtin_amdgcn_permlane32_swap(r[0], r[1], false, false);
-        const auto s23 = __builtin_amdgcn_permlane32_swap(r[2], r[3], false, false);
-        to = u32x4_t{s01[0], s23[0], s01[1], s23[1]};
-      }
-      v[i] = __builtin_bit_cast(f32x4_t, to);
-    }
-  }
-};
-template <int BLOCK> struct Sums;
-template <> struct Sums<16> { typedef f32x4_t type; };
-template <> struct Sums<32> { typedef f32x16_t type; };
+// A block of 16 rows of an operand, 16 k: value t is the lane's k 4 t + lane / 16 of row lane % 16.
+typedef f32x4_t Fragment;
 __device__ __forceinline__ f32x4_t matrix_step(float w, float a, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, c, 0, 0, 0); }
-__device__ __forceinline__ f32x16_t matrix_step(float w, float a, f32x16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(w, a, c, 0, 0, 0); }
-// where a lane's four sums q of a block lie: row of A, first column
-template <int BLOCK> __device__ __forceinline__ int sum_column(int lane, int q) { return BLOCK == 16 ? 4 * (lane >> 4) : 8 * q + 4 * (lane >> 5); }
+// A lane's four sums of 16 x 16 outputs: row lane % 16 of A, columns 4 (lane / 16) and on.
 
 // Four consecutive outputs of a row (as far as they exist): + bias, + old, in that order.  quads: every four lie on 16 bytes
 // and exist together.
@@ -258,113 +226,97 @@ __device__ __forceinline__ void store_outputs(float* __restrict__ C, const float
   }
 }
 
-// Hints for the order of what was written since the last such line: LDS reads and loads go out one by one between the products,
-// or two lane exchanges at a time.  All reads and loads ahead of the products made every wave wait for the others' at the LDS and
-// address units: 112 TFLOP/s at 2,048 x 4,096 x 4,096.
+// Hints for the order of what was written since the last such line: LDS reads and loads go out one by one between the products.
+// All of them ahead of the products made every wave wait for the others' at the LDS and address units: 112 TFLOP/s at
+// 2,048 x 4,096 x 4,096.
 template <int PRODUCTS, int READS, int LOADS>
 __device__ __forceinline__ void between_products() {
-  if constexpr (READS + LOADS == 0) {
+  constexpr int MOST = READS > LOADS ? READS : LOADS;
+  constexpr int EACH = MOST <= PRODUCTS ? 1 : (MOST + PRODUCTS - 1) / PRODUCTS;
 #pragma unroll
-    for (int i = 0; i < PRODUCTS; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one matrix instruction
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // two others
-    }
-  } else {
-    constexpr int MOST = READS > LOADS ? READS : LOADS;
-    constexpr int EACH = MOST <= PRODUCTS ? 1 : (MOST + PRODUCTS - 1) / PRODUCTS;
-#pragma unroll
-    for (int i = 0; i < PRODUCTS; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (i * EACH < READS) __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);   // LDS reads
-      if (i * EACH < LOADS) __builtin_amdgcn_sched_group_barrier(0x020, EACH, 0);   // loads
-    }
+  for (int i = 0; i < PRODUCTS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // one matrix instruction
+    if (i * EACH < READS) __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);   // LDS reads
+    if (i * EACH < LOADS) __builtin_amdgcn_sched_group_barrier(0x020, EACH, 0);   // loads
   }
   __builtin_amdgcn_sched_barrier(0);
 }
+// LDS reads of 16 k of TM + TN blocks: two blocks an instruction
+template <int TM, int TN> constexpr int READS_OF = 4 * ((TM + 1) / 2 + (TN + 1) / 2);
 
-// A workgroup's outputs over all of K: WM x WN waves, each TM x TN blocks of 32 x 32; steps of 32 k through STAGES stages, the
+// A workgroup's outputs over all of K: WM x WN waves, each TM x TN blocks of 16 x 16; steps of 32 k through STAGES stages, the
 // loads of STAGES - 1 steps in flight.  LDS rows are 128 bytes, unpadded (a load instruction fills 1 KB: 8 rows, lane L the 16
-// bytes at 16 L); chunk c of row r sits in slot c ^ (r % 8), so that 16 rows read the same chunk from different banks.  A wave
-// reads the operands of a half step while it multiplies the first half of the other and orders them during its second half.
-// SLABS: K has several.
+// bytes at 16 L); chunk c of row r sits in slot c ^ (r / 2 % 8): the 64 values of a block's next four k lie in 64 banks.  A wave
+// loads every WAVES-th 8 rows, so that its lanes' chunks are the same in all of them.  It reads the operands of a half step
+// while it multiplies the first half of the other.  SLABS: K has several.
 template <int TM, int TN, int WM, int WN, int STAGES, bool SLABS, bool ACCUMULATE>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                  const float* __restrict__ bias, float* __restrict__ C, int M,
                                                                  int N, int K, long long lda, long long ldc, bool quads) {
   typedef __attribute__((address_space(3))) void* lds_at;
-  typedef Fragment<32> Frag;
-  constexpr int WAVES = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, STEP = 32, ROW = STEP * 4;
+  constexpr int WAVES = WM * WN, BM = 16 * TM * WM, BN = 16 * TN * WN, STEP = 32, ROW = STEP * 4;
   constexpr int A_LOADS = BM / 8 / WAVES, W_LOADS = BN / 8 / WAVES, LOADS = A_LOADS + W_LOADS, STAGE = (BM + BN) * ROW;
-  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "tile rows must divide among the waves' loads");
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && WAVES % 2 == 0, "tile rows must divide among the waves' loads");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN, lr = Frag::row(lane);
+  const int wm = wave / WN, wn = wave % WN, lr = lane & 15;
   const int m_tiles = (M + BM - 1) / BM;
   const int m0 = blockIdx.x % m_tiles * BM, n0 = blockIdx.x / m_tiles * BN;
   const __amdgpu_buffer_rsrc_t a_view = row_view(A + (size_t)m0 * lda), w_view = row_view(W + (size_t)n0 * K);
-  const int ld_row = lane >> 3, ld_chunk = (lane & 7) ^ (lane >> 3);
+  const int ld_row = lane >> 3, ld_chunk = (lane & 7) ^ (lane >> 4) ^ (wave & 1) * 4;
   unsigned a_off[A_LOADS], w_off[W_LOADS];
 #pragma unroll
   for (int i = 0; i < A_LOADS; ++i)
-    a_off[i] = (unsigned)(min(m0 + (wave * A_LOADS + i) * 8 + ld_row, M - 1) - m0) * (unsigned)(lda * 4) + ld_chunk * 16;
+    a_off[i] = (unsigned)(min(m0 + (i * WAVES + wave) * 8 + ld_row, M - 1) - m0) * (unsigned)(lda * 4) + ld_chunk * 16;
 #pragma unroll
   for (int i = 0; i < W_LOADS; ++i)
-    w_off[i] = (unsigned)(min(n0 + (wave * W_LOADS + i) * 8 + ld_row, N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
+    w_off[i] = (unsigned)(min(n0 + (i * WAVES + wave) * 8 + ld_row, N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
   auto issue = [&](int stage, int step) {
-    unsigned char* to_a = lds + stage * STAGE + wave * A_LOADS * 1024;
-    unsigned char* to_w = lds + stage * STAGE + BM * ROW + wave * W_LOADS * 1024;
+    unsigned char* to_a = lds + stage * STAGE + wave * 1024;
+    unsigned char* to_w = to_a + BM * ROW;
     const unsigned kb = step * STEP + ld_chunk * 4 < K ? (unsigned)step * ROW : NO_CHUNK;
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_view, (lds_at)(to_a + i * 1024), 16, (int)(a_off[i] + kb), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_view, (lds_at)(to_a + i * WAVES * 1024), 16, (int)(a_off[i] + kb), 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_view, (lds_at)(to_w + i * 1024), 16, (int)(w_off[i] + kb), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_view, (lds_at)(to_w + i * WAVES * 1024), 16, (int)(w_off[i] + kb), 0, 0, 0);
   };
-  unsigned at_a[2], at_w[2];   // the lane's two chunks of the first half step; bit 6 of the place: the second half
+  unsigned at[4];                                      // the lane's four k of a block's first half step; bit 6 of the place: the second half
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const unsigned slot = (unsigned)((Frag::chunk(lane, i) ^ (lr & 7)) * 16);
-    at_a[i] = (unsigned)((wm * TM * 32 + lr) * ROW) + slot;
-    at_w[i] = (unsigned)((BM + wn * TN * 32 + lr) * ROW) + slot;
-  }
-  auto read = [&](int stage, int half, Frag (&fa)[TM], Frag (&fw)[TN]) {
+  for (int t = 0; t < 4; ++t) at[t] = (unsigned)(lr * ROW + ((t ^ (lr >> 1)) * 16) + (lane >> 4) * 4);
+  const unsigned at_a = wm * TM * 16 * ROW, at_w = (BM + wn * TN * 16) * ROW;
+  auto read = [&](int stage, int half, Fragment (&fa)[TM], Fragment (&fw)[TN]) {
     const unsigned char* base = lds + stage * STAGE;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int t = 0; t < 4; ++t) {
+      const unsigned char* from = base + (at[t] ^ (half * 64));
 #pragma unroll
-      for (int t = 0; t < TN; ++t) fw[t].v[i] = *(const f32x4_t*)(base + (at_w[i] ^ (half * 64)) + t * 32 * ROW);
+      for (int n = 0; n < TN; ++n) fw[n][t] = *(const float*)(from + at_w + n * 16 * ROW);
 #pragma unroll
-      for (int t = 0; t < TM; ++t) fa[t].v[i] = *(const f32x4_t*)(base + (at_a[i] ^ (half * 64)) + t * 32 * ROW);
+      for (int m = 0; m < TM; ++m) fa[m][t] = *(const float*)(from + at_a + m * 16 * ROW);
     }
   };
-  f32x16_t acc[TN][TM], slab[TN][TM], total[TN][TM];
+  f32x4_t acc[TN][TM], slab[TN][TM], total[TN][TM];
 #pragma unroll
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = slab[n][m] = total[n][m] = 0.f;
-  auto multiply = [&](const Frag (&fa)[TM], const Frag (&fw)[TN], int half) {
+  auto multiply = [&](const Fragment (&fa)[TM], const Fragment (&fw)[TN], int half) {
 #pragma unroll
-    for (int t = 4 * half; t < 4 * half + 4; ++t)
+    for (int t = 2 * half; t < 2 * half + 2; ++t)
 #pragma unroll
       for (int n = 0; n < TN; ++n)
 #pragma unroll
-        for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n](t), fa[m](t), acc[n][m]);
-  };
-  auto order = [&](Frag (&fa)[TM], Frag (&fw)[TN]) {
-#pragma unroll
-    for (int t = 0; t < TN; ++t) fw[t].order();
-#pragma unroll
-    for (int t = 0; t < TM; ++t) fa[t].order();
+        for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n][t], fa[m][t], acc[n][m]);
   };
   const int steps = (K + STEP - 1) / STEP;
-  Frag fa0[TM], fw0[TN], fa1[TM], fw1[TN];
+  Fragment fa0[TM], fw0[TN], fa1[TM], fw1[TN];
 #pragma unroll
   for (int i = 0; i < STAGES; ++i) issue(i, i);        // a step past the end loads zeros
   loads_but<(STAGES - 1) * LOADS>();
   __syncthreads();
   read(0, 0, fa0, fw0);
-  order(fa0, fw0);
   int stage = 0, s = 0;
   for (int slabs_done = 0; s < steps;) {
     // a range's steps in a loop of their own, which touches no sum but acc
@@ -373,19 +325,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
       const int next = stage + 1 == STAGES ? 0 : stage + 1;
       read(stage, 1, fa1, fw1);
       multiply(fa0, fw0, 0);
-      between_products<4 * TM * TN, 2 * (TM + TN), 0>();
-      order(fa1, fw1);
+      between_products<2 * TM * TN, READS_OF<TM, TN>, 0>();
       multiply(fa0, fw0, 1);
-      between_products<4 * TM * TN, 0, 0>();
+      __builtin_amdgcn_sched_barrier(0);
       loads_but<(STAGES - 2) * LOADS>();
       __syncthreads();                                 // step s + 1 is there, and nobody reads this step's stage any more
       read(next, 0, fa0, fw0);
       issue(stage, s + STAGES);
       multiply(fa1, fw1, 0);
-      between_products<4 * TM * TN, 2 * (TM + TN), LOADS>();
-      order(fa0, fw0);
+      between_products<2 * TM * TN, READS_OF<TM, TN>, LOADS>();
       multiply(fa1, fw1, 1);
-      between_products<4 * TM * TN, 0, 0>();
+      __builtin_amdgcn_sched_barrier(0);
       stage = next;
     }
     const bool slab_ends = ++slabs_done % SLAB_RANGES == 0 || s == steps;
@@ -408,39 +358,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
 #pragma unroll
     for (int n = 0; n < TN; ++n)
 #pragma unroll
-      for (int m = 0; m < TM; ++m) {
-        const f32x16_t& sum = SLABS ? total[n][m] : slab[n][m];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          store_outputs<ACCUMULATE>(C, bias, f32x4_t{sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]},
-                                    m0 + (wm * TM + m) * 32 + lr, n0 + (wn * TN + n) * 32 + sum_column<32>(lane, q), M, N, ldc, in_quads);
-      }
+      for (int m = 0; m < TM; ++m)
+        store_outputs<ACCUMULATE>(C, bias, SLABS ? total[n][m] : slab[n][m], m0 + (wm * TM + m) * 16 + lr,
+                                  n0 + (wn * TN + n) * 16 + 4 * (lane >> 4), M, N, ldc, in_quads);
   };
   if (quads) store(true);
   else store(false);
 }
 
-// A workgroup's BLOCK TM x BLOCK TN outputs over one slab (blockIdx.y), a range a wave.  A wave has stages of its own, of 16 k,
+// A workgroup's 16 TM x 16 TN outputs over one slab (blockIdx.y), a range a wave.  A wave has stages of its own, of 16 k,
 // and waits for no other before the ranges' sums meet.  LDS rows are 64 bytes (a load instruction: 16 rows); chunk c of row r
-// sits in slot c ^ (r / 4 % 4): a chunk of 16 rows lies in all banks.
-template <int BLOCK, int TM, int TN, int STAGES, bool PARTS, bool ACCUMULATE>
+// sits in slot c ^ (r / 4 % 4): the 64 values of a block's next four k lie in 64 banks.
+template <int TM, int TN, int STAGES, bool PARTS, bool ACCUMULATE>
 __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                         const float* __restrict__ bias, float* __restrict__ C,
                                                         float* __restrict__ parts, int M, int N, int K, long long lda,
                                                         long long ldc, bool quads) {
   typedef __attribute__((address_space(3))) void* lds_at;
-  typedef Fragment<BLOCK> Frag;
-  typedef typename Sums<BLOCK>::type Sum;
-  constexpr int STEP = 16, HALVES = BLOCK / 16, A_GROUPS = TM * HALVES, GROUPS = (TM + TN) * HALVES, STAGE = GROUPS * 1024;
-  constexpr int QUADS = BLOCK == 16 ? 1 : 4, SUM_QUADS = TM * TN * QUADS;
+  constexpr int STEP = 16, GROUPS = TM + TN, STAGE = GROUPS * 1024, SUM_QUADS = TM * TN;
   static_assert(SUM_QUADS * 1024 <= STAGES * STAGE, "the ranges' sums reuse the stages");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m_tiles = (M + BLOCK * TM - 1) / (BLOCK * TM);
-  const int m0 = blockIdx.x % m_tiles * (BLOCK * TM), n0 = blockIdx.x / m_tiles * (BLOCK * TN);
+  const int m_tiles = (M + 16 * TM - 1) / (16 * TM);
+  const int m0 = blockIdx.x % m_tiles * (16 * TM), n0 = blockIdx.x / m_tiles * (16 * TN);
   const int k_begin = blockIdx.y * SLAB_K + wave * RANGE_K, k_end = min(K, k_begin + RANGE_K);
   unsigned char* mine = lds + wave * (STAGES * STAGE);
-  Sum acc[TN][TM];
+  f32x4_t acc[TN][TM];
 #pragma unroll
   for (int n = 0; n < TN; ++n)
 #pragma unroll
@@ -451,55 +394,47 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
     unsigned off[GROUPS];
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g)
-      off[g] = (g < A_GROUPS ? (unsigned)(min(m0 + 16 * g + ld_row, M - 1) - m0) * (unsigned)(lda * 4)
-                             : (unsigned)(min(n0 + 16 * (g - A_GROUPS) + ld_row, N - 1) - n0) * (unsigned)(K * 4)) + ld_chunk * 16;
+      off[g] = (g < TM ? (unsigned)(min(m0 + 16 * g + ld_row, M - 1) - m0) * (unsigned)(lda * 4)
+                             : (unsigned)(min(n0 + 16 * (g - TM) + ld_row, N - 1) - n0) * (unsigned)(K * 4)) + ld_chunk * 16;
     auto issue = [&](int stage, int step) {
       unsigned char* to = mine + stage * STAGE;
       const unsigned kb = step * STEP + ld_chunk * 4 < left ? (unsigned)(step * STEP * 4) : NO_CHUNK;
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(g < A_GROUPS ? a_view : w_view, (lds_at)(to + g * 1024), 16, (int)(off[g] + kb), 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(g < TM ? a_view : w_view, (lds_at)(to + g * 1024), 16, (int)(off[g] + kb), 0, 0, 0);
     };
-    const int lr = Frag::row(lane);
-    unsigned at[HALVES];
+    const int lr = lane & 15;
+    unsigned at[4];                                    // the lane's four k of a block
 #pragma unroll
-    for (int i = 0; i < HALVES; ++i) at[i] = (unsigned)(lr * 64 + ((Frag::chunk(lane, i) ^ (lr >> 2 & 3)) * 16));
-    auto read = [&](int stage, Frag (&fa)[TM], Frag (&fw)[TN]) {
+    for (int t = 0; t < 4; ++t) at[t] = (unsigned)(lr * 64 + ((t ^ (lr >> 2)) * 16) + (lane >> 4) * 4);
+    auto read = [&](int stage, Fragment (&fa)[TM], Fragment (&fw)[TN]) {
       const unsigned char* base = mine + stage * STAGE;
 #pragma unroll
-      for (int i = 0; i < HALVES; ++i) {
+      for (int t = 0; t < 4; ++t) {
 #pragma unroll
-        for (int t = 0; t < TN; ++t) fw[t].v[i] = *(const f32x4_t*)(base + (TM + t) * HALVES * 1024 + at[i]);
+        for (int n = 0; n < TN; ++n) fw[n][t] = *(const float*)(base + (TM + n) * 1024 + at[t]);
 #pragma unroll
-        for (int t = 0; t < TM; ++t) fa[t].v[i] = *(const f32x4_t*)(base + t * HALVES * 1024 + at[i]);
+        for (int m = 0; m < TM; ++m) fa[m][t] = *(const float*)(base + m * 1024 + at[t]);
       }
     };
-    constexpr int INSTRUCTIONS = 4 * HALVES, FIRST = INSTRUCTIONS / 2;
-    auto multiply = [&](const Frag (&fa)[TM], const Frag (&fw)[TN], auto from, auto to) {
+    auto multiply = [&](const Fragment (&fa)[TM], const Fragment (&fw)[TN], int half) {
 #pragma unroll
-      for (int t = decltype(from)::value; t < decltype(to)::value; ++t)
+      for (int t = 2 * half; t < 2 * half + 2; ++t)
 #pragma unroll
         for (int n = 0; n < TN; ++n)
 #pragma unroll
-          for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n](t), fa[m](t), acc[n][m]);
-    };
-    auto order = [&](Frag (&fa)[TM], Frag (&fw)[TN]) {
-#pragma unroll
-      for (int t = 0; t < TN; ++t) fw[t].order();
-#pragma unroll
-      for (int t = 0; t < TM; ++t) fa[t].order();
+          for (int m = 0; m < TM; ++m) acc[n][m] = matrix_step(fw[n][t], fa[m][t], acc[n][m]);
     };
     const int steps = (left + STEP - 1) / STEP;
-    Frag fa0[TM], fw0[TN], fa1[TM], fw1[TN];
+    Fragment fa0[TM], fw0[TN], fa1[TM], fw1[TN];
 #pragma unroll
     for (int i = 0; i < STAGES; ++i) issue(i, i);      // a step past the end loads zeros
     loads_but<(STAGES - 1) * GROUPS>();
     asm volatile("" ::: "memory");
     read(0, fa0, fw0);
-    order(fa0, fw0);
     int stage = 0;
-    // fa, fw: this step's operands, in order; the next one's are read while their first half is multiplied
-    auto step = [&](int s, Frag (&fa)[TM], Frag (&fw)[TN], Frag (&na)[TM], Frag (&nw)[TN]) {
+    // fa, fw: this step's operands; the next one's are read while their first half is multiplied
+    auto step = [&](int s, Fragment (&fa)[TM], Fragment (&fw)[TN], Fragment (&na)[TM], Fragment (&nw)[TN]) {
       const int next = stage + 1 == STAGES ? 0 : stage + 1;
       __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this step's operands are in registers, its stage is free
       asm volatile("" ::: "memory");
@@ -507,11 +442,10 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
       loads_but<(STAGES - 1) * GROUPS>();              // step s + 1 is there
       asm volatile("" ::: "memory");
       read(next, na, nw);
-      multiply(fa, fw, std::integral_constant<int, 0>{}, std::integral_constant<int, FIRST>{});
-      between_products<FIRST * TM * TN, GROUPS, 0>();
-      order(na, nw);
-      multiply(fa, fw, std::integral_constant<int, FIRST>{}, std::integral_constant<int, INSTRUCTIONS>{});
-      between_products<FIRST * TM * TN, 0, 0>();
+      multiply(fa, fw, 0);
+      between_products<2 * TM * TN, READS_OF<TM, TN>, 0>();
+      multiply(fa, fw, 1);
+      __builtin_amdgcn_sched_barrier(0);
       stage = next;
     };
     int s = 0;
@@ -528,10 +462,7 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m)
-#pragma unroll
-      for (int q = 0; q < QUADS; ++q)
-        *(f32x4_t*)(sums + (((size_t)wave * SUM_QUADS + (n * TM + m) * QUADS + q) * 64 + lane) * 4) =
-            f32x4_t{acc[n][m][4 * q], acc[n][m][4 * q + 1], acc[n][m][4 * q + 2], acc[n][m][4 * q + 3]};
+      *(f32x4_t*)(sums + (((size_t)wave * SUM_QUADS + n * TM + m) * 64 + lane) * 4) = acc[n][m];
   __syncthreads();
 #pragma unroll
   for (int b0 = 0; b0 < SUM_QUADS; b0 += 4) {
@@ -540,8 +471,7 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < SLAB_RANGES; ++w) v += *(const f32x4_t*)(sums + (((size_t)w * SUM_QUADS + b) * 64 + lane) * 4);
-    const int q = b % QUADS, m = b / QUADS % TM, n = b / QUADS / TM;
-    const int row = m0 + BLOCK * m + Frag::row(lane), column = n0 + BLOCK * n + sum_column<BLOCK>(lane, q);
+    const int row = m0 + 16 * (b % TM) + (lane & 15), column = n0 + 16 * (b / TM) + 4 * (lane >> 4);
     if constexpr (PARTS) store_outputs<false>(parts + (size_t)blockIdx.y * M * N, nullptr, v, row, column, M, N, N, N % 4 == 0);
     else store_outputs<ACCUMULATE>(C, bias, v, row, column, M, N, ldc, quads);
   }
@@ -668,7 +598,7 @@ inline bool stores_quads(const float* C, const float* bias, int N, long long ldc
 template <int TM, int TN, int WM, int WN, int STAGES>
 int launch_rows(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, long long lda, long long ldc,
                 int accumulate, hipStream_t s) {
-  constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, lds_bytes = STAGES * (BM + BN) * 128;
+  constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, lds_bytes = STAGES * (BM + BN) * 128;
   static bool configured = false;
   if (!configured) {
     hipError_t e = hipSuccess;
@@ -688,15 +618,15 @@ int launch_rows(const float* A, const float* W, const float* bias, float* C, int
   return 0;
 }
 
-template <int BLOCK, int TM, int TN, int STAGES>
+template <int TM, int TN, int STAGES>
 int launch_slabs(const float* A, const float* W, const float* bias, float* C, float* parts, int M, int N, int K, long long lda,
                  long long ldc, int accumulate, hipStream_t s) {
-  constexpr int BM = BLOCK * TM, BN = BLOCK * TN, lds_bytes = 4 * STAGES * (BM + BN) * 64;
+  constexpr int BM = 16 * TM, BN = 16 * TN, lds_bytes = 4 * STAGES * (BM + BN) * 64;
   static bool configured = false;
   if (!configured) {
     hipError_t e = hipSuccess;
-    for (const void* f : {(const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, false>, (const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, true>,
-                          (const void*)gemm_slab_kernel<BLOCK, TM, TN, STAGES, true, false>})
+    for (const void* f : {(const void*)gemm_slab_kernel<TM, TN, STAGES, false, false>, (const void*)gemm_slab_kernel<TM, TN, STAGES, false, true>,
+                          (const void*)gemm_slab_kernel<TM, TN, STAGES, true, false>})
       if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return (int)e;
     configured = true;
@@ -704,90 +634,61 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
   const int slabs = (K + SLAB_K - 1) / SLAB_K;
   const bool quads = stores_quads(C, bias, N, ldc);
   const dim3 grid((unsigned)(((M + BM - 1) / BM) * ((N + BN - 1) / BN)), slabs);
-  if (slabs > 1) gemm_slab_kernel<BLOCK, TM, TN, STAGES, true, false><<<grid, 256, lds_bytes, s>>>(A, W, nullptr, nullptr, parts, M, N, K, lda, 0, false);
-  else if (accumulate) gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, true><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
-  else gemm_slab_kernel<BLOCK, TM, TN, STAGES, false, false><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
+  if (slabs > 1) gemm_slab_kernel<TM, TN, STAGES, true, false><<<grid, 256, lds_bytes, s>>>(A, W, nullptr, nullptr, parts, M, N, K, lda, 0, false);
+  else if (accumulate) gemm_slab_kernel<TM, TN, STAGES, false, true><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
+  else gemm_slab_kernel<TM, TN, STAGES, false, false><<<grid, 256, lds_bytes, s>>>(A, W, bias, C, nullptr, M, N, K, lda, ldc, quads);
   VK_LAUNCH_CHECK();
   if (slabs == 1) return 0;
   return accumulate ? launch_finish<float, true>(parts, bias, C, M, N, ldc, slabs, 1, s)
                     : launch_finish<float, false>(parts, bias, C, M, N, ldc, slabs, 1, s);
 }
 
-// Which kernel an all-32-bit product of aligned rows takes.  Both cut M x N into tiles, one a workgroup; the last round of
-// tiles over the 256 CUs is as long as a full one while the rounds are few.  Times in us as measured (weights from memory), of
-// a round and beside the rounds:
-//   slab, 16 x 32 outputs   2.9 + 3.9 a round (tiles x slabs)    9 x 1,152 x 896: 6.7 (14.1 as 64 x 64 tiles cut over workgroups)
-//         32 x 32           3.2 + 6.2                            128 x 1,152 x 896: 9.1 (15.0)
-//         48 x 32           4.5 + 9.3                            333 x 1,152 x 896: 14.2 (20.3)
-//   slabs of 64 columns: by how many a CU holds at a time (Residents)
-//         32 x 64           15, 26.5, 32 for 1, 2, 3             200 x 896 x 4,864: 34.6 (37.0 as 32 x 32)
-//         48 x 64           20.5, 33                             333 x 896 x 4,864: 44.0 (55.5 as 64 x 64 tiles cut over workgroups)
-//         64 x 64           23, 38.5                             64 x 1,536 x 8,960: 31 (40.3)
-//     and, with several slabs, 5 for adding the parts and their way through memory
-//   rows, 64 x 64           7.5 + 0.0193 K a round               2,048 x 2,560 x 2,048: 210 (232)
-//         32 x 128          8 + 0.0207 K                         65 x 17,920 x 1,536: 68.9 (92.9)
-//         64 x 128          8 + 0.0365 K                         333 x 9,728 x 896: 72.8 (81.7); 2,048 x 37,888 x 3,584: 4,757 (5,358)
-// A slab's wave has a chain of loads and sums of its own, and what hides it is other workgroups of the CU, not more of its own
-// stages: with 2 stages instead of 4 two workgroups of 64 x 64 fit, which take 0.91 of the time over 216 sizes from 12 to
-// 2,048 rows (0.75 to 0.98 at each), and with 3 instead of 4 three of 32 x 32 (0.96); the tiles of 48 x 64 and 32 x 64 read less
-// for each output than narrower ones and leave room for 2 and 3 on a CU.  The choice takes 0.966 of the time it took without these
-// (geometric mean), 0.72 at best (65 x 2,048 x 11,008: 60.9 against 84.2) and 1.05 at worst (256 x 2,560 x 2,048: 43.7 against 41.8).
-// Over 112 sizes from 9 to 2,048 rows it took 0.80 of the time of the 64 x 64 tiles cut over workgroups without them, and 1.07 of
-// it at worst.  Those keep a product where their cut of K is estimated to be faster (512 x 896 x 4,864), any other
-// type, and rows off 16 bytes.
-enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128, SLAB_32_64, SLAB_48_64 };
-
-inline double rounds(long long tiles) { return tiles <= 3 * 256 ? (double)((tiles + 255) / 256) : tiles / 256.0 + 0.35; }
-
-// The same estimate for the 64 x 64 tiles, as they are cut (matrix_units).
-inline double estimate_matrix(int M, int N, int K, int units) {
-  const double tiles = (double)((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
-  if (units == 0) return 7 + fmax(1.0, tiles / 256 + 0.3) * K * 0.0205;
-  const int cuts = (K + units * RANGE_K - 1) / (units * RANGE_K);
-  const double parts = (double)cuts * M * N * 8 / 6e6, per_cu = tiles * cuts / 256;
-  return units == 1 ? 9.5 + fmax(5.0, (per_cu + 0.35) * 5.2) + parts : 9 + fmax(19.5, (per_cu + 0.15) * 18.5) + parts;
-}
-
-// Slabs of 64 columns: `resident` of them run on a CU at a time, and together they take us[resident - 1] for theirs.  The last
-// ones to start share a CU with as many others as are left; past two full rounds those of several slabs overlap.  Weights
-// whose rows are a multiple of 8 KB apart arrive 1.06 times as slowly, and 32 x 64 falls behind over rows of more than 8,192
-// (200 x 2,048 x 11,008: 169 us, 149 as 64 x 64 tiles cut over workgroups).
-struct Residents { Direct form; int rows, resident; double us[3], long_rows; };
-inline double resident_rounds(const Residents& f, long long tiles, int K) {
-  const long long chip = 256ll * f.resident, full = tiles / chip, left = tiles % chip;
-  const double round = f.us[f.resident - 1], last = left ? f.us[(left + 255) / 256 - 1] : 0.0;
-  return (full >= 2 && K > SLAB_K ? ((double)tiles / chip - 0.2) * round : full * round + last) *
-         (K % 2048 == 0 ? 1.06 : 1.0) * (K > 8192 ? f.long_rows : 1.0);
-}
+// Which kernel an all-32-bit product of aligned rows takes.  Both cut M x N into tiles, one a workgroup, and a call lasts as
+// long as the CU with the most of them: us = beside + step (tiles of that CU), as measured (weights from memory):
+//   slab, 16 x 32 outputs   4 + 3.3 (tiles x slabs)      12 x 1,152 x 896: 6.8 us (14.2 as 64 x 64 tiles cut over workgroups)
+//         32 x 32           3.9 + 4.9                    200 x 1,152 x 896: 10.3 (18.4)
+//         48 x 32           3.9 + 6.8                    333 x 1,152 x 896: 12.4 (21.2)
+//         48 x 48           4.5 + 9.7                    333 x 9,728 x 896: 62.1 (80.7)
+//         48 x 64           4.2 + 12.8                   333 x 896 x 4,864: 40.3 (54.2)
+//         64 x 64           4.7 + 16.3                   333 x 2,048 x 11,008: 167 (191)
+//     and, with several slabs, 3 for adding the parts and their way through memory; the smaller tiles fall behind by a fifth
+//     where rows are longer than 8,192 (333 x 2,048 x 11,008: 190 as 48 x 48)
+//   rows, 64 x 64           4.1 + 0.0164 K, and 0.0045 K for every three on a CU     256 x 9,728 x 896: 53.6 (65.0)
+//         32 x 128          4.8 + 0.0159 K, 0.0038 K for every two                   65 x 17,920 x 1,536: 61.9 (91.7)
+//         64 x 128          3.5 + 0.0313 K, 0.0055 K for every two                   333 x 9,728 x 896: 68.0 (80.7)
+// Two or three stages leave room for a second or third workgroup on a CU, which hide a wave's own chain of loads better than a
+// deeper queue of its own does (a slab's 64 x 64 with four stages took 1.10 of the time with two).  Over 233 sizes from 12 to
+// 2,048 rows the choice takes 0.885 of the time of the kernels that exchanged lanes' values and had no tiles of 48 x 48
+// (geometric mean), 1.006 of it at worst, and 1.012 of the best form's.  The 64 x 64 tiles cut over workgroups are the fastest at
+// none of them; they keep any other type, and rows off 16 bytes.
+enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128, SLAB_48_48, SLAB_48_64 };
 
 Direct direct_plan(int M, int N, int K, long long part_floats) {
-  struct Form { Direct form; int rows, columns; double beside, round; };
-  constexpr Form slab_forms[] = {{SLAB_16_32, 16, 32, 2.9, 3.9}, {SLAB_32_32, 32, 32, 3.2, 6.2}, {SLAB_48_32, 48, 32, 4.5, 9.3}};
-  constexpr Residents wide_slabs[] = {{SLAB_32_64, 32, 3, {15.0, 26.5, 32.0}, 1.2}, {SLAB_48_64, 48, 2, {20.5, 33.0}, 1.0},
-                                       {SLAB_64_64, 64, 2, {23.0, 38.5}, 1.0}};
-  constexpr Form row_forms[] = {{ROWS_64_64, 64, 64, 7.5, 0.0193}, {ROWS_32_128, 32, 128, 8.0, 0.0207}, {ROWS_64_128, 64, 128, 8.0, 0.0365}};
+  struct Form { Direct form; int rows, columns, resident; double beside, step, together, over; };
+  constexpr Form slab_forms[] = {{SLAB_16_32, 16, 32, 4, 4.0, 3.3}, {SLAB_32_32, 32, 32, 5, 3.9, 4.9}, {SLAB_48_32, 48, 32, 4, 3.9, 6.8},
+                                 {SLAB_48_48, 48, 48, 3, 4.5, 9.7}, {SLAB_48_64, 48, 64, 2, 4.2, 12.8}, {SLAB_64_64, 64, 64, 2, 4.7, 16.3}};
+  constexpr Form row_forms[] = {{ROWS_64_64, 64, 64, 3, 4.1, 0.0164, 0.0045, 0.25}, {ROWS_32_128, 32, 128, 2, 4.8, 0.0159, 0.0038, 0.6},
+                                {ROWS_64_128, 64, 128, 2, 3.5, 0.0313, 0.0055, 0.5}};
   const long long slabs = (K + SLAB_K - 1) / SLAB_K;
-  const double parts = slabs == 1 ? 0.0 : 5.0 + (double)slabs * M * N * 8 / 6e6;
-  double best = 0.97 * estimate_matrix(M, N, K, part_floats > 0 ? matrix_units(M, N, K) : 0);
+  const double parts = slabs == 1 ? 0.0 : 3.0 + 1.1 * slabs * M * N * 8 / 6e6;
+  const double pitch = K % 2048 == 0 ? 1.04 : 1.0;     // weights whose rows are a multiple of 8 KB apart
+  double best = 1e300;
   Direct chosen = NOT_DIRECT;
-  auto tiles = [&](int rows, int columns) { return (long long)((M + rows - 1) / rows) * ((N + columns - 1) / columns); };
-  auto offer = [&](Direct form, long long count, double us) {
-    if (count <= 0xffffffffll / 256 && us < best) best = us, chosen = form;
+  auto offer = [&](const Form& f, long long tiles, double us) {
+    if (tiles <= 0xffffffffll / 256 && us < best) best = us, chosen = f.form;
   };
-  if (slabs == 1 || slabs * M * N <= part_floats) {
+  auto tiles_of = [&](const Form& f) { return (long long)((M + f.rows - 1) / f.rows) * ((N + f.columns - 1) / f.columns); };
+  if (slabs == 1 || slabs * M * N <= part_floats)
     for (const Form& f : slab_forms) {
-      const long long count = tiles(f.rows, f.columns);
-      offer(f.form, count, f.beside + f.round * rounds(count * slabs) + parts);
+      const long long tiles = tiles_of(f);
+      const double each = tiles * slabs / 256.0;       // past what is resident a CU short of its share waits for none; past 8 they even out
+      const double most = each > 8 ? each + 0.5 : each > f.resident ? ceil(each + 0.05) : ceil(each);
+      offer(f, tiles, (f.beside + f.step * most) * pitch * (K > 8192 && f.form != SLAB_64_64 ? 1.2 : 1.0) + parts);
     }
-    for (const Residents& f : wide_slabs) {
-      if (M <= 32) break;              // one row of tiles: narrower ones have more of the weight in flight (24 x 17,920 x 1,536: 40 against 45 us)
-      const long long count = tiles(f.rows, 64);
-      offer(f.form, count, resident_rounds(f, count * slabs, K) + parts);
-    }
-  }
   for (const Form& f : row_forms) {
-    const long long count = tiles(f.rows, f.columns);
-    offer(f.form, count, f.beside + f.round * K * rounds(count) * (K > SLAB_K && count <= 256 ? 1.07 : 1.0));
+    const long long tiles = tiles_of(f);
+    const double each = tiles / 256.0, most = ceil(each) > 2 * f.resident ? each + f.over : ceil(each);
+    offer(f, tiles, f.beside + (f.step * most + f.together * ceil(most / f.resident)) * K * pitch);
   }
   return chosen;
 }
@@ -795,15 +696,15 @@ Direct direct_plan(int M, int N, int K, long long part_floats) {
 int launch_direct(Direct form, const float* A, const float* W, const float* bias, float* C, float* parts, int M, int N, int K,
                   long long lda, long long ldc, int accumulate, hipStream_t s) {
   switch (form) {
-    case SLAB_16_32: return launch_slabs<16, 1, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_32_32: return launch_slabs<32, 1, 1, 3>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_48_32: return launch_slabs<16, 3, 2, 4>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_32_64: return launch_slabs<32, 1, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_48_64: return launch_slabs<16, 3, 4, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case SLAB_64_64: return launch_slabs<32, 2, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
-    case ROWS_64_64: return launch_rows<1, 1, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case ROWS_32_128: return launch_rows<1, 1, 1, 4, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
-    case ROWS_64_128: return launch_rows<1, 2, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_16_32: return launch_slabs<1, 2, 3>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_32_32: return launch_slabs<2, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_48_32: return launch_slabs<3, 2, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_48_48: return launch_slabs<3, 3, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_48_64: return launch_slabs<3, 4, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case SLAB_64_64: return launch_slabs<4, 4, 2>(A, W, bias, C, parts, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_64_64: return launch_rows<2, 2, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_32_128: return launch_rows<2, 2, 1, 4, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
+    case ROWS_64_128: return launch_rows<2, 4, 2, 2, 3>(A, W, bias, C, M, N, K, lda, ldc, accumulate, s);
     case NOT_DIRECT: break;
   }
   return VK_BAD_ARGUMENT;
