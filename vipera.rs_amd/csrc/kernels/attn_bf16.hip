@@ -63,6 +63,19 @@ __device__ __forceinline__ bf16x8 keep_before_end(bf16x8 v, int head, int tail) 
   return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & mask);
 }
 
+// Hints for the order of COUNT matrix instructions and the LDS reads of their operands, written since the last such line:
+// AHEAD reads first (0: they went out before), then one behind each product, READS altogether.  Left to itself the compiler
+// keeps one or two reads in flight.
+template <int COUNT, int AHEAD, int READS>
+__device__ __forceinline__ void reads_ahead() {
+  if constexpr (AHEAD > 0) __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+  for (int i = 0; i < COUNT; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if (i < READS - AHEAD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+}
+
 // A column's four lanes (lanes c, c + 16, c + 32, c + 48) combine their values with two lane swaps that run in the
 // vector ALU (v_permlane16_swap exchanges the odd 16-lane rows of one register with the even rows of another,
 // v_permlane32_swap the upper half of one with the lower half of another; with both registers holding v, the two
@@ -584,16 +597,20 @@ constexpr int PD_PARTIAL_ROW = HDP + 4;   // floats of a column's partial result
 // PARTS 2 (with SPLIT): the tile's 128 columns are shared between two workgroups of eight waves, each of which walks the tile's
 // positions, in the halves of the whole tile: every column's sums are those of PARTS 1. For items that are no more than the CUs:
 // what a step costs a CU is its waves' products, exponentials and LDS reads, behind one another. us, one workgroup a tile against two: 512 tokens
-// of 16 heads of 128 at 1,536 47.3 / 35.5, 1,000 of 12 28.2 / 22.3, 333 of 14 heads of 64 10.7 / 8.5, 1,200 of 16 (160 tiles) 31.3 /
-// 26.5, 1,834 of 16 (240) 28.2 / 28.1; a quarter of the columns a workgroup measured as a half does where it has a CU and up to
-// twice as long where it has not. With half the waves there are the registers to spread the next tile's loads over this one's parts and to
-// take the tile that holds the end in a loop of its own (38.2 to 35.5 of the first), which cost the other forms their second
-// workgroup a CU (61 to 82 us).
+// of 16 heads of 128 at 1,536 40.4 / 30.2, 1,000 of 12 24.0 / 18.5, 333 of 14 heads of 64 10.0 / 8.1, 1,200 of 16 (160 tiles) 26.7 /
+// 20.7, 1,834 of 16 (240) 24.6 / 24.9; a quarter of the columns a workgroup measured as a half does where it has a CU and up to
+// twice as long where it has not.
+//
+// A tile's loads go out before anything else of the last one, and its operands come from LDS four ahead of their products, the
+// first values while the exponentials run. us before and since, when a branch around the masking of the values past the end stood between
+// every two products and the compiler read one operand ahead: whole tiles, 2,048 tokens of 28 heads of 128 60.4 / 52.7; halved,
+// 512 of 16 at 1,536 44.2 / 40.4; shared by two workgroups 35.4 / 30.2 (their loads, spread over the tile, 33.0); cut, 200 of 12 at
+// 1,800 21.2 / 20.0. Eight ahead gained nothing where registers allow it.
 //
 // WIDE: the cache is 4 GB or more, and a load's address is 64 bits wide; else it is an offset behind a buffer descriptor, which
 // takes fewer vector instructions and registers (one prompt of 2,048 tokens, 28 heads, whole tiles 69.3 to 60.6 us, halved 59.5 to 57.2).
 template <bool SPLIT, bool CHUNKED, int PARTS, bool WIDE>
-__global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void attn_prefill_direct_kernel(
+__global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS, HDP <= 128 && PARTS == 1 ? 4 : 1) void attn_prefill_direct_kernel(
     const __bf16* __restrict__ q, long long q_stride, const __bf16* __restrict__ k_cache,
     const __bf16* __restrict__ v_cache, __bf16* __restrict__ out, const int* __restrict__ tiles,
     const int* __restrict__ entry_start, const int* __restrict__ entry_first_pos,
@@ -604,6 +621,7 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
   static_assert(PARTS == 1 || (SPLIT && PT_WAVES % PARTS == 0), "only halved tiles are shared");
   constexpr int WAVES = PT_WAVES / PARTS;                                           // of a half
   constexpr int PD_KLOADS = PD_KBYTES / 1024 / WAVES, PD_VLOADS = PD_VBYTES / 1024 / WAVES;   // load instructions per wave and tile
+  constexpr int READS = 4;                                                          // operands asked for ahead of their products
   typedef __attribute__((address_space(3))) void* lds_ptr;
   typedef __attribute__((address_space(1))) const void* global_ptr;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];  // [2][K tile | V^T tile]
@@ -676,8 +694,8 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
   // Per lane and load instruction: which page of a tile its chunk lies in and where in that page; both are the
   // same for every tile, since tiles start at multiples of 64 and the page size divides 64. Nothing is loaded
   // conditionally: a chunk outside [begin, end) reads a page of the same request inside that range, and its
-  // positions are masked, or weigh zero, for every column; the V^T operands of the tile that holds `end` are
-  // zeroed from `end` on (keep_before_end), since the slots there may hold anything.
+  // positions are masked, or weigh zero, for every column; the V^T rows of the tile that holds `end` are zeroed
+  // from `end` on in LDS (keep_values_before_end), since the slots there may hold anything.
   int k_tab[PD_KLOADS], v_tab[PD_VLOADS];
   unsigned k_in[PD_KLOADS], v_in[PD_VLOADS];
   const unsigned page_bytes = (unsigned)(kv_heads * bs * hd * 2);
@@ -713,19 +731,13 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)to, 16, (int)((unsigned)page * page_bytes + in), 0, 0, 0);
   };
-  auto issue = [&](int stage, int quarter) {   // a quarter of a tile's loads
+  auto issue = [&](int stage) {
     unsigned char* to_k = lds_half + stage * PD_STAGE + wave * PD_KLOADS * 1024;
     unsigned char* to_v = lds_half + stage * PD_STAGE + PD_KBYTES + wave * PD_VLOADS * 1024;
 #pragma unroll
-    for (int i = 0; i < PD_KLOADS; ++i)
-      if (i % 4 == quarter) load(k_cache, k_rsrc, k_page[i], k_in[i], to_k + i * 1024);
+    for (int i = 0; i < PD_KLOADS; ++i) load(k_cache, k_rsrc, k_page[i], k_in[i], to_k + i * 1024);
 #pragma unroll
-    for (int i = 0; i < PD_VLOADS; ++i)
-      if ((PD_KLOADS + i) % 4 == quarter) load(v_cache, v_rsrc, v_page[i], v_in[i], to_v + i * 1024);
-  };
-  auto issue_all = [&](int stage) {
-#pragma unroll
-    for (int quarter = 0; quarter < 4; ++quarter) issue(stage, quarter);
+    for (int i = 0; i < PD_VLOADS; ++i) load(v_cache, v_rsrc, v_page[i], v_in[i], to_v + i * 1024);
   };
 
   // a lane's operand addresses within a stage
@@ -743,20 +755,20 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
   const float cap_raw = softcap > 0.f ? softcap / scale : 0.f, cap_inv = softcap > 0.f ? scale / softcap : 0.f;
   const float* rel_row = ex.rel ? ex.rel + (size_t)h * (ex.rel_far + 1) : nullptr;
   const float inv_scale = 1.f / scale;
-  // `next` (PARTS 2): whether the next tile's loads go out between this one's parts, into `next_stage`
-  auto tile_body = [&](bool masked, int p0, const unsigned char* base, bool next, int next_stage) {
+  auto tile_body = [&](bool masked, int p0, const unsigned char* base) {
     // ---- scores: tile sub = 2 st + t holds positions p0 + 32 st + 8 g + 4 t + j in register j of lane group g
     f32x4 s[4];
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int st = 0; st < 2; ++st) {
+      s[2 * st] = s[2 * st + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8 kf = *(const bf16x8*)(base + k_at[ks] + ((sub >> 1) * 32 + (sub & 1) * 4) * PD_ROWB);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], acc, 0, 0, 0);
-      }
-      s[sub] = acc;
-      if (PARTS > 1 && (sub & 1) && next) issue(next_stage, sub >> 1);
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const bf16x8 kf = *(const bf16x8*)(base + k_at[ks] + (st * 32 + t * 4) * PD_ROWB);
+          s[2 * st + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[2 * st + t], 0, 0, 0);
+        }
+      reads_ahead<2 * KS, READS, 2 * KS>();
     }
     if (softcap > 0.f) {   // raw scores whose product with the scale is the capped score
 #pragma unroll
@@ -797,7 +809,11 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
     }
     // No branch around the weights: a column that sees nothing yet has m = -inf and only masked scores, which
     // give exp2(-inf - 0) = 0, as a masked score under a finite m does.
-    bf16x8 pf[2];
+    bf16x8 pf[2], vf[READS];   // the first values arrive while the exponentials run
+    auto value = [&](int i) { return *(const bf16x8*)(base + v_at[i % 2] + i / 2 * 16 * 128); };
+#pragma unroll
+    for (int i = 0; i < READS; ++i) vf[i] = value(i);
+    __builtin_amdgcn_sched_barrier(0);
     {
       const float mc = m_new > -INFINITY ? m_new * c2 : 0.f;
       float sum = 0.f;
@@ -809,26 +825,29 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
       }
       l += sum;
     }
-    if (PARTS > 1 && next) issue(next_stage, 2);
-    auto weigh = [&](auto tail) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        if (PARTS > 1 && dt == DT / 2 && next) issue(next_stage, 3);
+    for (int i = 0; i < 2 * DT; ++i) {
+      o[i / 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i % READS], pf[i % 2], o[i / 2], 0, 0, 0);
+      if (i + READS < 2 * DT) vf[i % READS] = value(i + READS);
+    }
+    reads_ahead<2 * DT, 0, 2 * DT - READS>();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The tile that holds `end`: a wave zeroes the values from there on in what it has loaded itself, before the barrier that
+  // hands the tile to the others.
+  const int my_p8 = ((lane & 7) ^ (lane >> 3)) * 8;   // the first of the lane's eight positions of a V^T row, in every load
+  auto keep_values_before_end = [&](int stage, int p0) {
+    wait_own_loads();   // a barrier alone does not wait for loads that write LDS
+    if (p0 + PT_KV <= end) return;
+    asm volatile("" ::: "memory");
+    unsigned char* loaded = lds_half + stage * PD_STAGE + PD_KBYTES + wave * PD_VLOADS * 1024 + lane * 16;
+    const int kept = end - (p0 + my_p8);
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          bf16x8 vf = *(const bf16x8*)(base + v_at[st] + dt * 16 * 128);
-          if (tail) {
-            const int kept = end - (p0 + st * 32 + lg * 8);
-            vf = keep_before_end(vf, kept, kept - 4);
-          }
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[st], o[dt], 0, 0, 0);
-        }
-      }
-    };
-    const bool tail = p0 + PT_KV > end;
-    if constexpr (PARTS == 1) weigh(tail);
-    else if (tail) weigh(std::true_type{});
-    else weigh(std::false_type{});
+    for (int i = 0; i < PD_VLOADS; ++i) {
+      bf16x8* at = (bf16x8*)(loaded + i * 1024);
+      *at = keep_before_end(*at, kept, kept - 4);
+    }
   };
 
   // this half's tiles: all of them, or with SPLIT the first or the second half of them (both halves pass the
@@ -837,9 +856,9 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
   const int my_tiles = half ? all_tiles - steps : steps;
   const int my_first = CHUNKED ? chunk * chunk_tiles : half ? steps : 0;   // in tiles of the walk
   lookup(walk.at(my_first));
-  if (my_tiles > 0) issue_all(0);
+  if (my_tiles > 0) issue(0);
   lookup(walk.at(my_first + 1));
-  wait_own_loads();
+  keep_values_before_end(0, walk.at(my_first));
   __syncthreads();
   int stage = 0;
   for (int i = 0; i < steps; ++i) {
@@ -847,18 +866,12 @@ __global__ __launch_bounds__((SPLIT ? 2 * PT_THREADS : PT_THREADS) / PARTS) void
     const bool next = i + 1 < my_tiles;   // into the stage that nobody reads any more: the barrier that ended the last tile
     const bool sees = i < my_tiles && p0 < wave_end && (p0 + PT_KV > wave_begin || p0 < ex.keep_first);
     const bool masked = !(p0 + PT_KV - 1 <= wave_first && p0 >= wave_lo_max);
-    if constexpr (PARTS == 1) {
-      if (next) {
-        issue_all(stage ^ 1);
-        lookup(walk.at(my_first + i + 2));
-      }
-      if (sees) tile_body(masked, p0, lds_half + stage * PD_STAGE, next, stage ^ 1);
-    } else {
-      if (sees) tile_body(masked, p0, lds_half + stage * PD_STAGE, next, stage ^ 1);
-      else if (next) issue_all(stage ^ 1);
-      if (next) lookup(walk.at(my_first + i + 2));
+    if (next) {
+      issue(stage ^ 1);
+      lookup(walk.at(my_first + i + 2));
     }
-    wait_own_loads();   // a barrier alone does not wait for loads that write LDS
+    if (sees) tile_body(masked, p0, lds_half + stage * PD_STAGE);
+    keep_values_before_end(stage ^ 1, next ? walk.at(my_first + i + 1) : 0);
     __syncthreads();
     stage ^= 1;
   }
