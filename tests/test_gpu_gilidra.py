@@ -394,6 +394,50 @@ def test_the_trace_runner_replays_a_schedule(tmp_path, g2):
         assert rel_err(got, np.stack(want)) < TOL["float32"]
 
 
+@pytest.mark.parametrize("taps,sizes", [(4, (2, 4, 128, 128)), (4, (1, 3, 64, 40)), (3, (2, 2, 256, 24)), (2, (3, 3, 64, 72))])
+def test_prompts_prepared_in_runs_give_the_bits_of_single_tokens(taps, sizes):
+    """delta_prepare of a step of 128 tokens or more, a run of four a thread, against the same tokens in steps of fewer: entries
+    that begin and end inside a run, at position 0 and behind a state, heads of one to four waves, channels that end inside a
+    workgroup."""
+    from vipera_rs_amd.ops import kernels
+
+    kv_heads, heads, dim, vdim = sizes
+    lengths, first = (77, 1, 2, 120, 3), (0, 5, 0, 40, 0)
+    channels, tokens = 2 * kv_heads * dim + heads * vdim, sum(lengths)
+    g = torch.Generator("cuda").manual_seed(channels + taps)
+    randn = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    proj, conv = randn(tokens, channels + 2 * heads + 3), randn(channels, taps)
+    state0, a_log, dt_bias = randn(6, (taps - 1) * channels + 7), randn(heads), randn(heads)
+    i32 = lambda a: torch.tensor(list(a), dtype=torch.int32, device="cuda")
+    starts = [0, *np.cumsum(lengths)]
+
+    def walk(most):
+        state = state0.clone()
+        qkv, beta, decay = (torch.full((tokens, n), float("nan"), device="cuda") for n in (channels, heads, heads))
+        done = [0] * len(lengths)
+        while any(d < n for d, n in zip(done, lengths)):
+            left, step = most, []
+            for e, n in enumerate(lengths):
+                take = min(n - done[e], left)
+                left -= take
+                if take:
+                    step.append((e, take))
+            rows = torch.tensor([starts[e] + done[e] + j for e, n in step for j in range(n)], device="cuda")
+            got = [torch.full((len(rows), n), float("nan"), device="cuda") for n in (channels, heads, heads)]
+            kernels.delta_prepare(proj[rows], conv, state, 7, i32(i for i, (_, n) in enumerate(step) for _ in range(n)),
+                                  i32(np.cumsum([0] + [n for _, n in step])), i32(first[e] + done[e] for e, _ in step),
+                                  i32(5 - e for e, _ in step), a_log, dt_bias, kv_heads, dim, heads, vdim, channels + 1,
+                                  channels + 1 + heads, 1e-6, *got, len(step))
+            for whole, part in zip((qkv, beta, decay), got):
+                whole[rows] = part
+            for e, n in step:
+                done[e] += n
+        return qkv, beta, decay, state
+
+    for whole, part in zip(walk(tokens), walk(13)):
+        assert torch.equal(whole, part)
+
+
 @pytest.mark.parametrize("rule", ["delta", "delta_channel", "wkv"])
 @pytest.mark.parametrize("sizes", [(1, 2, 20, 9), (2, 4, 64, 16), (1, 3, 72, 8), (2, 2, 128, 24), (1, 1, 200, 5)])
 def test_prompts_recurrences_in_whole_and_partial_blocks(rule, sizes):

@@ -88,6 +88,80 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     }
 }
 
+// The same for prompts' portions, every number formed as above: a thread per channel and PREP_RUN consecutive tokens of the
+// step, whose rows it asks for at once; the heads' sums of squares meet in LDS, a token's wave by wave as block_sum adds
+// them.  Above, a workgroup of one token and 128 channels of its head leaves half its threads idle and waits for entry, taps and
+// inputs one behind another, a few microseconds for a kilobyte.  dim: 64, 128 or 256, so that a head lies in one workgroup.
+// us with the state's rows after it, 4,096 channels of four taps, before and so: 2,048 tokens 74.0 / 26.3 (their rows' way from
+// and to memory takes some 15), 512 25.4 / 10.8, 128 9.9 / 7.9; 100 tokens of 2,048 channels 7.5 / 7.8.  Runs of 8: 25.4, 11.6 and
+// 10.4; of 16: 24.5, 16.1 and 15.3.
+constexpr int PREP_RUN = 4, PREP_RUN_TOKENS = 128;
+template <int TAPS>
+__global__ __launch_bounds__(256) void delta_prepare_run_kernel(
+    const float* __restrict__ proj, long long ldp, const float* __restrict__ conv, const float* __restrict__ state,
+    long long state_stride, long long conv_offset, const int* __restrict__ entry_of, const int* __restrict__ entry_start,
+    const int* __restrict__ entry_first, const int* __restrict__ slots, const float* __restrict__ a_log,
+    const float* __restrict__ dt_bias, int kv_heads, int dim, int heads, int vdim, int b_col, int a_col, float unit_eps,
+    float* __restrict__ qkv, long long ldq, float* __restrict__ beta, float* __restrict__ decay, int num_tokens) {
+  __shared__ float squares[PREP_RUN][4];
+  const int t0 = blockIdx.x * PREP_RUN, tokens = min(PREP_RUN, num_tokens - t0);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int unit_channels = 2 * kv_heads * dim, C = unit_channels + heads * vdim;
+  const int first = blockIdx.y * 256, c = first + threadIdx.x, from = min(c, C - 1);
+  const bool unit = first + wave * 64 < unit_channels;      // heads begin at multiples of 64
+  float w[TAPS], in[PREP_RUN + TAPS - 1], y[PREP_RUN];
+#pragma unroll
+  for (int i = 0; i < PREP_RUN + TAPS - 1; ++i)
+    in[i] = proj[(long long)min(max(t0 + i - (TAPS - 1), 0), num_tokens - 1) * ldp + from];
+#pragma unroll
+  for (int i = 0; i < TAPS; ++i) w[i] = conv[(long long)from * TAPS + i];
+#pragma unroll
+  for (int j = 0; j < PREP_RUN; ++j) {
+    const int t = min(t0 + j, num_tokens - 1), e = entry_of[t], offset = t - entry_start[e];
+    float sum = 0.f;
+    if (offset >= TAPS - 1) {
+#pragma unroll
+      for (int i = 0; i < TAPS; ++i) sum = fmaf(w[i], in[j + i], sum);
+    } else {       // the entry's first tokens: what came before them is the state, or nothing
+      const bool fresh = entry_first[e] == 0;
+      const float* old = state + (long long)slots[e] * state_stride + conv_offset + from;
+#pragma unroll
+      for (int i = 0; i < TAPS; ++i) {
+        const int before = TAPS - 1 - i - offset;      // tokens before the entry's first
+        sum = fmaf(w[i], before <= 0 ? in[j + i] : fresh ? 0.f : old[(long long)(TAPS - 1 - before) * C], sum);
+      }
+    }
+    y[j] = silu_f(sum);
+  }
+  if (unit) {
+#pragma unroll
+    for (int j = 0; j < PREP_RUN; ++j) {
+      const float sum = wave_sum(fmaf(y[j], y[j], 0.f));      // a square of its own, not a term of the first addition
+      if ((threadIdx.x & 63) == 0) squares[j][wave] = sum;
+    }
+  }
+  __syncthreads();
+  const int head_waves = dim / 64, head_wave = unit ? wave / head_waves * head_waves : 0;
+#pragma unroll
+  for (int j = 0; j < PREP_RUN; ++j) {
+    float scale = 1.f;
+    if (unit) {
+      float total = 0.f;
+      for (int i = 0; i < head_waves; ++i) total += squares[j][head_wave + i];
+      scale = 1.0f / sqrtf(total + unit_eps);
+      if (first + wave * 64 < kv_heads * dim) scale *= 1.0f / sqrtf((float)dim);
+    }
+    if (j < tokens && c < C) qkv[(long long)(t0 + j) * ldq + c] = y[j] * scale;
+  }
+  if (blockIdx.y == 0)
+    for (int i = threadIdx.x; i < tokens * heads; i += 256) {
+      const int t = t0 + i / heads, h = i % heads;
+      const float* p = proj + (long long)t * ldp;
+      beta[(long long)t * heads + h] = sigmoid_f(p[b_col + h]);
+      if (a_col >= 0) decay[(long long)t * heads + h] = expf(-expf(a_log[h]) * softplus_f(p[a_col + h] + dt_bias[h]));
+    }
+}
+
 // The convolution's inputs of an entry's last taps - 1 tokens become the state.  Grid (entries, ceil(C / 256)), a
 // thread per channel; runs after delta_prepare has read the old rows.
 __global__ __launch_bounds__(256) void conv_state_kernel(const float* __restrict__ proj, long long ldp, int taps, int C,
@@ -961,9 +1035,20 @@ extern "C" int vk_delta_prepare_strided(const float* proj, long long ldp, const 
   hipStream_t s = (hipStream_t)stream;
   const long long segments = 2LL * kv_heads + ((long long)heads * vdim + PREP_SPAN - 1) / PREP_SPAN;
   if (segments > 65535) return VK_UNSUPPORTED_SIZE;
-  delta_prepare_kernel<<<dim3(num_tokens, (unsigned)segments), 256, 0, s>>>(
-      proj, ldp, conv, taps, state, state_stride, conv_offset, entry_of, entry_start, entry_first, slots, a_log, dt_bias,
-      kv_heads, dim, heads, vdim, b_col, a_col, unit_eps, qkv, ldq, beta, decay);
+  const dim3 run_grid((num_tokens + PREP_RUN - 1) / PREP_RUN, (unsigned)((C + 255) / 256));
+#define VK_PREPARE_RUN(TAPS)                                                                                            \
+  delta_prepare_run_kernel<TAPS><<<run_grid, 256, 0, s>>>(proj, ldp, conv, state, state_stride, conv_offset, entry_of,   \
+                                                          entry_start, entry_first, slots, a_log, dt_bias, kv_heads, dim, \
+                                                          heads, vdim, b_col, a_col, unit_eps, qkv, ldq, beta, decay, num_tokens)
+  const bool runs = (dim == 64 || dim == 128 || dim == 256) && num_tokens >= PREP_RUN_TOKENS && run_grid.y <= 65535;
+  if (runs && taps == 4) VK_PREPARE_RUN(4);
+  else if (runs && taps == 3) VK_PREPARE_RUN(3);
+  else if (runs && taps == 2) VK_PREPARE_RUN(2);
+  else
+    delta_prepare_kernel<<<dim3(num_tokens, (unsigned)segments), 256, 0, s>>>(
+        proj, ldp, conv, taps, state, state_stride, conv_offset, entry_of, entry_start, entry_first, slots, a_log, dt_bias,
+        kv_heads, dim, heads, vdim, b_col, a_col, unit_eps, qkv, ldq, beta, decay);
+#undef VK_PREPARE_RUN
   VK_LAUNCH_CHECK();
   if (taps > 1) {
     conv_state_kernel<<<dim3(num_entries, (unsigned)((C + 255) / 256)), 256, 0, s>>>(
