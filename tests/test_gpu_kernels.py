@@ -1384,3 +1384,62 @@ def test_32_bit_prompt_attention_at_the_edges_of_its_tiles(heads, kv_heads, hd, 
         kernels.attn_prefill_f32(qkv, k, v, got, tiles, 64, ints(starts), ints(first), table, heads, kv_heads, hd, hd ** -0.5, window,
                                  softcap=cap, extras=extras)
         assert _rel(got.cpu(), want.cpu().double()) < 2e-6
+
+
+@pytest.mark.parametrize("rows,width", [(3, 64), (37, 132), (5, 1028), (9, 4100)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_passes_over_rows_in_fours_give_the_bits_of_one_number_at_a_time(rows, width, dtype):
+    """activation, swiglu, head_unpack_gate and scan_prepare where every row lies in pieces of four numbers, against the same
+    numbers in rows that do not (an odd stride or an odd width)."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator(DEV).manual_seed(width)
+    randn = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    odd = lambda x, spare=1: torch.cat([x, x[:, :spare]], dim=1)[:, :x.shape[1]]      # a view of rows one number longer
+    x, factor = randn(rows, width).to(dtype), randn(rows, width)
+    for kind in kernels.ACTIVATIONS:
+        for mul in (None, factor):
+            out, apart = torch.empty(rows, width, dtype=dtype, device=DEV), torch.empty(rows, width, dtype=dtype, device=DEV)
+            kernels.activation(x, kind, out, mul)
+            kernels.activation(odd(x), kind, apart, mul)
+            assert torch.equal(out, apart)
+    both, pairs = randn(rows, 2 * width).to(dtype), torch.empty(rows, width, dtype=dtype, device=DEV)
+    kernels.swiglu(both, pairs)
+    lone = torch.empty(rows, width + 1, dtype=dtype, device=DEV)
+    kernels.swiglu(torch.cat([odd(both[:, :width + 1])[:, :width], both[:, :1], both[:, width:], both[:, :1]], dim=1).contiguous(), lone)
+    assert torch.equal(pairs, lone[:, :width])
+    heads = randn(rows, 2 * width).to(dtype)                    # two heads of width - 4 in width columns each
+    gate, n = randn(rows, 2 * (width - 4)), width - 4
+    out, apart = (torch.empty(rows, 2 * n, dtype=dtype, device=DEV) for _ in range(2))
+    kernels.head_unpack_gate(heads, gate, "sigmoid", 2, n, width, out)
+    kernels.head_unpack_gate(heads, odd(gate), "sigmoid", 2, n, width, apart)
+    assert torch.equal(out, apart)
+    step, bias, z = randn(rows, width), randn(width), randn(rows, width)
+    ones, gates, alone = odd(step), torch.empty(rows, width, device=DEV), torch.empty(rows, width, device=DEV)
+    kernels.scan_prepare(ones, bias, odd(z), alone)
+    kernels.scan_prepare(step, bias, z, gates)
+    assert torch.equal(step, ones) and torch.equal(gates, alone)
+
+
+@pytest.mark.parametrize("tokens,width,dtype", [(514, 36, torch.bfloat16), (515, 1028, torch.float32), (640, 64, torch.bfloat16)])
+def test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, width, dtype):
+    """A step of 512 tokens or more against the same tokens in smaller steps: entries that begin inside a run, behind a state and at
+    position 0."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator(DEV).manual_seed(tokens)
+    h, mu = torch.randn(tokens, width, generator=g, device=DEV).to(dtype), torch.randn(3, width, generator=g, device=DEV)
+    saved = torch.randn(5, width + 8, generator=g, device=DEV)
+    i32 = lambda a: torch.tensor(list(a), dtype=torch.int32, device=DEV)
+    starts, first, slots = [0, 201, 202, 205, tokens], [0, 7, 0, 3], [4, 0, 2, 1]
+    whole, parts, left = torch.empty(3, tokens, width, dtype=dtype, device=DEV), torch.empty(3, tokens, width, dtype=dtype, device=DEV), saved.clone()
+    entry = lambda pieces: i32(i for i, (lo, hi) in enumerate(pieces) for _ in range(lo, hi))
+    all_of = list(zip(starts[:-1], starts[1:]))
+    kernels.token_shift(h, mu, left, 4, entry(all_of), i32(starts), i32(first), i32(slots), whole, 4)
+    one = saved.clone()
+    for e, (lo, hi) in enumerate(all_of):
+        for at in range(lo, hi, 150):
+            end = min(at + 150, hi)
+            piece = torch.empty(3, end - at, width, dtype=dtype, device=DEV)
+            kernels.token_shift(h[at:end].contiguous(), mu, one, 4, i32([0] * (end - at)), i32([0, end - at]), i32([first[e] + at - lo]), i32([slots[e]]),
+                                piece, 1)
+            parts[:, at:end] = piece
+    assert torch.equal(whole, parts) and torch.equal(left, one)

@@ -713,6 +713,59 @@ __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ 
   }
 }
 
+// The same for many tokens: four channels of SHIFT_RUN consecutive tokens a thread, so that a vector of factors is read once for
+// them and everything moves in pieces of four numbers.  2,048 tokens of 2,048 channels, six vectors, 16-bit: 27.0 -> 15.5 us;
+// 512 of them 14.0 -> 8.3.
+constexpr int SHIFT_RUN = 4;
+template <typename T>
+__global__ __launch_bounds__(256) void token_shift_run_kernel(const T* __restrict__ h, int width, const float* __restrict__ mu,
+                                                              int mixes, const float* __restrict__ state,
+                                                              long long state_stride, long long prev_offset,
+                                                              const int* __restrict__ entry_of,
+                                                              const int* __restrict__ entry_start,
+                                                              const int* __restrict__ entry_first,
+                                                              const int* __restrict__ slots, int num_tokens,
+                                                              T* __restrict__ out) {
+  typedef T four __attribute__((ext_vector_type(4)));
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  const int t0 = blockIdx.x * SHIFT_RUN, tokens = min(SHIFT_RUN, num_tokens - t0);
+  for (int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4; c < width; c += gridDim.y * blockDim.x * 4) {
+    four row[SHIFT_RUN + 1];       // the token before the first, then the run's
+#pragma unroll
+    for (int i = 0; i <= SHIFT_RUN; ++i)
+      row[i] = *(const four*)(h + (long long)min(max(t0 + i - 1, 0), num_tokens - 1) * width + c);
+    f32x4 cur[SHIFT_RUN], diff[SHIFT_RUN];
+#pragma unroll
+    for (int i = 0; i < SHIFT_RUN; ++i) {
+      const int t = min(t0 + i, num_tokens - 1), e = entry_of[t];
+      f32x4 prev;
+      if (t == entry_start[e]) {
+        prev = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (entry_first[e] != 0) prev = *(const f32x4*)(state + (long long)slots[e] * state_stride + prev_offset + c);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) prev[k] = to_float<T>(row[i][k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        cur[i][k] = to_float<T>(row[i + 1][k]);
+        diff[i][k] = prev[k] - cur[i][k];
+      }
+    }
+    for (int s = 0; s < mixes; ++s) {
+      const f32x4 m = *(const f32x4*)(mu + (long long)s * width + c);
+#pragma unroll
+      for (int i = 0; i < SHIFT_RUN; ++i) {
+        if (i >= tokens) break;
+        four mixed;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mixed[k] = from_float<T>(fmaf(diff[i][k], m[k], cur[i][k]));
+        *(four*)(out + ((long long)s * num_tokens + t0 + i) * width + c) = mixed;
+      }
+    }
+  }
+}
+
 // An entry's last h becomes the state's saved row; one workgroup per entry, after token_shift has read the old one.
 template <typename T>
 __global__ __launch_bounds__(256) void save_last_kernel(const T* __restrict__ h, int width, float* __restrict__ state,
@@ -729,27 +782,49 @@ __global__ __launch_bounds__(256) void save_last_kernel(const T* __restrict__ h,
 // ---------------------------------------------------------------------------------------------
 // Read-out of a recurrent head: o / rms(o) (per head, over its `vdim` channels) * weight * gate.
 // weight: [vdim] shared by the heads, or [heads * vdim]; gate: a column range of a [T, ldg] buffer of type TG,
-// as it is (`gate_silu` 0), through silu (1) or through the sigmoid (2).  One wave per (token, head).
-template <typename TG, typename TO>
+// as it is (`gate_silu` 0), through silu (1) or through the sigmoid (2).  One wave per (token, head).  N: 64 N >= vdim, a lane
+// asks for everything at once; 0: any width, read twice.  2,048 tokens of 16 heads of 128, 32-bit gates: 15.8 -> 12.3 us.
+template <typename TG, typename TO, int N>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ weight,
                                                              int weight_per_head, const TG* __restrict__ gate,
                                                              long long ldg, int gate_silu, float eps, int heads,
                                                              int vdim, int num_tokens, TO* __restrict__ out) {
   const int lane = threadIdx.x & (WAVE - 1);
-  const long long unit = (long long)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  if (unit >= (long long)num_tokens * heads) return;
-  const int t = (int)(unit / heads), h = (int)(unit % heads);
+  const long long unit = (long long)blockIdx.x * (blockDim.x / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const long long units = (long long)num_tokens * heads;
+  if (unit >= units) return;
+  const int t = units <= 0xffffffffll ? (int)((unsigned)unit / (unsigned)heads) : (int)(unit / heads), h = (int)(unit - (long long)t * heads);
   const float* src = o + unit * vdim;
-  float ss = 0.f;
-  for (int c = lane; c < vdim; c += WAVE) ss += src[c] * src[c];
-  ss = wave_sum(ss);
-  const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
-  for (int c = lane; c < vdim; c += WAVE) {
-    float g = to_float<TG>(gate[(long long)t * ldg + h * vdim + c]);
+  const TG* gates = gate + (long long)t * ldg + h * vdim;
+  const float* weights = weight + (weight_per_head ? h * vdim : 0);
+  auto result = [&](float x, float inv, float w, float g) {
     if (gate_silu == 1) g = silu_f(g);
     else if (gate_silu == 2) g = sigmoid_f(g);
-    const float w = weight[(weight_per_head ? h * vdim : 0) + c];
-    out[unit * vdim + c] = from_float<TO>(src[c] * inv * w * g);
+    return from_float<TO>(x * inv * w * g);
+  };
+  float ss = 0.f;
+  if constexpr (N > 0) {
+    float x[N], g[N], w[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = min(lane + i * WAVE, vdim - 1);
+      x[i] = src[c];
+      g[i] = to_float<TG>(gates[c]);
+      w[i] = weights[c];
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (lane + i * WAVE < vdim) ss = fmaf(x[i], x[i], ss);
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (lane + i * WAVE < vdim) out[unit * vdim + lane + i * WAVE] = result(x[i], inv, w[i], g[i]);
+  } else {
+    for (int c = lane; c < vdim; c += WAVE) ss += src[c] * src[c];
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
+    for (int c = lane; c < vdim; c += WAVE) out[unit * vdim + c] = result(src[c], inv, weights[c], to_float<TG>(gates[c]));
   }
 }
 
@@ -1259,17 +1334,29 @@ extern "C" int vk_token_shift(const void* h, int dtype, int width, const float* 
   // a step of few tokens spreads a row over several workgroups; a prompt's many tokens fill the GPU by themselves
   const unsigned spans = num_tokens >= 512 ? 1u : (unsigned)min(64, (width + 255) / 256);
   const dim3 tokens_grid(num_tokens, spans), entries_grid(num_entries, spans);
+  const int bytes = dtype == DT_F32 ? 4 : 2;
+  const bool runs = num_tokens >= 512 && width % 4 == 0 && state_stride % 4 == 0 && prev_offset % 4 == 0 &&
+                    (((uintptr_t)mu | (uintptr_t)state) & 15) == 0 && (((uintptr_t)h | (uintptr_t)out) % (4 * bytes)) == 0;
+  const dim3 runs_grid((num_tokens + SHIFT_RUN - 1) / SHIFT_RUN, (unsigned)min(64, (width + 1023) / 1024));
   if (dtype == DT_F32) {
-    token_shift_kernel<float><<<tokens_grid, 256, 0, s>>>((const float*)h, width, mu, mixes, state, state_stride,
-                                                         prev_offset, entry_of, entry_start, entry_first, slots,
-                                                         num_tokens, (float*)out);
+    if (runs)
+      token_shift_run_kernel<float><<<runs_grid, 256, 0, s>>>((const float*)h, width, mu, mixes, state, state_stride, prev_offset,
+                                                              entry_of, entry_start, entry_first, slots, num_tokens, (float*)out);
+    else
+      token_shift_kernel<float><<<tokens_grid, 256, 0, s>>>((const float*)h, width, mu, mixes, state, state_stride,
+                                                           prev_offset, entry_of, entry_start, entry_first, slots,
+                                                           num_tokens, (float*)out);
     VK_LAUNCH_CHECK();
     save_last_kernel<float><<<entries_grid, 256, 0, s>>>((const float*)h, width, state, state_stride, prev_offset,
                                                         entry_start, slots);
   } else if (dtype == DT_BF16) {
-    token_shift_kernel<bf16_t><<<tokens_grid, 256, 0, s>>>((const bf16_t*)h, width, mu, mixes, state, state_stride,
-                                                          prev_offset, entry_of, entry_start, entry_first, slots,
-                                                          num_tokens, (bf16_t*)out);
+    if (runs)
+      token_shift_run_kernel<bf16_t><<<runs_grid, 256, 0, s>>>((const bf16_t*)h, width, mu, mixes, state, state_stride, prev_offset,
+                                                               entry_of, entry_start, entry_first, slots, num_tokens, (bf16_t*)out);
+    else
+      token_shift_kernel<bf16_t><<<tokens_grid, 256, 0, s>>>((const bf16_t*)h, width, mu, mixes, state, state_stride,
+                                                            prev_offset, entry_of, entry_start, entry_first, slots,
+                                                            num_tokens, (bf16_t*)out);
     VK_LAUNCH_CHECK();
     save_last_kernel<bf16_t><<<entries_grid, 256, 0, s>>>((const bf16_t*)h, width, state, state_stride, prev_offset,
                                                          entry_start, slots);
@@ -1288,15 +1375,22 @@ extern "C" int vk_head_norm_gate(const float* o, const float* weight, int weight
   const long long units = (long long)num_tokens * heads;
   const unsigned blocks = (unsigned)((units + 3) / 4);
   hipStream_t s = (hipStream_t)stream;
-#define VK_HNG(TG, TO)                                                                                         \
-  head_norm_gate_kernel<TG, TO><<<blocks, 256, 0, s>>>(o, weight, weight_per_head, (const TG*)gate, ldg,      \
-                                                       gate_silu, eps, heads, vdim, num_tokens, (TO*)out)
+#define VK_HNG_N(TG, TO, N)                                                                                    \
+  head_norm_gate_kernel<TG, TO, N><<<blocks, 256, 0, s>>>(o, weight, weight_per_head, (const TG*)gate, ldg,   \
+                                                          gate_silu, eps, heads, vdim, num_tokens, (TO*)out)
+#define VK_HNG(TG, TO)                     \
+  do {                                     \
+    if (vdim <= 64) VK_HNG_N(TG, TO, 1);   \
+    else if (vdim <= 128) VK_HNG_N(TG, TO, 2); \
+    else VK_HNG_N(TG, TO, 0);              \
+  } while (0)
   if (gate_dtype == DT_F32 && out_dtype == DT_F32) VK_HNG(float, float);
   else if (gate_dtype == DT_F32 && out_dtype == DT_BF16) VK_HNG(float, bf16_t);
   else if (gate_dtype == DT_BF16 && out_dtype == DT_BF16) VK_HNG(bf16_t, bf16_t);
   else if (gate_dtype == DT_BF16 && out_dtype == DT_F32) VK_HNG(bf16_t, float);
   else return VK_BAD_ARGUMENT;
 #undef VK_HNG
+#undef VK_HNG_N
   VK_LAUNCH_CHECK();
   return 0;
 }

@@ -817,25 +817,52 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
 }
 
 // dt[t, c] <- softplus(dt[t, c] + dt_bias[c]) in place and gate[t, c] = silu(z[t, c]): what the scan of a prompt's
-// portion would otherwise compute token behind token.
-__global__ void scan_prepare_kernel(float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
-                                    const float* __restrict__ z, long long ldz, float* __restrict__ gate, int C,
-                                    long long total) {
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const long long t = idx / C;
-  const int c = (int)(idx % C);
-  dt[t * lddt + c] = scan_softplus(dt[t * lddt + c] + dt_bias[c]);
-  gate[idx] = scan_silu(z[t * ldz + c]);
+// portion would otherwise compute token behind token.  Grid (tokens, parts of 1,024 channels), four channels a thread: neighbours
+// (VEC: rows in 16 bytes) or 256 apart.  Bound by memory; a thread a number, which divided its index by C in 64 bits, took 36.4 us
+// for 1,834 tokens of 4,096 channels, this 28.4 (one number at a time 31).
+template <bool VEC>
+__global__ __launch_bounds__(256) void scan_prepare_kernel(float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
+                                                           const float* __restrict__ z, long long ldz, float* __restrict__ gate,
+                                                           int C) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  const long long t = blockIdx.x;
+  float* step = dt + t * lddt;
+  const float* from = z + t * ldz;
+  float* to = gate + t * C;
+  for (long long first = blockIdx.y * 1024LL; first < C; first += gridDim.y * 1024LL) {
+    if constexpr (VEC) {
+      const long long c = first + threadIdx.x * 4;
+      if (c >= C) return;
+      f32x4 d = *(const f32x4*)(step + c), g = *(const f32x4*)(from + c);
+      const f32x4 bias = *(const f32x4*)(dt_bias + c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] = scan_softplus(d[i] + bias[i]);
+        g[i] = scan_silu(g[i]);
+      }
+      *(f32x4*)(step + c) = d;
+      *(f32x4*)(to + c) = g;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long long c = first + i * 256 + threadIdx.x;
+        if (c >= C) return;
+        step[c] = scan_softplus(step[c] + dt_bias[c]);
+        to[c] = scan_silu(from[c]);
+      }
+    }
+  }
 }
 
 extern "C" int vk_scan_prepare(float* dt, long long lddt, const float* dt_bias, const float* z, long long ldz,
                                float* gate, int num_tokens, int C, void* stream) {
   if (num_tokens <= 0) return 0;
   if (C < 1) return VK_BAD_ARGUMENT;
-  const long long total = (long long)num_tokens * C;
-  scan_prepare_kernel<<<(unsigned)((total + 255) / 256), 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate,
-                                                                                       C, total);
+  const dim3 grid(num_tokens, (unsigned)min((C + 1023LL) / 1024, 65535LL));
+  const bool vec = C % 4 == 0 && lddt % 4 == 0 && ldz % 4 == 0 &&
+                   (((uintptr_t)dt | (uintptr_t)dt_bias | (uintptr_t)z | (uintptr_t)gate) & 15) == 0;
+  if (vec) scan_prepare_kernel<true><<<grid, 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C);
+  else scan_prepare_kernel<false><<<grid, 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C);
   VK_LAUNCH_CHECK();
   return 0;
 }
