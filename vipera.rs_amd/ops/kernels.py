@@ -989,7 +989,8 @@ def gemm_bf16_gated_act(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kin
 def gemm_bf16_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_per_wave: int = 1) -> None:
     """``out = up * silu(gate)`` where ``[gate, up] = a @ w.T`` and ``w`` interleaves gate and up rows in
     groups of 16.  ``out``: ``[tokens, w.shape[0] / 2]`` bfloat16.  ``rows_per_wave`` (up to 64 tokens): 1 or
-    2 tiles per wave of the LDS-shared kernel, 0 for the kernel with resident activations (up to 16
+    2 tiles per wave of the LDS-shared kernel (past 16 tokens only where K is no multiple of 64 or one of 2,048: tiles of
+    64 tokens are faster elsewhere, with the same bits), 0 for the kernel with resident activations (up to 16
     tokens, K a multiple of 128, ``tokens x K`` within LDS; refused otherwise), 3 for the tiled kernel that
     more than 64 tokens always take."""
     _dev(a, w, out)

@@ -157,7 +157,8 @@ def gated_rows_per_wave(m: int, n: int) -> int:
     A workgroup reads its weight rows and all of the activations; a CU's time goes with the bytes it pulls,
     so what counts is how many workgroups the busiest CU gets (whole rounds over 256 CUs while they are few;
     with three rounds or more the dispatcher evens them out) times the rows and padded tokens of each.
-    Measured at the 1.5B, 7B and 32B widths with 8 to 64 tokens; ties go to one tile."""
+    Measured at the 1.5B, 7B and 32B widths with 8 to 64 tokens; ties go to one tile.  Past 16 tokens the choice only counts where
+    the tiled kernel does not take the product in its place (:func:`kernels.gemm_bf16_gated`)."""
     padded = (m + 15) // 16 * 16
     def cost(rows: int) -> float:
         groups = (n + rows - 1) // rows
@@ -182,9 +183,9 @@ def gated_plan(m: int, n: int, k: int, cus: int = 256) -> int:
         # to 171 us against 185; at 64 the norm's own kernel, which only the tiled one saves, makes them even)
         return gated_rows_per_wave(m, n)
     if n * k >= 1e8 or m * n * k >= 1.5e9:
-        # a large weight, or many tokens on a small one: the tiled kernel (3) with its three LDS stages and tiles
-        # of 96 to 224 weight rows that fill the CUs in one round passes the LDS-shared one (7B widths at 17 to 64
-        # tokens: 51 to 54 us against 57 to 71; 32B: 102 to 106 against 110 to 120; 1.5B from 64 tokens)
+        # a large weight, or many tokens on a small one: the tiled kernel (3) with tiles of 64 tokens and of 64 to 224
+        # weight rows that fill the CUs in one round passes the LDS-shared one (7B widths at 17 to 64 tokens: 49 to
+        # 50 us against 57 to 71, and 51 to 54 in tiles of 128 tokens), and divides by the norm before it
         return 3
     return gated_rows_per_wave(m, n)
 
