@@ -1443,3 +1443,23 @@ def test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, wid
                                 piece, 1)
             parts[:, at:end] = piece
     assert torch.equal(whole, parts) and torch.equal(left, one)
+
+
+@pytest.mark.parametrize("tokens,heads,k,n", [(1, 2, 64, 64), (64, 3, 128, 192), (65, 2, 192, 100), (200, 1, 320, 33)])
+def test_products_per_head_in_tiles_of_64_give_the_bits_of_the_wide_ones(tokens, heads, k, n):
+    """K in whole steps of 64 against the same numbers with eight zeros more, which take the tiles of 128 x 128: tokens and outputs that
+    end inside a tile, one step and several, gated, outputs on 8 bytes and not."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator(DEV).manual_seed(tokens + k)
+    a, w = torch.randn(tokens, heads, k, generator=g, device=DEV).bfloat16(), torch.randn(heads, n, k, generator=g, device=DEV).bfloat16()
+    gate = torch.randn(tokens, heads, generator=g, device=DEV)
+    pad = lambda x: torch.nn.functional.pad(x, (0, 8)).contiguous()
+    for opened in (None, gate):
+        for spare in (0, 5):
+            out = [torch.full((tokens, heads * (n + spare)), 7.0, device=DEV).bfloat16() for _ in range(2)]
+            kernels.head_linear(a.reshape(tokens, -1), k, k, w, out[0], n + spare, gate=opened)
+            kernels.head_linear(pad(a).reshape(tokens, -1), k + 8, k + 8, pad(w), out[1], n + spare, gate=opened)
+            assert torch.equal(out[0], out[1])
+    want = torch.einsum("thk,hnk->thn", a.double().cpu(), w.double().cpu()) * torch.sigmoid(gate.double().cpu())[..., None]
+    got = out[0].reshape(tokens, heads, n + 5)[..., :n].double().cpu()
+    assert float((got - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())      # outputs are rounded to bfloat16

@@ -168,11 +168,14 @@ __global__ __launch_bounds__(256) void head_linear_kernel(const TA* __restrict__
 }
 
 // The same product on the matrix cores (bfloat16 in and out; K a multiple of 8, 16-byte rows): tiles of 128 tokens
-// x 128 outputs of one head, see group_tile.h.  Grid (ceil(T / 128), ceil(N / 128), heads).
+// x 128 outputs of one head, see group_tile.h.  Grid (ceil(T / 128), ceil(N / 128), heads).  quads: a lane's four consecutive
+// outputs leave as 8 bytes (2 bytes at a time, sixteen rows an instruction, 2,048
+// tokens of 16 heads, K 128, N 192 took 22.7 us, so 10.9).
 __global__ __launch_bounds__(256) void head_linear_mma_kernel(const __bf16* __restrict__ a, long long lda, long long sa,
                                                               const __bf16* __restrict__ w, __bf16* __restrict__ out,
                                                               long long ldo, long long so, int M, int N, int K,
-                                                              const float* __restrict__ gate, long long ldg) {
+                                                              const float* __restrict__ gate, long long ldg, bool quads) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int h = blockIdx.z, m0 = blockIdx.x * GT_TILE, n0 = blockIdx.y * GT_TILE;
   const __bf16* ah = a + (long long)h * sa;
@@ -189,12 +192,63 @@ __global__ __launch_bounds__(256) void head_linear_mma_kernel(const __bf16* __re
     __bf16* dst = out + (long long)m * ldo + (long long)h * so;
     const float open = head_gate(gate, ldg, m, h);
 #pragma unroll
-    for (int tn = 0; tn < 4; ++tn)
+    for (int tn = 0; tn < 4; ++tn) {
+      const int n = n0 + wn * 64 + tn * 16 + lg * 4;
+      bf16x4 v;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = n0 + wn * 64 + tn * 16 + lg * 4 + i;
-        if (n < N) dst[n] = (__bf16)(acc[tn][tm][i] * open);
+      for (int i = 0; i < 4; ++i) v[i] = (__bf16)(acc[tn][tm][i] * open);
+      if (quads) {
+        if (n < N) *(bf16x4*)(dst + n) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) dst[n + i] = v[i];
       }
+    }
+  }
+}
+
+// The same where K is a multiple of 64: operands straight into LDS, two steps asked for at once (K of 128 or 192, a head's width or
+// a compressed row, is two or three, which the tiles above take as round trips to memory one behind the other), in tiles of
+// 64 x 64 outputs, so that few tokens are many workgroups. Every output is the same sum. us before, with those tiles and so: 16 heads,
+// K 128, N 192, 64 tokens 8.2 / 5.6 / 3.4, 2,048 22.7 / 10.9 / 8.9; K 192, N 128, 64 tokens 10.0 / 7.4 / 4.0, 512 13.1 / 7.4 / 4.0. A third
+// stage, 128 x 64 and 128 x 128 outputs: the same to 1.4 times as long.
+constexpr int HEAD_TILE = 64;
+__global__ __launch_bounds__(256) void head_linear_direct_kernel(const __bf16* __restrict__ a, long long lda, long long sa,
+                                                                 const __bf16* __restrict__ w, __bf16* __restrict__ out,
+                                                                 long long ldo, long long so, int M, int N, int K,
+                                                                 const float* __restrict__ gate, long long ldg, bool quads) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int BM = HEAD_TILE, BN = HEAD_TILE, WM = 2, WN = 2, STAGES = 2, TM = BM / WM / 16, TN = BN / WN / 16;
+  const int h = blockIdx.z, m0 = blockIdx.x * BM, n0 = blockIdx.y * BN, rows = min(BM, M - m0);
+  const GtView w_view = gt_view(w + ((long long)h * N + n0) * K, GT_VIEW_BYTES);
+  gt_f32x4 acc[TN][TM];
+  group_tile_direct<BM, BN, WM, WN, STAGES>(
+      gt_view(a + (long long)h * sa + (long long)m0 * lda, GT_VIEW_BYTES),
+      [&](int r) { return r < rows ? (unsigned)r * (unsigned)(lda * 2) : GT_NO_ROW; }, w_view, w_view,
+      [&](int r) { return n0 + r < N ? (unsigned)r * (unsigned)(K * 2) : GT_NO_ROW; }, [](int) { return false; }, K, rows, lds, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm) {
+    const int m = m0 + wm * (BM / WM) + tm * 16 + lr;
+    if (m >= M) continue;
+    __bf16* dst = out + (long long)m * ldo + (long long)h * so;
+    const float open = head_gate(gate, ldg, m, h);
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      const int n = n0 + wn * (BN / WN) + tn * 16 + lg * 4;
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (__bf16)(acc[tn][tm][i] * open);
+      if (quads) {
+        if (n < N) *(bf16x4*)(dst + n) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) dst[n + i] = v[i];
+      }
+    }
   }
 }
 
@@ -247,12 +301,16 @@ extern "C" int vk_latent_q_rotate(const void* q, long long ldq, int q_head, int 
   return 0;
 }
 
+// Rows of up to that many numbers: a tile's bytes lie within a view.
+constexpr long long HEAD_DIRECT_ROW = 4000000;
+static_assert(HEAD_TILE * HEAD_DIRECT_ROW * 2 < GT_VIEW_BYTES, "a tile's rows lie within a view");
+
 extern "C" int vk_head_linear(const void* a, int a_dtype, long long lda, long long sa, const void* w, int w_dtype,
                               void* out, int out_dtype, long long ldo, long long so, int M, int N, int K, int heads,
                               const float* gate, long long ldg, void* stream) {
   if (M <= 0 || N <= 0 || heads <= 0) return 0;
   if (K < 1 || heads > 65535) return VK_BAD_ARGUMENT;
-  dim3 grid((M + 63) / 64, (N + 63) / 64, heads);
+  dim3 grid((M + 63) / 64, (N + 63) / 64, heads);   // of head_linear_direct_kernel as well
   if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
   hipStream_t s = (hipStream_t)stream;
   if (a_dtype == DT_F32 && w_dtype == DT_F32 && out_dtype == DT_F32)
@@ -260,6 +318,13 @@ extern "C" int vk_head_linear(const void* a, int a_dtype, long long lda, long lo
                                                                  ldo, so, M, N, K, gate, ldg);
   else if (a_dtype == DT_BF16 && w_dtype == DT_BF16 && out_dtype == DT_BF16 && K % 8 == 0 && lda % 8 == 0 && sa % 8 == 0 &&
            (((uintptr_t)a | (uintptr_t)w) & 15) == 0) {
+    const bool quads = N % 4 == 0 && ldo % 4 == 0 && so % 4 == 0 && ((uintptr_t)out & 7) == 0;
+    if (K % 64 == 0 && lda >= 0 && lda <= HEAD_DIRECT_ROW && K <= HEAD_DIRECT_ROW) {
+      head_linear_direct_kernel<<<grid, 256, gt_direct_lds<HEAD_TILE, HEAD_TILE, 2>(), s>>>(
+          (const __bf16*)a, lda, sa, (const __bf16*)w, (__bf16*)out, ldo, so, M, N, K, gate, ldg, quads);
+      VK_LAUNCH_CHECK();
+      return 0;
+    }
     static bool sized = false;
     if (!sized) {
       hipError_t e = hipFuncSetAttribute((const void*)head_linear_mma_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -269,7 +334,7 @@ extern "C" int vk_head_linear(const void* a, int a_dtype, long long lda, long lo
     }
     dim3 wide((M + GT_TILE - 1) / GT_TILE, (N + GT_TILE - 1) / GT_TILE, heads);
     head_linear_mma_kernel<<<wide, 256, GT_LDS_BYTES, s>>>((const __bf16*)a, lda, sa, (const __bf16*)w, (__bf16*)out, ldo,
-                                                           so, M, N, K, gate, ldg);
+                                                           so, M, N, K, gate, ldg, quads);
   } else if (a_dtype == DT_BF16 && w_dtype == DT_BF16 && out_dtype == DT_BF16)
     head_linear_kernel<bf16_t, bf16_t, bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)a, lda, sa, (const bf16_t*)w,
                                                                     (bf16_t*)out, ldo, so, M, N, K, gate, ldg);
