@@ -1463,3 +1463,27 @@ def test_products_per_head_in_tiles_of_64_give_the_bits_of_the_wide_ones(tokens,
     want = torch.einsum("thk,hnk->thn", a.double().cpu(), w.double().cpu()) * torch.sigmoid(gate.double().cpu())[..., None]
     got = out[0].reshape(tokens, heads, n + 5)[..., :n].double().cpu()
     assert float((got - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())      # outputs are rounded to bfloat16
+
+
+@pytest.mark.parametrize("tokens", [5, 70])
+@pytest.mark.parametrize("experts,top", [(1, 1), (5, 4), (33, 4), (64, 6), (130, 4)])
+def test_routes_by_lane_moves_are_the_largest_logits_lowest_id_first(tokens, experts, top):
+    """A token's choices over one and several experts a lane, whole numbers so that many are equal, and the grouping by expert: the
+    counts, the places and the tiles as a sort in plain code gives them."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(experts + tokens)
+    logits = torch.randint(-3, 4, (tokens, experts), generator=g).float()
+    logits[torch.rand(tokens, experts, generator=g) < 0.1] = float("-inf")
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    pairs = tokens * top
+    ids, offsets, order, tiles, count = i32(pairs), i32(experts + 1), i32(pairs), i32(2 * kernels.moe_max_tiles(pairs, experts, 64)), i32(1)
+    weights = torch.empty(pairs, device=DEV)
+    kernels.moe_route(logits.to(DEV), top, ids, weights, offsets, order, tiles, count)
+    want = [sorted(range(experts), key=lambda e: (-logits[t, e].item(), e))[:top] for t in range(tokens)]
+    assert ids.cpu().view(tokens, top).tolist() == want
+    flat = [e for row in want for e in row]
+    starts = [sum(x < e for x in flat) for e in range(experts + 1)]
+    assert offsets.tolist() == starts
+    placed = order.tolist()
+    assert sorted(placed) == list(range(pairs)) and all(flat[p] == e for e in range(experts) for p in placed[starts[e]:starts[e + 1]])
+    assert tiles.tolist()[:2 * count.item()] == [x for e in range(experts) for first in range(starts[e], starts[e + 1], 64) for x in (e, first)]

@@ -29,6 +29,47 @@ struct Routing {
   long long ld = 0;     // floats between two tokens' logits; 0: the number of experts (rows one behind the other)
 };
 
+// The value of lane ^ OFF, by the vector unit alone (a round trip through LDS stood behind each of a choice's six exchanges of
+// two numbers: route and grouping of 8 tokens, four of 32 experts, 6.9 us, so
+// and with the experts' running sums by lane moves 5.9; of 2,048 13.0 and 11.8).
+template <int OFF>
+__device__ __forceinline__ int lane_xor(int v, int lane) {
+  if constexpr (OFF == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);   // {the lower half's, the upper half's}
+    return lane & 32 ? s[0] : s[1];
+  } else if constexpr (OFF == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);   // {the even rows', the odd rows'}
+    return lane & 16 ? s[0] : s[1];
+  } else if constexpr (OFF == 8) {
+    return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true);             // a row turned by 8
+  } else if constexpr (OFF == 4) {
+    return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);   // ^ 7, ^ 3
+  } else if constexpr (OFF == 2) {
+    return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true);
+  } else {
+    return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);
+  }
+}
+// The better of two lanes' candidates OFF apart, then of all 64: the larger one, the lower id among equals; arg NO_CHOICE: none.
+constexpr int NO_CHOICE = 0x7fffffff;
+template <int OFF>
+__device__ __forceinline__ void better_of(float& best, int& arg, int lane) {
+  const float ob = __int_as_float(lane_xor<OFF>(__float_as_int(best), lane));
+  const int oa = lane_xor<OFF>(arg, lane);
+  if (oa != NO_CHOICE && (arg == NO_CHOICE || ob > best || (ob == best && oa < arg))) {
+    best = ob;
+    arg = oa;
+  }
+}
+__device__ __forceinline__ void best_of_wave(float& best, int& arg, int lane) {
+  better_of<32>(best, arg, lane);
+  better_of<16>(best, arg, lane);
+  better_of<8>(best, arg, lane);
+  better_of<4>(best, arg, lane);
+  better_of<2>(best, arg, lane);
+  better_of<1>(best, arg, lane);
+}
+
 __device__ __forceinline__ float choice_score(const Routing& how, const float* z, int e) {
   return how.all_scores == 3 ? 1.0f / (1.0f + expf(-z[e])) + (how.correction ? how.correction[e] : 0.f) : z[e];
 }
@@ -36,7 +77,6 @@ __device__ __forceinline__ float choice_score(const Routing& how, const float* z
 __device__ __forceinline__ void route_token(const float* __restrict__ logits, int experts, int top, int t, int lane,
                                             int* __restrict__ ids, float* __restrict__ weights,
                                             Routing how = Routing{1, 1, 0}) {
-  constexpr int NONE = 0x7fffffff;
   const float* z = logits + (long long)t * (how.ld ? how.ld : experts);
   unsigned long long taken = 0;
   if (how.groups > 1 && how.keep < how.groups) {
@@ -48,16 +88,9 @@ __device__ __forceinline__ void route_token(const float* __restrict__ logits, in
     unsigned long long kept = 0;
     for (int j = 0; j < how.keep; ++j) {
       float best = (lane < how.groups && !((kept >> lane) & 1ull)) ? score : -INFINITY;
-      int arg = (lane < how.groups && !((kept >> lane) & 1ull)) ? lane : NONE;
-      for (int off = WAVE / 2; off > 0; off >>= 1) {
-        const float ob = __shfl_xor(best, off, WAVE);
-        const int oa = __shfl_xor(arg, off, WAVE);
-        if (oa != NONE && (arg == NONE || ob > best || (ob == best && oa < arg))) {
-          best = ob;
-          arg = oa;
-        }
-      }
-      if (arg != NONE) kept |= 1ull << arg;
+      int arg = (lane < how.groups && !((kept >> lane) & 1ull)) ? lane : NO_CHOICE;
+      best_of_wave(best, arg, lane);
+      if (arg != NO_CHOICE) kept |= 1ull << arg;
     }
     for (int e = lane, i = 0; e < experts; e += WAVE, ++i)
       if (!((kept >> (e / size)) & 1ull)) taken |= 1ull << i;
@@ -71,25 +104,27 @@ __device__ __forceinline__ void route_token(const float* __restrict__ logits, in
     whole_sum = wave_sum(part);
   }
   float first = 0.f, sum = 0.f, mine = 0.f;      // lane j keeps the weight of choice j
+  const bool one_each = experts <= WAVE;         // a lane's only expert is scored once
+  const float own = one_each && lane < experts ? choice_score(how, z, lane) : 0.f;
   for (int j = 0; j < top; ++j) {
     float best = -INFINITY;
-    int arg = NONE;
-    for (int e = lane, i = 0; e < experts; e += WAVE, ++i) {
-      if ((taken >> i) & 1ull) continue;
-      const float v = choice_score(how, z, e);
-      if (arg == NONE || v > best) {   // ascending e: an equal later one does not replace
-        best = v;
-        arg = e;
+    int arg = NO_CHOICE;
+    if (one_each) {
+      if (lane < experts && !(taken & 1ull)) {
+        best = own;
+        arg = lane;
+      }
+    } else {
+      for (int e = lane, i = 0; e < experts; e += WAVE, ++i) {
+        if ((taken >> i) & 1ull) continue;
+        const float v = choice_score(how, z, e);
+        if (arg == NO_CHOICE || v > best) {      // ascending e: an equal later one does not replace
+          best = v;
+          arg = e;
+        }
       }
     }
-    for (int off = WAVE / 2; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, WAVE);
-      const int oa = __shfl_xor(arg, off, WAVE);
-      if (oa != NONE && (arg == NONE || ob > best || (ob == best && oa < arg))) {
-        best = ob;
-        arg = oa;
-      }
-    }
+    best_of_wave(best, arg, lane);
     if ((arg & (WAVE - 1)) == lane) taken |= 1ull << (arg / WAVE);
     if (j == 0) first = best;
     const float p = how.all_scores == 3 ? how.weight_scale / (1.0f + expf(-z[arg]))
@@ -106,6 +141,17 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
                                                         float* __restrict__ weights, Routing how) {
   const int t = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
   if (t < num_tokens) route_token(logits, experts, top, t, threadIdx.x & (WAVE - 1), ids, weights, how);
+}
+
+// The sum over a wave's lanes up to this one, by lane moves: within rows of sixteen, then a row's last lane to the next row and
+// that of the first half to the second.
+__device__ __forceinline__ int running_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
 }
 
 // One workgroup: counts per expert, offsets, the pairs' places, and the list of tiles.
@@ -136,13 +182,8 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
     for (int base = 0; base < experts; base += WAVE) {
       const int e = base + lane, count = e < experts ? counts[e] : 0, own = (count + tile_rows - 1) / tile_rows;
       int places = count, tiles_upto = own;
-      for (int off = 1; off < WAVE; off <<= 1) {
-        const int p = __shfl_up(places, off, WAVE), q = __shfl_up(tiles_upto, off, WAVE);
-        if (lane >= off) {
-          places += p;
-          tiles_upto += q;
-        }
-      }
+      places = running_sum(places);
+      tiles_upto = running_sum(tiles_upto);
       if (e < experts) {
         const int first = at + places - count;
         offsets[e] = first;
