@@ -2018,6 +2018,8 @@ TilePlan tile_plan(int M, int N, int K, long long partial_floats, bool gated, bo
 // 0.98 of the planned one's. us, planned to picked: 1,396 tokens on 2,048 rows of 1,536 21.4 -> 14.8, on 1,536
 // rows 19.7 -> 16.2, 1,383 on 2,048 of 2,048 24.4 -> 18.2, 1,000 on 4,608 of 3,584 49.0 -> 37.8, 1,014 on 3,584 of 3,584
 // 48.3 -> 38.8; gated: 1,396 on 17,920 of 1,536 89.8 -> 80.7, 622 on 5,120 of 2,048 25.0 -> 20.1, 311 on 22,016 46.1 -> 36.2.
+// The fit is with two stages of the weight's rows in 256x256, 256x192 and 128x128; the third one has since taken up to 7 % off their
+// steps in a full round and little off short ones, and the fit stands.
 // Every output is one sum over K in ascending steps of 32 whatever the tile, so the bits are the same.
 struct TileCost { int config, tokens, rows, resident; double beside, low, high, pair, alone, output; };
 constexpr TileCost WHOLE_TILES[] = {
