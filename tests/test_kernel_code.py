@@ -39,3 +39,34 @@ def test_whole_steps_of_an_odd_k_are_read_in_wide_loads(gemm_generic_code):
     for name, (both_32_bit, _, wide, body) in gemm_generic_code.items():
         if both_32_bit and not wide:
             assert body.count("global_load_dwordx4") >= 2, name
+
+
+@pytest.fixture(scope="module")
+def gemm_bf16_code(tmp_path_factory):
+    """The instructions of each kernel of the built library, by its name."""
+    tools = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(build._hipcc()))), "llvm", "bin")
+    if not os.path.exists(os.path.join(tools, "clang-offload-bundler")):
+        pytest.skip("needs ROCm's binary tools")
+    folder = tmp_path_factory.mktemp("library")
+    bundle, code = str(folder / "bundle"), str(folder / "code")
+    library = build.library_path("gemm_bf16") or build.compile_module("gemm_bf16")
+    for command in (["llvm-objcopy", f"--dump-section=.hip_fatbin={bundle}", library, os.devnull],
+                    ["clang-offload-bundler", "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={bundle}", f"--output={code}"]):
+        subprocess.run([os.path.join(tools, command[0]), *command[1:]], check=True, capture_output=True)
+    text = subprocess.run([os.path.join(tools, "llvm-objdump"), "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True).stdout
+    return dict(re.findall(r"^[0-9a-f]+ <(_ZN\S+)>:\n(.*?)(?=^\s*$|\Z)", text, re.S | re.M))
+
+
+def test_a_tile_with_as_many_stages_of_both_operands_works_out_one_place_a_step(gemm_bf16_code):
+    """Where the next step's rows lie is one choice of two (``s_cselect``) for what is read and one for what is asked for; with a
+    choice for each operand the 64x64 tiles that add K's ranges themselves took 8 to 10 % longer (512 x 2,048 x 2,048)."""
+    loops = 0
+    for name, body in gemm_bf16_code.items():
+        found = re.search(r"gemm_tile_direct_kernelI(?:Li\d+E){4}(?:f|DF16b)Lb\dELb\dELi(\d)ELb\dELi(\d)E", name)
+        if not found or found[1] != found[2]:
+            continue
+        for block in re.split(r"^\ts_c?branch\S*[^\n]*\n", body, flags=re.M):
+            if "v_mfma" in block and re.search(r"buffer_load_dwordx4 .* lds", block):
+                loops += 1
+                assert block.count("s_cselect") <= 2, name
+    assert loops >= 20
