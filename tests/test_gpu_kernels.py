@@ -532,6 +532,14 @@ def test_each_form_of_the_32_bit_product_sums_in_the_same_order(m, n, k, form):
         assert torch.equal(few, whole[rows]) and torch.equal(more, added[rows]), start
 
 
+@pytest.mark.parametrize("m,n,k,form", [(500, 130, 132, 1), (9, 33, 4, 1), (65, 4099, 132, 1), (17, 4099, 20, 2), (129, 2050, 4, 3), (257, 2050, 644, 9),
+                                        (501, 2050, 644, 8), (65, 9731, 36, 6), (333, 9731, 100, 7), (33, 9731, 64, 5), (2003, 9731, 16, 0),
+                                        (1001, 2050, 96, 0)])
+def test_a_32_bit_product_of_short_rows_takes_the_form_that_is_fast_there(m, n, k, form):
+    """Rows of less than 704 numbers, down to one step, beside each line of the choice (0: the 64 x 64 tiles)."""
+    test_each_form_of_the_32_bit_product_sums_in_the_same_order(m, n, k, form)
+
+
 @pytest.mark.parametrize("m,n,k,form", [(333, 9725, 900, 8), (39, 3037, 2052, 8), (35, 779, 11012, 8), (515, 1150, 900, 9),
                                         (36, 4979, 2052, 9), (333, 895, 4868, 9), (162, 4283, 1020, 4), (553, 105, 11012, 4)])
 def test_wide_slabs_of_the_32_bit_product_sum_in_the_same_order(m, n, k, form):

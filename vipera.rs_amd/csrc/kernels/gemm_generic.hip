@@ -659,36 +659,60 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
 // Two or three stages leave room for a second or third workgroup on a CU, which hide a wave's own chain of loads better than a
 // deeper queue of its own does (a slab's 64 x 64 with four stages took 1.10 of the time with two).  Over 233 sizes from 12 to
 // 2,048 rows the choice takes 0.885 of the time of the kernels that exchanged lanes' values and had no tiles of 48 x 48
-// (geometric mean), 1.006 of it at worst, and 1.012 of the best form's.  The 64 x 64 tiles cut over workgroups are the fastest at
-// none of them; they keep any other type, and rows off 16 bytes.
+// (geometric mean), 1.006 of it at worst, and 1.012 of the best form's; all of K 700 and more.  The 64 x 64 tiles cut over workgroups
+// are the fastest at none of them; they keep any other type, and rows off 16 bytes.
+// Below K 704 a slab's ranges are short or missing, while a walk over all of K has its first loads and its last stores to wait for:
+//   slab   the first tile takes what a range of K takes (256 of k or less), each further one on the CU `range` of a step for a whole
+//          range alone and all of it from K 704 on (the ranges share the CU's loads); `less` of `beside` falls away
+//   rows   `first` more beside it, `each` more a tile, and K in whole steps of 32
+//   the 64 x 64 tiles (two stages through registers, no slab to end), which pass both where K is a step or two
+// us, as chosen without that and now: 500 x 130 x 132 7.1 / 4.6, 65 x 4,096 x 132 7.7 / 5.8, 257 x 1,152 x 64 5.0 / 4.1, 9 x 9,728 x
+// 260 9.7 / 6.6, 2,500 x 9,728 x 16 36.4 / 26.9.  Over 1,430 sizes of K 4 to 1,000 the choice takes 0.89 of the time of the kernels that
+// exchanged lanes' values (1.03 without it) and 1.026 of the best form's; at worst 1.12 of theirs, 1,396 x 9,728 x 24 as 64 x 128, and 2,500 x
+// 1,024 x 1,000 as 48 x 32: rows that do not begin on 128 bytes cost the smaller slabs a fifth, which the choice does not tell apart.
 enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128, SLAB_48_48, SLAB_48_64 };
 
 Direct direct_plan(int M, int N, int K, long long part_floats) {
-  struct Form { Direct form; int rows, columns, resident; double beside, step, together, over; };
-  constexpr Form slab_forms[] = {{SLAB_16_32, 16, 32, 4, 4.0, 3.3}, {SLAB_32_32, 32, 32, 5, 3.9, 4.9}, {SLAB_48_32, 48, 32, 4, 3.9, 6.8},
-                                 {SLAB_48_48, 48, 48, 3, 4.5, 9.7}, {SLAB_48_64, 48, 64, 2, 4.2, 12.8}, {SLAB_64_64, 64, 64, 2, 4.7, 16.3}};
-  constexpr Form row_forms[] = {{ROWS_64_64, 64, 64, 3, 4.1, 0.0164, 0.0045, 0.25}, {ROWS_32_128, 32, 128, 2, 4.8, 0.0159, 0.0038, 0.6},
-                                {ROWS_64_128, 64, 128, 2, 3.5, 0.0313, 0.0055, 0.5}};
+  struct Slab { Direct form; int rows, columns, resident; double beside, step, less, range; };
+  struct Rows { Direct form; int rows, columns, resident; double beside, step, together, over, first, each; };
+  constexpr Slab slab_forms[] = {{SLAB_16_32, 16, 32, 4, 4.0, 3.3, 1.1, 0.41}, {SLAB_32_32, 32, 32, 5, 3.9, 4.9, 0.8, 0.41},
+                                 {SLAB_48_32, 48, 32, 4, 3.9, 6.8, 0.5, 0.41}, {SLAB_48_48, 48, 48, 3, 4.5, 9.7, 0.8, 0.45},
+                                 {SLAB_48_64, 48, 64, 2, 4.2, 12.8, 0.4, 0.55}, {SLAB_64_64, 64, 64, 2, 4.7, 16.3, 0.4, 0.55}};
+  constexpr Rows row_forms[] = {{ROWS_64_64, 64, 64, 3, 4.1, 0.0164, 0.0045, 0.25, -0.7, 0.6},
+                                {ROWS_32_128, 32, 128, 2, 4.8, 0.0159, 0.0038, 0.6, -1.3, 0.9},
+                                {ROWS_64_128, 64, 128, 2, 3.5, 0.0313, 0.0055, 0.5, 2.0, 0.6}};
+  constexpr int SHORT_K = 704, STEP_OR_TWO = 96;
   const long long slabs = (K + SLAB_K - 1) / SLAB_K;
   const double parts = slabs == 1 ? 0.0 : 3.0 + 1.1 * slabs * M * N * 8 / 6e6;
   const double pitch = K % 2048 == 0 ? 1.04 : 1.0;     // weights whose rows are a multiple of 8 KB apart
+  const double shorter = K < SHORT_K ? 1.0 - (double)K / SHORT_K : 0.0;
+  const int k16 = (K + 15) / 16 * 16, k32 = K < SHORT_K ? (K + 31) / 32 * 32 : K;
   double best = 1e300;
   Direct chosen = NOT_DIRECT;
-  auto offer = [&](const Form& f, long long tiles, double us) {
-    if (tiles <= 0xffffffffll / 256 && us < best) best = us, chosen = f.form;
+  auto tiles_of = [&](int rows, int columns) { return (long long)((M + rows - 1) / rows) * ((N + columns - 1) / columns); };
+  auto offer = [&](Direct form, long long tiles, double us) {
+    if (tiles <= 0xffffffffll / 256 && us < best) best = us, chosen = form;
   };
-  auto tiles_of = [&](const Form& f) { return (long long)((M + f.rows - 1) / f.rows) * ((N + f.columns - 1) / f.columns); };
   if (slabs == 1 || slabs * M * N <= part_floats)
-    for (const Form& f : slab_forms) {
-      const long long tiles = tiles_of(f);
+    for (const Slab& f : slab_forms) {
+      const long long tiles = tiles_of(f.rows, f.columns);
       const double each = tiles * slabs / 256.0;       // past what is resident a CU short of its share waits for none; past 8 they even out
       const double most = each > 8 ? each + 0.5 : each > f.resident ? ceil(each + 0.05) : ceil(each);
-      offer(f, tiles, (f.beside + f.step * most) * pitch * (K > 8192 && f.form != SLAB_64_64 ? 1.2 : 1.0) + parts);
+      const double ranges = (double)k16 / RANGE_K;
+      const double first = fmin(ranges, 1.0) * (1.0 - 0.03 * shorter);
+      const double further = ranges <= 1 ? 0.09 + (f.range - 0.09) * ranges
+                                         : fmin(1.0, f.range + (1.0 - f.range) * (k16 - RANGE_K) / (SHORT_K - RANGE_K));
+      const double us = (f.beside - f.less * shorter + f.step * (first + (most - 1) * further)) * pitch;
+      offer(f.form, tiles, us * (K > 8192 && f.form != SLAB_64_64 ? 1.2 : 1.0) + parts);
     }
-  for (const Form& f : row_forms) {
-    const long long tiles = tiles_of(f);
+  for (const Rows& f : row_forms) {
+    const long long tiles = tiles_of(f.rows, f.columns);
     const double each = tiles / 256.0, most = ceil(each) > 2 * f.resident ? each + f.over : ceil(each);
-    offer(f, tiles, f.beside + (f.step * most + f.together * ceil(most / f.resident)) * K * pitch);
+    offer(f.form, tiles, f.beside + (f.step * most + f.together * ceil(most / f.resident)) * k32 * pitch + shorter * (f.first + f.each * most));
+  }
+  if (K <= STEP_OR_TWO) {
+    const double us = 3.3 + 0.0117 * k16 + (0.42 + 0.0203 * k16) * fmax(1.0, tiles_of(TILE, TILE) / 256.0 + 0.3);
+    if (us < best) chosen = NOT_DIRECT;
   }
   return chosen;
 }
