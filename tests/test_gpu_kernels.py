@@ -1428,6 +1428,13 @@ def test_passes_over_rows_in_fours_give_the_bits_of_one_number_at_a_time(rows, w
     assert torch.equal(step, ones) and torch.equal(gates, alone)
 
 
+@pytest.mark.parametrize("rows,width", [(6143, 64), (6144, 64), (2979, 132), (97, 4100)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_passes_over_many_rows_in_fours_give_the_bits_of_one_number_at_a_time(rows, width, dtype):
+    """On both sides of the number from which a thread takes four, 393,216 of them."""
+    test_passes_over_rows_in_fours_give_the_bits_of_one_number_at_a_time(rows, width, dtype)
+
+
 @pytest.mark.parametrize("tokens,width,dtype", [(514, 36, torch.bfloat16), (515, 1028, torch.float32), (640, 64, torch.bfloat16)])
 def test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, width, dtype):
     """A step of 512 tokens or more against the same tokens in smaller steps: entries that begin inside a run, behind a state and at

@@ -412,10 +412,14 @@ extern "C" int vk_rope_kvwrite(void* qkv, int dtype, const int* positions, const
 }
 
 // ---------------------------------------------------------------------------------------------
-// The kernels below take V consecutive numbers of a row a thread: four where every row and pointer allows accesses of four,
-// else one.  They are bound by memory, which a thread a number, dividing its index by the row's width in 64 bits (some hundred
-// instructions), left half idle.  us, before and so: silu(a) b, 1,834 rows of 4,096, 32-bit 22.8 / 14.7, of 2,048 into 16 bits 11.5 /
-// 6.8; swiglu of 333 rows of 4,864 in 32 bits 5.5 / 4.2; 1,834 tokens of 16 gated heads of 128 11.7 / 7.0; 8 rows of 2,048 2.3 / 2.4.
+// The kernels below take V consecutive numbers of a row a thread: four where every row and pointer allows accesses of four and there
+// are FOURS_FROM numbers, else one.  Many numbers are bound by memory, which a thread a number, dividing its index by the row's width in 64
+// bits (some hundred instructions), left half idle.  us, before and so: silu(a) b, 1,834 rows of 4,096, 32-bit 22.8 / 14.7, of 2,048 into 16
+// bits 11.5 / 6.8; swiglu of 333 rows of 4,864 in 32 bits 5.5 / 4.2; 1,834 tokens of 16 gated heads of 128 11.7 / 7.0.  Few numbers are bound by
+// a thread's own chain, four exponentials behind one another instead of one.  us, a number and four a thread: silu(a) b, 8 rows of
+// 4,096 2.34 / 2.62, 128 of 2,048 2.55 / 2.69, 333 of 1,024 2.71 / 2.85, 128 of 4,096 3.04 / 2.85, 333 of 2,048 3.39 / 3.09; gated heads, 8 rows of
+// 2,048 2.35 / 2.56, 333 of 1,024 3.00 / 2.90, 333 of 2,048 3.84 / 3.17.
+constexpr long long FOURS_FROM = 3 << 17;
 template <typename T, int V> struct Pack { typedef T type __attribute__((ext_vector_type(V))); };
 struct RowColumn { long long row; int column; };
 __device__ __forceinline__ RowColumn row_column(long long index, int width, long long total) {
@@ -461,7 +465,7 @@ extern "C" int vk_swiglu(const void* gate_up, void* out, int dtype, int num_toke
   const long long total = (long long)num_tokens * inter;
   if (dtype != DT_F32 && dtype != DT_BF16) return VK_BAD_ARGUMENT;
   const int bytes = dtype == DT_F32 ? 4 : 2;
-  const bool fours = in_fours(gate_up, inter, bytes) && in_fours(out, inter, bytes);
+  const bool fours = total >= FOURS_FROM && in_fours(gate_up, inter, bytes) && in_fours(out, inter, bytes);
   const long long blocks = min((total / (fours ? 4 : 1) + 255) / 256, 65536ll);
   hipStream_t s = (hipStream_t)stream;
 #define VK_SWIGLU(T, V) swiglu_kernel<T, V><<<(int)blocks, 256, 0, s>>>((const T*)gate_up, (T*)out, inter, total, interleaved)
@@ -761,7 +765,7 @@ extern "C" int vk_activation(const void* in, int in_dtype, long long ldi, const 
   hipStream_t s = (hipStream_t)stream;
   if (mul == nullptr) mul_dtype = DT_F32;
   auto bytes = [](int dtype) { return dtype == DT_F32 ? 4 : 2; };
-  const bool fours = width % 4 == 0 && in_fours(in, ldi, bytes(in_dtype)) && in_fours(out, ldo, bytes(out_dtype)) &&
+  const bool fours = total >= FOURS_FROM && width % 4 == 0 && in_fours(in, ldi, bytes(in_dtype)) && in_fours(out, ldo, bytes(out_dtype)) &&
                      (!mul || in_fours(mul, ldm, bytes(mul_dtype)));
   const unsigned blocks = (unsigned)((total / (fours ? 4 : 1) + 255) / 256);
 #define VK_ACT_V(TI, TM, TO, V)                                                                                     \
@@ -957,7 +961,8 @@ extern "C" int vk_head_unpack_gate(const void* attn, int dtype, const float* g, 
   const long long total = (long long)num_tokens * heads * vdim;
   if (dtype != DT_F32 && dtype != DT_BF16) return VK_BAD_ARGUMENT;
   const int bytes = dtype == DT_F32 ? 4 : 2;
-  const bool fours = vdim % 4 == 0 && in_fours(attn, W, bytes) && in_fours(out, vdim, bytes) && (!g || in_fours(g, ldg, 4));
+  const bool fours = total >= FOURS_FROM && vdim % 4 == 0 && in_fours(attn, W, bytes) && in_fours(out, vdim, bytes) &&
+                     (!g || in_fours(g, ldg, 4));
   const unsigned blocks = (unsigned)((total / (fours ? 4 : 1) + 255) / 256);
   hipStream_t s = (hipStream_t)stream;
 #define VK_UNPACK(T, V) \
