@@ -1435,6 +1435,24 @@ def test_passes_over_many_rows_in_fours_give_the_bits_of_one_number_at_a_time(ro
     test_passes_over_rows_in_fours_give_the_bits_of_one_number_at_a_time(rows, width, dtype)
 
 
+@pytest.mark.parametrize("tokens,channels", [(1, 1), (7, 512), (1100, 508), (1023, 512), (1024, 512), (130, 4100), (997, 4001), (1049, 4001), (8300, 508)])
+def test_every_form_of_the_scans_preparation_gives_the_same_bits(tokens, channels):
+    """On both sides of the lines between a thread a number and four a thread, in rows on 16 bytes and off them: the bits of steps of
+    one token, and 64-bit."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator(DEV).manual_seed(tokens + channels)
+    wide, bias = torch.randn(tokens, 2 * channels + 4, generator=g, device=DEV) * 4, torch.randn(channels, generator=g, device=DEV)
+    for step, z in ((wide[:, :channels].clone(), wide[:, -channels:]), (wide.clone()[:, 1:channels + 1], wide[:, 1:channels + 1])):
+        first, gate = step.clone(), torch.full((tokens, channels), float("nan"), device=DEV)
+        kernels.scan_prepare(step, bias, z, gate)
+        assert _rel(step, torch.nn.functional.softplus(first.double() + bias.double())) < 2e-6
+        assert _rel(gate, torch.nn.functional.silu(z.double())) < 2e-6
+        for t in {0, tokens // 2, tokens - 1}:
+            one, alone = first[t:t + 1].clone(), torch.empty(1, channels, device=DEV)
+            kernels.scan_prepare(one, bias, z[t:t + 1], alone)
+            assert torch.equal(one, step[t:t + 1]) and torch.equal(alone, gate[t:t + 1])
+
+
 @pytest.mark.parametrize("tokens,width,dtype", [(514, 36, torch.bfloat16), (515, 1028, torch.float32), (640, 64, torch.bfloat16)])
 def test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, width, dtype):
     """A step of 512 tokens or more against the same tokens in smaller steps: entries that begin inside a run, behind a state and at

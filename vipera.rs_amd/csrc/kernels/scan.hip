@@ -818,8 +818,11 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
 
 // dt[t, c] <- softplus(dt[t, c] + dt_bias[c]) in place and gate[t, c] = silu(z[t, c]): what the scan of a prompt's
 // portion would otherwise compute token behind token.  Grid (tokens, parts of 1,024 channels), four channels a thread: neighbours
-// (VEC: rows in 16 bytes) or 256 apart.  Bound by memory; a thread a number, which divided its index by C in 64 bits, took 36.4 us
-// for 1,834 tokens of 4,096 channels, this 28.4 (one number at a time 31).
+// (VEC: rows in 16 bytes) or 256 apart.  Many numbers are bound by memory: 1,834 tokens of 4,096 channels take 26.1 us in fours, 28.4
+// 256 apart and 32.2 a thread a number (scan_prepare_each_kernel).  Few numbers are bound by a thread's own chain, four
+// exponentials and logarithms behind one another instead of one, and rows of few channels leave most of a workgroup idle: us, a thread
+// a number, in fours and 256 apart, 333 tokens of 64 channels 2.8 / 4.9 / 2.8, 128 of 2,048 3.5 / 3.9 / 4.7, 333 of 1,000 4.1 / 4.7 / 5.5, 128 of 4,096
+// 4.7 / 4.6 / 5.3, 4,096 of 256 7.2 / 7.2 / 6.6, 333 of 4,097 8.6 / - / 9.6, 1,834 of 4,097 31.9 / - / 28.6.
 template <bool VEC>
 __global__ __launch_bounds__(256) void scan_prepare_kernel(float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
                                                            const float* __restrict__ z, long long ldz, float* __restrict__ gate,
@@ -854,6 +857,21 @@ __global__ __launch_bounds__(256) void scan_prepare_kernel(float* __restrict__ d
   }
 }
 
+// The same, a thread a number; at most 2^32 - 256 of them, which is what a launch counts.
+__global__ __launch_bounds__(256) void scan_prepare_each_kernel(float* __restrict__ dt, long long lddt, const float* __restrict__ dt_bias,
+                                                                const float* __restrict__ z, long long ldz,
+                                                                float* __restrict__ gate, int C, unsigned total) {
+  const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+  if (idx >= total) return;
+  const unsigned t = idx / (unsigned)C, c = idx - t * (unsigned)C;
+  float* step = dt + t * lddt;
+  const float d = step[c], bias = dt_bias[c], g = z[t * ldz + c];
+  step[c] = scan_softplus(d + bias);
+  gate[idx] = scan_silu(g);
+}
+constexpr int SCAN_ROW = 512;                                        // channels from which a row is worth a workgroup,
+constexpr long long SCAN_FOURS = 1 << 19, SCAN_APART = 1 << 22;      // and numbers from which a thread takes four of it
+
 extern "C" int vk_scan_prepare(float* dt, long long lddt, const float* dt_bias, const float* z, long long ldz,
                                float* gate, int num_tokens, int C, void* stream) {
   if (num_tokens <= 0) return 0;
@@ -861,7 +879,10 @@ extern "C" int vk_scan_prepare(float* dt, long long lddt, const float* dt_bias, 
   const dim3 grid(num_tokens, (unsigned)min((C + 1023LL) / 1024, 65535LL));
   const bool vec = C % 4 == 0 && lddt % 4 == 0 && ldz % 4 == 0 &&
                    (((uintptr_t)dt | (uintptr_t)dt_bias | (uintptr_t)z | (uintptr_t)gate) & 15) == 0;
-  if (vec) scan_prepare_kernel<true><<<grid, 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C);
+  const long long total = (long long)num_tokens * C;
+  if ((C < SCAN_ROW || total < (vec ? SCAN_FOURS : SCAN_APART)) && total <= 0xffffff00ll)
+    scan_prepare_each_kernel<<<(unsigned)((total + 255) / 256), 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C, (unsigned)total);
+  else if (vec) scan_prepare_kernel<true><<<grid, 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C);
   else scan_prepare_kernel<false><<<grid, 256, 0, (hipStream_t)stream>>>(dt, lddt, dt_bias, z, ldz, gate, C);
   VK_LAUNCH_CHECK();
   return 0;
