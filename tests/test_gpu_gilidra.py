@@ -438,6 +438,13 @@ def test_prompts_prepared_in_runs_give_the_bits_of_single_tokens(taps, sizes):
         assert torch.equal(whole, part)
 
 
+@pytest.mark.parametrize("taps,sizes", [(4, (2, 8, 128, 128)), (4, (1, 31, 64, 33)), (3, (1, 4, 256, 256)), (2, (1, 25, 64, 41)),
+                                        (4, (6, 6, 64, 20)), (3, (5, 5, 64, 24)), (2, (6, 6, 128, 15))])
+def test_prompts_prepared_in_runs_at_the_lines_of_their_choice(taps, sizes):
+    """From 1,024 channels of values or 2,600 workgroups of a token each on (13 of them a token here), and just below either."""
+    test_prompts_prepared_in_runs_give_the_bits_of_single_tokens(taps, sizes)
+
+
 @pytest.mark.parametrize("rule", ["delta", "delta_channel", "wkv"])
 @pytest.mark.parametrize("sizes", [(1, 2, 20, 9), (2, 4, 64, 16), (1, 3, 72, 8), (2, 2, 128, 24), (1, 1, 200, 5)])
 def test_prompts_recurrences_in_whole_and_partial_blocks(rule, sizes):

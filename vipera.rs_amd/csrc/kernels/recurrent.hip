@@ -93,9 +93,14 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
 // them.  Above, a workgroup of one token and 128 channels of its head leaves half its threads idle and waits for entry, taps and
 // inputs one behind another, a few microseconds for a kilobyte.  dim: 64, 128 or 256, so that a head lies in one workgroup.
 // us with the state's rows after it, 4,096 channels of four taps, before and so: 2,048 tokens 74.0 / 26.3 (their rows' way from
-// and to memory takes some 15), 512 25.4 / 10.8, 128 9.9 / 7.9; 100 tokens of 2,048 channels 7.5 / 7.8.  Runs of 8: 25.4, 11.6 and
-// 10.4; of 16: 24.5, 16.1 and 15.3.
+// and to memory takes some 15), 512 25.4 / 10.8, 128 9.9 / 7.9.  Runs of 8: 25.4, 11.6 and 10.4; of 16: 24.5, 16.1 and 15.3.
+// A run's own chain is longer than a token's: it is taken where the workgroups above are more than the chip holds at once, or where
+// they walk 1,024 channels of values in four turns.  us, a token and a run a thread, one entry: 128 tokens of 2 key heads of 64 and 256
+// channels of values (640 workgroups) 6.6 / 8.0, of 4 of 128 and 512 (1,152) 7.5 / 8.2, of 4 of 128 and 1,024 (1,152) 9.8 / 8.2; 800 of 1 of
+// 128 and 66 (2,400) 6.9 / 7.4, 512 of 2 of 64 and 256 (2,560) 7.9 / 8.1, 300 of 4 of 128 and 512 (2,700) 9.5 / 8.4, 800 of 2 of 64 and 256
+// (4,000) 9.5 / 8.0.
 constexpr int PREP_RUN = 4, PREP_RUN_TOKENS = 128;
+constexpr long long PREP_RUN_BLOCKS = 2600;
 template <int TAPS>
 __global__ __launch_bounds__(256) void delta_prepare_run_kernel(
     const float* __restrict__ proj, long long ldp, const float* __restrict__ conv, const float* __restrict__ state,
@@ -1115,7 +1120,8 @@ extern "C" int vk_delta_prepare_strided(const float* proj, long long ldp, const 
   delta_prepare_run_kernel<TAPS><<<run_grid, 256, 0, s>>>(proj, ldp, conv, state, state_stride, conv_offset, entry_of,   \
                                                           entry_start, entry_first, slots, a_log, dt_bias, kv_heads, dim, \
                                                           heads, vdim, b_col, a_col, unit_eps, qkv, ldq, beta, decay, num_tokens)
-  const bool runs = (dim == 64 || dim == 128 || dim == 256) && num_tokens >= PREP_RUN_TOKENS && run_grid.y <= 65535;
+  const bool runs = (dim == 64 || dim == 128 || dim == 256) && num_tokens >= PREP_RUN_TOKENS && run_grid.y <= 65535 &&
+                    (num_tokens * segments >= PREP_RUN_BLOCKS || (long long)heads * vdim >= PREP_SPAN);
   if (runs && taps == 4) VK_PREPARE_RUN(4);
   else if (runs && taps == 3) VK_PREPARE_RUN(3);
   else if (runs && taps == 2) VK_PREPARE_RUN(2);
