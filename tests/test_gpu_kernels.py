@@ -1478,6 +1478,13 @@ def test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, wid
     assert torch.equal(whole, parts) and torch.equal(left, one)
 
 
+@pytest.mark.parametrize("tokens,width,dtype", [(515, 256, torch.float32), (515, 260, torch.bfloat16), (2047, 256, torch.bfloat16),
+                                                (2049, 256, torch.float32), (4099, 128, torch.bfloat16)])
+def test_token_shift_of_narrow_rows_gives_the_bits_of_single_tokens(tokens, width, dtype):
+    """On both sides of a row's turn of a workgroup and of the 524,288 numbers from which narrower rows go in runs."""
+    test_token_shift_in_runs_of_four_gives_the_bits_of_single_tokens(tokens, width, dtype)
+
+
 @pytest.mark.parametrize("tokens,heads,k,n", [(1, 2, 64, 64), (64, 3, 128, 192), (65, 2, 192, 100), (200, 1, 320, 33)])
 def test_products_per_head_in_tiles_of_64_give_the_bits_of_the_wide_ones(tokens, heads, k, n):
     """K in whole steps of 64 against the same numbers with eight zeros more, which take the tiles of 128 x 128: tokens and outputs that

@@ -720,8 +720,11 @@ __global__ __launch_bounds__(256) void token_shift_kernel(const T* __restrict__ 
 
 // The same for many tokens: four channels of SHIFT_RUN consecutive tokens a thread, so that a vector of factors is read once for
 // them and everything moves in pieces of four numbers.  2,048 tokens of 2,048 channels, six vectors, 16-bit: 27.0 -> 15.5 us;
-// 512 of them 14.0 -> 8.3.
-constexpr int SHIFT_RUN = 4;
+// 512 of them 14.0 -> 8.3.  A row of up to 256 channels is one turn of a workgroup above and a quarter of one here: there runs are for
+// many tokens.  us, six vectors, 16-bit: 512 tokens of 64 channels 4.8 / 5.7, of 256 5.0 / 5.6, of 320 6.0 / 6.0; 1,300 of 256 5.9 / 6.1, 2,048
+// of 192 6.1 / 6.1, of 256 6.5 / 6.3.
+constexpr int SHIFT_RUN = 4, SHIFT_TURN = 256;
+constexpr long long SHIFT_MANY = 1 << 19;
 template <typename T>
 __global__ __launch_bounds__(256) void token_shift_run_kernel(const T* __restrict__ h, int width, const float* __restrict__ mu,
                                                               int mixes, const float* __restrict__ state,
@@ -1341,7 +1344,7 @@ extern "C" int vk_token_shift(const void* h, int dtype, int width, const float* 
   const unsigned spans = num_tokens >= 512 ? 1u : (unsigned)min(64, (width + 255) / 256);
   const dim3 tokens_grid(num_tokens, spans), entries_grid(num_entries, spans);
   const int bytes = dtype == DT_F32 ? 4 : 2;
-  const bool runs = num_tokens >= 512 && width % 4 == 0 && state_stride % 4 == 0 && prev_offset % 4 == 0 &&
+  const bool runs = num_tokens >= 512 && (width > SHIFT_TURN || (long long)num_tokens * width >= SHIFT_MANY) && width % 4 == 0 && state_stride % 4 == 0 && prev_offset % 4 == 0 &&
                     (((uintptr_t)mu | (uintptr_t)state) & 15) == 0 && (((uintptr_t)h | (uintptr_t)out) % (4 * bytes)) == 0;
   const dim3 runs_grid((num_tokens + SHIFT_RUN - 1) / SHIFT_RUN, (unsigned)min(64, (width + 1023) / 1024));
   if (dtype == DT_F32) {
