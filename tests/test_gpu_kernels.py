@@ -639,6 +639,35 @@ def test_gemm_generic_needs_no_memory_for_its_parts():
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("m,n,k,slabs", [(333, 1152, 896, 0), (64, 1536, 8960, 9), (65, 17930, 1540, 0), (333, 1152, 1100, 2)])
+def test_a_32_bit_product_allocates_no_more_than_it_writes(m, n, k, slabs):
+    """With that memory, and with all that any types would take, the same form and the same bits; with less it is refused."""
+    import ctypes
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.build import load_module
+    g = torch.Generator(DEV).manual_seed(m + n + k)
+    a, w = torch.randn(m, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    out, all_parts = torch.empty(m, n, device=DEV), torch.empty(kernels._gemm_generic_parts(m, n, k), device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    kernels.gemm_generic(a, w, None, out)
+    assert torch.cuda.max_memory_allocated() - before <= slabs * m * n * 4 + 512
+    lib, other = load_module("gemm_generic"), torch.empty(m, n, device=DEV)
+    chosen = lib.vk_gemm_generic_form
+    chosen.argtypes, chosen.restype = [ctypes.c_int] * 3 + [ctypes.c_longlong], ctypes.c_int
+    assert chosen(m, n, k, slabs * m * n) == chosen(m, n, k, all_parts.numel())
+    p, split = ctypes.c_void_p, lib.vk_gemm_generic_split
+    def with_floats(floats):
+        return split(p(a.data_ptr()), 0, p(w.data_ptr()), 0, p(0), p(other.data_ptr()), 0, m, n, k, ctypes.c_longlong(k), ctypes.c_longlong(n), 0,
+                     p(all_parts.data_ptr()), ctypes.c_longlong(floats), p(torch.cuda.current_stream().cuda_stream))
+    assert with_floats(all_parts.numel()) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, other)
+    assert not slabs or with_floats(slabs * m * n - 1) != 0
+
+
 def test_gemm_generic_of_more_tiles_than_one_launch_takes():
     """Past 2^32 threads in its tiles a product is several launches: 1,048,576 x 65,600 outputs, 138 GB in bfloat16."""
     from vipera_rs_amd.ops import kernels

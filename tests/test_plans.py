@@ -177,6 +177,14 @@ def test_the_cut_of_a_32_bit_product_is_asked_for_once_for_a_size(monkeypatch):
     assert asked == ["vk_gemm_generic_workspace"] and first == kernels._gemm_generic_parts(77, 1155, 899) and len(asked) == 1
 
 
+def test_an_aligned_32_bit_product_asks_for_the_memory_that_its_form_writes():
+    from vipera_rs_amd.ops.kernels import _gemm_direct_parts, _gemm_generic_parts
+    assert _gemm_generic_parts(333, 1152, 896) == 4 * 333 * 1152 and _gemm_direct_parts(333, 1152, 896) == 0       # one slab
+    assert _gemm_generic_parts(64, 1536, 8960) == 35 * 64 * 1536 and _gemm_direct_parts(64, 1536, 8960) == 9 * 64 * 1536
+    assert _gemm_generic_parts(65, 17930, 1540) == 2 * 65 * 17930 and _gemm_direct_parts(65, 17930, 1540) == 0     # walks all of K
+    assert _gemm_generic_parts(2048, 9728, 8960) == 0 == _gemm_direct_parts(2048, 9728, 8960)
+
+
 def test_past_128_tokens_small_tiles_carry_out_a_128x128_plan_unless_its_tiles_fill_the_gpu():
     """The tiling and the ranges of K.  Tilings 9: 128x128, 13: 64x64 with K split, 14: 64x64 that walk K, 15: 128x64 that walk K."""
     from vipera_rs_amd.ops.kernels import gemm_bf16_tile_plan as plan

@@ -981,15 +981,28 @@ extern "C" long long vk_gemm_generic_workspace(int M, int N, int K) {
   return units ? (long long)((K + units * RANGE_K - 1) / (units * RANGE_K)) * M * N : 0;
 }
 
+// Those of them that the product leaves in memory where its operands are all 32-bit and aligned (direct_takes): one sum a slab in
+// the forms over slabs, none where K is one slab or a workgroup walks it. The form is the one that takes all of them into account.
+extern "C" long long vk_gemm_generic_direct_workspace(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= SLAB_K || K > DIRECT_MAX_ROW) return 0;
+  switch (direct_plan(M, N, K, vk_gemm_generic_workspace(M, N, K))) {
+    case NOT_DIRECT: case ROWS_64_64: case ROWS_32_128: case ROWS_64_128: return 0;
+    default: return (long long)((K + SLAB_K - 1) / SLAB_K) * M * N;
+  }
+}
+
 // The same product, with K split over workgroups where the tiles alone are too few. `parts`: a workspace of
-// vk_gemm_generic_workspace(M, N, K) floats, aligned to 16 bytes.
+// vk_gemm_generic_workspace(M, N, K) floats, or of vk_gemm_generic_direct_workspace(M, N, K) where that covers the operands, aligned
+// to 16 bytes.
 extern "C" int vk_gemm_generic_split(const void* A, int a_dtype, const void* W, int w_dtype, const float* bias, void* C,
                                      int c_dtype, int M, int N, int K, long long lda, long long ldc, int accumulate,
                                      float* parts, long long part_floats, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldc < N) return VK_BAD_ARGUMENT;
   if ((M + TILE - 1) / TILE > 65535) return VK_UNSUPPORTED_SIZE;
-  if (vk_gemm_generic_workspace(M, N, K) > part_floats || ((uintptr_t)parts & 15)) return VK_BAD_ARGUMENT;
+  const bool direct = direct_takes(A, a_dtype, W, w_dtype, c_dtype, K, lda);
+  const long long floats = direct ? vk_gemm_generic_direct_workspace(M, N, K) : vk_gemm_generic_workspace(M, N, K);
+  if (floats > part_floats || ((uintptr_t)parts & 15)) return VK_BAD_ARGUMENT;
   return dispatch(A, a_dtype, W, w_dtype, bias, C, c_dtype, M, N, K, lda, ldc, accumulate, parts, part_floats,
                   (hipStream_t)stream);
 }

@@ -228,11 +228,21 @@ def fill_normal(out: torch.Tensor, key: int, std: float, offset: float = 0.0) ->
 
 
 # ----------------------------------------------------------------------------------------------
+GEMM_DIRECT_MAX_ROW = 4000000     # numbers in a row of the 32-bit kernels that load straight into LDS
+
+
 @functools.lru_cache(maxsize=4096)
 def _gemm_generic_parts(m: int, n: int, k: int) -> int:
     """Floats of the sums that the tiled 32-bit product of these sizes leaves in memory between its two launches; 0: K is
     not cut.  Asked once for a size: a call into the library is 0.9 us of the 8 that a launch takes the host."""
     return _fn("gemm_generic", "vk_gemm_generic_workspace", [_i, _i, _i], restype=_ll)(m, n, k)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_direct_parts(m: int, n: int, k: int) -> int:
+    """The same where all operands are 32-bit and their rows start on 16 bytes: one sum a slab of 1,024 k, and none where K is one
+    slab or walked whole."""
+    return _fn("gemm_generic", "vk_gemm_generic_direct_workspace", [_i, _i, _i], restype=_ll)(m, n, k)
 
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
@@ -253,8 +263,9 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
         _need(out.dtype == torch.float32, "gemm: accumulation needs a float32 output")
     lda = a.stride(0) if m > 1 else max(a.stride(0), k)
     ldc = out.stride(0) if m > 1 else max(out.stride(0), n)
-    if (m <= 8 and a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0 and lda % 4 == 0
-            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and k < 65535 * 1024):
+    aligned = (a.dtype == torch.float32 and w.dtype == torch.float32 and k >= 4 and k % 4 == 0 and lda % 4 == 0
+               and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+    if m <= 8 and aligned and k < 65535 * 1024:
         # up to 8 tokens in 32-bit: a stream of the weights (the same sums in the same order as the tiled kernel, whose
         # matrix cores pass the stream's FMAs from there on: 9,728 x 896 at 8 tokens 21.2 us against 23.1, at 16 43.3 against
         # 22.7; 37,888 x 3,584 at 8 tokens 117 against 196, at 16 213 against 188; 151,936 x 896 113 against 206 and 212
@@ -267,7 +278,8 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     # K split over workgroups where the tiles are too few; the parts belong to this call alone, on whatever stream it runs.
     # Where the memory for them is not there a workgroup walks all of K instead: the same bits, more time.
     parts = None
-    floats = _gemm_generic_parts(m, n, k)
+    direct = aligned and out.dtype == torch.float32 and max(lda, k) <= GEMM_DIRECT_MAX_ROW
+    floats = _gemm_direct_parts(m, n, k) if direct else _gemm_generic_parts(m, n, k)
     if floats:
         try:
             parts = torch.empty(floats, dtype=torch.float32, device=a.device)
