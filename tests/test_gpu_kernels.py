@@ -187,6 +187,77 @@ def test_gated_products_of_up_to_64_tokens_take_tiles_of_64_with_the_same_bits(r
         assert _rel(got[0][0], up * gate / (1 + torch.exp(-gate))) < 8e-3
 
 
+@pytest.mark.parametrize("rows,tiling", [(96, 21), (96 * 256, 22), (96 * 256 + 32, 23), (160 * 256, 24), (224 * 256, 25)])
+@pytest.mark.parametrize("m,k", [(17, 320), (33, 1088), (64, 2112), (40, 768)])
+def test_tiles_of_64_tokens_give_the_bits_of_the_kernel_that_shares_the_activations(rows, tiling, m, k):
+    """That kernel takes up to 16 tokens at these K: every 16 tokens through it, K in several of its chunks of 256 and the rest of
+    one, and of five to 33 steps of the tiles."""
+    from vipera_rs_amd.ops import kernels
+    if kernels.compute_units(torch.device(DEV)) != 256:
+        pytest.skip("the widths follow the number of CUs")
+    g = torch.Generator(DEV).manual_seed(rows + m)
+    a = torch.randn(m, k, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn(rows, k, generator=g, device=DEV).to(torch.bfloat16)
+    got = torch.full((m, rows // 2), 7.0, dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_bf16_gated(a, w, got, 1)
+    assert kernels.gemm_bf16_tile_launched()[0] == tiling
+    for plan in (1, 2):
+        shared = torch.full((m, rows // 2), 7.0, dtype=torch.bfloat16, device=DEV)
+        for first in range(0, m, 16):
+            kernels.gemm_bf16_gated(a[first:first + 16], w, shared[first:first + 16], plan)
+        assert torch.equal(got, shared), plan
+
+
+@pytest.mark.parametrize("plan", [1, 2])
+@pytest.mark.parametrize("m,rows,k", [(24, 512, 2048), (33, 1056, 2048), (49, 96, 4096), (64, 8192, 2048), (64, 544, 264), (20, 160, 1032),
+                                      (48, 64, 520)])
+def test_the_kernel_that_shares_the_activations_takes_17_to_64_tokens_where_tiles_do_not(m, rows, k, plan):
+    """K a multiple of 2,048, where its workgroups start at chunks of their own, and K in no whole steps of 64: two to four blocks of
+    16 tokens give the bits of one block at a time, and 64-bit."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator(DEV).manual_seed(rows + m)
+    a = torch.randn(m, k, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn(rows, k, generator=g, device=DEV).to(torch.bfloat16)
+    out, blocks = (torch.full((m, rows // 2), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    before = kernels.gemm_bf16_tile_launched()
+    kernels.gemm_bf16_gated(a, w, out, plan)
+    for first in range(0, m, 16):
+        kernels.gemm_bf16_gated(a[first:first + 16], w, blocks[first:first + 16], plan)
+    assert kernels.gemm_bf16_tile_launched() == before          # no tile ran
+    assert torch.equal(out, blocks)
+    gate, up = (a.double() @ w.double().T).view(m, rows // 32, 2, 16).unbind(2)
+    gate, up = gate.reshape(m, -1), up.reshape(m, -1)
+    assert _rel(out, up * gate / (1 + torch.exp(-gate))) < 8e-3
+
+
+@pytest.mark.parametrize("tiling,other", [(5, 7), (6, 7), (9, 8)])
+def test_tiles_with_a_third_stage_of_the_weight_divide_by_a_norm_with_the_bits_of_the_others(tiling, other):
+    """The norm's sums follow the loop there, in LDS that held the stages: runs of K shorter than the stages, as long and longer,
+    against the tiles of as many threads a token, which add them before it."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(tiling)
+    for m, rows in ((257, 288), (300, 416)):
+        for k in (64, 128, 192, 256, 320, 1152):
+            a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+            w = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+            for groups in (1, 7, 70):
+                stride = kernels.follow_stride(m)
+                sumsq = (torch.rand(groups * stride, generator=g) * k / groups).to(DEV)
+                outs = [torch.full((m, rows // 2), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+                try:
+                    for one, out in zip((tiling, other), outs):
+                        kernels.gemm_bf16_force_tiling(one)
+                        kernels.gemm_bf16_gated_tile_scaled(a, w, out, sumsq, groups, 1e-5)
+                        assert kernels.gemm_bf16_tile_launched()[0] == one
+                finally:
+                    kernels.gemm_bf16_force_tiling(-1)
+                assert torch.equal(*outs), (m, rows, k, groups)
+                factor = 1 / torch.sqrt(sumsq.view(groups, stride)[:, :m].double().sum(0) / k + 1e-5)
+                gate, up = (a.double() @ w.double().T * factor[:, None]).view(m, rows // 32, 2, 16).unbind(2)
+                gate, up = gate.reshape(m, -1), up.reshape(m, -1)
+                assert _rel(outs[0], up * gate / (1 + torch.exp(-gate))) < 8e-3
+
+
 @pytest.mark.parametrize("m,n,k,tiling", [(1396, 1536, 1536, 16), (783, 4096, 2048, 17), (1000, 4608, 3584, 18), (2210, 4096, 1024, 19),
                                           (910, 9216, 2048, 20)])
 def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):

@@ -302,6 +302,12 @@ def test_gated_product_beside_its_twin(m, inter, k, plan):
     assert rel_err(got.float().numpy(), want.double().numpy()) < 8e-3
 
 
+@pytest.mark.parametrize("m,inter,k,plan", [(24, 64, 2048, 1), (33, 80, 2048, 2), (64, 256, 2048, 2), (64, 128, 264, 1), (49, 48, 520, 2)])
+def test_gated_product_of_17_to_64_tokens_off_the_tiles_beside_its_twin(m, inter, k, plan):
+    """K a multiple of 2,048 or in no whole steps of 64: two to four blocks of 16 tokens share the activations through LDS."""
+    test_gated_product_beside_its_twin(m, inter, k, plan)
+
+
 def _paged(T, kv_heads, hd, bs, dtype, seed, entries=1):
     """A cache whose pages are dealt out in a shuffled order, and its table: [entries, pages per entry]."""
     g = torch.Generator().manual_seed(seed)
