@@ -441,7 +441,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const __bf16* _
 // activations, so at the barrier the newest request of weights may stay in flight. Weights from memory, two stages to three: gate/up
 // of 2,048 tokens on 37,888 rows of 3,584 456 to 426 us (1.31 PFLOP/s), of 1,000 tokens 257 to 240, 1,396 on 17,920 of 1,536
 // 79.3 to 77.2; 256x192 tiles: 2,048 on 6,144 rows of 2,048 47.8 to 45.5, on 3,584 of 18,944 350 to 288; 128x128 tiles, two to a
-// CU: 1,396 on 17,920 of 1,536 92.1 to 88.2, on 1,536 of 8,960 115 to 98. No faster with a third one: 256x128 (three of both: 240
+// CU: 1,396 on 17,920 of 1,536 92.1 to 88.2, on 1,536 of 8,960 115 to 98. As the launcher chooses tiles for 350 products of 129 to 2,500
+// tokens, 256x256 take 0.99 of the time with two stages, 256x192 0.94 and 128x128 1.00 (0.93 to 1.03, and 1.06 for a gated 622
+// on 9,728 of 896). No faster with a third one: 256x128 (three of both: 240
 // us either way at 3,584 rows of 18,944), 192x192; slower: the weights' loads spread over the other half of the step.
 // group_tile_direct (group_tile.h) is the same loop over gathered rows; a change to one is to be weighed for the other.
 constexpr int DIRECT_ROW = BK * 2;  // bytes per LDS row
@@ -2025,8 +2027,11 @@ TilePlan tile_plan(int M, int N, int K, long long partial_floats, bool gated, bo
 // 0.98 of the planned one's. us, planned to picked: 1,396 tokens on 2,048 rows of 1,536 21.4 -> 14.8, on 1,536
 // rows 19.7 -> 16.2, 1,383 on 2,048 of 2,048 24.4 -> 18.2, 1,000 on 4,608 of 3,584 49.0 -> 37.8, 1,014 on 3,584 of 3,584
 // 48.3 -> 38.8; gated: 1,396 on 17,920 of 1,536 89.8 -> 80.7, 622 on 5,120 of 2,048 25.0 -> 20.1, 311 on 22,016 46.1 -> 36.2.
-// The fit is with two stages of the weight's rows in 256x256, 256x192 and 128x128; the third one has since taken up to 7 % off their
-// steps in a full round and little off short ones, and the fit stands.
+// The fit is with two stages of the weight's rows in 256x256, 256x192 and 128x128; the third one has since taken up to 5, 14 and 7 %
+// off such products, and the fit has not followed: it passes 256x192 by where that is now the fastest. Over 187 products of K 512
+// and more the choice takes 0.94 of the planned ones' time and 1.008 of the fastest tile's; the worst are planned as 256x192 and changed
+// for 192x128: 2,500 tokens on 3,584 rows of 3,584 70.5 us against 61.7, 2,048 on 4,608 of 3,584 71.4 against 65.1, 2,500 on 4,096 of
+// 2,048 45.8 against 41.9. Below K 512, 33 products, 1.03 and up to 1.19 (5 to 7 us a call).
 // Every output is one sum over K in ascending steps of 32 whatever the tile, so the bits are the same.
 struct TileCost { int config, tokens, rows, resident; double beside, low, high, pair, alone, output; };
 constexpr TileCost WHOLE_TILES[] = {

@@ -173,14 +173,17 @@ def gated_plan(m: int, n: int, k: int, cus: int = 256) -> int:
     enough over the ``cus`` workgroups (every CU with a pair of 16-row tiles at least, the busiest within 10 % of the
     mean: at 7B and 32B widths it measured 2 to 7 % faster than the LDS-shared kernel when its runs were still whole
     pairs, and it can divide by the norm before it, which saves that norm's kernel); else the LDS-shared kernel with
-    one or two tiles per wave."""
+    one or two tiles per wave.  Past 16 tokens :func:`kernels.gemm_bf16_gated` runs 1 and 2 on tiles of 64 tokens where these have
+    the same bits, K in whole steps of 64 but not of 2,048.  The norm before such a product stays a kernel of its own all the same:
+    dividing inside the product would round ``x * gain`` to bfloat16 instead of ``x * inv * gain``, which are other bits."""
     pairs, quads = n // 32, n // 8
     if gated_resident_fits(m, n, k) and pairs >= cus and -(-quads // cus) * cus <= 1.1 * quads:
         return 0
     if m <= 32 and k % 2048 == 0 and n * k >= 4e8:
         # the largest weights with rows a multiple of 4 KB apart, where the LDS-shared kernel's workgroups start at
-        # different chunks: it streams them faster than the tiled one (72B, 59,136 x 8,192, at 17 to 32 tokens: 164
-        # to 171 us against 185; at 64 the norm's own kernel, which only the tiled one saves, makes them even)
+        # different chunks: it streams them faster than the tiled one's tiles of 64 tokens (72B, 59,136 x 8,192: 167 to 170 us
+        # against 173 to 176 at 17 to 32 tokens, 169 and 174 at 33, 172 and 173 at 48, 181 and 176 at 64; from 33 on the norm's own
+        # kernel, which only the tiled one saves, makes up for it)
         return gated_rows_per_wave(m, n)
     if n * k >= 1e8 or m * n * k >= 1.5e9:
         # a large weight, or many tokens on a small one: the tiled kernel (3) with tiles of 64 tokens and of 64 to 224
