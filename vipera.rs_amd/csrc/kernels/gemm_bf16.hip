@@ -654,7 +654,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_direct_kernel(const __
       for (int j = 0; j < TM; ++j) acc[i][j] = folded[i][j] + acc[i][j];
   }
   if constexpr (W_MORE > 0) {
-    if (norm.sumsq) {
+    if (norm.sumsq) {    // from callers of the product alone: a model's steps divide in it up to 64 tokens, on other tiles
       __syncthreads();   // nobody reads a stage any more, and no load into one is in flight
       tile_norm_parts<BM, WAVES * 64>(norm, m0, M, tid, part_sums);
       __syncthreads();
