@@ -658,8 +658,8 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
 //         64 x 128          3.5 + 0.0313 K, 0.0055 K for every two                   333 x 9,728 x 896: 68.0 (80.7)
 // Two or three stages leave room for a second or third workgroup on a CU, which hide a wave's own chain of loads better than a
 // deeper queue of its own does (a slab's 64 x 64 with four stages took 1.10 of the time with two).  Over 233 sizes from 12 to
-// 2,048 rows and K 700 or more the choice takes 0.885 of the time of the kernels of commit 7de7731, which exchanged lanes' values and
-// had no tiles of 48 x 48 (geometric mean), 1.006 of it at worst, and 1.012 of the best form's.  The 64 x 64 tiles cut over workgroups
+// 2,048 rows and K 700 or more the choice takes 0.885 of the time of kernels that exchanged lanes' values, with as many stages and
+// without tiles of 48 x 48 (geometric mean), 1.006 of it at worst, and 1.012 of the best form's.  The 64 x 64 tiles cut over workgroups
 // are the fastest at none of them; they keep any other type, and rows off 16 bytes.
 // Below K 704 a slab's ranges are short or missing, while a walk over all of K has its first loads and its last stores to wait for:
 //   slab   the first tile takes what a range of K takes (256 of k or less), each further one on the CU `range` of a step for a whole
@@ -667,10 +667,10 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
 //   rows   `first` more beside it, `each` more a tile, and K in whole steps of 32
 //   the 64 x 64 tiles (two stages through registers, no slab to end), which pass both where K is a step or two
 // us, as chosen without that and now: 500 x 130 x 132 7.1 / 4.6, 65 x 4,096 x 132 7.7 / 5.8, 257 x 1,152 x 64 5.0 / 4.1, 9 x 9,728 x
-// 260 9.7 / 6.6, 2,500 x 9,728 x 16 36.4 / 26.9.  Over 1,430 sizes of K 4 to 1,000 the choice takes 0.89 of the time of the kernels of
-// commit eb72a37, the last before two workgroups shared a CU (1.03 without it), and 1.026 of the best form's; at worst 1.12 of theirs, 1,396 x
-// 9,728 x 24 as 64 x 128, and 2,500 x 1,024 x 1,000 as 48 x 32: rows that do not begin on 128 bytes cost the smaller slabs a fifth, which
-// the choice does not tell apart.
+// 260 9.7 / 6.6, 2,500 x 9,728 x 16 36.4 / 26.9.  Over 1,430 sizes of K 4 to 1,000 the choice takes 0.89 of the time of kernels that
+// exchanged lanes' values in three and four stages, one workgroup a CU (1.03 without it), and 1.026 of the best form's; at worst 1.12 of theirs,
+// 1,396 x 9,728 x 24 as 64 x 128, and 2,500 x 1,024 x 1,000 as 48 x 32: rows that do not begin on 128 bytes cost the smaller slabs a
+// fifth, which the choice does not tell apart.
 enum Direct { NOT_DIRECT, SLAB_16_32, SLAB_32_32, SLAB_48_32, SLAB_64_64, ROWS_64_64, ROWS_32_128, ROWS_64_128, SLAB_48_48, SLAB_48_64 };
 
 Direct direct_plan(int M, int N, int K, long long part_floats) {
