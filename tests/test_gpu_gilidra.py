@@ -505,3 +505,46 @@ def test_prompts_recurrences_in_whole_and_partial_blocks(rule, sizes):
     whole, cut = walk([lengths]), walk([(1, 2), (15, 1), (16, 14), (18, 0)])
     assert torch.equal(whole[0], cut[0]) and torch.equal(whole[1], cut[1])
     assert rel_err(whole[0].cpu().numpy(), want.reshape(tokens, -1)) < 4e-6     # dim terms a sum and 1 / (1 - keep) tokens' roundings
+
+
+@pytest.mark.parametrize("rule", ["delta", "delta_channel", "wkv"])
+@pytest.mark.parametrize("sizes", [(1, 2, 4, 9), (2, 4, 64, 16), (1, 3, 68, 8), (2, 2, 128, 24), (3, 6, 40, 130), (1, 60, 64, 20)])
+def test_prompts_recurrences_give_the_same_bits_from_rows_off_16_bytes(rule, sizes):
+    """Rows in whole pieces of 16 bytes go straight into LDS, 32 lanes a value channel (time mixing in blocks of 32 tokens, or of 16
+    for many workgroups); the same numbers a float further on in memory take the general walk: fresh and continued states, whole
+    blocks, remainders and a single token, every output and the states."""
+    from vipera_rs_amd.ops import kernels
+
+    kv_heads, heads, dim, vdim = sizes
+    vdim = dim if rule == "wkv" else vdim
+    lengths, firsts = (33, 1, 16, 70, 15, 32), (0, 5, 3, 0, 1, 2)
+    gen = torch.Generator("cuda").manual_seed(5)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    tokens, channels = sum(lengths), 2 * kv_heads * dim + heads * vdim
+    meta = (i32(np.cumsum([0, *lengths]).tolist()), i32(firsts), i32([3, 0, 6, 1, 4, 2]))
+    start = rand(8, heads * kernels.recurrent_head_floats(dim, vdim))
+    keep = torch.exp(-torch.exp(rand(tokens, heads, dim) - 2.0))
+    qkv = torch.cat([rand(tokens, channels) * dim ** -0.5, keep.flatten(1)], dim=1)
+    r, k, v, bonus, beta = rand(tokens, heads * dim), rand(tokens, heads * dim), rand(tokens, heads * dim), rand(heads * dim), torch.sigmoid(rand(tokens, heads))
+
+    def off_by(floats, t):
+        room = torch.empty(t.numel() + floats, device="cuda")
+        room[floats:] = t.reshape(-1)
+        return room[floats:].view(t.shape)
+
+    got = []
+    for floats in (0, 1):
+        state, out = start.clone(), torch.full((tokens, heads * vdim), float("nan"), device="cuda")
+        if rule == "wkv":
+            kernels.wkv_rule(*(off_by(floats, t) for t in (r, k, v, keep.flatten(1))), torch.zeros_like(bonus), bonus, state, *meta, dim,
+                             heads, out, len(lengths), decayed=True)
+        elif rule == "delta":
+            kernels.delta_rule(off_by(floats, qkv[:, :channels]), beta, keep[:, :, 0].contiguous(), state, *meta, kv_heads, dim, heads, vdim,
+                               out, len(lengths))
+        else:
+            kernels.delta_rule(off_by(floats, qkv)[:, :channels], beta, None, state, *meta, kv_heads, dim, heads, vdim, out, len(lengths),
+                               channel_decay_col=channels)
+        assert torch.isfinite(out).all()
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

@@ -441,6 +441,13 @@ __device__ __forceinline__ float rows_total(float v) {
 
 __device__ __forceinline__ float wave_total(float v) { return rows_total(row_sum16(v)); }
 
+// row 0 + row 1 to the lanes of both, row 2 + row 3 to theirs.
+__device__ __forceinline__ float pair_total(float v) {
+  const unsigned bits = (unsigned)__float_as_int(v);
+  const auto rows = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+  return __int_as_float((int)rows[0]) + __int_as_float((int)rows[1]);
+}
+
 // How a block gets into LDS: a wave takes whole pieces of sixty-four numbers of one token and one kind (k, q, ...), so
 // that where a piece begins is worked out by the scalar unit and a lane only adds its own number; the sixteen tokens'
 // eight values are 128 threads'.  A fetch only issues loads, the same number in every thread and none inside a
@@ -575,6 +582,243 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
   }
 }
 
+// Sums over the sixteen lanes of a row, of sixteen numbers a lane at once: of two numbers that are summed alike each lane passes
+// one on and keeps the other, so that a level of the tree (row_sum16's: neighbours, pairs, quads, eights) halves the numbers
+// that are left instead of taking all of them through it.  In the end lane j has number j's sum.
+template <int CTRL, int CTRL_ODD = 0>
+__device__ __forceinline__ float row_merge(bool odd, float even_number, float odd_number) {
+  const float kept = odd ? odd_number : even_number;
+  const int sent = __float_as_int(odd ? even_number : odd_number);
+  int moved;
+  if constexpr (CTRL_ODD == 0) {
+    moved = __builtin_amdgcn_update_dpp(0, sent, CTRL, 0xF, 0xF, false);
+  } else {       // lanes of the even quads through one move, of the odd ones through the other
+    moved = __builtin_amdgcn_update_dpp(0, sent, CTRL, 0xF, 0x5, false);
+    moved = __builtin_amdgcn_update_dpp(moved, sent, CTRL_ODD, 0xF, 0xA, false);
+  }
+  return kept + __int_as_float(moved);
+}
+struct RowMerge {
+  bool bit0, bit1, bit2, bit3;
+  __device__ __forceinline__ explicit RowMerge(int lane) : bit0(lane & 1), bit1(lane & 2), bit2(lane & 4), bit3(lane & 8) {}
+  __device__ __forceinline__ float quads(float a, float b, float c, float d) const {     // numbers 4 n .. 4 n + 3
+    return row_merge<0x4E>(bit1, row_merge<0xB1>(bit0, a, b), row_merge<0xB1>(bit0, c, d));
+  }
+  __device__ __forceinline__ float rows(const float (&q)[4]) const {                     // quads() of n = 0 .. 3
+    return row_merge<0x128>(bit3, row_merge<0x104, 0x114>(bit2, q[0], q[1]), row_merge<0x104, 0x114>(bit2, q[2], q[3]));
+  }
+};
+
+// 16 or 4 bytes a lane from memory into LDS, one lane's behind the other's from `to` on; past the view's end zeros.
+struct ScanView {
+  __amdgpu_buffer_rsrc_t rsrc;
+};
+__device__ __forceinline__ ScanView scan_view(const float* base, int bytes) {
+  return ScanView{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00020000)};
+}
+template <bool QUAD>
+__device__ __forceinline__ void scan_load_lds(const ScanView view, float* to, int offset) {
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  if constexpr (QUAD)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(view.rsrc, (lds_ptr)to, 16, offset, 0, 0, 0);
+  else
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(view.rsrc, (lds_ptr)to, 4, offset, 0, 0, 0);
+}
+
+// The delta rule for key widths up to 128 in whole pieces of 16 bytes, with every number formed as above: a value channel
+// has 32 lanes, each with the key channels of two of the 64 lanes above, and adds the two's parts itself where they would have
+// met first.  What bounds the walk is a wave's instructions: one goes out every 1.95 ns on a wave alone on its SIMD and little
+// faster on two, so that a token's step is worth what its instructions take (some 39 here for two value channels, 36 above for
+// one), and what a block costs besides is worth its share of sixteen tokens: here a block goes straight from memory into LDS in
+// pieces of 16 bytes, whose places are worked out once, and LDS reads and the read-out's products stand between the exchanges
+// of the update's sum, which would wait there.  us, above and here: 16 heads of 128 x 128, one entry of 2,048 tokens 287 / 219, of 512 77 / 60,
+// of 1,000 and 834 215 / 155, eight of 250 206 / 136; 8 heads, 2,048 tokens 265 / 209; 6 heads of 64 x 64, 512, 456 and 399 63 / 50; with
+// a decay per key channel, 16 heads 300 / 228.  Tokens of 31 and fewer cost the same either way.
+template <int Q, bool CH>
+__global__ __launch_bounds__(SCAN_COLS * 32) void delta_scan_direct_kernel(
+    const float* __restrict__ qkv, long long ldq, int g_col, const float* __restrict__ beta,
+    const float* __restrict__ decay, float* __restrict__ state, long long state_stride,
+    const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots,
+    int kv_heads, int dim, int heads, int vdim, int key_pad, int value_pad, float* __restrict__ out) {
+  constexpr int DP = 64 * Q, KINDS = CH ? 3 : 2, N = 2 * Q, WAVES = SCAN_COLS / 2;
+  constexpr int PIECES = KINDS * 4 * Q / WAVES, ROWS = 4 / Q;      // a wave's loads of a block (64 pieces of 16 bytes), rows each
+  static_assert(WAVES == 4, "two waves fetch the values, one beta, one the decay");
+  __shared__ __attribute__((aligned(16))) float rows[2][KINDS][REC_BLOCK][DP];
+  __shared__ float values[2][REC_BLOCK][SCAN_COLS];
+  __shared__ float gates[2][2][REC_BLOCK];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = tid >> 5, d0 = (lane & 31) * N;
+  const int v0 = blockIdx.z * SCAN_COLS, v = v0 + col;
+  const bool live = v < vdim;
+  const int kh = h / (heads / kv_heads);
+  const int start = entry_start[e], end = entry_start[e + 1];
+  if (start >= end) return;      // the whole workgroup
+  float* mine = state + (long long)slots[e] * state_stride + ((long long)h * value_pad + v) * key_pad + d0;
+  const bool fresh = entry_first[e] == 0, kept = v < value_pad;
+  float S[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) S[i] = (!fresh && kept && d0 + i < key_pad) ? mine[i] : 0.f;
+  const int row_bytes = (int)ldq * 4;
+  int piece_row[PIECES], piece_at[PIECES], piece_off[PIECES];
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int n = wave * PIECES + i, kind = n / (4 * Q), c = lane % (16 * Q) * 4;
+    piece_row[i] = n % (4 * Q) * ROWS + lane / (16 * Q);
+    piece_at[i] = c < dim ? ((kind == 0 ? kh * dim : kind == 1 ? (kv_heads + kh) * dim : g_col + h * dim) + c) * 4 : -1;
+    piece_off[i] = c < dim ? piece_row[i] * row_bytes + piece_at[i] : -1;
+  }
+  // the wave's single numbers: values (waves 0 and 1, a row's eight side by side), beta (2) and the decay (3)
+  const bool a_value = wave < 2, single = a_value || (lane < REC_BLOCK && !(CH && wave == 3));
+  const float* single_from = a_value ? qkv : wave == 2 ? beta : decay;
+  const int single_row = a_value ? tid >> 3 : lane, single_bytes = a_value ? row_bytes : heads * 4;
+  const int single_at = !a_value ? h * 4 : v0 + (tid & 7) < vdim ? (2 * kv_heads * dim + h * vdim + v0 + (tid & 7)) * 4 : -1;
+  const int single_off = single_at < 0 ? -1 : single_row * single_bytes + single_at;
+  float* const single_to = a_value ? &values[0][0][0] + wave * 64 : &gates[0][0][0] + (wave - 2) * REC_BLOCK;
+  const int single_next = a_value ? REC_BLOCK * SCAN_COLS : 2 * REC_BLOCK;
+  // a row past the entry's end is its last one, which nobody works on; what does not exist (-1) reads zeros
+  auto fetch = [&](int t0, int buf) {
+    const int last = min(REC_BLOCK, end - t0) - 1;
+    const ScanView view = scan_view(qkv + t0 * ldq, (last + 1) * row_bytes);
+    const ScanView single_view = scan_view(single_from + (long long)t0 * (single_bytes / 4), (last + 1) * single_bytes);
+    float* to = &rows[buf][0][0][0] + wave * PIECES * 256;
+    if (last == REC_BLOCK - 1) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) scan_load_lds<true>(view, to + i * 256, piece_off[i]);
+      if (single) scan_load_lds<false>(single_view, single_to + buf * single_next, single_off);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i)
+        scan_load_lds<true>(view, to + i * 256, piece_at[i] < 0 ? -1 : min(piece_row[i], last) * row_bytes + piece_at[i]);
+      if (single)
+        scan_load_lds<false>(single_view, single_to + buf * single_next,
+                             single_at < 0 ? -1 : min(single_row, last) * single_bytes + single_at);
+    }
+  };
+  auto lane_sum = [&](const float (&x)[N], const float (&y)[N]) {
+    float part[2] = {0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int i = 0; i < Q; ++i) part[p] = fmaf(x[p * Q + i], y[p * Q + i], part[p]);
+    return part[0] + part[1];
+  };
+  float outs = 0.f;      // lane j of every row: its row's part of token j's read-out, which nothing waits for
+  auto store = [&](int t0) {
+    const float o = pair_total(outs);
+    const int j = lane & 31;
+    if (live && j < min(REC_BLOCK, end - t0)) out[((long long)(t0 + j) * heads + h) * vdim + v] = o;
+  };
+  fetch(start, 0);
+  for (int t0 = start, buf = 0; t0 < end; t0 += REC_BLOCK, buf ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);     // the wave's loads of this block, asked for a block ago
+    __syncthreads();                        // everybody's; and nobody reads the block before any more
+    if (t0 > start) store(t0 - REC_BLOCK);
+    if (t0 + REC_BLOCK < end) fetch(t0 + REC_BLOCK, buf ^ 1);
+    const int count = min(REC_BLOCK, end - t0);
+    auto read_k = [&](int j, float (&kk)[N]) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) kk[i] = rows[buf][1][j][d0 + i];
+    };
+    auto read_q = [&](int j, float (&qq)[N]) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) qq[i] = rows[buf][0][j][d0 + i];
+    };
+    auto read_gates = [&](int j, float (&gg)[N], float& b) {
+      b = gates[buf][0][j];
+      const float g = CH ? 0.f : gates[buf][1][j];
+#pragma unroll
+      for (int i = 0; i < N; ++i) gg[i] = CH ? rows[buf][KINDS - 1][j][d0 + i] : g;
+    };
+    auto keep_out = [&](int j, float o) { outs = (lane & (REC_BLOCK - 1)) == j ? o : outs; };
+    constexpr int AHEAD = 2, READS = CH ? 5 : 4;      // a token's LDS reads go two tokens before its arithmetic
+    float kk[AHEAD + 1][N], qq[AHEAD + 2][N], gg[AHEAD + 1][N], b[AHEAD + 1], val[AHEAD + 1], part[2];
+    if (count == REC_BLOCK) {
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        read_k(j, kk[j]);
+        read_gates(j, gg[j], b[j]);
+        val[j] = values[buf][j][col];
+        read_q(j, qq[j]);
+      }
+      float o = 0.f, before = 0.f;     // lane sums of the read-outs of the token before and of the one before that
+#define VK_FENCE __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < REC_BLOCK; ++j) {
+        const int now = j % (AHEAD + 1), next = (j + AHEAD) % (AHEAD + 1);
+        const bool more = j + AHEAD < REC_BLOCK;
+        const float(&q)[N] = qq[(j + AHEAD + 1) % (AHEAD + 2)];
+        if (j + 1 < REC_BLOCK) __builtin_amdgcn_s_waitcnt(0xC07F | READS << 8);      // the token's LDS reads
+        else __builtin_amdgcn_s_waitcnt(0xC07F);
+        VK_FENCE
+        float held[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) held[i] = S[i];
+#pragma unroll
+        for (int i = 0; i < N; ++i) S[i] *= gg[now][i];
+        float dot = lane_sum(S, kk[now]);
+        VK_FENCE
+        before = o;
+        if (j > 0) {
+          part[0] = fmaf(held[0], q[0], 0.f);
+          part[1] = fmaf(held[Q], q[Q], 0.f);
+        }
+        VK_FENCE
+        dot = dpp_add<0xB1>(dot);
+        if (j > 1) before = dpp_add<0xB1>(before);
+        if (Q > 1 && j > 0) part[0] = fmaf(held[1], q[1], part[0]);
+        VK_FENCE
+        dot = dpp_add<0x4E>(dot);
+        if (j > 1) before = dpp_add<0x4E>(before);
+        if (Q > 1 && j > 0) part[1] = fmaf(held[Q + 1], q[Q + 1], part[1]);
+        VK_FENCE
+        dot = dpp_add<0x141>(dot);
+        if (j > 1) before = dpp_add<0x141>(before);
+        if (j > 0) o = part[0] + part[1];
+        VK_FENCE
+        dot = dpp_add<0x140>(dot);
+        if (j > 1) before = dpp_add<0x140>(before);
+        if (more) read_k(j + AHEAD, kk[next]);
+        VK_FENCE
+        if (more) {
+          read_gates(j + AHEAD, gg[next], b[next]);
+          val[next] = values[buf][j + AHEAD][col];
+        }
+        const float total = pair_total(dot);
+        if (more) read_q(j + AHEAD, qq[(j + AHEAD) % (AHEAD + 2)]);
+        if (j > 1) keep_out(j - 2, before);
+        VK_FENCE
+        const float u = b[now] * (val[now] - total);
+#pragma unroll
+        for (int i = 0; i < N; ++i) S[i] = fmaf(kk[now][i], u, S[i]);
+        VK_FENCE
+      }
+#undef VK_FENCE
+      const float last = lane_sum(S, qq[(REC_BLOCK - 1) % (AHEAD + 2)]);
+      keep_out(REC_BLOCK - 2, row_sum16(o));
+      keep_out(REC_BLOCK - 1, row_sum16(last));
+    } else {
+      for (int j = 0; j < count; ++j) {
+        read_k(j, kk[0]);
+        read_q(j, qq[0]);
+        read_gates(j, gg[0], b[0]);
+        val[0] = values[buf][j][col];
+#pragma unroll
+        for (int i = 0; i < N; ++i) S[i] *= gg[0][i];
+        const float u = b[0] * (val[0] - pair_total(row_sum16(lane_sum(S, kk[0]))));
+#pragma unroll
+        for (int i = 0; i < N; ++i) S[i] = fmaf(kk[0][i], u, S[i]);
+        keep_out(j, row_sum16(lane_sum(S, qq[0])));
+      }
+    }
+  }
+  store(start + (end - start - 1) / REC_BLOCK * REC_BLOCK);
+  if (kept) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (d0 + i < key_pad) mine[i] = S[i];
+  }
+}
+
 // An LDS row of a token: [r: 64Q | k: 64Q | w: 64Q | v: 8].
 template <int Q>
 __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
@@ -686,6 +930,139 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
   if (kept) {
 #pragma unroll
     for (int i = 0; i < Q; ++i)
+      if (d0 + i < key_pad) mine[i] = S[i];
+  }
+}
+
+// The time mixing for head widths up to 128 in whole pieces of 16 bytes and decays taken beforehand, shaped as
+// delta_scan_direct_kernel is, with every number formed as above: 32 lanes a value channel, some 16 instructions a token for two of
+// them (13 above for one).  Nothing waits for a token's sums over the lanes, so sixteen tokens' go through the tree together.  Blocks
+// of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here (in blocks of 32 /
+// 16): 32 heads of 64, one entry of 2,048 tokens 168 / 112 / 127, of 512 46 / 32 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
+// 512, 456 and 399 (768) 82 / 56 / 59, eight of 250 (2,048) 115 / 84 / 75.
+constexpr int WKV_LONG_BLOCKS = 3 * 256;      // workgroups up to which blocks are of 32 tokens
+template <int Q, int BLOCK>
+__global__ __launch_bounds__(SCAN_COLS * 32) void wkv_scan_direct_kernel(
+    const float* __restrict__ r, long long ldr, const float* __restrict__ k, long long ldk, const float* __restrict__ v,
+    long long ldv, const float* __restrict__ w, long long ldw, const float* __restrict__ bonus, float* __restrict__ state,
+    long long state_stride, const int* __restrict__ entry_start, const int* __restrict__ entry_first,
+    const int* __restrict__ slots, int dim, int heads, int key_pad, int value_pad, float* __restrict__ out) {
+  // rows of a load (64 pieces of 16 bytes) and a wave's loads of a kind
+  constexpr int DP = 64 * Q, N = 2 * Q, ROWS = 4 / Q, LOADS = BLOCK / ROWS / 4;
+  __shared__ __attribute__((aligned(16))) float rows[2][3][BLOCK][DP];
+  __shared__ float values[2][BLOCK][SCAN_COLS];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = tid >> 5, d0 = (lane & 31) * N;
+  const int v0 = blockIdx.z * SCAN_COLS, col_v = v0 + col;
+  const bool live = col_v < dim;
+  const int start = entry_start[e], end = entry_start[e + 1];
+  if (start >= end) return;      // the whole workgroup
+  float* mine = state + (long long)slots[e] * state_stride + ((long long)h * value_pad + col_v) * key_pad + d0;
+  const bool fresh = entry_first[e] == 0, kept = col_v < value_pad;
+  float S[N], U[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    S[i] = (!fresh && kept && d0 + i < key_pad) ? mine[i] : 0.f;
+    U[i] = d0 + i < dim ? bonus[h * dim + d0 + i] : 0.f;
+  }
+  const int first_row = wave * LOADS * ROWS + lane / (16 * Q), piece = lane % (16 * Q) * 4, value = v0 + (tid & 7);
+  const float* const from[3] = {r + h * dim, k + h * dim, w + h * dim};
+  const int row_bytes[3] = {(int)ldr * 4, (int)ldk * 4, (int)ldw * 4};
+  int off[3][LOADS];
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) off[n][i] = piece < dim ? (first_row + i * ROWS) * row_bytes[n] + piece * 4 : -1;
+  const int value_off = value < dim ? ((tid >> 3) * (int)ldv + value) * 4 : -1;
+  // a row past the entry's end is its last one, which nobody works on; what does not exist (-1) reads zeros
+  auto fetch = [&](int t0, int buf) {
+    const int last = min(BLOCK, end - t0) - 1;
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const ScanView view = scan_view(from[n] + (long long)t0 * (row_bytes[n] / 4), last * row_bytes[n] + dim * 4);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        int at = off[n][i];
+        if (last < BLOCK - 1 && piece < dim) at = min(first_row + i * ROWS, last) * row_bytes[n] + piece * 4;
+        scan_load_lds<true>(view, &rows[buf][n][(wave * LOADS + i) * ROWS][0], at);
+      }
+    }
+    if (wave * 8 < BLOCK) {
+      int at = value_off;
+      if (last < BLOCK - 1 && value < dim) at = (min(tid >> 3, last) * (int)ldv + value) * 4;
+      scan_load_lds<false>(scan_view(v + t0 * ldv + h * dim, (last * (int)ldv + dim) * 4), &values[buf][wave * 8][0], at);
+    }
+  };
+  const RowMerge merge(lane);
+  float outs[BLOCK / REC_BLOCK];      // lane j of every row: its row's part of token j's read-out, which nothing waits for
+  auto store = [&](int t0) {
+#pragma unroll
+    for (int half = 0; half < BLOCK / REC_BLOCK; ++half) {
+      const float o = pair_total(outs[half]);
+      const int j = half * REC_BLOCK + (lane & 31);
+      if (live && (lane & 31) < REC_BLOCK && j < end - t0) out[((long long)(t0 + j) * heads + h) * dim + col_v] = o;
+    }
+  };
+  fetch(start, 0);
+  for (int t0 = start, buf = 0; t0 < end; t0 += BLOCK, buf ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);     // the wave's loads of this block, asked for a block ago
+    __syncthreads();                        // everybody's; and nobody reads the block before any more
+    if (t0 > start) store(t0 - BLOCK);
+    if (t0 + BLOCK < end) fetch(t0 + BLOCK, buf ^ 1);
+    const int count = min(BLOCK, end - t0);
+    constexpr int AHEAD = Q == 1 ? 4 : 2;      // tokens read from LDS before the arithmetic of the AHEAD before them
+    float rr[2][AHEAD][N], kk[2][AHEAD][N], ww[2][AHEAD][N], val[2][AHEAD];
+    auto read = [&](int j, int of, int n) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        rr[of][n][i] = rows[buf][0][j][d0 + i];
+        kk[of][n][i] = rows[buf][1][j][d0 + i];
+        ww[of][n][i] = rows[buf][2][j][d0 + i];
+      }
+      val[of][n] = values[buf][j][col];
+    };
+    auto token = [&](int of, int n) {
+      float part[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float kv = kk[of][n][i] * val[of][n];
+        part[i / Q] = fmaf(fmaf(U[i], kv, S[i]), rr[of][n][i], part[i / Q]);
+        S[i] = fmaf(ww[of][n][i], S[i], kv);
+      }
+      return part[0] + part[1];
+    };
+    if (count == BLOCK) {
+#pragma unroll
+      for (int n = 0; n < AHEAD; ++n) read(n, 0, n);
+      float o[4], quads[4];
+#pragma unroll
+      for (int j = 0; j < BLOCK; j += AHEAD) {
+        const int of = j / AHEAD & 1;
+        if (j + AHEAD < BLOCK) {
+#pragma unroll
+          for (int n = 0; n < AHEAD; ++n) read(j + AHEAD + n, of ^ 1, n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) o[(j + n) % 4] = token(of, n);
+        if ((j + AHEAD) % 4 == 0) quads[j / 4 % 4] = merge.quads(o[0], o[1], o[2], o[3]);
+        if ((j + AHEAD) % REC_BLOCK == 0) outs[j / REC_BLOCK] = merge.rows(quads);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int j = 0; j < count; ++j) {
+        read(j, 0, 0);
+        const float o = row_sum16(token(0, 0));
+#pragma unroll
+        for (int half = 0; half < BLOCK / REC_BLOCK; ++half)
+          outs[half] = (lane & (REC_BLOCK - 1)) + half * REC_BLOCK == j ? o : outs[half];
+      }
+    }
+  }
+  store(start + (end - start - 1) / BLOCK * BLOCK);
+  if (kept) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
       if (d0 + i < key_pad) mine[i] = S[i];
   }
 }
@@ -1209,10 +1586,19 @@ extern "C" int vk_delta_rule_strided(const float* qkv, long long ldq, int g_col,
   delta_scan_kernel<Q, CH><<<scan_grid, SCAN_THREADS, 0, s>>>(qkv, ldq, g_col, beta, decay, state, state_stride,       \
                                                               entry_start, entry_first, slots, kv_heads, dim, heads,  \
                                                               vdim, key_pad, value_pad, out)
-    if (key_pad <= 64) { if (ch) VK_DELTA_SCAN(1, true); else VK_DELTA_SCAN(1, false); }
+#define VK_DELTA_DIRECT(Q, CH)                                                                                       \
+  delta_scan_direct_kernel<Q, CH><<<scan_grid, SCAN_COLS * 32, 0, s>>>(qkv, ldq, g_col, beta, decay, state,            \
+                                                                       state_stride, entry_start, entry_first, slots, \
+                                                                       kv_heads, dim, heads, vdim, key_pad, value_pad, out)
+    if (key_pad <= 128 && dim % 4 == 0 && ldq % 4 == 0 && ((uintptr_t)qkv & 15) == 0 && (!ch || g_col % 4 == 0)) {
+      if (key_pad <= 64) { if (ch) VK_DELTA_DIRECT(1, true); else VK_DELTA_DIRECT(1, false); }
+      else { if (ch) VK_DELTA_DIRECT(2, true); else VK_DELTA_DIRECT(2, false); }
+    }
+    else if (key_pad <= 64) { if (ch) VK_DELTA_SCAN(1, true); else VK_DELTA_SCAN(1, false); }
     else if (key_pad <= 128) { if (ch) VK_DELTA_SCAN(2, true); else VK_DELTA_SCAN(2, false); }
     else { if (ch) VK_DELTA_SCAN(4, true); else VK_DELTA_SCAN(4, false); }
 #undef VK_DELTA_SCAN
+#undef VK_DELTA_DIRECT
     VK_LAUNCH_CHECK();
     return 0;
   }
@@ -1313,10 +1699,21 @@ extern "C" int vk_wkv_rule(const float* r, long long ldr, const float* k, long l
   wkv_scan_kernel<Q><<<scan_grid, SCAN_THREADS, 0, s>>>(r, ldr, k, ldk, v, ldv, wraw, ldw, w0, bonus, state,          \
                                                         state_stride, entry_start, entry_first, slots, dim, heads,    \
                                                         key_pad, value_pad, decayed, out)
-    if (key_pad <= 64) VK_WKV_SCAN(1);
+#define VK_WKV_DIRECT(Q, BLOCK)                                                                                      \
+  wkv_scan_direct_kernel<Q, BLOCK><<<scan_grid, SCAN_COLS * 32, 0, s>>>(r, ldr, k, ldk, v, ldv, wraw, ldw, bonus,      \
+                                                                        state, state_stride, entry_start, entry_first, \
+                                                                        slots, dim, heads, key_pad, value_pad, out)
+    const bool pieces = dim % 4 == 0 && (ldr | ldk | ldw) % 4 == 0 && (((uintptr_t)r | (uintptr_t)k | (uintptr_t)wraw) & 15) == 0 &&
+                        std::max(std::max(ldr, ldk), std::max(ldv, ldw)) < (1 << 24);
+    const long long groups = (long long)num_entries * heads * (value_pad / SCAN_COLS);
+    if (decayed && pieces && key_pad <= 64 && groups <= WKV_LONG_BLOCKS) VK_WKV_DIRECT(1, 2 * REC_BLOCK);
+    else if (decayed && pieces && key_pad <= 64) VK_WKV_DIRECT(1, REC_BLOCK);
+    else if (decayed && pieces && key_pad <= 128) VK_WKV_DIRECT(2, REC_BLOCK);
+    else if (key_pad <= 64) VK_WKV_SCAN(1);
     else if (key_pad <= 128) VK_WKV_SCAN(2);
     else VK_WKV_SCAN(4);
 #undef VK_WKV_SCAN
+#undef VK_WKV_DIRECT
     VK_LAUNCH_CHECK();
     return 0;
   }
