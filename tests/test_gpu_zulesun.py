@@ -234,6 +234,12 @@ def test_prompts_portions_walk_to_the_same_bits(sizes):
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), f"{extra} more columns"
 
 
+@pytest.mark.parametrize("sizes", [(2, 64, 8), (1, 128, 4), (3, 128, 20), (5, 64, 36)])
+def test_prompts_portions_of_whole_pieces_walk_to_the_same_bits(sizes):
+    """64 and 128 key channels in rows of whole 16 bytes, which go straight into LDS (rows of one column more do not)."""
+    test_prompts_portions_walk_to_the_same_bits(sizes)
+
+
 @pytest.mark.parametrize("sizes", [(18, 5), (40, 16), (7, 33), (33, 20), (16, 64), (20, 65)])
 def test_a_prepared_selective_scan_walks_to_the_same_bits(sizes):
     """Steps and gates taken beforehand (the walk in blocks of tokens, up to 64 states) against those taken inside (token

@@ -8,6 +8,7 @@
 // The recurrence kernels keep a head's state matrix in registers, a column of it spread over four lanes, and walk an
 // entry's tokens in order; a sum over the key channels has one fixed order, whatever else is in the launch.
 #include "common.h"
+#include "scan_parts.h"
 
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -582,49 +583,6 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
   }
 }
 
-// Sums over the sixteen lanes of a row, of sixteen numbers a lane at once: of two numbers that are summed alike each lane passes
-// one on and keeps the other, so that a level of the tree (row_sum16's: neighbours, pairs, quads, eights) halves the numbers
-// that are left instead of taking all of them through it.  In the end lane j has number j's sum.
-template <int CTRL, int CTRL_ODD = 0>
-__device__ __forceinline__ float row_merge(bool odd, float even_number, float odd_number) {
-  const float kept = odd ? odd_number : even_number;
-  const int sent = __float_as_int(odd ? even_number : odd_number);
-  int moved;
-  if constexpr (CTRL_ODD == 0) {
-    moved = __builtin_amdgcn_update_dpp(0, sent, CTRL, 0xF, 0xF, false);
-  } else {       // lanes of the even quads through one move, of the odd ones through the other
-    moved = __builtin_amdgcn_update_dpp(0, sent, CTRL, 0xF, 0x5, false);
-    moved = __builtin_amdgcn_update_dpp(moved, sent, CTRL_ODD, 0xF, 0xA, false);
-  }
-  return kept + __int_as_float(moved);
-}
-struct RowMerge {
-  bool bit0, bit1, bit2, bit3;
-  __device__ __forceinline__ explicit RowMerge(int lane) : bit0(lane & 1), bit1(lane & 2), bit2(lane & 4), bit3(lane & 8) {}
-  __device__ __forceinline__ float quads(float a, float b, float c, float d) const {     // numbers 4 n .. 4 n + 3
-    return row_merge<0x4E>(bit1, row_merge<0xB1>(bit0, a, b), row_merge<0xB1>(bit0, c, d));
-  }
-  __device__ __forceinline__ float rows(const float (&q)[4]) const {                     // quads() of n = 0 .. 3
-    return row_merge<0x128>(bit3, row_merge<0x104, 0x114>(bit2, q[0], q[1]), row_merge<0x104, 0x114>(bit2, q[2], q[3]));
-  }
-};
-
-// 16 or 4 bytes a lane from memory into LDS, one lane's behind the other's from `to` on; past the view's end zeros.
-struct ScanView {
-  __amdgpu_buffer_rsrc_t rsrc;
-};
-__device__ __forceinline__ ScanView scan_view(const float* base, int bytes) {
-  return ScanView{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00020000)};
-}
-template <bool QUAD>
-__device__ __forceinline__ void scan_load_lds(const ScanView view, float* to, int offset) {
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  if constexpr (QUAD)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(view.rsrc, (lds_ptr)to, 16, offset, 0, 0, 0);
-  else
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(view.rsrc, (lds_ptr)to, 4, offset, 0, 0, 0);
-}
-
 // The delta rule for key widths up to 128 in whole pieces of 16 bytes, with every number formed as above: a value channel
 // has 32 lanes, each with the key channels of two of the 64 lanes above, and adds the two's parts itself where they would have
 // met first.  What bounds the walk is a wave's instructions: one goes out every 1.95 ns on a wave alone on its SIMD and little
@@ -676,16 +634,16 @@ __global__ __launch_bounds__(SCAN_COLS * 32) void delta_scan_direct_kernel(
   float* const single_to = a_value ? &values[0][0][0] + wave * 64 : &gates[0][0][0] + (wave - 2) * REC_BLOCK;
   const int single_next = a_value ? REC_BLOCK * SCAN_COLS : 2 * REC_BLOCK;
   // a row past the entry's end is its last one, which nobody works on; what does not exist (-1) reads zeros
+  const float *next_row = qkv + start * ldq, *next_single = single_from + (long long)start * (single_bytes / 4);     // of the block fetched next
   auto fetch = [&](int t0, int buf) {
-    const int last = min(REC_BLOCK, end - t0) - 1;
-    const ScanView view = scan_view(qkv + t0 * ldq, (last + 1) * row_bytes);
-    const ScanView single_view = scan_view(single_from + (long long)t0 * (single_bytes / 4), (last + 1) * single_bytes);
+    const ScanView view = scan_view(next_row, 0x7fffffff), single_view = scan_view(next_single, 0x7fffffff);
     float* to = &rows[buf][0][0][0] + wave * PIECES * 256;
-    if (last == REC_BLOCK - 1) {
+    if (t0 + REC_BLOCK <= end) {
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) scan_load_lds<true>(view, to + i * 256, piece_off[i]);
       if (single) scan_load_lds<false>(single_view, single_to + buf * single_next, single_off);
     } else {
+      const int last = end - 1 - t0;
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
         scan_load_lds<true>(view, to + i * 256, piece_at[i] < 0 ? -1 : min(piece_row[i], last) * row_bytes + piece_at[i]);
@@ -693,6 +651,8 @@ __global__ __launch_bounds__(SCAN_COLS * 32) void delta_scan_direct_kernel(
         scan_load_lds<false>(single_view, single_to + buf * single_next,
                              single_at < 0 ? -1 : min(single_row, last) * single_bytes + single_at);
     }
+    next_row += REC_BLOCK * ldq;
+    next_single += REC_BLOCK * (long long)(single_bytes / 4);
   };
   auto lane_sum = [&](const float (&x)[N], const float (&y)[N]) {
     float part[2] = {0.f, 0.f};
@@ -938,8 +898,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
 // delta_scan_direct_kernel is, with every number formed as above: 32 lanes a value channel, some 16 instructions a token for two of
 // them (13 above for one).  Nothing waits for a token's sums over the lanes, so sixteen tokens' go through the tree together.  Blocks
 // of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here (in blocks of 32 /
-// 16): 32 heads of 64, one entry of 2,048 tokens 168 / 112 / 127, of 512 46 / 32 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
-// 512, 456 and 399 (768) 82 / 56 / 59, eight of 250 (2,048) 115 / 84 / 75.
+// 16): 32 heads of 64, one entry of 2,048 tokens 168 / 108 / 127, of 512 46 / 31 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
+// 512, 456 and 399 (768) 82 / 55 / 59, eight of 250 (2,048) 115 / 84 / 75.
 constexpr int WKV_LONG_BLOCKS = 3 * 256;      // workgroups up to which blocks are of 32 tokens
 template <int Q, int BLOCK>
 __global__ __launch_bounds__(SCAN_COLS * 32) void wkv_scan_direct_kernel(
@@ -966,32 +926,39 @@ __global__ __launch_bounds__(SCAN_COLS * 32) void wkv_scan_direct_kernel(
     U[i] = d0 + i < dim ? bonus[h * dim + d0 + i] : 0.f;
   }
   const int first_row = wave * LOADS * ROWS + lane / (16 * Q), piece = lane % (16 * Q) * 4, value = v0 + (tid & 7);
-  const float* const from[3] = {r + h * dim, k + h * dim, w + h * dim};
-  const int row_bytes[3] = {(int)ldr * 4, (int)ldk * 4, (int)ldw * 4};
+  const float* next[3] = {r + start * ldr + h * dim, k + start * ldk + h * dim, w + start * ldw + h * dim};     // of the block fetched next
+  const float* next_value = v + start * ldv + h * dim;
+  const long long ld[3] = {ldr, ldk, ldw};
   int off[3][LOADS];
 #pragma unroll
   for (int n = 0; n < 3; ++n)
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) off[n][i] = piece < dim ? (first_row + i * ROWS) * row_bytes[n] + piece * 4 : -1;
+    for (int i = 0; i < LOADS; ++i) off[n][i] = piece < dim ? ((first_row + i * ROWS) * (int)ld[n] + piece) * 4 : -1;
   const int value_off = value < dim ? ((tid >> 3) * (int)ldv + value) * 4 : -1;
   // a row past the entry's end is its last one, which nobody works on; what does not exist (-1) reads zeros
   auto fetch = [&](int t0, int buf) {
-    const int last = min(BLOCK, end - t0) - 1;
+    const int last = end - 1 - t0;
+    if (last >= BLOCK - 1) {
 #pragma unroll
-    for (int n = 0; n < 3; ++n) {
-      const ScanView view = scan_view(from[n] + (long long)t0 * (row_bytes[n] / 4), last * row_bytes[n] + dim * 4);
+      for (int n = 0; n < 3; ++n)
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) {
-        int at = off[n][i];
-        if (last < BLOCK - 1 && piece < dim) at = min(first_row + i * ROWS, last) * row_bytes[n] + piece * 4;
-        scan_load_lds<true>(view, &rows[buf][n][(wave * LOADS + i) * ROWS][0], at);
-      }
+        for (int i = 0; i < LOADS; ++i)
+          scan_load_lds<true>(scan_view(next[n], 0x7fffffff), &rows[buf][n][(wave * LOADS + i) * ROWS][0], off[n][i]);
+      if (wave * 8 < BLOCK) scan_load_lds<false>(scan_view(next_value, 0x7fffffff), &values[buf][wave * 8][0], value_off);
+    } else {
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+          scan_load_lds<true>(scan_view(next[n], 0x7fffffff), &rows[buf][n][(wave * LOADS + i) * ROWS][0],
+                              piece < dim ? (min(first_row + i * ROWS, last) * (int)ld[n] + piece) * 4 : -1);
+      if (wave * 8 < BLOCK)
+        scan_load_lds<false>(scan_view(next_value, 0x7fffffff), &values[buf][wave * 8][0],
+                             value < dim ? (min(tid >> 3, last) * (int)ldv + value) * 4 : -1);
     }
-    if (wave * 8 < BLOCK) {
-      int at = value_off;
-      if (last < BLOCK - 1 && value < dim) at = (min(tid >> 3, last) * (int)ldv + value) * 4;
-      scan_load_lds<false>(scan_view(v + t0 * ldv + h * dim, (last * (int)ldv + dim) * 4), &values[buf][wave * 8][0], at);
-    }
+#pragma unroll
+    for (int n = 0; n < 3; ++n) next[n] += BLOCK * ld[n];
+    next_value += BLOCK * ldv;
   };
   const RowMerge merge(lane);
   float outs[BLOCK / REC_BLOCK];      // lane j of every row: its row's part of token j's read-out, which nothing waits for

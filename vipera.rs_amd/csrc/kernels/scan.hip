@@ -16,6 +16,7 @@
 // by a kernel ahead, for a prompt's portion, where every wave would pay for it token behind token.
 #include "common.h"
 #include "conv_state.h"
+#include "scan_parts.h"
 
 __device__ __forceinline__ float scan_silu(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float scan_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -288,6 +289,153 @@ __global__ __launch_bounds__(RUN_THREADS) void decay_run_kernel(const float* __r
   }
 }
 
+// The same for 64 or 128 key channels in rows of whole 16 bytes, with every number formed as above: a block goes straight from memory
+// into LDS, in the order in which the lanes read it, from places that are worked out once; two tokens' products, states and sums are
+// three runs of instructions none of which waits for the one before it; and sixteen tokens' sums go through the lanes together.
+// What bounds it is a token's instructions (32 for 8 key channels a lane, of which one goes out every 1.95 ns on a wave alone on
+// its SIMD) and a block's branches and barrier.  us, above and here: 16 heads of 128 x 128, one entry of 2,048 tokens 219 / 182, of 512 59 /
+// 50, of 1,000 and 834 150 / 113, of 512, 456 and 399 82 / 63, eight of 250 104 / 86; 31 tokens cost the same either way.
+template <int R>
+__global__ __launch_bounds__(RUN_THREADS) void decay_run_direct_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, long long ldqk, const float* __restrict__ v, long long ldv,
+    const float* __restrict__ decay, float* __restrict__ state, long long state_stride, const int* __restrict__ entry_start,
+    const int* __restrict__ entry_first, const int* __restrict__ slots, int heads, int vdim, float* __restrict__ o) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int KEYS = 16 * R, BLOCK = 16, QUADS = KEYS / 4;      // QUADS: 16-byte pieces of a row
+  constexpr int ROWS = 64 / QUADS, LOADS = BLOCK / ROWS / RUN_WAVES;     // rows a load, a wave's loads of a block's keys
+  __shared__ __attribute__((aligned(16))) float kq[2][2][BLOCK][KEYS];
+  __shared__ float vals[2][BLOCK][RUN_COLS];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, part = lane & 15;
+  const int v0 = blockIdx.z * RUN_COLS, mine = (tid >> 6) * 4 + (lane >> 4), vch = v0 + mine;
+  const bool live = vch < vdim;
+  const int vcol = h * vdim + min(vch, vdim - 1);
+  const int t0 = entry_start[e], t1 = entry_start[e + 1];
+  if (t1 <= t0) return;       // the whole workgroup
+  const bool fresh = entry_first[e] == 0;
+  const float rate = decay[h];
+  float* row = state + (long long)slots[e] * state_stride + ((long long)h * vdim + min(vch, vdim - 1)) * KEYS + part * R;
+  float s[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const float old = row[r];
+    s[r] = fresh ? 0.f : old;
+  }
+  // in LDS a row's pieces stand as the sixteen lanes' first, then their second ones, so that these read them without bank conflicts
+  const int slot = lane % QUADS, piece = slot % 16 * (R / 4) + slot / 16, first_row = wave * LOADS * ROWS + lane / QUADS;
+  const int row_bytes = (int)ldqk * 4, value_bytes = (int)ldv * 4;
+  const int piece_at = (h * KEYS + piece * 4) * 4, value_at = (h * vdim + min(v0 + tid % RUN_COLS, vdim - 1)) * 4;
+  int off[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) off[i] = (first_row + i * ROWS) * row_bytes + piece_at;
+  const int value_off = tid / RUN_COLS * value_bytes + value_at;
+  // where the block that is fetched next begins; a row past the entry's end is its last one, which nobody works on
+  const float *next_k = k + t0 * ldqk, *next_q = q + t0 * ldqk, *next_v = v + t0 * ldv;
+  auto fetch = [&](int first, int buf) {
+    const ScanView keys = scan_view(next_k, 0x7fffffff), queries = scan_view(next_q, 0x7fffffff), values = scan_view(next_v, 0x7fffffff);
+    float *to_k = &kq[buf][0][wave * LOADS * ROWS][0], *to_q = &kq[buf][1][wave * LOADS * ROWS][0], *to_v = &vals[buf][wave * 64 / RUN_COLS][0];
+    if (first + BLOCK <= t1) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        scan_load_lds<true>(keys, to_k + i * 256, off[i]);
+        scan_load_lds<true>(queries, to_q + i * 256, off[i]);
+      }
+      scan_load_lds<false>(values, to_v, value_off);
+    } else {
+      const int last = t1 - 1 - first;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int at = min(first_row + i * ROWS, last) * row_bytes + piece_at;
+        scan_load_lds<true>(keys, to_k + i * 256, at);
+        scan_load_lds<true>(queries, to_q + i * 256, at);
+      }
+      scan_load_lds<false>(values, to_v, min(tid / RUN_COLS, last) * value_bytes + value_at);
+    }
+    next_k += BLOCK * ldqk;
+    next_q += BLOCK * ldqk;
+    next_v += BLOCK * ldv;
+  };
+  const RowMerge merge(lane);
+  float sums = 0.f;    // lane j of a channel's sixteen: token j's sum
+  float* to = o + (long long)(t0 + part) * heads * vdim + vcol;
+  auto store = [&](int first) {
+    if (live && part < t1 - first) *to = sums;
+    to += (long long)BLOCK * heads * vdim;
+  };
+  fetch(t0, 0);
+  for (int tb = t0, buf = 0; tb < t1; tb += BLOCK, buf ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);     // the wave's loads of this block, asked for a block ago
+    __syncthreads();                        // everybody's; and nobody reads the block before any more
+    if (tb > t0) store(tb - BLOCK);
+    if (tb + BLOCK < t1) fetch(tb + BLOCK, buf ^ 1);
+    auto token = [&](const float (&kj)[R], const float (&qj)[R], float value) {
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        s[r] = fmaf(rate, s[r], kj[r] * value);
+        sum = fmaf(s[r], qj[r], sum);
+      }
+      return sum;
+    };
+    auto read = [&](int j, float (&kj)[R], float (&qj)[R], float& value) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        kj[r] = kq[buf][0][j][r / 4 * 64 + part * 4 + r % 4];
+        qj[r] = kq[buf][1][j][r / 4 * 64 + part * 4 + r % 4];
+      }
+      value = vals[buf][j][mine];
+    };
+    const int count = min(BLOCK, t1 - tb);
+    if (count == BLOCK) {
+      float kp[2][2][R], qp[2][2][R], vp[2][2], sum[4], quads[4];     // two tokens at a time, the next two's reads before them
+      read(0, kp[0][0], qp[0][0], vp[0][0]);
+      read(1, kp[0][1], qp[0][1], vp[0][1]);
+#pragma unroll
+      for (int j = 0; j < BLOCK; j += 2) {
+        const int now = j / 2 & 1;
+        if (j + 2 < BLOCK) {
+          read(j + 2, kp[now ^ 1][0], qp[now ^ 1][0], vp[now ^ 1][0]);
+          read(j + 3, kp[now ^ 1][1], qp[now ^ 1][1], vp[now ^ 1][1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float first[R], chain[2] = {0.f, 0.f};      // the state after the first of the two tokens; their sums, in turn
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < R; ++r) kp[now][n][r] *= vp[now][n];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) first[r] = fmaf(rate, s[r], kp[now][0][r]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r] = fmaf(rate, first[r], kp[now][1][r]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          chain[0] = fmaf(first[r], qp[now][0][r], chain[0]);
+          chain[1] = fmaf(s[r], qp[now][1][r], chain[1]);
+        }
+        sum[j % 4] = chain[0];
+        sum[j % 4 + 1] = chain[1];
+        if (j % 4 == 2) quads[j / 4] = merge.quads(sum[0], sum[1], sum[2], sum[3]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      sums = merge.rows(quads);
+    } else {
+      for (int j = 0; j < count; ++j) {
+        float kj[R], qj[R], value;
+        read(j, kj, qj, value);
+        const float sum = row16_sum(token(kj, qj, value));
+        sums = part == j ? sum : sums;
+      }
+    }
+  }
+  store(t0 + (t1 - t0 - 1) / BLOCK * BLOCK);
+  if (live) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) row[r] = s[r];
+  }
+}
+
 extern "C" long long vk_decay_rule_head_floats(int dim, int vdim) { return (long long)vdim * 16 * lanes_share(dim); }
 
 static int launch_decay_rule(const float* q, const float* k, long long ldqk, const float* v, long long ldv, int act,
@@ -312,15 +460,20 @@ static int launch_decay_rule(const float* q, const float* k, long long ldqk, con
   if (quads) VK_RUN_AS(RR, true, true);         \
   else if (dim == 16 * RR) VK_RUN_AS(RR, true, false); \
   else VK_RUN_AS(RR, false, false)
+#define VK_RUN_DIRECT(RR)                                                                                                     \
+  decay_run_direct_kernel<RR><<<run_grid, RUN_THREADS, 0, s>>>(q, k, ldqk, v, ldv, decay, state, state_stride, entry_start,     \
+                                                               entry_first, slots, heads, vdim, o)
+    const bool direct = quads && ldqk < (1 << 24) && ldv < (1 << 24);
     switch (share) {
       case 1: VK_RUN(1); break;
       case 2: VK_RUN(2); break;
-      case 4: VK_RUN(4); break;
-      case 8: VK_RUN(8); break;
+      case 4: if (direct) VK_RUN_DIRECT(4); else VK_RUN(4); break;
+      case 8: if (direct) VK_RUN_DIRECT(8); else VK_RUN(8); break;
       default: VK_RUN(16); break;
     }
 #undef VK_RUN
 #undef VK_RUN_AS
+#undef VK_RUN_DIRECT
     VK_LAUNCH_CHECK();
     return 0;
   }
@@ -672,15 +825,14 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 }
 
 // The same for prompts' portions (`prepared`) and up to 64 states, with every token's sum and state formed exactly as above.  A
-// workgroup of four waves (sixteen channels) takes the tokens in blocks of sixteen through two LDS stages, where a state's (a
-// channel's) numbers of neighbouring tokens lie side by side, so that a lane reads four tokens' at once; a block's numbers are on
-// their way into registers while the block before is worked on.  A whole block is unrolled without a branch: the exponentials,
+// workgroup of four waves (sixteen channels) takes the tokens in blocks (of 32 for a state a lane, else of 16) through two LDS stages, where a
+// state's (a channel's) numbers of neighbouring tokens lie side by side, so that a lane reads four tokens' at once; a block's numbers
+// are on their way into registers while the block before is worked on.  A whole block is unrolled without a branch: the exponentials,
 // products and exchanges of neighbouring tokens, which wait for nothing but the state's one FMA a token, fill each other's
-// latencies.  Lane j of a channel's sixteen keeps token j's sum and finishes that token's output, so that a block's gate, skip and
-// store are one instruction each.  Now the vector instructions of a token bound it (about 25 and an exponential for a state a
-// lane); above it was their latencies, one behind the other on a wave a SIMD.  ALL: N = 16 R.  4,096 channels of 16 states,
-// against that walk: portions of 1,000 and 834 tokens 278 -> 118 us, one of 2,048 473 -> 172 us, of 512 120 -> 45 us.  Beyond
-// 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
+// latencies, and sixteen tokens' sums go through the lanes together.  Lane j of a channel's sixteen ends up with token j's sum and
+// finishes that token's output.  What bounds it is the instructions (about 23 a token for a state a lane, fourteen of them the
+// exponential).  ALL: N = 16 R.  4,096 channels of 16 states, with blocks of 16 and every token's sum by itself, and so: portions of
+// 1,000 and 834 tokens 120 -> 111 us, one of 2,048 178 -> 159, of 512 50 -> 44, eight of 250 101 -> 93.  Beyond 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
 template <int R, bool ALL, typename TO>
 __global__ __launch_bounds__(256) void selective_run_kernel(
     const float* __restrict__ x, const float* __restrict__ dt, long long lddt, const float* __restrict__ bmat,
@@ -689,7 +841,8 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
     const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots, int C, int N,
     TO* __restrict__ out) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int BLOCK = 16, ROW = BLOCK + 4, STATES = 16 * R;
+  constexpr int HALVES = R == 1 ? 2 : 1, BLOCK = 16 * HALVES, ROW = BLOCK + 4, STATES = 16 * R;
+  constexpr int BC_TOKENS = 256 / STATES, BC_LOADS = BLOCK / BC_TOKENS;
   __shared__ __attribute__((aligned(16))) float bc[2][2][STATES][ROW];     // B and C: [state][token]
   __shared__ __attribute__((aligned(16))) float xdz[2][3][16][ROW];        // x, dt and the gate: [channel][token]
   const int e = blockIdx.x, tid = threadIdx.x;
@@ -711,34 +864,45 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
     a[r] = -expf(a_log[(long long)ch * N + (ALL ? n : min(n, N - 1))]);
   }
   const float d = skip[ch];
-  // this thread's numbers of a block: state tid % STATES of tokens tid / STATES + i (256 / STATES), channel tid % 16 of token
-  // tid / 16; a token past the end is the last one again
+  // this thread's numbers of a block: state tid % STATES of tokens tid / STATES + i (256 / STATES), channel tid % 16 of tokens
+  // tid / 16 + 16 i; a token past the end is the last one again
   const int state_of = tid % STATES, bc_token = tid / STATES, ch_token = tid / 16;
   const int bc_col = ALL ? state_of : min(state_of, N - 1);
   const long long ch_col = min((int)blockIdx.y * 16 + tid % 16, C - 1);
-  float held_b[R], held_c[R], held_x, held_dt, held_z;
+  float held_b[BC_LOADS], held_c[BC_LOADS], held_x[HALVES], held_dt[HALVES], held_z[HALVES];
   auto fetch = [&](int first) {
+    const bool whole = first + BLOCK <= t1;
+    const float *bs = bmat + first * ldbc + bc_col, *cs = cmat + first * ldbc + bc_col;
+    const float *xs = x + (long long)first * C + ch_col, *dts = dt + first * lddt + ch_col, *zs = z + first * ldz + ch_col;
+    const int last = t1 - 1 - first;
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const long long at = (long long)min(first + bc_token + i * (256 / STATES), t1 - 1) * ldbc + bc_col;
-      held_b[i] = bmat[at];
-      held_c[i] = cmat[at];
+    for (int i = 0; i < BC_LOADS; ++i) {
+      const int j = bc_token + i * BC_TOKENS, at = (whole ? j : min(j, last)) * (int)ldbc;
+      held_b[i] = bs[at];
+      held_c[i] = cs[at];
     }
-    const long long t = min(first + ch_token, t1 - 1);
-    held_x = x[t * C + ch_col];
-    held_dt = dt[t * lddt + ch_col];
-    held_z = z[t * ldz + ch_col];
+#pragma unroll
+    for (int i = 0; i < HALVES; ++i) {
+      const int j = ch_token + i * 16, at = whole ? j : min(j, last);
+      held_x[i] = xs[at * C];
+      held_dt[i] = dts[at * (int)lddt];
+      held_z[i] = zs[at * (int)ldz];
+    }
   };
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-      bc[buf][0][state_of][bc_token + i * (256 / STATES)] = held_b[i];
-      bc[buf][1][state_of][bc_token + i * (256 / STATES)] = held_c[i];
+    for (int i = 0; i < BC_LOADS; ++i) {
+      bc[buf][0][state_of][bc_token + i * BC_TOKENS] = held_b[i];
+      bc[buf][1][state_of][bc_token + i * BC_TOKENS] = held_c[i];
     }
-    xdz[buf][0][tid % 16][ch_token] = held_x;
-    xdz[buf][1][tid % 16][ch_token] = held_dt;
-    xdz[buf][2][tid % 16][ch_token] = held_z;
+#pragma unroll
+    for (int i = 0; i < HALVES; ++i) {
+      xdz[buf][0][tid % 16][ch_token + i * 16] = held_x[i];
+      xdz[buf][1][tid % 16][ch_token + i * 16] = held_dt[i];
+      xdz[buf][2][tid % 16][ch_token + i * 16] = held_z[i];
+    }
   };
+  const RowMerge merge(lane);
   fetch(t0);
   stage(0);
   __syncthreads();
@@ -746,9 +910,10 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
   for (int tb = t0; tb < t1; tb += BLOCK, buf ^= 1) {
     const bool more = tb + BLOCK < t1;
     if (more) fetch(tb + BLOCK);
-    float sums = 0.f;
+    float sums[HALVES] = {};
     const int count = min(BLOCK, t1 - tb);
     if (count == BLOCK) {
+      float quads[4];
       f32x4 x4[2], dt4[2], b4[2][R], c4[2][R];     // four tokens at a time, the next four's reads before them
       auto read = [&](int j4, int to) {
         x4[to] = *(const f32x4*)&xdz[buf][0][mine][j4];
@@ -786,10 +951,8 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[j] = row16_sum(sum[j]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sums = part == j4 + j ? sum[j] : sums;
+        quads[j4 / 4 % 4] = merge.quads(sum[0], sum[1], sum[2], sum[3]);
+        if (j4 % 16 == 12) sums[j4 / 16] = merge.rows(quads);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
@@ -802,11 +965,16 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
           sum = fmaf(s[r], in[r] ? bc[buf][1][part * R + r][j] : 0.f, sum);
         }
         sum = row16_sum(sum);
-        sums = part == j ? sum : sums;
+#pragma unroll
+        for (int half = 0; half < HALVES; ++half) sums[half] = part + half * 16 == j ? sum : sums[half];
       }
     }
-    if (live && part < count)
-      out[(long long)(tb + part) * C + ch] = from_float<TO>(fmaf(d, xdz[buf][0][mine][part], sums) * xdz[buf][2][mine][part]);
+#pragma unroll
+    for (int half = 0; half < HALVES; ++half) {
+      const int j = part + half * 16;
+      if (live && j < count)
+        out[(long long)(tb + j) * C + ch] = from_float<TO>(fmaf(d, xdz[buf][0][mine][j], sums[half]) * xdz[buf][2][mine][j]);
+    }
     if (more) stage(buf ^ 1);
     __syncthreads();
   }
@@ -904,12 +1072,14 @@ extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long l
   if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
   hipStream_t s = (hipStream_t)stream;
   const dim3 run_grid(num_entries, (C + 15) / 16);
+  // the walk in blocks counts a block's numbers from its first token in 32 bits
+  const bool runs = prepared && C < (1 << 26) && lddt < (1 << 26) && ldbc < (1 << 26) && ldz < (1 << 26);
 #define VK_SS_RUN(RR, ALL, TO)                                                                                        \
   selective_run_kernel<RR, ALL, TO><<<run_grid, 256, 0, s>>>(x, dtraw, lddt, bmat, cmat, ldbc, a_log, skip, z, ldz, state, \
                                                              state_stride, entry_start, entry_first, slots, C, N, (TO*)out)
 #define VK_SS(RR, TO)                                                                                               \
   if constexpr (RR <= 4) {                                                                                          \
-    if (prepared) {                                                                                                 \
+    if (runs) {                                                                                                     \
       if (N == 16 * RR) VK_SS_RUN(RR, true, TO);                                                                    \
       else VK_SS_RUN(RR, false, TO);                                                                                \
       break;                                                                                                        \
