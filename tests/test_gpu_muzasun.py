@@ -498,3 +498,33 @@ def test_the_trace_runner_replays_a_schedule(tmp_path, m1):
     for step, want in rows.items():
         got = np.fromfile(out / f"{step}.f32", dtype="<f4").reshape(len(want), cfg["vocab"])
         assert rel_err(got, np.stack(want)) < TOL["float32"]
+
+
+@pytest.mark.parametrize("sizes", [(1, 4, 9), (2, 64, 16), (3, 68, 8), (2, 128, 24), (6, 40, 130), (40, 64, 20)])
+def test_prompts_memory_gives_the_same_bits_from_rows_off_16_bytes(sizes):
+    """Rows in whole pieces of 16 bytes go straight into LDS, 32 lanes a value channel; the same numbers a float further on in memory
+    take the general walk: fresh and continued states, whole blocks, remainders and a single token, every output and the states."""
+    from vipera_rs_amd.ops import kernels
+
+    heads, dim, vdim = sizes
+    lengths, firsts = (33, 1, 16, 70, 15, 32), (0, 5, 3, 0, 1, 2)
+    gen = torch.Generator("cuda").manual_seed(7)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    tokens, keys, columns = sum(lengths), heads * dim, 2 * heads * dim + heads * vdim + 2 * heads
+    pitch = (columns + 3) // 4 * 4
+    meta = (i32(np.cumsum([0, *lengths]).tolist()), i32(firsts), i32([3, 0, 6, 1, 4, 2]))
+    start = rand(8, kernels.memory_state_floats(heads, dim, vdim))
+    proj = rand(tokens, pitch)
+    proj[:, columns - heads:columns] += 3.0      # forget gates as they are met
+    got = []
+    for floats in (0, 1):
+        room = torch.empty(proj.numel() + floats, device="cuda")
+        given = room[floats:].view(proj.shape)
+        given.copy_(proj)
+        state, out = start.clone(), torch.full((tokens, heads * vdim), float("nan"), device="cuda")
+        kernels.memory_rule(given[:, :columns], 0, keys, 2 * keys, columns - 2 * heads, columns - heads, dim ** -0.5, 15.0, state, *meta,
+                            dim, heads, vdim, out, len(lengths))
+        assert torch.isfinite(out).all()
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

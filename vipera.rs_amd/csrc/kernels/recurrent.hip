@@ -1433,6 +1433,211 @@ __global__ __launch_bounds__(SCAN_THREADS) void memory_scan_kernel(
   if (tid == 0) my_m[0] = m;
 }
 
+// The matrix memory for key widths up to 128 in whole pieces of 16 bytes, with 32 lanes a value channel as in
+// delta_scan_direct_kernel and every number formed as above.  What bounds it is a wave's instructions, some 20 a token for two value
+// channels (25 above for one) and as many as six tokens' besides for a block.  What a token needs once for all its value channels
+// is done before the walk: the wave that has fetched a piece of q or k multiplies it by the scale or by the token's share on its way
+// into LDS, and lane j of a row reads token j's gates itself, whose exponentials are taken among the products of the block before.
+// Four tokens' LDS reads go before the arithmetic of the four before them, sixteen tokens' sums through the lanes together, and a
+// wave works out n . q for four tokens of a block.  (Loads straight into LDS, scaled there: the compiler has every later LDS read of the
+// rows wait for them, 253 us a prompt of 2,048.)  us, above and here, with the gates' kernel: 16 heads of 128 x 128, one entry of 2,048
+// tokens 373 / 233, of 512 97 / 62, of 1,000 and 834 254 / 152, of 512, 456 and 399 200 / 95, eight of 250 251 / 126; 8 heads, 2,048 tokens
+// 361 / 223; 6 heads of 64 x 64, 512, 456 and 399 80 / 49; 31 tokens 13 / 11.
+template <int Q>
+__global__ __launch_bounds__(SCAN_COLS * 32) void memory_scan_direct_kernel(
+    const float* __restrict__ proj, long long ldp, MemoryColumns col, float q_scale,
+    float* __restrict__ state, long long state_stride, long long n_offset, long long m_offset,
+    const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots, int dim,
+    int heads, int vdim, int key_pad, int value_pad, float* __restrict__ out) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int DP = 64 * Q, N = 2 * Q, WAVES = SCAN_COLS / 2, GROUP = REC_BLOCK / WAVES;
+  constexpr int PIECES = 2 * Q, ROWS = 4 / Q;      // a wave's loads of a block (64 pieces of 16 bytes), rows each
+  static_assert(WAVES == 4 && GROUP == 4, "two waves fetch q, two k; a wave's n . q are of four tokens");
+  __shared__ __attribute__((aligned(16))) float rows[2][2][REC_BLOCK][DP];
+  __shared__ float values[2][REC_BLOCK][SCAN_COLS];
+  __shared__ float dens[2][REC_BLOCK];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int who = tid >> 5, d0 = (lane & 31) * N, jj = lane & (REC_BLOCK - 1);
+  const int v0 = blockIdx.z * SCAN_COLS, v = v0 + who;
+  const bool live = v < vdim;
+  const int start = entry_start[e], end = entry_start[e + 1];
+  if (start >= end) return;      // the whole workgroup
+  float* row0 = state + (long long)slots[e] * state_stride;
+  float* mine = row0 + ((long long)h * value_pad + v) * key_pad + d0;
+  float* my_n = row0 + n_offset + ((long long)h * gridDim.z + blockIdx.z) * key_pad + d0;
+  float* my_m = row0 + m_offset + (long long)h * gridDim.z + blockIdx.z;
+  const bool fresh = entry_first[e] == 0;
+  float S[N], norm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const bool in = !fresh && d0 + i < key_pad;
+    S[i] = in ? mine[i] : 0.f;
+    norm[i] = in ? my_n[i] : 0.f;
+  }
+  float m = fresh ? 0.f : my_m[0];
+  const int row_bytes = (int)ldp * 4, piece = lane % (16 * Q) * 4;
+  const bool a_query = wave < 2;
+  const int piece_at = piece < dim ? ((a_query ? col.q : col.k) + h * dim + piece) * 4 : -1;
+  const int first_row = (wave & 1) * PIECES * ROWS + lane / (16 * Q);
+  const int value_at = v0 + (tid & 7) < vdim ? (col.v + h * vdim + v0 + (tid & 7)) * 4 : -1;
+  int piece_off[PIECES];
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) piece_off[i] = piece_at < 0 ? -1 : (first_row + i * ROWS) * row_bytes + piece_at;
+  const int value_off = value_at < 0 ? -1 : (tid >> 3) * row_bytes + value_at;
+  // a row past the entry's end is its last one, which nobody works on; what does not exist (-1) reads zeros
+  f32x4 held[PIECES];
+  float held_value = 0.f;
+  auto fetch = [&](int t0) {
+    const int last = min(REC_BLOCK, end - t0) - 1;
+    const ScanView view = scan_view(proj + t0 * ldp, (last + 1) * row_bytes);
+    const bool whole = last == REC_BLOCK - 1;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      held[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+          view.rsrc, whole || piece_at < 0 ? piece_off[i] : min(first_row + i * ROWS, last) * row_bytes + piece_at, 0, 0));
+    if (a_query)
+      held_value = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+          view.rsrc, whole || value_at < 0 ? value_off : min(tid >> 3, last) * row_bytes + value_at, 0, 0));
+  };
+  float li, lf;      // token jj's gates, of the block behind the one whose exponentials are next
+  auto fetch_gates = [&](int t0) {
+    const float* gates = proj + min(t0 + jj, end - 1) * ldp + h;
+    li = gates[col.i];
+    lf = gates[col.f];
+  };
+  // A block's running maxima in closed form, as above, of `count` tokens from the maximum m on.
+  struct Gates { float keep, take, floor, m; };
+  auto gates_of = [&](float li_j, float lf_j, float m, int count) {
+    float F = lf_j;
+    F += row_shifted<1>(F, 0.f);
+    F += row_shifted<2>(F, 0.f);
+    F += row_shifted<4>(F, 0.f);
+    F += row_shifted<8>(F, 0.f);
+    float p = li_j - F;
+    p = fmaxf(p, row_shifted<1>(p, -INFINITY));
+    p = fmaxf(p, row_shifted<2>(p, -INFINITY));
+    p = fmaxf(p, row_shifted<4>(p, -INFINITY));
+    p = fmaxf(p, row_shifted<8>(p, -INFINITY));
+    const float m_j = F + fmaxf(m, p), m_before = row_shifted<1>(m_j, m);
+    return Gates{expf(lf_j + m_before - m_j), expf(li_j - m_j), expf(-m_j),
+                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m_j), count - 1))};
+  };
+  // the wave's pieces of a block, times the scale (q) or the tokens' shares (k), into LDS
+  auto share = [&](int buf, float take) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const float taken = __shfl(take, first_row + i * ROWS, 64);
+      *(f32x4*)(&rows[buf][0][0][0] + (wave * PIECES + i) * 256 + lane * 4) = held[i] * (a_query ? q_scale : taken);
+    }
+    if (a_query) values[buf][tid >> 3][tid & 7] = held_value;
+  };
+  const RowMerge merge(lane);
+  float tops = 0.f, floor_before = 0.f;      // lane j of every row: its row's part of token j's S^T q, and the token's floor
+  auto store = [&](int t0, int buf) {
+    const float top = pair_total(tops);
+    if (live && (lane & 31) < min(REC_BLOCK, end - t0))
+      out[((long long)(t0 + jj) * heads + h) * vdim + v] = top / (fmaxf(fabsf(dens[buf][jj]), floor_before) + 1e-6f);
+  };
+  fetch_gates(start);
+  fetch(start);
+  Gates now = gates_of(li, lf, m, min(REC_BLOCK, end - start));
+  share(0, now.take);
+  fetch_gates(start + REC_BLOCK);
+  for (int t0 = start, buf = 0; t0 < end; t0 += REC_BLOCK, buf ^= 1) {
+    const int count = min(REC_BLOCK, end - t0);
+    const bool more = t0 + REC_BLOCK < end;
+    // what was asked for a block ago, the gates among it: asked for here, or the compiler waits for them behind the loads below
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();                        // everybody's part of the block; and nobody reads the block before any more
+    float kk[2][GROUP][N], qq[2][GROUP][N], val[2][GROUP], quads[GROUP];
+    auto read = [&](int j, int of, int n) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        kk[of][n][i] = rows[buf][1][j][d0 + i];
+        qq[of][n][i] = rows[buf][0][j][d0 + i];
+      }
+      val[of][n] = values[buf][j][who];
+    };
+#pragma unroll
+    for (int n = 0; n < GROUP; ++n) read(n, 0, n);
+    if (t0 > start) store(t0 - REC_BLOCK, buf ^ 1);
+    floor_before = now.floor;
+    const float next_li = li, next_lf = lf;
+    if (more) fetch(t0 + REC_BLOCK);
+    fetch_gates(t0 + 2 * REC_BLOCK);
+    auto lane_sum = [&](const float (&x)[N], const float (&y)[N]) {
+      float part[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < N; ++i) part[i / Q] = fmaf(x[i], y[i], part[i / Q]);
+      return part[0] + part[1];
+    };
+    auto token = [&](int j, int of, int n) {
+      const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.keep), j));
+#pragma unroll
+      for (int i = 0; i < N; ++i) S[i] = fmaf(kk[of][n][i], val[of][n], a * S[i]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) norm[i] = fmaf(a, norm[i], kk[of][n][i]);
+      return lane_sum(S, qq[of][n]);
+    };
+    Gates next = now;
+    if (count == REC_BLOCK) {
+      auto group = [&](int g, auto with_dens) {
+        if (g == 1) next = gates_of(next_li, next_lf, now.m, min(REC_BLOCK, end - t0 - REC_BLOCK));
+        float num[GROUP], den[GROUP];
+#pragma unroll
+        for (int n = 0; n < GROUP; ++n) {
+          num[n] = token(g * GROUP + n, g & 1, n);
+          if constexpr (decltype(with_dens)::value) den[n] = lane_sum(norm, qq[g & 1][n]);
+        }
+        quads[g] = merge.quads(num[0], num[1], num[2], num[3]);
+        if constexpr (decltype(with_dens)::value) {      // lane n of every four: token n's
+          float d = merge.quads(den[0], den[1], den[2], den[3]);
+          int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x104, 0xF, 0x5, false);
+          moved = __builtin_amdgcn_update_dpp(moved, __float_as_int(d), 0x114, 0xF, 0xA, false);
+          d += __int_as_float(moved);
+          d = pair_total(dpp_add<0x128>(d));
+          if (lane < GROUP) dens[buf][g * GROUP + lane] = d;
+        }
+      };
+#pragma unroll
+      for (int g = 0; g < WAVES; ++g) {
+        if (g + 1 < WAVES) {
+#pragma unroll
+          for (int n = 0; n < GROUP; ++n) read((g + 1) * GROUP + n, (g + 1) & 1, n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (wave == g) group(g, std::integral_constant<bool, true>{});      // the whole wave or none of it
+        else group(g, std::integral_constant<bool, false>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (more) share(buf ^ 1, next.take);      // asked for a block ago
+      tops = merge.rows(quads);
+    } else {
+      for (int j = 0; j < count; ++j) {
+        read(j, 0, 0);
+        const float num = row_sum16(token(j, 0, 0));
+        tops = jj == j ? num : tops;
+        if (wave == j / GROUP) {
+          const float den = pair_total(row_sum16(lane_sum(norm, qq[0][0])));
+          if (lane == 0) dens[buf][j] = den;
+        }
+      }
+    }
+    m = now.m;
+    now = next;
+  }
+  __syncthreads();     // the last block's n . q are in LDS
+  const int blocks = (end - start - 1) / REC_BLOCK;
+  store(start + blocks * REC_BLOCK, blocks & 1);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (d0 + i < key_pad) {
+      mine[i] = S[i];
+      if (tid < 32) my_n[i] = norm[i];
+    }
+  if (tid == 0) my_m[0] = m;
+}
+
 // x[t, c] = exp(-exp(x[t, c] + w0[c])) in place: time mixing's decay, for a step whose recurrence reads it many times.
 __global__ void decay_kernel(float* __restrict__ x, const float* __restrict__ w0, int width, long long count) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1628,10 +1833,18 @@ extern "C" int vk_memory_rule(float* proj, long long ldp, int num_tokens, int q_
   memory_scan_kernel<Q><<<scan_grid, SCAN_THREADS, 0, s>>>(proj, ldp, col, q_scale, state, state_stride, n_offset,     \
                                                            m_offset, entry_start, entry_first, slots, dim, heads, vdim, \
                                                            key_pad, value_pad, out)
-    if (key_pad <= 64) VK_MEMORY_SCAN(1);
+#define VK_MEMORY_DIRECT(Q)                                                                                          \
+  memory_scan_direct_kernel<Q><<<scan_grid, SCAN_COLS * 32, 0, s>>>(proj, ldp, col, q_scale, state, state_stride,      \
+                                                                    n_offset, m_offset, entry_start, entry_first,     \
+                                                                    slots, dim, heads, vdim, key_pad, value_pad, out)
+    const bool pieces = (dim | q_col | k_col) % 4 == 0 && ldp % 4 == 0 && ((uintptr_t)proj & 15) == 0;
+    if (pieces && key_pad <= 64) VK_MEMORY_DIRECT(1);
+    else if (pieces && key_pad <= 128) VK_MEMORY_DIRECT(2);
+    else if (key_pad <= 64) VK_MEMORY_SCAN(1);
     else if (key_pad <= 128) VK_MEMORY_SCAN(2);
     else VK_MEMORY_SCAN(4);
 #undef VK_MEMORY_SCAN
+#undef VK_MEMORY_DIRECT
     VK_LAUNCH_CHECK();
     return 0;
   }
