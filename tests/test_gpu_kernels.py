@@ -1627,3 +1627,36 @@ def test_routes_by_lane_moves_are_the_largest_logits_lowest_id_first(tokens, exp
     placed = order.tolist()
     assert sorted(placed) == list(range(pairs)) and all(flat[p] == e for e in range(experts) for p in placed[starts[e]:starts[e + 1]])
     assert tiles.tolist()[:2 * count.item()] == [x for e in range(experts) for first in range(starts[e], starts[e + 1], 64) for x in (e, first)]
+
+
+# every form of the 32-bit product, at sizes with remainders of its tiles, and one of several slabs in each form that walks them
+@pytest.mark.parametrize("m,inter,k", [
+    (9, 4, 132), (17, 20, 896), (17, 2404, 896), (130, 1004, 896), (333, 516, 1024), (700, 4868, 1024), (50, 4868, 64), (50, 4864, 132),
+    (17, 8968, 260), (65, 4868, 1536), (333, 4864, 132), (333, 2404, 1028), (333, 2404, 896), (65, 8962, 896), (130, 2405, 896)])
+def test_gated_32_bit_product_has_the_bits_of_product_and_gate(m, inter, k):
+    from vipera_rs_amd.ops import kernels
+
+    gen = torch.Generator("cuda").manual_seed(m + inter + k)
+    a = torch.randn(m, k, generator=gen, device="cuda")
+    w = torch.randn(2 * inter, k, generator=gen, device="cuda") * k ** -0.5
+    a[0, 0] = 1e30     # a row of gates far out on both sides
+    both, want = torch.empty(m, 2 * inter, device="cuda"), torch.empty(m, inter, device="cuda")
+    kernels.gemm_generic(a, w, None, both)
+    kernels.swiglu(both, want)
+    got = torch.full((m, inter), float("nan"), device="cuda")
+    assert kernels.gemm_generic_gated(a, w, got)
+    assert torch.equal(got, want)
+    strided = torch.empty(m, k + 4, device="cuda")
+    strided[:, :k] = a
+    assert kernels.gemm_generic_gated(strided[:, :k], w, got.fill_(0.0)) and torch.equal(got, want)
+
+
+def test_gated_32_bit_product_leaves_what_it_cannot_take():
+    from vipera_rs_amd.ops import kernels
+
+    a, w, out = torch.ones(65, 1028, device="cuda"), torch.ones(24, 1028, device="cuda"), torch.zeros(65, 12, device="cuda")
+    assert not kernels.gemm_generic_gated(a, w, out)                                   # parts of its sums in memory
+    assert not kernels.gemm_generic_gated(a[:8, :64], w[:, :64].contiguous(), out[:8])      # a stream of the weights
+    room = torch.ones(65 * 64 + 1, device="cuda")
+    assert not kernels.gemm_generic_gated(room[1:].view(65, 64), w[:, :64].contiguous(), out)     # rows off 16 bytes
+    assert not out.any()

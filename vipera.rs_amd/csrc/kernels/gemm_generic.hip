@@ -226,6 +226,14 @@ __device__ __forceinline__ void store_outputs(float* __restrict__ C, const float
   }
 }
 
+// Four outputs of a gated product: up * silu(gate).
+__device__ __forceinline__ f32x4_t gated_outputs(f32x4_t gate, f32x4_t up) {
+  f32x4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = up[e] * (gate[e] / (1.0f + expf(-gate[e])));
+  return v;
+}
+
 // Hints for the order of what was written since the last such line: LDS reads and loads go out one by one between the products.
 // All of them ahead of the products made every wave wait for the others' at the LDS and address units: 112 TFLOP/s at
 // 2,048 x 4,096 x 4,096.
@@ -249,7 +257,9 @@ template <int TM, int TN> constexpr int READS_OF = 4 * ((TM + 1) / 2 + (TN + 1) 
 // bytes at 16 L); chunk c of row r sits in slot c ^ (r / 2 % 8): the 64 values of a block's next four k lie in 64 banks.  A wave
 // loads every WAVES-th 8 rows, so that its lanes' chunks are the same in all of them.  It reads the operands of a half step
 // while it multiplies the first half of the other.  SLABS: K has several.
-template <int TM, int TN, int WM, int WN, int STAGES, bool SLABS, bool ACCUMULATE>
+// GATED: W is [gate; up], N rows each, and C's N columns up * silu(gate); every second block of 16 rows of a tile is up's of the
+// outputs whose gates the block before it has, so that a lane has both sums of an output.
+template <int TM, int TN, int WM, int WN, int STAGES, bool SLABS, bool ACCUMULATE, bool GATED = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                                  const float* __restrict__ bias, float* __restrict__ C, int M,
                                                                  int N, int K, long long lda, long long ldc, bool quads) {
@@ -261,7 +271,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, lr = lane & 15;
   const int m_tiles = (M + BM - 1) / BM;
-  const int m0 = blockIdx.x % m_tiles * BM, n0 = blockIdx.x / m_tiles * BN;
+  const int m0 = blockIdx.x % m_tiles * BM, n0 = blockIdx.x / m_tiles * (GATED ? BN / 2 : BN);
+  static_assert(!GATED || (TN % 2 == 0 && !ACCUMULATE), "blocks of gate and up in pairs");
   const __amdgpu_buffer_rsrc_t a_view = row_view(A + (size_t)m0 * lda), w_view = row_view(W + (size_t)n0 * K);
   const int ld_row = lane >> 3, ld_chunk = (lane & 7) ^ (lane >> 4) ^ (wave & 1) * 4;
   unsigned a_off[A_LOADS], w_off[W_LOADS];
@@ -269,8 +280,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
   for (int i = 0; i < A_LOADS; ++i)
     a_off[i] = (unsigned)(min(m0 + (i * WAVES + wave) * 8 + ld_row, M - 1) - m0) * (unsigned)(lda * 4) + ld_chunk * 16;
 #pragma unroll
-  for (int i = 0; i < W_LOADS; ++i)
-    w_off[i] = (unsigned)(min(n0 + (i * WAVES + wave) * 8 + ld_row, N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
+  for (int i = 0; i < W_LOADS; ++i) {
+    const int r = (i * WAVES + wave) * 8 + ld_row;
+    if constexpr (GATED)
+      w_off[i] = (unsigned)((r & 16 ? N : 0) + min(n0 + (r / 32 * 16 + r % 16), N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
+    else
+      w_off[i] = (unsigned)(min(n0 + r, N - 1) - n0) * (unsigned)(K * 4) + ld_chunk * 16;
+  }
   auto issue = [&](int stage, int step) {
     unsigned char* to_a = lds + stage * STAGE + wave * 1024;
     unsigned char* to_w = to_a + BM * ROW;
@@ -354,6 +370,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
       }
   }
   loads_but<0>();                                      // no load may write LDS that the next workgroup has
+  if constexpr (GATED) {
+#pragma unroll
+    for (int n = 0; n < TN; n += 2)
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+        store_outputs<false>(C, nullptr, SLABS ? gated_outputs(total[n][m], total[n + 1][m]) : gated_outputs(slab[n][m], slab[n + 1][m]),
+                             m0 + (wm * TM + m) * 16 + lr, n0 + (wn * TN + n) * 8 + 4 * (lane >> 4), M, N, ldc, quads);
+    return;
+  }
   auto store = [&](bool in_quads) {
 #pragma unroll
     for (int n = 0; n < TN; ++n)
@@ -369,7 +394,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const float* __
 // A workgroup's 16 TM x 16 TN outputs over one slab (blockIdx.y), a range a wave.  A wave has stages of its own, of 16 k,
 // and waits for no other before the ranges' sums meet.  LDS rows are 64 bytes (a load instruction: 16 rows); chunk c of row r
 // sits in slot c ^ (r / 4 % 4): the 64 values of a block's next four k lie in 64 banks.
-template <int TM, int TN, int STAGES, bool PARTS, bool ACCUMULATE>
+// GATED: as in gemm_rows_kernel, but a block's first eight rows are gate's and its others up's of the same eight outputs, as a
+// tile may have an odd number of blocks: the sums of an output are 32 lanes apart.
+template <int TM, int TN, int STAGES, bool PARTS, bool ACCUMULATE, bool GATED = false>
 __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                         const float* __restrict__ bias, float* __restrict__ C,
                                                         float* __restrict__ parts, int M, int N, int K, long long lda,
@@ -380,7 +407,8 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m_tiles = (M + 16 * TM - 1) / (16 * TM);
-  const int m0 = blockIdx.x % m_tiles * (16 * TM), n0 = blockIdx.x / m_tiles * (16 * TN);
+  const int m0 = blockIdx.x % m_tiles * (16 * TM), n0 = blockIdx.x / m_tiles * (GATED ? 8 * TN : 16 * TN);
+  static_assert(!GATED || (!PARTS && !ACCUMULATE), "the gate needs whole sums");
   const int k_begin = blockIdx.y * SLAB_K + wave * RANGE_K, k_end = min(K, k_begin + RANGE_K);
   unsigned char* mine = lds + wave * (STAGES * STAGE);
   f32x4_t acc[TN][TM];
@@ -393,9 +421,11 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
     const int ld_row = lane >> 2, ld_chunk = (lane & 3) ^ (lane >> 4), left = k_end - k_begin;
     unsigned off[GROUPS];
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g)
+    for (int g = 0; g < GROUPS; ++g) {
+      const int w_row = GATED ? (ld_row & 8 ? N : 0) + min(n0 + 8 * (g - TM) + (ld_row & 7), N - 1) : min(n0 + 16 * (g - TM) + ld_row, N - 1);
       off[g] = (g < TM ? (unsigned)(min(m0 + 16 * g + ld_row, M - 1) - m0) * (unsigned)(lda * 4)
-                             : (unsigned)(min(n0 + 16 * (g - TM) + ld_row, N - 1) - n0) * (unsigned)(K * 4)) + ld_chunk * 16;
+                             : (unsigned)(w_row - n0) * (unsigned)(K * 4)) + ld_chunk * 16;
+    }
     auto issue = [&](int stage, int step) {
       unsigned char* to = mine + stage * STAGE;
       const unsigned kb = step * STEP + ld_chunk * 4 < left ? (unsigned)(step * STEP * 4) : NO_CHUNK;
@@ -471,6 +501,15 @@ __global__ __launch_bounds__(256) void gemm_slab_kernel(const float* __restrict_
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < SLAB_RANGES; ++w) v += *(const f32x4_t*)(sums + (((size_t)w * SUM_QUADS + b) * 64 + lane) * 4);
+    if constexpr (GATED) {
+      f32x4_t up;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(v[e], 32, 64);
+      if (lane < 32)
+        store_outputs<false>(C, nullptr, gated_outputs(v, up), m0 + 16 * (b % TM) + (lane & 15), n0 + 8 * (b / TM) + 4 * (lane >> 4), M, N,
+                             ldc, quads);
+      continue;
+    }
     const int row = m0 + 16 * (b % TM) + (lane & 15), column = n0 + 16 * (b / TM) + 4 * (lane >> 4);
     if constexpr (PARTS) store_outputs<false>(parts + (size_t)blockIdx.y * M * N, nullptr, v, row, column, M, N, N, N % 4 == 0);
     else store_outputs<ACCUMULATE>(C, bias, v, row, column, M, N, ldc, quads);
@@ -641,6 +680,43 @@ int launch_slabs(const float* A, const float* W, const float* bias, float* C, fl
   if (slabs == 1) return 0;
   return accumulate ? launch_finish<float, true>(parts, bias, C, M, N, ldc, slabs, 1, s)
                     : launch_finish<float, false>(parts, bias, C, M, N, ldc, slabs, 1, s);
+}
+
+// The gated forms: C [M, N] from W [2 N, K]; K is one slab where a workgroup owns a slab.
+template <int TM, int TN, int WM, int WN, int STAGES>
+int launch_rows_gated(const float* A, const float* W, float* C, int M, int N, int K, long long lda, long long ldc, hipStream_t s) {
+  constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, lds_bytes = STAGES * (BM + BN) * 128;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipSuccess;
+    for (const void* f : {(const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, false, false, true>, (const void*)gemm_rows_kernel<TM, TN, WM, WN, STAGES, true, false, true>})
+      if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  const unsigned tiles = (unsigned)(((M + BM - 1) / BM) * ((N + BN / 2 - 1) / (BN / 2)));
+  const bool quads = stores_quads(C, nullptr, N, ldc);
+  if (K <= SLAB_K) gemm_rows_kernel<TM, TN, WM, WN, STAGES, false, false, true><<<tiles, 64 * WM * WN, lds_bytes, s>>>(A, W, nullptr, C, M, N, K, lda, ldc, quads);
+  else gemm_rows_kernel<TM, TN, WM, WN, STAGES, true, false, true><<<tiles, 64 * WM * WN, lds_bytes, s>>>(A, W, nullptr, C, M, N, K, lda, ldc, quads);
+  VK_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int TM, int TN, int STAGES>
+int launch_slab_gated(const float* A, const float* W, float* C, int M, int N, int K, long long lda, long long ldc, hipStream_t s) {
+  constexpr int BM = 16 * TM, BN = 16 * TN, lds_bytes = 4 * STAGES * (BM + BN) * 64;
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_slab_kernel<TM, TN, STAGES, false, false, true>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  const unsigned tiles = (unsigned)(((M + BM - 1) / BM) * ((N + BN / 2 - 1) / (BN / 2)));
+  gemm_slab_kernel<TM, TN, STAGES, false, false, true><<<tiles, 256, lds_bytes, s>>>(A, W, nullptr, C, nullptr, M, N, K, lda, ldc,
+                                                                                     stores_quads(C, nullptr, N, ldc));
+  VK_LAUNCH_CHECK();
+  return 0;
 }
 
 // Which kernel an all-32-bit product of aligned rows takes.  Both cut M x N into tiles, one a workgroup, and a call lasts as
@@ -960,9 +1036,43 @@ int dispatch(const void* A, int a_dtype, const void* W, int w_dtype, const float
 }
 }  // namespace
 
+extern "C" long long vk_gemm_generic_workspace(int M, int N, int K);
+
 // The kernel that an all-32-bit product of aligned rows takes with a workspace of part_floats (direct_plan); 0: the 64 x 64 tiles.
 extern "C" int vk_gemm_generic_form(int M, int N, int K, long long part_floats) {
   return M <= 0 || N <= 0 || K <= 0 || (K & 3) || K > DIRECT_MAX_ROW ? 0 : (int)direct_plan(M, N, K, part_floats);
+}
+
+// A gated product, C [M, N] = up * silu(gate) with W = [gate; up], N rows each, all 32-bit and rows on 16 bytes, in the form and the bits
+// of the product of 2 N rows.  Whether it is taken: where that form leaves no parts in memory and W lies within a view.  The gate as a
+// launch of its own waits for the product and passes its sums through memory.  us, product and gate in two launches and here: 333 x (2 x
+// 4,864) x 896 78.2 / 69.2, of 64 rows 25.8 / 23.8, of 17 17.6 / 16.0; 65 x (2 x 8,960) x 1,536 72.0 / 65.0, of 400 rows 235 / 222.
+static Direct gated_plan(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || (K & 3) || K > DIRECT_MAX_ROW || 2ll * N * K * 4 >= VIEW_BYTES) return NOT_DIRECT;
+  const Direct form = direct_plan(M, 2 * N, K, vk_gemm_generic_workspace(M, 2 * N, K));
+  const bool slab = form != ROWS_64_64 && form != ROWS_32_128 && form != ROWS_64_128;
+  return slab && K > SLAB_K ? NOT_DIRECT : form;
+}
+extern "C" int vk_gemm_generic_gated_takes(int M, int N, int K) { return gated_plan(M, N, K) != NOT_DIRECT; }
+
+extern "C" int vk_gemm_generic_gated(const float* A, const float* W, float* C, int M, int N, int K, long long lda, long long ldc,
+                                     void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || lda < K || ldc < N || lda % 4 || lda > DIRECT_MAX_ROW || (((uintptr_t)A | (uintptr_t)W) & 15)) return VK_BAD_ARGUMENT;
+  hipStream_t s = (hipStream_t)stream;
+  switch (gated_plan(M, N, K)) {
+    case SLAB_16_32: return launch_slab_gated<1, 2, 3>(A, W, C, M, N, K, lda, ldc, s);
+    case SLAB_32_32: return launch_slab_gated<2, 2, 2>(A, W, C, M, N, K, lda, ldc, s);
+    case SLAB_48_32: return launch_slab_gated<3, 2, 2>(A, W, C, M, N, K, lda, ldc, s);
+    case SLAB_48_48: return launch_slab_gated<3, 3, 2>(A, W, C, M, N, K, lda, ldc, s);
+    case SLAB_48_64: return launch_slab_gated<3, 4, 2>(A, W, C, M, N, K, lda, ldc, s);
+    case SLAB_64_64: return launch_slab_gated<4, 4, 2>(A, W, C, M, N, K, lda, ldc, s);
+    case ROWS_64_64: return launch_rows_gated<2, 2, 2, 2, 3>(A, W, C, M, N, K, lda, ldc, s);
+    case ROWS_32_128: return launch_rows_gated<2, 2, 1, 4, 3>(A, W, C, M, N, K, lda, ldc, s);
+    case ROWS_64_128: return launch_rows_gated<2, 4, 2, 2, 3>(A, W, C, M, N, K, lda, ldc, s);
+    case NOT_DIRECT: break;
+  }
+  return VK_UNSUPPORTED_SIZE;
 }
 
 // Without a workspace: no sums go through memory. dtypes: 0 = float, 1 = bfloat16. lda / ldc are row strides in elements.

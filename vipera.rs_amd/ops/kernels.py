@@ -245,6 +245,29 @@ def _gemm_direct_parts(m: int, n: int, k: int) -> int:
     return _fn("gemm_generic", "vk_gemm_generic_direct_workspace", [_i, _i, _i], restype=_ll)(m, n, k)
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_gated_takes(m: int, inter: int, k: int) -> bool:
+    return bool(_fn("gemm_generic", "vk_gemm_generic_gated_takes", [_i, _i, _i])(m, inter, k))
+
+
+def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """``out = up(a) * silu(gate(a))`` of 32-bit operands with ``w = [gate; up]``, in the product's own launch and with the bits of
+    :func:`gemm_generic` and :func:`swiglu` behind it; False, and nothing launched, where these are to be used: up to 8 tokens, which are a
+    stream of the weights, rows off 16 bytes, and sizes whose product leaves parts of its sums in memory."""
+    _dev(a, w, out)
+    m, k = a.shape
+    inter = out.shape[1]
+    if not (m > 8 and a.dtype == w.dtype == out.dtype == torch.float32 and w.shape == (2 * inter, k) and out.shape[0] == m):
+        return False
+    lda = a.stride(0)
+    if not (a.stride(1) == 1 and lda >= k and w.is_contiguous() and out.is_contiguous() and lda % 4 == 0 and k % 4 == 0
+            and lda <= GEMM_DIRECT_MAX_ROW and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _gemm_gated_takes(m, inter, k)):
+        return False
+    fn = _fn("gemm_generic", "vk_gemm_generic_gated", [_p, _p, _p, _i, _i, _i, _ll, _ll, _p])
+    _status(fn(_ptr(a), _ptr(w), _ptr(out), m, inter, k, lda, inter, _stream()), "gemm_generic_gated")
+    return True
+
+
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                  accumulate: bool = False) -> None:
     """``out (+)= a @ w.T + bias`` with every product and sum in 32 bits; ``a`` and ``out`` may be row-strided views."""
