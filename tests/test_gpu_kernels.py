@@ -278,6 +278,27 @@ def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):
     assert torch.equal(out, other)
 
 
+@pytest.mark.parametrize("m,n,k,tiling,before,cut", [(1396, 1536, 8960, 20, 6, 4), (1201, 896, 4864, 18, 7, 4), (400, 900, 4864, 17, 9, 8),
+                                                     (311, 3584, 4736, 18, 9, 4), (400, 4608, 3584, 18, 7, 2), (130, 5120, 13824, 20, 6, 8)])
+def test_a_plan_of_several_ranges_is_carried_out_with_the_same_bits(m, n, k, tiling, before, cut):
+    """The tile that is picked and the one of the estimate by whole rounds, with the same cut of K; results of either kind."""
+    from vipera_rs_amd.ops import kernels
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    old = torch.randn(m, n, generator=g).to(DEV)
+    for dtype, accumulate in ((torch.float32, False), (torch.bfloat16, False), (torch.float32, True)):
+        out, other = old.to(dtype), old.to(dtype)
+        kernels.gemm_bf16(a, w, None, out, accumulate)
+        assert kernels.gemm_bf16_tile_launched()[:2] == (tiling, cut)
+        try:
+            kernels.gemm_bf16_force_tiling(before, cut)
+            kernels.gemm_bf16(a, w, None, other, accumulate)
+        finally:
+            kernels.gemm_bf16_force_tiling(-1)
+        assert torch.equal(out, other)
+
+
 @pytest.mark.parametrize("m,n,k", [(399, 4288, 512), (288, 8320, 1024), (1435, 5440, 256), (695, 5440, 2048), (1805, 8896, 512),
                                    (512, 1056, 2048), (512, 64, 2048), (330, 7488, 7168), (100, 4608, 3584), (700, 4096, 2040)])
 def test_a_product_launches_the_tile_that_the_plan_names_and_works_it_out_once(m, n, k):

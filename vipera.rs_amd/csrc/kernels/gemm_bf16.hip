@@ -2003,11 +2003,15 @@ int smaller_tiles(int M, int N, int K, int ranges) {
   return small * ranges <= 4LL * g_compute_units ? 13 : 9;
 }
 
+int split_tile(int planned, int M, int N, int K, int ranges);
+
 // What launch_tile carries out: `scaled`: with a norm's factors.
 TilePlan tile_plan(int M, int N, int K, long long partial_floats, bool gated, bool scaled) {
   const bool direct = (K & 63) == 0;
   TilePlan plan = choose_tile_plan(M, N, K, partial_floats, direct, gated);
   if (direct && plan.config == 9 && M > 128 && !scaled) plan.config = smaller_tiles(M, N, K, plan.ranges);
+  if (direct && plan.config >= 5 && plan.config <= 7 && plan.ranges > 1 && M > 128 && !scaled)
+    plan.config = split_tile(plan.config, M, N, K, plan.ranges);
   return plan;
 }
 
@@ -2040,8 +2044,8 @@ constexpr TileCost WHOLE_TILES[] = {
     {15, 128, 64, 2, 2.6, 0.28, 0.41, 0.69, 0.75, 0.091}, {16, 192, 64, 1, 3.7, 0.34, 0.44, 0, 0, 0.153},
     {17, 128, 128, 1, 3.2, 0.41, 0.53, 0, 0, 0.174},    {18, 192, 128, 1, 5.3, 0.48, 0.59, 0, 0, 0.148},
     {19, 192, 128, 2, 3.0, 0.71, 0.94, 1.32, 0.40, 0.115}, {20, 192, 192, 1, 6.4, 0.63, 0.96, 0, 0, 0.100}};
-double whole_tile_us(const TileCost& t, int M, int N, int K, double output_bytes) {
-  const long long groups = (long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows);
+double whole_tile_us(const TileCost& t, int M, int N, int K, double output_bytes, int ranges = 1) {
+  const long long groups = (long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows) * ranges;
   const long long full = groups / g_compute_units;
   const double rest = (double)(groups % g_compute_units) / g_compute_units;
   const double last = rest > 0 ? t.low + (t.high - t.low) * rest : 0;
@@ -2050,7 +2054,7 @@ double whole_tile_us(const TileCost& t, int M, int N, int K, double output_bytes
     rounds = full / 2 * t.pair + last;
     if (full & 1) rounds = full / 2 * t.pair + t.high + (rest > 0 ? (t.pair - t.high) * (t.alone + (1 - t.alone) * rest) : 0);
   }
-  return t.beside + K / 64 * rounds + t.output * 1e-6 * M * N * output_bytes;
+  return t.beside + (ranges == 1 ? K / 64 : ((K + ranges - 1) / ranges + 63) / 64) * rounds + t.output * 1e-6 * M * N * output_bytes * ranges;
 }
 // output_bytes: per product row and token (a gated product writes one 16-bit result for two rows).
 int whole_tile(int planned, int M, int N, int K, double output_bytes) {
@@ -2065,6 +2069,33 @@ int whole_tile(int planned, int M, int N, int K, double output_bytes) {
         (long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows) > g_compute_units)
       continue;
     const double us = whole_tile_us(t, M, N, K, output_bytes);
+    if (us < best_us) {
+      best_us = us;
+      best = t.config;
+    }
+  }
+  return best;
+}
+
+// The same for a plan of several ranges: whether 128x128, 192x128 or 192x192 with three LDS stages carries its
+// ranges out in one round (a range is K / ranges deep, and its sums are written in 32 bits). The larger tiles come to three quarters of a
+// round or less there, or the 128x128 ones to a little more than one: 1,396 tokens on 1,536 rows of 8,960 in four ranges are 192
+// tiles of 256x192 and 256 of 192x192. Over the 70 products of the sizes above, 130 to 2,000 tokens, that are planned so, the choice takes 0.958
+// of the planned tiles' time, 1.02 of it at worst, and 1.003 of the fastest tile's; with the other tiles, or several rounds of these, among
+// the candidates the estimate is off by up to 1.14. us, planned and picked: 1,396 on 1,536 of 8,960 56.8 / 49.8, 1,200 on 896 of 4,864
+// 29.9 / 25.2, 311 on 3,584 of 18,944 81.1 / 61.5, 400 on 4,608 of 3,584 35.7 / 30.1, 1,200 on 2,048 of 4,096 38.9 / 34.3. The cut of K
+// stays as it was, and so do the bits. A plan of tiles of 256 tokens names the tile that is picked; 128x128 tiles are asked for
+// where they carry the plan out, in four ranges or more.
+int split_tile(int planned, int M, int N, int K, int ranges) {
+  int best = planned;
+  double best_us = -1;
+  for (const TileCost& t : WHOLE_TILES)
+    if (t.config == planned) best_us = 0.98 * whole_tile_us(t, M, N, K, 4.0, ranges);
+  if (best_us < 0) return planned;
+  for (const TileCost& t : WHOLE_TILES) {
+    if (t.config != 17 && t.config != 18 && t.config != 20) continue;
+    if ((long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows) * ranges > g_compute_units) continue;
+    const double us = whole_tile_us(t, M, N, K, 4.0, ranges);
     if (us < best_us) {
       best_us = us;
       best = t.config;
@@ -2112,6 +2143,7 @@ TilePlan carried_out(int M, int N, int K, long long partial_floats, bool gated, 
     ++g_tile_launched.plans;
     TilePlan plan = tile_plan(M, N, K, (long long)most_ranges * M * N, gated, scaled);
     if ((K & 63) == 0 && M > 128 && plan.ranges == 1 && !scaled) plan.config = whole_tile(plan.config, M, N, K, output_bytes);
+    if ((K & 63) == 0 && M > 128 && plan.ranges >= 4 && plan.config == 9 && !scaled) plan.config = split_tile(9, M, N, K, plan.ranges);
     if ((K & 63) == 0 && M <= 64 && gated) plan.config = few_tokens_tile(N);
     kept = Kept{M, N, K, form, plan};
   }
