@@ -751,3 +751,37 @@ def test_the_trace_runner_replays_a_schedule(tmp_path, r1):
     for step, want in rows.items():
         got = np.fromfile(out / f"{step}.f32", dtype="<f4").reshape(len(want), cfg["vocab"])
         assert rel_err(got, np.stack(want)) < TOL["float32"]
+
+
+@pytest.mark.parametrize("plain, weigh_input", [("relu2", False), (None, True)])
+@pytest.mark.parametrize("tokens, width, ff, experts, top", [(37, 64, 64, 5, 2), (192, 320, 192, 3, 1), (193, 192, 448, 1, 1), (700, 192, 448, 3, 2)])
+def test_experts_in_tiles_of_192_places_give_the_bits_of_128(tokens, width, ff, experts, top, plain, weigh_input):
+    """Experts with no pairs, a tile's exactly, one more and several tiles; columns that end inside a tile, rows further apart than they
+    are long."""
+    from vipera_rs_amd.ops import kernels
+
+    g = torch.Generator(device="cuda").manual_seed(tokens + ff)
+    h = torch.randn(tokens, width + 64, device="cuda", generator=g).to(torch.bfloat16)[:, :width]
+    z = torch.randn(tokens, experts, device="cuda", generator=g) + (torch.arange(experts, device="cuda") == 1) * 2.0
+    if experts > 3:
+        z[:, 3] = -30.0                                   # nobody's choice
+    gate, up = ((torch.randn(experts, ff, width, device="cuda", generator=g) * width ** -0.5).to(torch.bfloat16) for _ in range(2))
+    down = (torch.randn(experts, width, ff, device="cuda", generator=g) * ff ** -0.5).to(torch.bfloat16)
+    got = []
+    for tile_rows in (128, 192):
+        _, w, offsets, order, tiles, count = route(kernels, z, top, tile_rows)
+        act = torch.full((tokens * top, ff), float("nan"), dtype=torch.bfloat16, device="cuda")
+        pair_out, residual = torch.full((tokens * top, width), float("nan"), device="cuda"), torch.empty(tokens, width, device="cuda")
+        kernels.moe_experts(h, None if plain else gate, up, down, offsets, order, tiles, count, w, top, float("inf"), 1.0, act, pair_out,
+                            residual, False, weigh_input, tile_rows, plain=plain)
+        assert torch.isfinite(residual).all()
+        got.append((pair_out, residual))      # by pair and token: a pair's place among its expert's is any
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_tiles_of_192_places_are_for_216_to_288_pairs_an_expert():
+    from vipera_rs_amd.ops import kernels
+
+    rows = lambda tokens, gated=True: kernels.moe_tile_rows(torch.empty(tokens, 2048, dtype=torch.bfloat16, device="cuda"), 2048, 1024, 4 * tokens, 32, gated)
+    assert [rows(n) for n in (1400, 1727, 1728, 2048)] == [128, 128, 192, 192] and rows(3000) == 256
+    assert [rows(n, False) for n in (1727, 1728, 2304, 2305)] == [128, 192, 192, 128]

@@ -2,7 +2,7 @@
 //
 // A step's T tokens each choose `top` of E experts: P = T * top pairs, pair p = t * top + j.  The pairs are
 // grouped by expert (`order[i]` is the pair at sorted place i, `offsets[e]` the first place of expert e) and cut
-// into tiles of 64 places (128 or 256 on the matrix cores, 16 where a step has few pairs) that never span two experts; a
+// into tiles of 64 places (128, 192 or 256 on the matrix cores, 16 where a step has few pairs) that never span two experts; a
 // product's workgroup owns one tile and some output columns.  The grid is sized for the most tiles there can be, and workgroups past `num_tiles` (which only the
 // device knows) leave at once.  Which place a pair gets depends on the order in which the counters were bumped,
 // but no value does: a pair's row is computed alone, an FMA chain in k order per output element, and the
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void moe_down_mma_kernel(const __bf16* __restr
 // through one L2.  Grid (a multiple of eight at or above the tiles there can be, column blocks): a row of the grid holds a column
 // block's share of every XCD, so that the numbers run on from row to row.  In one row they passed the 2^32 threads that a launch takes.
 template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
-__global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
+__global__ __launch_bounds__(WM* WN * 64, (2 * gt_direct_lds<BM, BN, STAGES>() <= 160 * 1024 ? WM * WN / 2 : WM * WN / 4)) void moe_direct_kernel(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
                                                                  const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
                                                                  const int* __restrict__ offsets,
                                                                  const int* __restrict__ order, const int* __restrict__ tiles,
@@ -495,12 +495,9 @@ __global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* _
   if (at >= own * blocks) return;
   const int tile = t0 + at % own, n0 = at / own * COLUMNS;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  __shared__ unsigned rows[BM];
   const int e = tiles[2 * tile], first = tiles[2 * tile + 1];
   const int count = min(BM, offsets[e + 1] - first);
-  for (int i = threadIdx.x; i < BM; i += WM * WN * 64)
-    rows[i] = i < count ? (unsigned)((FORM == 2 ? first + i : order[first + i] / top) * ldi * 2) : GT_NO_ROW;
-  __syncthreads();
+  auto row = [&](int r) { return r < count ? (unsigned)((FORM == 2 ? first + r : order[first + r] / top) * ldi * 2) : GT_NO_ROW; };
   // weight row r of the tile: the wave's rows are its columns of the gate, then the same columns of up
   auto column = [&](int r) {
     if constexpr (FORM != 0) return n0 + r;
@@ -510,7 +507,7 @@ __global__ __launch_bounds__(WM* WN * 64) void moe_direct_kernel(const __bf16* _
   const long long matrix = (long long)e * N * K, matrix_bytes = (long long)N * K * 2;
   gt_f32x4 acc[TN][TM];
   group_tile_direct<BM, BN, WM, WN, STAGES>(
-      gt_view(in, in_bytes), [&](int r) { return rows[r]; }, gt_view(w0 + matrix, matrix_bytes), gt_view(w1 + matrix, matrix_bytes),
+      gt_view(in, in_bytes), row, gt_view(w0 + matrix, matrix_bytes), gt_view(w1 + matrix, matrix_bytes),
       [&](int r) { const int c = column(r); return c < N ? (unsigned)c * (unsigned)K * 2u : GT_NO_ROW; },
       [&](int r) { return FORM == 0 && (r / (TN * 8)) % 2 == 1; }, K, count, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN, lr = lane & 15, lg = lane >> 4;
@@ -562,11 +559,13 @@ static int launch_direct(const __bf16* in, long long in_rows, long long ldi, con
   return 0;
 }
 
-// Tiles of 128 x 128 outputs (two workgroups a CU) or 256 x 256 (one): moe_tile_rows in ops/kernels.py chooses.  Tiles of
+// Tiles of 128 x 128 or 192 x 128 outputs (two workgroups a CU; the second's stages are all of its LDS, so that lanes find their rows
+// themselves) or 256 x 256 (one): moe_tile_rows in ops/kernels.py chooses.  Tiles of
 // 320 x 128 were measured too: the fastest where 256 pairs fall to every expert alike (2,048 tokens 180 us against 204 with the
 // weighted sum), the slowest as soon as the experts differ (239 to 247 against 198 to 205), so they are not in.
 template <int FORM, typename... Args>
 static int launch_direct_tiles(int tile_rows, Args... args) {
+  if (tile_rows == GT_MIDDLE) return launch_direct<FORM, GT_MIDDLE, 128, 4, 2, 2>(args...);
   if (tile_rows == GT_WIDE) return launch_direct<FORM, GT_WIDE, 256, 2, 4, 2>(args...);
   return launch_direct<FORM, GT_TILE, 128, 2, 4, 2>(args...);
 }
@@ -718,7 +717,7 @@ extern "C" int vk_moe_max_tiles(int pairs, int experts, int tile_rows) {
   return (pairs + tile_rows - 1) / tile_rows + (experts < pairs ? experts : pairs);
 }
 
-// Whether the products of these operands run on the matrix cores (tiles of 128 or 16 places) or as 32-bit FMAs (64).
+// Whether the products of these operands run on the matrix cores (tiles of 128 and more or 16 places) or as 32-bit FMAs (64).
 static inline bool moe_on_matrix_cores(int dtype, int width, int ff, long long ldh) {
   return dtype == DT_BF16 && width % 8 == 0 && ff % 8 == 0 && ldh % 8 == 0;
 }
@@ -732,7 +731,7 @@ static inline bool moe_loads_direct(int width, int ff, int num_tokens, int top, 
 extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int groups, int keep,
                             int all_scores, const float* correction, float weight_scale, long long ld, int* ids,
                             float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
-  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE)
+  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE && tile_rows != GT_MIDDLE)
     return VK_BAD_ARGUMENT;
   if (groups < 1 || keep < 1 || keep > groups || experts % groups != 0) return VK_BAD_ARGUMENT;
   if (groups > WAVE) return VK_UNSUPPORTED_SIZE;
@@ -803,7 +802,7 @@ extern "C" int vk_moe_experts(const void* h, long long ldh, const void* wg, cons
       __bf16* a = (__bf16*)act;
       const int max_tiles = vk_moe_max_tiles(pairs, experts, tile_rows);
       int status;
-      if (tile_rows != GT_TILE && tile_rows != GT_WIDE) return VK_BAD_ARGUMENT;
+      if (tile_rows != GT_TILE && tile_rows != GT_MIDDLE && tile_rows != GT_WIDE) return VK_BAD_ARGUMENT;
       if (plain)
         status = launch_direct_tiles<1>(tile_rows, x, (long long)num_tokens, ldh, u, u, offsets, order, tiles, num_tiles, max_tiles,
                                         top, width, ff, limit, alpha, plain, in_weights, a, (float*)nullptr, s);

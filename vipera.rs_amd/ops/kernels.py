@@ -1419,14 +1419,20 @@ MOE_STREAM_PAIRS = 10     # pairs per expert, on average, up to which the expert
 
 def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int, gated: bool = True) -> int:
     """Places per tile of the experts' products for activations ``h`` of ``pairs`` (token, choice) pairs: on the matrix cores
-    (bfloat16, widths that are multiples of 8) 128 or 256, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The
+    (bfloat16, widths that are multiples of 8) 128, 192 or 256, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The
     grouping has to be made for the same number.
 
     With widths in whole steps of 64 the tiles are 128 x 128 outputs (two workgroups a CU) or 256 x 256 (one), and a chip full
     of the second takes 1.6 times as long as one of the first (32 experts of 1,024 x 2,048, gate and up: 60 against 37 us, down
     37 against 23).  Experts are taken to fill their last tile to a half, as they do when tokens prefer some of them:
     3,000 tokens, top 4 of 32, products and sum 267 us in tiles of 128, 217 to 231 in 256 (282 where half the tokens choose
-    one expert); 2,048 tokens 198 to 205 and 206 to 214; 1,383 tokens 150 to 164 and 133 (all experts alike) to 192."""
+    one expert); 2,048 tokens 198 to 205 and 206 to 214; 1,383 tokens 150 to 164 and 133 (all experts alike) to 192.
+
+    192 where 216 to 288 pairs fall to an expert: two tiles of 192 x 128 instead of two or three of 128 x 128, two workgroups a CU as
+    these, whole rounds less (32 experts of 1,024 x 2,048, products and sum in tiles of 128 and 192: 2,048 tokens 204 and 202 us, without
+    a gate 163 and 150; in a medium Gilidra's prompt of 2,048 tokens 17 us a layer).  A tile takes up to 1.4 times as long, so that outside of
+    these it loses (1,400 tokens 168 and 184, 2,500 without a gate 183 and 191), or gains where some experts just pass 128 pairs, which
+    is not known here (512 tokens 143 and 119, and 99 and 102 where none does)."""
     if not (h.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and h.stride(0) % 8 == 0):
         return 64
     if pairs <= MOE_STREAM_PAIRS * experts:
@@ -1440,7 +1446,9 @@ def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int
         fills = lambda n: max(1.0, tiles * -(-n // columns) / slots)
         return fills(2 * ff if gated else ff) * width + fills(width) * ff
 
-    return 256 if 1.6 * cost(256, 256, 256) < 0.95 * cost(128, 128, 512) else 128
+    if 1.6 * cost(256, 256, 256) < 0.95 * cost(128, 128, 512):
+        return 256
+    return 192 if 216 * experts <= pairs <= 288 * experts else 128
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 64) -> int:
@@ -1467,7 +1475,7 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     _f32(weights, "moe_route: weights")
     _need(ids.numel() == tokens * top and weights.numel() == tokens * top and order.numel() == tokens * top
           and offsets.numel() == experts + 1 and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and num_tiles.numel() == 1 and tile_rows in (16, 64, 128, 256), "moe_route: output sizes")
+          and num_tiles.numel() == 1 and tile_rows in (16, 64, 128, 192, 256), "moe_route: output sizes")
     _need(1 <= keep <= groups <= 64 and experts % groups == 0 and (keep == groups or keep * (experts // groups) >= top),
           f"moe_route: {keep} of {groups} groups of {experts} experts for top {top}")
     mode = {"sigmoid": 2, "steered": 3}.get(all_scores, 1 if all_scores else 0)
@@ -1521,7 +1529,7 @@ def moe_experts(h: torch.Tensor, w_gate: Optional[torch.Tensor], w_up: torch.Ten
     _i32(offsets, order, tiles, num_tiles)
     _need(offsets.numel() == experts + 1 and order.numel() == tokens * top
           and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, 128, 256),
+          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, 128, 192, 256),
           "moe_experts: grouping (made by moe_route with the tile_rows that moe_tile_rows gives)")
     fn = _fn("moe", "vk_moe_experts", [_p, _ll, _p, _p, _p, _i, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f, _f, _i, _p, _p,
                                        _p, _i, _i, _p, _p, _ll, _p, _p])
