@@ -279,7 +279,9 @@ def test_a_plan_of_one_range_is_carried_out_with_the_same_bits(m, n, k, tiling):
 
 
 @pytest.mark.parametrize("m,n,k,tiling,before,cut", [(1396, 1536, 8960, 20, 6, 4), (1201, 896, 4864, 18, 7, 4), (400, 900, 4864, 17, 9, 8),
-                                                     (311, 3584, 4736, 18, 9, 4), (400, 4608, 3584, 18, 7, 2), (130, 5120, 13824, 20, 6, 8)])
+                                                     (311, 3584, 4736, 18, 9, 4), (400, 4608, 3584, 18, 7, 2), (130, 5120, 13824, 20, 6, 8),
+                                                     (311, 1024, 4096, 16, 13, 8), (200, 1530, 8960, 17, 13, 8), (622, 1536, 8960, 17, 14, 4),
+                                                     (130, 3580, 3584, 16, 14, 4)])
 def test_a_plan_of_several_ranges_is_carried_out_with_the_same_bits(m, n, k, tiling, before, cut):
     """The tile that is picked and the one of the estimate by whole rounds, with the same cut of K; results of either kind."""
     from vipera_rs_amd.ops import kernels

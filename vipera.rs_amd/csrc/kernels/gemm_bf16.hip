@@ -2086,22 +2086,37 @@ int whole_tile(int planned, int M, int N, int K, double output_bytes) {
 // 29.9 / 25.2, 311 on 3,584 of 18,944 81.1 / 61.5, 400 on 4,608 of 3,584 35.7 / 30.1, 1,200 on 2,048 of 4,096 38.9 / 34.3. The cut of K
 // stays as it was, and so do the bits. A plan of tiles of 256 tokens names the tile that is picked; 128x128 tiles are asked for
 // where they carry the plan out, in four ranges or more.
-int split_tile(int planned, int M, int N, int K, int ranges) {
-  int best = planned;
-  double best_us = -1;
-  for (const TileCost& t : WHOLE_TILES)
-    if (t.config == planned) best_us = 0.98 * whole_tile_us(t, M, N, K, 4.0, ranges);
-  if (best_us < 0) return planned;
+int one_round_tile(int planned, double limit_us, int M, int N, int K, int ranges, bool narrow) {
   for (const TileCost& t : WHOLE_TILES) {
-    if (t.config != 17 && t.config != 18 && t.config != 20) continue;
+    if (t.config != 17 && t.config != 18 && t.config != 20 && !(narrow && t.config == 16)) continue;
     if ((long long)((M + t.tokens - 1) / t.tokens) * ((N + t.rows - 1) / t.rows) * ranges > g_compute_units) continue;
     const double us = whole_tile_us(t, M, N, K, 4.0, ranges);
-    if (us < best_us) {
-      best_us = us;
-      best = t.config;
+    if (us < limit_us) {
+      limit_us = us;
+      planned = t.config;
     }
   }
-  return best;
+  return planned;
+}
+int split_tile(int planned, int M, int N, int K, int ranges) {
+  for (const TileCost& t : WHOLE_TILES)
+    if (t.config == planned) return one_round_tile(planned, 0.98 * whole_tile_us(t, M, N, K, 4.0, ranges), M, N, K, ranges, false);
+  return planned;
+}
+
+// The same where 64x64 tiles were to carry several ranges out, with 192x64 among those offered: in place of split ones (13) that
+// are more than two a CU, and of ones that walk K (14) where the estimate with the sums' way through memory and a second launch is below
+// 0.95 of the walk's (2.5 us and 0.27 a step of 64). Of 101 products planned as small tiles 18 change, to 0.88 of their time, 0.94 at worst:
+// us, 130 tokens on 2,048 rows of 8,192 22.1 / 18.2, 311 on 2,048 of 4,096 22.3 / 18.2, 622 on 896 of 4,864 21.5 / 18.3, and walked 622 on
+// 1,536 of 8,960 40.4 / 32.9, 512 on 2,048 of 8,192 35.2 / 29.6. Up to two a CU the split small tiles stay ahead by 4 to 15 %.
+int split_small_tile(int planned, int M, int N, int K, int ranges) {
+  const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  if (planned == 13 && small * ranges > 2LL * g_compute_units) return one_round_tile(13, 1e30, M, N, K, ranges, true);
+  if (planned == 14) {
+    const double sums = (2.0 * ranges + 1.0) * 4.0 * M * N / 6e6 + 3.0;
+    return one_round_tile(14, 0.95 * (2.5 + 0.27 * (K / 64)) - sums, M, N, K, ranges, true);
+  }
+  return planned;
 }
 
 // The gated product of up to 64 tokens: tiles of 64 tokens and of the fewest weight rows with which every tile finds a CU; past
@@ -2143,7 +2158,9 @@ TilePlan carried_out(int M, int N, int K, long long partial_floats, bool gated, 
     ++g_tile_launched.plans;
     TilePlan plan = tile_plan(M, N, K, (long long)most_ranges * M * N, gated, scaled);
     if ((K & 63) == 0 && M > 128 && plan.ranges == 1 && !scaled) plan.config = whole_tile(plan.config, M, N, K, output_bytes);
-    if ((K & 63) == 0 && M > 128 && plan.ranges >= 4 && plan.config == 9 && !scaled) plan.config = split_tile(9, M, N, K, plan.ranges);
+    if ((K & 63) == 0 && M > 128 && plan.ranges > 1 && !scaled)
+      plan.config = plan.config != 9 ? split_small_tile(plan.config, M, N, K, plan.ranges)
+                    : plan.ranges >= 4 ? split_tile(9, M, N, K, plan.ranges) : 9;
     if ((K & 63) == 0 && M <= 64 && gated) plan.config = few_tokens_tile(N);
     kept = Kept{M, N, K, form, plan};
   }
