@@ -779,9 +779,24 @@ def test_experts_in_tiles_of_192_places_give_the_bits_of_128(tokens, width, ff, 
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
-def test_tiles_of_192_places_are_for_216_to_288_pairs_an_expert():
+@pytest.mark.parametrize("counts, columns, want", [
+    ((128,) * 32, (2048, 2048), 128),              # one round of either
+    ((129,) + (50,) * 31, (2048, 2048), 192),      # a second round for one pair, where 192 places are one
+    ((193,) + (50,) * 31, (2048, 2048), 128),      # two rounds of either
+    ((256,) * 16 + (257,) * 16, (2048, 2048), 192), ((0, 300, 129, 0, 128, 1), (512, 320), 128),
+    ((129,) + (50,) * 40, (1024, 1024), 128), ((129,) * 70, (1024, 512), 192), ((100,) * 70, (1024, 512), 128), ((129,) * 64, (1024, 1024), 192)])
+def test_pairs_are_grouped_in_the_tiles_of_fewer_rounds(counts, columns, want):
+    """Two workgroups a CU, of 256; every choice of every token is given, top 1."""
     from vipera_rs_amd.ops import kernels
 
-    rows = lambda tokens, gated=True: kernels.moe_tile_rows(torch.empty(tokens, 2048, dtype=torch.bfloat16, device="cuda"), 2048, 1024, 4 * tokens, 32, gated)
-    assert [rows(n) for n in (1400, 1727, 1728, 2048)] == [128, 128, 192, 192] and rows(3000) == 256
-    assert [rows(n, False) for n in (1727, 1728, 2304, 2305)] == [128, 192, 192, 128]
+    experts, pairs = len(counts), sum(counts)
+    chosen = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(pairs)]
+    z = torch.nn.functional.one_hot(chosen, experts).float().cuda()
+    i32 = lambda n: torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    rows = kernels.MOE_EITHER_ROWS
+    ids, offsets, order, tiles, count = i32(pairs), i32(experts + 1), i32(pairs), i32(2 * kernels.moe_max_tiles(pairs, experts, rows)), i32(1)
+    kernels.moe_route(z, 1, ids, torch.empty(pairs, device="cuda"), offsets, order, tiles, count, rows, columns=columns)
+    edges = np.cumsum([0, *counts])
+    listed = [(e, edges[e] + i) for e in range(experts) for i in range(0, counts[e], want)]
+    assert count.item() == len(listed) | (1 << 30 if want == 192 else 0)
+    assert tiles.view(-1, 2)[:len(listed)].tolist() == [list(map(int, t)) for t in listed]

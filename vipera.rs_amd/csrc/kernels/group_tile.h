@@ -104,6 +104,7 @@ __device__ __forceinline__ void group_tile_mma(ARow a_row, WRow w_row, int K, un
 // Every row's place is a byte offset of its own, so rows may be gathered; a row that does not exist has GT_NO_ROW and
 // reads zero without touching memory.
 constexpr int GT_MIDDLE = 192, GT_WIDE = 256;                    // rows of activations of its larger tiles
+constexpr int GT_EITHER = 96;                                    // in a tile's place: 128 or 192, as the groups' sizes say
 constexpr unsigned GT_NO_ROW = 0x80000000u;                      // past the end of every view; so are the steps behind it
 constexpr long long GT_VIEW_BYTES = 0x7fffffffll;                // views are shorter than GT_NO_ROW
 

@@ -154,13 +154,28 @@ __device__ __forceinline__ int running_sum(int v) {
   return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
 }
 
+// Rounds of workgroups that so many tiles are in the experts' two products, two a CU; column blocks of the products.
+struct Rounds {
+  int up, down;
+  __device__ __forceinline__ long long of(int tiles) const {
+    constexpr int AT_ONCE = 512;
+    return ((long long)tiles * up + AT_ONCE - 1) / AT_ONCE + ((long long)tiles * down + AT_ONCE - 1) / AT_ONCE;
+  }
+};
+constexpr int TILES_OF_192 = 1 << 30;     // in num_tiles: the tiles are of 192 places
+
 // One workgroup: counts per expert, offsets, the pairs' places, and the list of tiles.
-//   offsets [E + 1], order [P], tiles [max_tiles][2] = (expert, first place), num_tiles [1]
+//   offsets [E + 1], order [P], tiles [max_tiles][2] = (expert, first place), num_tiles [1] (with TILES_OF_192)
+// tile_rows GT_EITHER: tiles of 192 places where these are fewer rounds of workgroups than those of 128. A round of the wider
+// ones takes some 1.15 times as long where an expert has one tile and up to 1.4 times with full ones, and one of them that is
+// hardly begun as long as a full one. us, products and sum of 32 experts of 1,024 x 2,048 in tiles of 128 and 192: 512 tokens of which the
+// favourite expert has more than 128 143 and 119, none 99 and 102; 1,400 (as many rounds) 168 and 184; 2,048 204 and 202; without a gate 1,700
+// 156 and 142, 2,500 (as many) 183 and 191; 16 experts of 512 x 1,024, 2,000 tokens 76 and 63.
 // With `logits`: the same workgroup routes the step's tokens first, a wave per token in turn (a step of few tokens:
 // one launch instead of two).
 __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict__ logits, int top, int num_tokens,
                                                          float* __restrict__ weights, int* __restrict__ ids, int pairs,
-                                                         int experts, int tile_rows, int* __restrict__ offsets,
+                                                         int experts, int tile_rows, Rounds rounds, int* __restrict__ offsets,
                                                          int* __restrict__ order, int* __restrict__ tiles,
                                                          int* __restrict__ num_tiles, Routing how) {
   extern __shared__ int shared[];      // counts [E], cursor [E]
@@ -179,11 +194,34 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
   if (threadIdx.x < WAVE) {          // one wave: running sums over the experts, 64 at a time
     const int lane = threadIdx.x;
     int at = 0, tile = 0;
+    // up to 64 experts the choice falls out of the sums below, both kinds of tiles in one number
+    if (tile_rows == GT_EITHER && (experts > WAVE || pairs > 8000000)) {
+      int narrow = 0, wide = 0;
+      for (int base = 0; base < experts; base += WAVE) {
+        const int e = base + lane, count = e < experts ? counts[e] : 0;
+        narrow += (count + GT_TILE - 1) / GT_TILE;
+        wide += (count + GT_MIDDLE - 1) / GT_MIDDLE;
+      }
+      narrow = __shfl(running_sum(narrow), WAVE - 1, WAVE);
+      wide = __shfl(running_sum(wide), WAVE - 1, WAVE);
+      tile_rows = rounds.of(wide) < rounds.of(narrow) ? GT_MIDDLE : GT_TILE;
+    }
     for (int base = 0; base < experts; base += WAVE) {
-      const int e = base + lane, count = e < experts ? counts[e] : 0, own = (count + tile_rows - 1) / tile_rows;
-      int places = count, tiles_upto = own;
-      places = running_sum(places);
-      tiles_upto = running_sum(tiles_upto);
+      const int e = base + lane, count = e < experts ? counts[e] : 0;
+      const int places = running_sum(count);
+      int own, tiles_upto;
+      if (tile_rows == GT_EITHER) {
+        own = (count + GT_TILE - 1) / GT_TILE | (count + GT_MIDDLE - 1) / GT_MIDDLE << 16;
+        tiles_upto = running_sum(own);
+        const unsigned all = (unsigned)__shfl(tiles_upto, WAVE - 1, WAVE);
+        const int part = rounds.of((int)(all >> 16)) < rounds.of((int)(all & 0xffff)) ? 16 : 0;
+        tile_rows = part ? GT_MIDDLE : GT_TILE;
+        own = (int)((unsigned)own >> part & 0xffff);
+        tiles_upto = (int)((unsigned)tiles_upto >> part & 0xffff);
+      } else {
+        own = (count + tile_rows - 1) / tile_rows;
+        tiles_upto = running_sum(own);
+      }
       if (e < experts) {
         const int first = at + places - count;
         offsets[e] = first;
@@ -198,7 +236,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
     }
     if (lane == 0) {
       offsets[experts] = at;
-      num_tiles[0] = tile;
+      num_tiles[0] = tile | (tile_rows == GT_MIDDLE ? TILES_OF_192 : 0);
     }
   }
   __syncthreads();
@@ -237,7 +275,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ 
                                                           const int* __restrict__ num_tiles, int top, int width, int ff,
                                                           float limit, float alpha, int plain,
                                                           const float* __restrict__ in_weights, T* __restrict__ act) {
-  if ((int)blockIdx.x >= num_tiles[0]) return;
+  if ((int)blockIdx.x >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   __shared__ float As[16][MOE_TILE + 4];
   __shared__ float Gs[GATED ? 16 : 1][MOE_TILE + 4];
   __shared__ float Us[16][MOE_TILE + 4];
@@ -301,7 +339,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ act
                                                        const int* __restrict__ offsets, const int* __restrict__ order,
                                                        const int* __restrict__ tiles, const int* __restrict__ num_tiles,
                                                        int width, int ff, float* __restrict__ pair_out) {
-  if ((int)blockIdx.x >= num_tiles[0]) return;
+  if ((int)blockIdx.x >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   __shared__ float As[16][MOE_TILE + 4];
   __shared__ float Ws[16][MOE_TILE + 4];
   const int e = tiles[2 * blockIdx.x], first = tiles[2 * blockIdx.x + 1];
@@ -358,7 +396,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_mma_kernel(const __bf16* __re
                                                               int ff, float limit, float alpha,
                                                               const float* __restrict__ in_weights,
                                                               __bf16* __restrict__ act) {
-  if ((int)blockIdx.x >= num_tiles[0]) return;
+  if ((int)blockIdx.x >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   __shared__ int rows[GT_TILE];
   const int e = tiles[2 * blockIdx.x], first = tiles[2 * blockIdx.x + 1];
@@ -402,7 +440,7 @@ __global__ __launch_bounds__(256) void moe_up_mma_kernel(const __bf16* __restric
                                                          const int* __restrict__ num_tiles, int top, int width, int ff,
                                                          int plain, const float* __restrict__ in_weights,
                                                          __bf16* __restrict__ act) {
-  if ((int)blockIdx.x >= num_tiles[0]) return;
+  if ((int)blockIdx.x >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   __shared__ int rows[GT_TILE];
   const int e = tiles[2 * blockIdx.x], first = tiles[2 * blockIdx.x + 1];
@@ -438,7 +476,7 @@ __global__ __launch_bounds__(256) void moe_down_mma_kernel(const __bf16* __restr
                                                            const int* __restrict__ tiles,
                                                            const int* __restrict__ num_tiles, int width, int ff,
                                                            float* __restrict__ pair_out) {
-  if ((int)blockIdx.x >= num_tiles[0]) return;
+  if ((int)blockIdx.x >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int e = tiles[2 * blockIdx.x], first = tiles[2 * blockIdx.x + 1];
   const int count = min(GT_TILE, offsets[e + 1] - first);
@@ -480,16 +518,14 @@ __global__ __launch_bounds__(256) void moe_down_mma_kernel(const __bf16* __restr
 // through one L2.  Grid (a multiple of eight at or above the tiles there can be, column blocks): a row of the grid holds a column
 // block's share of every XCD, so that the numbers run on from row to row.  In one row they passed the 2^32 threads that a launch takes.
 template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
-__global__ __launch_bounds__(WM* WN * 64, (2 * gt_direct_lds<BM, BN, STAGES>() <= 160 * 1024 ? WM * WN / 2 : WM * WN / 4)) void moe_direct_kernel(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
-                                                                 const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
-                                                                 const int* __restrict__ offsets,
-                                                                 const int* __restrict__ order, const int* __restrict__ tiles,
-                                                                 const int* __restrict__ num_tiles, int top, int K, int N,
-                                                                 float limit, float alpha, int plain,
-                                                                 const float* __restrict__ in_weights,
-                                                                 __bf16* __restrict__ act, float* __restrict__ pair_out) {
+__device__ __forceinline__ void moe_direct_tile(const __bf16* __restrict__ in, long long in_bytes, long long ldi,
+                                                const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
+                                                const int* __restrict__ offsets, const int* __restrict__ order,
+                                                const int* __restrict__ tiles, int count_tiles, int top, int K, int N, float limit,
+                                                float alpha, int plain, const float* __restrict__ in_weights,
+                                                __bf16* __restrict__ act, float* __restrict__ pair_out) {
   constexpr int COLUMNS = FORM == 0 ? BN / 2 : BN, TM = BM / WM / 16, TN = BN / WN / 16;
-  const int blocks = (N + COLUMNS - 1) / COLUMNS, count_tiles = num_tiles[0];
+  const int blocks = (N + COLUMNS - 1) / COLUMNS;
   const int xcd = blockIdx.x & 7, at = (blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3);
   const int t0 = (int)((long long)count_tiles * xcd / 8), own = (int)((long long)count_tiles * (xcd + 1) / 8) - t0;
   if (at >= own * blocks) return;
@@ -536,38 +572,48 @@ __global__ __launch_bounds__(WM* WN * 64, (2 * gt_direct_lds<BM, BN, STAGES>() <
   }
 }
 
-template <int FORM, int BM, int BN, int WM, int WN, int STAGES>
-static int launch_direct(const __bf16* in, long long in_rows, long long ldi, const __bf16* w0, const __bf16* w1,
-                         const int* offsets, const int* order, const int* tiles, const int* num_tiles, int max_tiles, int top,
-                         int K, int N, float limit, float alpha, int plain, const float* in_weights, __bf16* act,
-                         float* pair_out, hipStream_t s) {
-  constexpr int COLUMNS = FORM == 0 ? BN / 2 : BN, lds_bytes = gt_direct_lds<BM, BN, STAGES>();
-  static bool sized = false;
-  if (!sized) {
-    const hipError_t e = hipFuncSetAttribute((const void*)moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) return (int)e;
-    sized = true;
-  }
-  // an XCD has at most ceil(tiles / 8) of the tiles, whatever their number turns out to be
-  const dim3 grid(8 * ((max_tiles + 7) / 8), (N + COLUMNS - 1) / COLUMNS);
-  if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
-  moe_direct_kernel<FORM, BM, BN, WM, WN, STAGES><<<grid, WM * WN * 64, lds_bytes, s>>>(
-      in, ((in_rows - 1) * ldi + K) * 2, ldi, w0, w1, offsets, order, tiles, num_tiles, top, K, N, limit, alpha, plain, in_weights,
-      act, pair_out);
-  VK_LAUNCH_CHECK();
-  return 0;
-}
-
-// Tiles of 128 x 128 or 192 x 128 outputs (two workgroups a CU; the second's stages are all of its LDS, so that lanes find their rows
-// themselves) or 256 x 256 (one): moe_tile_rows in ops/kernels.py chooses.  Tiles of
+// Tiles of 128 x 128 or 192 x 128 outputs, as the grouping has them (two workgroups a CU; the wider one's stages are all of its LDS, so
+// that lanes find their rows themselves), or 256 x 256 (one): moe_tile_rows in ops/kernels.py chooses.  Tiles of
 // 320 x 128 were measured too: the fastest where 256 pairs fall to every expert alike (2,048 tokens 180 us against 204 with the
 // weighted sum), the slowest as soon as the experts differ (239 to 247 against 198 to 205), so they are not in.
-template <int FORM, typename... Args>
-static int launch_direct_tiles(int tile_rows, Args... args) {
-  if (tile_rows == GT_MIDDLE) return launch_direct<FORM, GT_MIDDLE, 128, 4, 2, 2>(args...);
-  if (tile_rows == GT_WIDE) return launch_direct<FORM, GT_WIDE, 256, 2, 4, 2>(args...);
-  return launch_direct<FORM, GT_TILE, 128, 2, 4, 2>(args...);
+template <int FORM, bool WIDE>
+__global__ __launch_bounds__(512, WIDE ? 2 : 4) void moe_direct_kernel(
+    const __bf16* __restrict__ in, long long in_bytes, long long ldi, const __bf16* __restrict__ w0, const __bf16* __restrict__ w1,
+    const int* __restrict__ offsets, const int* __restrict__ order, const int* __restrict__ tiles, const int* __restrict__ num_tiles,
+    int top, int K, int N, float limit, float alpha, int plain, const float* __restrict__ in_weights, __bf16* __restrict__ act,
+    float* __restrict__ pair_out) {
+  const int listed = num_tiles[0], count = listed & (TILES_OF_192 - 1);
+#define VK_TILE(BM, BN, WM, WN)                                                                                        \
+  moe_direct_tile<FORM, BM, BN, WM, WN, 2>(in, in_bytes, ldi, w0, w1, offsets, order, tiles, count, top, K, N, limit, alpha, plain, \
+                                           in_weights, act, pair_out)
+  if constexpr (WIDE) VK_TILE(GT_WIDE, 256, 2, 4);
+  else if (listed & TILES_OF_192) VK_TILE(GT_MIDDLE, 128, 4, 2);
+  else VK_TILE(GT_TILE, 128, 2, 4);
+#undef VK_TILE
+}
+
+template <int FORM>
+static int launch_direct_tiles(int tile_rows, const __bf16* in, long long in_rows, long long ldi, const __bf16* w0, const __bf16* w1,
+                               const int* offsets, const int* order, const int* tiles, const int* num_tiles, int max_tiles, int top,
+                               int K, int N, float limit, float alpha, int plain, const float* in_weights, __bf16* act,
+                               float* pair_out, hipStream_t s) {
+  const bool wide = tile_rows == GT_WIDE;
+  const int columns = (wide ? 256 : 128) / (FORM == 0 ? 2 : 1);
+  constexpr int wide_bytes = gt_direct_lds<GT_WIDE, 256, 2>(), bytes = gt_direct_lds<GT_MIDDLE, 128, 2>();
+  const auto kernel = wide ? &moe_direct_kernel<FORM, true> : &moe_direct_kernel<FORM, false>;
+  static bool sized[2] = {false, false};
+  if (!sized[wide]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, wide ? wide_bytes : bytes);
+    if (e != hipSuccess) return (int)e;
+    sized[wide] = true;
+  }
+  // an XCD has at most ceil(tiles / 8) of the tiles, whatever their number turns out to be
+  const dim3 grid(8 * ((max_tiles + 7) / 8), (N + columns - 1) / columns);
+  if (grid.y > 65535) return VK_UNSUPPORTED_SIZE;
+  kernel<<<grid, 512, wide ? wide_bytes : bytes, s>>>(in, ((in_rows - 1) * ldi + K) * 2, ldi, w0, w1, offsets, order, tiles, num_tiles, top,
+                                                      K, N, limit, alpha, plain, in_weights, act, pair_out);
+  VK_LAUNCH_CHECK();
+  return 0;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -585,7 +631,7 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const __bf16* __restric
                                                          int top, int K, int N, float limit, float alpha, int plain,
                                                          const float* __restrict__ in_weights, __bf16* __restrict__ act,
                                                          float* __restrict__ pair_out) {
-  if ((int)blockIdx.y >= num_tiles[0]) return;
+  if ((int)blockIdx.y >= (num_tiles[0] & (TILES_OF_192 - 1))) return;
   __shared__ gt_f32x4 part[4][2][WAVE];
   const int e = tiles[2 * blockIdx.y], first = tiles[2 * blockIdx.y + 1];
   const int count = min(MOE_FEW, offsets[e + 1] - first);
@@ -728,10 +774,13 @@ static inline bool moe_loads_direct(int width, int ff, int num_tokens, int top, 
          (long long)num_tokens * top * ff * 2 <= GT_VIEW_BYTES && (long long)width * ff * 2 <= GT_VIEW_BYTES;
 }
 
-extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int groups, int keep,
+// up_blocks, down_blocks: column blocks of the experts' products in tiles of 128 columns, for tile_rows GT_EITHER.
+extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int up_blocks,
+                            int down_blocks, int groups, int keep,
                             int all_scores, const float* correction, float weight_scale, long long ld, int* ids,
                             float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
-  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE && tile_rows != GT_MIDDLE)
+  if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE && tile_rows != GT_MIDDLE &&
+      (tile_rows != GT_EITHER || up_blocks < 1 || down_blocks < 1))
     return VK_BAD_ARGUMENT;
   if (groups < 1 || keep < 1 || keep > groups || experts % groups != 0) return VK_BAD_ARGUMENT;
   if (groups > WAVE) return VK_UNSUPPORTED_SIZE;
@@ -751,7 +800,7 @@ extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_t
     VK_LAUNCH_CHECK();
   }
   moe_group_kernel<<<1, 1024, (size_t)experts * 2 * sizeof(int), s>>>(together ? logits : nullptr, top, num_tokens,
-                                                                       weights, ids, (int)pairs, experts, tile_rows,
+                                                                       weights, ids, (int)pairs, experts, tile_rows, Rounds{up_blocks, down_blocks},
                                                                        offsets, order, tiles, num_tiles, how);
   VK_LAUNCH_CHECK();
   return 0;
@@ -800,9 +849,9 @@ extern "C" int vk_moe_experts(const void* h, long long ldh, const void* wg, cons
     if (moe_loads_direct(width, ff, num_tokens, top, ldh)) {
       const __bf16 *x = (const __bf16*)h, *g = (const __bf16*)wg, *u = (const __bf16*)wu, *d = (const __bf16*)wd;
       __bf16* a = (__bf16*)act;
-      const int max_tiles = vk_moe_max_tiles(pairs, experts, tile_rows);
+      const int max_tiles = vk_moe_max_tiles(pairs, experts, tile_rows == GT_EITHER ? GT_TILE : tile_rows);
       int status;
-      if (tile_rows != GT_TILE && tile_rows != GT_MIDDLE && tile_rows != GT_WIDE) return VK_BAD_ARGUMENT;
+      if (tile_rows != GT_TILE && tile_rows != GT_MIDDLE && tile_rows != GT_EITHER && tile_rows != GT_WIDE) return VK_BAD_ARGUMENT;
       if (plain)
         status = launch_direct_tiles<1>(tile_rows, x, (long long)num_tokens, ldh, u, u, offsets, order, tiles, num_tiles, max_tiles,
                                         top, width, ff, limit, alpha, plain, in_weights, a, (float*)nullptr, s);

@@ -1414,6 +1414,7 @@ def head_linear(a: torch.Tensor, a_head_stride: int, k: int, w: torch.Tensor, ou
 
 
 # --- mixture of experts ---------------------------------------------------------------------------
+MOE_EITHER_ROWS = 96      # in the place of a tile's rows: 128 or 192, as the experts' counts say
 MOE_STREAM_PAIRS = 10     # pairs per expert, on average, up to which the experts' products are streams of the weights
 
 
@@ -1428,11 +1429,8 @@ def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int
     3,000 tokens, top 4 of 32, products and sum 267 us in tiles of 128, 217 to 231 in 256 (282 where half the tokens choose
     one expert); 2,048 tokens 198 to 205 and 206 to 214; 1,383 tokens 150 to 164 and 133 (all experts alike) to 192.
 
-    192 where 216 to 288 pairs fall to an expert: two tiles of 192 x 128 instead of two or three of 128 x 128, two workgroups a CU as
-    these, whole rounds less (32 experts of 1,024 x 2,048, products and sum in tiles of 128 and 192: 2,048 tokens 204 and 202 us, without
-    a gate 163 and 150; in a medium Gilidra's prompt of 2,048 tokens 17 us a layer).  A tile takes up to 1.4 times as long, so that outside of
-    these it loses (1,400 tokens 168 and 184, 2,500 without a gate 183 and 191), or gains where some experts just pass 128 pairs, which
-    is not known here (512 tokens 143 and 119, and 99 and 102 where none does)."""
+    Instead of 128 the answer is :data:`MOE_EITHER_ROWS` there: the grouping takes tiles of 192 x 128 outputs, two workgroups a CU as
+    well, where they are fewer rounds of workgroups than those of 128 x 128, which it sees from the experts' counts."""
     if not (h.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and h.stride(0) % 8 == 0):
         return 64
     if pairs <= MOE_STREAM_PAIRS * experts:
@@ -1446,9 +1444,7 @@ def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int
         fills = lambda n: max(1.0, tiles * -(-n // columns) / slots)
         return fills(2 * ff if gated else ff) * width + fills(width) * ff
 
-    if 1.6 * cost(256, 256, 256) < 0.95 * cost(128, 128, 512):
-        return 256
-    return 192 if 216 * experts <= pairs <= 288 * experts else 128
+    return 256 if 1.6 * cost(256, 256, 256) < 0.95 * cost(128, 128, 512) else MOE_EITHER_ROWS
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 64) -> int:
@@ -1458,14 +1454,15 @@ def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 64) -> int:
 def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.Tensor, offsets: torch.Tensor,
               order: torch.Tensor, tiles: torch.Tensor, num_tiles: torch.Tensor, tile_rows: int = 64,
               groups: int = 1, keep: int = 1, all_scores=False, correction: Optional[torch.Tensor] = None,
-              weight_scale: float = 1.0) -> None:
+              weight_scale: float = 1.0, columns: Tuple[int, int] = (0, 0)) -> None:
     """Each token's ``top`` largest router logits (lowest id first among equals) with the softmax over those, and the
     (token, choice) pairs grouped by expert: ``offsets [E + 1]``, ``order [T * top]``, ``tiles [max, 2]``.
     ``groups`` > 1: the experts form that many equal groups of neighbours and only those of the ``keep`` groups with
     the largest logits can be chosen.  ``all_scores``: the weights are the chosen experts' shares of the softmax over
     all experts (they do not add up to one); ``all_scores="sigmoid"``: the weight of a chosen expert is the sigmoid of its
     own logit, not renormalized; ``all_scores="steered"``: the experts are chosen by ``sigmoid(logit) + correction[e]``
-    (``correction`` [experts] 32-bit or None) and a chosen expert's weight is ``weight_scale * sigmoid(logit)``."""
+    (``correction`` [experts] 32-bit or None) and a chosen expert's weight is ``weight_scale * sigmoid(logit)``.  ``columns``: the weight
+    rows of the experts' two products (gate and up both), for ``tile_rows`` :data:`MOE_EITHER_ROWS`."""
     _dev(logits, ids, weights, offsets, order, tiles, num_tiles)
     tokens, experts = logits.shape
     _f32s(logits, "moe_route: logits")      # rows may lie further apart than they are long (a view of some columns)
@@ -1475,7 +1472,7 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     _f32(weights, "moe_route: weights")
     _need(ids.numel() == tokens * top and weights.numel() == tokens * top and order.numel() == tokens * top
           and offsets.numel() == experts + 1 and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and num_tiles.numel() == 1 and tile_rows in (16, 64, 128, 192, 256), "moe_route: output sizes")
+          and num_tiles.numel() == 1 and tile_rows in (16, 64, MOE_EITHER_ROWS, 128, 192, 256), "moe_route: output sizes")
     _need(1 <= keep <= groups <= 64 and experts % groups == 0 and (keep == groups or keep * (experts // groups) >= top),
           f"moe_route: {keep} of {groups} groups of {experts} experts for top {top}")
     mode = {"sigmoid": 2, "steered": 3}.get(all_scores, 1 if all_scores else 0)
@@ -1483,8 +1480,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
         _dev(correction)
         _need(mode == 3 and correction.dtype == torch.float32 and correction.is_contiguous()
               and correction.numel() == experts, "moe_route: one 32-bit correction per expert, with steered scores")
-    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
-    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, int(groups), int(keep), mode, _ptr(correction),
+    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
+    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, -(-columns[0] // 128), -(-columns[1] // 128), int(groups), int(keep), mode, _ptr(correction),
                float(weight_scale), logits.stride(0) if tokens > 1 else experts, _ptr(ids), _ptr(weights), _ptr(offsets),
                _ptr(order), _ptr(tiles), _ptr(num_tiles), _stream()), "moe_route")
 
@@ -1529,7 +1526,7 @@ def moe_experts(h: torch.Tensor, w_gate: Optional[torch.Tensor], w_up: torch.Ten
     _i32(offsets, order, tiles, num_tiles)
     _need(offsets.numel() == experts + 1 and order.numel() == tokens * top
           and tiles.numel() >= 2 * moe_max_tiles(tokens * top, experts, tile_rows)
-          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, 128, 192, 256),
+          and (tile_rows == 64) == (moe_tile_rows(h, width, ff, 0, 1) == 64) and tile_rows in (16, 64, MOE_EITHER_ROWS, 128, 192, 256),
           "moe_experts: grouping (made by moe_route with the tile_rows that moe_tile_rows gives)")
     fn = _fn("moe", "vk_moe_experts", [_p, _ll, _p, _p, _p, _i, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f, _f, _i, _p, _p,
                                        _p, _i, _i, _p, _p, _ll, _p, _p])
