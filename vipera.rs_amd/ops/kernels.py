@@ -1420,7 +1420,7 @@ MOE_STREAM_PAIRS = 10     # pairs per expert, on average, up to which the expert
 
 def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int, gated: bool = True) -> int:
     """Places per tile of the experts' products for activations ``h`` of ``pairs`` (token, choice) pairs: on the matrix cores
-    (bfloat16, widths that are multiples of 8) 128, 192 or 256, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The
+    (bfloat16, widths that are multiples of 8) 128, 128 or 192 (:data:`MOE_EITHER_ROWS`) or 256, or 16 where few pairs fall to an expert; 64 as 32-bit FMAs.  The
     grouping has to be made for the same number.
 
     With widths in whole steps of 64 the tiles are 128 x 128 outputs (two workgroups a CU) or 256 x 256 (one), and a chip full
