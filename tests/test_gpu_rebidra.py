@@ -800,3 +800,16 @@ def test_pairs_are_grouped_in_the_tiles_of_fewer_rounds(counts, columns, want):
     listed = [(e, edges[e] + i) for e in range(experts) for i in range(0, counts[e], want)]
     assert count.item() == len(listed) | (1 << 30 if want == 192 else 0)
     assert tiles.view(-1, 2)[:len(listed)].tolist() == [list(map(int, t)) for t in listed]
+
+
+@pytest.mark.parametrize("counts, columns, want", [
+    ((204, 214, 172, 211, 166, 216, 170, 183), (28672, 4096), 128),     # us in tiles of 128 and 192: 819 and 1,139, no XCD has fewer tiles
+    ((238, 80, 319, 92, 282, 190, 187, 148), (16384, 2048), 128),       # 306 and 379
+    ((285, 38, 168, 54, 96, 55, 231, 97), (28672, 4096), 128),          # 886 and 1,067
+    ((99, 31, 45, 92, 63, 137, 78, 55), (28672, 4096), 192),            # 830 and 671: a ninth tile is one XCD's second
+    ((127, 109, 104, 149, 134, 124, 133, 144), (28672, 4096), 192),     # 960 and 684
+    ((181, 237, 197, 184, 132, 142, 324, 139), (28672, 4096), 192),     # 1,143 and 1,065
+    ((100,) * 96 + (150,) * 32, (1536, 2048), 128)])                    # nine rounds of those of 192 for ten of 128
+def test_pairs_are_grouped_in_the_tiles_that_cost_less(counts, columns, want):
+    """A round of tiles of 192 places costs more than one of 128, and rounds are an XCD's, which has an eighth of the tiles."""
+    test_pairs_are_grouped_in_the_tiles_of_fewer_rounds(counts, columns, want)

@@ -154,23 +154,37 @@ __device__ __forceinline__ int running_sum(int v) {
   return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
 }
 
-// Rounds of workgroups that so many tiles are in the experts' two products, two a CU; column blocks of the products.
+// What so many tiles cost in the experts' two products: their rounds of workgroups times a round's length. An XCD has an eighth of
+// the tiles with all their column blocks (moe_direct_tile), `slots` workgroups at once; a last round of up to half as many has one a CU and
+// takes two thirds of a full one. A round is as long as K and some 600 more (K 2,048 37 us, K 1,024 23).
 struct Rounds {
-  int up, down;
-  __device__ __forceinline__ long long of(int tiles) const {
-    constexpr int AT_ONCE = 512;
-    return ((long long)tiles * up + AT_ONCE - 1) / AT_ONCE + ((long long)tiles * down + AT_ONCE - 1) / AT_ONCE;
+  int up, down, up_k, down_k, slots;     // column blocks and K of the two products
+  __device__ __forceinline__ float of(int blocks, int own) const {
+    const float n = (float)blocks * (float)own, full = floorf(n * (1.0f / slots)), rest = n - full * slots;
+    return full + (rest <= 0.f ? 0.f : 2.f * rest <= slots ? 2.f / 3.f : 1.f);
   }
+  __device__ __forceinline__ float cost(int tiles) const {
+    const int own = (tiles + 7) / 8;
+    return of(up, own) * (up_k + 600) + of(down, own) * (down_k + 600);
+  }
+  __device__ __forceinline__ bool prefer_192(int narrow, int wide) const { return 1.3f * cost(wide) < cost(narrow); }
 };
 constexpr int TILES_OF_192 = 1 << 30;     // in num_tiles: the tiles are of 192 places
 
+// Tiles of 192 or of a power of two places; a division by a variable is a chain of some thirty instructions in front of the sums.
+__device__ __forceinline__ int tiles_of(int count, int rows) {
+  return rows == GT_MIDDLE ? (count + GT_MIDDLE - 1) / GT_MIDDLE : (int)((unsigned)(count + rows - 1) >> (__ffs(rows) - 1));
+}
+
 // One workgroup: counts per expert, offsets, the pairs' places, and the list of tiles.
 //   offsets [E + 1], order [P], tiles [max_tiles][2] = (expert, first place), num_tiles [1] (with TILES_OF_192)
-// tile_rows GT_EITHER: tiles of 192 places where these are fewer rounds of workgroups than those of 128. A round of the wider
-// ones takes some 1.15 times as long where an expert has one tile and up to 1.4 times with full ones, and one of them that is
-// hardly begun as long as a full one. us, products and sum of 32 experts of 1,024 x 2,048 in tiles of 128 and 192: 512 tokens of which the
-// favourite expert has more than 128 143 and 119, none 99 and 102; 1,400 (as many rounds) 168 and 184; 2,048 204 and 202; without a gate 1,700
-// 156 and 142, 2,500 (as many) 183 and 191; 16 experts of 512 x 1,024, 2,000 tokens 76 and 63.
+// tile_rows GT_EITHER: tiles of 192 places where these cost less than those of 128 at 1.3 times as much a round (1.15 where an expert has
+// one tile, 1.4 with full ones, and one tile that is hardly begun takes as long as a full one), else of 128. Nine shapes of 8 to 256
+// experts, 300 to 2,500 tokens, four spreads of choices each (108 steps, weights from memory): the choice takes 0.964 of the time of 128
+// alone, the faster of the two each time would take 0.960, and one choice is more than 2 % behind 128 (8 experts of 8,192 x 2,048, 768 tokens,
+// 309 / 324 us). Counting a round of either as much and over the whole chip instead of an XCD took 0.984, seventeen of them 2 % and more behind.
+// us, products and sum in tiles of 128 and 192: 8 experts of 14,336 x 4,096, 300 tokens with a ninth tile in those of 128 830 / 671, 768 tokens 819 /
+// 1,139 (sixteen and twelve tiles); 32 of 1,024 x 2,048, 1,000 tokens, none past 192 pairs 163 / 137; 16 of 512 x 1,024, 2,000 tokens 73 / 60.
 // With `logits`: the same workgroup routes the step's tokens first, a wave per token in turn (a step of few tokens:
 // one launch instead of two).
 __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict__ logits, int top, int num_tokens,
@@ -204,7 +218,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
       }
       narrow = __shfl(running_sum(narrow), WAVE - 1, WAVE);
       wide = __shfl(running_sum(wide), WAVE - 1, WAVE);
-      tile_rows = rounds.of(wide) < rounds.of(narrow) ? GT_MIDDLE : GT_TILE;
+      tile_rows = rounds.prefer_192(narrow, wide) ? GT_MIDDLE : GT_TILE;
     }
     for (int base = 0; base < experts; base += WAVE) {
       const int e = base + lane, count = e < experts ? counts[e] : 0;
@@ -214,12 +228,12 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
         own = (count + GT_TILE - 1) / GT_TILE | (count + GT_MIDDLE - 1) / GT_MIDDLE << 16;
         tiles_upto = running_sum(own);
         const unsigned all = (unsigned)__shfl(tiles_upto, WAVE - 1, WAVE);
-        const int part = rounds.of((int)(all >> 16)) < rounds.of((int)(all & 0xffff)) ? 16 : 0;
+        const int part = rounds.prefer_192((int)(all & 0xffff), (int)(all >> 16)) ? 16 : 0;
         tile_rows = part ? GT_MIDDLE : GT_TILE;
         own = (int)((unsigned)own >> part & 0xffff);
         tiles_upto = (int)((unsigned)tiles_upto >> part & 0xffff);
       } else {
-        own = (count + tile_rows - 1) / tile_rows;
+        own = tiles_of(count, tile_rows);
         tiles_upto = running_sum(own);
       }
       if (e < experts) {
@@ -774,13 +788,12 @@ static inline bool moe_loads_direct(int width, int ff, int num_tokens, int top, 
          (long long)num_tokens * top * ff * 2 <= GT_VIEW_BYTES && (long long)width * ff * 2 <= GT_VIEW_BYTES;
 }
 
-// up_blocks, down_blocks: column blocks of the experts' products in tiles of 128 columns, for tile_rows GT_EITHER.
+// For tile_rows GT_EITHER: column blocks of the experts' products in tiles of 128 columns, their K, and the device's CUs.
 extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int up_blocks,
-                            int down_blocks, int groups, int keep,
-                            int all_scores, const float* correction, float weight_scale, long long ld, int* ids,
-                            float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
+                            int down_blocks, int up_k, int down_k, int compute_units, int groups, int keep, int all_scores,
+                            const float* correction, float weight_scale, long long ld, int* ids, float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
   if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE && tile_rows != GT_MIDDLE &&
-      (tile_rows != GT_EITHER || up_blocks < 1 || down_blocks < 1))
+      (tile_rows != GT_EITHER || up_blocks < 1 || down_blocks < 1 || up_k < 1 || down_k < 1 || compute_units < 8))
     return VK_BAD_ARGUMENT;
   if (groups < 1 || keep < 1 || keep > groups || experts % groups != 0) return VK_BAD_ARGUMENT;
   if (groups > WAVE) return VK_UNSUPPORTED_SIZE;
@@ -800,7 +813,8 @@ extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_t
     VK_LAUNCH_CHECK();
   }
   moe_group_kernel<<<1, 1024, (size_t)experts * 2 * sizeof(int), s>>>(together ? logits : nullptr, top, num_tokens,
-                                                                       weights, ids, (int)pairs, experts, tile_rows, Rounds{up_blocks, down_blocks},
+                                                                       weights, ids, (int)pairs, experts, tile_rows,
+                                                                       Rounds{up_blocks, down_blocks, up_k, down_k, compute_units / 8 * 2},
                                                                        offsets, order, tiles, num_tiles, how);
   VK_LAUNCH_CHECK();
   return 0;

@@ -1430,7 +1430,7 @@ def moe_tile_rows(h: torch.Tensor, width: int, ff: int, pairs: int, experts: int
     one expert); 2,048 tokens 198 to 205 and 206 to 214; 1,383 tokens 150 to 164 and 133 (all experts alike) to 192.
 
     Instead of 128 the answer is :data:`MOE_EITHER_ROWS` there: the grouping takes tiles of 192 x 128 outputs, two workgroups a CU as
-    well, where they are fewer rounds of workgroups than those of 128 x 128, which it sees from the experts' counts."""
+    well, where their rounds of workgroups cost less than those of 128 x 128, which it sees from the experts' counts."""
     if not (h.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and h.stride(0) % 8 == 0):
         return 64
     if pairs <= MOE_STREAM_PAIRS * experts:
@@ -1454,7 +1454,7 @@ def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 64) -> int:
 def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.Tensor, offsets: torch.Tensor,
               order: torch.Tensor, tiles: torch.Tensor, num_tiles: torch.Tensor, tile_rows: int = 64,
               groups: int = 1, keep: int = 1, all_scores=False, correction: Optional[torch.Tensor] = None,
-              weight_scale: float = 1.0, columns: Tuple[int, int] = (0, 0)) -> None:
+              weight_scale: float = 1.0, columns: Tuple[int, int] = (0, 0), gated: bool = True) -> None:
     """Each token's ``top`` largest router logits (lowest id first among equals) with the softmax over those, and the
     (token, choice) pairs grouped by expert: ``offsets [E + 1]``, ``order [T * top]``, ``tiles [max, 2]``.
     ``groups`` > 1: the experts form that many equal groups of neighbours and only those of the ``keep`` groups with
@@ -1462,7 +1462,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     all experts (they do not add up to one); ``all_scores="sigmoid"``: the weight of a chosen expert is the sigmoid of its
     own logit, not renormalized; ``all_scores="steered"``: the experts are chosen by ``sigmoid(logit) + correction[e]``
     (``correction`` [experts] 32-bit or None) and a chosen expert's weight is ``weight_scale * sigmoid(logit)``.  ``columns``: the weight
-    rows of the experts' two products (gate and up both), for ``tile_rows`` :data:`MOE_EITHER_ROWS`."""
+    rows of the experts' two products (gate and up both if ``gated``), by which ``tile_rows`` :data:`MOE_EITHER_ROWS` chooses.
+    ``num_tiles``: how many tiles are listed, with bit 30 set where they have 192 places."""
     _dev(logits, ids, weights, offsets, order, tiles, num_tiles)
     tokens, experts = logits.shape
     _f32s(logits, "moe_route: logits")      # rows may lie further apart than they are long (a view of some columns)
@@ -1480,8 +1481,9 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
         _dev(correction)
         _need(mode == 3 and correction.dtype == torch.float32 and correction.is_contiguous()
               and correction.numel() == experts, "moe_route: one 32-bit correction per expert, with steered scores")
-    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
-    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, -(-columns[0] // 128), -(-columns[1] // 128), int(groups), int(keep), mode, _ptr(correction),
+    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
+    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, -(-columns[0] // 128), -(-columns[1] // 128), columns[1],
+               columns[0] // 2 if gated else columns[0], compute_units(logits.device), int(groups), int(keep), mode, _ptr(correction),
                float(weight_scale), logits.stride(0) if tokens > 1 else experts, _ptr(ids), _ptr(weights), _ptr(offsets),
                _ptr(order), _ptr(tiles), _ptr(num_tiles), _stream()), "moe_route")
 

@@ -166,7 +166,7 @@ class MixtureOfExperts(FeedForward):
         weights = torch.empty(pairs, dtype=torch.float32, device=device)
         kernels.moe_route(logits, self.top, ids, weights, offsets, order, tiles, num_tiles, tile_rows,
                           groups=self.groups, keep=self.keep, all_scores=self.all_scores, correction=self.correction,
-                          weight_scale=self.weight_scale, columns=((1 if self.plain else 2) * self.inter, self.hidden))
+                          weight_scale=self.weight_scale, columns=((1 if self.plain else 2) * self.inter, self.hidden), gated=self.plain is None)
         act = self.runtime.empty((pairs, self.inter))
         pair_out = torch.empty((pairs, self.hidden), dtype=torch.float32, device=device)
         extra = None
