@@ -813,3 +813,26 @@ def test_pairs_are_grouped_in_the_tiles_of_fewer_rounds(counts, columns, want):
 def test_pairs_are_grouped_in_the_tiles_that_cost_less(counts, columns, want):
     """A round of tiles of 192 places costs more than one of 128, and rounds are an XCD's, which has an eighth of the tiles."""
     test_pairs_are_grouped_in_the_tiles_of_fewer_rounds(counts, columns, want)
+
+
+def test_a_grouping_without_the_products_columns_has_tiles_of_128_places():
+    """For what moe_tile_rows answers, with nothing by which to choose between 128 and 192 places."""
+    from vipera_rs_amd.ops import kernels
+
+    tokens, width, ff, experts, top = 200, 192, 128, 4, 2
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = torch.randn(tokens, width, device="cuda", generator=g).to(torch.bfloat16)
+    z = torch.randn(tokens, experts, device="cuda", generator=g) + (torch.arange(experts, device="cuda") == 1) * 2.0
+    gate, up = ((torch.randn(experts, ff, width, device="cuda", generator=g) * width ** -0.5).to(torch.bfloat16) for _ in range(2))
+    down = (torch.randn(experts, width, ff, device="cuda", generator=g) * ff ** -0.5).to(torch.bfloat16)
+    rows = kernels.moe_tile_rows(h, width, ff, tokens * top, experts)
+    assert rows == kernels.MOE_EITHER_ROWS
+    got = []
+    for tile_rows in (rows, 128):
+        _, w, offsets, order, tiles, count = route(kernels, z, top, tile_rows)
+        act, pair_out = torch.empty(tokens * top, ff, dtype=torch.bfloat16, device="cuda"), torch.empty(tokens * top, width, device="cuda")
+        residual = torch.empty(tokens, width, device="cuda")
+        kernels.moe_experts(h, gate, up, down, offsets, order, tiles, count, w, top, float("inf"), 1.0, act, pair_out, residual, False,
+                            tile_rows=tile_rows)
+        got.append((offsets, count, tiles[:2 * count.item()], pair_out, residual))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

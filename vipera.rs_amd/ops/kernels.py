@@ -1462,8 +1462,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
     all experts (they do not add up to one); ``all_scores="sigmoid"``: the weight of a chosen expert is the sigmoid of its
     own logit, not renormalized; ``all_scores="steered"``: the experts are chosen by ``sigmoid(logit) + correction[e]``
     (``correction`` [experts] 32-bit or None) and a chosen expert's weight is ``weight_scale * sigmoid(logit)``.  ``columns``: the weight
-    rows of the experts' two products (gate and up both if ``gated``), by which ``tile_rows`` :data:`MOE_EITHER_ROWS` chooses.
-    ``num_tiles``: how many tiles are listed, with bit 30 set where they have 192 places."""
+    rows of the experts' two products (gate and up both if ``gated``), by which ``tile_rows`` :data:`MOE_EITHER_ROWS` chooses; without
+    them its tiles have 128 places.  ``num_tiles``: how many tiles are listed, with bit 30 set where they have 192 places."""
     _dev(logits, ids, weights, offsets, order, tiles, num_tiles)
     tokens, experts = logits.shape
     _f32s(logits, "moe_route: logits")      # rows may lie further apart than they are long (a view of some columns)
@@ -1476,6 +1476,8 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
           and num_tiles.numel() == 1 and tile_rows in (16, 64, MOE_EITHER_ROWS, 128, 192, 256), "moe_route: output sizes")
     _need(1 <= keep <= groups <= 64 and experts % groups == 0 and (keep == groups or keep * (experts // groups) >= top),
           f"moe_route: {keep} of {groups} groups of {experts} experts for top {top}")
+    if tile_rows == MOE_EITHER_ROWS and min(columns) < 1:
+        tile_rows = 128
     mode = {"sigmoid": 2, "steered": 3}.get(all_scores, 1 if all_scores else 0)
     if correction is not None:
         _dev(correction)
