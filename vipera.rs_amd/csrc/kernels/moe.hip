@@ -159,15 +159,14 @@ __device__ __forceinline__ int running_sum(int v) {
 // takes two thirds of a full one. A round is as long as K and some 600 more (K 2,048 37 us, K 1,024 23).
 struct Rounds {
   int up, down, up_k, down_k, slots;     // column blocks and K of the two products
-  __device__ __forceinline__ float of(int blocks, int own) const {
-    const float n = (float)blocks * (float)own, full = floorf(n * (1.0f / slots)), rest = n - full * slots;
-    return full + (rest <= 0.f ? 0.f : 2.f * rest <= slots ? 2.f / 3.f : 1.f);
+  // By a whole wave: of every four lanes one takes one of the products in tiles of 128 or (the last two) of 192 places.
+  __device__ __forceinline__ bool prefer_192(int narrow, int wide, int lane) const {
+    const float n = (float)(lane & 1 ? down : up) * (float)(((lane & 2 ? wide : narrow) + 7) / 8);
+    const float full = floorf(n * (1.0f / slots)), rest = n - full * slots;
+    const float cost = (full + (rest <= 0.f ? 0.f : 2.f * rest <= slots ? 2.f / 3.f : 1.f)) * ((lane & 1 ? down_k : up_k) + 600);
+    const float both = cost + __shfl_xor(cost, 1, WAVE);
+    return 1.3f * __shfl(both, 2, WAVE) < __shfl(both, 0, WAVE);
   }
-  __device__ __forceinline__ float cost(int tiles) const {
-    const int own = (tiles + 7) / 8;
-    return of(up, own) * (up_k + 600) + of(down, own) * (down_k + 600);
-  }
-  __device__ __forceinline__ bool prefer_192(int narrow, int wide) const { return 1.3f * cost(wide) < cost(narrow); }
 };
 constexpr int TILES_OF_192 = 1 << 30;     // in num_tiles: the tiles are of 192 places
 
@@ -205,56 +204,47 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const float* __restrict
   __syncthreads();
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) atomicAdd(&counts[ids[p]], 1);
   __syncthreads();
+  const int lane = threadIdx.x & (WAVE - 1);
   if (threadIdx.x < WAVE) {          // one wave: running sums over the experts, 64 at a time
-    const int lane = threadIdx.x;
-    int at = 0, tile = 0;
-    // up to 64 experts the choice falls out of the sums below, both kinds of tiles in one number
-    if (tile_rows == GT_EITHER && (experts > WAVE || pairs > 8000000)) {
-      int narrow = 0, wide = 0;
-      for (int base = 0; base < experts; base += WAVE) {
-        const int e = base + lane, count = e < experts ? counts[e] : 0;
-        narrow += (count + GT_TILE - 1) / GT_TILE;
-        wide += (count + GT_MIDDLE - 1) / GT_MIDDLE;
-      }
-      narrow = __shfl(running_sum(narrow), WAVE - 1, WAVE);
-      wide = __shfl(running_sum(wide), WAVE - 1, WAVE);
-      tile_rows = rounds.prefer_192(narrow, wide) ? GT_MIDDLE : GT_TILE;
-    }
+    int at = 0;
     for (int base = 0; base < experts; base += WAVE) {
-      const int e = base + lane, count = e < experts ? counts[e] : 0;
-      const int places = running_sum(count);
-      int own, tiles_upto;
-      if (tile_rows == GT_EITHER) {
-        own = (count + GT_TILE - 1) / GT_TILE | (count + GT_MIDDLE - 1) / GT_MIDDLE << 16;
-        tiles_upto = running_sum(own);
-        const unsigned all = (unsigned)__shfl(tiles_upto, WAVE - 1, WAVE);
-        const int part = rounds.prefer_192((int)(all & 0xffff), (int)(all >> 16)) ? 16 : 0;
-        tile_rows = part ? GT_MIDDLE : GT_TILE;
-        own = (int)((unsigned)own >> part & 0xffff);
-        tiles_upto = (int)((unsigned)tiles_upto >> part & 0xffff);
-      } else {
-        own = tiles_of(count, tile_rows);
-        tiles_upto = running_sum(own);
-      }
-      if (e < experts) {
-        const int first = at + places - count;
-        offsets[e] = first;
-        cursor[e] = first;
-        for (int i = 0, to = tile + tiles_upto - own; i < own; ++i, ++to) {
-          tiles[2 * to] = e;
-          tiles[2 * to + 1] = first + i * tile_rows;
-        }
-      }
+      const int e = base + lane, count = e < experts ? counts[e] : 0, places = running_sum(count);
+      if (e < experts) offsets[e] = cursor[e] = at + places - count;
       at += __shfl(places, WAVE - 1, WAVE);
-      tile += __shfl(tiles_upto, WAVE - 1, WAVE);
     }
-    if (lane == 0) {
-      offsets[experts] = at;
-      num_tiles[0] = tile | (tile_rows == GT_MIDDLE ? TILES_OF_192 : 0);
+    if (lane == 0) offsets[experts] = at;
+  }
+  const int placing = blockDim.x - WAVE;
+  if (threadIdx.x >= placing && tile_rows == GT_EITHER) {      // the last wave chooses while the first sums
+    int narrow = 0, wide = 0;
+    for (int e = lane; e < experts; e += WAVE) {
+      narrow += tiles_of(counts[e], GT_TILE);
+      wide += tiles_of(counts[e], GT_MIDDLE);
     }
+    narrow = __shfl(running_sum(narrow), WAVE - 1, WAVE);
+    wide = __shfl(running_sum(wide), WAVE - 1, WAVE);
+    tile_rows = rounds.prefer_192(narrow, wide, lane) ? GT_MIDDLE : GT_TILE;
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) order[atomicAdd(&cursor[ids[p]], 1)] = p;
+  if (threadIdx.x < placing) {
+    for (int p = threadIdx.x; p < pairs; p += placing) order[atomicAdd(&cursor[ids[p]], 1)] = p;
+    return;
+  }
+  // The last wave lists the tiles meanwhile: nothing here waits for them.  us, routing and grouping, with choice and list between the
+  // sums and the placing (the list alone before there was a choice) and here: 32 experts, top 4, 512 tokens 7.53 (7.44) / 7.43, 2,048 11.57 (11.53)
+  // / 11.45; 128, top 8, 1,500 21.0 (20.7) / 20.3; 256, top 8, 2,048 28.1 (27.6) / 26.9; 90 tokens on 32 6.81 (6.67) / 6.80.
+  int at = 0, tile = 0;
+  for (int base = 0; base < experts; base += WAVE) {
+    const int e = base + lane, count = e < experts ? counts[e] : 0, own = tiles_of(count, tile_rows);
+    const int places = running_sum(count), tiles_upto = running_sum(own);
+    for (int i = 0, to = tile + tiles_upto - own; i < own; ++i, ++to) {
+      tiles[2 * to] = e;
+      tiles[2 * to + 1] = at + places - count + i * tile_rows;
+    }
+    at += __shfl(places, WAVE - 1, WAVE);
+    tile += __shfl(tiles_upto, WAVE - 1, WAVE);
+  }
+  if (lane == 0) num_tiles[0] = tile | (tile_rows == GT_MIDDLE ? TILES_OF_192 : 0);
 }
 
 // ---------------------------------------------------------------------------------------------
