@@ -221,6 +221,15 @@ def test_256x128_tiles_with_few_last_tokens_keep_their_deep_ranges():
     assert carried(945, 1536, 8960) == 18                                              # 42.2 and 39.8
 
 
+def test_split_small_tiles_give_way_where_the_larger_ones_are_faster():
+    """13: 64x64 with K split, 16: 192x64, 17: 128x128; us of the small tiles and of those picked, or of 17 where they stay."""
+    from vipera_rs_amd.ops.kernels import gemm_bf16_tile_carried_out as carried
+    assert carried(204, 1152, 6912) == 13 and carried(250, 1152, 6912) == 13      # 18.2 and 18.7, 19.6 and 19.8: 576 small tiles
+    assert carried(204, 1280, 5120) == 17 and carried(204, 2560, 4096) == 17      # 16.9 and 16.8, 20.1 and 19.0: 640
+    assert carried(319, 896, 4864) == 16 and carried(572, 512, 8192) == 16        # 15.0 and 14.9, 17.9 and 17.2: 560 and 576
+    assert carried(200, 1024, 4096) == 13                                         # 512, two a CU
+
+
 def _walked(reach, tokens, window, keep_first=0):
     """Steps that the kernel's walk makes of a tile of so many tokens whose last one sees ``reach`` positions (TileWalk)."""
     pos = reach - tokens

@@ -2117,10 +2117,16 @@ int split_tile(int planned, int M, int N, int K, int ranges) {
 // are more than two a CU, and of ones that walk K (14) where the estimate with the sums' way through memory and a second launch is below
 // 0.95 of the walk's (2.5 us and 0.27 a step of 64). Of 101 products planned as small tiles 18 change, to 0.88 of their time, 0.94 at worst:
 // us, 130 tokens on 2,048 rows of 8,192 22.1 / 18.2, 311 on 2,048 of 4,096 22.3 / 18.2, 622 on 896 of 4,864 21.5 / 18.3, and walked 622 on
-// 1,536 of 8,960 40.4 / 32.9, 512 on 2,048 of 8,192 35.2 / 29.6. Up to two a CU the split small tiles stay ahead by 4 to 15 %.
+// 1,536 of 8,960 40.4 / 32.9, 512 on 2,048 of 8,192 35.2 / 29.6. Up to two a CU the split small tiles stay ahead by 4 to 15 %; past two
+// they are not estimated: what comes in one round takes their place, 128x128 tiles from nine for four CUs on (204 to 250 tokens on 1,152 rows of
+// 6,912 in eight ranges, 576 small tiles, 18.2 to 19.6 / 18.7 to 19.8 us; 204 on 1,280 of 5,120, 640, 16.9 / 16.8, 204 on 2,560 of 4,096 in four 20.1 /
+// 19.0). Of 138 further products past two a CU 134 change, to 0.90 of their time, 0.997 at worst.
 int split_small_tile(int planned, int M, int N, int K, int ranges) {
   const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  if (planned == 13 && small * ranges > 2LL * g_compute_units) return one_round_tile(13, 1e30, M, N, K, ranges, true);
+  if (planned == 13 && small * ranges > 2LL * g_compute_units) {
+    const int picked = one_round_tile(13, 1e30, M, N, K, ranges, true);
+    return picked == 17 && small * ranges * 4 <= 9LL * g_compute_units ? 13 : picked;
+  }
   if (planned == 14) {
     const double sums = (2.0 * ranges + 1.0) * 4.0 * M * N / 6e6 + 3.0;
     return one_round_tile(14, 0.95 * (2.5 + 0.27 * (K / 64)) - sums, M, N, K, ranges, true);
