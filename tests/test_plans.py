@@ -185,6 +185,19 @@ def test_an_aligned_32_bit_product_asks_for_the_memory_that_its_form_writes():
     assert _gemm_generic_parts(2048, 9728, 8960) == 0 == _gemm_direct_parts(2048, 9728, 8960)
 
 
+def test_a_gated_32_bit_product_is_one_launch_where_that_is_faster():
+    """us of product and gate in two launches and in one."""
+    from vipera_rs_amd.ops.kernels import _gemm_gated_takes as takes, gemm_generic_gated_pays as pays
+    for slower in ((400, 4096, 1024), (494, 2148, 948),          # 75 and 83, 51 and 61: 4.5 and 2.9 tiles of 48 x 64 a CU
+                   (441, 3396, 932), (550, 9720, 968),           # 67 and 75, 206 and 228: 2.9 and 10.7 of 64 x 64
+                   (231, 6056, 956)):                            # 74 and 76: 4.9 of 48 x 48
+        assert takes(*slower) and not pays(*slower)
+    for faster in ((333, 4864, 896), (17, 4864, 896), (130, 4864, 896), (65, 8960, 1536), (512, 4096, 1024),     # 68 and 65, 16 and 14, 34 and 32, ...
+                   (138, 10328, 948), (635, 5812, 992), (742, 1688, 988)):          # 3.8 of 48 x 64, 7.1 of 64 x 64, 6.6 of 48 x 32
+        assert takes(*faster) and pays(*faster)
+    assert not pays(65, 12, 1028) and not takes(65, 12, 1028)
+
+
 def test_past_128_tokens_small_tiles_carry_out_a_128x128_plan_unless_its_tiles_fill_the_gpu():
     """The tiling and the ranges of K.  Tilings 9: 128x128, 13: 64x64 with K split, 14: 64x64 that walk K, 15: 128x64 that walk K."""
     from vipera_rs_amd.ops.kernels import gemm_bf16_tile_plan as plan

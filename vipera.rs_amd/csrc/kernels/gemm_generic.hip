@@ -1055,6 +1055,26 @@ static Direct gated_plan(int M, int N, int K) {
 }
 extern "C" int vk_gemm_generic_gated_takes(int M, int N, int K) { return gated_plan(M, N, K) != NOT_DIRECT; }
 
+// Whether it is the faster way there too. Past one round the larger slabs' workgroups end in step with the others of their CU when they apply the
+// gate, and the next ones come to a CU in twos (48 x 48: threes): where the last round has fewer for a CU than its places, some CUs get a
+// tile more than the product's launch gives any. us, product and gate in two launches and here: 400 x (2 x 4,096) x 1,024, 4.5 tiles of 48 x 64 a CU, 75 / 83;
+// 494 x (2 x 2,148) x 948, 2.9, 51 / 61; 441 x (2 x 3,396) x 932, 2.9 of 64 x 64, 67 / 75; 231 x (2 x 6,056) x 956, 4.9 of 48 x 48, 74 / 76. Of 209 such sizes of the
+// four larger slabs 83 stay here, in 0.96 of the time, 1.03 at worst, and 126 would take 1.03, 1.2 at worst; of 530 others none takes longer here.
+extern "C" int vk_gemm_generic_gated_pays(int M, int N, int K) {
+  const Direct form = gated_plan(M, N, K);
+  auto most = [&](int rows, int columns) {
+    const long long tiles = (long long)((M + rows - 1) / rows) * ((2ll * N + columns - 1) / columns);
+    return (tiles + 255) / 256;
+  };
+  switch (form) {
+    case NOT_DIRECT: return 0;
+    case SLAB_48_48: return most(48, 48) <= 3 || most(48, 48) % 3 != 2;
+    case SLAB_48_64: return most(48, 64) <= 2 || most(48, 64) == 4;
+    case SLAB_64_64: return most(64, 64) <= 8 && (most(64, 64) == 1 || most(64, 64) % 2 == 0);
+    default: return 1;
+  }
+}
+
 extern "C" int vk_gemm_generic_gated(const float* A, const float* W, float* C, int M, int N, int K, long long lda, long long ldc,
                                      void* stream) {
   if (M <= 0 || N <= 0) return 0;

@@ -250,6 +250,12 @@ def _gemm_gated_takes(m: int, inter: int, k: int) -> bool:
     return bool(_fn("gemm_generic", "vk_gemm_generic_gated_takes", [_i, _i, _i])(m, inter, k))
 
 
+@functools.lru_cache(maxsize=4096)
+def gemm_generic_gated_pays(m: int, inter: int, k: int) -> bool:
+    """Whether :func:`gemm_generic_gated` is faster than :func:`gemm_generic` and :func:`swiglu`, where it takes the operands."""
+    return bool(_fn("gemm_generic", "vk_gemm_generic_gated_pays", [_i, _i, _i])(m, inter, k))
+
+
 def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     """``out = up(a) * silu(gate(a))`` of 32-bit operands with ``w = [gate; up]``, in the product's own launch and with the bits of
     :func:`gemm_generic` and :func:`swiglu` behind it; False, and nothing launched, where these are to be used: up to 8 tokens, which are a
