@@ -267,6 +267,31 @@ def test_a_prepared_selective_scan_walks_to_the_same_bits(sizes):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("lengths", [(70, 33, 48, 17, 1, 63), (32, 40), (31, 20, 5), (300,)])
+@pytest.mark.parametrize("sizes", [(18, 5), (40, 16), (33, 20)])
+def test_a_prepared_selective_scan_of_long_and_short_portions_walks_to_the_same_bits(sizes, lengths):
+    """In blocks of 32 tokens from 32 tokens an entry on (up to 16 states), with whole blocks, whole halves of one and remainders."""
+    from vipera_rs_amd.ops import kernels
+
+    channels, states = sizes
+    entries, tokens, floats = len(lengths), sum(lengths), channels * kernels.selective_scan_channel_floats(states)
+    g = torch.Generator("cuda").manual_seed(tokens + channels)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    meta = (i32(np.cumsum([0, *lengths]).tolist()), i32([0, 7, 3, 0, 1, 2][:entries]), i32([3, 0, 5, 1, 2, 6][:entries]))
+    start, x, z, dt, low = rand(7, floats + 3), rand(tokens, channels), rand(tokens, channels), rand(tokens, channels), rand(tokens, 3 + 2 * states)
+    a_log, skip, dt_bias = rand(channels, states), rand(channels), rand(channels) - 1.0
+    got = []
+    for prepared in (False, True):
+        state, out, step, gate = start.clone(), torch.full_like(x, float("nan")), dt.clone(), z.clone()
+        if prepared:
+            kernels.scan_prepare(step, dt_bias, z, gate)
+        kernels.selective_scan(x, step, dt_bias, low[:, 3:3 + states], low[:, 3 + states:], a_log, skip, gate, state, *meta, out,
+                               entries, prepared)
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 # --- each mechanism alone: models of one layer ---------------------------------------------------------------------
 def only_left(part):
     return Z.parallel(part, Z.right(16, 4, 2, 2), 1.0, 0.0)

@@ -825,15 +825,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 }
 
 // The same for prompts' portions (`prepared`) and up to 64 states, with every token's sum and state formed exactly as above.  A
-// workgroup of four waves (sixteen channels) takes the tokens in blocks (of 32 for a state a lane, else of 16) through two LDS stages, where a
+// workgroup of four waves (sixteen channels) takes the tokens in blocks (of 32 for a state a lane and 32 tokens an entry, else of 16) through two LDS stages, where a
 // state's (a channel's) numbers of neighbouring tokens lie side by side, so that a lane reads four tokens' at once; a block's numbers
 // are on their way into registers while the block before is worked on.  A whole block is unrolled without a branch: the exponentials,
 // products and exchanges of neighbouring tokens, which wait for nothing but the state's one FMA a token, fill each other's
 // latencies, and sixteen tokens' sums go through the lanes together.  Lane j of a channel's sixteen ends up with token j's sum and
 // finishes that token's output.  What bounds it is the instructions (about 23 a token for a state a lane, fourteen of them the
 // exponential).  ALL: N = 16 R.  4,096 channels of 16 states, with blocks of 16 and every token's sum by itself, and so: portions of
-// 1,000 and 834 tokens 120 -> 111 us, one of 2,048 178 -> 159, of 512 50 -> 44, eight of 250 101 -> 93.  Beyond 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
-template <int R, bool ALL, typename TO>
+// 1,000 and 834 tokens 120 -> 111 us, one of 2,048 178 -> 159, of 512 50 -> 44, eight of 250 101 -> 93.  Short entries have no block of 32 and pay for
+// its stages: in blocks of 32 and of 16, 64 of 20 tokens 72 -> 62 us, 30 of 5 16.4 -> 13.5, one of 16 5.1 -> 4.0.  Beyond 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
+template <int R, int BLOCK, bool ALL, typename TO>
 __global__ __launch_bounds__(256) void selective_run_kernel(
     const float* __restrict__ x, const float* __restrict__ dt, long long lddt, const float* __restrict__ bmat,
     const float* __restrict__ cmat, long long ldbc, const float* __restrict__ a_log, const float* __restrict__ skip,
@@ -841,7 +842,7 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
     const int* __restrict__ entry_start, const int* __restrict__ entry_first, const int* __restrict__ slots, int C, int N,
     TO* __restrict__ out) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int HALVES = R == 1 ? 2 : 1, BLOCK = 16 * HALVES, ROW = BLOCK + 4, STATES = 16 * R;
+  constexpr int HALVES = BLOCK / 16, ROW = BLOCK + 4, STATES = 16 * R;
   constexpr int BC_TOKENS = 256 / STATES, BC_LOADS = BLOCK / BC_TOKENS;
   __shared__ __attribute__((aligned(16))) float bc[2][2][STATES][ROW];     // B and C: [state][token]
   __shared__ __attribute__((aligned(16))) float xdz[2][3][16][ROW];        // x, dt and the gate: [channel][token]
@@ -869,24 +870,39 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
   const int state_of = tid % STATES, bc_token = tid / STATES, ch_token = tid / 16;
   const int bc_col = ALL ? state_of : min(state_of, N - 1);
   const long long ch_col = min((int)blockIdx.y * 16 + tid % 16, C - 1);
-  float held_b[BC_LOADS], held_c[BC_LOADS], held_x[HALVES], held_dt[HALVES], held_z[HALVES];
+  float held_b[BC_LOADS] = {}, held_c[BC_LOADS] = {}, held_x[HALVES] = {}, held_dt[HALVES] = {}, held_z[HALVES] = {};
   auto fetch = [&](int first) {
-    const bool whole = first + BLOCK <= t1;
-    const float *bs = bmat + first * ldbc + bc_col, *cs = cmat + first * ldbc + bc_col;
-    const float *xs = x + (long long)first * C + ch_col, *dts = dt + first * lddt + ch_col, *zs = z + first * ldz + ch_col;
-    const int last = t1 - 1 - first;
+    if constexpr (HALVES == 1) {
 #pragma unroll
-    for (int i = 0; i < BC_LOADS; ++i) {
-      const int j = bc_token + i * BC_TOKENS, at = (whole ? j : min(j, last)) * (int)ldbc;
-      held_b[i] = bs[at];
-      held_c[i] = cs[at];
-    }
+      for (int i = 0; i < BC_LOADS; ++i) {
+        const long long at = (long long)min(first + bc_token + i * BC_TOKENS, t1 - 1) * ldbc + bc_col;
+        held_b[i] = bmat[at];
+        held_c[i] = cmat[at];
+      }
+      const long long t = min(first + ch_token, t1 - 1);
+      held_x[0] = x[t * C + ch_col];
+      held_dt[0] = dt[t * lddt + ch_col];
+      held_z[0] = z[t * ldz + ch_col];
+    } else {
+      const bool whole = first + BLOCK <= t1;
+      const float *bs = bmat + first * ldbc + bc_col, *cs = cmat + first * ldbc + bc_col;
+      const float *xs = x + (long long)first * C + ch_col, *dts = dt + first * lddt + ch_col, *zs = z + first * ldz + ch_col;
+      const int last = t1 - 1 - first;
 #pragma unroll
-    for (int i = 0; i < HALVES; ++i) {
-      const int j = ch_token + i * 16, at = whole ? j : min(j, last);
-      held_x[i] = xs[at * C];
-      held_dt[i] = dts[at * (int)lddt];
-      held_z[i] = zs[at * (int)ldz];
+      for (int i = 0; i < BC_LOADS; ++i) {
+        if (HALVES == 2 && i > 0 && last < 16) break;      // nobody reads what would be there
+        const int j = bc_token + i * BC_TOKENS, at = (whole ? j : min(j, last)) * (int)ldbc;
+        held_b[i] = bs[at];
+        held_c[i] = cs[at];
+      }
+#pragma unroll
+      for (int i = 0; i < HALVES; ++i) {
+        if (i > 0 && last < 16) break;
+        const int j = ch_token + i * 16, at = whole ? j : min(j, last);
+        held_x[i] = xs[at * C];
+        held_dt[i] = dts[at * (int)lddt];
+        held_z[i] = zs[at * (int)ldz];
+      }
     }
   };
   auto stage = [&](int buf) {
@@ -912,7 +928,8 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
     if (more) fetch(tb + BLOCK);
     float sums[HALVES] = {};
     const int count = min(BLOCK, t1 - tb);
-    if (count == BLOCK) {
+    auto walk = [&](auto tokens) {      // the block's first ones
+      constexpr int TOKENS = decltype(tokens)::value;
       float quads[4];
       f32x4 x4[2], dt4[2], b4[2][R], c4[2][R];     // four tokens at a time, the next four's reads before them
       auto read = [&](int j4, int to) {
@@ -926,9 +943,9 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
       };
       read(0, 0);
 #pragma unroll
-      for (int j4 = 0; j4 < BLOCK; j4 += 4) {
+      for (int j4 = 0; j4 < TOKENS; j4 += 4) {
         const int now = j4 / 4 & 1;
-        if (j4 + 4 < BLOCK) read(j4 + 4, now ^ 1);
+        if (j4 + 4 < TOKENS) read(j4 + 4, now ^ 1);
         __builtin_amdgcn_sched_barrier(0);
         // in phases, each of them over the four tokens, so that none of their chains is waited for alone
         float keep[4][R], add[4][R], sum[4];
@@ -955,8 +972,13 @@ __global__ __launch_bounds__(256) void selective_run_kernel(
         if (j4 % 16 == 12) sums[j4 / 16] = merge.rows(quads);
         __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    if (count == BLOCK) {
+      walk(std::integral_constant<int, BLOCK>{});
     } else {
-      for (int j = 0; j < count; ++j) {
+      const int walked = HALVES == 2 && count >= 16 ? 16 : 0;
+      if (HALVES == 2 && walked) walk(std::integral_constant<int, 16>{});
+      for (int j = walked; j < count; ++j) {
         const float step = xdz[buf][1][mine][j], dtx = step * xdz[buf][0][mine][j];
         float sum = 0.f;
 #pragma unroll
@@ -1062,7 +1084,7 @@ extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long l
                                  const float* bmat, const float* cmat, long long ldbc, const float* a_log,
                                  const float* skip, const float* z, long long ldz, float* state,
                                  long long state_stride, const int* entry_start, const int* entry_first,
-                                 const int* slots, int num_entries, int C, int N, int prepared, void* out,
+                                 const int* slots, int num_entries, int num_tokens, int C, int N, int prepared, void* out,
                                  int out_dtype, void* stream) {
   if (num_entries <= 0) return 0;
   if (C < 1 || N < 1) return VK_BAD_ARGUMENT;
@@ -1073,15 +1095,19 @@ extern "C" int vk_selective_scan(const float* x, const float* dtraw, long long l
   hipStream_t s = (hipStream_t)stream;
   const dim3 run_grid(num_entries, (C + 15) / 16);
   // the walk in blocks counts a block's numbers from its first token in 32 bits
+  const bool long_blocks = num_tokens >= 32ll * num_entries;
   const bool runs = prepared && C < (1 << 26) && lddt < (1 << 26) && ldbc < (1 << 26) && ldz < (1 << 26);
-#define VK_SS_RUN(RR, ALL, TO)                                                                                        \
-  selective_run_kernel<RR, ALL, TO><<<run_grid, 256, 0, s>>>(x, dtraw, lddt, bmat, cmat, ldbc, a_log, skip, z, ldz, state, \
-                                                             state_stride, entry_start, entry_first, slots, C, N, (TO*)out)
+#define VK_SS_RUN(RR, BLOCK, ALL, TO)                                                                                 \
+  selective_run_kernel<RR, BLOCK, ALL, TO><<<run_grid, 256, 0, s>>>(x, dtraw, lddt, bmat, cmat, ldbc, a_log, skip, z, ldz, \
+                                                                    state, state_stride, entry_start, entry_first, slots, \
+                                                                    C, N, (TO*)out)
 #define VK_SS(RR, TO)                                                                                               \
   if constexpr (RR <= 4) {                                                                                          \
     if (runs) {                                                                                                     \
-      if (N == 16 * RR) VK_SS_RUN(RR, true, TO);                                                                    \
-      else VK_SS_RUN(RR, false, TO);                                                                                \
+      if (RR == 1 && long_blocks && N == 16) VK_SS_RUN(1, 32, true, TO);                                            \
+      else if (RR == 1 && long_blocks) VK_SS_RUN(1, 32, false, TO);                                                 \
+      else if (N == 16 * RR) VK_SS_RUN(RR, 16, true, TO);                                                           \
+      else VK_SS_RUN(RR, 16, false, TO);                                                                            \
       break;                                                                                                        \
     }                                                                                                               \
   }                                                                                                                 \

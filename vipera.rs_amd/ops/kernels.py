@@ -1850,10 +1850,10 @@ def selective_scan(x: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, b: 
     _i32(entry_start, entry_first_pos, slots)
     _entries_ok((entry_start, entry_first_pos, slots), num_entries)
     fn = _fn("scan", "vk_selective_scan", [_p, _p, _ll, _p, _p, _p, _ll, _p, _p, _p, _ll, _p, _ll, _p, _p, _p, _i, _i, _i,
-                                           _i, _p, _i, _p])
+                                           _i, _i, _p, _i, _p])
     _status(fn(_ptr(x), _ptr(dt), dt.stride(0), _ptr(dt_bias), _ptr(b), _ptr(c), b.stride(0), _ptr(a_log), _ptr(skip),
                _ptr(z), z.stride(0), _ptr(state), state.stride(0), _ptr(entry_start), _ptr(entry_first_pos), _ptr(slots),
-               num_entries, channels, states, 1 if prepared else 0, _ptr(out), _dt(out, "out"), _stream()),
+               num_entries, tokens, channels, states, 1 if prepared else 0, _ptr(out), _dt(out, "out"), _stream()),
             "selective_scan")
 
 
