@@ -548,3 +548,31 @@ def test_prompts_recurrences_give_the_same_bits_from_rows_off_16_bytes(rule, siz
         assert torch.isfinite(out).all()
         got.append((out, state))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("lengths", [(70, 33, 64, 48, 7), (32, 32), (31, 40, 16), (300,)])
+@pytest.mark.parametrize("heads, dim", [(1, 4), (3, 40), (2, 64), (40, 64)])
+def test_time_mixing_in_long_and_short_blocks_gives_the_same_bits_from_rows_off_16_bytes(heads, dim, lengths):
+    """Blocks of 32 tokens from 32 tokens an entry on, up to 768 workgroups (40 heads of 64 are 320 an entry), else of 16, with whole
+    blocks and remainders; the same numbers a float further on in memory take the general walk."""
+    from vipera_rs_amd.ops import kernels
+
+    gen = torch.Generator("cuda").manual_seed(6)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    entries, tokens, width = len(lengths), sum(lengths), heads * dim
+    meta = (i32(np.cumsum([0, *lengths]).tolist()), i32([0, 5, 3, 0, 1][:entries]), i32([3, 0, 5, 1, 4][:entries]))
+    start, bonus = rand(6, heads * kernels.recurrent_head_floats(dim, dim)), rand(width)
+    rows = [rand(tokens, width) for _ in range(3)] + [torch.exp(-torch.exp(rand(tokens, width) - 2.0))]
+    got = []
+    for floats in (0, 1):
+        given = []
+        for t in rows:
+            room = torch.empty(t.numel() + floats, device="cuda")
+            given.append(room[floats:].view(t.shape).copy_(t))
+        assert all((t.data_ptr() % 16 == 0) == (floats == 0) for t in given)
+        state, out = start.clone(), torch.full((tokens, width), float("nan"), device="cuda")
+        kernels.wkv_rule(*given, torch.zeros_like(bonus), bonus, state, *meta, dim, heads, out, entries, decayed=True)
+        assert torch.isfinite(out).all()
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

@@ -899,7 +899,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
 // them (13 above for one).  Nothing waits for a token's sums over the lanes, so sixteen tokens' go through the tree together.  Blocks
 // of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here (in blocks of 32 /
 // 16): 32 heads of 64, one entry of 2,048 tokens 168 / 108 / 127, of 512 46 / 31 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
-// 512, 456 and 399 (768) 82 / 55 / 59, eight of 250 (2,048) 115 / 84 / 75.
+// 512, 456 and 399 (768) 82 / 55 / 59, eight of 250 (2,048) 115 / 84 / 75.  Entries that have no block of 32
+// are walked in blocks of 16: 31 tokens in either 6.5 / 6.0, 16 tokens 5.0 / 4.3.
 constexpr int WKV_LONG_BLOCKS = 3 * 256;      // workgroups up to which blocks are of 32 tokens
 template <int Q, int BLOCK>
 __global__ __launch_bounds__(SCAN_COLS * 32) void wkv_scan_direct_kernel(
@@ -1865,8 +1866,8 @@ extern "C" int vk_memory_rule(float* proj, long long ldp, int num_tokens, int q_
 extern "C" int vk_wkv_rule(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv,
                            const float* wraw, long long ldw, const float* w0, const float* bonus, float* state,
                            long long state_stride, const int* entry_start, const int* entry_first, const int* slots,
-                           int dim, int heads, float* out, int num_entries, int short_entries, int decayed,
-                           void* stream) {
+                           int dim, int heads, float* out, int num_entries, int num_tokens, int short_entries,
+                           int decayed, void* stream) {
   if (num_entries <= 0) return 0;
   if (heads < 1 || dim < 1) return VK_BAD_ARGUMENT;
   if (dim > 256 || heads > 65535) return VK_UNSUPPORTED_SIZE;
@@ -1886,7 +1887,8 @@ extern "C" int vk_wkv_rule(const float* r, long long ldr, const float* k, long l
     const bool pieces = dim % 4 == 0 && (ldr | ldk | ldw) % 4 == 0 && (((uintptr_t)r | (uintptr_t)k | (uintptr_t)wraw) & 15) == 0 &&
                         std::max(std::max(ldr, ldk), std::max(ldv, ldw)) < (1 << 24);
     const long long groups = (long long)num_entries * heads * (value_pad / SCAN_COLS);
-    if (decayed && pieces && key_pad <= 64 && groups <= WKV_LONG_BLOCKS) VK_WKV_DIRECT(1, 2 * REC_BLOCK);
+    const bool long_blocks = groups <= WKV_LONG_BLOCKS && num_tokens >= 32ll * num_entries;
+    if (decayed && pieces && key_pad <= 64 && long_blocks) VK_WKV_DIRECT(1, 2 * REC_BLOCK);
     else if (decayed && pieces && key_pad <= 64) VK_WKV_DIRECT(1, REC_BLOCK);
     else if (decayed && pieces && key_pad <= 128) VK_WKV_DIRECT(2, REC_BLOCK);
     else if (key_pad <= 64) VK_WKV_SCAN(1);

@@ -1294,10 +1294,10 @@ def wkv_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wraw: torch.Tens
     if dim > RECURRENT_MAX_KEY_DIM:
         raise UnsupportedError(f"wkv_rule: a head width of {dim} is above the kernel's limit of {RECURRENT_MAX_KEY_DIM}")
     fn = _fn("recurrent", "vk_wkv_rule",
-             [_p, _ll, _p, _ll, _p, _ll, _p, _ll, _p, _p, _p, _ll, _p, _p, _p, _i, _i, _p, _i, _i, _i, _p])
+             [_p, _ll, _p, _ll, _p, _ll, _p, _ll, _p, _p, _p, _ll, _p, _p, _p, _i, _i, _p, _i, _i, _i, _i, _p])
     _status(fn(_ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(wraw), wraw.stride(0), _ptr(w0),
                _ptr(bonus), _ptr(state), state.stride(0), _ptr(entry_start), _ptr(entry_first), _ptr(slots), dim, heads,
-               _ptr(out), num_entries, 1 if short_entries else 0, 1 if decayed else 0, _stream()), "wkv_rule")
+               _ptr(out), num_entries, tokens, 1 if short_entries else 0, 1 if decayed else 0, _stream()), "wkv_rule")
 
 
 def token_shift(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, prev_offset: int, entry_of: torch.Tensor,
