@@ -508,10 +508,9 @@ def test_prompts_recurrences_in_whole_and_partial_blocks(rule, sizes):
 
 
 @pytest.mark.parametrize("rule", ["delta", "delta_channel", "wkv"])
-@pytest.mark.parametrize("sizes", [(1, 2, 4, 9), (2, 4, 64, 16), (1, 3, 68, 8), (2, 2, 128, 24), (3, 6, 40, 130), (1, 60, 64, 20)])
+@pytest.mark.parametrize("sizes", [(2, 4, 4, 9), (2, 4, 64, 16), (1, 3, 68, 8), (2, 2, 128, 24), (3, 6, 40, 130), (1, 60, 64, 20)])
 def test_prompts_recurrences_give_the_same_bits_from_rows_off_16_bytes(rule, sizes):
-    """Rows in whole pieces of 16 bytes go straight into LDS, 32 lanes a value channel (time mixing in blocks of 32 tokens, or of 16
-    for many workgroups); the same numbers a float further on in memory take the general walk: fresh and continued states, whole
+    """Rows in whole pieces of 16 bytes go straight into LDS, 32 lanes a value channel; the same numbers a float further on in memory take the general walk: fresh and continued states, whole
     blocks, remainders and a single token, every output and the states."""
     from vipera_rs_amd.ops import kernels
 
@@ -531,8 +530,11 @@ def test_prompts_recurrences_give_the_same_bits_from_rows_off_16_bytes(rule, siz
     def off_by(floats, t):
         room = torch.empty(t.numel() + floats, device="cuda")
         room[floats:] = t.reshape(-1)
-        return room[floats:].view(t.shape)
+        given = room[floats:].view(t.shape)
+        assert given.stride(0) % 4 == 0 and given.data_ptr() % 16 == 4 * floats     # what the two walks are told apart by
+        return given
 
+    assert dim % 4 == 0 and channels % 4 == 0      # the column of the decays
     got = []
     for floats in (0, 1):
         state, out = start.clone(), torch.full((tokens, heads * vdim), float("nan"), device="cuda")

@@ -900,7 +900,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
 // of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here (in blocks of 32 /
 // 16): 32 heads of 64, one entry of 2,048 tokens 168 / 108 / 127, of 512 46 / 31 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
 // 512, 456 and 399 (768) 82 / 55 / 59, eight of 250 (2,048) 115 / 84 / 75.  Entries that have no block of 32
-// are walked in blocks of 16: 31 tokens in either 6.5 / 6.0, 16 tokens 5.0 / 4.3.
+// are walked in blocks of 16: 31 tokens of 16 heads in either 6.5 / 5.6, 16 tokens 5.0 / 4.0.
 constexpr int WKV_LONG_BLOCKS = 3 * 256;      // workgroups up to which blocks are of 32 tokens
 template <int Q, int BLOCK>
 __global__ __launch_bounds__(SCAN_COLS * 32) void wkv_scan_direct_kernel(
