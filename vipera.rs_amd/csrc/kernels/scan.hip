@@ -456,10 +456,12 @@ static int launch_decay_rule(const float* q, const float* k, long long ldqk, con
 #define VK_RUN_AS(RR, ALL, VEC)                                                                                              \
   decay_run_kernel<RR, ALL, VEC><<<run_grid, RUN_THREADS, 0, s>>>(q, k, ldqk, v, ldv, decay, state, state_stride, entry_start, \
                                                                   entry_first, slots, heads, dim, vdim, o)
+#define VK_RUN_EACH(RR)                                \
+  if (dim == 16 * RR) VK_RUN_AS(RR, true, false);      \
+  else VK_RUN_AS(RR, false, false)
 #define VK_RUN(RR)                              \
   if (quads) VK_RUN_AS(RR, true, true);         \
-  else if (dim == 16 * RR) VK_RUN_AS(RR, true, false); \
-  else VK_RUN_AS(RR, false, false)
+  else VK_RUN_EACH(RR)
 #define VK_RUN_DIRECT(RR)                                                                                                     \
   decay_run_direct_kernel<RR><<<run_grid, RUN_THREADS, 0, s>>>(q, k, ldqk, v, ldv, decay, state, state_stride, entry_start,     \
                                                                entry_first, slots, heads, vdim, o)
@@ -467,11 +469,12 @@ static int launch_decay_rule(const float* q, const float* k, long long ldqk, con
     switch (share) {
       case 1: VK_RUN(1); break;
       case 2: VK_RUN(2); break;
-      case 4: if (direct) VK_RUN_DIRECT(4); else VK_RUN(4); break;
-      case 8: if (direct) VK_RUN_DIRECT(8); else VK_RUN(8); break;
+      case 4: if (direct) VK_RUN_DIRECT(4); else VK_RUN_EACH(4); break;
+      case 8: if (direct) VK_RUN_DIRECT(8); else VK_RUN_EACH(8); break;
       default: VK_RUN(16); break;
     }
 #undef VK_RUN
+#undef VK_RUN_EACH
 #undef VK_RUN_AS
 #undef VK_RUN_DIRECT
     VK_LAUNCH_CHECK();
