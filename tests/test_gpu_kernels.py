@@ -1683,3 +1683,22 @@ def test_gated_32_bit_product_leaves_what_it_cannot_take():
     room = torch.ones(65 * 64 + 1, device="cuda")
     assert not kernels.gemm_generic_gated(room[1:].view(65, 64), w[:, :64].contiguous(), out)     # rows off 16 bytes
     assert not out.any()
+
+
+def test_gated_32_bit_layer_may_write_over_its_input():
+    from vipera_rs_amd.ops import kernels
+    from vipera_rs_amd.ops.linear import linear_gated
+
+    gen = torch.Generator("cuda").manual_seed(8)
+    m, k = 130, 896
+    room, w = torch.randn(2 * m, k, generator=gen, device="cuda"), torch.randn(2 * k, k, generator=gen, device="cuda") * k ** -0.5
+    for at in (0, 7, 129, 130):                # the input's own rows, rows that overlap with them, and the next ones
+        a = room.clone()[:m]
+        out = a.as_strided((m, k), (k, 1), at * k)
+        assert kernels.gemm_generic_gated(a, w, torch.empty_like(a))
+        want = torch.empty_like(a)
+        linear_gated(a, w, want, False)
+        if at < m:
+            assert not kernels.gemm_generic_gated(a, w, out)
+        linear_gated(a, w, out, False)
+        assert torch.equal(out, want)

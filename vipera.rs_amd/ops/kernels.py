@@ -259,7 +259,8 @@ def gemm_generic_gated_pays(m: int, inter: int, k: int) -> bool:
 def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     """``out = up(a) * silu(gate(a))`` of 32-bit operands with ``w = [gate; up]``, in the product's own launch and with the bits of
     :func:`gemm_generic` and :func:`swiglu` behind it; False, and nothing launched, where these are to be used: up to 8 tokens, which are a
-    stream of the weights, rows off 16 bytes, and sizes whose product leaves parts of its sums in memory."""
+    stream of the weights, rows off 16 bytes, sizes whose product leaves parts of its sums in memory, and an ``out`` in ``a``'s own
+    memory, which workgroups would overwrite while others read it."""
     _dev(a, w, out)
     m, k = a.shape
     inter = out.shape[1]
@@ -267,7 +268,8 @@ def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> b
         return False
     lda = a.stride(0)
     if not (a.stride(1) == 1 and lda >= k and w.is_contiguous() and out.is_contiguous() and lda % 4 == 0 and k % 4 == 0
-            and lda <= GEMM_DIRECT_MAX_ROW and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _gemm_gated_takes(m, inter, k)):
+            and lda <= GEMM_DIRECT_MAX_ROW and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _gemm_gated_takes(m, inter, k)
+            and (out.data_ptr() >= a.data_ptr() + 4 * ((m - 1) * lda + k) or out.data_ptr() + 4 * m * inter <= a.data_ptr())):
         return False
     fn = _fn("gemm_generic", "vk_gemm_generic_gated", [_p, _p, _p, _i, _i, _i, _ll, _ll, _p])
     _status(fn(_ptr(a), _ptr(w), _ptr(out), m, inter, k, lda, inter, _stream()), "gemm_generic_gated")
