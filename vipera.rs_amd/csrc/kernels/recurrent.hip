@@ -589,9 +589,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void delta_scan_kernel(
 // faster on two, so that a token's step is worth what its instructions take (some 39 here for two value channels, 36 above for
 // one), and what a block costs besides is worth its share of sixteen tokens: here a block goes straight from memory into LDS in
 // pieces of 16 bytes, whose places are worked out once, and LDS reads and the read-out's products stand between the exchanges
-// of the update's sum, which would wait there.  us, above and here: 16 heads of 128 x 128, one entry of 2,048 tokens 287 / 219, of 512 77 / 60,
-// of 1,000 and 834 215 / 155, eight of 250 206 / 136; 8 heads, 2,048 tokens 265 / 209; 6 heads of 64 x 64, 512, 456 and 399 63 / 50; with
-// a decay per key channel, 16 heads 300 / 228.  Tokens of 31 and fewer cost the same either way.
+// of the update's sum, which would wait there.  us, above and here, launches behind one another in a graph: 16 heads of 128 x 128, one entry of
+// 2,048 tokens 259 / 200, of 512 67 / 53, of 1,000 and 834 194 / 135, eight of 250 169 / 114, of 31 8.1 / 7.4; 8 heads, 2,048 tokens 255 / 196; 6 heads of
+// 64 x 64, 512, 456 and 399 59 / 46; with a decay per key channel, 16 heads 277 / 209.
 template <int Q, bool CH>
 __global__ __launch_bounds__(SCAN_COLS * 32) void delta_scan_direct_kernel(
     const float* __restrict__ qkv, long long ldq, int g_col, const float* __restrict__ beta,
@@ -897,9 +897,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void wkv_scan_kernel(
 // The time mixing for head widths up to 128 in whole pieces of 16 bytes and decays taken beforehand, shaped as
 // delta_scan_direct_kernel is, with every number formed as above: 32 lanes a value channel, some 16 instructions a token for two of
 // them (13 above for one).  Nothing waits for a token's sums over the lanes, so sixteen tokens' go through the tree together.  Blocks
-// of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here (in blocks of 32 /
-// 16): 32 heads of 64, one entry of 2,048 tokens 168 / 108 / 127, of 512 46 / 31 / 36, of 1,000 and 834 (512 workgroups) 124 / 82 / 87, of
-// 512, 456 and 399 (768) 82 / 55 / 59, eight of 250 (2,048) 115 / 84 / 75.  Entries that have no block of 32
+// of 32 tokens cost half as much besides, but leave room for three workgroups a CU instead of six.  us, above and here, as
+// chosen: 32 heads of 64, one entry of 2,048 tokens 154 / 96, of 512 41 / 27, of 1,000 and 834 (512 workgroups) 109 / 70, of 512, 456 and 399
+// (768) 71 / 47, eight of 250 (2,048) 96 / 70; in blocks of 32 / 16, when a block's places were still worked out anew: 108 / 127, 31 / 36, 82 / 87, 55 / 59, 84 / 75.  Entries that have no block of 32
 // are walked in blocks of 16: 31 tokens of 16 heads in either 6.5 / 5.6, 16 tokens 5.0 / 4.0.
 constexpr int WKV_LONG_BLOCKS = 3 * 256;      // workgroups up to which blocks are of 32 tokens
 template <int Q, int BLOCK>
@@ -1435,15 +1435,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void memory_scan_kernel(
 }
 
 // The matrix memory for key widths up to 128 in whole pieces of 16 bytes, with 32 lanes a value channel as in
-// delta_scan_direct_kernel and every number formed as above.  What bounds it is a wave's instructions, some 20 a token for two value
-// channels (25 above for one) and as many as six tokens' besides for a block.  What a token needs once for all its value channels
+// delta_scan_direct_kernel and every number formed as above.  What bounds it is a wave's instructions, in the assembly some 780 for a
+// block of sixteen tokens and two value channels: twenty a token are the recurrence, as many again its LDS reads, the sums through the lanes and n . q, and
+// the rest the block's, 49 a token together or 95 ns at one every 1.95 ns; a token takes 110, and what the others pass with was not measured.  What a token needs once for all its value channels
 // is done before the walk: the wave that has fetched a piece of q or k multiplies it by the scale or by the token's share on its way
 // into LDS, and lane j of a row reads token j's gates itself, whose exponentials are taken among the products of the block before.
 // Four tokens' LDS reads go before the arithmetic of the four before them, sixteen tokens' sums through the lanes together, and a
 // wave works out n . q for four tokens of a block.  (Loads straight into LDS, scaled there: the compiler has every later LDS read of the
-// rows wait for them, 253 us a prompt of 2,048.)  us, above and here, with the gates' kernel: 16 heads of 128 x 128, one entry of 2,048
-// tokens 373 / 233, of 512 97 / 62, of 1,000 and 834 254 / 152, of 512, 456 and 399 200 / 95, eight of 250 251 / 126; 8 heads, 2,048 tokens
-// 361 / 223; 6 heads of 64 x 64, 512, 456 and 399 80 / 49; 31 tokens 13 / 11.
+// rows wait for them, 253 us a prompt of 2,048.)  us, above and here, with the gates' kernel, launches behind one another in a graph: 16 heads of 128 x
+// 128, one entry of 2,048 tokens 363 / 227, of 512 96 / 62, of 1,000 and 834 255 / 151, of 512, 456 and 399 200 / 94, eight of 250 251 / 124; 8 heads,
+// 2,048 tokens 362 / 225; 6 heads of 64 x 64, 512, 456 and 399 81 / 50; 31 tokens 13 / 11.
 template <int Q>
 __global__ __launch_bounds__(SCAN_COLS * 32) void memory_scan_direct_kernel(
     const float* __restrict__ proj, long long ldp, MemoryColumns col, float q_scale,

@@ -293,8 +293,8 @@ __global__ __launch_bounds__(RUN_THREADS) void decay_run_kernel(const float* __r
 // into LDS, in the order in which the lanes read it, from places that are worked out once; two tokens' products, states and sums are
 // three runs of instructions none of which waits for the one before it; and sixteen tokens' sums go through the lanes together.
 // What bounds it is a token's instructions (32 for 8 key channels a lane, of which one goes out every 1.95 ns on a wave alone on
-// its SIMD) and a block's branches and barrier.  us, above and here: 16 heads of 128 x 128, one entry of 2,048 tokens 219 / 182, of 512 59 /
-// 50, of 1,000 and 834 150 / 113, of 512, 456 and 399 82 / 63, eight of 250 104 / 86; 31 tokens cost the same either way.
+// its SIMD) and a block's branches and barrier.  us, above and here, launches behind one another in a graph: 16 heads of 128 x 128, one entry of 2,048
+// tokens 210 / 171, of 512 55 / 45, of 1,000 and 834 139 / 103, of 512, 456 and 399 72 / 54, eight of 250 84 / 74, of 31 7.0 / 6.5.
 template <int R>
 __global__ __launch_bounds__(RUN_THREADS) void decay_run_direct_kernel(
     const float* __restrict__ q, const float* __restrict__ k, long long ldqk, const float* __restrict__ v, long long ldv,
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 // latencies, and sixteen tokens' sums go through the lanes together.  Lane j of a channel's sixteen ends up with token j's sum and
 // finishes that token's output.  What bounds it is the instructions (about 23 a token for a state a lane, fourteen of them the
 // exponential).  ALL: N = 16 R.  4,096 channels of 16 states, with blocks of 16 and every token's sum by itself, and so: portions of
-// 1,000 and 834 tokens 120 -> 111 us, one of 2,048 178 -> 159, of 512 50 -> 44, eight of 250 101 -> 93.  Short entries have no block of 32 and pay for
+// 1,000 and 834 tokens 108 -> 95 us, one of 2,048 165 -> 144, of 512 44 -> 39, eight of 250 85 -> 74.  Short entries have no block of 32 and pay for
 // its stages: in blocks of 32 and of 16, 64 of 20 tokens 72 -> 62 us, 30 of 5 16.4 -> 13.5, one of 16 5.1 -> 4.0.  Beyond 64 states a lane's registers and the stages grow past what the chip holds at once, and the walk above stays.
 template <int R, int BLOCK, bool ALL, typename TO>
 __global__ __launch_bounds__(256) void selective_run_kernel(

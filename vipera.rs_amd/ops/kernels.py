@@ -800,8 +800,9 @@ TILE_TILINGS = {0: "128x128 staged", 2: "256x128 staged", 3: "128x256 staged", 4
 
 def gemm_bf16_tile_plan(m: int, n: int, k: int, gated: bool = False) -> Tuple[int, int]:
     """The tiling (a key of ``TILE_TILINGS``) and the number of ranges of K that the tiled kernel of :func:`gemm_bf16` (or
-    :func:`gemm_bf16_gated`) plans for these sizes; the ranges decide the bits.  A plan of one range, or of 128x128 tiles,
-    may be carried out by another tiling with the same bits: :func:`gemm_bf16_tile_carried_out`."""
+    :func:`gemm_bf16_gated`) plans for these sizes; the ranges decide the bits.  A plan of one range, or of several in
+    128x128 or 64x64 tiles, may be carried out by another tiling with the same bits: :func:`gemm_bf16_tile_carried_out`.  For a plan of
+    several ranges in tiles of 256 tokens the tiling is the one that carries it out."""
     tiling, ranges = _i(), _i()
     fn = _fn("gemm_bf16", "vk_gemm_bf16_tile_plan", [_i, _i, _i, _ll, _i, _p, _p])
     _status(fn(m, n, k, min(8 * m * n, _TILE_WORKSPACE_FLOATS), 1 if gated else 0, ctypes.addressof(tiling),
