@@ -778,12 +778,24 @@ static inline bool moe_loads_direct(int width, int ff, int num_tokens, int top, 
          (long long)num_tokens * top * ff * 2 <= GT_VIEW_BYTES && (long long)width * ff * 2 <= GT_VIEW_BYTES;
 }
 
-// For tile_rows GT_EITHER: column blocks of the experts' products in tiles of 128 columns, their K, and the device's CUs.
-extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int up_blocks,
-                            int down_blocks, int up_k, int down_k, int compute_units, int groups, int keep, int all_scores,
+static int compute_units() {
+  static const int units = [] {
+    int device = 0, count = 0;
+    const bool known = hipGetDevice(&device) == hipSuccess &&
+                       hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && count >= 8;
+    return known ? count : 256;
+  }();
+  return units;
+}
+
+// up_rows (of gate and up both if gated), down_rows: the weight rows of an expert's products, by which tile_rows GT_EITHER chooses; 0: not
+// known, tiles of 128 places.
+extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_tokens, int tile_rows, int up_rows,
+                            int down_rows, int gated, int groups, int keep, int all_scores,
                             const float* correction, float weight_scale, long long ld, int* ids, float* weights, int* offsets, int* order, int* tiles, int* num_tiles, void* stream) {
+  if (tile_rows == GT_EITHER && (up_rows < 1 || down_rows < 1)) tile_rows = GT_TILE;
   if (tile_rows != MOE_TILE && tile_rows != GT_TILE && tile_rows != MOE_FEW && tile_rows != GT_WIDE && tile_rows != GT_MIDDLE &&
-      (tile_rows != GT_EITHER || up_blocks < 1 || down_blocks < 1 || up_k < 1 || down_k < 1 || compute_units < 8))
+      tile_rows != GT_EITHER)
     return VK_BAD_ARGUMENT;
   if (groups < 1 || keep < 1 || keep > groups || experts % groups != 0) return VK_BAD_ARGUMENT;
   if (groups > WAVE) return VK_UNSUPPORTED_SIZE;
@@ -804,7 +816,8 @@ extern "C" int vk_moe_route(const float* logits, int experts, int top, int num_t
   }
   moe_group_kernel<<<1, 1024, (size_t)experts * 2 * sizeof(int), s>>>(together ? logits : nullptr, top, num_tokens,
                                                                        weights, ids, (int)pairs, experts, tile_rows,
-                                                                       Rounds{up_blocks, down_blocks, up_k, down_k, compute_units / 8 * 2},
+                                                                       Rounds{(up_rows + 127) / 128, (down_rows + 127) / 128, down_rows,
+                                                                              gated ? up_rows / 2 : up_rows, compute_units() / 8 * 2},
                                                                        offsets, order, tiles, num_tiles, how);
   VK_LAUNCH_CHECK();
   return 0;

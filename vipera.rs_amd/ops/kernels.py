@@ -256,23 +256,25 @@ def gemm_generic_gated_pays(m: int, inter: int, k: int) -> bool:
     return bool(_fn("gemm_generic", "vk_gemm_generic_gated_pays", [_i, _i, _i])(m, inter, k))
 
 
-def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+def gemm_generic_gated(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, where_faster: bool = False) -> bool:
     """``out = up(a) * silu(gate(a))`` of 32-bit operands with ``w = [gate; up]``, in the product's own launch and with the bits of
     :func:`gemm_generic` and :func:`swiglu` behind it; False, and nothing launched, where these are to be used: up to 8 tokens, which are a
     stream of the weights, rows off 16 bytes, sizes whose product leaves parts of its sums in memory, and an ``out`` in ``a``'s own
-    memory, which workgroups would overwrite while others read it."""
+    memory, which workgroups would overwrite while others read it; with ``where_faster`` also sizes that take longer so
+    (:func:`gemm_generic_gated_pays`)."""
     _dev(a, w, out)
     m, k = a.shape
     inter = out.shape[1]
     if not (m > 8 and a.dtype == w.dtype == out.dtype == torch.float32 and w.shape == (2 * inter, k) and out.shape[0] == m):
         return False
-    lda = a.stride(0)
+    lda, a_at, w_at, out_at = a.stride(0), a.data_ptr(), w.data_ptr(), out.data_ptr()
     if not (a.stride(1) == 1 and lda >= k and w.is_contiguous() and out.is_contiguous() and lda % 4 == 0 and k % 4 == 0
-            and lda <= GEMM_DIRECT_MAX_ROW and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _gemm_gated_takes(m, inter, k)
-            and (out.data_ptr() >= a.data_ptr() + 4 * ((m - 1) * lda + k) or out.data_ptr() + 4 * m * inter <= a.data_ptr())):
+            and lda <= GEMM_DIRECT_MAX_ROW and a_at % 16 == 0 and w_at % 16 == 0
+            and (out_at >= a_at + 4 * ((m - 1) * lda + k) or out_at + 4 * m * inter <= a_at)
+            and (gemm_generic_gated_pays if where_faster else _gemm_gated_takes)(m, inter, k)):
         return False
     fn = _fn("gemm_generic", "vk_gemm_generic_gated", [_p, _p, _p, _i, _i, _i, _ll, _ll, _p])
-    _status(fn(_ptr(a), _ptr(w), _ptr(out), m, inter, k, lda, inter, _stream()), "gemm_generic_gated")
+    _status(fn(a_at, w_at, out_at, m, inter, k, lda, inter, _stream()), "gemm_generic_gated")
     return True
 
 
@@ -1485,16 +1487,13 @@ def moe_route(logits: torch.Tensor, top: int, ids: torch.Tensor, weights: torch.
           and num_tiles.numel() == 1 and tile_rows in (16, 64, MOE_EITHER_ROWS, 128, 192, 256), "moe_route: output sizes")
     _need(1 <= keep <= groups <= 64 and experts % groups == 0 and (keep == groups or keep * (experts // groups) >= top),
           f"moe_route: {keep} of {groups} groups of {experts} experts for top {top}")
-    if tile_rows == MOE_EITHER_ROWS and min(columns) < 1:
-        tile_rows = 128
     mode = {"sigmoid": 2, "steered": 3}.get(all_scores, 1 if all_scores else 0)
     if correction is not None:
         _dev(correction)
         _need(mode == 3 and correction.dtype == torch.float32 and correction.is_contiguous()
               and correction.numel() == experts, "moe_route: one 32-bit correction per expert, with steered scores")
-    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
-    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, -(-columns[0] // 128), -(-columns[1] // 128), columns[1],
-               columns[0] // 2 if gated else columns[0], compute_units(logits.device), int(groups), int(keep), mode, _ptr(correction),
+    fn = _fn("moe", "vk_moe_route", [_p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _f, _ll, _p, _p, _p, _p, _p, _p, _p])
+    _status(fn(_ptr(logits), experts, top, tokens, tile_rows, columns[0], columns[1], gated, int(groups), int(keep), mode, _ptr(correction),
                float(weight_scale), logits.stride(0) if tokens > 1 else experts, _ptr(ids), _ptr(weights), _ptr(offsets),
                _ptr(order), _ptr(tiles), _ptr(num_tiles), _stream()), "moe_route")
 

@@ -206,8 +206,7 @@ def linear_gated(a: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, in
         if m > 4 or plan == 0:
             kernels.gemm_bf16_gated(a, w_gate_up, out, rows_per_wave=plan)
             return out
-    if (not interleaved and a.dtype == torch.float32 and kernels.gemm_generic_gated_pays(m, n // 2, k)
-            and kernels.gemm_generic_gated(a, w_gate_up, out)):
+    if not interleaved and kernels.gemm_generic_gated(a, w_gate_up, out, where_faster=True):
         return out
     gate_up = torch.empty((m, n), dtype=out.dtype, device=out.device)
     linear(a, w_gate_up, None, gate_up)
