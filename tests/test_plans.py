@@ -230,7 +230,8 @@ def test_256x128_tiles_with_few_last_tokens_keep_their_deep_ranges():
     assert carried(575, 2048, 11008) == 7 and carried(572, 2048, 8192) == 7            # 45.2 and 47.7, 35.7 and 39.0: 63 tokens in the last tile
     assert carried(1315, 2048, 11008) == 7 and carried(940, 3072, 8192) == 7           # 74.4 and 80.1, 62.3 and 64.5
     assert carried(649, 4096, 14336) == 18 and carried(1241, 1792, 7168) == 18         # 98.4 and 83.0, 56.3 and 46.2
-    assert carried(575, 2560, 10240) == 7 and carried(575, 2048, 4096) == 18           # ranges of 2,560 (47.0 and 45.4) and 1,024 (27.0 and 25.6)
+    assert carried(575, 2560, 10240) == 18 and carried(575, 2048, 4096) == 18          # 47.0 and 45.4: 240 tiles; 27.0 and 25.6: ranges of 1,024
+    assert carried(134, 3584, 18944) == 18 and carried(1032, 2560, 10240) == 18        # 46.9 and 44.5: a single tile of tokens; 69 and 62
     assert carried(945, 1536, 8960) == 18                                              # 42.2 and 39.8
 
 

@@ -2098,16 +2098,18 @@ int one_round_tile(int planned, double limit_us, int M, int N, int K, int ranges
   }
   return planned;
 }
-// 256x128 tiles whose last tokens are few are not changed for deep ranges: rows that do not exist cost their waves nothing, the tiles of 192 tokens
-// have as many rows that do, and it is the work that a deep range takes. us, 256x128 and 192x128: 575 tokens on 2,048 rows of 11,008 in four
-// ranges 45.2 / 47.7, 572 of 8,192 35.7 / 39.0, 1,315 of 11,008 in two 74.4 / 80.1, 940 on 3,072 of 8,192 62.3 / 64.5. Of 263 products planned as 256x128 on
-// 25 shapes of 512 to 4,608 rows, 131 to 2,000 tokens, 77 stay; the others take 0.91 of the time, 1.015 at worst.
-bool stays_256x128(int M, int K, int ranges) {
-  const long long wide = (M + 255) / 256 * 256, narrow = (M + 191) / 192 * 192;
-  return (K / ranges >= 2048 && wide * 10 > narrow * 11) || (K / ranges >= 4096 && wide * 20 > narrow * 21);
+// 256x128 tiles stay for deep ranges where they multiply a tenth more tokens than 192x128 ones and are at most three for four CUs: rows that do
+// not exist cost their waves nothing, so the smaller tiles' work is as much, and a deep range takes as long as its work. us, 256x128 and 192x128: 575
+// tokens on 2,048 rows of 11,008 in four ranges 45.2 / 47.7, 572 of 8,192 35.7 / 39.0, 1,315 of 11,008 in two 74.4 / 80.1, 940 on 3,072 of 8,192 (a
+// fifteenth more, ranges of 4,096) 62.3 / 64.5. Of 263 products planned as 256x128 on 25 shapes of 512 to 4,608 rows, 131 to 2,000 tokens, 40 stay, which
+// would take as long on average (0.91 to 1.09), and the others take 0.914 of the time, 1.002 at worst.
+bool stays_256x128(int M, int N, int K, int ranges) {
+  const long long wide = (M + 255) / 256, narrow = (M + 191) / 192, tiles = wide * ((N + 127) / 128) * ranges;
+  if (wide == 1 || tiles * 4 > 3LL * g_compute_units || K / ranges < 2048) return false;
+  return wide * 256 * 100 > narrow * 192 * (K / ranges >= 4096 ? 105 : 112);
 }
 int split_tile(int planned, int M, int N, int K, int ranges) {
-  if (planned == 7 && stays_256x128(M, K, ranges)) return planned;
+  if (planned == 7 && stays_256x128(M, N, K, ranges)) return planned;
   for (const TileCost& t : WHOLE_TILES)
     if (t.config == planned) return one_round_tile(planned, 0.98 * whole_tile_us(t, M, N, K, 4.0, ranges), M, N, K, ranges, false);
   return planned;
