@@ -242,6 +242,9 @@ def test_split_small_tiles_give_way_where_the_larger_ones_are_faster():
     assert carried(204, 1280, 5120) == 17 and carried(204, 2560, 4096) == 17      # 16.9 and 16.8, 20.1 and 19.0: 640
     assert carried(319, 896, 4864) == 16 and carried(572, 512, 8192) == 16        # 15.0 and 14.9, 17.9 and 17.2: 560 and 576
     assert carried(200, 1024, 4096) == 13                                         # 512, two a CU
+    # 14: 64x64 that walk K
+    assert carried(771, 896, 4864) == 14 and carried(797, 1024, 8192) == 17       # 17.5 and 19.4, 32.3 and 27.5
+    assert carried(568, 1536, 8960) == 17 and carried(133, 3584, 3584) == 16      # 42.2 and 30.2, 17.6 and 16.9
 
 
 def _walked(reach, tokens, window, keep_first=0):

@@ -2117,7 +2117,7 @@ int split_tile(int planned, int M, int N, int K, int ranges) {
 
 // The same where 64x64 tiles were to carry several ranges out, with 192x64 among those offered: in place of split ones (13) that
 // are more than two a CU, and of ones that walk K (14) where the estimate with the sums' way through memory and a second launch is below
-// 0.95 of the walk's (2.5 us and 0.27 a step of 64). Of 101 products planned as small tiles 18 change, to 0.88 of their time, 0.94 at worst:
+// 0.95 of the walk's (2.5 us and 0.27 a step of 64, 0.20 below 1,024 rows: 771 tokens on 896 of 4,864 17.5, 19.4 as 128x128). Of 101 products planned as small tiles 18 change, to 0.88 of their time, 0.94 at worst:
 // us, 130 tokens on 2,048 rows of 8,192 22.1 / 18.2, 311 on 2,048 of 4,096 22.3 / 18.2, 622 on 896 of 4,864 21.5 / 18.3, and walked 622 on
 // 1,536 of 8,960 40.4 / 32.9, 512 on 2,048 of 8,192 35.2 / 29.6. Up to two a CU the split small tiles stay ahead by 4 to 15 %; past two
 // they are not estimated: what comes in one round takes their place, 128x128 tiles from nine for four CUs on (204 to 250 tokens on 1,152 rows of
@@ -2131,7 +2131,7 @@ int split_small_tile(int planned, int M, int N, int K, int ranges) {
   }
   if (planned == 14) {
     const double sums = (2.0 * ranges + 1.0) * 4.0 * M * N / 6e6 + 3.0;
-    return one_round_tile(14, 0.95 * (2.5 + 0.27 * (K / 64)) - sums, M, N, K, ranges, true);
+    return one_round_tile(14, 0.95 * (2.5 + (N < 1024 ? 0.20 : 0.27) * (K / 64)) - sums, M, N, K, ranges, true);
   }
   return planned;
 }
